@@ -614,6 +614,35 @@ def test_truncated_sampler_matches_oracle(dtype, V, T, top_k, top_p):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("V", [512, 8704, 32768])
+@pytest.mark.parametrize("top_k,top_p", [(1, 0.5), (3, 0.3), (40, 0.999), (511, 0.6), (511, 1.0), (0, 0.02), (0, 0.9999)])
+def test_truncated_sampler_threshold_on_hard_rows(V, top_k, top_p):
+    """The kept set on rows that put the radix walk on its edges - all logits equal, two values, one value far above the rest,
+    values that differ in the last bit only, logits so low that every mass rounds to zero - against the definition on the
+    same exponentials (read back as thresholds): every key above the threshold is kept and the cut is the smallest such."""
+    from ultraviolet_amd.kernels.fused_sample import sample_filtered
+    g = torch.Generator().manual_seed(V + top_k)
+    r = torch.randn(V, generator=g) * 3
+    rows = [torch.full((V,), 1.5), torch.where(r > 0, 2.0, -2.0), torch.where(torch.arange(V) == V - 7, 30.0, -3.0), 4.0 + r.sign() * 2 ** -7,
+            torch.full((V,), -200.0), r]
+    x = torch.stack(rows).bfloat16()
+    u = torch.tensor([0.0, 0.3, 0.999999, 0.5, 0.7, 0.1])
+    t, _, thr = sample_filtered(x.to(DEV), u.to(DEV), SC, 1.0, top_k, top_p, return_threshold=True)
+    t, thr = t.cpu().numpy(), thr.cpu().double().numpy()
+    e = np.exp(SC[0] / (1.0 + np.exp(-(to_np(x).astype(np.float64) + SC[1]) / SC[2])) - SC[0])
+    for i in range(len(rows)):
+        s = np.sort(e[i])[::-1]
+        n = int((e[i] >= s[top_k - 1]).sum()) if 0 < top_k < V else V
+        if top_p < 1.0:
+            c = np.cumsum(s[:n])
+            n = int((e[i] >= s[min(np.searchsorted(c, top_p * c[-1] * (1 - 1e-9)), n - 1)]).sum()) if c[-1] > 2.0 ** -20 else int((e[i] == s[0]).sum())
+        kept = e[i] >= thr[i] * (1 - 2e-6)
+        assert kept[t[i]]
+        # (a cut that the last bits of the exponentials move takes or leaves values within rounding of each other)
+        assert abs(int(kept.sum()) - n) <= 2 or np.ptp(s[min(kept.sum(), n) - 1:max(kept.sum(), n)]) <= 1e-2 * s[n - 1], (i, int(kept.sum()), n)
+
+
+@pytest.mark.gpu
 def test_truncated_sampler_off_equals_plain_and_seeded_draw():
     from ultraviolet_amd.kernels.fused_sample import fused_sample, fused_sample_seeded, sample_filtered
     g = torch.Generator().manual_seed(9)

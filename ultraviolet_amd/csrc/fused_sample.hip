@@ -173,133 +173,176 @@ __global__ __launch_bounds__(NT) void sample_kernel(const void* a_x, int64_t a_s
 // least the k-th largest, then of those the smallest prefix by probability whose mass reaches top_p (the token that
 // crosses it included, ties of the last kept value all kept), and draw from what is kept by inverse CDF in index order.
 // Everything is decided on e = exp((z - a)/T), which is positive and monotone in the logit, so its fp32 bit pattern
-// orders the tokens: both thresholds are found by a radix select over those 32 bits, 8 bits per sweep of the row (the row
-// stays in cache between sweeps).  The nucleus select walks the digits by probability mass; masses are summed as 32.32
-// fixed point in 64-bit integers, so the histogram does not depend on the order in which lanes add to it.  The behaviour
-// log-prob is that of the unfiltered softmax, as the reference records it (model.py:1161-1169).
+// orders the tokens: both thresholds are found by a radix select over those 32 bits.  The behaviour log-prob is that of the
+// unfiltered softmax, as the reference records it (model.py:1161-1169).
+//
+// What bounds it: one row per workgroup is a serial chain of selects, so the chain is kept short.  The row is read once and
+// its exponentials stay in registers (1024 threads x 32 elements); the digits are 12 + 10 + 10 bits, so a threshold takes
+// three histograms, and the first digit (8 exponent bits and 3 of the mantissa) already spreads a row over tens of
+// bins, which keeps the LDS atomics of a wave from meeting on one address.  A bin holds the count (16 bits) and the mass
+// (48 bits, 32.32 fixed point: sums do not depend on the order of the additions) of its keys in one 64-bit word, so one
+// histogram serves both selects: the nucleus walk starts on the histograms that the top-k walk left and only builds new
+// ones for the bins in which it ends elsewhere.  200 rows x 32768, top_k 50 + top_p 0.95: 203 us for eleven sweeps of the
+// row with 8-bit digits, one thread walking each histogram; 27 us as it is now.
+constexpr unsigned long long BIN_ONE = 1ull << 48, BIN_MASS = BIN_ONE - 1;
+
+// floor(e * 2^32) for 0 <= e <= 1
+__device__ __forceinline__ unsigned long long fix32(float e) {
+  const uint32_t b = __float_as_uint(e);
+  const int sh = (int)(b >> 23) - 118;   // e = m * 2^(exponent - 150)
+  const uint32_t m = (b & 0x7fffffu) | 0x800000u;
+  return sh >= 0 ? (unsigned long long)m << sh : (unsigned long long)(sh > -24 ? m >> -sh : 0u);
+}
+
+struct BinPick { unsigned int digit, cnt_above; unsigned long long mass_above, mass; };
+
+// The bin of a histogram of 1024 * PER bins in which a walk from the largest key down ends: by count (the bin with the
+// want-th largest key) or by mass (the first bin at which the mass reaches `want`; the largest key's bin when want is 0).
+// All 1024 threads call it; total is the whole histogram's word.
+template <int PER, bool BY_MASS>
+__device__ __forceinline__ BinPick pick_bin(const unsigned long long* h, unsigned long long want, unsigned long long* wtot, BinPick* sh,
+                                            unsigned long long& total) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  unsigned long long v[PER], sum = 0;
+#pragma unroll
+  for (int i = 0; i < PER; i++) {
+    v[i] = h[1024 * PER - 1 - (tid * PER + i)];
+    sum += v[i];
+  }
+  unsigned long long incl = sum;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const unsigned long long t = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += t;
+  }
+  if (lane == 63) wtot[wave] = incl;
+  __syncthreads();
+  unsigned long long run = incl - sum;
+  total = 0;
+#pragma unroll
+  for (int w = 0; w < 16; w++) {
+    const unsigned long long t = wtot[w];
+    if (w < wave) run += t;
+    total += t;
+  }
+#pragma unroll
+  for (int i = 0; i < PER; i++) {
+    const unsigned long long above = run;
+    run += v[i];
+    const unsigned long long ca = above >> 48, c = v[i] >> 48, ma = above & BIN_MASS, m = v[i] & BIN_MASS;
+    const bool here = BY_MASS ? c > 0 && (want == 0 ? ca == 0 : ma < want && ma + m >= want) : ca < want && ca + c >= want;
+    if (here) *sh = BinPick{(unsigned int)(1024 * PER - 1 - (tid * PER + i)), (unsigned int)ca, ma, m};
+  }
+  __syncthreads();
+  const BinPick r = *sh;
+  __syncthreads();   // (the next pick writes wtot and sh)
+  return r;
+}
+
 template <int DT>
-__global__ __launch_bounds__(256) void sample_filtered_kernel(SampleParams P) {
+__global__ __launch_bounds__(1024) void sample_filtered_kernel(SampleParams P) {
   __shared__ float csum[64 + 4];
-  __shared__ unsigned int hcnt[256];
-  __shared__ unsigned long long hmass[256];
-  __shared__ unsigned int sh_prefix, sh_krem;
-  __shared__ unsigned long long sh_mhi, sh_zk;
+  __shared__ unsigned long long h1[4096], h2[1024], h3[1024], wtot[16];
+  __shared__ BinPick sh;
   const int row = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, tid = threadIdx.x;
   const char* xr = (const char*)P.x + (int64_t)row * P.stride * (DT == UVMI_F32 ? 4 : 2);
-  const int nchunks = P.V / CHUNK;
-  const int nvec = P.V / 8;
-  auto fix = [](float e) -> unsigned long long { return (unsigned long long)((double)e * 4294967296.0); };
+  const int nchunks = P.V / CHUNK;   // <= 64: wave w holds chunks w, w + 16, w + 32, w + 48
 
-  // ---- unfiltered sum S (for the log-prob), in the order of the unfiltered kernel
-  for (int c = wave; c < nchunks; c += 4) {
-    float v[8];
-    load8<DT>(xr, c * 64 + lane, v);
-    float s = 0.f;
+  float e[4][8];
 #pragma unroll
-    for (int j = 0; j < 8; j++) s += e_of(v[j], P);
-    s = wave_sum(s);
-    if (lane == 0) csum[c] = s;
+  for (int q = 0; q < 4; q++) {
+    const int c = wave + 16 * q;
+    if (c < nchunks) load8<DT>(xr, c * 64 + lane, e[q]);
+  }
+  for (int i = tid; i < 4096; i += 1024) h1[i] = 0;
+  h2[tid] = 0;
+  h3[tid] = 0;
+  // ---- unfiltered chunk sums (for the log-prob), in the order of the unfiltered kernel
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const int c = wave + 16 * q;
+    if (c < nchunks) {
+      float s = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        e[q][j] = e_of(e[q][j], P);
+        s += e[q][j];
+      }
+      s = wave_sum(s);
+      if (lane == 0) csum[c] = s;
+    }
   }
   __syncthreads();
   float S = 0.f;
-  for (int c = 0; c < nchunks; c++) S += csum[c];
-  __syncthreads();
+  if (wave == 0)
+    for (int c = 0; c < nchunks; c++) S += csum[c];
 
-  // ---- top-k: the k-th largest key
-  unsigned int thr = 0;  // keep keys >= thr
-  if (P.top_k > 0 && P.top_k < P.V) {
-    unsigned int prefix = 0, mask = 0, krem = (unsigned int)P.top_k;
-    for (int shift = 24; shift >= 0; shift -= 8) {
-      hcnt[tid] = 0;
-      __syncthreads();
-      for (int i = tid; i < nvec; i += 256) {
-        float v[8];
-        load8<DT>(xr, i, v);
+  // keys whose bits above SHIFT + NBITS equal `prefix` into h, by the NBITS bits at SHIFT
+  auto histogram = [&](unsigned long long* h, int shift, int nbits, unsigned int prefix) {
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+      if (wave + 16 * q < nchunks) {
 #pragma unroll
         for (int j = 0; j < 8; j++) {
-          const unsigned int key = __float_as_uint(e_of(v[j], P));
-          if ((key & mask) == prefix) atomicAdd(&hcnt[(key >> shift) & 255u], 1u);
+          const unsigned int key = __float_as_uint(e[q][j]);
+          if (nbits + shift == 32 || (key >> (shift + nbits)) == prefix)
+            atomicAdd(&h[(key >> shift) & ((1u << nbits) - 1u)], BIN_ONE | fix32(e[q][j]));
         }
       }
-      __syncthreads();
-      if (tid == 0) {
-        unsigned int c = 0;
-        int d = 255;
-        for (; d > 0; d--) {
-          if (c + hcnt[d] >= krem) break;
-          c += hcnt[d];
-        }
-        sh_prefix = prefix | ((unsigned int)d << shift);
-        sh_krem = krem - c;
-      }
-      __syncthreads();
-      prefix = sh_prefix; krem = sh_krem;
-      mask |= 255u << shift;
-      __syncthreads();
-    }
-    thr = prefix;
+    __syncthreads();
+  };
+  auto clear = [&](unsigned long long* h) { h[tid] = 0; };
+
+  histogram(h1, 20, 12, 0);
+  unsigned int thr = 0, d1 = 0, d2 = 0;   // keep keys >= thr
+  unsigned long long zk = 0, above1 = 0, above2 = 0, tot;
+  const bool by_count = P.top_k > 0 && P.top_k < P.V;
+  if (by_count) {
+    unsigned int krem = (unsigned int)P.top_k;
+    BinPick b = pick_bin<4, false>(h1, krem, wtot, &sh, tot);
+    d1 = b.digit; krem -= b.cnt_above; above1 = b.mass_above;
+    histogram(h2, 10, 10, d1);
+    b = pick_bin<1, false>(h2, krem, wtot, &sh, tot);
+    d2 = b.digit; krem -= b.cnt_above; above2 = b.mass_above;
+    histogram(h3, 0, 10, (d1 << 10) | d2);
+    b = pick_bin<1, false>(h3, krem, wtot, &sh, tot);
+    thr = (d1 << 20) | (d2 << 10) | b.digit;
+    zk = above1 + above2 + b.mass_above + b.mass;
   }
-
-  // ---- nucleus: the smallest key whose mass of strictly larger keys is below top_p * (mass of the top-k set)
+  // ---- nucleus: the smallest key whose mass of strictly larger keys is below top_p * (mass of the top-k set).  Bins above
+  // the top-k threshold's are whole, so a walk that ends in one of them never meets a key below the threshold.
   if (P.top_p < 1.0f) {
-    if (tid == 0) sh_zk = 0;
-    __syncthreads();
-    unsigned long long part = 0;
-    for (int i = tid; i < nvec; i += 256) {
-      float v[8];
-      load8<DT>(xr, i, v);
-#pragma unroll
-      for (int j = 0; j < 8; j++) {
-        const float e = e_of(v[j], P);
-        if (__float_as_uint(e) >= thr) part += fix(e);
-      }
-    }
-    atomicAdd(&sh_zk, part);
-    __syncthreads();
     const double tp = P.top_p > 0.f ? (double)P.top_p : 0.0;
-    const unsigned long long target = (unsigned long long)(tp * (double)sh_zk);
-    unsigned int prefix = 0, mask = 0;
-    unsigned long long mhi = 0;
-    for (int shift = 24; shift >= 0; shift -= 8) {
-      hcnt[tid] = 0;
-      hmass[tid] = 0;
-      __syncthreads();
-      for (int i = tid; i < nvec; i += 256) {
-        float v[8];
-        load8<DT>(xr, i, v);
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-          const float e = e_of(v[j], P);
-          const unsigned int key = __float_as_uint(e);
-          if (key >= thr && (key & mask) == prefix) {
-            const unsigned int d = (key >> shift) & 255u;
-            atomicAdd(&hcnt[d], 1u);
-            atomicAdd(&hmass[d], fix(e));
-          }
-        }
-      }
-      __syncthreads();
-      if (tid == 0) {
-        // walk the digits downwards; `run` is the mass above the digit.  The last non-empty digit reached while run <
-        // target holds the cut; when even the largest key fails (top_p = 0) it is kept anyway, as the first token is.
-        unsigned long long run = mhi, above = mhi;
-        int dsel = -1;
-        for (int d = 255; d >= 0; d--) {
-          if (hcnt[d] == 0) continue;
-          if (dsel >= 0 && run >= target) break;
-          dsel = d; above = run;
-          run += hmass[d];
-        }
-        if (dsel < 0) dsel = 0;
-        sh_prefix = prefix | ((unsigned int)dsel << shift);
-        sh_mhi = above;
-      }
-      __syncthreads();
-      prefix = sh_prefix; mhi = sh_mhi;
-      mask |= 255u << shift;
-      __syncthreads();
+    if (!by_count) {
+      pick_bin<4, true>(h1, 0, wtot, &sh, tot);
+      zk = tot & BIN_MASS;
     }
-    thr = prefix;  // (a key of the top-k set, so >= the top-k threshold)
+    unsigned long long want = (unsigned long long)(tp * (double)zk);
+    bool same = by_count;   // the walk is still on the top-k threshold's path: its histogram of this level is there
+    if (!(same && want > above1)) {
+      const BinPick b = pick_bin<4, true>(h1, want, wtot, &sh, tot);
+      same = same && b.digit == d1;
+      d1 = b.digit; above1 = b.mass_above;
+    }
+    want -= want ? above1 : 0;
+    if (!same) {
+      clear(h2);
+      __syncthreads();
+      histogram(h2, 10, 10, d1);
+    }
+    if (!(same && want > above2)) {
+      const BinPick b = pick_bin<1, true>(h2, want, wtot, &sh, tot);
+      same = same && b.digit == d2;
+      d2 = b.digit; above2 = b.mass_above;
+    }
+    want -= want ? above2 : 0;
+    if (!same) {
+      clear(h3);
+      __syncthreads();
+      histogram(h3, 0, 10, (d1 << 10) | d2);
+    }
+    const BinPick b = pick_bin<1, true>(h3, want, wtot, &sh, tot);
+    thr = (d1 << 20) | (d2 << 10) | b.digit;
   }
   auto e_kept = [&](float x) -> float {
     const float e = e_of(x, P);
@@ -307,14 +350,16 @@ __global__ __launch_bounds__(256) void sample_filtered_kernel(SampleParams P) {
   };
 
   // ---- draw from the kept tokens: chunk sums, then the chunk, the lane, the element (as the unfiltered kernel)
-  for (int c = wave; c < nchunks; c += 4) {
-    float v[8];
-    load8<DT>(xr, c * 64 + lane, v);
-    float s = 0.f;
 #pragma unroll
-    for (int j = 0; j < 8; j++) s += e_kept(v[j]);
-    s = wave_sum(s);
-    if (lane == 0) csum[c] = s;
+  for (int q = 0; q < 4; q++) {
+    const int c = wave + 16 * q;
+    if (c < nchunks) {
+      float s = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; j++) s += __float_as_uint(e[q][j]) >= thr ? e[q][j] : 0.f;
+      s = wave_sum(s);
+      if (lane == 0) csum[c] = s;
+    }
   }
   __syncthreads();
   if (wave != 0) return;
@@ -344,13 +389,13 @@ __global__ __launch_bounds__(256) void sample_filtered_kernel(SampleParams P) {
   // so the chosen chunk always holds a kept token unless rounding pushed target past the total: then walk back)
   while (ck > 0 && (ck > 0 ? __shfl(incl, ck - 1, 64) : 0.f) >= Sk) ck--;
   const float before = ck > 0 ? __shfl(incl, ck - 1, 64) : 0.f;
-  float v[8], e[8];
+  float v[8], ek[8];
   load8<DT>(xr, ck * 64 + lane, v);
   float ls = 0.f;
 #pragma unroll
   for (int j = 0; j < 8; j++) {
-    e[j] = e_kept(v[j]);
-    ls += e[j];
+    ek[j] = e_kept(v[j]);
+    ls += ek[j];
   }
   float linc = ls;
 #pragma unroll
@@ -375,7 +420,7 @@ __global__ __launch_bounds__(256) void sample_filtered_kernel(SampleParams P) {
   bool found = false;
 #pragma unroll
   for (int j = 0; j < 8; j++) {
-    const float ej = __shfl(e[j], ln, 64), xj = __shfl(v[j], ln, 64);
+    const float ej = __shfl(ek[j], ln, 64), xj = __shfl(v[j], ln, 64);
     if (ej > 0.f && !found) {
       run += ej;
       sel = ln * 8 + j; xsel = xj;
@@ -486,7 +531,7 @@ extern "C" int uvmi_fused_sample(const uvmi_sample_args* a, void* stream) {
   }
   const bool filtered = !greedy && (P.top_k > 0 || P.top_p < 1.0f);
   hipStream_t st = (hipStream_t)stream;
-  const dim3 grid(a->B), blk(256);
+  const dim3 grid(a->B), blk(filtered ? 1024 : 256);
 #define UVMI_S(K)                                                                          \
   do {                                                                                     \
     if (a->x_dtype == UVMI_F16) hipLaunchKernelGGL((K<UVMI_F16>), grid, blk, 0, st, P);    \
