@@ -6,6 +6,7 @@ Mirror of ultraviolet/kernels/decode_attn.py of the reference (`decode_attention
 from __future__ import annotations
 
 import ctypes as C
+import functools
 
 import torch
 from torch import Tensor
@@ -13,17 +14,22 @@ from torch import Tensor
 from .. import _lib as L
 
 
+@functools.lru_cache(maxsize=None)
+def _device_cus(index: int) -> int:
+    """Compute units of a device, asked once per device."""
+    with torch.cuda.device(index):
+        cus = L.lib().uvmi_device_cus()
+    if cus <= 0:
+        raise L.UvmiError(L.lib().uvmi_last_error().decode())
+    return cus
+
+
 def default_splits(n_bk: int, ctx: int, device=None, min_chunk: int = 256, waves: int = 1) -> int:
     """Splits per (row, kv head) (reference: decode_attn.py:121-129, re-derived for MI355X).  Each (row, kv head,
     split) is one workgroup whose 4 waves stream interleaved key tiles, so a row is only cut when there are fewer rows
     than `waves` workgroups per compute unit, and never into chunks shorter than min_chunk keys."""
-    if device is not None:
-        with torch.cuda.device(device):
-            cus = L.lib().uvmi_device_cus()
-    else:
-        cus = L.lib().uvmi_device_cus()
-    if cus <= 0:
-        raise L.UvmiError(L.lib().uvmi_last_error().decode())
+    index = None if device is None else torch.device(device).index
+    cus = _device_cus(torch.cuda.current_device() if index is None else index)
     want = -(-waves * cus // max(int(n_bk), 1))
     return int(max(1, min(want, max(1, int(ctx) // min_chunk), 64)))
 
@@ -53,23 +59,15 @@ def build_attn_args(q, k_cache, v_cache, pos, starts, scale, window, ring, k_sca
     if num_splits > 1:
         ws_bytes = L.lib().uvmi_decode_attn_workspace_bytes(B, H, KH, hd, num_splits)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
-    a = L.AttnArgs()
-    a.q, a.q_dtype, a.sqb, a.sqh = q.data_ptr(), L.dtype_code(q.dtype), q.stride(0), q.stride(1)
-    a.k_cache, a.v_cache, a.kv_dtype = k_cache.data_ptr(), v_cache.data_ptr(), L.dtype_code(k_cache.dtype)
-    a.skb, a.skh, a.sks = k_cache.stride(0), k_cache.stride(1), k_cache.stride(2)
-    a.svb, a.svh, a.svs = v_cache.stride(0), v_cache.stride(1), v_cache.stride(2)
-    if int8:
-        a.k_scale, a.v_scale = k_scale.data_ptr(), v_scale.data_ptr()
-        a.ssb, a.ssh, a.stb, a.sth = k_scale.stride(0), k_scale.stride(1), v_scale.stride(0), v_scale.stride(1)
-    a.pos, a.starts, a.idx_dtype = pos.data_ptr(), starts.data_ptr(), L.dtype_code(pos.dtype)
     if rows is not None:
         assert rows.dtype == pos.dtype and rows.is_contiguous() and rows.numel() == B
-        a.rows = rows.data_ptr()
-    a.out, a.out_dtype, a.sob, a.soh = out.data_ptr(), L.dtype_code(out.dtype), out.stride(0), out.stride(1)
-    a.B, a.H, a.KH, a.S, a.hd = B, H, KH, S, hd
-    a.scale, a.window, a.ring, a.num_splits = float(scale), int(window), int(bool(ring)), int(num_splits)
-    a.chunk_keys = int(chunk_keys)
-    a.workspace, a.workspace_bytes = (ws.data_ptr() if ws is not None else None), ws_bytes
+    dt = L.dtype_code
+    # (one positional construction: forty attribute assignments cost 4 us, half of a small launch's host time)
+    a = L.AttnArgs(q.data_ptr(), dt(q.dtype), *q.stride()[:2], k_cache.data_ptr(), v_cache.data_ptr(), dt(k_cache.dtype), *k_cache.stride()[:3],
+                   *v_cache.stride()[:3], *((k_scale.data_ptr(), v_scale.data_ptr(), *k_scale.stride()[:2], *v_scale.stride()[:2]) if int8 else
+                                            (None, None, 0, 0, 0, 0)),
+                   pos.data_ptr(), starts.data_ptr(), dt(pos.dtype), None if rows is None else rows.data_ptr(), out.data_ptr(), dt(out.dtype),
+                   *out.stride()[:2], B, H, KH, S, hd, scale, window, ring, num_splits, chunk_keys, None if ws is None else ws.data_ptr(), ws_bytes)
     if post is not None:
         vhat, gate, xsa, round_dtype = post
         assert vhat.dtype == torch.float32 and vhat.is_contiguous()
@@ -184,7 +182,13 @@ def decode_attention(q: Tensor, k_cache: Tensor, v_cache: Tensor, pos: Tensor, s
     q = q.contiguous() if q.stride(-1) != 1 else q
     if pos.dtype != starts.dtype:
         starts = starts.to(pos.dtype)
-    return _decode_attn_op(q, k_cache, v_cache, pos.contiguous(), starts.contiguous(), float(scale), int(window),
+    pos, starts = pos.contiguous(), starts.contiguous()
+    if type(q) is Tensor and not q.requires_grad and not torch.compiler.is_compiling():
+        # eager calls on plain tensors launch directly: the dispatcher's round trip through the registered op costs more host
+        # time than the launch (23 us a call against an 8 us kernel on 256 rows of up to 1024 keys)
+        out = torch.empty(q.shape, device=q.device, dtype=torch.float32 if out_fp32 else q.dtype)
+        return _launch(q, k_cache, v_cache, pos, starts, scale, window, ring, k_scale, v_scale, num_splits, out, chunk_keys, rows)
+    return _decode_attn_op(q, k_cache, v_cache, pos, starts, float(scale), int(window),
                            bool(ring), k_scale, v_scale, int(num_splits), bool(out_fp32), int(chunk_keys), rows)
 
 
