@@ -41,7 +41,7 @@ extern "C" {
 #define UVMI_I64 5
 
 /* Revision of the argument structs below (uvmi_version() returns the value the library was built with). */
-#define UVMI_ABI_VERSION 4
+#define UVMI_ABI_VERSION 5
 int uvmi_version(void);
 const char* uvmi_last_error(void);
 /* Number of compute units of the current device (used by the split heuristics); <0 on error. */
@@ -259,6 +259,9 @@ typedef struct uvmi_prefill_attn_args {
   const float* post_vhat;                  /* (N, KH, hd) fp32 normalized v of every token (uvmi_qkv_post vhat_out) */
   const float* post_gate;                  /* (N, H) fp32 gate values (uvmi_qkv_post gate_out), or NULL */
   const float* post_xsa;                   /* (H,) tanh(alpha) fp32, or NULL */
+  /* Optional output of the rows' softmax statistics for the backward (MFMA kernel only): lse_out (H, lse_stride) fp32, the
+   * log2 of each row's sum of exp2(scale log2(e) q . k); lse_stride >= N. */
+  float* lse_out; int64_t lse_stride;
 } uvmi_prefill_attn_args;
 /* The MFMA kernel runs when hd == 64, H / KH <= 8, q and k/v share a 16-bit dtype and rows are 16-byte aligned
  * (probabilities are rounded to that dtype for P.V, accumulation is fp32); anything else that uvmi_decode_attn's
@@ -272,8 +275,8 @@ int uvmi_prefill_attn_path(const uvmi_prefill_attn_args* a);
 /* Backward of uvmi_prefill_attn: replaces mathk::varlen_attn_bwd (ultraviolet/kernels/varlen_attn.py:56-66, the
  * aten._efficient_attention_backward call with K / V expanded to the query heads and their gradients summed back over the
  * group).  All tensors contiguous: q, o, go, dq (N, H, hd); k, v, dk, dv (N, KH, hd), one 16-bit dtype, head_dim 64;
- * cu_seqlens (n_seg + 1,) as in the forward.  The row log-sum-exp is recomputed (the forward does not return it).  fp32
- * arithmetic on the vector units (a first, plain form: no matrix cores).  workspace: (2 N H) fp32 (lse and go . o). */
+ * cu_seqlens (n_seg + 1,) as in the forward.  Up to 8 query heads per kv head run on the matrix cores, larger groups in a plain
+ * fp32 form.  The rows' log-sum-exp comes from the forward (lse), or is recomputed by a forward pass without output. */
 typedef struct uvmi_prefill_attn_bwd_args {
   const void* q; const void* k; const void* v; const void* o; const void* go; int dtype;
   void* dq; void* dk; void* dv;
@@ -282,6 +285,9 @@ typedef struct uvmi_prefill_attn_bwd_args {
   float scale;
   int window;                              /* 0 = none */
   void* workspace; size_t workspace_bytes; /* >= uvmi_prefill_attn_bwd_workspace_bytes(N, H) */
+  /* Optional: what the forward call left - its statistics (uvmi_prefill_attn_args.lse_out with a pitch lse_stride >=
+   * N + 32 that is a multiple of 4; 16-byte aligned) and its workspace, which holds the segment table of the same cu_seqlens. */
+  const float* lse; int64_t lse_stride; const void* fwd_workspace;
 } uvmi_prefill_attn_bwd_args;
 int uvmi_prefill_attn_bwd(const uvmi_prefill_attn_bwd_args* a, void* stream);
 size_t uvmi_prefill_attn_bwd_workspace_bytes(int N, int H);

@@ -348,6 +348,7 @@ static int check_prefill(const uvmi_prefill_attn_args* a) {
   UVMI_REQUIRE(a->workspace && a->workspace_bytes >= need, UVMI_EWORKSPACE, "uvmi_prefill_attn: workspace of %zu bytes needed, %zu given",
                need, a->workspace_bytes);
   UVMI_REQUIRE(((uintptr_t)a->workspace % 16) == 0, UVMI_EWORKSPACE, "uvmi_prefill_attn: workspace must be 16-byte aligned");
+  UVMI_REQUIRE(!a->lse_out || a->lse_stride >= a->N, UVMI_EINVAL, "uvmi_prefill_attn: lse_stride %lld below N", (long long)a->lse_stride);
   return UVMI_OK;
 }
 
@@ -448,6 +449,7 @@ extern "C" int uvmi_prefill_attn(const uvmi_prefill_attn_args* a, void* stream) 
     UVMI_REQUIRE(prefill_mfma_ok(a), UVMI_EUNSUPPORTED, "uvmi_prefill_attn: the fused post epilogue needs the MFMA kernel (head_dim 64, 16-bit q / k / v)");
     UVMI_REQUIRE(((uintptr_t)a->post_vhat % 16) == 0, UVMI_EINVAL, "uvmi_prefill_attn: post_vhat must be 16-byte aligned");
   }
+  UVMI_REQUIRE(!a->lse_out || prefill_mfma_ok(a), UVMI_EUNSUPPORTED, "uvmi_prefill_attn: lse_out needs the MFMA kernel (head_dim 64, 16-bit q / k / v)");
   if (!prefill_mfma_ok(a)) {
     // every packed token is a decode row whose "cache" is the packed K / V of the call (batch stride 0)
     uvmi_attn_args d = {};
@@ -460,6 +462,6 @@ extern "C" int uvmi_prefill_attn(const uvmi_prefill_attn_args* a, void* stream) 
     d.scale = a->scale; d.window = a->window; d.ring = 0; d.num_splits = 1;
     return uvmi_decode_attn(&d, stream);
   }
-  return launch_mfma(a, seg_start, nullptr, 0, st);
+  return launch_mfma(a, seg_start, a->lse_out, a->lse_stride, st);
 }
 

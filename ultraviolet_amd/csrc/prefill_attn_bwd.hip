@@ -232,7 +232,7 @@ __global__ __launch_bounds__(64) void bwd_dkv_kernel(BwdParams P) {
 
 // ------------------------------------------------------------------------------------------------ the MFMA form
 // Same mathematics on the matrix cores, on the forward kernel's operand layouts (prefill_attn.hip):
-//   * the forward kernel is run once more without storing an output, for the rows' log-sum-exp (log2 domain);
+//   * the rows' log-sum-exp (log2 domain) is the forward's, or comes from one more run of the forward kernel without output;
 //   * bwd_dq_mfma: a workgroup owns 16 query rows of one kv head, wave w the query heads 2w, 2w+1 of the group.  K and V
 //     super-tiles (32 keys) are staged once per workgroup in LDS.  S^T = K Q^T and dP^T = V dO^T have the same shape: a lane
 //     of either accumulator holds 4 consecutive keys of one query row for two 16-key tiles, so p = exp2(c s - lse) and
@@ -246,7 +246,8 @@ __global__ __launch_bounds__(64) void bwd_dkv_kernel(BwdParams P) {
 struct BwdMParams {
   const void* q; const void* k; const void* v; const void* o; const void* go;
   void* dq; void* dk; void* dv;
-  const float* lse; float* dsum; int64_t ls;   // (H, ls) each: log2-domain log-sum-exp of a row, and D = go . o
+  const float* lse; int64_t lse_ld;            // (H, lse_ld): log2-domain log-sum-exp of a row
+  float* dsum; int64_t ls;                      // (H, ls): D = go . o
   const int32_t* seg_start;                     // (ls,) first token of each token's sequence (entries >= N unused)
   const void* cu; int idx64, n_seg;
   int N, H, KH, G, window, n_wg;
@@ -358,7 +359,7 @@ __global__ __launch_bounds__(256) void bwd_dq_mfma(BwdMParams P) {
     for (int i = 0; i < 4; i++) d = dot2w<DT>(GO[hh][1][i], o1[i], dot2w<DT>(GO[hh][0][i], o0[i], d));
     d = psum32(psum16(d));
     Dr[hh] = d;
-    lse2[hh] = row_ok ? P.lse[(int64_t)head * P.ls + row] : INFINITY;
+    lse2[hh] = row_ok ? P.lse[(int64_t)head * P.lse_ld + row] : INFINITY;
     if (hok[hh] && g == 0 && row < P.N) P.dsum[(int64_t)head * P.ls + row] = row_ok ? d : 0.f;
   }
   pf4 dQ[2][4];
@@ -511,7 +512,7 @@ __global__ __launch_bounds__(256) void bwd_dkv_mfma(BwdMParams P) {
     pA = mfma16<DT>(GA[1], Vb[1], pA);
     pB = mfma16<DT>(GA[3], Vb[1], pB);
     // statistics of this lane's queries tq + 4g + i (tile A) and tq + 16 + 4g + i (tile B)
-    const float* lp = P.lse + (int64_t)head * P.ls + tq + 4 * g;
+    const float* lp = P.lse + (int64_t)head * P.lse_ld + tq + 4 * g;
     const float* dp = P.dsum + (int64_t)head * P.ls + tq + 4 * g;
     const float4 la = *(const float4*)lp, lb = *(const float4*)(lp + 16), da = *(const float4*)dp, db = *(const float4*)(dp + 16);
     const float lA[4] = {la.x, la.y, la.z, la.w}, lB[4] = {lb.x, lb.y, lb.z, lb.w};
@@ -609,11 +610,22 @@ extern "C" int uvmi_prefill_attn_bwd(const uvmi_prefill_attn_bwd_args* a, void* 
     f.cu_seqlens = a->cu_seqlens; f.idx_dtype = a->idx_dtype; f.n_seg = a->n_seg;
     f.N = a->N; f.H = a->H; f.KH = a->KH; f.hd = a->hd; f.scale = a->scale; f.window = a->window;
     UVMI_REQUIRE(a->scale > 0.f, UVMI_EUNSUPPORTED, "uvmi_prefill_attn_bwd: scale must be positive");
-    int rc = prefill_attn_stats(&f, seg, pidx, lse, ls, stream);
-    if (rc) return rc;
+    const float* stats = lse;
+    int64_t stats_ld = ls;
+    const int32_t* seg_start = seg;
+    if (a->lse) {   // the forward kept them: no pass of its own (43 us of 290 for forward and backward of 31 700 tokens)
+      UVMI_REQUIRE(a->fwd_workspace && ((uintptr_t)a->lse % 16) == 0 && a->lse_stride >= a->N + 32 && a->lse_stride % 4 == 0, UVMI_EINVAL,
+                   "uvmi_prefill_attn_bwd: lse must be 16-byte aligned with a pitch of at least N + 32 that is a multiple of 4, beside fwd_workspace");
+      stats = a->lse;
+      stats_ld = a->lse_stride;
+      seg_start = (const int32_t*)a->fwd_workspace;
+    } else {
+      int rc = prefill_attn_stats(&f, seg, pidx, lse, ls, stream);
+      if (rc) return rc;
+    }
     BwdMParams M;
     M.q = a->q; M.k = a->k; M.v = a->v; M.o = a->o; M.go = a->go; M.dq = a->dq; M.dk = a->dk; M.dv = a->dv;
-    M.lse = lse; M.dsum = dsum; M.ls = ls; M.seg_start = seg;
+    M.lse = stats; M.lse_ld = stats_ld; M.dsum = dsum; M.ls = ls; M.seg_start = seg_start;
     M.cu = a->cu_seqlens; M.idx64 = a->idx_dtype == UVMI_I64 ? 1 : 0; M.n_seg = a->n_seg;
     M.N = a->N; M.H = a->H; M.KH = a->KH; M.G = G; M.window = a->window;
     M.scale = a->scale; M.scale_log2 = a->scale * 1.4426950408889634f;

@@ -29,13 +29,14 @@ def _args(q, k, v, cu, scale, window, out, ws):
 
 def packed_attention(q: Tensor, k: Tensor, v: Tensor, cu_seqlens: Tensor, scale: float, window: int | None = None,
                      out: Tensor | None = None, out_fp32: bool = False, workspace: Tensor | None = None,
-                     segments_ready: bool = False, post: tuple | None = None) -> Tensor:
+                     segments_ready: bool = False, post: tuple | None = None, lse_out: Tensor | None = None) -> Tensor:
     """q (N, H, hd) fp16 / bf16, k / v (N, K, hd) (same dtype for the MFMA kernel; fp32 runs the generic kernel),
     cu_seqlens (S+1,) int32 / int64 on the device.  Returns (N, H, hd) in q's dtype (fp32 with out_fp32), or fills `out`.
     `workspace` (uint8, >= uvmi_prefill_attn_workspace_bytes(N)) avoids the allocation; segments_ready: it already holds
     the segment table of these cu_seqlens (an earlier call).  post = (vhat (N, K, hd) fp32, gate (N, H) fp32 or None, xsa
     (H,) fp32 or None) applies Attention.post (XSA, per-head gate; ultraviolet/model.py:321-333) in the kernel's epilogue
-    (MFMA kernel only)."""
+    (MFMA kernel only).  lse_out (H, >= N) fp32: also returns the rows' softmax statistics in it, for
+    packed_attention_backward (MFMA kernel only)."""
     L.require_cuda(q, k, v, cu_seqlens)
     assert q.dim() == 3 and k.dim() == 3 and v.shape == k.shape and k.size(0) == q.size(0) and k.size(2) == q.size(2)
     assert q.size(1) % k.size(1) == 0, "H must be a multiple of K"
@@ -59,6 +60,9 @@ def packed_attention(q: Tensor, k: Tensor, v: Tensor, cu_seqlens: Tensor, scale:
     assert workspace.dtype == torch.uint8 and workspace.numel() >= need
     a = _args(q, k, v, cu_seqlens, scale, window, out, workspace)
     a.segments_ready = int(bool(segments_ready))
+    if lse_out is not None:
+        assert lse_out.dtype == torch.float32 and lse_out.dim() == 2 and lse_out.size(0) == q.size(1) and lse_out.stride(1) == 1
+        a.lse_out, a.lse_stride = lse_out.data_ptr(), lse_out.stride(0)
     if post is not None:
         vhat, gate, xsa = post
         assert vhat.dtype == torch.float32 and vhat.is_contiguous() and vhat.shape == (N, k.size(1), q.size(2))
@@ -81,9 +85,11 @@ def packed_attention_path(q: Tensor, k: Tensor, v: Tensor, cu_seqlens: Tensor, s
 
 
 def packed_attention_backward(go: Tensor, q: Tensor, k: Tensor, v: Tensor, o: Tensor, cu_seqlens: Tensor, scale: float,
-                              window: int | None = None) -> tuple[Tensor, Tensor, Tensor]:
+                              window: int | None = None, saved: tuple | None = None) -> tuple[Tensor, Tensor, Tensor]:
     """(dq, dk, dv) of packed_attention for the output gradient go: q, o, go (N, H, 64), k, v (N, K, 64), one 16-bit dtype
-    (reference: mathk::varlen_attn_bwd, varlen_attn.py:56-66; gradients of K / V are summed over the heads of a group)."""
+    (reference: mathk::varlen_attn_bwd, varlen_attn.py:56-66; gradients of K / V are summed over the heads of a group).
+    saved = (lse, workspace) of the forward call (packed_attention's lse_out with statistics_pitch(N) columns, and its
+    workspace): without it the statistics are formed by one more pass of the forward kernel."""
     L.require_cuda(go, q, k, v, o, cu_seqlens)
     assert q.dim() == 3 and k.dim() == 3 and k.shape == v.shape and q.shape == o.shape == go.shape
     assert q.dtype == k.dtype == v.dtype == o.dtype == go.dtype
@@ -95,26 +101,42 @@ def packed_attention_backward(go: Tensor, q: Tensor, k: Tensor, v: Tensor, o: Te
     a = L.PrefillAttnBwdArgs(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), go.data_ptr(), L.dtype_code(q.dtype),
                              dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), cu_seqlens.data_ptr(), L.dtype_code(cu_seqlens.dtype),
                              cu_seqlens.numel() - 1, N, H, k.size(1), hd, float(scale), int(window or 0), ws.data_ptr(), ws.numel())
+    if saved is not None:
+        lse, fwd_ws = saved
+        a.lse, a.lse_stride, a.fwd_workspace = lse.data_ptr(), lse.stride(0), fwd_ws.data_ptr()
     L.check(L.lib().uvmi_prefill_attn_bwd(C.byref(a), L.stream_ptr(q)), "uvmi_prefill_attn_bwd")
     return dq, dk, dv
 
 
+def statistics_pitch(N: int) -> int:
+    """Row pitch of the (H, pitch) statistics a forward call leaves for its backward (whole 32-token tiles are read)."""
+    return (N + 31) // 32 * 32 + 32
+
+
 class _PackedAttention(torch.autograd.Function):
     """packed_attention with the backward above (the reference registers its pair of custom ops with autograd the same
-    way, varlen_attn.py:69-84)."""
+    way, varlen_attn.py:69-84), on the (1, N, ..) tensors themselves: a select in front of it would cost a zero fill and a copy
+    of every gradient.  Where the MFMA kernels run, the forward keeps its row statistics and segment table for the backward."""
 
     @staticmethod
     def forward(ctx, q, k, v, cu_seqlens, scale, window):
-        o = packed_attention(q, k, v, cu_seqlens, scale, window)
-        ctx.save_for_backward(q, k, v, o, cu_seqlens)
+        q0, k0, v0 = (t[0] if t.stride(3) == 1 else t[0].contiguous() for t in (q, k, v))
+        N, H, hd = q0.shape
+        out = torch.empty(q0.shape, dtype=q.dtype, device=q.device)
+        ws = torch.empty(L.lib().uvmi_prefill_attn_workspace_bytes(N), dtype=torch.uint8, device=q.device)
+        keep = N > 0 and L.lib().uvmi_prefill_attn_path(C.byref(_args(q0, k0, v0, cu_seqlens, scale, window, out, ws))) == 1
+        lse = torch.empty(H, statistics_pitch(N), dtype=torch.float32, device=q.device) if keep else None
+        packed_attention(q0, k0, v0, cu_seqlens, scale, window, out=out, workspace=ws, lse_out=lse)
+        out = out[None]
+        ctx.save_for_backward(q, k, v, out, cu_seqlens, *((lse, ws) if keep else ()))
         ctx.scale, ctx.window = scale, window
-        return o
+        return out
 
     @staticmethod
     def backward(ctx, go):
-        q, k, v, o, cu = ctx.saved_tensors
-        dq, dk, dv = packed_attention_backward(go, q, k, v, o, cu, ctx.scale, ctx.window)
-        return dq, dk, dv, None, None, None
+        q, k, v, o, cu, *saved = ctx.saved_tensors
+        dq, dk, dv = packed_attention_backward(go[0], q[0], k[0], v[0], o[0], cu, ctx.scale, ctx.window, saved=tuple(saved) or None)
+        return dq[None], dk[None], dv[None], None, None, None
 
 
 def varlen_attention(q: Tensor, k: Tensor, v: Tensor, cu_seqlens: Tensor, max_seqlen: int, scale: float,
@@ -124,7 +146,7 @@ def varlen_attention(q: Tensor, k: Tensor, v: Tensor, cu_seqlens: Tensor, max_se
     Differentiable in q, k, v (16-bit inputs, head_dim 64)."""
     assert q.dim() == 4 and q.size(0) == 1 and k.size(0) == 1 and v.size(0) == 1
     if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
-        return _PackedAttention.apply(q[0], k[0], v[0], cu_seqlens, float(scale), int(window or 0))[None]
+        return _PackedAttention.apply(q, k, v, cu_seqlens, float(scale), int(window or 0))
     return packed_attention(q[0], k[0], v[0], cu_seqlens, scale, window)[None]
 
 
