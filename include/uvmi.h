@@ -208,6 +208,8 @@ int uvmi_decode_attn_noalloc(const uvmi_attn_args* a, void* stream);
 #define UVMI_GEMM_STORE 0
 #define UVMI_GEMM_SWIGLU 1
 #define UVMI_GEMM_RESID 2
+#define UVMI_GEMM_SOFTCAP 4 /* C (M, N) fp32 = ca * sigmoid((x + cb) / cap_c) of the product x rounded to `dtype`: the logits of
+                               the tied head (model.py:824-827); uvmi_gemm_tn_ex, direct-to-LDS forms only (config 0, 5, 6) */
 int uvmi_gemm_tn_supported(int dtype, int64_t M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc, int epilogue);
 int uvmi_gemm_tn(const void* a, const void* w, void* c, int dtype, int64_t M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc,
                  int epilogue, void* stream);
@@ -230,6 +232,7 @@ typedef struct uvmi_gemm_args {
                                               128 x 128; 4: tiled, 64 x 64; 5: 256 x 256 tiles, 6: 128 x 128 tiles, both with slabs
                                               loaded straight into LDS (need K >= 128, C and resid 16-byte aligned, ldc,
                                               ldr % 8 == 0) - for tuning and tests */
+  float cap_c;                             /* SOFTCAP: the cap is ca * sigmoid((x + cb) / cap_c) */
 } uvmi_gemm_args;
 int uvmi_gemm_tn_ex(const uvmi_gemm_args* a, void* stream);
 
@@ -358,7 +361,7 @@ typedef struct uvmi_qkv_post_args {
   void* q_out; int q_dtype;            /* (n, H, hd) F16, BF16 or F32 */
   void* k_out; void* v_out;            /* (n, KH, hd) in dtype, or NULL */
   int8_t* k_cache; int8_t* v_cache;    /* (B, KH, S, hd) or NULL (no append) */
-  uint16_t* k_scale; uint16_t* v_scale;
+  uint16_t* k_scale; uint16_t* v_scale; /* both NULL: the caches hold values of dtype (16 bits) and k, v are stored as they are */
   int64_t scb, sch, scs, ssb, ssh;     /* cache / scale strides */
   int64_t n, vocab;
   int H, KH, hd, d, ve_ch, n_pairs, S, ring, has_ve, rope;
@@ -394,6 +397,25 @@ int uvmi_swiglu(const void* gu, int dtype, int64_t rows, int f, void* out, void*
  * is never written.  f % 8 == 0, d % 2 == 0. */
 int uvmi_swiglu_norm(const void* gu, const void* h, int dtype, int64_t rows, int f, int d, float eps, void* out,
                      void* stream);
+
+/* uvmi_embed_norm (tok != NULL: x is the table) and uvmi_add_norm as one argument block for uvmi_run_ops.  advance: an
+ * optional (rows,) array of positions the launch counts up by one - a decode step ends with st.pos += 1
+ * (fast_decode.py:332), which would otherwise be a launch of its own. */
+struct uvmi_norm_args {
+  const void* x; const void* y; const int64_t* tok; int64_t vocab; int dtype;
+  float a, b; int64_t rows; int d; float eps;
+  void* h_out; void* n_out; int64_t* advance;
+};
+
+/* A sequence of launches in one call: the layers of a pass without a host language between them.  kinds[i] says which
+ * entry point args[i] is for; the launches go to `stream` in order, and the first one that fails ends the call with its
+ * code and message.  The argument blocks are read before the call returns. */
+#define UVMI_OP_GEMM 0          /* uvmi_gemm_args */
+#define UVMI_OP_DECODE_ATTN 1   /* uvmi_attn_args */
+#define UVMI_OP_QKV_POST 2      /* uvmi_qkv_post_args */
+#define UVMI_OP_PREFILL_ATTN 3  /* uvmi_prefill_attn_args */
+#define UVMI_OP_NORM 4          /* struct uvmi_norm_args */
+int uvmi_run_ops(const int* kinds, const void* const* args, int n_ops, void* stream);
 
 /* ------------------------------------------------------------------------------------------------------------
  * On-device continuous batching: the slot table of generate_continuous (ultraviolet/model.py:1283-1350) and

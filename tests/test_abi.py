@@ -279,3 +279,30 @@ def test_weight_stamp_is_stable_on_a_real_module():
     assert fd._weights_stamp(p) == s2
     p._sd["w"].add_(1)
     assert fd._weights_stamp(p) != s2
+
+
+def test_run_ops_checks_its_list_and_the_norm_block_follows_the_header(tmp_path):
+    """uvmi_run_ops refuses unknown kinds, missing arguments and bad operations before it launches anything; the norm operation's
+    block is laid out as the header's."""
+    import subprocess
+    from ultraviolet_amd import _lib
+    lib = _lib.lib()
+    run = lambda kinds, args: lib.uvmi_run_ops((C.c_int * len(kinds))(*kinds), (C.c_void_p * len(args))(*args), len(kinds), None)
+    assert run([], []) == 0
+    assert lib.uvmi_run_ops(None, None, 1, None) == -1
+    assert run([99], [C.addressof(_lib.NormArgs())]) == -1 and b"unknown kind" in lib.uvmi_last_error()
+    assert run([_lib.OP_NORM], [None]) == -1
+    for kind, cls in ((_lib.OP_GEMM, _lib.GemmArgs), (_lib.OP_DECODE_ATTN, _lib.AttnArgs), (_lib.OP_QKV_POST, _lib.QkvPostArgs), (_lib.OP_NORM, _lib.NormArgs)):
+        a = cls()
+        assert run([kind], [C.addressof(a)]) == -1, cls
+    src = tmp_path / "norm.c"
+    names = [f[0] for f in _lib.NormArgs._fields_]
+    src.write_text('#include <stddef.h>\n#include <stdio.h>\n#include "uvmi.h"\nint main(void) {\n  printf("%zu\\n", sizeof(struct uvmi_norm_args));\n' +
+                   "".join(f'  printf("%zu\\n", offsetof(struct uvmi_norm_args, {n}));\n' for n in names) + "  return 0;\n}\n")
+    exe = tmp_path / "norm"
+    subprocess.run(["gcc", "-I", os.path.join(ROOT, "include"), str(src), "-o", str(exe)], check=True)
+    got = [int(x) for x in subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split()]
+    assert got == [C.sizeof(_lib.NormArgs)] + [getattr(_lib.NormArgs, n).offset for n in names]
+    hdr = open(os.path.join(ROOT, "include", "uvmi.h")).read()
+    kinds = dict(re.findall(r"#define UVMI_OP_(\w+) (\d+)", hdr))
+    assert {k: int(v) for k, v in kinds.items()} == {n[3:]: getattr(_lib, n) for n in dir(_lib) if n.startswith("OP_")}

@@ -702,3 +702,67 @@ def test_bf16_engine_greedy_against_the_bf16_oracle_reports_every_divergence():
             print(f"row {b}: identical for all 64 steps")
     assert all(g_ < 0.15 for g_ in gaps), gaps
     assert (ref[:, 0] == out[:, 0]).sum() >= 6  # (the first token comes from the prefill alone: most rows agree on it)
+
+
+@pytest.mark.parametrize("kv_dtype", ["int8", "fp16"])
+def test_recorded_passes_rebind_to_other_calls(kv_dtype):
+    """A pass that reuses a state's recorded launch list - other token tensors, other row counts on either side of the plans'
+    thresholds, another prompt set, a state of more rows than the step - gives what a fresh state gives bit for bit; positions
+    of all rows move by one; new weights and replaced cache tensors are picked up."""
+    from ultraviolet_amd.engine import KVState, UVWeights, random_params
+    cfg, params, eng, _ = _setup(dtype=torch.bfloat16, window=64)
+    rng = np.random.default_rng(3)
+    B, max_len = 224, 96
+    mk = lambda: KVState(cfg, B, max_len, DEV, kv_dtype=kv_dtype, dtype=torch.bfloat16)
+    same = lambda a, b: all(torch.equal(x, y) for x, y in zip(a.k + a.v, b.k + b.v)) and torch.equal(a.pos, b.pos) and torch.equal(a.starts, b.starts)
+    old = mk()
+    for round_ in range(3):
+        new = mk()
+        for a, b in zip(new.k + new.v + [new.pos, new.starts], old.k + old.v + [old.pos, old.starts]):
+            a.copy_(b)
+        if kv_dtype == "int8":
+            for a, b in zip(new.k_scale + new.v_scale, old.k_scale + old.v_scale):
+                a.copy_(b)
+        if round_ == 2:
+            eng.w.load_(random_params(cfg, 9, perturb=0.06))       # other residual scalars: launch arguments of the list
+            old.k[1] = old.k[1].clone()
+        prompts = _prompts(cfg, rng.integers(1, 30, size=(5, 40, 61)[round_]), seed=round_)
+        rows = rng.permutation(B)[:len(prompts)].tolist()
+        outs = [eng.prefill(prompts, rows, st).clone() for st in (old, new)]
+        assert torch.equal(*outs) and same(old, new)
+        for n in (3, 192, 193, B, 1):
+            p0 = old.pos.clone()
+            tok = torch.from_numpy(rng.integers(1, cfg.vocab_size, size=n)).to(DEV)
+            outs = [eng.decode_step(tok.clone(), st).clone() for st in (old, new)]
+            assert torch.equal(*outs) and same(old, new) and torch.equal(old.pos, p0 + 1)
+        pk = eng.pack_prompts(_prompts(cfg, (7, 20), seed=50 + round_), [B - 1, B - 2], max_len)
+        nd = 5 + round_
+        rows_d = torch.arange(nd, device=DEV)
+        tok = torch.from_numpy(rng.integers(1, cfg.vocab_size, size=nd)).to(DEV)
+        outs = [[t.clone() for t in eng.mixed_step(pk, tok, st.pos[:nd].clone(), st.starts[:nd].clone(), rows_d, st)] for st in (old, new)]
+        assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1]) and same(old, new)
+
+
+def test_unquantized_prefill_appends_what_it_attends():
+    """The post-processing kernel's append to an unquantized cache: the bytes of buf k / v at their slots (a ring keeps a
+    prompt's last S), nothing else; a cache of another 16-bit type takes them cast."""
+    from ultraviolet_amd.engine import KVState
+    cfg, _, eng, _ = _setup(dtype=torch.bfloat16, window=32)
+    prompts = _prompts(cfg, (40, 3, 33), seed=4)
+    for dt in (torch.bfloat16, torch.float16):
+        st = KVState(cfg, 4, 64, DEV, kv_dtype="fp16", dtype=dt)
+        for t in st.k + st.v:
+            t.fill_(7.0)
+        eng.prefill(prompts, [2, 0, 1], st, left_pad=False)
+        l = cfg.n_layers - 1                                # the buffers hold the last layer's k and v
+        exp_k, exp_v = torch.full_like(st.k[l], 7.0), torch.full_like(st.v[l], 7.0)
+        S, i = st.k[l].size(2), 0
+        for p, row in zip(prompts, (2, 0, 1)):
+            for t in range(len(p)):
+                if cfg.is_global(l) or t >= len(p) - S:
+                    s_ = t if cfg.is_global(l) else t % S
+                    exp_k[row, :, s_], exp_v[row, :, s_] = eng.buf["k"][i].to(dt), eng.buf["v"][i].to(dt)
+                i += 1
+        assert torch.equal(exp_k, st.k[l]) and torch.equal(exp_v, st.v[l])
+        if not cfg.is_global(0):
+            assert (st.k[0][3] == 7.0).all() and (st.k[0][0, :, 3:] == 7.0).all()

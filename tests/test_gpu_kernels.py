@@ -913,3 +913,27 @@ def test_attention_probe_runs_the_engine_shape_and_refuses_the_rest():
     a3, alive3 = build_attn_args(q, k, v, pos.int(), starts.int(), 0.14125, 0, False, ks, vs, 1, out)
     assert L.lib().uvmi_decode_attn_probe(C.byref(a3), 1, stream) != 0                    # 32-bit indices
     assert b"probe" in L.lib().uvmi_last_error()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K,norm,config", [(1, 512, 128, False, 0), (130, 1040, 640, True, 6), (257, 2048, 192, False, 5), (300, 32768, 640, True, 0)])
+def test_gemm_softcap_epilogue(dtype, M, N, K, norm, config):
+    """The head GEMM with the softcap in its epilogue: ca * sigmoid((x + cb) / cap_c) in fp32 of the product rounded to the
+    activation type, against float64 (a product that rounds the other way moves the logit by one step of its grid)."""
+    from ultraviolet_amd.kernels.gemm import SOFTCAP, gemm_tn
+    g = torch.Generator().manual_seed(M + N)
+    a, w = torch.randn(M, K, generator=g).to(dtype), (torch.randn(N, K, generator=g) * 0.3).to(dtype)
+    eps = 1e-6 if norm else None
+    got = gemm_tn(a.to(DEV), w.to(DEV), epilogue=SOFTCAP, norm_eps=eps, ca=23.0, cb=5.0, cap_c=7.5, config=config)
+    assert got.dtype == torch.float32 and got.shape == (M, N)
+    x = a.double() @ w.double().T
+    if norm:
+        x = x * torch.rsqrt(a.double().pow(2).mean(1, keepdim=True) + eps)
+    step = x.abs() * 2.0 ** (-8 if dtype == torch.bfloat16 else -11) + 1e-6
+    cap = lambda v: 23.0 * torch.sigmoid((v + 5.0) / 7.5)
+    lo, hi = cap(x - step) - 2e-5, cap(x + step) + 2e-5
+    got = got.cpu().double()
+    assert bool(((got >= lo) & (got <= hi)).all())
+    exact = 23.0 * torch.sigmoid((x.to(dtype).double() + 5.0) / 7.5)
+    assert float(((got - exact).abs() < 1e-5).double().mean()) > 0.97

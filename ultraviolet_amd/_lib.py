@@ -51,7 +51,8 @@ class AttnQkvFuse(C.Structure):
 class GemmArgs(C.Structure):
     _fields_ = [("a", C.c_void_p), ("w", C.c_void_p), ("c", C.c_void_p), ("dtype", C.c_int), ("M", C.c_int64), ("N", C.c_int),
                 ("K", C.c_int), ("lda", C.c_int64), ("ldw", C.c_int64), ("ldc", C.c_int64), ("epilogue", C.c_int), ("norm_a", C.c_int),
-                ("eps", C.c_float), ("resid", C.c_void_p), ("ldr", C.c_int64), ("ca", C.c_float), ("cb", C.c_float), ("config", C.c_int)]
+                ("eps", C.c_float), ("resid", C.c_void_p), ("ldr", C.c_int64), ("ca", C.c_float), ("cb", C.c_float), ("config", C.c_int),
+                ("cap_c", C.c_float)]
 
 
 class PrefillAttnArgs(C.Structure):
@@ -121,6 +122,14 @@ class SampleCommit(C.Structure):
                 ("starts_c", C.c_void_p), ("req_c", C.c_void_p), ("cnt_c", C.c_void_p), ("retire_p", C.c_float), ("seed", C.c_uint64)]
 
 
+class NormArgs(C.Structure):   # struct uvmi_norm_args: an operation of uvmi_run_ops
+    _fields_ = [("x", C.c_void_p), ("y", C.c_void_p), ("tok", C.c_void_p), ("vocab", C.c_int64), ("dtype", C.c_int),
+                ("a", C.c_float), ("b", C.c_float), ("rows", C.c_int64), ("d", C.c_int), ("eps", C.c_float),
+                ("h_out", C.c_void_p), ("n_out", C.c_void_p), ("advance", C.c_void_p)]
+
+
+OP_GEMM, OP_DECODE_ATTN, OP_QKV_POST, OP_PREFILL_ATTN, OP_NORM = range(5)   # UVMI_OP_*
+
 _lib = None
 ABI_VERSION = 5   # UVMI_ABI_VERSION of include/uvmi.h
 
@@ -180,6 +189,7 @@ def lib() -> C.CDLL:
         L.uvmi_sched_plan_admit.argtypes = [C.POINTER(SchedState), C.c_int, C.c_int, C.c_int] + [C.c_void_p] * 7
         L.uvmi_sched_step_plan.argtypes = ([C.POINTER(SchedState), C.c_int] + [C.c_void_p] * 6 + [C.c_int, C.c_int, C.c_int] +
                                            [C.c_void_p] * 12)
+        L.uvmi_run_ops.argtypes = [C.c_void_p, C.c_void_p, C.c_int, C.c_void_p]
         L.uvmi_rope_table.argtypes = [C.c_void_p, C.c_int, C.c_int64, C.c_int, C.c_void_p, C.c_void_p]
         L.uvmi_gemm_tn_supported.argtypes = [C.c_int, C.c_int64, C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_int64, C.c_int]
         L.uvmi_gemm_tn_ex.argtypes = [C.POINTER(GemmArgs), C.c_void_p]
@@ -212,4 +222,4 @@ EXPORTS = ["uvmi_version", "uvmi_last_error", "uvmi_device_cus", "uvmi_quantize_
            "uvmi_default_splits", "uvmi_decode_attn_path", "uvmi_decode_attn_noalloc", "uvmi_decode_attn_probe", "uvmi_prefill_attn", "uvmi_prefill_attn_workspace_bytes",
            "uvmi_prefill_attn_path", "uvmi_fused_sample", "uvmi_philox4x32_10",
            "uvmi_embed_norm", "uvmi_add_norm", "uvmi_qkv_post", "uvmi_attn_post", "uvmi_swiglu", "uvmi_swiglu_norm",
-           "uvmi_prefill_attn_bwd", "uvmi_prefill_attn_bwd_workspace_bytes", "uvmi_sched_compact", "uvmi_sched_commit", "uvmi_sched_commit_dense", "uvmi_sched_admit", "uvmi_sched_expand", "uvmi_sched_harvest", "uvmi_sched_plan_admit", "uvmi_sched_step_plan", "uvmi_rope_table", "uvmi_gemm_tn_supported", "uvmi_gemm_tn", "uvmi_gemm_tn_ex"]
+           "uvmi_prefill_attn_bwd", "uvmi_prefill_attn_bwd_workspace_bytes", "uvmi_sched_compact", "uvmi_sched_commit", "uvmi_sched_commit_dense", "uvmi_sched_admit", "uvmi_sched_expand", "uvmi_sched_harvest", "uvmi_sched_plan_admit", "uvmi_sched_step_plan", "uvmi_run_ops", "uvmi_rope_table", "uvmi_gemm_tn_supported", "uvmi_gemm_tn", "uvmi_gemm_tn_ex"]

@@ -400,7 +400,7 @@ static int skinny_bn(int K, int epilogue) {  // widest strip that fits 64 KB of 
 
 extern "C" int uvmi_gemm_tn_supported(int dtype, int64_t M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc, int epilogue) {
   if (dtype != UVMI_F16 && dtype != UVMI_BF16) return 0;
-  if (epilogue != UVMI_GEMM_STORE && epilogue != UVMI_GEMM_SWIGLU && epilogue != UVMI_GEMM_RESID) return 0;
+  if (epilogue != UVMI_GEMM_STORE && epilogue != UVMI_GEMM_SWIGLU && epilogue != UVMI_GEMM_RESID && epilogue != UVMI_GEMM_SOFTCAP) return 0;
   if (M < 0 || M > (1 << 16) || N <= 0 || K <= 0 || K % 64 != 0 || K > 8192) return 0;  // (the skinny forms add K <= 1984 / 960)
   if (N % (epilogue == UVMI_GEMM_SWIGLU ? 32 : 16) != 0) return 0;
   if (lda < K || ldw < K || lda % 8 != 0 || ldw % 8 != 0 || ldc % 4 != 0) return 0;
@@ -439,6 +439,9 @@ extern "C" int uvmi_gemm_tn_ex(const uvmi_gemm_args* a, void* stream) {
   if (a->epilogue == UVMI_GEMM_RESID)
     UVMI_REQUIRE(a->resid && ((uintptr_t)a->resid % 8) == 0 && a->ldr % 4 == 0 && a->ldr >= a->N, UVMI_EINVAL,
                  "uvmi_gemm_tn: the RESID epilogue needs an 8-byte aligned residual with a pitch that is a multiple of 4 and >= N");
+  if (a->epilogue == UVMI_GEMM_SOFTCAP)
+    UVMI_REQUIRE(big_ok(a) && a->cap_c != 0.f && (a->config == 0 || a->config >= 5), UVMI_EUNSUPPORTED,
+                 "uvmi_gemm_tn: the SOFTCAP epilogue needs K >= 128, a 16-byte aligned C with ldc %% 8 == 0, a non-zero cap_c and config 0, 5 or 6");
   UVMI_REQUIRE(!a->norm_a || a->eps >= 0.f, UVMI_EINVAL, "uvmi_gemm_tn: negative eps");
   UVMI_REQUIRE(a->config >= 0 && a->config <= 6, UVMI_EINVAL, "uvmi_gemm_tn: config %d", a->config);
   if (a->M == 0) return UVMI_OK;
@@ -461,7 +464,7 @@ extern "C" int uvmi_gemm_tn_ex(const uvmi_gemm_args* a, void* stream) {
     UVMI_CHECK_LAUNCH("uvmi_gemm_tn(direct to LDS)");
     return UVMI_OK;
   }
-  if (a->config == 6) {
+  if (a->config == 6 || a->epilogue == UVMI_GEMM_SOFTCAP) {
     UVMI_REQUIRE(big_ok(a), UVMI_EUNSUPPORTED,
                  "uvmi_gemm_tn: config %d (tiles loaded straight into LDS) needs K >= 128, C (and the residual) 16-byte aligned, ldc (ldr) %% 8 == 0", a->config);
     gemm_big_launch(a, 128, (hipStream_t)stream);

@@ -36,7 +36,7 @@ struct BigParams {
   int64_t ldc, ldr;     // elements
   int M, N, K, tiles_m, tiles_n;
   int rowsplit;
-  float eps, ca, cb;
+  float eps, ca, cb, cap_c;
 };
 
 #define UVMI_LDSP(p) ((__attribute__((address_space(3))) void*)(p))
@@ -64,7 +64,8 @@ template <int DT> __device__ __forceinline__ void unpack2(uint32_t w, float& lo,
 }
 
 // EPI 0: C = A W^T (M, N).  EPI 1: W rows are [gate 16 | up 16] slabs; C = silu(gate) * up, (M, N / 2).
-// EPI 2: C = ca * R + cb * (A W^T).  NORM: A stands for its RMS-normalised rows.
+// EPI 2: C = ca * R + cb * (A W^T).  EPI 3: C fp32 = ca * sigmoid((x + cb) / cap_c) of the rounded product x.  NORM: A stands
+// for its RMS-normalised rows.
 // FI: 16-row fragments per wave along M: 8 - the 256 x 256 tile on 8 waves (2 x 4); 4 - a 128 x 128 tile on 4 waves (2 x 2,
 // 64 x 64 per wave, two workgroups per compute unit) for passes whose 256 x 256 tiles would not fill the device.  (A
 // 64 x 64 tile on 2 waves was measured too: no faster than the tiled kernel's 64 x 64 form at 2 k rows.)
@@ -296,6 +297,19 @@ void gemm_big_kernel(BigParams P) {
             wds[e] = gpack<DT>(P.ca * x0 + P.cb * p0, P.ca * x1 + P.cb * p1);
           }
         }
+        if (EPI == 3) {
+          float* fp = (float*)P.c + (int64_t)row * P.ldc + n;
+          const float k2 = -1.4426950408889634f / P.cap_c;
+          auto cap = [&](float x) { return P.ca * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f((x + P.cb) * k2)); };
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            float p0, p1, p2, p3;
+            unpack2<DT>(wds[2 * e], p0, p1);
+            unpack2<DT>(wds[2 * e + 1], p2, p3);
+            *(float4*)(fp + 4 * e) = float4{cap(p0), cap(p1), cap(p2), cap(p3)};
+          }
+          continue;
+        }
         uint16_t* cp = (uint16_t*)P.c + (int64_t)row * P.ldc + n;
         *(uint4*)cp = uint4{wds[0], wds[1], wds[2], wds[3]};
         *(uint4*)(cp + 8) = uint4{wds[4], wds[5], wds[6], wds[7]};
@@ -312,6 +326,7 @@ static void launch_big(const uvmi_gemm_args* a, const BigParams& P, hipStream_t 
   const bool norm = a->norm_a != 0;
   if (a->epilogue == UVMI_GEMM_RESID) { if (norm) UVMI_GO(2, true); else UVMI_GO(2, false); }
   else if (a->epilogue == UVMI_GEMM_SWIGLU) { if (norm) UVMI_GO(1, true); else UVMI_GO(1, false); }
+  else if (a->epilogue == UVMI_GEMM_SOFTCAP) { if (norm) UVMI_GO(3, true); else UVMI_GO(3, false); }
   else { if (norm) UVMI_GO(0, true); else UVMI_GO(0, false); }
 #undef UVMI_GO
 }
@@ -324,7 +339,7 @@ void gemm_big_launch(const uvmi_gemm_args* a, int tile, hipStream_t st) {
   P.M = (int)a->M; P.N = a->N; P.K = a->K;
   P.tiles_m = (int)((a->M + tile - 1) / tile);
   P.tiles_n = (a->N + tile - 1) / tile;
-  P.eps = a->eps; P.ca = a->ca; P.cb = a->cb;
+  P.eps = a->eps; P.ca = a->ca; P.cb = a->cb; P.cap_c = a->cap_c;
   const double bytes_a = (double)a->M * a->K, bytes_w = (double)a->N * a->K;
   P.rowsplit = bytes_a / 8 + bytes_w < bytes_a + bytes_w / 8;
   if (a->dtype == UVMI_F16) { if (tile == 256) launch_big<UVMI_F16, 8>(a, P, st); else launch_big<UVMI_F16, 4>(a, P, st); }

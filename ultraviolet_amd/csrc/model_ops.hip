@@ -81,11 +81,13 @@ __device__ __forceinline__ void st8(void* p, int64_t i, const float (&v)[8]) {
 template <int DT, int MODE>
 __global__ __launch_bounds__(256) void norm_kernel(const void* __restrict__ xin, const void* __restrict__ yin,
                                                    const int64_t* __restrict__ tok, int64_t vocab, float a, float b,
-                                                   void* __restrict__ xout, void* __restrict__ nout, int64_t rows, int d, float eps) {
+                                                   void* __restrict__ xout, void* __restrict__ nout, int64_t rows, int d, float eps,
+                                                   int64_t* __restrict__ advance) {
   constexpr int NP = 16;  // pairs per lane: d <= 2048
   const int lane = threadIdx.x & 63;
   const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (r >= rows) return;
+  if (advance && lane == 0) advance[r]++;
   const int np = d / 2;
   float v0[NP], v1[NP];
   float ss = 0.f;
@@ -290,7 +292,11 @@ __global__ __launch_bounds__(256) void qkv_post_kernel(QkvArgs A) {
       const float nv = sqrtf(wave_sum(v * v));
       A.vhat_out[(r * A.KH + kh) * 64 + lane] = v / fmaxf(nv, A.xsa_eps);
     }
-    if (wr) {  // int8 append, same arithmetic as the standalone quantizer
+    if (wr && !A.k_scale) {   // an unquantized cache: the values as they are
+      const int64_t at = row * A.scb + kh * A.sch + slot * A.scs + lane;
+      elem<DT>::st(A.k_cache, at, k);
+      elem<DT>::st(A.v_cache, at, v);
+    } else if (wr) {  // int8 append, same arithmetic as the standalone quantizer
       const float vals[2] = {k, v};
       int8_t* caches[2] = {A.k_cache, A.v_cache};
       uint16_t* scales[2] = {A.k_scale, A.v_scale};
@@ -403,7 +409,10 @@ __global__ __launch_bounds__(256) void qkv_post_fast_kernel(QkvArgs A) {
   const int64_t slot = A.ring ? (p % A.S) : p;
   bool wr = A.k_cache && row >= 0 && p >= 0 && slot < A.S;
   if (wr && A.ring && A.last_pos) wr = p > lastp - A.S;
-  if (wr) {
+  if (wr && !A.k_scale) {
+    elem<DT>::st(A.k_cache, row * A.scb + slot * A.scs + lane, k);
+    elem<DT>::st(A.v_cache, row * A.scb + slot * A.scs + lane, v);
+  } else if (wr) {
     const float vals[2] = {k, v};
     int8_t* caches[2] = {A.k_cache, A.v_cache};
     uint16_t* scales[2] = {A.k_scale, A.v_scale};
@@ -536,26 +545,35 @@ static void dispatch_dt(int dt, F&& f) {
   else f(std::integral_constant<int, UVMI_F32>{});
 }
 
+namespace uvmi {
+int norm_run(const uvmi_norm_args* a, void* stream) {
+  const bool embed = a->tok != nullptr;
+  UVMI_REQUIRE(a->x && (embed || a->y) && a->n_out, UVMI_EINVAL, "uvmi_%s_norm: null pointer", embed ? "embed" : "add");
+  UVMI_REQUIRE(is_float_dtype(a->dtype) && a->rows >= 0 && a->d > 0 && a->d % 2 == 0 && a->d <= 2048 && (!embed || a->vocab > 0), UVMI_EINVAL,
+               "uvmi_%s_norm: bad arguments", embed ? "embed" : "add");
+  if (a->rows == 0) return UVMI_OK;
+  const dim3 grid((unsigned)((a->rows + 3) / 4)), blk(256);
+  dispatch_dt(a->dtype, [&](auto DT) {
+    constexpr int D = decltype(DT)::value;
+    if (embed) hipLaunchKernelGGL((norm_kernel<D, 0>), grid, blk, 0, (hipStream_t)stream, a->x, nullptr, a->tok, a->vocab, 0.f, 0.f, a->h_out, a->n_out, a->rows, a->d, a->eps, a->advance);
+    else hipLaunchKernelGGL((norm_kernel<D, 1>), grid, blk, 0, (hipStream_t)stream, a->x, a->y, nullptr, 0, a->a, a->b, a->h_out, a->n_out, a->rows, a->d, a->eps, a->advance);
+  });
+  UVMI_CHECK_LAUNCH(embed ? "uvmi_embed_norm" : "uvmi_add_norm");
+  return UVMI_OK;
+}
+}  // namespace uvmi
+
 extern "C" int uvmi_embed_norm(const void* table, int dtype, int64_t vocab, const int64_t* tok, int64_t rows, int d, float eps,
                                void* x_out, void* n_out, void* stream) {
-  UVMI_REQUIRE(table && tok && n_out, UVMI_EINVAL, "uvmi_embed_norm: null pointer");
-  UVMI_REQUIRE(is_float_dtype(dtype) && rows >= 0 && d > 0 && d % 2 == 0 && d <= 2048 && vocab > 0, UVMI_EINVAL, "uvmi_embed_norm: bad arguments");
-  if (rows == 0) return UVMI_OK;
-  const dim3 grid((unsigned)((rows + 3) / 4)), blk(256);
-  dispatch_dt(dtype, [&](auto DT) { hipLaunchKernelGGL((norm_kernel<decltype(DT)::value, 0>), grid, blk, 0, (hipStream_t)stream, table, nullptr, tok, vocab, 0.f, 0.f, x_out, n_out, rows, d, eps); });
-  UVMI_CHECK_LAUNCH("uvmi_embed_norm");
-  return UVMI_OK;
+  UVMI_REQUIRE(tok, UVMI_EINVAL, "uvmi_embed_norm: null pointer");
+  const uvmi_norm_args a{table, nullptr, tok, vocab, dtype, 0.f, 0.f, rows, d, eps, x_out, n_out, nullptr};
+  return norm_run(&a, stream);
 }
 
 extern "C" int uvmi_add_norm(const void* x, const void* y, int dtype, float a, float b, int64_t rows, int d, float eps, void* h_out,
                              void* n_out, void* stream) {
-  UVMI_REQUIRE(x && y && n_out, UVMI_EINVAL, "uvmi_add_norm: null pointer");
-  UVMI_REQUIRE(is_float_dtype(dtype) && rows >= 0 && d > 0 && d % 2 == 0 && d <= 2048, UVMI_EINVAL, "uvmi_add_norm: bad arguments");
-  if (rows == 0) return UVMI_OK;
-  const dim3 grid((unsigned)((rows + 3) / 4)), blk(256);
-  dispatch_dt(dtype, [&](auto DT) { hipLaunchKernelGGL((norm_kernel<decltype(DT)::value, 1>), grid, blk, 0, (hipStream_t)stream, x, y, nullptr, 0, a, b, h_out, n_out, rows, d, eps); });
-  UVMI_CHECK_LAUNCH("uvmi_add_norm");
-  return UVMI_OK;
+  const uvmi_norm_args n{x, y, nullptr, 0, dtype, a, b, rows, d, eps, h_out, n_out, nullptr};
+  return norm_run(&n, stream);
 }
 
 extern "C" int uvmi_qkv_post(const uvmi_qkv_post_args* a, void* stream) {
@@ -576,7 +594,8 @@ extern "C" int uvmi_qkv_post(const uvmi_qkv_post_args* a, void* stream) {
   UVMI_REQUIRE(((uintptr_t)a->qkv % 16) == 0 && ((uintptr_t)a->q_out % 16) == 0, UVMI_EUNSUPPORTED, "uvmi_qkv_post: qkv and q_out must be 16-byte aligned");
   UVMI_REQUIRE(!a->has_ve || (a->ve_table && a->tok && a->vocab > 0 && (a->ext_logits || (a->xn && a->ve_gate && a->ve_ch > 0 && a->ve_ch <= 64))), UVMI_EINVAL,
                "uvmi_qkv_post: value-embedding inputs missing");
-  UVMI_REQUIRE(!a->k_cache || (a->v_cache && a->k_scale && a->v_scale && a->S > 0), UVMI_EINVAL, "uvmi_qkv_post: incomplete cache arguments");
+  UVMI_REQUIRE(!a->k_cache || (a->v_cache && !a->k_scale == !a->v_scale && (a->k_scale || a->dtype != UVMI_F32) && a->S > 0), UVMI_EINVAL,
+               "uvmi_qkv_post: incomplete cache arguments");
   if (a->n == 0) return UVMI_OK;
   QkvArgs A;
   A.qkv = a->qkv; A.xn = a->xn; A.ve_table = a->ve_table; A.ve_gate = a->ve_gate; A.tok = a->tok; A.pos = a->pos; A.rows = a->rows;

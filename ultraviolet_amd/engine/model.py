@@ -16,13 +16,13 @@ import torch
 from torch import Tensor
 
 from .. import _lib as L
-from ..kernels.decode_attn import (build_attn_args, build_fused_args, decode_attention, decode_attention_fused, decode_attention_post,
-                                   rope_table)
-from ..kernels.gemm import RESID, SWIGLU, gemm_tn
+from ..kernels.decode_attn import build_attn_args, build_fused_args, decode_attention, rope_table
+from ..kernels.gemm import RESID, SOFTCAP, STORE, SWIGLU, gemm_args, gemm_supported, gemm_tn
 from ..kernels.kv_quant import kv_write
-from ..kernels.varlen_attn import packed_attention
+from ..kernels.varlen_attn import packed_attention, packed_attention_args
 from ..kernels.fused_sample import fused_sample_seeded, greedy_sample
 from .config import UVConfig
+from .plan import PassPlan, launch
 from .weights import UVWeights
 
 
@@ -144,22 +144,45 @@ class UVEngine:
         self.fold_down_rows = (int(fold_down_rows[0]), int(fold_down_rows[1]))
         self.head_own_rows = 288       # decode steps of at most this many rows run the head GEMM on this library's kernel (own_head_ok)
         self.hidden_is_raw = False
+        self._rec = None               # the PassPlan being recorded (None: operations are launched as they come)
         self._rope_tabs: dict[int, Tensor] = {}  # rotation tables by position count, kept for the engine's life (graphs hold them)
         if self.fuse_qkv:
             self.buf["qkvx"] = e(n, UVWeights.qkv_ext_rows(cfg))
         self.pf_ws = torch.empty(L.lib().uvmi_prefill_attn_workspace_bytes(n), dtype=torch.uint8, device=dev)  # fails now if the library is missing
 
     # ------------------------------------------------------------------------------------------------ kernels
+    # An operation is launched at once, or appended to the plan being recorded (_planned), where the names given for its
+    # fields say which per-call values they hold: n the token rows of the pass, tok / pos / rows / last / starts / cu the
+    # addresses of its arrays, Np / nd the prompt tokens and decode rows of a mixed pass, *_d addresses of its decode part.
+    def _op(self, kind: int, args, keep=(), **per_call):
+        if self._rec is None:
+            launch(kind, args, L.stream_ptr(self.buf["x"]))
+        else:
+            self._rec.op(kind, args, keep, **per_call)
+
+    def _lib_gemm(self, n: int, fn):
+        """A GEMM of the vendor library on the first n rows of the engine's buffers: fn(n)."""
+        if self._rec is None:
+            fn(n)
+        else:
+            self._rec.call(lambda values: fn(values["n"]))
+
+    def _gemm(self, a: Tensor, w: Tensor, out: Tensor, epilogue: int = STORE, **kw):
+        g = gemm_args(a, w, out, epilogue, **kw)
+        self._op(L.OP_GEMM, g, (a, w, out), M="n")
+
     def _embed_norm(self, tok: Tensor, n: int):
         b = self.buf
-        rc = L.lib().uvmi_embed_norm(self.w.embed.data_ptr(), self.dt_code, self.cfg.vocab_size, tok.data_ptr(), n,
-                                     self.cfg.d_model, self.eps, b["x"].data_ptr(), b["xn"].data_ptr(), L.stream_ptr(tok))
-        L.check(rc, "uvmi_embed_norm")
+        self._op(L.OP_NORM, L.NormArgs(x=self.w.embed.data_ptr(), tok=tok.data_ptr(), vocab=self.cfg.vocab_size, dtype=self.dt_code, rows=n,
+                                       d=self.cfg.d_model, eps=self.eps, h_out=b["x"].data_ptr(), n_out=b["xn"].data_ptr()),
+                 (self.w.embed, tok), rows="n", tok="tok")
 
-    def _add_norm(self, x: Tensor, y: Tensor, a: float, bb: float, n: int, h_out: Tensor | None, n_out: Tensor):
-        rc = L.lib().uvmi_add_norm(x.data_ptr(), y.data_ptr(), self.dt_code, a, bb, n, self.cfg.d_model, self.eps,
-                                   None if h_out is None else h_out.data_ptr(), n_out.data_ptr(), L.stream_ptr(x))
-        L.check(rc, "uvmi_add_norm")
+    def _add_norm(self, x: Tensor, y: Tensor, a: float, bb: float, n: int, h_out: Tensor | None, n_out: Tensor, advance: Tensor | None = None):
+        """h_out = a x + bb y, n_out = its norm; advance: positions of the rows to count up in the same launch."""
+        args = L.NormArgs(x=x.data_ptr(), y=y.data_ptr(), dtype=self.dt_code, a=a, b=bb, rows=n, d=self.cfg.d_model, eps=self.eps,
+                          h_out=None if h_out is None else h_out.data_ptr(), n_out=n_out.data_ptr(),
+                          advance=None if advance is None else advance.data_ptr())
+        self._op(L.OP_NORM, args, (), rows="n", **({} if advance is None else {"advance": "pos"}))
 
     def _qkv_post(self, l: int, tok: Tensor, pos: Tensor, rows: Tensor | None, last_pos: Tensor | None, st: KVState | None,
                   n: int, write_cache: bool = True, ext: bool = False):
@@ -172,19 +195,28 @@ class UVEngine:
         if ext:
             a.qkv_ld, a.ext_logits = b["qkvx"].stride(0), 1
         has_ve = cfg.has_ve(l)
+        per_call = dict(n="n", pos="pos")
         if has_ve:
             a.ve_table, a.ve_gate, a.tok = self.w.value_embed.data_ptr(), W["ve_gate"].data_ptr(), tok.data_ptr()
+            per_call["tok"] = "tok"
         a.pos = pos.data_ptr()
-        a.rows = None if rows is None else rows.data_ptr()
-        a.last_pos = None if last_pos is None else last_pos.data_ptr()
+        if rows is not None:
+            a.rows = rows.data_ptr()
+            per_call["rows"] = "rows"
+        if last_pos is not None:
+            a.last_pos = last_pos.data_ptr()
+            per_call["last_pos"] = "last"
         a.inv_freq = self.w.inv_freq.data_ptr()
         a.q_out, a.q_dtype = b["q"].data_ptr(), L.dtype_code(self.q_dtype)
         a.k_out, a.v_out = b["k"].data_ptr(), b["v"].data_ptr()
-        if st is not None and write_cache and st.quantized:
+        write_cache = st is not None and write_cache
+        fused_write = write_cache and self._append_fused(st)
+        if fused_write:   # int8 codes and scales, or (a cache of the activation type) the values as they are
             kc, ks = st.k[l], st.k_scale[l]
-            a.k_cache, a.v_cache, a.k_scale, a.v_scale = kc.data_ptr(), st.v[l].data_ptr(), ks.data_ptr(), st.v_scale[l].data_ptr()
-            a.scb, a.sch, a.scs, a.ssb, a.ssh = kc.stride(0), kc.stride(1), kc.stride(2), ks.stride(0), ks.stride(1)
-            a.S = kc.size(2)
+            a.k_cache, a.v_cache, a.S = kc.data_ptr(), st.v[l].data_ptr(), kc.size(2)
+            a.scb, a.sch, a.scs = kc.stride(0), kc.stride(1), kc.stride(2)
+            if st.quantized:
+                a.k_scale, a.v_scale, a.ssb, a.ssh = ks.data_ptr(), st.v_scale[l].data_ptr(), ks.stride(0), ks.stride(1)
         a.n, a.vocab = n, cfg.vocab_size
         a.H, a.KH, a.hd, a.d, a.ve_ch, a.n_pairs = cfg.n_heads, cfg.n_kv_heads, cfg.head_dim, cfg.d_model, cfg.ve_gate_channels, cfg.n_pairs
         a.ring, a.has_ve = int(not glob), int(has_ve)
@@ -197,14 +229,19 @@ class UVEngine:
             a.vhat_out, a.xsa_eps = b["vhat"].data_ptr(), float(cfg.xsa_eps)
         if W["attn_gate"] is not None:
             a.gate_w, a.gate_ch, a.gate_out = W["attn_gate"].data_ptr(), cfg.gate_ch, b["gate"].data_ptr()
-        L.check(L.lib().uvmi_qkv_post(C.byref(a), L.stream_ptr(pos)), "uvmi_qkv_post")
-        if st is not None and write_cache and not st.quantized:
-            self._write_kv16(l, pos, rows, last_pos, st, n)
+        self._op(L.OP_QKV_POST, a, (tok, pos, rows, last_pos), **per_call)
+        if write_cache and not fused_write:
+            self._write_kv_cast(l, pos, rows, last_pos, st, n)
 
-    def _write_kv16(self, l: int, pos: Tensor, rows: Tensor | None, last_pos: Tensor | None, st: KVState, n: int):
-        """Unquantized caches: buf k / v of the n rows go to slot pos (pos % S on a ring) of their cache rows - the two
-        kv_write calls of the reference's step (fast_decode.py:291-294, 315-317).  Dropped, as the int8 append drops them:
-        padding rows, positions past a linear cache, and prompt positions a ring will not keep (older than last_pos - S)."""
+    def _append_fused(self, st: KVState) -> bool:
+        """Whether the post-processing kernel appends to this state's caches (int8, or unquantized in the activation type)."""
+        return st.quantized or st.k[0].dtype == self.dtype
+
+    def _write_kv_cast(self, l: int, pos: Tensor, rows: Tensor | None, last_pos: Tensor | None, st: KVState, n: int):
+        """Unquantized caches of another type than the activations: buf k / v of the n rows go, cast, to slot pos (pos % S on a
+        ring) of their cache rows - the two kv_write calls of the reference's step (fast_decode.py:291-294, 315-317).
+        Dropped, as the fused append drops them: padding rows, positions past a linear cache, and prompt positions a ring
+        will not keep (older than last_pos - S)."""
         cfg, b = self.cfg, self.buf
         K = cfg.n_kv_heads
         S = st.k[l].size(2)
@@ -242,6 +279,13 @@ class UVEngine:
         L.check(rc, "uvmi_swiglu_norm")
 
     # ------------------------------------------------------------------------------------------------ trunk
+    def cache_attention_plannable(self, l: int, st: KVState) -> bool:
+        """Whether layer l's attention over the cache is one launch with the fused XSA + gate epilogue: the MFMA kernel streams
+        32-key tiles (rings need S % 32 == 0, linear int8 caches S % 4 == 0) and serves int8 caches and caches in the q dtype."""
+        cfg, S = self.cfg, st.k[l].size(2)
+        mfma_cache = self.q_dtype != torch.float32 and (st.quantized or st.k[l].dtype == self.q_dtype)
+        return (mfma_cache and cfg.xsa and cfg.n_heads // cfg.n_kv_heads <= 8 and S % (4 if cfg.is_global(l) else 32) == 0 and S >= 32)
+
     def cache_attention(self, l: int, q: Tensor, st: KVState, pos: Tensor, starts: Tensor, n: int, rows: Tensor | None = None,
                         off: int = 0):
         """Decode attention of layer l over the cache (int8, or unquantized) with the fused XSA + gate epilogue for the n rows that sit at
@@ -249,17 +293,25 @@ class UVEngine:
         the fused epilogue does not apply, returns the plain attention output for _attn_post."""
         cfg, b, W = self.cfg, self.buf, self.w.layers[l]
         glob = cfg.is_global(l)
-        S = st.k[l].size(2)
-        kw = dict(window=0 if glob else cfg.window, ring=not glob, k_scale=st.k_scale[l], v_scale=st.v_scale[l], rows=rows)
-        # the MFMA kernel (which carries the epilogue) streams 32-key tiles: rings need S % 32 == 0, linear int8 caches
-        # S % 4 == 0; it serves int8 caches and caches in the q dtype
-        mfma_cache = q.dtype != torch.float32 and (st.quantized or (st.k[l].dtype == q.dtype and q.dtype in (torch.float16, torch.bfloat16)))
-        if mfma_cache and cfg.xsa and cfg.n_heads // cfg.n_kv_heads <= 8 and S % (4 if glob else 32) == 0 and S >= 32:
+        window = 0 if glob else cfg.window
+        if self.cache_attention_plannable(l, st) and q.dtype == self.q_dtype:
+            if rows is not None:
+                rows = rows.to(pos.dtype).contiguous()
             out = b["zg"][off:off + n].view(n, cfg.n_heads, cfg.head_dim)
-            decode_attention_post(q, st.k[l], st.v[l], pos, starts, cfg.attn_scale, vhat=b["vhat"][off:off + n],
-                                  gate=None if W["attn_gate"] is None else b["gate"][off:off + n], xsa=W["xsa"], out=out, **kw)
+            gate = None if W["attn_gate"] is None else b["gate"][off:off + n]
+            a, keep = build_attn_args(q, st.k[l], st.v[l], pos.contiguous(), starts.contiguous(), cfg.attn_scale, window, not glob, st.k_scale[l],
+                                      st.v_scale[l], 1, out, 0, rows, (b["vhat"][off:off + n], gate, W["xsa"], out.dtype))
+            self._op(L.OP_DECODE_ATTN, a, (keep, q, pos, starts), B="nd", q="q_d", post_vhat="vhat_d", out="zg_d", pos="pos_d", starts="starts_d",
+                     **({} if gate is None else {"post_gate": "gate_d"}), **({} if rows is None else {"rows": "rows_d"}))
             return None
-        return decode_attention(q, st.k[l], st.v[l], pos, starts, cfg.attn_scale, num_splits=1, **kw)
+        return decode_attention(q, st.k[l], st.v[l], pos, starts, cfg.attn_scale, num_splits=1, window=window, ring=not glob, k_scale=st.k_scale[l],
+                                v_scale=st.v_scale[l], rows=rows)
+
+    def prompt_attention_plannable(self) -> bool:
+        """Whether the packed prompts' attention is one launch with the fused XSA + gate epilogue (16-bit engine)."""
+        cfg = self.cfg
+        return (cfg.xsa and self.dtype in (torch.bfloat16, torch.float16) and self.q_dtype == self.dtype and cfg.head_dim == 64
+                and cfg.n_heads // cfg.n_kv_heads <= 8)
 
     def prompt_attention(self, l: int, q: Tensor, N: int, cu: Tensor):
         """Causal (windowed on local layers) attention of the N packed prompt tokens at the head of the call's buffers over
@@ -268,14 +320,15 @@ class UVEngine:
         _attn_post.  The segment table of cu is built by layer 0's call and reused by the other layers of the pass."""
         cfg, b, W = self.cfg, self.buf, self.w.layers[l]
         w = 0 if cfg.is_global(l) else cfg.window
-        kw = dict(workspace=self.pf_ws, segments_ready=l > 0)
-        if (cfg.xsa and self.dtype in (torch.bfloat16, torch.float16) and self.q_dtype == self.dtype and cfg.head_dim == 64
-                and cfg.n_heads // cfg.n_kv_heads <= 8):
+        if self.prompt_attention_plannable():
+            if N == 0:
+                return None
             out = b["zg"][:N].view(N, cfg.n_heads, cfg.head_dim)
-            packed_attention(q, b["k"][:N], b["v"][:N], cu, cfg.attn_scale, w, out=out,
-                             post=(b["vhat"][:N], None if W["attn_gate"] is None else b["gate"][:N], W["xsa"]), **kw)
+            a = packed_attention_args(q, b["k"][:N], b["v"][:N], cu, cfg.attn_scale, w, out, self.pf_ws, segments_ready=l > 0,
+                                      post=(b["vhat"][:N], None if W["attn_gate"] is None else b["gate"][:N], W["xsa"]))
+            self._op(L.OP_PREFILL_ATTN, a, (q, out, cu), N="Np", cu_seqlens="cu", n_seg="n_seg")
             return None
-        return packed_attention(q, b["k"][:N], b["v"][:N], cu, cfg.attn_scale, w, **kw)
+        return packed_attention(q, b["k"][:N], b["v"][:N], cu, cfg.attn_scale, w, workspace=self.pf_ws, segments_ready=l > 0)
 
     def fused_layer_ok(self, l: int, st: KVState) -> bool:
         """Whether layer l's decode attention can take the fused path: the MFMA kernel streams 32-key tiles."""
@@ -303,12 +356,10 @@ class UVEngine:
     def fused_cache_attention(self, l: int, tok: Tensor, st: KVState, pos: Tensor, starts: Tensor, n: int, rows: Tensor | None = None):
         """Decode attention of layer l straight from buf qkvx (the extended projection of the n rows): QK-norm, rotation,
         value embedding, int8 append, attention over lo..pos, XSA and gate in one launch; writes buf zg."""
-        cfg, b, W = self.cfg, self.buf, self.w.layers[l]
-        glob = cfg.is_global(l)
-        out = b["zg"][:n].view(n, cfg.n_heads, cfg.head_dim)
-        decode_attention_fused(b["qkvx"][:n], cfg.n_heads, st.k[l], st.v[l], pos, starts, cfg.attn_scale, window=0 if glob else cfg.window,
-                               ring=not glob, k_scale=st.k_scale[l], v_scale=st.v_scale[l], xsa=W["xsa"], out=out,
-                               fuse=self._fuse_dict(l, tok, st), rows=rows)
+        a, keep = self.fused_attention_args(l, self.buf["qkvx"], tok, st, pos, starts, n, rows)
+        if self._rec is not None and self.cfg.has_ve(l):
+            self._rec.field(keep[0][2], "tok", "tok")
+        self._op(L.OP_DECODE_ATTN, a, (keep, pos, starts), B="n", pos="pos", starts="starts", **({} if rows is None else {"rows": "rows"}))
 
     def fused_attention_args(self, l: int, qkvx: Tensor, tok: Tensor, st: KVState, pos: Tensor, starts: Tensor, n: int,
                              rows: Tensor | None = None):
@@ -332,72 +383,163 @@ class UVEngine:
                                (b["vhat"][:n], None if W["attn_gate"] is None else b["gate"][:n], W["xsa"], out.dtype))
 
     def _trunk(self, tok: Tensor, pos: Tensor, n: int, attn, rows=None, last_pos=None, st: KVState | None = None,
-               fused_attn=None, defer_final_norm: bool = False) -> Tensor:
+               fused_attn=None, defer_final_norm: bool = False, advance: bool = False) -> Tensor:
         """n token rows through all layers; attn(l, q (n, H, hd)) -> z (n, H, hd) (or None when it wrote the post-processed
         result to buf zg itself) runs after K/V of the layer have been appended to the cache and written unquantized to
         buf k / v.  Returns the final normed hidden (n, d) (a buffer).  defer_final_norm: a plan whose last block leaves the
         hidden un-normalised returns it as it is and sets self.hidden_is_raw - the caller's head GEMM then carries the final
-        norm as the row scale of its product (head_of), and the norm launch goes away."""
+        norm as the row scale of its product (head_of), and the norm launch goes away.  advance: the final norm's launch
+        counts pos up by one."""
         cfg, b = self.cfg, self.buf
         assert n <= self.max_tokens
         self._embed_norm(tok, n)
         x, xn = b["x"][:n], b["xn"][:n]
+        adv = pos if advance else None
+        self.hidden_is_raw = False
+        raw = True          # the last block leaves buf x un-normalised
+        kind = self._pass_kind(n, fused_attn is not None, st)
+        if kind == "lean":
+            self._layers_lean(n, fused_attn)
+        elif kind == "folded":
+            self._layers_folded(n, fused_attn)
+        elif kind == "packed":
+            self._layers_packed(n, tok, pos, rows, last_pos, st, attn)
+        else:
+            raw = self._layers_plain(n, tok, pos, rows, last_pos, st, attn, fused_attn)
+        if raw:
+            if defer_final_norm and self.own_head_ok(n):
+                self.hidden_is_raw = True
+                return x
+            self._add_norm(x, x, 1.0, 0.0, n, None, b["xn"], adv)   # the final norm
+        elif advance:
+            pos.add_(1)
+        return xn
+
+    def _pass_kind(self, n: int, fused: bool, st: KVState | None) -> str:
+        """The launch plan of a pass of n rows: "lean" and "folded" for decode rows whose every layer takes the fused
+        attention, "packed" for prompts, mixed passes and the unfused attention of a 16-bit engine, "plain" for the rest
+        (fp32, widths the GEMMs do not take, plans switched off)."""
+        cfg = self.cfg
+        ok16 = self.dtype != torch.float32
+        il = all("gu_il" in W for W in self.w.layers)
+        div = cfg.d_model % 64 == 0 and (cfg.n_heads * cfg.head_dim) % 64 == 0
+        if fused and ok16 and all(self.fused_layer_ok(l, st) for l in range(cfg.n_layers)):
+            skinny = n <= self.skinny_rows and div and cfg.d_model <= 960
+            if skinny and self.lean and il and cfg.d_ff % 64 == 0 and cfg.d_ff <= 1984:
+                return "lean"
+            if self.fold and not skinny and cfg.d_ff % 8 == 0:
+                return "folded"
+        if not fused and ok16 and self.fold and self.tiled_prefill and self.fuse_qkv and il and div and cfg.d_ff % 64 == 0:
+            return "packed"
+        return "plain"
+
+    def _keep_projection(self, l: int, n: int):
+        if self.qkvx_keep is not None:   # a benchmark re-issues this layer's launch later on the same projection
+            self.qkvx_keep[l][:n].copy_(self.buf["qkvx"][:n])
+
+    def _project_qkv(self, l: int, n: int, own: bool = True, **kw):
+        """buf qkvx = the extended projection (q, k, v and the gates' logits) of the n rows, with the block's pre-norm as the
+        row scale of the product (layer 0: the embedding's norm exists already); own: on this library's GEMM."""
+        b, W = self.buf, self.w.layers[l]
+        if not own:
+            if l > 0:
+                self._add_norm(b["x"], b["x"], 1.0, 0.0, n, None, b["xn"])
+            self._lib_gemm(n, lambda n: torch.mm(b["xn"][:n], W["wqkv_ext"].t(), out=b["qkvx"][:n]))
+        elif l == 0:
+            self._gemm(b["xn"][:n], W["wqkv_ext"], b["qkvx"][:n], **kw)
+        else:
+            self._gemm(b["x"][:n], W["wqkv_ext"], b["qkvx"][:n], norm_eps=self.eps, **kw)
+
+    def _layers_lean(self, n: int, fused_attn):
+        """Decode passes of few rows: every projection on the skinny GEMM, the residual updates in the epilogues of the output
+        and down projections, both pre-norms as row scales of the products that read them.  Five launches per layer."""
+        b = self.buf
+        x, h, zg, act = b["x"][:n], b["h"][:n], b["zg"][:n], b["act"][:n]
+        for l, W in enumerate(self.w.layers):
+            self._project_qkv(l, n)
+            self._keep_projection(l, n)
+            fused_attn(l)
+            self._gemm(zg, W["wo"], h, RESID, resid=x, ca=W["resid_attn"], cb=W["post_attn"])
+            self._gemm(h, W["gu_il"], act, SWIGLU, norm_eps=self.eps)
+            self._gemm(act, W["down"], x, RESID, resid=h, ca=W["resid_mlp"], cb=W["post_mlp"])
+
+    def _layers_folded(self, n: int, fused_attn):
+        """Decode passes of many rows, five launches per layer: QKV projection with the block's pre-norm as a row scale, fused
+        attention, output projection with the residual update in place, gate-up projection with the MLP's pre-norm and the
+        SwiGLU in its epilogue (the (n, 2 f) intermediate and the normalised hidden are never written), down projection with the
+        residual update (the vendor library's C = alpha A B + beta C outside fold_down_rows: at K = d_ff it is still the
+        faster kernel there)."""
+        cfg, b = self.cfg, self.buf
+        x, zg, act = b["x"][:n], b["zg"][:n], b["act"][:n]
+        gc = self.gemm_config
+        sk_ok = cfg.d_model % 64 == 0 and (cfg.n_heads * cfg.head_dim) % 64 == 0
+        sk_qkv, sk_o = sk_ok and n <= self.fold_qkv_rows, sk_ok and n <= self.fold_o_rows
+        for l, W in enumerate(self.w.layers):
+            self._project_qkv(l, n, sk_qkv, config=gc)
+            self._keep_projection(l, n)
+            fused_attn(l)
+            # x <- resid_attn * x + post_attn * (zg @ wo.T), in place (every element is read and written by the same lane)
+            if sk_o:
+                self._gemm(zg, W["wo"], x, RESID, resid=x, ca=W["resid_attn"], cb=W["post_attn"], config=gc)
+            else:
+                self._lib_gemm(n, lambda n, W=W: torch.addmm(b["x"][:n], b["zg"][:n], W["wo"].t(), beta=W["resid_attn"], alpha=W["post_attn"], out=b["x"][:n]))
+            if sk_ok and "gu_il" in W and n <= self.fold_gu_rows:
+                self._gemm(x, W["gu_il"], act, SWIGLU, norm_eps=self.eps, config=gc)
+            else:
+                def gate_up(n, W=W):
+                    torch.mm(b["x"][:n], W["gu"].t(), out=b["gu"][:n])
+                    self._swiglu_norm(b["x"][:n], n)
+                self._lib_gemm(n, gate_up)
+            # x <- resid_mlp * x + post_mlp * (act @ down.T)
+            self._down(l, n, sk_ok and self.fold_down_rows[0] <= n <= self.fold_down_rows[1] and cfg.d_ff % 64 == 0)
+
+    def _down(self, l: int, n: int, own: bool):
+        """x <- resid_mlp * x + post_mlp * (act @ down.T), in place."""
+        b, W = self.buf, self.w.layers[l]
+        if own:
+            self._gemm(b["act"][:n], W["down"], b["x"][:n], RESID, resid=b["x"][:n], ca=W["resid_mlp"], cb=W["post_mlp"], config=self.gemm_config)
+        else:
+            self._lib_gemm(n, lambda n: torch.addmm(b["x"][:n], b["act"][:n], W["down"].t(), beta=W["resid_mlp"], alpha=W["post_mlp"], out=b["x"][:n]))
+
+    def _layers_packed(self, n: int, tok, pos, rows, last_pos, st, attn):
+        """Prompts, mixed passes and the unfused attention of a 16-bit engine: the extended projection with the pre-norm in it,
+        the post-processing kernel (which takes the gates' logits from the projection and appends to the cache), the
+        attention launches, output and down projections with the residual update in place, gate-up with the pre-norm and
+        the SwiGLU.  The normalised hidden is not written between blocks (it is formed on demand for a layer whose attention
+        leaves its epilogue to _attn_post)."""
+        cfg, b = self.cfg, self.buf
+        x, zg, act = b["x"][:n], b["zg"][:n], b["act"][:n]
+        gc = self.gemm_config
+        own_down = n <= self.skinny_rows or n >= self.big_rows or self.fold_down_rows[0] <= n <= self.fold_down_rows[1]
+        for l, W in enumerate(self.w.layers):
+            self._project_qkv(l, n, n <= self.fold_qkv_rows, config=gc)
+            self._qkv_post(l, tok, pos, rows, last_pos, st, n, ext=True)
+            z = attn(l, b["q"][:n])
+            if z is not None:
+                if l > 0:
+                    self._add_norm(x, x, 1.0, 0.0, n, None, b["xn"])
+                self._attn_post(l, z, n)
+            self._gemm(zg, W["wo"], x, RESID, resid=x, ca=W["resid_attn"], cb=W["post_attn"], config=gc)
+            self._gemm(x, W["gu_il"], act, SWIGLU, norm_eps=self.eps, config=gc)
+            self._down(l, n, own_down)
+
+    def _layers_plain(self, n: int, tok, pos, rows, last_pos, st, attn, fused_attn) -> bool:
+        """The reference's order of operations on the vendor library's GEMMs (16-bit passes of few rows: on the skinny GEMM),
+        one launch per step between them: fp32 engines, widths the other plans do not take.  Returns whether buf x was
+        left un-normalised (else buf xn holds the final norm)."""
+        cfg, b = self.cfg, self.buf
+        x, xn = b["x"][:n], b["xn"][:n]
         skinny_rows = self.skinny_rows if fused_attn is not None else max(self.skinny_rows, self.general_skinny_rows)
         skinny = n <= skinny_rows and cfg.d_model % 64 == 0 and cfg.d_model <= 960 and (cfg.n_heads * cfg.head_dim) % 64 == 0
         mm = (lambda a, w, out: gemm_tn(a, w, out)) if skinny else (lambda a, w, out: torch.mm(a, w.t(), out=out))
-        # Small passes whose every layer takes the fused attention never need the normalised hidden in memory: the block's
-        # second residual update then rides on the down projection and the next block's pre-norm on its QKV projection (a row
-        # scale of the product), and only the final norm is a launch of its own.
-        lean = (skinny and fused_attn is not None and self.lean
-                and all("gu_il" in W and self.fused_layer_ok(l, st) for l, W in enumerate(self.w.layers))
-                and cfg.d_ff % 64 == 0 and cfg.d_ff <= 1984)
-        # Larger passes under the same condition keep the library GEMMs but still never add a launch for a residual update or
-        # for the MLP's pre-norm: both residual updates are the library's own C = alpha A B + beta C on the hidden in place,
-        # and the pre-norm is a row scale inside the SwiGLU launch (7 launches per layer where the general path has 8; 6 while
-        # the QKV projection with the pre-norm in it is still faster on the skinny kernel).
-        folded = (not skinny and fused_attn is not None and self.fold and self.dtype != torch.float32
-                  and all(self.fused_layer_ok(l, st) for l in range(cfg.n_layers)) and cfg.d_ff % 8 == 0)
-        self.hidden_is_raw = False
-        if folded:
-            return self._trunk_folded(n, fused_attn, defer_final_norm)
         fold_mlp = not skinny and self.dtype != torch.float32 and cfg.d_ff % 8 == 0 and self.fold
-        tiled_gu = (fold_mlp and self.tiled_prefill and n >= 448 and cfg.d_model % 64 == 0
-                    and all("gu_il" in W for W in self.w.layers))
-        # Passes of the general path with many rows (a packed prefill, a mixed step): the QKV and output projections run on this
-        # library's GEMM (64 x 64 / 128 x 128 tiles, 256 x 256 from big_rows rows on - faster than the vendor library's at these
-        # shapes), the output projection with the residual update in place; from big_rows rows on the down projection too.
-        own = (fold_mlp and tiled_gu and (cfg.n_heads * cfg.head_dim) % 64 == 0 and cfg.d_ff % 64 == 0 and cfg.d_model % 8 == 0)
-        own_down = own and n >= self.big_rows
-        if own:
-            mm = lambda a, w, out: gemm_tn(a, w, out, config=self.gemm_config)
-        # ... and with the extended projection (q, k, v and the gates' logits) the block's pre-norm rides on the QKV GEMM as a
-        # row scale and the post-processing reads the logits from the projection: the normalised hidden is not written between
-        # blocks (it is formed on demand for a layer whose attention leaves its epilogue to _attn_post)
-        own_ext = own and self.fuse_qkv and fused_attn is None and all("wqkv_ext" in W for W in self.w.layers)
-        x_is_normed = True   # buf xn holds rmsnorm(x)
         for l, W in enumerate(self.w.layers):
             if fused_attn is not None and self.fused_layer_ok(l, st):
                 # decode rows of a 16-bit engine: the projection also forms the gate logits, and fused_attn(l) does the
                 # post-processing, the cache append, the attention and its epilogue in one launch (writes buf zg)
-                if x_is_normed:
-                    mm(xn, W["wqkv_ext"], b["qkvx"][:n])
-                else:
-                    gemm_tn(x, W["wqkv_ext"], b["qkvx"][:n], norm_eps=self.eps)
-                if self.qkvx_keep is not None:   # a benchmark re-issues this layer's launch later on the same projection
-                    self.qkvx_keep[l][:n].copy_(b["qkvx"][:n])
+                mm(xn, W["wqkv_ext"], b["qkvx"][:n])
+                self._keep_projection(l, n)
                 fused_attn(l)
-            elif own_ext:
-                if x_is_normed:
-                    gemm_tn(xn, W["wqkv_ext"], b["qkvx"][:n], config=self.gemm_config)
-                else:
-                    gemm_tn(x, W["wqkv_ext"], b["qkvx"][:n], norm_eps=self.eps, config=self.gemm_config)
-                self._qkv_post(l, tok, pos, rows, last_pos, st, n, ext=True)
-                z = attn(l, b["q"][:n])
-                if z is not None:
-                    if not x_is_normed:
-                        self._add_norm(x, x, 1.0, 0.0, n, None, b["xn"])
-                        x_is_normed = True
-                    self._attn_post(l, z, n)
             else:
                 mm(xn, W["wqkv"], b["qkv"][:n])
                 self._qkv_post(l, tok, pos, rows, last_pos, st, n)
@@ -406,30 +548,17 @@ class UVEngine:
                     self._attn_post(l, z, n)
             if skinny and "gu_il" in W:
                 # the residual update rides on the output projection (h = resid_attn * x + post_attn * a) and the MLP's
-                # pre-norm on the gate-up projection (a row scale of the product), whose epilogue is the SwiGLU: two
-                # launches where the general path has five
+                # pre-norm on the gate-up projection (a row scale of the product), whose epilogue is the SwiGLU
                 gemm_tn(b["zg"][:n], W["wo"], b["h"][:n], epilogue=RESID, resid=x, ca=W["resid_attn"], cb=W["post_attn"])
                 gemm_tn(b["h"][:n], W["gu_il"], b["act"][:n], epilogue=SWIGLU, norm_eps=self.eps)
             elif fold_mlp:
-                # 16-bit passes of any size and attention path: both residual updates are the library's C = alpha A B + beta C
-                # on the hidden in place and the MLP's pre-norm is the row scale inside the SwiGLU launch; the block ends
-                # with the norm the next block's projection and post-processing read
-                if own:
-                    gemm_tn(b["zg"][:n], W["wo"], x, epilogue=RESID, resid=x, ca=W["resid_attn"], cb=W["post_attn"], config=self.gemm_config)
-                else:
-                    torch.addmm(x, b["zg"][:n], W["wo"].t(), beta=W["resid_attn"], alpha=W["post_attn"], out=x)
-                if tiled_gu:   # the tiled GEMM with the pre-norm and the SwiGLU in it: the (n, 2 f) product is never written
-                    gemm_tn(x, W["gu_il"], b["act"][:n], epilogue=SWIGLU, norm_eps=self.eps, config=self.gemm_config)
-                else:
-                    torch.mm(x, W["gu"].t(), out=b["gu"][:n])
-                    self._swiglu_norm(x, n)
-                if own_down:
-                    gemm_tn(b["act"][:n], W["down"], x, epilogue=RESID, resid=x, ca=W["resid_mlp"], cb=W["post_mlp"], config=self.gemm_config)
-                else:
-                    torch.addmm(x, b["act"][:n], W["down"].t(), beta=W["resid_mlp"], alpha=W["post_mlp"], out=x)
-                if own_ext:
-                    x_is_normed = False
-                else:
+                # both residual updates are the library's C = alpha A B + beta C on the hidden in place and the MLP's pre-norm
+                # is the row scale inside the SwiGLU launch; the block ends with the norm the next block reads
+                torch.addmm(x, b["zg"][:n], W["wo"].t(), beta=W["resid_attn"], alpha=W["post_attn"], out=x)
+                torch.mm(x, W["gu"].t(), out=b["gu"][:n])
+                self._swiglu_norm(x, n)
+                torch.addmm(x, b["act"][:n], W["down"].t(), beta=W["resid_mlp"], alpha=W["post_mlp"], out=x)
+                if l + 1 < cfg.n_layers:
                     self._add_norm(x, x, 1.0, 0.0, n, None, b["xn"])
                 continue
             else:
@@ -438,68 +567,37 @@ class UVEngine:
                 self._add_norm(x, b["a"][:n], W["resid_attn"], W["post_attn"], n, b["h"], b["xn"])
                 mm(xn, W["gu"], b["gu"][:n])
                 self._swiglu(n)
-            if lean:
-                # x = resid_mlp * h + post_mlp * m in the down projection's epilogue (in place of the residual-add + norm launch)
-                gemm_tn(b["act"][:n], W["down"], x, epilogue=RESID, resid=b["h"][:n], ca=W["resid_mlp"], cb=W["post_mlp"])
-                x_is_normed = False
-            else:
-                torch.mm(b["act"][:n], W["down"].t(), out=b["m"][:n])   # (K = d_ff: 26 K-steps per strip, the library is faster)
-                # x = resid_mlp * h + post_mlp * m ; xn = rmsnorm(x) (next block's pre-norm, or the final norm)
-                self._add_norm(b["h"][:n], b["m"][:n], W["resid_mlp"], W["post_mlp"], n, b["x"], b["xn"])
-        if not x_is_normed:
-            if defer_final_norm and self.own_head_ok(n):
-                self.hidden_is_raw = True
-                return x
-            self._add_norm(x, x, 1.0, 0.0, n, None, b["xn"])   # the final norm
-        return xn
+            torch.mm(b["act"][:n], W["down"].t(), out=b["m"][:n])   # (K = d_ff: 26 K-steps per strip, the library is faster)
+            # x = resid_mlp * h + post_mlp * m ; xn = rmsnorm(x) (next block's pre-norm, or the final norm)
+            self._add_norm(b["h"][:n], b["m"][:n], W["resid_mlp"], W["post_mlp"], n, b["x"], b["xn"])
+        return fold_mlp
 
-    def _trunk_folded(self, n: int, fused_attn, defer_final_norm: bool = False) -> Tensor:
-        """The layers of _trunk for a pass of many rows whose every layer takes the fused attention; buf x and xn hold the
-        embedded rows and their norm on entry.  Five launches per layer: QKV projection with the block's pre-norm as a row
-        scale, fused attention, output projection with the residual update in place, gate-up projection with the MLP's
-        pre-norm and the SwiGLU in its epilogue (the tiled GEMM of this library: the (n, 2 f) intermediate and the
-        normalised hidden are never written), down projection with the residual update (the vendor library's
-        C = alpha A B + beta C: at K = d_ff it is still the faster kernel)."""
-        cfg, b = self.cfg, self.buf
-        x, xn = b["x"][:n], b["xn"][:n]
-        gc = self.gemm_config
-        sk_ok = cfg.d_model % 64 == 0 and (cfg.n_heads * cfg.head_dim) % 64 == 0
-        sk_qkv, sk_o = sk_ok and n <= self.fold_qkv_rows, sk_ok and n <= self.fold_o_rows
-        for l, W in enumerate(self.w.layers):
-            if l == 0:      # (the embedding's norm exists already: the same product as on the general path, bit for bit -
-                            # the tiled GEMM of this library from 448 rows, where the general path takes it too)
-                if sk_qkv and n >= 448:
-                    gemm_tn(xn, W["wqkv_ext"], b["qkvx"][:n], config=gc)
-                else:
-                    torch.mm(xn, W["wqkv_ext"].t(), out=b["qkvx"][:n])
-            elif sk_qkv:
-                gemm_tn(x, W["wqkv_ext"], b["qkvx"][:n], norm_eps=self.eps, config=gc)
-            else:
-                self._add_norm(x, x, 1.0, 0.0, n, None, b["xn"])
-                torch.mm(xn, W["wqkv_ext"].t(), out=b["qkvx"][:n])
-            if self.qkvx_keep is not None:
-                self.qkvx_keep[l][:n].copy_(b["qkvx"][:n])
-            fused_attn(l)
-            # x <- resid_attn * x + post_attn * (zg @ wo.T), in place (every element is read and written by the same lane)
-            if sk_o:
-                gemm_tn(b["zg"][:n], W["wo"], x, epilogue=RESID, resid=x, ca=W["resid_attn"], cb=W["post_attn"], config=gc)
-            else:
-                torch.addmm(x, b["zg"][:n], W["wo"].t(), beta=W["resid_attn"], alpha=W["post_attn"], out=x)
-            if sk_ok and "gu_il" in W and n <= self.fold_gu_rows:
-                gemm_tn(x, W["gu_il"], b["act"][:n], epilogue=SWIGLU, norm_eps=self.eps, config=gc)
-            else:
-                torch.mm(x, W["gu"].t(), out=b["gu"][:n])
-                self._swiglu_norm(x, n)
-            # x <- resid_mlp * x + post_mlp * (act @ down.T)
-            if sk_ok and self.fold_down_rows[0] <= n <= self.fold_down_rows[1] and cfg.d_ff % 64 == 0:
-                gemm_tn(b["act"][:n], W["down"], x, epilogue=RESID, resid=x, ca=W["resid_mlp"], cb=W["post_mlp"], config=gc)
-            else:
-                torch.addmm(x, b["act"][:n], W["down"].t(), beta=W["resid_mlp"], alpha=W["post_mlp"], out=x)
-        if defer_final_norm and self.own_head_ok(n):
-            self.hidden_is_raw = True
-            return x
-        self._add_norm(x, x, 1.0, 0.0, n, None, b["xn"])   # the final norm
-        return xn
+    # ---- recorded passes
+    def _planned(self, what: str, st: KVState, kind: str, n: int, values: dict, record) -> Tensor:
+        """Run the pass that record() makes, from its recorded launch list: recorded on the state the first time a pass of this
+        shape class runs on it, then only re-bound to the call's row counts and addresses (values).  The list is recorded
+        again when an object it rests on is another one (weights, cache tensors, a switch of the launch plans)."""
+        own_down = n <= self.skinny_rows or n >= self.big_rows or self.fold_down_rows[0] <= n <= self.fold_down_rows[1]
+        key = (id(self), what, kind, n <= self.fold_qkv_rows, n <= self.fold_o_rows, n <= self.fold_gu_rows, own_down,
+               self.fold_down_rows[0] <= n <= self.fold_down_rows[1], self.gemm_config, getattr(self.w, "scalar_epoch", 0))
+        guard = (self.w, *st.k, *st.v, *st.k_scale, *st.v_scale)
+        plans = st.__dict__.setdefault("_pass_plans", {})
+        plan = plans.get(key)
+        if plan is None or len(plan.guard) != len(guard) or any(a is not b for a, b in zip(plan.guard, guard)):
+            if len(plans) >= 16:
+                plans.clear()
+            plan = PassPlan()
+            self._rec = plan
+            try:
+                record()
+            finally:
+                self._rec = None
+            plan.guard = guard
+            plan.engine = self          # (keeps id(self) from being reused while the plan lives)
+            plans[key] = plan.close()
+        plan.run(values, L.stream_ptr(self.buf["x"]))
+        self.hidden_is_raw = False
+        return self.buf["xn"][:n]
 
     def own_head_ok(self, n: int) -> bool:
         """Whether head_of runs the head GEMM of n rows on this library's kernel with the final norm in it: 16-bit engines up
@@ -529,7 +627,15 @@ class UVEngine:
         return torch.mm(hidden, self.w.embed.t())
 
     def logits(self, hidden: Tensor) -> Tensor:
+        """Softcapped fp32 logits of the normed hidden (MathLM.logits, model.py:824-827): on a 16-bit engine one GEMM whose
+        epilogue rounds the product to the activation type and applies the softcap (the library's GEMM and the five
+        elementwise passes over the (n, V) output took 130 us at 512 rows)."""
         a, bb, c = self.cfg.softcap
+        W = self.w.embed
+        if hidden.dtype in (torch.bfloat16, torch.float16) and hidden.dim() == 2 and hidden.size(0) > 0 and hidden.dtype == W.dtype and W.size(1) >= 128 and W.size(0) % 16 == 0:
+            hidden = hidden.contiguous()
+            if gemm_supported(hidden, W, SOFTCAP):
+                return gemm_tn(hidden, W, epilogue=SOFTCAP, ca=a, cb=bb, cap_c=c)
         return a * torch.sigmoid((self.head(hidden).float() + bb) / c)
 
     # ------------------------------------------------------------------------------------------------ decode
@@ -541,6 +647,19 @@ class UVEngine:
         B = tok.numel()
         pos, starts = st.pos, st.starts
         ns = num_splits or {}
+        fused = None
+        if self.fuse_qkv and not num_splits and fuse:
+            fused = lambda l: self.fused_cache_attention(l, tok, st, pos, starts, B)
+            kind = self._pass_kind(B, True, st)
+            if kind in ("lean", "folded") and self.qkvx_keep is None:
+                assert B <= self.max_tokens and B <= st.B and tok.dtype == torch.int64 and tok.is_contiguous()
+                whole = B == pos.numel()     # (a step of fewer rows than the state has still moves every position)
+                h = self._planned("decode" if whole else "decode-part", st, kind, B,
+                                  dict(n=B, tok=tok.data_ptr(), pos=pos.data_ptr(), starts=starts.data_ptr()),
+                                  lambda: self._trunk(tok, pos, B, None, st=st, fused_attn=fused, advance=whole))
+                if not whole:
+                    st.pos.add_(1)
+                return h
 
         def attn(l, q):
             key = "global" if cfg.is_global(l) else "local"
@@ -550,9 +669,6 @@ class UVEngine:
             return decode_attention(q, st.k[l], st.v[l], pos, starts, cfg.attn_scale, window=0 if glob else cfg.window, ring=not glob,
                                     k_scale=st.k_scale[l], v_scale=st.v_scale[l], num_splits=ns[key])
 
-        fused = None
-        if self.fuse_qkv and not num_splits and fuse:
-            fused = lambda l: self.fused_cache_attention(l, tok, st, pos, starts, B)
         h = self._trunk(tok, pos, B, attn, st=st, fused_attn=fused)
         st.pos.add_(1)
         return h
@@ -623,7 +739,16 @@ class UVEngine:
                 self._attn_post(l, zd, nd, off=Np)
             return None
 
-        return self._trunk(tok[:N], pos[:N], N, attn, rows=rows[:N], last_pos=last[:N], st=st)
+        run = lambda: self._trunk(tok[:N], pos[:N], N, attn, rows=rows[:N], last_pos=last[:N], st=st)
+        if (Np > 0 and nd > 0 and self._pass_kind(N, False, st) == "packed" and self.prompt_attention_plannable() and self._append_fused(st)
+                and all(self.cache_attention_plannable(l, st) for l in range(cfg.n_layers))):
+            assert all(t.dtype == torch.int64 and t.stride(0) == 1 for t in (tok, pos, rows, last, starts_d))
+            at = lambda name: b[name].data_ptr() + Np * b[name].stride(0) * b[name].element_size()
+            values = dict(n=N, Np=Np, nd=nd, tok=tok.data_ptr(), pos=pos.data_ptr(), rows=rows.data_ptr(), last=last.data_ptr(), cu=cu.data_ptr(),
+                          n_seg=cu.numel() - 1, pos_d=pos_d.data_ptr(), rows_d=rows_d.data_ptr(), starts_d=starts_d.data_ptr(),
+                          q_d=at("q"), vhat_d=at("vhat"), gate_d=at("gate"), zg_d=at("zg"))
+            return self._planned("mixed", st, "packed", N, values, run)
+        return run()
 
     @torch.no_grad()
     def prefill(self, prompts: list[list[int]], rows: list[int], st: KVState, left_pad: bool = True) -> Tensor:
@@ -639,7 +764,13 @@ class UVEngine:
         def attn(l, q):
             return self.prompt_attention(l, q, N, pk["cu"])
 
-        h = self._trunk(pk["tok"], pk["pos"], N, attn, rows=pk["row"], last_pos=pk["last"], st=st)
+        tok, pos, row, last, cu = pk["tok"], pk["pos"], pk["row"], pk["last"], pk["cu"]
+        run = lambda: self._trunk(tok, pos, N, attn, rows=row, last_pos=last, st=st)
+        if self._pass_kind(N, False, st) == "packed" and self.prompt_attention_plannable() and self._append_fused(st):
+            h = self._planned("prefill", st, "packed", N, dict(n=N, Np=N, tok=tok.data_ptr(), pos=pos.data_ptr(), rows=row.data_ptr(), last=last.data_ptr(),
+                                                                cu=cu.data_ptr(), n_seg=cu.numel() - 1), run)
+        else:
+            h = run()
         self.bind_prompts(pk, st)
         return h.index_select(0, pk["last_idx"])
 

@@ -1,0 +1,73 @@
+"""The launch list of a forward pass, prepared once and issued with one native call per pass (uvmi_run_ops).
+
+A pass is ~50 launches whose arguments are the same from call to call except for the number of token rows and the addresses
+of the per-call arrays.  Preparing them one by one from Python costs ~12 us each, twice what the GPU needs for the launch
+on a small batch; a prepared list costs ~3 us a launch.  A list holds argument blocks (addresses and sizes), never
+results: every launch runs on every call."""
+from __future__ import annotations
+
+import ctypes as C
+
+from .. import _lib as L
+
+
+class PassPlan:
+    def __init__(self):
+        self.items = []     # ("ops", [(kind, args struct)]) or ("call", function of the pass's values), in launch order
+        self.keep = []      # what the argument blocks point into
+        self.fields = {}    # name of a per-call value -> [(struct, field)] that hold it
+        self.bound = {}     # the values they hold now
+        self.guard = ()     # objects whose identity the recorded addresses rest on
+
+    def op(self, kind: int, args, keep=(), **per_call):
+        """A launch; per_call: field of args (or (struct, field)) = name of the per-call value it holds."""
+        if not self.items or self.items[-1][0] != "ops":
+            self.items.append(("ops", []))
+        self.items[-1][1].append((kind, args))
+        self.keep.append((args, keep))
+        for field, name in per_call.items():
+            self.field(args, field, name)
+
+    def field(self, struct, field: str, name: str):
+        self.fields.setdefault(name, []).append((struct, field))
+
+    def call(self, fn):
+        """Work between the launches that is not this library's (a GEMM of the vendor library)."""
+        self.items.append(("call", fn))
+
+    def close(self):
+        self.segments = []
+        for what, item in self.items:
+            if what == "ops":
+                kinds = (C.c_int * len(item))(*[k for k, _ in item])
+                args = (C.c_void_p * len(item))(*[C.addressof(a) for _, a in item])
+                item = (kinds, args, len(item))
+            self.segments.append((what, item))
+        return self
+
+    def run(self, values: dict, stream: int):
+        """values: the pass's row counts and addresses by name; only the fields of values that changed are rewritten."""
+        for name, v in values.items():
+            if self.bound.get(name, self) != v:
+                self.bound[name] = v
+                for s, f in self.fields.get(name, ()):
+                    setattr(s, f, v)
+        run_ops = L.lib().uvmi_run_ops
+        for what, item in self.segments:
+            if what == "ops":
+                rc = run_ops(*item, stream)
+                if rc:
+                    L.check(rc, "uvmi_run_ops")
+            else:
+                item(values)
+
+
+_ENTRY = {L.OP_GEMM: "uvmi_gemm_tn_ex", L.OP_DECODE_ATTN: "uvmi_decode_attn", L.OP_QKV_POST: "uvmi_qkv_post", L.OP_PREFILL_ATTN: "uvmi_prefill_attn"}
+
+
+def launch(kind: int, args, stream: int):
+    """One operation at once."""
+    if kind in _ENTRY:
+        L.check(getattr(L.lib(), _ENTRY[kind])(C.byref(args), stream), _ENTRY[kind])
+    else:
+        L.check(L.lib().uvmi_run_ops((C.c_int * 1)(kind), (C.c_void_p * 1)(C.addressof(args)), 1, stream), "uvmi_run_ops")

@@ -10,7 +10,7 @@ from torch import Tensor
 
 from .. import _lib as L
 
-STORE, SWIGLU, RESID = 0, 1, 2
+STORE, SWIGLU, RESID, SOFTCAP = 0, 1, 2, 4
 
 
 def gemm_supported(a: Tensor, w: Tensor, epilogue: int = STORE) -> bool:
@@ -23,25 +23,33 @@ def gemm_supported(a: Tensor, w: Tensor, epilogue: int = STORE) -> bool:
                                                n_out, epilogue))
 
 
+def gemm_args(a: Tensor, w: Tensor, out: Tensor, epilogue: int = STORE, *, norm_eps: float | None = None, resid: Tensor | None = None,
+              ca: float = 1.0, cb: float = 1.0, cap_c: float = 0.0, config: int = 0):
+    """The uvmi_gemm_args block of gemm_tn."""
+    M, K = a.shape
+    N = w.size(0)
+    assert out.shape == (M, N // 2 if epilogue == SWIGLU else N) and out.dtype == (torch.float32 if epilogue == SOFTCAP else a.dtype)
+    assert out.stride(1) == 1 and a.stride(1) == 1 and w.stride(1) == 1
+    rp, ldr = None, 0
+    if epilogue == RESID:
+        assert resid is not None and resid.shape == (M, N) and resid.dtype == a.dtype and resid.stride(1) == 1
+        rp, ldr = resid.data_ptr(), resid.stride(0)
+    return L.GemmArgs(a.data_ptr(), w.data_ptr(), out.data_ptr(), L.dtype_code(a.dtype), M, N, K, a.stride(0), w.stride(0), out.stride(0),
+                      epilogue, norm_eps is not None, norm_eps or 0.0, rp, ldr, ca, cb, config, cap_c)
+
+
 def gemm_tn(a: Tensor, w: Tensor, out: Tensor | None = None, epilogue: int = STORE, *, norm_eps: float | None = None,
-            resid: Tensor | None = None, ca: float = 1.0, cb: float = 1.0, config: int = 0) -> Tensor:
+            resid: Tensor | None = None, ca: float = 1.0, cb: float = 1.0, cap_c: float = 0.0, config: int = 0) -> Tensor:
     """a (M, K) @ w (N, K).T -> (M, N); with epilogue=SWIGLU w is interleave_gate_up(w_gate, w_up) and the result is
     silu(a @ w_gate.T) * (a @ w_up.T), (M, N / 2); with epilogue=RESID the result is ca * resid + cb * (a @ w.T) (the
-    block's residual update, ultraviolet/model.py:567-571).  norm_eps: a stands for rmsnorm(a) with that epsilon (the
+    block's residual update, ultraviolet/model.py:567-571); with epilogue=SOFTCAP it is ca * sigmoid((x + cb) / cap_c) in fp32
+    of the rounded product x (the logits, model.py:824-827).  norm_eps: a stands for rmsnorm(a) with that epsilon (the
     pre-norm of the block folded into the projection as a row scale of the product).  Raises UvmiError for shapes the
     kernel does not take.  config (tuning / tests): 0 built-in choice, 1 the 64-row workgroup form, 2 the 16-row form whose
     waves split K."""
-    M, K = a.shape
-    N = w.size(0)
-    n_out = N // 2 if epilogue == SWIGLU else N
     if out is None:
-        out = torch.empty(M, n_out, dtype=a.dtype, device=a.device)
-    assert out.shape == (M, n_out) and out.dtype == a.dtype and out.stride(1) == 1 and a.stride(1) == 1 and w.stride(1) == 1
-    g = L.GemmArgs(a.data_ptr(), w.data_ptr(), out.data_ptr(), L.dtype_code(a.dtype), M, N, K, a.stride(0), w.stride(0), out.stride(0),
-                   epilogue, 0 if norm_eps is None else 1, 0.0 if norm_eps is None else float(norm_eps), None, 0, float(ca), float(cb), int(config))
-    if epilogue == RESID:
-        assert resid is not None and resid.shape == (M, N) and resid.dtype == a.dtype and resid.stride(1) == 1
-        g.resid, g.ldr = resid.data_ptr(), resid.stride(0)
+        out = torch.empty(a.size(0), w.size(0) // 2 if epilogue == SWIGLU else w.size(0), dtype=torch.float32 if epilogue == SOFTCAP else a.dtype, device=a.device)
+    g = gemm_args(a, w, out, epilogue, norm_eps=norm_eps, resid=resid, ca=ca, cb=cb, cap_c=cap_c, config=config)
     L.check(L.lib().uvmi_gemm_tn_ex(C.byref(g), L.stream_ptr(a)), "uvmi_gemm_tn")
     return out
 

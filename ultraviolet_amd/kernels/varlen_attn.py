@@ -58,6 +58,15 @@ def packed_attention(q: Tensor, k: Tensor, v: Tensor, cu_seqlens: Tensor, scale:
     if workspace is None:
         workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
     assert workspace.dtype == torch.uint8 and workspace.numel() >= need
+    a = packed_attention_args(q, k, v, cu_seqlens, scale, window, out, workspace, segments_ready, post, lse_out)
+    L.check(L.lib().uvmi_prefill_attn(C.byref(a), L.stream_ptr(q)), "uvmi_prefill_attn")
+    return out
+
+
+def packed_attention_args(q: Tensor, k: Tensor, v: Tensor, cu_seqlens: Tensor, scale: float, window: int | None, out: Tensor, workspace: Tensor,
+                          segments_ready: bool = False, post: tuple | None = None, lse_out: Tensor | None = None):
+    """The uvmi_prefill_attn_args block of packed_attention."""
+    N = q.size(0)
     a = _args(q, k, v, cu_seqlens, scale, window, out, workspace)
     a.segments_ready = int(bool(segments_ready))
     if lse_out is not None:
@@ -73,8 +82,7 @@ def packed_attention(q: Tensor, k: Tensor, v: Tensor, cu_seqlens: Tensor, scale:
         if xsa is not None:
             assert xsa.dtype == torch.float32 and xsa.is_contiguous() and xsa.numel() == q.size(1)
             a.post_xsa = xsa.data_ptr()
-    L.check(L.lib().uvmi_prefill_attn(C.byref(a), L.stream_ptr(q)), "uvmi_prefill_attn")
-    return out
+    return a
 
 
 def packed_attention_path(q: Tensor, k: Tensor, v: Tensor, cu_seqlens: Tensor, scale: float, window: int | None = None) -> int:
