@@ -183,8 +183,11 @@ __global__ __launch_bounds__(NT) void sample_kernel(const void* a_x, int64_t a_s
 // (48 bits, 32.32 fixed point: sums do not depend on the order of the additions) of its keys in one 64-bit word, so one
 // histogram serves both selects: the nucleus walk starts on the histograms that the top-k walk left and only builds new
 // ones for the bins in which it ends elsewhere.  200 rows x 32768, top_k 50 + top_p 0.95: 203 us for eleven sweeps of the
-// row with 8-bit digits, one thread walking each histogram; 27 us as it is now.
+// row with 8-bit digits, one thread walking each histogram; 13.6 us as it is now (top-k cuts of at most 256 through the
+// candidate list: the exponentials 2.8, the bound 2, collecting and ranking 2.5, the draw 2.5, launch and loads 4); 23 us for
+// top_p alone, which needs the histogram of the whole row (9 us: 512 wave-wide 64-bit LDS atomics of ~40 clocks each).
 constexpr unsigned long long BIN_ONE = 1ull << 48, BIN_MASS = BIN_ONE - 1;
+constexpr unsigned int CAND = 512;   // most candidates of a top-k select that are ranked key by key
 
 // floor(e * 2^32) for 0 <= e <= 1
 __device__ __forceinline__ unsigned long long fix32(float e) {
@@ -194,14 +197,31 @@ __device__ __forceinline__ unsigned long long fix32(float e) {
   return sh >= 0 ? (unsigned long long)m << sh : (unsigned long long)(sh > -24 ? m >> -sh : 0u);
 }
 
+// inclusive prefix sum over the 64 lanes by DPP row shifts and broadcasts (a shuffle through the LDS crossbar per step and word
+// would be most of a pick's time)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ unsigned long long scan_step(unsigned long long v) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, CTRL, ROWS, 0xf, false);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), CTRL, ROWS, 0xf, false);
+  return v + (((unsigned long long)hi << 32) | lo);
+}
+__device__ __forceinline__ unsigned long long wave_scan(unsigned long long v) {
+  v = scan_step<0x111, 0xf>(v);   // row_shr 1, 2, 4, 8
+  v = scan_step<0x112, 0xf>(v);
+  v = scan_step<0x114, 0xf>(v);
+  v = scan_step<0x118, 0xf>(v);
+  v = scan_step<0x142, 0xa>(v);   // lane 15 of rows 0, 2 -> rows 1, 3
+  return scan_step<0x143, 0xc>(v);  // lane 31 -> rows 2, 3
+}
+
 struct BinPick { unsigned int digit, cnt_above; unsigned long long mass_above, mass; };
 
 // The bin of a histogram of 1024 * PER bins in which a walk from the largest key down ends: by count (the bin with the
 // want-th largest key) or by mass (the first bin at which the mass reaches `want`; the largest key's bin when want is 0).
-// All 1024 threads call it; total is the whole histogram's word.
+// All 1024 threads call it; share > 0: `want` is set to that share of the whole histogram's mass first.
 template <int PER, bool BY_MASS>
-__device__ __forceinline__ BinPick pick_bin(const unsigned long long* h, unsigned long long want, unsigned long long* wtot, BinPick* sh,
-                                            unsigned long long& total) {
+__device__ __forceinline__ BinPick pick_bin(const unsigned long long* h, unsigned long long& want, unsigned long long* wtot, BinPick* sh,
+                                            double share = 0.0) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   unsigned long long v[PER], sum = 0;
 #pragma unroll
@@ -209,22 +229,18 @@ __device__ __forceinline__ BinPick pick_bin(const unsigned long long* h, unsigne
     v[i] = h[1024 * PER - 1 - (tid * PER + i)];
     sum += v[i];
   }
-  unsigned long long incl = sum;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const unsigned long long t = __shfl_up(incl, o, 64);
-    if (lane >= o) incl += t;
-  }
+  const unsigned long long incl = wave_scan(sum);
   if (lane == 63) wtot[wave] = incl;
   __syncthreads();
   unsigned long long run = incl - sum;
-  total = 0;
+  unsigned long long total = 0;
 #pragma unroll
   for (int w = 0; w < 16; w++) {
     const unsigned long long t = wtot[w];
     if (w < wave) run += t;
     total += t;
   }
+  if (BY_MASS && share > 0.0) want = (unsigned long long)(share * (double)(total & BIN_MASS));
 #pragma unroll
   for (int i = 0; i < PER; i++) {
     const unsigned long long above = run;
@@ -241,9 +257,10 @@ __device__ __forceinline__ BinPick pick_bin(const unsigned long long* h, unsigne
 
 template <int DT>
 __global__ __launch_bounds__(1024) void sample_filtered_kernel(SampleParams P) {
-  __shared__ float csum[64 + 4];
+  __shared__ float csum[64 + 4], csum_all[64];
   __shared__ unsigned long long h1[4096], h2[1024], h3[1024], wtot[16];
   __shared__ BinPick sh;
+  __shared__ unsigned int cand[CAND], n_cand;
   const int row = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, tid = threadIdx.x;
   const char* xr = (const char*)P.x + (int64_t)row * P.stride * (DT == UVMI_F32 ? 4 : 2);
   const int nchunks = P.V / CHUNK;   // <= 64: wave w holds chunks w, w + 16, w + 32, w + 48
@@ -253,6 +270,19 @@ __global__ __launch_bounds__(1024) void sample_filtered_kernel(SampleParams P) {
   for (int q = 0; q < 4; q++) {
     const int c = wave + 16 * q;
     if (c < nchunks) load8<DT>(xr, c * 64 + lane, e[q]);
+  }
+  float u = 0.f;   // (requested with the row: the draw at the end of the chain needs it at once)
+  if (wave == 0) {
+    if (P.u) {
+      u = P.u[row];
+    } else {
+      const uint64_t rid = (uint64_t)P.req_id[row], ti = (uint64_t)P.tok_idx[row];
+      const uint32_t ctr[4] = {(uint32_t)ti, (uint32_t)rid, (uint32_t)(rid >> 32), DOMAIN_SAMPLE};
+      const uint32_t key[2] = {(uint32_t)P.seed, (uint32_t)(P.seed >> 32)};
+      uint32_t o[4];
+      philox4x32_10(ctr, key, o);
+      u = (float)(o[0] >> 8) * 5.9604644775390625e-08f;  // 2^-24
+    }
   }
   for (int i = tid; i < 4096; i += 1024) h1[i] = 0;
   h2[tid] = 0;
@@ -269,80 +299,160 @@ __global__ __launch_bounds__(1024) void sample_filtered_kernel(SampleParams P) {
         s += e[q][j];
       }
       s = wave_sum(s);
-      if (lane == 0) csum[c] = s;
+      if (lane == 0) csum_all[c] = s;
     }
   }
   __syncthreads();
-  float S = 0.f;
-  if (wave == 0)
-    for (int c = 0; c < nchunks; c++) S += csum[c];
 
-  // keys whose bits above SHIFT + NBITS equal `prefix` into h, by the NBITS bits at SHIFT
-  auto histogram = [&](unsigned long long* h, int shift, int nbits, unsigned int prefix) {
+  unsigned int thr = 0;   // keep keys >= thr
+  const bool by_count = P.top_k > 0 && P.top_k < P.V;
+  const double share = P.top_p > 0.f ? (double)P.top_p : 0.0;
+  unsigned int mx = 0, top = 0;   // the thread's largest key, the row's
+#pragma unroll
+  for (int q = 0; q < 4; q++)
+    if (wave + 16 * q < nchunks) {
+#pragma unroll
+      for (int j = 0; j < 8; j++) mx = max(mx, __float_as_uint(e[q][j]));
+    }
+  {
+    const float wm = wave_max(__uint_as_float(mx));
+    if (lane == 0) wtot[wave] = __float_as_uint(wm);
+    if (tid == 0) n_cand = 0;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < 16; w++) top = max(top, (unsigned int)wtot[w]);
+    top >>= 16;
+    __syncthreads();
+  }
+  // ---- top-k of at most 256: the threads' largest keys bound the k-th largest key from below (k of them are at least as
+  // large), so only keys from that bound's bin up can matter.  They are about a hundred of the 32 768 and are collected in LDS.
+  // There a key's rank and the mass above it are counted key by key, which gives both cuts at once; rows whose candidates
+  // are too many for that (long runs of equal logits) take the histograms.
+  bool ranked = false;
+  if (by_count && P.top_k <= 256) {
+    atomicAdd(&h1[4095u - min(4095u, top - (mx >> 16))], BIN_ONE);
+    __syncthreads();
+    unsigned long long k_th = (unsigned long long)P.top_k;
+    const unsigned int digit = pick_bin<4, false>(h1, k_th, wtot, &sh).digit;
+    const unsigned int low = digit ? (top - (4095u - digit)) << 16 : 0u;
+    for (int i = tid; i < 4096; i += 1024) h1[i] = 0;
 #pragma unroll
     for (int q = 0; q < 4; q++)
       if (wave + 16 * q < nchunks) {
 #pragma unroll
         for (int j = 0; j < 8; j++) {
           const unsigned int key = __float_as_uint(e[q][j]);
-          if (nbits + shift == 32 || (key >> (shift + nbits)) == prefix)
-            atomicAdd(&h[(key >> shift) & ((1u << nbits) - 1u)], BIN_ONE | fix32(e[q][j]));
+          if (key >= low) {
+            const unsigned int at = atomicAdd(&n_cand, 1u);
+            if (at < CAND) cand[at] = key;
+          }
         }
       }
     __syncthreads();
-  };
-  auto clear = [&](unsigned long long* h) { h[tid] = 0; };
-
-  histogram(h1, 20, 12, 0);
-  unsigned int thr = 0, d1 = 0, d2 = 0;   // keep keys >= thr
-  unsigned long long zk = 0, above1 = 0, above2 = 0, tot;
-  const bool by_count = P.top_k > 0 && P.top_k < P.V;
-  if (by_count) {
-    unsigned int krem = (unsigned int)P.top_k;
-    BinPick b = pick_bin<4, false>(h1, krem, wtot, &sh, tot);
-    d1 = b.digit; krem -= b.cnt_above; above1 = b.mass_above;
-    histogram(h2, 10, 10, d1);
-    b = pick_bin<1, false>(h2, krem, wtot, &sh, tot);
-    d2 = b.digit; krem -= b.cnt_above; above2 = b.mass_above;
-    histogram(h3, 0, 10, (d1 << 10) | d2);
-    b = pick_bin<1, false>(h3, krem, wtot, &sh, tot);
-    thr = (d1 << 20) | (d2 << 10) | b.digit;
-    zk = above1 + above2 + b.mass_above + b.mass;
+    ranked = n_cand <= CAND;
   }
-  // ---- nucleus: the smallest key whose mass of strictly larger keys is below top_p * (mass of the top-k set).  Bins above
-  // the top-k threshold's are whole, so a walk that ends in one of them never meets a key below the threshold.
-  if (P.top_p < 1.0f) {
-    const double tp = P.top_p > 0.f ? (double)P.top_p : 0.0;
-    if (!by_count) {
-      pick_bin<4, true>(h1, 0, wtot, &sh, tot);
-      zk = tot & BIN_MASS;
+  if (ranked) {
+    // every wave compares the candidates with a sixteenth of the list: h1 gathers their counts (larger keys in the low word,
+    // equal ones in the high word), h2 the mass of the larger keys
+    const unsigned int n = n_cand;
+    for (unsigned int i = lane; i < n; i += 64) {
+      const unsigned int mine = cand[i];
+      unsigned long long cnt = 0, mgt = 0;
+      for (unsigned int j = wave; j < n; j += 16) {
+        const unsigned int key = cand[j];
+        const unsigned long long m = fix32(__uint_as_float(key));
+        cnt += key > mine ? 1ull : (key == mine ? 1ull << 32 : 0ull);
+        mgt += key > mine ? m : 0ull;
+      }
+      if (cnt) atomicAdd(&h1[i], cnt);
+      if (mgt) atomicAdd(&h2[i], mgt);
     }
-    unsigned long long want = (unsigned long long)(tp * (double)zk);
-    bool same = by_count;   // the walk is still on the top-k threshold's path: its histogram of this level is there
-    if (!(same && want > above1)) {
-      const BinPick b = pick_bin<4, true>(h1, want, wtot, &sh, tot);
-      same = same && b.digit == d1;
-      d1 = b.digit; above1 = b.mass_above;
+    __syncthreads();
+    // (equal keys write the same words)
+    unsigned int mine = 0, gt = 0, eq = 0;
+    if (tid < (int)n) {
+      mine = cand[tid];
+      gt = (unsigned int)h1[tid];
+      eq = (unsigned int)(h1[tid] >> 32);
+      if (gt < (unsigned int)P.top_k && gt + eq >= (unsigned int)P.top_k) sh = BinPick{mine, gt, h2[tid], eq * fix32(__uint_as_float(mine))};
     }
-    want -= want ? above1 : 0;
-    if (!same) {
-      clear(h2);
+    __syncthreads();
+    const BinPick b = sh;
+    thr = b.digit;
+    __syncthreads();
+    if (P.top_p < 1.0f) {
+      const unsigned long long want = (unsigned long long)(share * (double)(b.mass_above + b.mass));
+      if (tid < (int)n && (want == 0 ? gt == 0 : h2[tid] < want && h2[tid] + eq * fix32(__uint_as_float(mine)) >= want)) sh.digit = mine;
       __syncthreads();
+      thr = sh.digit;
+    }
+  }
+  // ---- the general form: radix selects over histograms of the whole row, by digits of 12 + 10 + 10 bits.  (Digits counted from
+  // the row's largest key in 128 bins per octave were measured too: no faster - a wave's 64-bit LDS atomics take ~40 clocks
+  // whether their addresses meet or not.)
+  if (!ranked) {
+    auto histogram = [&](unsigned long long* h, int shift, int nbits, unsigned int prefix) {
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        if (wave + 16 * q < nchunks) {
+#pragma unroll
+          for (int j = 0; j < 8; j++) {
+            unsigned int key = __float_as_uint(e[q][j]);
+            asm volatile("" : "+v"(key));   // (what is derived from a key is formed again in every pass: kept, it would spill)
+            if (nbits + shift == 32 || (key >> (shift + nbits)) == prefix)
+              atomicAdd(&h[(key >> shift) & ((1u << nbits) - 1u)], BIN_ONE | fix32(__uint_as_float(key)));
+          }
+        }
+      __syncthreads();
+    };
+    auto clear = [&]() { h2[tid] = 0; h3[tid] = 0; };
+    for (int i = tid; i < 4096; i += 1024) h1[i] = 0;
+    clear();
+    __syncthreads();
+    unsigned int d1 = 0, d2 = 0;
+    unsigned long long above1 = 0, above2 = 0, want = 0;
+    histogram(h1, 20, 12, 0);
+    if (by_count) {
+      unsigned long long krem = (unsigned long long)P.top_k;
+      BinPick b = pick_bin<4, false>(h1, krem, wtot, &sh);
+      d1 = b.digit; krem -= b.cnt_above; above1 = b.mass_above;
       histogram(h2, 10, 10, d1);
-    }
-    if (!(same && want > above2)) {
-      const BinPick b = pick_bin<1, true>(h2, want, wtot, &sh, tot);
-      same = same && b.digit == d2;
-      d2 = b.digit; above2 = b.mass_above;
-    }
-    want -= want ? above2 : 0;
-    if (!same) {
-      clear(h3);
-      __syncthreads();
+      b = pick_bin<1, false>(h2, krem, wtot, &sh);
+      d2 = b.digit; krem -= b.cnt_above; above2 = b.mass_above;
       histogram(h3, 0, 10, (d1 << 10) | d2);
+      b = pick_bin<1, false>(h3, krem, wtot, &sh);
+      thr = (d1 << 20) | (d2 << 10) | b.digit;
+      want = (unsigned long long)(share * (double)(above1 + above2 + b.mass_above + b.mass));
     }
-    const BinPick b = pick_bin<1, true>(h3, want, wtot, &sh, tot);
-    thr = (d1 << 20) | (d2 << 10) | b.digit;
+    // ---- nucleus: the smallest key whose mass of strictly larger keys is below top_p * (mass of the top-k set).  Bins above
+    // the top-k threshold's are whole, so a walk that ends in one of them never meets a key below the threshold.
+    if (P.top_p < 1.0f) {
+      bool same = by_count;   // the walk is still on the top-k threshold's path: its histogram of this level is there
+      if (!(same && want > above1)) {
+        const BinPick b = pick_bin<4, true>(h1, want, wtot, &sh, by_count ? 0.0 : share);
+        same = same && b.digit == d1;
+        d1 = b.digit; above1 = b.mass_above;
+      }
+      want -= want ? above1 : 0;
+      if (!same) {
+        clear();
+        __syncthreads();
+        histogram(h2, 10, 10, d1);
+      }
+      if (!(same && want > above2)) {
+        const BinPick b = pick_bin<1, true>(h2, want, wtot, &sh);
+        same = same && b.digit == d2;
+        d2 = b.digit; above2 = b.mass_above;
+      }
+      want -= want ? above2 : 0;
+      if (!same) {
+        h3[tid] = 0;
+        __syncthreads();
+        histogram(h3, 0, 10, (d1 << 10) | d2);
+      }
+      const BinPick b = pick_bin<1, true>(h3, want, wtot, &sh);
+      thr = (d1 << 20) | (d2 << 10) | b.digit;
+    }
   }
   auto e_kept = [&](float x) -> float {
     const float e = e_of(x, P);
@@ -370,17 +480,7 @@ __global__ __launch_bounds__(1024) void sample_filtered_kernel(SampleParams P) {
     if (lane >= o) incl += t;
   }
   const float Sk = __shfl(incl, 63, 64);
-  float u;
-  if (P.u) {
-    u = P.u[row];
-  } else {
-    const uint64_t rid = (uint64_t)P.req_id[row], ti = (uint64_t)P.tok_idx[row];
-    const uint32_t ctr[4] = {(uint32_t)ti, (uint32_t)rid, (uint32_t)(rid >> 32), DOMAIN_SAMPLE};
-    const uint32_t key[2] = {(uint32_t)P.seed, (uint32_t)(P.seed >> 32)};
-    uint32_t o[4];
-    philox4x32_10(ctr, key, o);
-    u = (float)(o[0] >> 8) * 5.9604644775390625e-08f;  // 2^-24
-  }
+  const float S = wave_sum(lane < nchunks ? csum_all[lane] : 0.f);
   const float target = (1.0f - u) * Sk;
   const unsigned long long below = __ballot(lane < nchunks && incl < target);
   int ck = __popcll(below);
