@@ -484,6 +484,26 @@ int uvmi_sched_admit(const uvmi_sched_state* s, int n, const int64_t* slots, con
 int uvmi_sched_expand(const uvmi_sched_state* s, int n_adm, int n_tokens, const int64_t* cu_seqlens, const int64_t* adm_slot,
                       const int64_t* adm_start, int64_t* pos_t, int64_t* row_t, int64_t* last_t, int64_t* last_idx, void* stream);
 
+/* The per-token tables of a prefill or mixed pass in one launch (prefill_packed_host's index tensors, fast_decode.py:210-269,
+ * the packing of a left-padded batch, fast_decode.py:70-134, and the binding of the cache rows): prompt a holds packed
+ * tokens cu[a] .. cu[a + 1] - 1, its first token sits at position start[a] of cache row row[a].  For packed token i of prompt a:
+ * pos_t = start[a] + i - cu[a], row_t = row[a], last_t = the prompt's last position, and tok_t = tok[i], or with idx_ld > 0 the
+ * token of a right-aligned (n, idx_ld) matrix (tok[a * idx_ld + idx_ld - (cu[a + 1] - i)]).  nd decode rows follow at n_tokens ..:
+ * tok_d, pos_d, rows_d, and pos_d once more as their last position.  last_idx[a] = cu[a + 1] - 1.  Optional outputs (NULL: not
+ * written): pos_t with tok_t, row_t and last_t, last_idx, the state's st_pos / st_starts of the rows, device copies of cu, row,
+ * start and of the prompts' end positions, and check_out = check_in[0 .. n).  cu, row, start, tok and check_out may be pinned host
+ * memory (n <= 2047 then): the launch reads a small table where the host wrote it, and a copy of its own would cost more. */
+struct uvmi_prompt_tables_args {
+  int n, n_tokens, nd; int64_t idx_ld;
+  const int64_t* cu; const int64_t* row; const int64_t* start; const int64_t* tok;
+  const int64_t* tok_d; const int64_t* pos_d; const int64_t* rows_d;
+  int64_t* tok_t; int64_t* pos_t; int64_t* row_t; int64_t* last_t; int64_t* last_idx;
+  int64_t* st_pos; int64_t* st_starts;
+  int64_t* cu_out; int64_t* row_out; int64_t* start_out; int64_t* end_out;
+  const int64_t* check_in; int64_t* check_out;
+};
+int uvmi_prompt_tables(const struct uvmi_prompt_tables_args* a, void* stream);
+
 /* The admission of a step decided on the device - the free-slot choice and the FIFO queue that the reference keeps in
  * host Python (StreamGen._refill, scripts/rl_stream.py:76-93; generate_continuous' refill, ultraviolet/model.py:1293-1314).
  * Takes prompts from the head of the staged ring while a reusable slot (slot_req < 0, not held) is left, at most admit_cap

@@ -295,14 +295,15 @@ def test_run_ops_checks_its_list_and_the_norm_block_follows_the_header(tmp_path)
     for kind, cls in ((_lib.OP_GEMM, _lib.GemmArgs), (_lib.OP_DECODE_ATTN, _lib.AttnArgs), (_lib.OP_QKV_POST, _lib.QkvPostArgs), (_lib.OP_NORM, _lib.NormArgs)):
         a = cls()
         assert run([kind], [C.addressof(a)]) == -1, cls
-    src = tmp_path / "norm.c"
-    names = [f[0] for f in _lib.NormArgs._fields_]
-    src.write_text('#include <stddef.h>\n#include <stdio.h>\n#include "uvmi.h"\nint main(void) {\n  printf("%zu\\n", sizeof(struct uvmi_norm_args));\n' +
-                   "".join(f'  printf("%zu\\n", offsetof(struct uvmi_norm_args, {n}));\n' for n in names) + "  return 0;\n}\n")
-    exe = tmp_path / "norm"
-    subprocess.run(["gcc", "-I", os.path.join(ROOT, "include"), str(src), "-o", str(exe)], check=True)
-    got = [int(x) for x in subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split()]
-    assert got == [C.sizeof(_lib.NormArgs)] + [getattr(_lib.NormArgs, n).offset for n in names]
+    for cname, cls in (("uvmi_norm_args", _lib.NormArgs), ("uvmi_prompt_tables_args", _lib.PromptTablesArgs)):
+        src = tmp_path / "layout.c"
+        names = [f[0] for f in cls._fields_]
+        src.write_text('#include <stddef.h>\n#include <stdio.h>\n#include "uvmi.h"\nint main(void) {\n' + f'  printf("%zu\\n", sizeof(struct {cname}));\n' +
+                       "".join(f'  printf("%zu\\n", offsetof(struct {cname}, {n}));\n' for n in names) + "  return 0;\n}\n")
+        exe = tmp_path / cname
+        subprocess.run(["gcc", "-I", os.path.join(ROOT, "include"), str(src), "-o", str(exe)], check=True)
+        got = [int(x) for x in subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split()]
+        assert got == [C.sizeof(cls)] + [getattr(cls, n).offset for n in names]
     hdr = open(os.path.join(ROOT, "include", "uvmi.h")).read()
     kinds = dict(re.findall(r"#define UVMI_OP_(\w+) (\d+)", hdr))
     assert {k: int(v) for k, v in kinds.items()} == {n[3:]: getattr(_lib, n) for n in dir(_lib) if n.startswith("OP_")}

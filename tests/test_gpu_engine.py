@@ -766,3 +766,42 @@ def test_unquantized_prefill_appends_what_it_attends():
         assert torch.equal(exp_k, st.k[l]) and torch.equal(exp_v, st.v[l])
         if not cfg.is_global(0):
             assert (st.k[0][3] == 7.0).all() and (st.k[0][0, :, 3:] == 7.0).all()
+
+
+@pytest.mark.parametrize("n,hi,left_pad", [(1, 1, True), (1, 300, False), (37, 40, True), (2047, 3, True), (2048, 2, False)])
+def test_packed_prompt_tables_match_their_definition(n, hi, left_pad):
+    """Per-token tables, prompt table and the binding of the rows (tables of up to 2047 prompts are read from the host's memory,
+    longer ones from the device's), from token lists and from a right-aligned matrix, against numpy."""
+    from ultraviolet_amd.engine import KVState
+    cfg, _, eng, _ = _setup(dtype=torch.bfloat16)
+    eng.max_tokens = 8192
+    rng = np.random.default_rng(n + hi)
+    lens = rng.integers(1, hi + 1, size=n)
+    prompts = _prompts(cfg, lens, seed=n)
+    B = n + 3
+    rows = rng.permutation(B)[:n]
+    st = KVState(cfg, B, 320, DEV)
+    st.pos.fill_(-5)
+    st.starts.fill_(-6)
+    T = int(lens.max())
+    start = (T - lens) if left_pad else np.zeros(n, np.int64)
+    cu = np.concatenate([[0], np.cumsum(lens)])
+    exp = dict(tok=np.concatenate(prompts), pos=np.concatenate([s + np.arange(m) for s, m in zip(start, lens)]), row=np.repeat(rows, lens),
+               last=np.repeat(start + lens - 1, lens), cu=cu, last_idx=cu[1:] - 1, rows=rows, starts=start, ends=start + lens)
+    pk = eng._pack(prompts, rows.tolist(), 320, left_pad, st)
+    pos, starts = np.full(B, -5), np.full(B, -6)
+    pos[rows], starts[rows] = start + lens, start
+    assert np.array_equal(st.pos.cpu().numpy(), pos) and np.array_equal(st.starts.cpu().numpy(), starts)
+    packs = [pk]
+    if left_pad and n < 2048:
+        idx = torch.zeros(n, T, dtype=torch.long)
+        for a, p in enumerate(prompts):
+            idx[a, T - len(p):] = torch.as_tensor(p)
+        seen = torch.arange(n, device=DEV) * 3
+        packs.append(eng._pack(None, rows.tolist(), 320, True, None, idx.to(DEV), lens, check=seen))
+        assert np.array_equal(packs[1]["check"](), np.arange(n) * 3)
+    for pk in packs:
+        for k, v in exp.items():
+            assert np.array_equal(pk[k].cpu().numpy(), v), k
+    with pytest.raises(IndexError):
+        eng._pack(prompts, [B] * n, 320, left_pad, st)

@@ -128,6 +128,16 @@ class NormArgs(C.Structure):   # struct uvmi_norm_args: an operation of uvmi_run
                 ("h_out", C.c_void_p), ("n_out", C.c_void_p), ("advance", C.c_void_p)]
 
 
+class PromptTablesArgs(C.Structure):   # struct uvmi_prompt_tables_args
+    _fields_ = [("n", C.c_int), ("n_tokens", C.c_int), ("nd", C.c_int), ("idx_ld", C.c_int64),
+                ("cu", C.c_void_p), ("row", C.c_void_p), ("start", C.c_void_p), ("tok", C.c_void_p),
+                ("tok_d", C.c_void_p), ("pos_d", C.c_void_p), ("rows_d", C.c_void_p),
+                ("tok_t", C.c_void_p), ("pos_t", C.c_void_p), ("row_t", C.c_void_p), ("last_t", C.c_void_p), ("last_idx", C.c_void_p),
+                ("st_pos", C.c_void_p), ("st_starts", C.c_void_p),
+                ("cu_out", C.c_void_p), ("row_out", C.c_void_p), ("start_out", C.c_void_p), ("end_out", C.c_void_p),
+                ("check_in", C.c_void_p), ("check_out", C.c_void_p)]
+
+
 OP_GEMM, OP_DECODE_ATTN, OP_QKV_POST, OP_PREFILL_ATTN, OP_NORM = range(5)   # UVMI_OP_*
 
 _lib = None
@@ -189,6 +199,7 @@ def lib() -> C.CDLL:
         L.uvmi_sched_plan_admit.argtypes = [C.POINTER(SchedState), C.c_int, C.c_int, C.c_int] + [C.c_void_p] * 7
         L.uvmi_sched_step_plan.argtypes = ([C.POINTER(SchedState), C.c_int] + [C.c_void_p] * 6 + [C.c_int, C.c_int, C.c_int] +
                                            [C.c_void_p] * 12)
+        L.uvmi_prompt_tables.argtypes = [C.POINTER(PromptTablesArgs), C.c_void_p]
         L.uvmi_run_ops.argtypes = [C.c_void_p, C.c_void_p, C.c_int, C.c_void_p]
         L.uvmi_rope_table.argtypes = [C.c_void_p, C.c_int, C.c_int64, C.c_int, C.c_void_p, C.c_void_p]
         L.uvmi_gemm_tn_supported.argtypes = [C.c_int, C.c_int64, C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_int64, C.c_int]
@@ -222,4 +233,4 @@ EXPORTS = ["uvmi_version", "uvmi_last_error", "uvmi_device_cus", "uvmi_quantize_
            "uvmi_default_splits", "uvmi_decode_attn_path", "uvmi_decode_attn_noalloc", "uvmi_decode_attn_probe", "uvmi_prefill_attn", "uvmi_prefill_attn_workspace_bytes",
            "uvmi_prefill_attn_path", "uvmi_fused_sample", "uvmi_philox4x32_10",
            "uvmi_embed_norm", "uvmi_add_norm", "uvmi_qkv_post", "uvmi_attn_post", "uvmi_swiglu", "uvmi_swiglu_norm",
-           "uvmi_prefill_attn_bwd", "uvmi_prefill_attn_bwd_workspace_bytes", "uvmi_sched_compact", "uvmi_sched_commit", "uvmi_sched_commit_dense", "uvmi_sched_admit", "uvmi_sched_expand", "uvmi_sched_harvest", "uvmi_sched_plan_admit", "uvmi_sched_step_plan", "uvmi_run_ops", "uvmi_rope_table", "uvmi_gemm_tn_supported", "uvmi_gemm_tn", "uvmi_gemm_tn_ex"]
+           "uvmi_prefill_attn_bwd", "uvmi_prefill_attn_bwd_workspace_bytes", "uvmi_sched_compact", "uvmi_sched_commit", "uvmi_sched_commit_dense", "uvmi_sched_admit", "uvmi_sched_expand", "uvmi_sched_harvest", "uvmi_sched_plan_admit", "uvmi_sched_step_plan", "uvmi_run_ops", "uvmi_prompt_tables", "uvmi_rope_table", "uvmi_gemm_tn_supported", "uvmi_gemm_tn", "uvmi_gemm_tn_ex"]

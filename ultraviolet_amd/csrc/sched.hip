@@ -333,6 +333,59 @@ static int check_state(const uvmi_sched_state* s, const char* who) {
   return UVMI_OK;
 }
 
+// One thread per packed token / decode row / prompt.  cu, row and start may lie in pinned host memory, so every workgroup takes
+// them into LDS once (where a token finds its prompt by binary search) instead of walking them over the bus; a table of more
+// than PT_MAX prompts is in device memory and searched there.
+constexpr int PT_MAX = 2047;
+__global__ __launch_bounds__(256) void prompt_tables_kernel(uvmi_prompt_tables_args A) {
+  __shared__ int scu[PT_MAX + 1], srow[PT_MAX], sst[PT_MAX];
+  const int tid = threadIdx.x, i = blockIdx.x * 256 + tid;
+  const bool lds = A.n <= PT_MAX;
+  const bool token = A.pos_t && i < A.n_tokens;
+  const int64_t t_own = token && A.idx_ld == 0 ? A.tok[i] : 0;
+  if (lds) {
+    for (int a = tid; a < A.n; a += 256) {
+      scu[a] = (int)A.cu[a];
+      srow[a] = (int)A.row[a];
+      sst[a] = (int)A.start[a];
+    }
+    if (tid == 0 && A.n > 0) scu[A.n] = (int)A.cu[A.n];
+  }
+  __syncthreads();
+  auto cu = [&](int a) -> int64_t { return lds ? scu[a] : A.cu[a]; };
+  auto row = [&](int a) -> int64_t { return lds ? srow[a] : A.row[a]; };
+  auto start = [&](int a) -> int64_t { return lds ? sst[a] : A.start[a]; };
+  if (i < A.n) {
+    const int64_t b = cu(i), e = cu(i + 1), r = row(i), s = start(i);
+    if (A.last_idx) A.last_idx[i] = e - 1;
+    if (A.st_pos) {
+      A.st_starts[r] = s;
+      A.st_pos[r] = s + e - b;
+    }
+    if (A.cu_out) {
+      A.cu_out[i] = b;
+      if (i == A.n - 1) A.cu_out[A.n] = e;
+      A.row_out[i] = r; A.start_out[i] = s; A.end_out[i] = s + e - b;
+    }
+    if (A.check_out) A.check_out[i] = A.check_in[i];
+  }
+  if (!A.pos_t || i >= A.n_tokens + A.nd) return;
+  if (i >= A.n_tokens) {
+    const int j = i - A.n_tokens;
+    const int64_t p = A.pos_d[j];
+    A.tok_t[i] = A.tok_d[j]; A.pos_t[i] = p; A.row_t[i] = A.rows_d[j]; A.last_t[i] = p;
+    return;
+  }
+  int lo = 0, hi = A.n;   // cu[lo] <= i < cu[hi]
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (cu(mid) <= i) lo = mid; else hi = mid;
+  }
+  const int64_t b = cu(lo), e = cu(lo + 1), s = start(lo);
+  A.tok_t[i] = A.idx_ld > 0 ? A.tok[lo * A.idx_ld + A.idx_ld - (e - i)] : t_own;
+  A.pos_t[i] = s + i - b; A.row_t[i] = row(lo); A.last_t[i] = s + e - b - 1;
+}
+
 }  // namespace uvmi
 
 using namespace uvmi;
@@ -434,5 +487,23 @@ extern "C" int uvmi_sched_harvest(const uvmi_sched_state* s, int64_t seen, int m
   UVMI_REQUIRE(seen >= 0 && max_rows > 0 && max_rows <= 65535 && hdr && tok_dst, UVMI_EINVAL, "uvmi_sched_harvest: bad arguments");
   hipLaunchKernelGGL(sched_harvest_kernel, dim3(max_rows), dim3(256), 0, (hipStream_t)stream, *s, seen, max_rows, hdr, tok_dst, lp_dst);
   UVMI_CHECK_LAUNCH("uvmi_sched_harvest");
+  return UVMI_OK;
+}
+
+extern "C" int uvmi_prompt_tables(const uvmi_prompt_tables_args* a, void* stream) {
+  UVMI_REQUIRE(a && a->n >= 0 && a->n_tokens >= 0 && a->nd >= 0 && a->idx_ld >= 0, UVMI_EINVAL, "uvmi_prompt_tables: bad sizes");
+  UVMI_REQUIRE(a->n == 0 || (a->cu && a->row && a->start), UVMI_EINVAL, "uvmi_prompt_tables: null prompt table");
+  UVMI_REQUIRE(a->n > 0 || a->n_tokens == 0, UVMI_EINVAL, "uvmi_prompt_tables: tokens without a prompt");
+  UVMI_REQUIRE(!a->st_pos == !a->st_starts, UVMI_EINVAL, "uvmi_prompt_tables: st_pos and st_starts go together");
+  UVMI_REQUIRE(!a->cu_out || (a->row_out && a->start_out && a->end_out), UVMI_EINVAL, "uvmi_prompt_tables: incomplete copies of the prompt table");
+  UVMI_REQUIRE(!a->check_out || a->check_in, UVMI_EINVAL, "uvmi_prompt_tables: check_out without check_in");
+  if (a->pos_t) {
+    UVMI_REQUIRE(a->tok_t && a->row_t && a->last_t && (a->n_tokens == 0 || a->tok), UVMI_EINVAL, "uvmi_prompt_tables: null token table");
+    UVMI_REQUIRE(a->nd == 0 || (a->tok_d && a->pos_d && a->rows_d), UVMI_EINVAL, "uvmi_prompt_tables: null decode rows");
+  }
+  const int64_t tokens = a->pos_t ? (int64_t)a->n_tokens + a->nd : 0, n = tokens > a->n ? tokens : a->n;
+  if (n == 0) return UVMI_OK;
+  hipLaunchKernelGGL(prompt_tables_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, *a);
+  UVMI_CHECK_LAUNCH("uvmi_prompt_tables");
   return UVMI_OK;
 }

@@ -144,6 +144,7 @@ class UVEngine:
         self.fold_down_rows = (int(fold_down_rows[0]), int(fold_down_rows[1]))
         self.head_own_rows = 288       # decode steps of at most this many rows run the head GEMM on this library's kernel (own_head_ok)
         self.hidden_is_raw = False
+        self._stage, self._stage_at = [(None, None)] * 2, 0   # pinned tables and the events of the launches that read them (_staging)
         self._rec = None               # the PassPlan being recorded (None: operations are launched as they come)
         self._rope_tabs: dict[int, Tensor] = {}  # rotation tables by position count, kept for the engine's life (graphs hold them)
         if self.fuse_qkv:
@@ -383,13 +384,14 @@ class UVEngine:
                                (b["vhat"][:n], None if W["attn_gate"] is None else b["gate"][:n], W["xsa"], out.dtype))
 
     def _trunk(self, tok: Tensor, pos: Tensor, n: int, attn, rows=None, last_pos=None, st: KVState | None = None,
-               fused_attn=None, defer_final_norm: bool = False, advance: bool = False) -> Tensor:
+               fused_attn=None, defer_final_norm: bool = False, advance: bool = False, final_norm: bool = True) -> Tensor:
         """n token rows through all layers; attn(l, q (n, H, hd)) -> z (n, H, hd) (or None when it wrote the post-processed
         result to buf zg itself) runs after K/V of the layer have been appended to the cache and written unquantized to
         buf k / v.  Returns the final normed hidden (n, d) (a buffer).  defer_final_norm: a plan whose last block leaves the
         hidden un-normalised returns it as it is and sets self.hidden_is_raw - the caller's head GEMM then carries the final
-        norm as the row scale of its product (head_of), and the norm launch goes away.  advance: the final norm's launch
-        counts pos up by one."""
+        norm as the row scale of its product (head_of), and the norm launch goes away; final_norm False: likewise at any row
+        count, for a caller that norms the few rows it needs itself (_normed).  advance: the final norm's launch counts pos up
+        by one."""
         cfg, b = self.cfg, self.buf
         assert n <= self.max_tokens
         self._embed_norm(tok, n)
@@ -407,7 +409,7 @@ class UVEngine:
         else:
             raw = self._layers_plain(n, tok, pos, rows, last_pos, st, attn, fused_attn)
         if raw:
-            if defer_final_norm and self.own_head_ok(n):
+            if not final_norm or (defer_final_norm and self.own_head_ok(n)):
                 self.hidden_is_raw = True
                 return x
             self._add_norm(x, x, 1.0, 0.0, n, None, b["xn"], adv)   # the final norm
@@ -594,10 +596,17 @@ class UVEngine:
                 self._rec = None
             plan.guard = guard
             plan.engine = self          # (keeps id(self) from being reused while the plan lives)
+            plan.raw = self.hidden_is_raw
             plans[key] = plan.close()
         plan.run(values, L.stream_ptr(self.buf["x"]))
-        self.hidden_is_raw = False
-        return self.buf["xn"][:n]
+        self.hidden_is_raw = plan.raw
+        return self.buf["x" if plan.raw else "xn"][:n]
+
+    def _normed(self, rows: Tensor) -> Tensor:
+        """The final norm of some rows of what _trunk returned, in place where it still has to be taken."""
+        if self.hidden_is_raw and rows.size(0):
+            self._add_norm(rows, rows, 1.0, 0.0, rows.size(0), None, rows)
+        return rows
 
     def own_head_ok(self, n: int) -> bool:
         """Whether head_of runs the head GEMM of n rows on this library's kernel with the final norm in it: 16-bit engines up
@@ -674,29 +683,80 @@ class UVEngine:
         return h
 
     # ------------------------------------------------------------------------------------------------ prefill
-    def pack_prompts(self, prompts: list[list[int]], rows: list[int], max_len: int, left_pad: bool = True) -> dict:
-        """Host-built packed indices of a prefill call (reference: prefill_packed_host, fast_decode.py:210-269): per packed
-        token its id, position, cache row and the last position of its prompt; cu_seqlens; the packed index of every
-        prompt's last token; per prompt the cache row, start and end position.  All as device tensors."""
-        dev = self.device
-        lens = np.fromiter((len(p) for p in prompts), dtype=np.int64, count=len(prompts))
+    def _staging(self, n: int):
+        """n int64 of pinned host memory out of a small ring, and the event to record behind the launch that reads it: a buffer
+        is handed out again only after that launch."""
+        self._stage_at = (self._stage_at + 1) % len(self._stage)
+        buf, ev = self._stage[self._stage_at]
+        if ev is not None:
+            ev.synchronize()
+        if buf is None or buf.numel() < n:
+            buf, ev = torch.empty(max(1024, n + n // 4), dtype=torch.int64, pin_memory=True), torch.cuda.Event()
+            self._stage[self._stage_at] = (buf, ev)
+        return buf, ev
+
+    def _pack(self, prompts, rows, max_len: int, left_pad: bool, st: KVState | None = None, idx: Tensor | None = None, lens=None,
+              check: Tensor | None = None) -> dict:
+        """pack_prompts; st: also bind its rows to the prompts; idx (n, T) with lens instead of prompts: right-aligned prompts
+        already on the device; check: n int64 of the device that the caller wants to see: pk["check"]() waits for this launch
+        and gives them.  The launch reads the host's tables in pinned memory: a copy to the device would make the host wait
+        for the passes still running (pageable memory) or cost the GPU 20 us (pinned memory)."""
+        if idx is None:
+            lens = np.fromiter((len(p) for p in prompts), dtype=np.int64, count=len(prompts))
+        n = len(lens)
         assert lens.min() > 0
         T = int(lens.max())
         assert T <= max_len
-        starts = (T - lens) if left_pad else np.zeros_like(lens)
-        cu = np.zeros(len(prompts) + 1, dtype=np.int64)
-        cu[1:] = np.cumsum(lens)
-        N = int(cu[-1])
+        N = int(lens.sum())
         assert N <= self.max_tokens, f"{N} prefill tokens exceed the engine's max_tokens {self.max_tokens}"
-        x = np.concatenate([np.asarray(p, dtype=np.int64) for p in prompts])   # (prompts may be lists or int arrays)
-        seg = np.repeat(np.arange(len(prompts), dtype=np.int64), lens)
-        pos = np.arange(N, dtype=np.int64) - cu[:-1][seg] + starts[seg]
         rows_np = np.asarray(rows, dtype=np.int64)
-        # one host -> device copy for all nine arrays
-        parts = [x, pos, rows_np[seg], (starts + lens - 1)[seg], cu, cu[1:] - 1, rows_np, starts, starts + lens]
-        flat = torch.from_numpy(np.concatenate(parts)).to(dev)
-        tok, pos_t, row, last, cu_t, last_idx, rows_t, starts_t, ends = flat.split([len(a) for a in parts])
-        return dict(N=N, tok=tok, pos=pos_t, row=row, last=last, cu=cu_t, last_idx=last_idx, rows=rows_t, starts=starts_t, ends=ends)
+        assert len(rows_np) == n
+        n_tok = N if idx is None else 0
+        buf, ev = self._staging(4 * n + 1 + n_tok)
+        h = buf.numpy()
+        h[0] = 0
+        np.cumsum(lens, out=h[1:n + 1])
+        h[n + 1:2 * n + 1] = rows_np
+        h[2 * n + 1:3 * n + 1] = (T - lens) if left_pad else 0
+        if idx is None:
+            np.concatenate([np.asarray(p, dtype=np.int64) for p in prompts], out=h[4 * n + 1:4 * n + 1 + N])   # (prompts may be lists or int arrays)
+        pinned = n <= 2047
+        host = buf if pinned else buf[:4 * n + 1 + n_tok].to(self.device)
+        src = host.data_ptr()
+        out = torch.empty(4 * N + 5 * n + 1, dtype=torch.int64, device=self.device)
+        tok, pos, row, last, last_idx, cu_t, rows_t, starts_t, ends = out.split([N, N, N, N, n, n + 1, n, n, n])
+        pk = dict(N=N, tok=tok, pos=pos, row=row, last=last, cu=cu_t, last_idx=last_idx, rows=rows_t, starts=starts_t, ends=ends,
+                  rows_h=(int(rows_np.min()), int(rows_np.max())))
+        at = out.data_ptr()
+        a = L.PromptTablesArgs(n=n, n_tokens=N, idx_ld=0 if idx is None else idx.size(1), cu=src, row=src + 8 * (n + 1), start=src + 8 * (2 * n + 1),
+                               tok=src + 8 * (4 * n + 1) if idx is None else idx.data_ptr(), tok_t=at, pos_t=at + 8 * N, row_t=at + 16 * N, last_t=at + 24 * N,
+                               last_idx=at + 32 * N, cu_out=cu_t.data_ptr(), row_out=rows_t.data_ptr(), start_out=starts_t.data_ptr(), end_out=ends.data_ptr())
+        if st is not None:
+            self._check_rows(pk, st)
+            a.st_pos, a.st_starts = st.pos.data_ptr(), st.starts.data_ptr()
+        if check is not None:
+            assert pinned and check.dtype == torch.int64 and check.is_contiguous() and check.numel() == n
+            a.check_in, a.check_out = check.data_ptr(), src + 8 * (3 * n + 1)
+
+            def seen():
+                ev.synchronize()
+                return h[3 * n + 1:4 * n + 1].copy()
+            pk["check"] = seen
+        L.check(L.lib().uvmi_prompt_tables(C.byref(a), L.stream_ptr(out)), "uvmi_prompt_tables")
+        ev.record()
+        return pk
+
+    @staticmethod
+    def _check_rows(pk: dict, st: KVState):
+        if pk["rows_h"][0] < 0 or pk["rows_h"][1] >= st.pos.numel():
+            raise IndexError(f"cache rows {pk['rows_h'][0]}..{pk['rows_h'][1]} of a state with {st.pos.numel()} rows")
+
+    def pack_prompts(self, prompts: list[list[int]], rows: list[int], max_len: int, left_pad: bool = True) -> dict:
+        """Packed indices of a prefill call (reference: prefill_packed_host, fast_decode.py:210-269): per packed token its id,
+        position, cache row and the last position of its prompt; cu_seqlens; the packed index of every prompt's last token; per
+        prompt the cache row, start and end position.  All as device tensors: the host uploads the tokens and one line
+        per prompt, a launch forms the per-token tables."""
+        return self._pack(prompts, rows, max_len, left_pad)
 
     @staticmethod
     def bind_prompts(pk: dict, st: KVState):
@@ -714,17 +774,26 @@ class UVEngine:
         Returns the final normed hidden of each prompt's last token and of each decode row.  Does not advance st.pos of
         the decode rows (the caller's slot table does), but binds the prompts' rows."""
         Np, nd = pk["N"], tok_d.numel()
-        tok, pos = torch.cat([pk["tok"], tok_d]), torch.cat([pk["pos"], pos_d])
-        rows, last = torch.cat([pk["row"], rows_d]), torch.cat([pk["last"], pos_d])
-        h = self.mixed_trunk(tok, pos, rows, last, Np, nd, pk["cu"], starts_d, st)
-        self.bind_prompts(pk, st)
-        return h.index_select(0, pk["last_idx"]), h[Np:Np + nd]
+        N = Np + nd
+        tables = torch.empty(4, N, dtype=torch.int64, device=self.device)
+        tok, pos, rows, last = tables.unbind(0)
+        tok_d, pos_d, rows_d = (t.to(torch.int64).contiguous() for t in (tok_d, pos_d, rows_d))
+        self._check_rows(pk, st)
+        a = L.PromptTablesArgs(n=pk["rows"].numel(), n_tokens=Np, nd=nd, cu=pk["cu"].data_ptr(), row=pk["rows"].data_ptr(), start=pk["starts"].data_ptr(),
+                               tok=pk["tok"].data_ptr(), tok_d=tok_d.data_ptr(), pos_d=pos_d.data_ptr(), rows_d=rows_d.data_ptr(), tok_t=tok.data_ptr(),
+                               pos_t=pos.data_ptr(), row_t=rows.data_ptr(), last_t=last.data_ptr())
+        L.check(L.lib().uvmi_prompt_tables(C.byref(a), L.stream_ptr(tables)), "uvmi_prompt_tables")
+        h = self.mixed_trunk(tok, pos, rows, last, Np, nd, pk["cu"], starts_d, st, final_norm=False)
+        b = L.PromptTablesArgs(n=a.n, cu=a.cu, row=a.row, start=a.start, st_pos=st.pos.data_ptr(), st_starts=st.starts.data_ptr())
+        L.check(L.lib().uvmi_prompt_tables(C.byref(b), L.stream_ptr(tables)), "uvmi_prompt_tables")   # (after the pass: pos_d may be a view of st.pos)
+        return self._normed(h.index_select(0, pk["last_idx"])), self._normed(h[Np:N])
 
     def mixed_trunk(self, tok: Tensor, pos: Tensor, rows: Tensor, last: Tensor, Np: int, nd: int, cu: Tensor, starts_d: Tensor,
-                    st: KVState) -> Tensor:
+                    st: KVState, final_norm: bool = True) -> Tensor:
         """The pass of mixed_step over already concatenated per-token arrays (Np packed prompt tokens, then nd decode rows;
         cu: the prompts' cu_seqlens on the device).  Allocation-free apart from the packed attention output, so a caller
-        that builds the arrays on the device can capture it in a graph.  Returns the final normed hidden (Np + nd, d)."""
+        that builds the arrays on the device can capture it in a graph.  Returns the final normed hidden (Np + nd, d); final_norm
+        False: as in _trunk."""
         cfg, b = self.cfg, self.buf
         N = Np + nd
         assert N <= self.max_tokens, f"{N} token rows exceed the engine's max_tokens {self.max_tokens}"
@@ -739,7 +808,7 @@ class UVEngine:
                 self._attn_post(l, zd, nd, off=Np)
             return None
 
-        run = lambda: self._trunk(tok[:N], pos[:N], N, attn, rows=rows[:N], last_pos=last[:N], st=st)
+        run = lambda: self._trunk(tok[:N], pos[:N], N, attn, rows=rows[:N], last_pos=last[:N], st=st, final_norm=final_norm)
         if (Np > 0 and nd > 0 and self._pass_kind(N, False, st) == "packed" and self.prompt_attention_plannable() and self._append_fused(st)
                 and all(self.cache_attention_plannable(l, st) for l in range(cfg.n_layers))):
             assert all(t.dtype == torch.int64 and t.stride(0) == 1 for t in (tok, pos, rows, last, starts_d))
@@ -747,7 +816,7 @@ class UVEngine:
             values = dict(n=N, Np=Np, nd=nd, tok=tok.data_ptr(), pos=pos.data_ptr(), rows=rows.data_ptr(), last=last.data_ptr(), cu=cu.data_ptr(),
                           n_seg=cu.numel() - 1, pos_d=pos_d.data_ptr(), rows_d=rows_d.data_ptr(), starts_d=starts_d.data_ptr(),
                           q_d=at("q"), vhat_d=at("vhat"), gate_d=at("gate"), zg_d=at("zg"))
-            return self._planned("mixed", st, "packed", N, values, run)
+            return self._planned("mixed" if final_norm else "mixed-raw", st, "packed", N, values, run)
         return run()
 
     @torch.no_grad()
@@ -758,21 +827,32 @@ class UVEngine:
         positions (token j of a prompt of length n sits at T - n + j, T = longest prompt of the call) so the cache
         layout equals the reference's; left_pad=False starts every prompt at position 0.  Sets st.pos / st.starts of the
         rows and returns the final normed hidden of each prompt's last token (len(prompts), d)."""
-        pk = self.pack_prompts(prompts, rows, st.max_len, left_pad)
-        N, b, cfg = pk["N"], self.buf, self.cfg
+        return self._prefill(self._pack(prompts, rows, st.max_len, left_pad, st), st)
+
+    @torch.no_grad()
+    def prefill_matrix(self, idx: Tensor, lens, rows, st: KVState, check: Tensor | None = None):
+        """prefill(left_pad=True) of the prompts that stand right-aligned in idx (n, T), an int64 matrix on the engine's device: the
+        last lens[a] (host) tokens of row a.  The token ids never visit the host.  check: also returns a function that gives
+        these n int64 of the device without waiting for the pass."""
+        assert idx.dtype == torch.int64 and idx.is_contiguous() and idx.size(0) == len(lens) and idx.size(1) >= int(lens.max())
+        pk = self._pack(None, rows, st.max_len, True, st, idx, lens, check)
+        h = self._prefill(pk, st)
+        return h if check is None else (h, pk["check"])
+
+    def _prefill(self, pk: dict, st: KVState) -> Tensor:
+        N = pk["N"]
 
         def attn(l, q):
             return self.prompt_attention(l, q, N, pk["cu"])
 
         tok, pos, row, last, cu = pk["tok"], pk["pos"], pk["row"], pk["last"], pk["cu"]
-        run = lambda: self._trunk(tok, pos, N, attn, rows=row, last_pos=last, st=st)
+        run = lambda: self._trunk(tok, pos, N, attn, rows=row, last_pos=last, st=st, final_norm=False)
         if self._pass_kind(N, False, st) == "packed" and self.prompt_attention_plannable() and self._append_fused(st):
             h = self._planned("prefill", st, "packed", N, dict(n=N, Np=N, tok=tok.data_ptr(), pos=pos.data_ptr(), rows=row.data_ptr(), last=last.data_ptr(),
                                                                 cu=cu.data_ptr(), n_seg=cu.numel() - 1), run)
         else:
             h = run()
-        self.bind_prompts(pk, st)
-        return h.index_select(0, pk["last_idx"])
+        return self._normed(h.index_select(0, pk["last_idx"]))   # (the norm of the prompts' last rows only)
 
     # ------------------------------------------------------------------------------------------------ generation
     @torch.no_grad()
