@@ -247,6 +247,18 @@ def test_backward_many_tiles_and_padding_tokens(dtype, H, K, window):
         assert np.linalg.norm(a[:N] - b) / np.linalg.norm(b) < (5e-3 if dtype == torch.float16 else 2e-2)
 
 
+@pytest.mark.parametrize("H,K", [(3, 1), (7, 1), (10, 2)])
+@pytest.mark.parametrize("n", [32, 33, 63, 65, 97])
+def test_backward_odd_head_groups_at_block_edges(H, K, n):
+    """Head groups that end inside a pair of heads, with keys and queries that end at and around the edges of the 32- and 64-row
+    blocks; a sequence boundary and a window inside a block."""
+    for lens, window in (([n], None), ([n - 20, 20], 24)):
+        got, ref = _grad_case(lens, H, K, torch.bfloat16, window, seed=n)
+        for a, b in zip(got, ref):
+            assert np.isfinite(a).all()
+            assert np.abs(a - b).max() <= 2 * 2.0 ** -7 * np.abs(b).max() + 1e-6, (lens, np.abs(a - b).max(), np.abs(b).max())
+
+
 def test_backward_rejects_what_it_cannot_do():
     from ultraviolet_amd import _lib as L
     from ultraviolet_amd.kernels.varlen_attn import packed_attention_backward

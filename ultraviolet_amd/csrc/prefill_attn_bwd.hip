@@ -238,8 +238,8 @@ __global__ __launch_bounds__(64) void bwd_dkv_kernel(BwdParams P) {
 //     of either accumulator holds 4 consecutive keys of one query row for two 16-key tiles, so p = exp2(c s - lse) and
 //     ds = p (dp - D) are lane-local, and the 8 values of ds, rounded to the input type, are the lane's slice of the B
 //     operand of dQ^T += K^T dS^T (K^T operands from 8-byte LDS reads regrouped with v_perm_b32, as V^T in the forward);
-//   * bwd_dkv_mfma: the transposed problem.  A workgroup owns 64 keys of one kv head (16 per wave) and walks (query tile of
-//     32, query head): the tile's Q and dO rows are staged in LDS; S = Q K^T and dP = dO V^T leave 4 consecutive queries
+//   * bwd_dkv_mfma: the transposed problem.  A workgroup owns 64 keys of one kv head and walks (query tile of 32, pair of query
+//     heads): the tile's Q and dO rows are staged in LDS; S = Q K^T and dP = dO V^T leave 4 consecutive queries
 //     of one key in a lane for two 16-query tiles, exactly the B-operand slices of dV^T += dO^T P and dK^T += Q^T dS, which
 //     accumulate over the tiles and over the heads of the group in registers.
 // Probabilities and ds are rounded to the input type for their second products; everything else is fp32.
@@ -445,129 +445,208 @@ __global__ __launch_bounds__(256) void bwd_dq_mfma(BwdMParams P) {
   }
 }
 
+// dk / dv.  What bounds it is the vector work per (query, key) pair (an exponential and ~8 instructions) and, before it was
+// pipelined, the round trips of the staged tiles: 31 700 tokens, window 256, took 130 us with 16 keys per wave, one tile in flight and
+// the statistics read from global memory inside the arithmetic; 72 us as it is now:
+//   * a wave owns 32 keys, so the operands of a query tile (16 KB of LDS reads, 32 permutes) serve two 16-key columns; the
+//     workgroup's waves are 2 key groups x 2 heads of a pair, which add their sums through LDS at the end;
+//   * the pair's Q and dO tiles and their statistics go from global memory straight into one of three LDS stages, two
+//     iterations ahead of their use (no staging registers; a wave's 1 KB load is 8 rows, the chunk swizzle is applied to the
+//     global address); an iteration waits for the loads of the one before last only;
+//   * the queries a key sees are an index range, key .. min(end of its sequence, key + window), found once per lane: the loop
+//     reads no tables.
+struct DkvStage { unsigned char t[4][4096]; float st[4][64]; };   // Q of head 0, 1, dO of head 0, 1; lse of head 0, 1, D of head 0, 1
+
 template <int DT>
-__global__ __launch_bounds__(256) void bwd_dkv_mfma(BwdMParams P) {
-  __shared__ __attribute__((aligned(16))) unsigned char smem[2][2][4096];  // [half][Q, dO][32 queries x 128 B]
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void bwd_dkv_mfma(BwdMParams P) {
+  // (one object per stage: the compiler can then tell that reads of one stage do not touch the stage a load is filling)
+  __shared__ __attribute__((aligned(1024))) DkvStage s0, s1, s2;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int per = gridDim.x >> 3;
   const int bid = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
   if (bid >= P.n_wg) return;
   const int kvh = bid % P.KH, kb = bid / P.KH;
   const int n = lane & 15, g = lane >> 4;   // accumulator column n = key, group g = queries 4g .. 4g+3 of a 16-query tile
-  const int G = P.G;
+  const int kg = wave & 1, hg = wave >> 1;
+  const int G = P.G, GP = (G + 1) >> 1;     // head pairs
   const float c = P.scale_log2;
   int n_end = (int)load_index(P.cu, P.idx64, P.n_seg);
   n_end = n_end < 0 ? 0 : (n_end > P.N ? P.N : n_end);
   const int jw0 = kb * 64, jw_last = min(jw0 + 63, n_end - 1);
-  const int key = jw0 + 16 * wave + n;
-  const bool key_ok = key < n_end;
-  const int keyc = key < P.N ? key : P.N - 1;
-  // ---- K^T / V^T operands (B side: lane = key n, dims 32 s + 8 g ..)
-  pu4 Kb[2], Vb[2];
-  {
-    const int64_t base = ((int64_t)keyc * P.KH + kvh) * 64 + 8 * g;
-    Kb[0] = *(const pu4*)((const uint16_t*)P.k + base);
-    Kb[1] = *(const pu4*)((const uint16_t*)P.k + base + 32);
-    Vb[0] = *(const pu4*)((const uint16_t*)P.v + base);
-    Vb[1] = *(const pu4*)((const uint16_t*)P.v + base + 32);
-  }
-  pf4 dK[4], dV[4];
+  const int key0 = jw0 + 32 * kg + n;       // column block b: key0 + 16 b
+  // ---- K^T / V^T operands (B side: lane = key, dims 32 s + 8 g ..)
+  pu4 Kb[2][2], Vb[2][2];
 #pragma unroll
-  for (int t = 0; t < 4; t++) dK[t] = dV[t] = pf4{0.f, 0.f, 0.f, 0.f};
-  // queries that may see a key of this workgroup: jw0 .. qend - 1 (its keys' segment may end earlier: checked per tile)
-  int qend = n_end;
-  if (P.window > 0 && jw_last + P.window < qend) qend = jw_last + P.window;
-  const int n_tiles = jw0 < n_end ? (qend - jw0 + 31) >> 5 : 0;
-  const int n_it = n_tiles * G;
-  const int lrow = tid >> 3, lch = tid & 7;
-  const uint32_t st_off = lds_chunk_off(lrow, lch);
-  pu4 rq, rg;
-  auto fetch = [&](int it) {
-    const int itc = min(it, max(n_it - 1, 0));
-    const int tq = jw0 + 32 * (itc / G), head = kvh * G + itc % G;
-    const int64_t r = ((int64_t)min(tq + lrow, P.N - 1) * P.H + head) * 64 + 8 * lch;
-    rq = *(const pu4*)((const uint16_t*)P.q + r);
-    rg = *(const pu4*)((const uint16_t*)P.go + r);
+  for (int b = 0; b < 2; b++) {
+    const int64_t base = ((int64_t)min(key0 + 16 * b, P.N - 1) * P.KH + kvh) * 64 + 8 * g;
+    Kb[b][0] = *(const pu4*)((const uint16_t*)P.k + base);
+    Kb[b][1] = *(const pu4*)((const uint16_t*)P.k + base + 32);
+    Vb[b][0] = *(const pu4*)((const uint16_t*)P.v + base);
+    Vb[b][1] = *(const pu4*)((const uint16_t*)P.v + base + 32);
+  }
+  pf4 dK[2][4], dV[2][4];
+#pragma unroll
+  for (int b = 0; b < 2; b++)
+#pragma unroll
+    for (int t = 0; t < 4; t++) dK[b][t] = dV[b][t] = pf4{0.f, 0.f, 0.f, 0.f};
+  // ---- sequences of the first and the last key (the last s with cu[s] <= key), 64 probes at a time
+  auto seq_of = [&](int j) {
+    int lo = 0, hi = P.n_seg;   // cu[lo] <= j, and hi == n_seg or cu[hi] > j
+    while (hi - lo > 1) {
+      const int step = (hi - lo + 63) >> 6, at = lo + (lane + 1) * step;
+      const bool below = at < hi && load_index(P.cu, P.idx64, at) <= j;
+      lo += __popcll(__ballot(below)) * step;
+      hi = min(hi, lo + step);
+    }
+    return lo;
   };
-  auto park = [&](int half) {
-    *(pu4*)(&smem[half][0][st_off]) = rq;
-    *(pu4*)(&smem[half][1][st_off]) = rg;
-  };
-  auto step = [&](int half, int tq, int head, bool interior) {
-    pu4 QA[4], GA[4], QT[4], GT[4];
-    pu2 rt[8];
-    read_rows_a(smem[half][0], n, g, QA);
-    read_rows_a(smem[half][1], n, g, GA);
-    read_rows_t(smem[half][0], n, g, rt);
-    transpose_ops(rt, QT);
-    read_rows_t(smem[half][1], n, g, rt);
-    transpose_ops(rt, GT);
-    pf4 sA = pf4{0.f, 0.f, 0.f, 0.f}, sB = sA, pA = sA, pB = sA;
-    sA = mfma16<DT>(QA[0], Kb[0], sA);
-    sB = mfma16<DT>(QA[2], Kb[0], sB);
-    pA = mfma16<DT>(GA[0], Vb[0], pA);
-    pB = mfma16<DT>(GA[2], Vb[0], pB);
-    sA = mfma16<DT>(QA[1], Kb[1], sA);
-    sB = mfma16<DT>(QA[3], Kb[1], sB);
-    pA = mfma16<DT>(GA[1], Vb[1], pA);
-    pB = mfma16<DT>(GA[3], Vb[1], pB);
-    // statistics of this lane's queries tq + 4g + i (tile A) and tq + 16 + 4g + i (tile B)
-    const float* lp = P.lse + (int64_t)head * P.lse_ld + tq + 4 * g;
-    const float* dp = P.dsum + (int64_t)head * P.ls + tq + 4 * g;
-    const float4 la = *(const float4*)lp, lb = *(const float4*)(lp + 16), da = *(const float4*)dp, db = *(const float4*)(dp + 16);
-    const float lA[4] = {la.x, la.y, la.z, la.w}, lB[4] = {lb.x, lb.y, lb.z, lb.w};
-    const float dA[4] = {da.x, da.y, da.z, da.w}, dB[4] = {db.x, db.y, db.z, db.w};
-    float p[8], ds[8];
+  int first_end = 0, last_end = 0, hi_q[2] = {0, 0};   // ends of those sequences; key block b is seen by queries key .. hi_q[b] - 1
+  if (jw0 < n_end) {
+    const int sf = seq_of(jw0), sl = seq_of(jw_last);
+    first_end = min((int)load_index(P.cu, P.idx64, sf + 1), n_end);
+    last_end = min((int)load_index(P.cu, P.idx64, sl + 1), n_end);
+    hi_q[0] = hi_q[1] = last_end;
+    for (int s = sl - 1; s >= sf; s--) {
+      const int e = (int)load_index(P.cu, P.idx64, s + 1);
+#pragma unroll
+      for (int b = 0; b < 2; b++)
+        if (key0 + 16 * b < e) hi_q[b] = e;
+    }
+#pragma unroll
+    for (int b = 0; b < 2; b++) {
+      if (P.window > 0) hi_q[b] = min(hi_q[b], key0 + 16 * b + P.window);
+      if (key0 + 16 * b >= n_end) hi_q[b] = 0;
+    }
+  }
+  const int qend = P.window > 0 ? min(last_end, jw_last + P.window) : last_end;
+  const int n_it = jw0 < n_end ? ((qend - jw0 + 31) >> 5) * GP : 0;
+
+  // ---- loader: wave w fills tile w and statistics row w of a stage: Q / dO of head w % 2, four loads of 8 rows
+  const int lrow = lane >> 3, lch = lane & 7;
+  const uint16_t* lsrc = (const uint16_t*)(wave < 2 ? P.q : P.go);
+  const float* lst = wave < 2 ? P.lse : P.dsum;
+  const int64_t lst_ld = wave < 2 ? P.lse_ld : P.ls;
+  int f_t = 0, f_p = 0;   // tile and head pair of the next request
+  auto issue = [&](DkvStage& S) {
+    const int tq = jw0 + 32 * f_t, head = kvh * G + min(2 * f_p + (wave & 1), G - 1);
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      p[i] = __builtin_amdgcn_exp2f(fmaf(sA[i], c, -lA[i]));
-      p[4 + i] = __builtin_amdgcn_exp2f(fmaf(sB[i], c, -lB[i]));
-      ds[i] = p[i] * (pA[i] - dA[i]);
-      ds[4 + i] = p[4 + i] * (pB[i] - dB[i]);
+      const int r = 8 * i + lrow;
+      const uint16_t* src = lsrc + ((int64_t)min(tq + r, P.N - 1) * P.H + head) * 64 + 8 * (lch ^ ((r >> 1) & 7));
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)(S.t[wave] + 1024 * i), 16, 0, 0);
     }
-    if (!interior) {   // (selects, not products: the statistics of a query past the last token are whatever the workspace held)
-      const int4 sa = *(const int4*)(P.seg_start + tq + 4 * g), sb = *(const int4*)(P.seg_start + tq + 16 + 4 * g);
-      const int sA_[4] = {sa.x, sa.y, sa.z, sa.w}, sB_[4] = {sb.x, sb.y, sb.z, sb.w};
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(lst + head * lst_ld + min(tq + (lane & 31), P.N - 1)),
+                                     (__attribute__((address_space(3))) void*)S.st[wave], 4, 0, 0);
+    if (++f_p == GP) { f_p = 0; f_t = min(f_t + 1, max((qend - jw0 - 1) >> 5, 0)); }   // (past the last tile: re-reads of it, into a stage nobody uses)
+  };
+  int c_t = 0, c_p = 0;   // tile and head pair of the next arithmetic
+  auto step = [&](const DkvStage& S) {
+    const int tq = jw0 + 32 * c_t;
+    const bool live = 2 * c_p + hg < G;   // (an odd last head has no partner)
+    // no mask needed when every query of the tile follows every key, in the first key's sequence and window
+    const bool interior = tq >= jw0 + 63 && tq + 31 < first_end && (P.window == 0 || tq + 31 - jw0 < P.window);
+    if (++c_p == GP) { c_p = 0; c_t++; }
+    if (!live) return;
+    const unsigned char* sq = S.t[hg];
+    const unsigned char* sg = S.t[2 + hg];
+    pu4 QA[4], GA[4];
+    read_rows_a(sq, n, g, QA);
+    read_rows_a(sg, n, g, GA);
+    // statistics of this lane's queries tq + 4g + i (tile A) and tq + 16 + 4g + i (tile B)
+    const pf4 lA = *(const pf4*)(S.st[hg] + 4 * g), lB = *(const pf4*)(S.st[hg] + 16 + 4 * g);
+    const pf4 dA = *(const pf4*)(S.st[2 + hg] + 4 * g), dB = *(const pf4*)(S.st[2 + hg] + 16 + 4 * g);
+    pu4 PB[2], SB[2];
+#pragma unroll
+    for (int b = 0; b < 2; b++) {
+      pf4 sA = pf4{0.f, 0.f, 0.f, 0.f}, sB = sA, pA = sA, pB = sA;
+      sA = mfma16<DT>(QA[0], Kb[b][0], sA);
+      sB = mfma16<DT>(QA[2], Kb[b][0], sB);
+      pA = mfma16<DT>(GA[0], Vb[b][0], pA);
+      pB = mfma16<DT>(GA[2], Vb[b][0], pB);
+      sA = mfma16<DT>(QA[1], Kb[b][1], sA);
+      sB = mfma16<DT>(QA[3], Kb[b][1], sB);
+      pA = mfma16<DT>(GA[1], Vb[b][1], pA);
+      pB = mfma16<DT>(GA[3], Vb[b][1], pB);
+      float p[8], ds[8];
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        const int ia = tq + 4 * g + i, ib = ia + 16;
-        const bool va = key_ok && ia < n_end && key <= ia && (P.window == 0 || ia - key < P.window) && sA_[i] <= key;
-        const bool vb = key_ok && ib < n_end && key <= ib && (P.window == 0 || ib - key < P.window) && sB_[i] <= key;
-        if (!va) { p[i] = 0.f; ds[i] = 0.f; }
-        if (!vb) { p[4 + i] = 0.f; ds[4 + i] = 0.f; }
+        p[i] = __builtin_amdgcn_exp2f(fmaf(sA[i], c, -lA[i]));
+        p[4 + i] = __builtin_amdgcn_exp2f(fmaf(sB[i], c, -lB[i]));
+        ds[i] = p[i] * (pA[i] - dA[i]);
+        ds[4 + i] = p[4 + i] * (pB[i] - dB[i]);
       }
-    }
-    const pu4 PB = pu4{pack2<DT>(p[0], p[1]), pack2<DT>(p[2], p[3]), pack2<DT>(p[4], p[5]), pack2<DT>(p[6], p[7])};
-    const pu4 SB = pu4{pack2<DT>(ds[0], ds[1]), pack2<DT>(ds[2], ds[3]), pack2<DT>(ds[4], ds[5]), pack2<DT>(ds[6], ds[7])};
+      if (!interior) {   // (selects, not products: the statistics of a query past the last token are whatever the workspace held)
+        const int key = key0 + 16 * b;
 #pragma unroll
-    for (int t = 0; t < 4; t++) {
-      dV[t] = mfma16<DT>(GT[t], PB, dV[t]);
-      dK[t] = mfma16<DT>(QT[t], SB, dK[t]);
+        for (int i = 0; i < 8; i++) {
+          const int iq = tq + 4 * g + (i & 3) + 16 * (i >> 2);
+          if (iq < key || iq >= hi_q[b]) { p[i] = 0.f; ds[i] = 0.f; }
+        }
+      }
+      PB[b] = pu4{pack2<DT>(p[0], p[1]), pack2<DT>(p[2], p[3]), pack2<DT>(p[4], p[5]), pack2<DT>(p[6], p[7])};
+      SB[b] = pu4{pack2<DT>(ds[0], ds[1]), pack2<DT>(ds[2], ds[3]), pack2<DT>(ds[4], ds[5]), pack2<DT>(ds[6], ds[7])};
     }
+    pu2 rt[8];
+    pu4 T[4];
+    read_rows_t(sg, n, g, rt);
+    transpose_ops(rt, T);
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+      for (int b = 0; b < 2; b++) dV[b][t] = mfma16<DT>(T[t], PB[b], dV[b][t]);
+    read_rows_t(sq, n, g, rt);
+    transpose_ops(rt, T);
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+      for (int b = 0; b < 2; b++) dK[b][t] = mfma16<DT>(T[t], SB[b], dK[b][t]);
   };
   if (n_it > 0) {
-    fetch(0);
-    park(0);
+    // iteration i: request i + 2 into the stage that i - 1 used (every wave is done with it: the barrier), multiply i, wait
+    // until i + 1 has landed (its 5 loads are all but the newest 5)
+    issue(s0);
+    issue(s1);
+    __builtin_amdgcn_s_waitcnt(0x0f75);   // vmcnt(5)
     __syncthreads();
-    bool interior = false;
-    for (int it = 0; it < n_it; it++) {
-      const int tq = jw0 + 32 * (it / G), hh = it % G;
-      if (hh == 0) {   // workgroup-uniform: the first query of the tile starts a later sequence than the last key's - done
-        if (P.seg_start[min(tq, P.N - 1)] > jw_last) break;
-        // no mask needed when every query of the tile follows every key, in the first key's sequence and window
-        interior = tq >= jw0 + 63 && tq + 31 < n_end && jw0 + 63 < n_end && P.seg_start[tq + 31] <= jw0 &&
-                   (P.window == 0 || tq + 31 - jw0 < P.window);
-      }
-      fetch(it + 1);
-      step(it & 1, tq, kvh * G + hh, interior);
-      park((it + 1) & 1);
-      __syncthreads();
+#define UVMI_DKV(CUR, NEXT2)                                             \
+  do {                                                                   \
+    issue(NEXT2);                                                        \
+    step(CUR);                                                           \
+    __builtin_amdgcn_s_waitcnt(0x0f75);                                  \
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      \
+  } while (0)
+    int it = 0;
+    for (; it + 3 <= n_it; it += 3) {
+      UVMI_DKV(s0, s2);
+      UVMI_DKV(s1, s0);
+      UVMI_DKV(s2, s1);
     }
+    if (it < n_it) UVMI_DKV(s0, s2);
+    if (it + 1 < n_it) UVMI_DKV(s1, s0);
+#undef UVMI_DKV
+    __builtin_amdgcn_s_waitcnt(0x0f70);   // the requests past the last iteration have landed before LDS is used again
+    __syncthreads();
   }
-  if (key < P.N) {   // (zeros for padding tokens)
-    const int64_t off = ((int64_t)key * P.KH + kvh) * 64 + 16 * g;
-    store_dims16<DT>(P.dk, off, dK, P.scale);
-    store_dims16<DT>(P.dv, off, dV, 1.0f);
+  // ---- the two heads of a pair meet in LDS: head 0's wave finishes dk of its keys, head 1's dv
+  float* mine = (float*)(kg ? &s1 : &s0) + (hg ? 0 : 2048) + lane;        // what the partner takes: [register][lane]
+  const float* theirs = (const float*)(kg ? &s1 : &s0) + (hg ? 2048 : 0) + lane;
+#pragma unroll
+  for (int b = 0; b < 2; b++)
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) mine[((b * 4 + t) * 4 + i) * 64] = hg ? dK[b][t][i] : dV[b][t][i];
+  __syncthreads();
+#pragma unroll
+  for (int b = 0; b < 2; b++) {
+    pf4 acc[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) acc[t][i] = (hg ? dV[b][t][i] : dK[b][t][i]) + theirs[((b * 4 + t) * 4 + i) * 64];
+    const int key = key0 + 16 * b;
+    if (key < P.N)   // (zeros for padding tokens)
+      store_dims16<DT>(hg ? P.dv : P.dk, ((int64_t)key * P.KH + kvh) * 64 + 16 * g, acc, hg ? 1.0f : P.scale);
   }
 }
 
