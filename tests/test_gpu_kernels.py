@@ -701,6 +701,38 @@ def test_skinny_gemm_norm_and_resid_fusions(dtype, M, K, N):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [(1, 16, 64), (16, 32, 576), (17, 48, 512), (31, 96, 640), (33, 160, 1088), (64, 64, 448), (65, 80, 1664), (1100, 656, 640)])
+def test_streaming_gemm_edges(dtype, M, N, K):
+    """The streaming form's tiles (16 x 16, 16 x 32, 32 x 32, 32 x 64, 64 x 64 by config, and the built-in choice) at the edges of
+    tiles and with every split of K over the waves: fewer slabs than waves, uneven shares, one slab."""
+    from ultraviolet_amd.kernels.gemm import RESID, SWIGLU, gemm_tn, interleave_gate_up
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a = (torch.randn(M, K, device="cuda", generator=g) * 2).to(dtype)
+    w = (torch.randn(N, K, device="cuda", generator=g) / K ** 0.5).to(dtype)
+    r = torch.randn(M, N, device="cuda", generator=g).to(dtype)
+    ulp, eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11, 1e-6
+    ad = a.double()
+    an = ad * torch.rsqrt((ad * ad).mean(-1, keepdim=True) + eps)
+    ref, prod = an @ w.double().t(), (ad @ w.double().t()).to(dtype).double()
+    want = 0.75 * r.double() + 1.25 * prod
+    for config in (2, 7, 8, 1, 4, 0):
+        full = torch.full((M, N + 4), 7.0, device="cuda", dtype=dtype)
+        gemm_tn(a, w, full[:, :N], norm_eps=eps, config=config)
+        assert bool(((full[:, :N].double() - ref).abs() <= ulp * ref.abs().clamp_min(1.0) + 1e-5 * K ** 0.5).all()), config
+        assert bool((full[:, N:] == 7.0).all())
+        x = r.clone()
+        gemm_tn(a, w, x, epilogue=RESID, resid=x, ca=0.75, cb=1.25, config=config)
+        assert bool(((x.double() - want).abs() <= ulp * want.abs().clamp_min(1.0) + 2.5 * ulp * prod.abs().clamp_min(1.0)).all()), config
+        if N % 32 == 0 and (K <= 960 or config not in (1, 2)):
+            f = N // 2
+            gg, uu = ((an @ v.double().t()).to(dtype).double() for v in (w[:f], w[f:]))
+            ra = (gg * torch.sigmoid(gg)).to(dtype).double() * uu
+            act = gemm_tn(a, interleave_gate_up(w[:f].contiguous(), w[f:].contiguous()), epilogue=SWIGLU, norm_eps=eps, config=config)
+            assert bool(((act.double() - ra).abs() <= 4 * ulp * ra.abs().clamp_min(1.0) + 4 * ulp * (gg.abs() + uu.abs())).all()), config
+
+
+@pytest.mark.gpu
 def test_tiled_gemm_at_prefill_row_counts():
     """The projections of a packed prefill pass at its size (33 216 rows, the mixed-batch config): gate-up with the pre-norm
     and SwiGLU, and the output projection with the residual update in place, on both tile shapes and on the shape the

@@ -1,0 +1,344 @@
+// 16-bit GEMM for steps of up to a few thousand rows: C[M, N] = A[M, K] . W[N, K]^T, fp32 accumulation, with the epilogues of
+// the other forms - SwiGLU on interleaved gate / up slabs, the block's residual update, the RMS pre-norm as a row scale.  These
+// are the F.linear calls of the reference's fused inference path (ultraviolet/model.py:302-335 attention projections,
+// 388-391 MLP) with what surrounds them (:566-571).
+//
+// What bounds it: 0.7 - 4.3 MB of weights that the previous layers have pushed out of the L2, and activations that another XCD
+// wrote: a launch lasts as long as the round trips to the last-level cache that it puts in sequence, then as long as a compute
+// unit takes to pull its tiles through the L2 (64 bytes per clock).  To keep that pipe full for one trip of ~1 us takes ~150 KB in
+// flight per compute unit, which is what LDS holds.  So:
+//   * the NW waves of a workgroup split K: wave w takes the 64-wide slabs w, w + NW, .. of the tile's rows of A and W, from global
+//     memory straight into its own part of LDS (16 bytes per lane, a 1 KB load is 8 rows), R slabs ahead, and multiplies them
+//     into its own accumulators of the whole tile.  A wave waits for its own loads only: the loop has no barrier, no staging
+//     registers and no LDS stores, and an operand fragment is read from LDS once per 16-row fragment of the other side;
+//   * small problems have all their slabs in flight within the first few hundred cycles;
+//   * LDS rows are 128 bytes with the 16-byte chunk index xor-ed with (row / 2) % 8 (the lane fetches the chunk that belongs at
+//     its place), so the 16-row operand reads (lane (r, g) reads chunk 4 s + g of row r) touch every bank once;
+//   * the MFMA's A input is the weight fragment and its B input the activation fragment, so an accumulator holds C^T: a lane
+//     has 4 consecutive columns of one row and stores them as one 8-byte write;
+//   * the partial sums meet in LDS (the slabs' space) behind the kernel's only barrier; a wave adds and finishes its share of the
+//     fragments.  The residual of that share is requested before anything else, the squares of NORM are summed from the
+//     operand fragments as they pass;
+//   * rows past M or N are clamped to the last one (computed, not stored);
+//   * individual scalar arguments rather than a parameter block: they arrive in SGPRs with the wave.
+// us per launch in a stream of launches with 20 layers' weights in turn (N x K: 656 x 640 with NORM | 640 x 512 RESID | 3328 x 640
+// NORM, SWIGLU | 640 x 1664 RESID), and in brackets what the forms took that it replaced (a whole weight strip parked in LDS
+// behind a barrier below 448 rows, 64 x 64 tiles through registers from there on):
+//      1 row   2.7 [3.9] | 2.5 [3.8] | 3.4 [4.7] | 2.9 [4.3]        64 rows   2.8 [4.4] | 2.5 [4.3] | 3.9 [6.0] | 3.2 [5.3]
+//    256 rows  3.6 [5.6] | 3.0 [5.4] | 5.8 [6.5] | 4.6 [9.2]       512 rows   4.4 [6.2] | 3.7 [5.2] | 8.1 [8.7] | 5.9 [8.9]
+//   2048 rows  7.9 [8.4] | 6.7 [7.4] |     -     | 12.1 [13.7]
+#include "common.h"
+#include "gemm_util.h"
+
+namespace uvmi {
+
+struct StreamParams {
+  const void* a; const void* w; void* c; const void* r;
+  int64_t ldc, ldr;     // elements
+  uint32_t lda2, ldw2;  // row pitches in bytes
+  int M, N, K, tiles_m, tiles_n, rowsplit;
+  float eps, ca, cb;
+};
+
+#define UVMI_GLBP(p) ((const __attribute__((address_space(1))) void*)(p))
+#define UVMI_LDSP(p) ((__attribute__((address_space(3))) void*)(p))
+
+// s + the squares of the 8 values of an operand word
+template <int DT>
+__device__ __forceinline__ float sumsq8(gu4 v, float s) {
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    float lo, hi;
+    if (DT == UVMI_BF16) { lo = __uint_as_float(v[i] << 16); hi = __uint_as_float(v[i] & 0xffff0000u); }
+    else { lo = half_bits_to_float((uint16_t)(v[i] & 0xffff)); hi = half_bits_to_float((uint16_t)(v[i] >> 16)); }
+    s = fmaf(lo, lo, s);
+    s = fmaf(hi, hi, s);
+  }
+  return s;
+}
+
+template <int N> __device__ __forceinline__ void wait_vm() {   // all but the newest N loads have landed
+  static_assert(N >= 0 && N < 64, "vmcnt has six bits");
+  __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N >> 4) << 14));
+}
+
+// EPI 0: C = A W^T (M, N).  EPI 1: W rows are [gate 16 | up 16] slabs; C = silu(gate) * up, (M, N / 2); a tile of 16 columns
+// takes 8 gate rows and their 8 up rows.  EPI 2: C = ca * R + cb * (A W^T).  NORM: A stands for its RMS-normalised rows.
+template <int DT, int BM, int BN, int NW, int R, int EPI, bool NORM>
+__global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(const void* a_a, const void* a_w, uint32_t a_lda2, uint32_t a_ldw2, int a_M, int a_N,
+                                                              int a_K, int a_tiles_m, int a_tiles_n, int a_rowsplit, const void* a_r,
+                                                              void* a_c, int64_t a_ldc, int64_t a_ldr, float a_eps, float a_ca, float a_cb) {
+  const StreamParams P = {a_a, a_w, a_c, a_r, a_ldc, a_ldr, a_lda2, a_ldw2, a_M, a_N, a_K, a_tiles_m, a_tiles_n, a_rowsplit, a_eps, a_ca, a_cb};
+  constexpr int FM = BM / 16, FN = BN / 16, F = FM * FN;
+  constexpr int ROWS = BM + BN, LOADS = ROWS / 8;          // a load instruction moves 8 rows of 128 bytes
+  constexpr int FW = (F + NW - 1) / NW;                    // fragments per wave in the epilogue
+  static_assert(R == 1 || R == 2, "slabs of a wave in flight");
+  static_assert(F * 1024 <= ROWS * 128, "a wave's partial sums fit its slab's space");
+  // (one object per stage: the compiler can then tell that reads of one do not touch the one a load is filling)
+  __shared__ __attribute__((aligned(1024))) unsigned char s0[NW * ROWS * 128];
+  __shared__ __attribute__((aligned(1024))) unsigned char s1[R > 1 ? NW * ROWS * 128 : 16];
+  __shared__ float sSS[NORM ? NW * BM : 1];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int T = P.tiles_m * P.tiles_n, per = (T + 7) / 8;
+  const int L = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+  if (L >= T) return;
+  const int bn = P.rowsplit ? L % P.tiles_n : L / P.tiles_m, bm = P.rowsplit ? L / P.tiles_n : L % P.tiles_m;
+  const int m0 = bm * BM, n0 = bn * BN;
+  const int r = lane & 15, g = lane >> 4;
+
+  // ---- loader: load i of a slab moves its rows 8 i .. 8 i + 7 (the tile's rows of A, then of W)
+  const int lr = lane >> 3;
+  const unsigned char* gp[LOADS];
+#pragma unroll
+  for (int i = 0; i < LOADS; i++) {
+    const int row = 8 * i + lr;
+    const int sw = (lane & 7) ^ ((row >> 1) & 7);
+    if (8 * i < BM) gp[i] = (const unsigned char*)P.a + (uint32_t)min(m0 + row, P.M - 1) * (size_t)P.lda2 + 16 * sw;
+    else {
+      const int j = row - BM;
+      const int wr = EPI == 1 && BN == 16 ? (n0 & ~31) + ((n0 & 16) >> 1) + (j & 7) + ((j & 8) << 1) : n0 + j;
+      gp[i] = (const unsigned char*)P.w + (uint32_t)min(wr, P.N - 1) * (size_t)P.ldw2 + 16 * sw;
+    }
+  }
+  const int nk = P.K / 64;
+  const int nw = (nk - wave + NW - 1) / NW;                // slabs of this wave: wave, wave + NW, ..
+  const int lds0 = wave * (ROWS * 128);
+  auto issue = [&](unsigned char* S, int i) {
+    const int ko = (wave + NW * i) * 128;
+#pragma unroll
+    for (int l = 0; l < LOADS; l++) __builtin_amdgcn_global_load_lds(UVMI_GLBP(gp[l] + ko), UVMI_LDSP(S + lds0 + 1024 * l), 16, 0, 0);
+  };
+
+  // ---- this wave's share of the output, and its residual
+  uint2 res[FW];
+  int f_of[FW];
+#pragma unroll
+  for (int i = 0; i < FW; i++) f_of[i] = wave * FW + i;
+  if (EPI == 2) {
+#pragma unroll
+    for (int i = 0; i < FW; i++) {
+      const int fi = f_of[i] / FN, fj = f_of[i] % FN;
+      const int row = m0 + 16 * fi + r, n = n0 + 16 * fj;
+      res[i] = uint2{0u, 0u};
+      if (f_of[i] < F && row < P.M && n < P.N) res[i] = *(const uint2*)((const uint16_t*)P.r + (int64_t)row * P.ldr + n + 4 * g);
+    }
+  }
+  if (nw > 0) issue(s0, 0);
+  if (R > 1 && nw > 1) issue(s1, 1);
+
+  gf4 acc[FM][FN];
+  float ss[FM];
+#pragma unroll
+  for (int i = 0; i < FM; i++) {
+    ss[i] = 0.f;
+#pragma unroll
+    for (int j = 0; j < FN; j++) acc[i][j] = gf4{0.f, 0.f, 0.f, 0.f};
+  }
+  const uint32_t ld0 = (uint32_t)r * 128 + (uint32_t)((g ^ ((r >> 1) & 7)) << 4), ld1 = (uint32_t)r * 128 + (uint32_t)(((4 + g) ^ ((r >> 1) & 7)) << 4);
+  auto slab = [&](unsigned char* S, int i) {
+    if (R > 1 && i + 1 < nw) wait_vm<LOADS>(); else wait_vm<0>();   // (loads land in order)
+    asm volatile("" ::: "memory");
+    const unsigned char* A = S + lds0;
+    const unsigned char* B = A + BM * 128;
+    gu4 af[2][FM], wf[2][FN];
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+#pragma unroll
+      for (int j = 0; j < FN; j++) wf[s][j] = *(const gu4*)(B + 2048 * j + (s ? ld1 : ld0));
+#pragma unroll
+      for (int f = 0; f < FM; f++) af[s][f] = *(const gu4*)(A + 2048 * f + (s ? ld1 : ld0));
+    }
+    if (i + R < nw) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the slab is in registers: its place may be filled again
+      issue(S, i + R);
+    }
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+#pragma unroll
+      for (int f = 0; f < FM; f++) {
+#pragma unroll
+        for (int j = 0; j < FN; j++) acc[f][j] = gmfma<DT>(wf[s][j], af[s][f], acc[f][j]);
+        if (NORM) ss[f] = sumsq8<DT>(af[s][f], ss[f]);
+      }
+    }
+  };
+  int i = 0;
+  if constexpr (R == 1) {
+    for (; i < nw; i++) slab(s0, i);
+  } else {
+    for (; i + 2 <= nw; i += 2) { slab(s0, i); slab(s1, i + 1); }
+    if (i < nw) slab(s0, i);
+  }
+
+  // ---- the waves' partial sums meet in LDS
+  if (NORM) {
+#pragma unroll
+    for (int f = 0; f < FM; f++) {
+      float v = ss[f];
+      v += __shfl_xor(v, 16, 64);
+      v += __shfl_xor(v, 32, 64);
+      if (g == 0) sSS[wave * BM + 16 * f + r] = v;
+    }
+  }
+  auto part = [&](int w, int f) { return (gf4*)(s0 + w * (ROWS * 128) + 1024 * f) + lane; };   // fragment f of wave w's sums
+#pragma unroll
+  for (int fi = 0; fi < FM; fi++)
+#pragma unroll
+    for (int fj = 0; fj < FN; fj++) *part(wave, fi * FN + fj) = acc[fi][fj];
+  __syncthreads();
+  gf4 o[FW];
+  float rn[FW];
+#pragma unroll
+  for (int q = 0; q < FW; q++) {
+    const int f = f_of[q];
+    if (F % NW != 0 && f >= F) break;
+    gf4 v = *part(0, f);
+#pragma unroll
+    for (int w = 1; w < NW; w++) v += *part(w, f);
+    rn[q] = 1.0f;
+    if (NORM) {
+      const int rl = 16 * (f / FN) + r;
+      float t = sSS[rl];
+#pragma unroll
+      for (int w = 1; w < NW; w++) t += sSS[w * BM + rl];
+      rn[q] = rsqrtf(t / (float)P.K + P.eps);
+    }
+    o[q] = v;
+  }
+  if constexpr (EPI == 1 && BN == 16) {
+#pragma unroll
+    for (int q = 0; q < FW; q++) {
+      const int f = f_of[q], row = m0 + 16 * f + r;
+      float x[4];
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        const float gv = ground<DT>(o[q][t] * rn[q]), uv = __shfl_xor(gv, 32, 64);
+        x[t] = silu_round<DT>(gv) * uv;
+      }
+      if (f >= F || row >= P.M || g >= 2) continue;
+      uint16_t* cp = (uint16_t*)P.c + (int64_t)row * P.ldc + (n0 >> 1) + 4 * g;
+      *(uint2*)cp = uint2{gpack<DT>(x[0], x[1]), gpack<DT>(x[2], x[3])};
+    }
+  } else if constexpr (EPI == 1) {
+    if constexpr (FW % 2 == 0) {
+#pragma unroll
+      for (int q = 0; q < FW; q += 2) {
+        const int f = f_of[q], row = m0 + 16 * (f / FN) + r, n = n0 + 16 * (f % FN);
+        if (row >= P.M || n >= P.N) continue;
+        float x[4];
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+          const float gv = ground<DT>(o[q][t] * rn[q]), uv = ground<DT>(o[q + 1][t] * rn[q]);
+          x[t] = silu_round<DT>(gv) * uv;
+        }
+        uint16_t* cp = (uint16_t*)P.c + (int64_t)row * P.ldc + (n >> 1) + 4 * g;
+        *(uint2*)cp = uint2{gpack<DT>(x[0], x[1]), gpack<DT>(x[2], x[3])};
+      }
+    } else {                                               // one fragment per wave: the even ones take their pair's other half
+      static_assert(FW == 1, "");
+      const int f = f_of[0], row = m0 + 16 * (f / FN) + r, n = n0 + 16 * (f % FN);
+      if (f >= F || f % 2 || row >= P.M || n >= P.N) return;
+      gf4 u = *part(0, f + 1);
+#pragma unroll
+      for (int w = 1; w < NW; w++) u += *part(w, f + 1);
+      float x[4];
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        const float gv = ground<DT>(o[0][t] * rn[0]), uv = ground<DT>(u[t] * rn[0]);
+        x[t] = silu_round<DT>(gv) * uv;
+      }
+      uint16_t* cp = (uint16_t*)P.c + (int64_t)row * P.ldc + (n >> 1) + 4 * g;
+      *(uint2*)cp = uint2{gpack<DT>(x[0], x[1]), gpack<DT>(x[2], x[3])};
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < FW; q++) {
+      const int f = f_of[q], row = m0 + 16 * (f / FN) + r, n = n0 + 16 * (f % FN);
+      if (f >= F || row >= P.M || n >= P.N) continue;
+      float x[4];
+#pragma unroll
+      for (int t = 0; t < 4; t++) x[t] = o[q][t] * rn[q];
+      if (EPI == 2) {
+        float y[4];
+        if (DT == UVMI_BF16) {
+          y[0] = __uint_as_float(res[q].x << 16); y[1] = __uint_as_float(res[q].x & 0xffff0000u);
+          y[2] = __uint_as_float(res[q].y << 16); y[3] = __uint_as_float(res[q].y & 0xffff0000u);
+        } else {
+          y[0] = half_bits_to_float((uint16_t)(res[q].x & 0xffff)); y[1] = half_bits_to_float((uint16_t)(res[q].x >> 16));
+          y[2] = half_bits_to_float((uint16_t)(res[q].y & 0xffff)); y[3] = half_bits_to_float((uint16_t)(res[q].y >> 16));
+        }
+#pragma unroll
+        for (int t = 0; t < 4; t++) x[t] = P.ca * y[t] + P.cb * ground<DT>(x[t]);
+      }
+      uint16_t* cp = (uint16_t*)P.c + (int64_t)row * P.ldc + n + 4 * g;
+      *(uint2*)cp = uint2{gpack<DT>(x[0], x[1]), gpack<DT>(x[2], x[3])};
+    }
+  }
+}
+
+template <int DT, int BM, int BN, int NW, int R>
+static void launch_stream(const uvmi_gemm_args* a, StreamParams& P, hipStream_t st) {
+  P.tiles_m = (int)((a->M + BM - 1) / BM);
+  P.tiles_n = (a->N + BN - 1) / BN;
+  const int T = P.tiles_m * P.tiles_n;
+  const dim3 grid((unsigned)(((T + 7) / 8) * 8)), blk(64 * NW);
+#define UVMI_GO(EPI, NORM) hipLaunchKernelGGL((gemm_stream_kernel<DT, BM, BN, NW, R, EPI, NORM>), grid, blk, 0, st, P.a, P.w, P.lda2, P.ldw2, P.M, P.N, P.K, P.tiles_m, P.tiles_n, P.rowsplit, P.r, P.c, P.ldc, P.ldr, P.eps, P.ca, P.cb)
+  const bool norm = a->norm_a != 0;
+  if (a->epilogue == UVMI_GEMM_RESID) { if (norm) UVMI_GO(2, true); else UVMI_GO(2, false); }
+  else if (a->epilogue == UVMI_GEMM_SWIGLU) {
+    if (norm) UVMI_GO(1, true); else UVMI_GO(1, false);
+  } else { if (norm) UVMI_GO(0, true); else UVMI_GO(0, false); }
+#undef UVMI_GO
+}
+
+// The tiles, from the smallest: (BM, BN, NW, R).  LDS: 64, 48, 64, 96 / 48, 64 KB.  The smallest tile takes 8 waves (K of 512 or
+// 640: one or two slabs each, all in flight at once).
+template <int DT>
+static void launch_form(const uvmi_gemm_args* a, int form, bool single_round, StreamParams& P, hipStream_t st) {
+  switch (form) {
+    case 0: launch_stream<DT, 16, 16, 8, 2>(a, P, st); break;
+    case 1: launch_stream<DT, 16, 32, 4, 2>(a, P, st); break;
+    case 2: launch_stream<DT, 32, 32, 4, 2>(a, P, st); break;
+    case 3:   // two slabs per wave ahead where a compute unit has one workgroup; else one, and three workgroups fit (384 rows, N 3328: 7.3 against 11.3 us)
+      if (single_round) launch_stream<DT, 32, 64, 4, 2>(a, P, st);
+      else launch_stream<DT, 32, 64, 4, 1>(a, P, st);
+      break;
+    default: launch_stream<DT, 64, 64, 4, 1>(a, P, st); break;
+  }
+}
+
+static int64_t stream_tiles(const uvmi_gemm_args* a, int form) {
+  static const int bm[5] = {16, 16, 32, 32, 64}, bn[5] = {16, 32, 32, 64, 64};
+  return ((a->M + bm[form] - 1) / bm[form]) * ((a->N + bn[form] - 1) / bn[form]);
+}
+
+// The smallest tile that leaves a compute unit about one workgroup: smaller ones re-read the operands more often, larger ones
+// leave compute units idle and a longer chain of slabs per wave (640 columns, K 1664, 128 rows: 16 x 16 4.0 us, 16 x 32 3.7, 32 x 32
+// 4.5; 512 rows: 16 x 32 6.7, 32 x 32 6.8, 32 x 64 5.9, 64 x 64 7.9).  A short K ends before a second workgroup on the unit
+// hurts: 7 / 4 per unit up to K = 768 (640 columns, K 512, 256 rows: 16 x 32, 320 tiles, 3.0 us; 32 x 32, 160 tiles, 3.1).
+// -1: more than that even of 64 x 64 tiles.
+int gemm_stream_form(const uvmi_gemm_args* a, int cus) {
+  const int64_t most = a->K <= 768 ? (int64_t)cus * 7 / 4 : cus;
+  for (int f = 0; f < 5; f++)
+    if (stream_tiles(a, f) <= most) return f;
+  return -1;
+}
+
+// Arguments are validated by the caller (uvmi_gemm_tn_ex).
+void gemm_stream_launch(const uvmi_gemm_args* a, int form, int cus, hipStream_t st) {
+  StreamParams P;
+  P.a = a->a; P.w = a->w; P.c = a->c; P.r = a->resid;
+  P.lda2 = (uint32_t)a->lda * 2; P.ldw2 = (uint32_t)a->ldw * 2; P.ldc = a->ldc; P.ldr = a->ldr;
+  P.M = (int)a->M; P.N = a->N; P.K = a->K;
+  P.eps = a->eps; P.ca = a->ca; P.cb = a->cb;
+  // tiles are dealt to the XCDs in contiguous runs, by row blocks or by weight strips, whichever leaves the smaller working set
+  // per XCD (an eighth of A plus all of W, or all of A plus an eighth of W)
+  const double bytes_a = (double)a->M * a->K, bytes_w = (double)a->N * a->K;
+  P.rowsplit = bytes_a / 8 + bytes_w < bytes_a + bytes_w / 8;
+  const bool single_round = stream_tiles(a, form) <= cus;
+  if (a->dtype == UVMI_F16) launch_form<UVMI_F16>(a, form, single_round, P, st);
+  else launch_form<UVMI_BF16>(a, form, single_round, P, st);
+}
+
+}  // namespace uvmi

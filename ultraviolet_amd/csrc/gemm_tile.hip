@@ -1,12 +1,12 @@
-// Tiled 16-bit GEMM for the projections of a large decode step (several hundred to a few thousand rows):
-// C[M, N] = A[M, K] . W[N, K]^T with fp32 accumulation and the epilogues of the skinny kernel (gemm.hip) - SwiGLU on
-// interleaved gate / up slabs, the block's residual update, the RMS pre-norm as a row scale.  These are the F.linear calls
-// of the reference's fused inference path (ultraviolet/model.py:302-335, 388-391) with what surrounds them (:566-571).
+// Tiled 16-bit GEMM for many rows whose outputs (or residuals) are not aligned for the 16-byte stores of the direct-to-LDS form
+// (gemm_big.hip): C[M, N] = A[M, K] . W[N, K]^T with fp32 accumulation and the epilogues of the streaming kernel
+// (gemm_stream.hip) - SwiGLU on interleaved gate / up slabs, the block's residual update, the RMS pre-norm as a row scale.
+// These are the F.linear calls of the reference's fused inference path (ultraviolet/model.py:302-335, 388-391) with what
+// surrounds them (:566-571).
 //
 // At this size a projection is a contraction of 1 - 9 GFLOP whose operands (a few MB) live in the L2 / last-level cache:
 // the kernel is bound by how fast a compute unit can feed its matrix cores from LDS.
-//   * a workgroup of 4 waves (2 x 2) owns a BM x BN tile (128 x 128, or 64 x 64 when the larger tile would leave compute
-//     units idle); K is walked in slabs of 64;
+//   * a workgroup of 4 waves (2 x 2) owns a BM x BN tile (128 x 128); K is walked in slabs of 64;
 //   * a slab of A and of W is fetched by 16-byte buffer loads (8 consecutive lanes on one 128-byte row segment) into
 //     registers while the previous slab is multiplied, then parked in the other half of a double-buffered LDS tile: one
 //     barrier per slab;
@@ -242,20 +242,18 @@ static void launch_tile(const uvmi_gemm_args* a, const TileParams& P, hipStream_
 #undef UVMI_GO
 }
 
-// Arguments are validated by the caller (uvmi_gemm_tn_ex).  big: 128 x 128 tiles with two slabs in flight, else 64 x 64 with four.
-void gemm_tile_launch(const uvmi_gemm_args* a, bool big, hipStream_t st) {
+// Arguments are validated by the caller (uvmi_gemm_tn_ex).
+void gemm_tile_launch(const uvmi_gemm_args* a, hipStream_t st) {
   TileParams P;
   P.a = a->a; P.w = a->w; P.c = a->c; P.r = a->resid;
   P.lda2 = (uint32_t)a->lda * 2; P.ldw2 = (uint32_t)a->ldw * 2; P.ldc = a->ldc; P.ldr = a->ldr;
   P.M = (int)a->M; P.N = a->N; P.K = a->K;
-  const int bm = big ? 128 : 64;
-  P.tiles_m = (int)((a->M + bm - 1) / bm);
-  P.tiles_n = (a->N + bm - 1) / bm;
+  P.tiles_m = (int)((a->M + 127) / 128);
+  P.tiles_n = (a->N + 127) / 128;
   P.eps = a->eps; P.ca = a->ca; P.cb = a->cb;
   const double bytes_a = (double)a->M * a->K, bytes_w = (double)a->N * a->K;
   P.rowsplit = bytes_a / 8 + bytes_w < bytes_a + bytes_w / 8;
-  if (a->dtype == UVMI_F16) { if (big) launch_tile<UVMI_F16, 128, 128, 2>(a, P, st); else launch_tile<UVMI_F16, 64, 64, 4>(a, P, st); }
-  else { if (big) launch_tile<UVMI_BF16, 128, 128, 2>(a, P, st); else launch_tile<UVMI_BF16, 64, 64, 4>(a, P, st); }
+  if (a->dtype == UVMI_F16) launch_tile<UVMI_F16, 128, 128, 2>(a, P, st); else launch_tile<UVMI_BF16, 128, 128, 2>(a, P, st);
 }
 
 }  // namespace uvmi

@@ -93,18 +93,18 @@ def rms_norm_eps(dtype: torch.dtype) -> float:
 class UVEngine:
     def __init__(self, weights: UVWeights, max_tokens: int, skinny_rows: int = 192, fold_qkv_rows: int = 1 << 30, fold_o_rows: int = 1 << 30,
                  fold_gu_rows: int = 1 << 30, lean: bool = True, fold: bool = True, gemm_config: int = 0,
-                 tiled_prefill: bool = True, big_rows: int = 12288, fold_down_rows: tuple = (800, 1632), general_skinny_rows: int = 384):
+                 tiled_prefill: bool = True, big_rows: int = 12288, fold_down_rows: tuple = (0, 5120), general_skinny_rows: int = 384):
         """max_tokens: largest number of token rows one forward call processes (decode rows + packed prefill tokens).
-        skinny_rows: decode passes of at most this many rows run every projection on the skinny GEMM (general_skinny_rows:
-        the same for passes of the general path); fold_qkv_rows, fold_o_rows,
+        skinny_rows: decode passes of at most this many rows run every projection on this library's GEMM, the residual updates out of
+        place (general_skinny_rows: the same for passes of the plain path); fold_qkv_rows, fold_o_rows,
         fold_gu_rows: above skinny_rows, row counts up to which the QKV projection (with the pre-norm), the output
         projection (with the residual update) and the gate-up projection (with the pre-norm and the SwiGLU) run on this
         library's GEMM kernels instead of the vendor library's (see _trunk_folded); lean / fold: the launch plans that drop
         the residual-add and norm launches (off: the general path); gemm_config: form of the hand-written GEMM (0: its own
         choice by size; tests force the tiled forms at a few rows); big_rows: passes of the general path with at least this
         many rows (a packed prefill, a mixed pass) run the down projection too on this library's GEMM, whose 256 x 256 tile
-        form is faster than the vendor library there (the other three projections run on it from 448 rows); fold_down_rows:
-        (first, last) row count of decode passes whose down projection runs on this library's tiled GEMM.  The defaults are the measured
+        form is as fast as the vendor library there; fold_down_rows: (first, last) row count of passes whose down projection runs
+        on this library's GEMM.  The defaults are the measured
         optimum on UV-50M."""
         self.w, self.cfg = weights, weights.cfg
         cfg, dt, dev = self.cfg, weights.dtype, weights.device
@@ -124,23 +124,20 @@ class UVEngine:
         # post-processing to the attention kernel (one launch less per layer)
         self.fuse_qkv = dt in (torch.bfloat16, torch.float16) and cfg.n_heads // cfg.n_kv_heads <= 8 and cfg.n_pairs in (0, 16)
         self.qkvx_keep = None
-        # Passes of at most this many rows run every projection on the skinny GEMM (the down projection with the block's
-        # second residual update in its epilogue); above it the folded plan (tiled GEMMs, the vendor library for the down
-        # projection).  Measured on UV-50M decode steps inside a rollout: 0.369 against 0.388 ms at 192 rows, 0.424 against
-        # 0.415 at 256, 0.466 against 0.460 at 320, equal at 384.
+        # Decode passes of at most this many rows keep the block's two hiddens apart (h and x); above it the folded plan updates
+        # one in place.
         self.skinny_rows = int(skinny_rows) if dt in (torch.bfloat16, torch.float16) else 0
-        # passes of the general path (prefill, mixed steps, layers without the fused attention) keep the skinny GEMM up to
-        # this many rows: their alternative below 448 rows is the vendor library with separate SwiGLU and norm launches
+        # passes of the plain path run on this library's GEMM up to this many rows: their alternative is the vendor library with
+        # separate SwiGLU and norm launches
         self.general_skinny_rows = int(general_skinny_rows) if dt in (torch.bfloat16, torch.float16) else 0
-        # above skinny_rows the skinny kernel still carries the QKV projection (with the pre-norm) and the output projection
-        # (with the residual update) up to these many rows
+        # above skinny_rows: row counts up to which the QKV, output and gate-up projections run on this library's GEMM
         self.fold_qkv_rows = int(fold_qkv_rows)
         self.fold_o_rows, self.fold_gu_rows = int(fold_o_rows), int(fold_gu_rows)
         self.lean, self.fold, self.gemm_config = bool(lean), bool(fold), int(gemm_config)
         self.tiled_prefill = bool(tiled_prefill)
         self.big_rows = int(big_rows)
-        # the folded plan's down projection runs on this library's tiled GEMM between these row counts (measured inside the
-        # decode step: 4 - 11 us per step faster than the vendor library's there, slower below and above)
+        # the down projection runs on this library's GEMM between these row counts (per launch 5.9 against the vendor library's
+        # 8.5 us at 512 rows, 13.5 against 14.2 at 3072, 19.3 against 19.9 at 4608, 21.6 against 19.3 at 6144)
         self.fold_down_rows = (int(fold_down_rows[0]), int(fold_down_rows[1]))
         self.head_own_rows = 288       # decode steps of at most this many rows run the head GEMM on this library's kernel (own_head_ok)
         self.hidden_is_raw = False
@@ -426,8 +423,8 @@ class UVEngine:
         il = all("gu_il" in W for W in self.w.layers)
         div = cfg.d_model % 64 == 0 and (cfg.n_heads * cfg.head_dim) % 64 == 0
         if fused and ok16 and all(self.fused_layer_ok(l, st) for l in range(cfg.n_layers)):
-            skinny = n <= self.skinny_rows and div and cfg.d_model <= 960
-            if skinny and self.lean and il and cfg.d_ff % 64 == 0 and cfg.d_ff <= 1984:
+            skinny = n <= self.skinny_rows and div
+            if skinny and self.lean and il and cfg.d_ff % 64 == 0:
                 return "lean"
             if self.fold and not skinny and cfg.d_ff % 8 == 0:
                 return "folded"
@@ -453,7 +450,7 @@ class UVEngine:
             self._gemm(b["x"][:n], W["wqkv_ext"], b["qkvx"][:n], norm_eps=self.eps, **kw)
 
     def _layers_lean(self, n: int, fused_attn):
-        """Decode passes of few rows: every projection on the skinny GEMM, the residual updates in the epilogues of the output
+        """Decode passes of few rows: every projection on this library's GEMM, the residual updates in the epilogues of the output
         and down projections, both pre-norms as row scales of the products that read them.  Five launches per layer."""
         b = self.buf
         x, h, zg, act = b["x"][:n], b["h"][:n], b["zg"][:n], b["act"][:n]
@@ -469,8 +466,7 @@ class UVEngine:
         """Decode passes of many rows, five launches per layer: QKV projection with the block's pre-norm as a row scale, fused
         attention, output projection with the residual update in place, gate-up projection with the MLP's pre-norm and the
         SwiGLU in its epilogue (the (n, 2 f) intermediate and the normalised hidden are never written), down projection with the
-        residual update (the vendor library's C = alpha A B + beta C outside fold_down_rows: at K = d_ff it is still the
-        faster kernel there)."""
+        residual update (the vendor library's C = alpha A B + beta C outside fold_down_rows)."""
         cfg, b = self.cfg, self.buf
         x, zg, act = b["x"][:n], b["zg"][:n], b["act"][:n]
         gc = self.gemm_config
@@ -526,7 +522,7 @@ class UVEngine:
             self._down(l, n, own_down)
 
     def _layers_plain(self, n: int, tok, pos, rows, last_pos, st, attn, fused_attn) -> bool:
-        """The reference's order of operations on the vendor library's GEMMs (16-bit passes of few rows: on the skinny GEMM),
+        """The reference's order of operations on the vendor library's GEMMs (16-bit passes of few rows: on this one's),
         one launch per step between them: fp32 engines, widths the other plans do not take.  Returns whether buf x was
         left un-normalised (else buf xn holds the final norm)."""
         cfg, b = self.cfg, self.buf

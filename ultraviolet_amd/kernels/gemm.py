@@ -45,8 +45,7 @@ def gemm_tn(a: Tensor, w: Tensor, out: Tensor | None = None, epilogue: int = STO
     block's residual update, ultraviolet/model.py:567-571); with epilogue=SOFTCAP it is ca * sigmoid((x + cb) / cap_c) in fp32
     of the rounded product x (the logits, model.py:824-827).  norm_eps: a stands for rmsnorm(a) with that epsilon (the
     pre-norm of the block folded into the projection as a row scale of the product).  Raises UvmiError for shapes the
-    kernel does not take.  config (tuning / tests): 0 built-in choice, 1 the 64-row workgroup form, 2 the 16-row form whose
-    waves split K."""
+    kernel does not take.  config (tuning / tests): 0 built-in choice, else a form of the kernel (uvmi_gemm_args.config)."""
     if out is None:
         out = torch.empty(a.size(0), w.size(0) // 2 if epilogue == SWIGLU else w.size(0), dtype=torch.float32 if epilogue == SOFTCAP else a.dtype, device=a.device)
     g = gemm_args(a, w, out, epilogue, norm_eps=norm_eps, resid=resid, ca=ca, cb=cb, cap_c=cap_c, config=config)
