@@ -1,0 +1,60 @@
+"""Which calls of decode_attention may launch past the dispatcher: those that no transform, mode, tracer or gradient sees.
+No GPU: the launch and the registered op are replaced by recorders."""
+import pytest
+import torch
+from torch.utils._python_dispatch import TorchDispatchMode
+
+from ultraviolet_amd.kernels import decode_attn as D
+
+
+class _Passing(TorchDispatchMode):
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+class _Subclass(torch.Tensor):
+    pass
+
+
+@pytest.fixture
+def route(monkeypatch):
+    """call(q, k, v) -> "launch" or "op"."""
+    taken = []
+    monkeypatch.setattr(D.L, "require_cuda", lambda *t: None)
+    monkeypatch.setattr(D, "_launch", lambda q, *a, **k: taken.append("launch") or torch.zeros_like(q))
+    monkeypatch.setattr(D, "_decode_attn_op", lambda q, *a, **k: taken.append("op") or torch.zeros_like(q))
+    idx = torch.zeros(2, dtype=torch.long)
+
+    def call(q, k, v):
+        D.decode_attention(q, k, v, idx, idx, 0.1, num_splits=1)
+        return taken.pop()
+    return call
+
+
+def _qkv():
+    return torch.randn(2, 8, 64).half(), torch.randn(2, 1, 32, 64).half(), torch.randn(2, 1, 32, 64).half()
+
+
+def test_plain_call_launches(route):
+    assert route(*_qkv()) == "launch"
+
+
+@pytest.mark.parametrize("which", [0, 1, 2])
+def test_gradient_and_subclass_of_any_operand_reach_the_op(route, which):
+    t = list(_qkv())
+    t[which] = t[which].clone().requires_grad_()
+    assert route(*t) == "op"
+    t = list(_qkv())
+    t[which] = t[which].as_subclass(_Subclass)
+    assert route(*t) == "op"
+
+
+def test_modes_and_transforms_reach_the_op(route):
+    with _Passing():
+        assert route(*_qkv()) == "op"
+    with torch.autograd.forward_ad.dual_level():
+        assert route(*_qkv()) == "op"
+    seen = []
+    q, k, v = _qkv()
+    torch.func.vmap(lambda a: (seen.append(route(a, k, v)), a)[1])(q[None])
+    assert seen == ["op"]

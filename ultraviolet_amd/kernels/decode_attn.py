@@ -10,6 +10,7 @@ import functools
 
 import torch
 from torch import Tensor
+from torch.autograd import forward_ad
 
 from .. import _lib as L
 
@@ -22,6 +23,15 @@ def _device_cus(index: int) -> int:
     if cus <= 0:
         raise L.UvmiError(L.lib().uvmi_last_error().decode())
     return cus
+
+
+def plain_eager(*tensors: Tensor | None) -> bool:
+    """Whether a call on these tensors is seen by nothing but the caller, so that it may launch without the dispatcher: plain
+    tensors that record no gradient, no compile or trace, no functorch transform (vmap, jvp, grad), no dispatch or function
+    mode (fake tensors, proxies, counters), no forward-mode level."""
+    return (all(t is None or (type(t) is Tensor and not t.requires_grad) for t in tensors) and not torch.compiler.is_compiling()
+            and not torch.jit.is_tracing() and torch._C._functorch.peek_interpreter_stack() is None and torch._C._len_torch_dispatch_stack() == 0
+            and torch._C._len_torch_function_stack() == 0 and forward_ad._current_level < 0)
 
 
 def default_splits(n_bk: int, ctx: int, device=None, min_chunk: int = 256, waves: int = 1) -> int:
@@ -183,7 +193,7 @@ def decode_attention(q: Tensor, k_cache: Tensor, v_cache: Tensor, pos: Tensor, s
     if pos.dtype != starts.dtype:
         starts = starts.to(pos.dtype)
     pos, starts = pos.contiguous(), starts.contiguous()
-    if type(q) is Tensor and not q.requires_grad and not torch.compiler.is_compiling():
+    if plain_eager(q, k_cache, v_cache, pos, starts, k_scale, v_scale, rows):
         # eager calls on plain tensors launch directly: the dispatcher's round trip through the registered op costs more host
         # time than the launch (23 us a call against an 8 us kernel on 256 rows of up to 1024 keys)
         out = torch.empty(q.shape, device=q.device, dtype=torch.float32 if out_fp32 else q.dtype)
