@@ -726,6 +726,9 @@ def test_recorded_passes_rebind_to_other_calls(kv_dtype):
         if round_ == 2:
             eng.w.load_(random_params(cfg, 9, perturb=0.06))       # other residual scalars: launch arguments of the list
             old.k[1] = old.k[1].clone()
+            gone = old.v[0].data
+            old.v[0].data = gone.clone()                           # the same object elsewhere
+            gone.fill_(1)
         prompts = _prompts(cfg, rng.integers(1, 30, size=(5, 40, 61)[round_]), seed=round_)
         rows = rng.permutation(B)[:len(prompts)].tolist()
         outs = [eng.prefill(prompts, rows, st).clone() for st in (old, new)]

@@ -578,10 +578,12 @@ class UVEngine:
         own_down = n <= self.skinny_rows or n >= self.big_rows or self.fold_down_rows[0] <= n <= self.fold_down_rows[1]
         key = (id(self), what, kind, n <= self.fold_qkv_rows, n <= self.fold_o_rows, n <= self.fold_gu_rows, own_down,
                self.fold_down_rows[0] <= n <= self.fold_down_rows[1], self.gemm_config, getattr(self.w, "scalar_epoch", 0))
-        guard = (self.w, *st.k, *st.v, *st.k_scale, *st.v_scale)
+        caches = [t for t in (*st.k, *st.v, *st.k_scale, *st.v_scale) if t is not None]
+        guard = (self.w, *caches)
         plans = st.__dict__.setdefault("_pass_plans", {})
         plan = plans.get(key)
-        if plan is None or len(plan.guard) != len(guard) or any(a is not b for a, b in zip(plan.guard, guard)):
+        at = tuple(map(Tensor.data_ptr, caches))   # (a cache may keep its object and move, as with `.data = `)
+        if plan is None or len(plan.guard) != len(guard) or any(a is not b for a, b in zip(plan.guard, guard)) or plan.at != at:
             if len(plans) >= 16:
                 plans.clear()
             plan = PassPlan()
@@ -590,7 +592,7 @@ class UVEngine:
                 record()
             finally:
                 self._rec = None
-            plan.guard = guard
+            plan.guard, plan.at = guard, at
             plan.engine = self          # (keeps id(self) from being reused while the plan lives)
             plan.raw = self.hidden_is_raw
             plans[key] = plan.close()
@@ -657,7 +659,9 @@ class UVEngine:
             fused = lambda l: self.fused_cache_attention(l, tok, st, pos, starts, B)
             kind = self._pass_kind(B, True, st)
             if kind in ("lean", "folded") and self.qkvx_keep is None:
-                assert B <= self.max_tokens and B <= st.B and tok.dtype == torch.int64 and tok.is_contiguous()
+                assert B <= self.max_tokens and B <= st.B
+                # (a recorded list takes addresses only, so what its launches assume of the arrays is checked on every call)
+                assert all(t.dtype == torch.int64 and t.is_contiguous() and t.numel() >= B for t in (tok, pos, starts))
                 whole = B == pos.numel()     # (a step of fewer rows than the state has still moves every position)
                 h = self._planned("decode" if whole else "decode-part", st, kind, B,
                                   dict(n=B, tok=tok.data_ptr(), pos=pos.data_ptr(), starts=starts.data_ptr()),

@@ -18,6 +18,7 @@ class PassPlan:
         self.fields = {}    # name of a per-call value -> [(struct, field)] that hold it
         self.bound = {}     # the values they hold now
         self.guard = ()     # objects whose identity the recorded addresses rest on
+        self.at = ()        # the addresses of those that a caller could move
 
     def op(self, kind: int, args, keep=(), **per_call):
         """A launch; per_call: field of args (or (struct, field)) = name of the per-call value it holds."""
