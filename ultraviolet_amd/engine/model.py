@@ -90,6 +90,23 @@ def rms_norm_eps(dtype: torch.dtype) -> float:
     return cands[int(np.argmin([abs(y - r) for r in refs]))]
 
 
+class _Stage:
+    """A pinned host buffer that launches read in place, and the event behind the last of them.  The allocator does not know
+    of such readers, so the buffer waits for them before it goes."""
+
+    buf = event = None
+
+    def wait(self):
+        if self.event is not None:
+            self.event.synchronize()
+
+    def __del__(self):
+        try:
+            self.wait()
+        except Exception:   # the runtime is already gone (interpreter exit)
+            pass
+
+
 class UVEngine:
     def __init__(self, weights: UVWeights, max_tokens: int, skinny_rows: int = 192, fold_qkv_rows: int = 1 << 30, fold_o_rows: int = 1 << 30,
                  fold_gu_rows: int = 1 << 30, lean: bool = True, fold: bool = True, gemm_config: int = 0,
@@ -141,7 +158,7 @@ class UVEngine:
         self.fold_down_rows = (int(fold_down_rows[0]), int(fold_down_rows[1]))
         self.head_own_rows = 288       # decode steps of at most this many rows run the head GEMM on this library's kernel (own_head_ok)
         self.hidden_is_raw = False
-        self._stage, self._stage_at = [(None, None)] * 2, 0   # pinned tables and the events of the launches that read them (_staging)
+        self._stage, self._stage_at = [_Stage() for _ in range(2)], 0   # (_staging)
         self._rec = None               # the PassPlan being recorded (None: operations are launched as they come)
         self._rope_tabs: dict[int, Tensor] = {}  # rotation tables by position count, kept for the engine's life (graphs hold them)
         if self.fuse_qkv:
@@ -685,15 +702,13 @@ class UVEngine:
     # ------------------------------------------------------------------------------------------------ prefill
     def _staging(self, n: int):
         """n int64 of pinned host memory out of a small ring, and the event to record behind the launch that reads it: a buffer
-        is handed out again only after that launch."""
+        is handed out again, or given back to the allocator, only after that launch."""
         self._stage_at = (self._stage_at + 1) % len(self._stage)
-        buf, ev = self._stage[self._stage_at]
-        if ev is not None:
-            ev.synchronize()
-        if buf is None or buf.numel() < n:
-            buf, ev = torch.empty(max(1024, n + n // 4), dtype=torch.int64, pin_memory=True), torch.cuda.Event()
-            self._stage[self._stage_at] = (buf, ev)
-        return buf, ev
+        st = self._stage[self._stage_at]
+        st.wait()
+        if st.buf is None or st.buf.numel() < n:
+            st.buf, st.event = torch.empty(max(1024, n + n // 4), dtype=torch.int64, pin_memory=True), torch.cuda.Event()
+        return st.buf, st.event
 
     def _pack(self, prompts, rows, max_len: int, left_pad: bool, st: KVState | None = None, idx: Tensor | None = None, lens=None,
               check: Tensor | None = None) -> dict:
@@ -743,7 +758,7 @@ class UVEngine:
                 return h[3 * n + 1:4 * n + 1].copy()
             pk["check"] = seen
         L.check(L.lib().uvmi_prompt_tables(C.byref(a), L.stream_ptr(out)), "uvmi_prompt_tables")
-        ev.record()
+        ev.record(torch.cuda.current_stream(self.device))
         return pk
 
     @staticmethod
