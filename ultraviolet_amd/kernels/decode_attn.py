@@ -25,13 +25,27 @@ def _device_cus(index: int) -> int:
     return cus
 
 
-def plain_eager(*tensors: Tensor | None) -> bool:
-    """Whether a call on these tensors is seen by nothing but the caller, so that it may launch without the dispatcher: plain
+def _key_sets() -> frozenset:
+    """Dispatch keys that a thread has switched on outside every mode, transform and trace: with and without inference mode."""
+    keys = torch._C.DispatchKeySet(torch._C.DispatchKey.BackendSelect)
+    return frozenset((keys.raw_repr(), keys.add(torch._C.DispatchKey.ADInplaceOrView).raw_repr()))
+
+
+_PLAIN_KEYS = _key_sets()
+
+
+def plain_eager(q: Tensor, k: Tensor, v: Tensor, k_scale: Tensor | None, v_scale: Tensor | None) -> bool:
+    """Whether a call on these operands is seen by nothing but the caller, so that it may launch without the dispatcher: plain
     tensors that record no gradient, no compile or trace, no functorch transform (vmap, jvp, grad), no dispatch or function
-    mode (fake tensors, proxies, counters), no forward-mode level."""
-    return (all(t is None or (type(t) is Tensor and not t.requires_grad) for t in tensors) and not torch.compiler.is_compiling()
-            and not torch.jit.is_tracing() and torch._C._functorch.peek_interpreter_stack() is None and torch._C._len_torch_dispatch_stack() == 0
-            and torch._C._len_torch_function_stack() == 0 and forward_ad._current_level < 0)
+    mode (fake tensors, proxies, counters), no forward-mode level.  (Modes, transforms and traces switch dispatch keys on.)"""
+    if (torch.compiler.is_compiling() or torch._C._dispatch_tls_local_include_set().raw_repr() not in _PLAIN_KEYS
+            or torch._C._len_torch_function_stack() or forward_ad._current_level >= 0):
+        return False
+    if type(q) is not Tensor or type(k) is not Tensor or type(v) is not Tensor or q.requires_grad:
+        return False
+    if k_scale is None or v_scale is None:
+        return not (k.requires_grad or v.requires_grad)
+    return type(k_scale) is Tensor and type(v_scale) is Tensor and not (k_scale.requires_grad or v_scale.requires_grad or k.requires_grad or v.requires_grad)
 
 
 def default_splits(n_bk: int, ctx: int, device=None, min_chunk: int = 256, waves: int = 1) -> int:
@@ -193,7 +207,7 @@ def decode_attention(q: Tensor, k_cache: Tensor, v_cache: Tensor, pos: Tensor, s
     if pos.dtype != starts.dtype:
         starts = starts.to(pos.dtype)
     pos, starts = pos.contiguous(), starts.contiguous()
-    if plain_eager(q, k_cache, v_cache, pos, starts, k_scale, v_scale, rows):
+    if plain_eager(q, k_cache, v_cache, k_scale, v_scale):
         # eager calls on plain tensors launch directly: the dispatcher's round trip through the registered op costs more host
         # time than the launch (23 us a call against an 8 us kernel on 256 rows of up to 1024 keys)
         out = torch.empty(q.shape, device=q.device, dtype=torch.float32 if out_fp32 else q.dtype)
