@@ -74,6 +74,20 @@ def test_few_and_many_rows_on_long_caches(dtype, B, S, ring):
     _attn_check(q, k, v, ks, vs, pos, starts, 1.13 / 8, window=S if ring else 0, ring=ring)
 
 
+@pytest.mark.parametrize("KH,B,S,ring", [(1, 256, 512, False), (1, 257, 512, False), (2, 128, 544, True), (8, 5, 512, False), (1, 7, 32, False),
+                                         (1, 256, 64, True), (1, 257, 64, False), (4, 64, 160, False)])
+def test_waves_per_row_at_the_edges_of_their_rule(KH, B, S, ring):
+    """One item per compute unit and one more, caches of 512 slots and less: rows whose last tile is each wave's first, second and
+    none, and rows that end one key before and after a tile of the last wave."""
+    q, k, v, ks, vs = attn_case(B, KH, 8 // KH, 64, S, True, dtype=torch.bfloat16)
+    g = torch.Generator().manual_seed(B + S)
+    pos = torch.randint(0, S if not ring else 3 * S, (B,), generator=g)
+    edges = [p for p in (0, 30, 31, 32, 127, 128, 223, 224, 255, 256, 257, 480, S - 1) if p < S][:B]
+    pos[:len(edges)] = torch.tensor(edges)
+    starts = torch.where(torch.arange(B) % 3 == 2, pos // 2, torch.zeros_like(pos))
+    _attn_check(q, k, v, ks, vs, pos, starts, 1.13 / 8, window=S if ring else 0, ring=ring, splits=1)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("B,S,ring,G", [(3, 1056, False, 8), (200, 1056, False, 8), (300, 2080, False, 4), (40, 1024, True, 8), (64, 256, True, 2),
                                         (50, 100, False, 8)])

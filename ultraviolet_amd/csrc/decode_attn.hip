@@ -180,15 +180,15 @@ struct AttnState {
 // arithmetic: every tile is loaded exactly as in the real kernel and folded into the state with a few xors; 2 - its
 // arithmetic without the stream: tiles are made up in registers, nothing is loaded from the cache.
 template <int QDT, int ODT, int WPR, bool FUSE, bool KV16 = false, bool FAST = false, int PROBE = 0>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4)))
+__global__ __launch_bounds__(WPR > 4 ? 64 * WPR : 256) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_rows, const void* a_q, int64_t a_items, int a_idx64,
                        int a_splits, int a_kh, AttnParams P) {
   P.pos = a_pos; P.starts = a_starts; P.rows = a_rows; P.n_items = a_items; P.idx64 = a_idx64; P.splits = a_splits; P.KH = a_kh;
   if constexpr (FAST) { P.idx64 = 1; P.splits = 1; P.KH = 1; P.G = 8; P.H = 8; P.hd = 64; P.chunk_keys = 0; }
   if (FUSE) P.f_qkv = a_q; else P.q = a_q;
-  constexpr int IPB = 4 / WPR;  // items per block
-  __shared__ __attribute__((aligned(16))) float sh_o[4][16][68];
-  __shared__ __attribute__((aligned(16))) float sh_ml[4][16][4];
+  constexpr int BW = WPR > 4 ? WPR : 4, IPB = BW / WPR;  // waves and items per block
+  __shared__ __attribute__((aligned(16))) float sh_o[BW][16][68];
+  __shared__ __attribute__((aligned(16))) float sh_ml[BW][16][4];
   __shared__ float sh_post[4][80];  // epilogue operands of the item whose first wave this is: v_hat[64], gate[8], xsa[8]
   __shared__ float sh_cur[FUSE ? 4 : 1][72];  // own key of that item: score per head [8], dequantised v [64]
   __shared__ __attribute__((aligned(16))) uint16_t sh_q[FUSE ? 4 : 1][8][64];  // the item's q as fp16 operand words
@@ -810,7 +810,8 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
   if (g == 0) *(float4*)&sh_ml[wave][m][0] = float4{m2, lsum, ps, 0.f};
   if (WPR > 1) __syncthreads(); else __builtin_amdgcn_wave_barrier();
   if (!live) return;
-  constexpr int NV = 8 / WPR, TPH = 64 / NV;       // values per thread, threads per head
+  if (WPR > 4 && wsub >= 4) return;                // (four waves cover the item's 512 outputs, 2 each)
+  constexpr int NV = 8 / (WPR > 4 ? 4 : WPR), TPH = 64 / NV;   // values per thread, threads per head
   const int ti = wsub * 64 + lane;
   const int eh = ti / TPH, d0 = (ti % TPH) * NV;   // head and first dim of this thread
   float mw[2 * WPR], mall = -INFINITY;
@@ -1231,6 +1232,16 @@ static int decode_attn_launch(const uvmi_attn_args* a, void* ws, size_t ws_bytes
       const int64_t slots = (int64_t)cus * 16;
       while (wpr > 1 && P.n_items * wpr > slots && P.n_items * (wpr / 2) <= slots) wpr /= 2;
       if (wpr == 4 && P.n_items * 5 > slots) wpr = 2;
+      // Up to one item per compute unit a launch lasts as long as its longest row: four waves whatever the length (fused, rows of
+      // 8 .. 64 keys, 37 rows: 5.3 us with 4, 5.9 with 1; 16 .. 128 keys: 5.3 with 4, 5.7 with 2), eight from 512 keys on (an
+      // int8 cache, 64 rows of 64 .. 512 keys 6.1 us against 6.5 with 4, 128 .. 1024 7.1 / 7.9, 256 .. 2048 9.2 / 10.6; 256
+      // rows 6.3 / 6.6, 7.7 / 8.3, 10.7 / 11.6; sixteen: 9.8 at 64 rows of 2048).  Above that eight gain nothing (448 rows of
+      // up to 1024 keys 10.1 / 9.9), nor do they on a 16-bit cache, whose waves keep twice the bytes in flight (64 rows of up to
+      // 1024 keys 10.1 / 9.4); of 256 keys a wave has two tiles with four waves already (5.6 / 5.7).
+      if (P.n_items <= cus) {
+        if (wpr < 4) wpr = 4;
+        if (ctx >= 512 && !kv16 && a->num_splits == 1 && !probe) wpr = 8;
+      }
       // Rows of a known, short length - a window or ring of at most 512 keys, 16 tiles - are a chain of latencies rather than
       // a stream: they run fastest with about one wave per SIMD (measured on 256-key rings: 4 waves per row up to ~300 rows,
       // 2 up to ~650, 1 beyond; 500 rows 6.1 us with 2 against 6.9 with 4, 1000 rows 9.5 us with 1 against 9.8 with 2).  With
@@ -1243,27 +1254,31 @@ static int decode_attn_launch(const uvmi_attn_args* a, void* ws, size_t ws_bytes
     }
     P.gran = 32 * wpr;
     if (P.chunk_keys) P.chunk_keys = (P.chunk_keys + P.gran - 1) / P.gran * P.gran;
-    const int ipb = 4 / wpr;
-    const dim3 grid((unsigned)((P.n_items + ipb - 1) / ipb)), blk(256);
+    const int ipb = wpr > 4 ? 1 : 4 / wpr;
+    const dim3 grid((unsigned)((P.n_items + ipb - 1) / ipb)), blk(wpr > 4 ? 64 * wpr : 256);
 #define UVMI_LEAD P.pos, P.starts, P.rows, (a->fuse ? P.f_qkv : P.q), P.n_items, P.idx64, P.splits, P.KH
 #define UVMI_L(QD, OD)                                                                                \
   do {                                                                                                \
-    if (wpr == 4) hipLaunchKernelGGL((attn_mfma_i8_hd64<QD, OD, 4, false>), grid, blk, 0, st, UVMI_LEAD, P);      \
+    if (wpr == 8) hipLaunchKernelGGL((attn_mfma_i8_hd64<QD, OD, 8, false>), grid, blk, 0, st, UVMI_LEAD, P);      \
+    else if (wpr == 4) hipLaunchKernelGGL((attn_mfma_i8_hd64<QD, OD, 4, false>), grid, blk, 0, st, UVMI_LEAD, P);      \
     else if (wpr == 2) hipLaunchKernelGGL((attn_mfma_i8_hd64<QD, OD, 2, false>), grid, blk, 0, st, UVMI_LEAD, P); \
     else hipLaunchKernelGGL((attn_mfma_i8_hd64<QD, OD, 1, false>), grid, blk, 0, st, UVMI_LEAD, P);               \
   } while (0)
 #define UVMI_LF(QD)                                                                                   \
   do {                                                                                                \
-    if (fast && wpr == 4) hipLaunchKernelGGL((attn_mfma_i8_hd64<QD, QD, 4, true, false, true>), grid, blk, 0, st, UVMI_LEAD, P);       \
+    if (fast && wpr == 8) hipLaunchKernelGGL((attn_mfma_i8_hd64<QD, QD, 8, true, false, true>), grid, blk, 0, st, UVMI_LEAD, P);       \
+    else if (fast && wpr == 4) hipLaunchKernelGGL((attn_mfma_i8_hd64<QD, QD, 4, true, false, true>), grid, blk, 0, st, UVMI_LEAD, P);       \
     else if (fast && wpr == 2) hipLaunchKernelGGL((attn_mfma_i8_hd64<QD, QD, 2, true, false, true>), grid, blk, 0, st, UVMI_LEAD, P);  \
     else if (fast) hipLaunchKernelGGL((attn_mfma_i8_hd64<QD, QD, 1, true, false, true>), grid, blk, 0, st, UVMI_LEAD, P);              \
+    else if (wpr == 8) hipLaunchKernelGGL((attn_mfma_i8_hd64<QD, QD, 8, true>), grid, blk, 0, st, UVMI_LEAD, P);  \
     else if (wpr == 4) hipLaunchKernelGGL((attn_mfma_i8_hd64<QD, QD, 4, true>), grid, blk, 0, st, UVMI_LEAD, P);  \
     else if (wpr == 2) hipLaunchKernelGGL((attn_mfma_i8_hd64<QD, QD, 2, true>), grid, blk, 0, st, UVMI_LEAD, P);  \
     else hipLaunchKernelGGL((attn_mfma_i8_hd64<QD, QD, 1, true>), grid, blk, 0, st, UVMI_LEAD, P);                \
   } while (0)
 #define UVMI_LFAST(QD)                                                                                \
   do {                                                                                                \
-    if (wpr == 4) hipLaunchKernelGGL((attn_mfma_i8_hd64<QD, QD, 4, false, false, true>), grid, blk, 0, st, UVMI_LEAD, P);      \
+    if (wpr == 8) hipLaunchKernelGGL((attn_mfma_i8_hd64<QD, QD, 8, false, false, true>), grid, blk, 0, st, UVMI_LEAD, P);      \
+    else if (wpr == 4) hipLaunchKernelGGL((attn_mfma_i8_hd64<QD, QD, 4, false, false, true>), grid, blk, 0, st, UVMI_LEAD, P);      \
     else if (wpr == 2) hipLaunchKernelGGL((attn_mfma_i8_hd64<QD, QD, 2, false, false, true>), grid, blk, 0, st, UVMI_LEAD, P); \
     else hipLaunchKernelGGL((attn_mfma_i8_hd64<QD, QD, 1, false, false, true>), grid, blk, 0, st, UVMI_LEAD, P);               \
   } while (0)
