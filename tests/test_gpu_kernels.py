@@ -963,7 +963,8 @@ def test_attention_probe_runs_the_engine_shape_and_refuses_the_rest():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("M,N,K,norm,config", [(1, 512, 128, False, 0), (130, 1040, 640, True, 6), (257, 2048, 192, False, 5), (300, 32768, 640, True, 0)])
+@pytest.mark.parametrize("M,N,K,norm,config", [(1, 512, 128, False, 0), (130, 1040, 640, True, 6), (257, 2048, 192, False, 5), (300, 32768, 640, True, 0),
+                                               (383, 32768, 128, False, 0), (385, 32768, 192, True, 0), (512, 32768, 128, False, 0), (513, 32768, 128, False, 0)])
 def test_gemm_softcap_epilogue(dtype, M, N, K, norm, config):
     """The head GEMM with the softcap in its epilogue: ca * sigmoid((x + cb) / cap_c) in fp32 of the product rounded to the
     activation type, against float64 (a product that rounds the other way moves the logit by one step of its grid)."""

@@ -54,10 +54,14 @@ extern "C" int uvmi_gemm_tn_ex(const uvmi_gemm_args* a, void* stream) {
                "uvmi_gemm_tn: K = %d is beyond config 1, 2 (1984; 960 with SWIGLU)", a->K);
   if (a->M == 0) return UVMI_OK;
   // (also a product of fewer rows whose 256 x 256 tiles still come to two rounds of the device or more - the tied head,
-  // 2048 x 32768: 104 us against 129 us on 128 x 128 tiles)
+  // 2048 x 32768: 104 us against 129 us on 128 x 128 tiles - or, none of their columns padding, to one full round where 128 x 128
+  // tiles, two to a compute unit, take a second one: 512 x 32768 26.6 us against 29.9, with the softcap 33.7 against 47.7 and
+  // from 384 rows on 28.3 against 35.6; 288 rows 27.9 against 26.4, 384 without the softcap 26.6 against 24.1)
   int cus = uvmi_device_cus();
   if (cus <= 0) cus = 256;
-  const bool many_big_tiles = a->M >= 1024 && ((a->M + 255) / 256) * (((int64_t)a->N + 255) / 256) >= 2 * (int64_t)cus;
+  const int64_t t128 = ((a->M + 127) / 128) * (((int64_t)a->N + 127) / 128), t256 = ((a->M + 255) / 256) * (((int64_t)a->N + 255) / 256);
+  const bool one_round = a->N % 256 == 0 && a->M >= (a->epilogue == UVMI_GEMM_SOFTCAP ? 384 : 512) && t256 <= cus && 8 * t256 >= 7 * (int64_t)cus && t128 > 2 * (int64_t)cus;
+  const bool many_big_tiles = one_round || (a->M >= 1024 && t256 >= 2 * (int64_t)cus);
   if (a->config == 5 || (a->config == 0 && (many_big_tiles || a->M >= (a->epilogue == UVMI_GEMM_SWIGLU ? BIG_MIN_ROWS_SWIGLU : BIG_MIN_ROWS)) && big_ok(a))) {
     UVMI_REQUIRE(big_ok(a), UVMI_EUNSUPPORTED,
                  "uvmi_gemm_tn: config 5 (256 x 256 tiles) needs K >= 128, C (and the residual) 16-byte aligned, ldc (ldr) %% 8 == 0");
@@ -80,7 +84,6 @@ extern "C" int uvmi_gemm_tn_ex(const uvmi_gemm_args* a, void* stream) {
   // The streaming form while one of its tiles leaves a compute unit about one workgroup (gemm_stream_form) and, on 64 x 64 tiles,
   // until 128 x 128 tiles fill enough of the device: 9/16 of it (N 656, K 640: 10.2 against 11.2 us at 3072 rows), with a longer
   // K, where a tile's chain of slabs is longer, 4/5 (640 columns, K 1664: at 4608 rows 21.0 against 19.3, at 6144 21.6 against 24.5).
-  const int64_t t128 = ((a->M + 127) / 128) * ((a->N + 127) / 128);
   static const int of_config[9] = {-1, 3, 0, -1, 4, -1, -1, 1, 2};
   int form = a->config == 0 ? gemm_stream_form(a, cus) : of_config[a->config];
   if (a->config == 0 && form < 0 && (a->K <= 768 ? 16 * t128 < 9 * (int64_t)cus : 5 * t128 < 4 * (int64_t)cus)) form = 4;

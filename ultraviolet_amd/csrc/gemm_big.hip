@@ -19,9 +19,12 @@
 //     slab k + 1 lands in the other; its operand reads run one MFMA group (8 MFMAs) ahead of their use, and before its
 //     last group it waits for slab k + 1, refills its own stage with slab k + 2 and requests slab k + 1's first operands:
 //     one barrier per slab, no bubble between slabs;
-//   * the accumulator holds C^T fragments (a lane has 4 consecutive columns of one row); the epilogue converts, transposes
-//     4 x 4 across the lane groups with permlane swaps, and each lane stores 16 consecutive columns - whole 128-byte lines
-//     per row instead of 8-byte pieces;
+//   * the accumulator holds C^T fragments (a lane has 4 consecutive columns of one row); the epilogue converts and swaps
+//     lanes so that the 4 lane groups of a row store 64 consecutive bytes (RESID: 16 columns per lane).  fp32 logits are
+//     stored as they lie: 4 columns are 16 bytes (512 x 32768 with the softcap 52.8 us behind the 4 x 4 transpose, 47.7 so,
+//     33.7 on 256 x 256 tiles; 128 rows 17.8 / 14.2; 256 rows 24.2 / 18.0);
+//   * no loads are made past the last slab (they were, to keep the loop free of branches: the epilogue then waited for them;
+//     1 - 3 % of a launch);
 //   * tiles are dealt to the XCDs in contiguous runs, as in the tiled kernel.
 // One workgroup per compute unit (128 KB of LDS, 2 waves per SIMD).  K >= 128; C and the residual 16-byte aligned with
 // pitches that are multiples of 8 elements (the caller checks).
@@ -42,9 +45,16 @@ struct BigParams {
 #define UVMI_LDSP(p) ((__attribute__((address_space(3))) void*)(p))
 #define UVMI_GLBP(p) ((const __attribute__((address_space(1))) void*)(p))
 
+// Two dwords x, y per lane in lane groups g = lane / 16 (x0 .. x3, y0 .. y3) -> x = (x0, x2, y0, y2), y = (x1, x3, y1, y3).
+// (permlane32_swap exchanges the upper 32 lanes of its first operand with the lower 32 of its second, permlane16_swap does the
+// same inside each half.)
+__device__ __forceinline__ void xpose_pair(uint32_t& x, uint32_t& y) {
+  auto s = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+  auto t = __builtin_amdgcn_permlane16_swap(s[0], s[1], false, false);
+  x = t[0]; y = t[1];
+}
 // 4 x 4 transpose of one dword per (register j, lane group g = lane / 16): afterwards register j of group g holds what
-// register g of group j held.  (permlane32_swap exchanges the upper 32 lanes of its first operand with the lower 32 of its
-// second, permlane16_swap does the same inside each half.)
+// register g of group j held.
 __device__ __forceinline__ void xpose4(uint32_t (&x)[4]) {
   auto s0 = __builtin_amdgcn_permlane32_swap(x[0], x[2], false, false);
   auto s1 = __builtin_amdgcn_permlane32_swap(x[1], x[3], false, false);
@@ -107,8 +117,8 @@ void gemm_big_kernel(BigParams P) {
   }
   const unsigned char* ga = (const unsigned char*)P.a;
   const unsigned char* gw = (const unsigned char*)P.w;
-  auto issue = [&](unsigned char* sa, unsigned char* sb, int kt) {   // (past the last slab: the last slab again, into a stage nobody reads)
-    const uint32_t ko = (uint32_t)(kt < nk ? kt : nk - 1) * 128;
+  auto issue = [&](unsigned char* sa, unsigned char* sb, int kt) {
+    const uint32_t ko = (uint32_t)kt * 128;
 #pragma unroll
     for (int i = 0; i < 4; i++)
       __builtin_amdgcn_global_load_lds(UVMI_GLBP(ga + offA[i] + ko), UVMI_LDSP(sa + (4 * wave + i) * 1024), 16, 0, 0);
@@ -191,7 +201,7 @@ void gemm_big_kernel(BigParams P) {
     mm1(4, f0, w1); UVMI_SB(); read_a(SA, 1, 6, f1); UVMI_SB(); mm7(4, f0, w1); sumsq(2, f0); UVMI_SB();                 \
     __builtin_amdgcn_s_waitcnt(0x0f70);                                                                                  \
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");                                                      \
-    issue(SA, SB_, (k) + 2);                                                                                             \
+    if ((k) + 2 < nk) issue(SA, SB_, (k) + 2);                                                                           \
     read_b(SBN, 0, w0); read_a(SAN, 0, 0, f0); UVMI_SB();                                                                \
     mm1(6, f1, w1); mm7(6, f1, w1); sumsq(3, f1); UVMI_SB();                                                             \
   } while (0)
@@ -204,7 +214,7 @@ void gemm_big_kernel(BigParams P) {
     mm1(0, f2, w1); UVMI_SB(); read_a(SA, 1, 2, X); UVMI_SB(); mm7(0, f2, w1); sumsq(0, f2); UVMI_SB();                  \
     __builtin_amdgcn_s_waitcnt(0x0f70);                                                                                  \
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");                                                      \
-    issue(SA, SB_, (k) + 2);                                                                                             \
+    if ((k) + 2 < nk) issue(SA, SB_, (k) + 2);                                                                           \
     read_b(SBN, 0, w0); read_a(SAN, 0, 0, Y); UVMI_SB();                                                                 \
     mm1(2, X, w1); mm7(2, X, w1); sumsq(1, X); UVMI_SB();                                                                \
   } while (0)
@@ -225,7 +235,6 @@ void gemm_big_kernel(BigParams P) {
 #undef UVMI_ITER4
 #undef UVMI_ITER
 #undef UVMI_SB
-  __builtin_amdgcn_s_waitcnt(0x0f70);   // the loads past the last slab have landed before LDS is reused or the wave ends
 
   // ---- row scales of the pre-norm: the 4 lane groups of a row add their sums; LDS carries the scales to every wave
   float rn[FI];
@@ -272,7 +281,35 @@ void gemm_big_kernel(BigParams P) {
         uint16_t* cp = (uint16_t*)P.c + (int64_t)row * P.ldc + n;
         *(uint4*)cp = uint4{x0[0], x0[1], x1[0], x1[1]};
       }
+    } else if (EPI == 3) {   // fp32: 4 columns are 16 bytes, the 4 lane groups of a row store 64 consecutive ones
+      const float k2 = -1.4426950408889634f / P.cap_c;
+      auto cap = [&](float x) { return P.ca * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f((ground<DT>(x * rn[i]) + P.cb) * k2)); };
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const int n = n0 + 64 * wn + 16 * j + 4 * g;
+        if (row < P.M && n < P.N)
+          *(float4*)((float*)P.c + (int64_t)row * P.ldc + n) = float4{cap(acc[i][j][0]), cap(acc[i][j][1]), cap(acc[i][j][2]), cap(acc[i][j][3])};
+      }
+    } else if (EPI == 0) {
+#pragma unroll
+      for (int s = 0; s < 2; s++) {
+        // columns 16 (2 s + j) + 4 g .. of fragments j = 0, 1 -> the 8 consecutive columns 32 s + 8 g ..: the 4 lane groups of a row
+        // store 64 consecutive bytes (pieces of 16 bytes 32 apart: 33 216 x 656 x 640 51.9 us, so 49.2)
+        uint32_t x[2][2];
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+          const gf4 v = acc[i][2 * s + j] * rn[i];
+          x[j][0] = gpack<DT>(v[0], v[1]);
+          x[j][1] = gpack<DT>(v[2], v[3]);
+        }
+        xpose_pair(x[0][0], x[1][0]);
+        xpose_pair(x[0][1], x[1][1]);
+        const int n = n0 + 64 * wn + 32 * s + 8 * g;
+        if (row < P.M && n < P.N) *(uint4*)((uint16_t*)P.c + (int64_t)row * P.ldc + n) = uint4{x[0][0], x[0][1], x[1][0], x[1][1]};
+      }
     } else {
+      // (with the stores of EPI 0 here the residual's loads come in the same pieces: 0 - 3 % slower; requested in the last iteration
+      // but one, the residual costs 56 registers and 10 % of the K = 1664 product)
       uint32_t lo[4], hi[4];
 #pragma unroll
       for (int j = 0; j < 4; j++) {
@@ -285,30 +322,15 @@ void gemm_big_kernel(BigParams P) {
       const int n = n0 + 64 * wn + 16 * g;
       if (row < P.M && n < P.N) {
         uint32_t wds[8] = {lo[0], hi[0], lo[1], hi[1], lo[2], hi[2], lo[3], hi[3]};
-        if (EPI == 2) {
-          const uint16_t* rp = (const uint16_t*)P.r + (int64_t)row * P.ldr + n;
-          const uint4 q0 = *(const uint4*)rp, q1 = *(const uint4*)(rp + 8);
-          const uint32_t rw[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+        const uint16_t* rp = (const uint16_t*)P.r + (int64_t)row * P.ldr + n;
+        const uint4 q0 = *(const uint4*)rp, q1 = *(const uint4*)(rp + 8);
+        const uint32_t rw[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
 #pragma unroll
-          for (int e = 0; e < 8; e++) {
-            float p0, p1, x0, x1;
-            unpack2<DT>(wds[e], p0, p1);   // the product, already rounded to the activation type
-            unpack2<DT>(rw[e], x0, x1);
-            wds[e] = gpack<DT>(P.ca * x0 + P.cb * p0, P.ca * x1 + P.cb * p1);
-          }
-        }
-        if (EPI == 3) {
-          float* fp = (float*)P.c + (int64_t)row * P.ldc + n;
-          const float k2 = -1.4426950408889634f / P.cap_c;
-          auto cap = [&](float x) { return P.ca * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f((x + P.cb) * k2)); };
-#pragma unroll
-          for (int e = 0; e < 4; e++) {
-            float p0, p1, p2, p3;
-            unpack2<DT>(wds[2 * e], p0, p1);
-            unpack2<DT>(wds[2 * e + 1], p2, p3);
-            *(float4*)(fp + 4 * e) = float4{cap(p0), cap(p1), cap(p2), cap(p3)};
-          }
-          continue;
+        for (int e = 0; e < 8; e++) {
+          float p0, p1, x0, x1;
+          unpack2<DT>(wds[e], p0, p1);   // the product, already rounded to the activation type
+          unpack2<DT>(rw[e], x0, x1);
+          wds[e] = gpack<DT>(P.ca * x0 + P.cb * p0, P.ca * x1 + P.cb * p1);
         }
         uint16_t* cp = (uint16_t*)P.c + (int64_t)row * P.ldc + n;
         *(uint4*)cp = uint4{wds[0], wds[1], wds[2], wds[3]};
