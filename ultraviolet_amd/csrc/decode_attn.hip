@@ -73,11 +73,13 @@ __device__ __forceinline__ int load_idx32(const void* p, int is64, int64_t i) {
 }
 // own_key_apart: the key at the row's own position is not in the cache yet (the kernel forms it itself), so the streamed
 // range ends one position earlier.
-__device__ __forceinline__ RowPlan plan_row(const AttnParams& P, int b, bool own_key_apart = false, bool uncut = false) {
+struct RowIdx { int pos, start, row; };   // a row's entries of the index arrays, as loaded
+__device__ __forceinline__ RowIdx load_row(const AttnParams& P, int b) {
+  return RowIdx{load_idx32(P.pos, P.idx64, b), load_idx32(P.starts, P.idx64, b), load_idx32(P.rows ? P.rows : P.pos, P.idx64, b)};
+}
+__device__ __forceinline__ RowPlan plan_row(const AttnParams& P, const RowIdx& ri, int b, bool own_key_apart = false, bool uncut = false) {
   RowPlan r;
-  const int pv = load_idx32(P.pos, P.idx64, b);
-  const int st = load_idx32(P.starts, P.idx64, b);
-  const int rv = load_idx32(P.rows ? P.rows : P.pos, P.idx64, b);
+  const int pv = ri.pos, st = ri.start, rv = ri.row;
   r.cb = P.rows ? rv : b;               // cache row of this query row
   const int pc = r.cb < 0 ? -1 : pv;    // padding row of a compacted batch: no keys, output zeros
   if (r.cb < 0) r.cb = 0;               // (dead rows have no keys; keep addresses valid)
@@ -181,8 +183,8 @@ struct AttnState {
 // arithmetic without the stream: tiles are made up in registers, nothing is loaded from the cache.
 template <int QDT, int ODT, int WPR, bool FUSE, bool KV16 = false, bool FAST = false, int PROBE = 0>
 __global__ __launch_bounds__(WPR > 4 ? 64 * WPR : 256) __attribute__((amdgpu_waves_per_eu(4, 4)))
-void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_rows, const void* a_q, int64_t a_items, int a_idx64,
-                       int a_splits, int a_kh, AttnParams P) {
+void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_rows, const void* a_q, const void* a_tok, int a_items,
+                       int a_idx64, int a_splits, int a_kh, AttnParams P) {
   P.pos = a_pos; P.starts = a_starts; P.rows = a_rows; P.n_items = a_items; P.idx64 = a_idx64; P.splits = a_splits; P.KH = a_kh;
   if constexpr (FAST) { P.idx64 = 1; P.splits = 1; P.KH = 1; P.G = 8; P.H = 8; P.hd = 64; P.chunk_keys = 0; }
   if (FUSE) P.f_qkv = a_q; else P.q = a_q;
@@ -209,6 +211,14 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
   const uint32_t bk = P.splits == 1 ? it32 : it32 / (uint32_t)P.splits;
   const int b = __builtin_amdgcn_readfirstlane((int)(P.KH == 1 ? bk : bk / (uint32_t)P.KH));
   const int h = __builtin_amdgcn_readfirstlane((int)(P.KH == 1 ? 0u : bk % (uint32_t)P.KH));
+  // The row's indices are requested first, all at once: their addresses come with the wave (preloaded arguments), so they share
+  // the trip to memory that the rest of the arguments takes.  (a_tok is some readable index array where there is no token.  One
+  // after the other, as the compiler places them by itself, they are two to three trips more before the first K / V request.)
+  RowIdx ri = load_row(P, b);
+  int tok_idx = FUSE ? load_idx32(a_tok, P.idx64, b) : 0;
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (FUSE) asm volatile("" : "+s"(ri.pos), "+s"(ri.start), "+s"(ri.row), "+s"(tok_idx));
+  else asm volatile("" : "+s"(ri.pos), "+s"(ri.start), "+s"(ri.row));
   const int m = lane & 15, g = lane >> 4;  // A/B operand (row, group) == accumulator (column, group)
   const int strm = m >> 3, head = m & 7;
   const int G = P.G;
@@ -236,7 +246,7 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
     vlog = rowp[P.f_ext + P.H + h];
     raw_a = rowp[(P.H + (WPR > 1 && wsub == VW ? P.KH : 0) + h) * 64 + lane];
     if (WPR == 1) raw_v = rowp[(P.H + P.KH + h) * 64 + lane];
-    own_tok = P.f_has_ve ? (int64_t)load_idx32(P.f_tok, P.idx64, b) : 0;
+    own_tok = P.f_has_ve ? tok_idx : 0;
     own_tok = own_tok < 0 ? 0 : (own_tok >= P.f_vocab ? P.f_vocab - 1 : own_tok);
   }
   // Operands of the fused epilogue are requested now, with q, and parked in LDS once q has arrived, so that the
@@ -249,7 +259,7 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
   const float* pg_src = !FUSE && has_post && P.post_gate ? P.post_gate + (int64_t)b * P.H + hsafe : anyf;
   const float* px_src = has_post && P.post_xsa ? P.post_xsa + hsafe : anyf;
   const float pv_val = *pv_src, pg_val = *pg_src, px_val = *px_src;
-  const RowPlan rp = plan_row(P, b, FUSE, FAST);
+  const RowPlan rp = plan_row(P, ri, b, FUSE, FAST);
   // FUSE: the row of the rotation table (cos / sin of the row's position per frequency, already rounded to the activation
   // type): prep_q reads its 32 values as scalars, the lane that owns dim d of the own key reads its own pair
   const int rope_row = rp.pc < 0 ? 0 : (rp.pc < P.f_rope_n ? rp.pc : P.f_rope_n - 1);
@@ -941,7 +951,7 @@ __global__ __launch_bounds__(64) void attn_generic(AttnParams P) {
     qs[i] = elem<QDT>::ld(P.q, (int64_t)b * P.sqb + (int64_t)(h * G + gi) * P.sqh + d);
   }
   __syncthreads();
-  const RowPlan rp = plan_row(P, b);
+  const RowPlan rp = plan_row(P, load_row(P, b), b);
   if (sid >= rp.nsplit) return;
   struct { int s0, s1; } c;
   c.s0 = rp.a0 + sid * rp.chunk;
@@ -1048,7 +1058,7 @@ __global__ __launch_bounds__(256) void attn_combine(AttnParams P) {
   const int64_t bk = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (bk >= (int64_t)P.B * P.KH) return;
   const int b = (int)(bk / P.KH), h = (int)(bk % P.KH);
-  const RowPlan rp = plan_row(P, b);
+  const RowPlan rp = plan_row(P, load_row(P, b), b);
   if (rp.nsplit <= 1) return;
   for (int gi = 0; gi < P.G; gi++) {
     float mx = -INFINITY;
@@ -1256,7 +1266,7 @@ static int decode_attn_launch(const uvmi_attn_args* a, void* ws, size_t ws_bytes
     if (P.chunk_keys) P.chunk_keys = (P.chunk_keys + P.gran - 1) / P.gran * P.gran;
     const int ipb = wpr > 4 ? 1 : 4 / wpr;
     const dim3 grid((unsigned)((P.n_items + ipb - 1) / ipb)), blk(wpr > 4 ? 64 * wpr : 256);
-#define UVMI_LEAD P.pos, P.starts, P.rows, (a->fuse ? P.f_qkv : P.q), P.n_items, P.idx64, P.splits, P.KH
+#define UVMI_LEAD P.pos, P.starts, P.rows, (a->fuse ? P.f_qkv : P.q), (a->fuse && P.f_has_ve ? P.f_tok : P.pos), (int)P.n_items, P.idx64, P.splits, P.KH
 #define UVMI_L(QD, OD)                                                                                \
   do {                                                                                                \
     if (wpr == 8) hipLaunchKernelGGL((attn_mfma_i8_hd64<QD, OD, 8, false>), grid, blk, 0, st, UVMI_LEAD, P);      \
