@@ -99,7 +99,7 @@ __device__ __forceinline__ RowPlan plan_row(const AttnParams& P, const RowIdx& r
   }
   // (integer divisions by run-time values cost a few dozen instructions each, here on the way to the row's first tile
   // request: the granule is a power of two, and an uncut row - every decode step of the engine - divides by nothing)
-  const int gr = P.gran;  // 32, 64 or 128
+  const int gr = P.gran;  // a power of two from 32 up
   const int per = P.splits == 1 ? span : (int)(((uint32_t)span + (uint32_t)P.splits - 1u) / (uint32_t)P.splits);
   int chunk = (per + gr - 1) & ~(gr - 1);
   if (chunk < P.chunk_keys) chunk = P.chunk_keys;
@@ -181,11 +181,12 @@ struct AttnState {
 // PROBE (uvmi_decode_attn_probe; measurement only, the output is meaningless): 1 - the kernel's memory stream without its
 // arithmetic: every tile is loaded exactly as in the real kernel and folded into the state with a few xors; 2 - its
 // arithmetic without the stream: tiles are made up in registers, nothing is loaded from the cache.
-template <int QDT, int ODT, int WPR, bool FUSE, bool KV16 = false, bool FAST = false, int PROBE = 0>
+template <int QDT, int ODT, int WPR, bool FUSE, bool KV16 = false, bool FAST = false, int PROBE = 0, bool BYSLOT = false>
 __global__ __launch_bounds__(WPR > 4 ? 64 * WPR : 256) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_rows, const void* a_q, const void* a_tok, int a_items,
                        int a_idx64, int a_splits, int a_kh, AttnParams P) {
   P.pos = a_pos; P.starts = a_starts; P.rows = a_rows; P.n_items = a_items; P.idx64 = a_idx64; P.splits = a_splits; P.KH = a_kh;
+  if constexpr (BYSLOT) P.ring = 1;
   if constexpr (FAST) { P.idx64 = 1; P.splits = 1; P.KH = 1; P.G = 8; P.H = 8; P.hd = 64; P.chunk_keys = 0; }
   if (FUSE) P.f_qkv = a_q; else P.q = a_q;
   constexpr int BW = WPR > 4 ? WPR : 4, IPB = BW / WPR;  // waves and items per block
@@ -211,14 +212,16 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
   const uint32_t bk = P.splits == 1 ? it32 : it32 / (uint32_t)P.splits;
   const int b = __builtin_amdgcn_readfirstlane((int)(P.KH == 1 ? bk : bk / (uint32_t)P.KH));
   const int h = __builtin_amdgcn_readfirstlane((int)(P.KH == 1 ? 0u : bk % (uint32_t)P.KH));
-  // The row's indices are requested first, all at once: their addresses come with the wave (preloaded arguments), so they share
-  // the trip to memory that the rest of the arguments takes.  (a_tok is some readable index array where there is no token.  One
-  // after the other, as the compiler places them by itself, they are two to three trips more before the first K / V request.)
+  // FUSE: the row's indices are requested first, all at once: their addresses come with the wave (preloaded arguments), so they
+  // share the trip to memory that the rest of the arguments takes.  (a_tok is some readable index array where there is no token.
+  // One after the other, as the compiler places them by itself, they are two to three trips more before the first K / V request.
+  // Unfused, q is requested ahead of them: 1000 rows of up to 4096 keys 62.3 us against 62.7.)
   RowIdx ri = load_row(P, b);
   int tok_idx = FUSE ? load_idx32(a_tok, P.idx64, b) : 0;
-  __builtin_amdgcn_sched_barrier(0);
-  if constexpr (FUSE) asm volatile("" : "+s"(ri.pos), "+s"(ri.start), "+s"(ri.row), "+s"(tok_idx));
-  else asm volatile("" : "+s"(ri.pos), "+s"(ri.start), "+s"(ri.row));
+  if constexpr (FUSE) {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" : "+s"(ri.pos), "+s"(ri.start), "+s"(ri.row), "+s"(tok_idx));
+  }
   const int m = lane & 15, g = lane >> 4;  // A/B operand (row, group) == accumulator (column, group)
   const int strm = m >> 3, head = m & 7;
   const int G = P.G;
@@ -268,6 +271,18 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
   const int s0 = rp.a0 + sid * rp.chunk;
   const int s1 = live ? min(s0 + rp.chunk, rp.p + 1) : s0;
   const int lo_eff = max(rp.lo, s0);
+  // BYSLOT: a row that has been once around its ring, where the window is the whole ring, has its keys streamed by slot, not by
+  // position.  The window's first position is rarely a multiple of 32, so by position a ring of S slots takes S / 32 + 1 tiles
+  // (256 slots: 9, a third round for 4 waves), by slot S / 32.  Slots below wx hold the positions from wb up, the others those of
+  // one turn before; in the tile with both, positions from s1 on stand for the position S below.  (Straight-line selects: a branch
+  // here would separate the loads above from the first tile's.  Rings of 256, 64 rows 6.0 -> 5.55 us, 512 rows 7.2 -> 7.05, 1000
+  // rows 10.3 -> 9.7; 16-bit cache 6.4 -> 6.0, 9.5 -> 9.4, 16.3 -> 15.7.  Rows that have not wrapped pay up to 0.1 us for the
+  // selects, which is why caches that cannot wrap run without them.)
+  const int turn = BYSLOT ? P.S : 0x7fffffff;
+  const int wrapped = BYSLOT ? -(int)(s1 > turn) : 0;   // all ones or zero
+  const int wx = s1 & (turn - 1) & wrapped, wb = s1 - wx;
+  auto tile_pos = [&](int u) { return BYSLOT ? u + ((wb - (u >= wx ? turn : 0)) & wrapped) : u; };   // position of tile u's first key
+  auto outside = [&](int t) { return t < lo_eff || (t >= s1 && (!BYSLOT || !wrapped || t - turn < lo_eff)); };
 
   // ---- Q^T operands: lane (n, g) holds q[head][16g + 8s + j] as fp16 (bf16 inputs are converted; exact for
   // 2^-14 <= |q| <= 65504).  The K operand carries a +1152 bias, cancelled by starting the accumulator at
@@ -552,8 +567,8 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
       u4 a0 = T.kA[0], a1 = T.kA[1], b0 = T.kB[0], b1 = T.kB[1];
       if (edge) {
         const u4 z = u4{0u, 0u, 0u, 0u};
-        if (tb + m < lo_eff || tb + m >= s1) { a0 = z; a1 = z; }
-        if (tb + 16 + m < lo_eff || tb + 16 + m >= s1) { b0 = z; b1 = z; }
+        if (outside(tb + m)) { a0 = z; a1 = z; }
+        if (outside(tb + 16 + m)) { b0 = z; b1 = z; }
       }
       acc = mfma_kv<QDT>(as_h8(a0.x, a0.y, a0.z, a0.w), QA0, acc);
       acc = mfma_kv<QDT>(as_h8(a1.x, a1.y, a1.z, a1.w), QA1, acc);
@@ -584,7 +599,7 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
       const int t0 = tb + 16 * strm + 4 * g;
 #pragma unroll
       for (int i = 0; i < 4; i++)
-        if (t0 + i < lo_eff || t0 + i >= s1) { t[i] = -INFINITY; vsf[i] = 0.f; }
+        if (outside(t0 + i)) { t[i] = -INFINITY; vsf[i] = 0.f; }
     }
     // The reference point of a column's exponentials only has to stay within 2^LAZY of its true maximum (probabilities up
     // to 2^LAZY are as exact in fp16 / fp32 as those below 1), so the common tile compares each lane's own scores with
@@ -644,8 +659,8 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
 #pragma unroll
         for (int j = 0; j < 4; j++) {
           const int ka = tb + 4 * g + j, kb = ka + 16;
-          if (ka < lo_eff || ka >= s1) va_[j] = u2{0u, 0u};
-          if (kb < lo_eff || kb >= s1) vb_[j] = u2{0u, 0u};
+          if (outside(ka)) va_[j] = u2{0u, 0u};
+          if (outside(kb)) vb_[j] = u2{0u, 0u};
         }
       }
       constexpr uint32_t LO = 0x05040100u, HI = 0x07060302u;
@@ -675,8 +690,8 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
     // before the current tile is consumed (past the end the current tile is re-read, a cache hit), so that no
     // branch separates load issue from use and the wait counters stay exact.
     constexpr int STEP = 32 * WPR;
-    const int s1f = P.ring ? s1 : min(s1, S & ~31);
-    int tb = s0 + 32 * wsub;
+    const int s1f = BYSLOT && wrapped ? S : P.ring ? s1 : min(s1, S & ~31);
+    int tb = (s0 & ~wrapped) + 32 * wsub;
     const bool has = tb < s1f;
     int slot = has ? ring_slot(P, tb) : 0;
     auto next_slot = [&](int sl, int t) {
@@ -726,21 +741,25 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
         if (WPR == 1) own_v(raw_v, raw_ve);
       }
     }
+    auto stepu = [&](const TileX& T, int u) {
+      const int t = tile_pos(u);
+      step(T, t, t < lo_eff || t + 32 > s1);
+    };
     if (has) {
       while (true) {
         slot = next_slot(slot, tb);
         load_tile(slot, TB);
-        step(TA, tb, tb < lo_eff || tb + 32 > s1);
+        stepu(TA, tb);
         tb += STEP;
         if (tb >= s1f) break;
         slot = next_slot(slot, tb);
         load_tile(slot, TA);
-        step(TB, tb, tb < lo_eff || tb + 32 > s1);
+        stepu(TB, tb);
         tb += STEP;
         if (tb >= s1f) break;
       }
     }
-    if (tb < s1) {  // linear cache ending inside this super-tile (at most one wave of the item gets here)
+    if (!P.ring && tb < s1) {  // linear cache ending inside this super-tile (at most one wave of the item gets here)
       TileX TT;
       load_tail(tb, TT);
       step(TT, tb, true);
@@ -1274,6 +1293,13 @@ static int decode_attn_launch(const uvmi_attn_args* a, void* ws, size_t ws_bytes
     else if (wpr == 2) hipLaunchKernelGGL((attn_mfma_i8_hd64<QD, OD, 2, false>), grid, blk, 0, st, UVMI_LEAD, P); \
     else hipLaunchKernelGGL((attn_mfma_i8_hd64<QD, OD, 1, false>), grid, blk, 0, st, UVMI_LEAD, P);               \
   } while (0)
+#define UVMI_LS(QD, W, FU, K16, FA) hipLaunchKernelGGL((attn_mfma_i8_hd64<QD, QD, W, FU, K16, FA, 0, true>), grid, blk, 0, st, UVMI_LEAD, P)
+#define UVMI_LBS(QD, FU, K16, FA)                                                                     \
+  do {                                                                                                \
+    if (wpr == 4) UVMI_LS(QD, 4, FU, K16, FA);                                                        \
+    else if (wpr == 2) UVMI_LS(QD, 2, FU, K16, FA);                                                   \
+    else UVMI_LS(QD, 1, FU, K16, FA);                                                                 \
+  } while (0)
 #define UVMI_LF(QD)                                                                                   \
   do {                                                                                                \
     if (fast && wpr == 8) hipLaunchKernelGGL((attn_mfma_i8_hd64<QD, QD, 8, true, false, true>), grid, blk, 0, st, UVMI_LEAD, P);       \
@@ -1306,6 +1332,8 @@ static int decode_attn_launch(const uvmi_attn_args* a, void* ws, size_t ws_bytes
   } while (0)
     const int od = a->out_dtype;  // rows that fit one chunk are written directly even when num_splits > 1
     // the engine's decode-step shape has an instantiation of its own (see FAST)
+    // rings that are streamed by slot once they have wrapped (BYSLOT): the window is the ring, S a power of two
+    const bool by_slot = a->ring && a->window == a->S && (a->S & (a->S - 1)) == 0 && a->num_splits == 1 && !probe;
     const bool fast = !kv16 && a->num_splits == 1 && a->KH == 1 && a->H == 8 && a->idx_dtype == UVMI_I64;
     if (probe) {
       UVMI_REQUIRE(fast && !a->fuse && od == a->q_dtype && a->q_dtype == UVMI_BF16, UVMI_EUNSUPPORTED,
@@ -1318,6 +1346,11 @@ static int decode_attn_launch(const uvmi_attn_args* a, void* ws, size_t ws_bytes
   } while (0)
       if (probe == 1) UVMI_LP(1); else UVMI_LP(2);
 #undef UVMI_LP
+    } else if (by_slot && kv16 && a->fuse && wpr <= 4) {
+      if (a->q_dtype == UVMI_F16) UVMI_LBS(UVMI_F16, true, true, false); else UVMI_LBS(UVMI_BF16, true, true, false);
+    } else if (by_slot && fast && od == a->q_dtype && wpr <= 4) {
+      if (a->fuse) { if (a->q_dtype == UVMI_F16) UVMI_LBS(UVMI_F16, true, false, true); else UVMI_LBS(UVMI_BF16, true, false, true); }
+      else { if (a->q_dtype == UVMI_F16) UVMI_LBS(UVMI_F16, false, false, true); else UVMI_LBS(UVMI_BF16, false, false, true); }
     } else if (kv16 && a->fuse) {
       if (a->q_dtype == UVMI_F16) UVMI_LF16(UVMI_F16); else UVMI_LF16(UVMI_BF16);
     } else if (kv16) {
@@ -1338,6 +1371,8 @@ static int decode_attn_launch(const uvmi_attn_args* a, void* ws, size_t ws_bytes
 #undef UVMI_L
 #undef UVMI_LF
 #undef UVMI_LFAST
+#undef UVMI_LS
+#undef UVMI_LBS
 #undef UVMI_L16
 #undef UVMI_LF16
 #undef UVMI_LEAD
