@@ -808,3 +808,37 @@ def test_packed_prompt_tables_match_their_definition(n, hi, left_pad):
             assert np.array_equal(pk[k].cpu().numpy(), v), k
     with pytest.raises(IndexError):
         eng._pack(prompts, [B] * n, 320, left_pad, st)
+
+
+@pytest.mark.parametrize("kv_dtype", ["int8", "fp16"])
+def test_ring_of_a_short_cache_keeps_its_length(kv_dtype):
+    """A ring that a short max_len cuts below the window has max_len slots for its user (their fills and copies see no other
+    shape) and runs on whole tiles: prefill, steps and row copies give what a state of whole tiles gives bit for bit, and a
+    state whose tensors are replaced runs on those."""
+    from ultraviolet_amd.engine import KVState
+    cfg, _, eng, _ = _setup(dtype=torch.bfloat16, window=64)
+    prompts, B = _prompts(cfg, (40, 3, 33), seed=4), 5
+    a, b = (KVState(cfg, B, n, DEV, kv_dtype=kv_dtype, dtype=torch.bfloat16) for n in (50, 64))
+    l = [i for i in range(cfg.n_layers) if not cfg.is_global(i)][0]
+    assert a.k[l].size(2) == a.v[l].size(2) == a.local_len == 50 and a.slots(l) == 64 and b.slots(l) == 64 and a.max_len == 64
+    for st in (a, b):
+        g = torch.Generator(device=DEV).manual_seed(7)
+        st.k[l][:, :, :50] = torch.randint(-5, 6, st.k[l][:, :, :50].shape, generator=g, device=DEV).to(st.k[l].dtype)
+    for step in range(4):
+        if step == 0:
+            outs = [eng.prefill(prompts, [2, 0, 1], st, left_pad=False).clone() for st in (a, b)]
+        elif step == 2:
+            for st in (a, b):
+                st.copy_rows(torch.tensor([2, 0], device=DEV), torch.tensor([3, 4], device=DEV), 41)
+        tok = torch.arange(B, device=DEV) + 9
+        outs = [eng.decode_step(tok, st).clone() for st in (a, b)]
+        assert torch.equal(*outs)
+    for i in range(cfg.n_layers):
+        n = a.k[i].size(2)
+        assert torch.equal(a.k[i], b.k[i][:, :, :n]) and torch.equal(a.v[i], b.v[i][:, :, :n])
+    a.k[l], a.v[l] = a.k[l].clone(), a.v[l].clone()
+    if kv_dtype == "int8":
+        a.k_scale[l], a.v_scale[l] = a.k_scale[l].clone(), a.v_scale[l].clone()
+    assert a.slots(l) == 50
+    outs = [eng.decode_step(tok, st).float() for st in (a, b)]
+    assert float((outs[0] - outs[1]).norm() / outs[1].norm()) < 0.05   # (the generic kernel: bf16 roundings of four layers)

@@ -33,10 +33,11 @@ class KVState:
     reference's name for "unquantized") keeps k, v in `dtype`, the activation type, with no scales."""
 
     def __init__(self, cfg: UVConfig, B: int, max_len: int, device="cuda", kv_dtype: str = "int8", dtype=torch.bfloat16):
-        # Global caches are allocated with S rounded up to 32 slots: the MFMA attention kernel streams 32-key tiles and
-        # needs S % 4 == 0 for its 8-byte scale loads (other S fall back to the generic kernel).  A ring of a full window keeps
-        # its length; one that a short max_len cuts below the window never wraps, so it is rounded up like a global cache (the
-        # generic kernel takes 123 us where the MFMA kernel takes 5.6 on 16 rows of up to 128 keys).
+        # Global caches have S rounded up to 32 slots: the MFMA attention kernel streams 32-key tiles and needs S % 4 == 0 for its
+        # 8-byte scale loads (other S fall back to the generic kernel).  A ring of a full window keeps its length; one that a short
+        # max_len cuts below the window never wraps: it keeps its length too, but as the front of an allocation of whole
+        # tiles, on which the kernels run (cache(); the generic kernel takes 123 us where the MFMA kernel takes 5.6 on 16 rows of
+        # up to 128 keys).
         self.local_len = min(cfg.window, max_len)
         max_len = (max_len + 31) // 32 * 32
         ring = min(cfg.window, max_len)
@@ -46,15 +47,31 @@ class KVState:
         cdt = torch.int8 if self.quantized else dtype
         dev = torch.device(device)
         self.k, self.v, self.k_scale, self.v_scale = [], [], [], []
+        self._whole = []   # per layer the whole allocations where k, v and the scales are the front of them, else None
         for l in range(cfg.n_layers):
-            S = max_len if cfg.is_global(l) else ring
+            S, front = (max_len, max_len) if cfg.is_global(l) else (ring, self.local_len)
             shp = (B, cfg.n_kv_heads, S, cfg.head_dim)
-            self.k.append(torch.zeros(shp, dtype=cdt, device=dev))
-            self.v.append(torch.zeros(shp, dtype=cdt, device=dev))
-            self.k_scale.append(torch.zeros(shp[:3], dtype=torch.float16, device=dev) if self.quantized else None)
-            self.v_scale.append(torch.zeros(shp[:3], dtype=torch.float16, device=dev) if self.quantized else None)
+            whole = [torch.zeros(shp, dtype=cdt, device=dev) for _ in range(2)]
+            whole += [torch.zeros(shp[:3], dtype=torch.float16, device=dev) if self.quantized else None for _ in range(2)]
+            self._whole.append(whole if front < S else None)
+            for ts, t in zip((self.k, self.v, self.k_scale, self.v_scale), whole):
+                ts.append(t if t is None or front == S else t[:, :, :front])
         self.pos = torch.zeros(B, dtype=torch.long, device=dev)
         self.starts = torch.zeros(B, dtype=torch.long, device=dev)
+
+    def cache(self, l: int) -> tuple:
+        """k, v, k_scale, v_scale of layer l as the kernels take them: the whole allocations, as long as the layer's tensors are
+        still the front of them, else the tensors."""
+        ts = (self.k[l], self.v[l], self.k_scale[l], self.v_scale[l])
+        whole = self._whole[l]
+        if whole is None or any(t is not None and (t.data_ptr() != w.data_ptr() or t.stride() != w.stride()) for t, w in zip(ts, whole)):
+            return ts
+        return tuple(whole)
+
+    def slots(self, l: int) -> int:
+        """Slots of cache(l)'s rows (of its k; the launch checks the rest)."""
+        k, whole = self.k[l], self._whole[l]
+        return k.size(2) if whole is None or k.data_ptr() != whole[0].data_ptr() else whole[0].size(2)
 
     def nbytes(self) -> int:
         return sum(t.numel() * t.element_size() for t in self.k + self.v + self.k_scale + self.v_scale if t is not None)
@@ -65,7 +82,7 @@ class KVState:
         int64 on the device).  A sequence's cache depends only on its own tokens and quantisation is per row, so a prompt
         shared by several sequences is prefilled once and copied: the copies hold the bytes their own prefill would write."""
         for l in range(self.cfg.n_layers):
-            for t in (self.k[l], self.v[l], self.k_scale[l], self.v_scale[l]):
+            for t in self.cache(l):
                 if t is not None:
                     n = min(upto, t.size(2))
                     t[dst, :, :n] = t[src, :, :n]
@@ -225,11 +242,11 @@ class UVEngine:
         write_cache = st is not None and write_cache
         fused_write = write_cache and self._append_fused(st)
         if fused_write:   # int8 codes and scales, or (a cache of the activation type) the values as they are
-            kc, ks = st.k[l], st.k_scale[l]
-            a.k_cache, a.v_cache, a.S = kc.data_ptr(), st.v[l].data_ptr(), kc.size(2)
+            kc, vc, ks, vs = st.cache(l)
+            a.k_cache, a.v_cache, a.S = kc.data_ptr(), vc.data_ptr(), kc.size(2)
             a.scb, a.sch, a.scs = kc.stride(0), kc.stride(1), kc.stride(2)
             if st.quantized:
-                a.k_scale, a.v_scale, a.ssb, a.ssh = ks.data_ptr(), st.v_scale[l].data_ptr(), ks.stride(0), ks.stride(1)
+                a.k_scale, a.v_scale, a.ssb, a.ssh = ks.data_ptr(), vs.data_ptr(), ks.stride(0), ks.stride(1)
         a.n, a.vocab = n, cfg.vocab_size
         a.H, a.KH, a.hd, a.d, a.ve_ch, a.n_pairs = cfg.n_heads, cfg.n_kv_heads, cfg.head_dim, cfg.d_model, cfg.ve_gate_channels, cfg.n_pairs
         a.ring, a.has_ve = int(not glob), int(has_ve)
@@ -257,7 +274,8 @@ class UVEngine:
         will not keep (older than last_pos - S)."""
         cfg, b = self.cfg, self.buf
         K = cfg.n_kv_heads
-        S = st.k[l].size(2)
+        kc, vc = st.cache(l)[:2]
+        S = kc.size(2)
         ring = not cfg.is_global(l)
         row = torch.arange(n, device=pos.device) if rows is None else rows[:n]
         p = pos[:n]
@@ -267,8 +285,8 @@ class UVEngine:
             ok &= p > last_pos[:n] - S
         flat = (row[:, None] * K + torch.arange(K, device=pos.device)[None, :]) * S + slot[:, None]
         flat = torch.where(ok[:, None], flat, torch.full_like(flat, -1)).reshape(-1).contiguous()
-        kv_write(st.k[l], None, flat, b["k"][:n])
-        kv_write(st.v[l], None, flat, b["v"][:n])
+        kv_write(kc, None, flat, b["k"][:n])
+        kv_write(vc, None, flat, b["v"][:n])
 
     def _attn_post(self, l: int, z: Tensor, n: int, off: int = 0):
         """XSA + gate of rows off..off+n of the call (z holds just those rows); writes buf zg[off:off+n]."""
@@ -295,7 +313,7 @@ class UVEngine:
     def cache_attention_plannable(self, l: int, st: KVState) -> bool:
         """Whether layer l's attention over the cache is one launch with the fused XSA + gate epilogue: the MFMA kernel streams
         32-key tiles (rings need S % 32 == 0, linear int8 caches S % 4 == 0) and serves int8 caches and caches in the q dtype."""
-        cfg, S = self.cfg, st.k[l].size(2)
+        cfg, S = self.cfg, st.slots(l)
         mfma_cache = self.q_dtype != torch.float32 and (st.quantized or st.k[l].dtype == self.q_dtype)
         return (mfma_cache and cfg.xsa and cfg.n_heads // cfg.n_kv_heads <= 8 and S % (4 if cfg.is_global(l) else 32) == 0 and S >= 32)
 
@@ -312,13 +330,13 @@ class UVEngine:
                 rows = rows.to(pos.dtype).contiguous()
             out = b["zg"][off:off + n].view(n, cfg.n_heads, cfg.head_dim)
             gate = None if W["attn_gate"] is None else b["gate"][off:off + n]
-            a, keep = build_attn_args(q, st.k[l], st.v[l], pos.contiguous(), starts.contiguous(), cfg.attn_scale, window, not glob, st.k_scale[l],
-                                      st.v_scale[l], 1, out, 0, rows, (b["vhat"][off:off + n], gate, W["xsa"], out.dtype))
+            k, v, ks, vs = st.cache(l)
+            a, keep = build_attn_args(q, k, v, pos.contiguous(), starts.contiguous(), cfg.attn_scale, window, not glob, ks, vs, 1, out, 0, rows, (b["vhat"][off:off + n], gate, W["xsa"], out.dtype))
             self._op(L.OP_DECODE_ATTN, a, (keep, q, pos, starts), B="nd", q="q_d", post_vhat="vhat_d", out="zg_d", pos="pos_d", starts="starts_d",
                      **({} if gate is None else {"post_gate": "gate_d"}), **({} if rows is None else {"rows": "rows_d"}))
             return None
-        return decode_attention(q, st.k[l], st.v[l], pos, starts, cfg.attn_scale, num_splits=1, window=window, ring=not glob, k_scale=st.k_scale[l],
-                                v_scale=st.v_scale[l], rows=rows)
+        k, v, ks, vs = st.cache(l)
+        return decode_attention(q, k, v, pos, starts, cfg.attn_scale, num_splits=1, window=window, ring=not glob, k_scale=ks, v_scale=vs, rows=rows)
 
     def prompt_attention_plannable(self) -> bool:
         """Whether the packed prompts' attention is one launch with the fused XSA + gate epilogue (16-bit engine)."""
@@ -345,7 +363,7 @@ class UVEngine:
 
     def fused_layer_ok(self, l: int, st: KVState) -> bool:
         """Whether layer l's decode attention can take the fused path: the MFMA kernel streams 32-key tiles."""
-        S = st.k[l].size(2)
+        S = st.slots(l)
         return self.fuse_qkv and (st.quantized or st.k[l].dtype == self.dtype) and S % 32 == 0 and S >= 32
 
     def rope_table(self, n_positions: int) -> Tensor:
@@ -382,8 +400,8 @@ class UVEngine:
         cfg, b, W = self.cfg, self.buf, self.w.layers[l]
         glob = cfg.is_global(l)
         out = b["zg"][:n].view(n, cfg.n_heads, cfg.head_dim)
-        return build_fused_args(qkvx[:n], cfg.n_heads, st.k[l], st.v[l], pos, starts, cfg.attn_scale, 0 if glob else cfg.window, not glob,
-                                st.k_scale[l], st.v_scale[l], W["xsa"], out, self._fuse_dict(l, tok, st), rows)
+        k, v, ks, vs = st.cache(l)
+        return build_fused_args(qkvx[:n], cfg.n_heads, k, v, pos, starts, cfg.attn_scale, 0 if glob else cfg.window, not glob, ks, vs, W["xsa"], out, self._fuse_dict(l, tok, st), rows)
 
     def cache_attention_args(self, l: int, st: KVState, pos: Tensor, starts: Tensor, n: int, rows: Tensor | None = None):
         """The uvmi_attn_args struct cache_attention would launch for layer l on the engine's buffers (fused path only):
@@ -391,8 +409,8 @@ class UVEngine:
         cfg, b, W = self.cfg, self.buf, self.w.layers[l]
         glob = cfg.is_global(l)
         out = b["zg"][:n].view(n, cfg.n_heads, cfg.head_dim)
-        return build_attn_args(b["q"][:n], st.k[l], st.v[l], pos, starts, cfg.attn_scale, 0 if glob else cfg.window, not glob,
-                               st.k_scale[l], st.v_scale[l], 1, out, 0, rows,
+        k, v, ks, vs = st.cache(l)
+        return build_attn_args(b["q"][:n], k, v, pos, starts, cfg.attn_scale, 0 if glob else cfg.window, not glob, ks, vs, 1, out, 0, rows,
                                (b["vhat"][:n], None if W["attn_gate"] is None else b["gate"][:n], W["xsa"], out.dtype))
 
     def _trunk(self, tok: Tensor, pos: Tensor, n: int, attn, rows=None, last_pos=None, st: KVState | None = None,
@@ -759,8 +777,9 @@ class UVEngine:
             if ns.get(key) in (None, 1):
                 return self.cache_attention(l, q, st, pos, starts, B)
             glob = cfg.is_global(l)
-            return decode_attention(q, st.k[l], st.v[l], pos, starts, cfg.attn_scale, window=0 if glob else cfg.window, ring=not glob,
-                                    k_scale=st.k_scale[l], v_scale=st.v_scale[l], num_splits=ns[key])
+            k, v, ks, vs = st.cache(l)
+            return decode_attention(q, k, v, pos, starts, cfg.attn_scale, window=0 if glob else cfg.window, ring=not glob,
+                                    k_scale=ks, v_scale=vs, num_splits=ns[key])
 
         h = self._trunk(tok, pos, B, attn, st=st, fused_attn=fused)
         st.pos.add_(1)
