@@ -610,73 +610,6 @@ class UVEngine:
         the call's row counts and addresses (values).  The list is recorded again when an object it rests on is another one or
         elsewhere (weights, cache tensors, a switch of the launch plans)."""
         own_down = n <= self.skinny_rows or n >= self.big_rows or self.fold_down_rows[0] <= n <= self.fold_down_rows[1]
-        for l, W in enumerate(self.w.layers):
-            self._project_qkv(l, n, n <= self.fold_qkv_rows, config=gc)
-            self._qkv_post(l, tok, pos, rows, last_pos, st, n, ext=True)
-            z = attn(l, b["q"][:n])
-            if z is not None:
-                if l > 0:
-                    self._add_norm(x, x, 1.0, 0.0, n, None, b["xn"])
-                self._attn_post(l, z, n)
-            self._gemm(zg, W["wo"], x, RESID, resid=x, ca=W["resid_attn"], cb=W["post_attn"], config=gc)
-            self._gemm(x, W["gu_il"], act, SWIGLU, norm_eps=self.eps, config=gc)
-            self._down(l, n, own_down)
-
-    def _layers_plain(self, n: int, tok, pos, rows, last_pos, st, attn, fused_attn) -> bool:
-        """The reference's order of operations on the vendor library's GEMMs (16-bit passes of few rows: on this one's),
-        one launch per step between them: fp32 engines, widths the other plans do not take.  Returns whether buf x was
-        left un-normalised (else buf xn holds the final norm)."""
-        cfg, b = self.cfg, self.buf
-        x, xn = b["x"][:n], b["xn"][:n]
-        skinny_rows = self.skinny_rows if fused_attn is not None else max(self.skinny_rows, self.general_skinny_rows)
-        skinny = n <= skinny_rows and cfg.d_model % 64 == 0 and cfg.d_model <= 960 and (cfg.n_heads * cfg.head_dim) % 64 == 0
-        mm = (lambda a, w, out: gemm_tn(a, w, out)) if skinny else (lambda a, w, out: torch.mm(a, w.t(), out=out))
-        fold_mlp = not skinny and self.dtype != torch.float32 and cfg.d_ff % 8 == 0 and self.fold
-        for l, W in enumerate(self.w.layers):
-            if fused_attn is not None and self.fused_layer_ok(l, st):
-                # decode rows of a 16-bit engine: the projection also forms the gate logits, and fused_attn(l) does the
-                # post-processing, the cache append, the attention and its epilogue in one launch (writes buf zg)
-                mm(xn, W["wqkv_ext"], b["qkvx"][:n])
-                self._keep_projection(l, n)
-                fused_attn(l)
-            else:
-                mm(xn, W["wqkv"], b["qkv"][:n])
-                self._qkv_post(l, tok, pos, rows, last_pos, st, n)
-                z = attn(l, b["q"][:n])
-                if z is not None:   # None: the attention kernel already applied XSA + gate and wrote buf zg
-                    self._attn_post(l, z, n)
-            if skinny and "gu_il" in W:
-                # the residual update rides on the output projection (h = resid_attn * x + post_attn * a) and the MLP's
-                # pre-norm on the gate-up projection (a row scale of the product), whose epilogue is the SwiGLU
-                gemm_tn(b["zg"][:n], W["wo"], b["h"][:n], epilogue=RESID, resid=x, ca=W["resid_attn"], cb=W["post_attn"])
-                gemm_tn(b["h"][:n], W["gu_il"], b["act"][:n], epilogue=SWIGLU, norm_eps=self.eps)
-            elif fold_mlp:
-                # both residual updates are the library's C = alpha A B + beta C on the hidden in place and the MLP's pre-norm
-                # is the row scale inside the SwiGLU launch; the block ends with the norm the next block reads
-                torch.addmm(x, b["zg"][:n], W["wo"].t(), beta=W["resid_attn"], alpha=W["post_attn"], out=x)
-                torch.mm(x, W["gu"].t(), out=b["gu"][:n])
-                self._swiglu_norm(x, n)
-                torch.addmm(x, b["act"][:n], W["down"].t(), beta=W["resid_mlp"], alpha=W["post_mlp"], out=x)
-                if l + 1 < cfg.n_layers:
-                    self._add_norm(x, x, 1.0, 0.0, n, None, b["xn"])
-                continue
-            else:
-                mm(b["zg"][:n], W["wo"], b["a"][:n])
-                # h = resid_attn * x + post_attn * a ; n = rmsnorm(h)
-                self._add_norm(x, b["a"][:n], W["resid_attn"], W["post_attn"], n, b["h"], b["xn"])
-                mm(xn, W["gu"], b["gu"][:n])
-                self._swiglu(n)
-            torch.mm(b["act"][:n], W["down"].t(), out=b["m"][:n])   # (K = d_ff: 26 K-steps per strip, the library is faster)
-            # x = resid_mlp * h + post_mlp * m ; xn = rmsnorm(x) (next block's pre-norm, or the final norm)
-            self._add_norm(b["h"][:n], b["m"][:n], W["resid_mlp"], W["post_mlp"], n, b["x"], b["xn"])
-        return fold_mlp
-
-    # ---- recorded passes
-    def _planned(self, what: str, st: KVState, kind: str, n: int, values: dict, record) -> Tensor:
-        """Run the pass that record() makes, from its recorded launch list: recorded on the state the first time a pass of this
-        shape class runs on it (launched as it is recorded, so a state's first pass waits for nothing), then only re-bound to the call's row counts and addresses (values).  The list is recorded
-        again when an object it rests on is another one (weights, cache tensors, a switch of the launch plans)."""
-        own_down = n <= self.skinny_rows or n >= self.big_rows or self.fold_down_rows[0] <= n <= self.fold_down_rows[1]
         key = (id(self), what, kind, n <= self.fold_qkv_rows, n <= self.fold_o_rows, n <= self.fold_gu_rows, own_down,
                self.fold_down_rows[0] <= n <= self.fold_down_rows[1], self.gemm_config, getattr(self.w, "scalar_epoch", 0))
         caches = [t for t in (*st.k, *st.v, *st.k_scale, *st.v_scale) if t is not None]
