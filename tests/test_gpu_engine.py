@@ -842,3 +842,71 @@ def test_ring_of_a_short_cache_keeps_its_length(kv_dtype):
     assert a.slots(l) == 50
     outs = [eng.decode_step(tok, st).float() for st in (a, b)]
     assert float((outs[0] - outs[1]).norm() / outs[1].norm()) < 0.05   # (the generic kernel: bf16 roundings of four layers)
+
+
+_LEFT_TO_POST = {   # configurations whose attention leaves XSA and gate to the separate launch: what is not the default
+    "no-xsa": (dict(xsa=False, window=64), "int8", None), "window-48": (dict(window=48), "int8", None),
+    "other-16-bit-cache": (dict(window=64), "fp16", {torch.bfloat16: torch.float16, torch.float16: torch.bfloat16}),
+}
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("lens,nd", [((20, 15), 25), ((150, 131, 170, 144, 90, 200, 163, 155), 100)], ids=["60-rows", "1303-rows"])
+@pytest.mark.parametrize("case", list(_LEFT_TO_POST))
+def test_mixed_step_of_a_16bit_engine_whose_attention_leaves_its_epilogue(case, lens, nd, dtype):
+    """Mixed passes where prompts or decode rows leave XSA and gate to the separate launch, which forms the gate from the block's
+    normalised input: final hiddens against the same engine's prefill and decode step, and against an fp32 engine on the same
+    kind of cache.  The mixed pass is another rounding of the same function, so it may stand as far from the fp32 engine as
+    the separate passes do (half as far again: 2-norms over 2 .. 100 rows) and from these at most the two distances' root sum
+    of squares (with the same room)."""
+    from ultraviolet_amd.engine import KVState, UVEngine, UVWeights
+    over, kv, cdt = _LEFT_TO_POST[case]
+    cfg, params, eng, _ = _setup(dtype=dtype, **over)
+    cdt = dtype if cdt is None else cdt[dtype]
+    new, old = _prompts(cfg, lens, seed=6), _prompts(cfg, np.random.default_rng(1).integers(3, 70, size=nd), seed=5)
+    rows_d, rows_p = torch.arange(nd, device=DEV), list(range(nd, nd + len(new)))
+    tok = torch.from_numpy(np.random.default_rng(7).integers(1, cfg.vocab_size, size=nd)).to(DEV)
+    outs = []
+    for e, mixed in ((eng, True), (eng, False), (UVEngine(UVWeights(cfg, params, torch.float32, DEV), 8192), False)):
+        e.max_tokens = max(e.max_tokens, sum(map(len, old)))
+        if e.buf["x"].size(0) < e.max_tokens:
+            e = UVEngine(e.w, e.max_tokens)
+        st = KVState(cfg, nd + len(new), 256, DEV, kv_dtype=kv, dtype=cdt)
+        e.prefill(old, rows_d.tolist(), st, left_pad=False)
+        if mixed:
+            pk = e.pack_prompts(new, rows_p, st.max_len, left_pad=False)
+            hp, hd = e.mixed_step(pk, tok, st.pos[:nd].clone(), st.starts[:nd].clone(), rows_d, st)
+        else:
+            hp = e.prefill(new, rows_p, st, left_pad=False).clone()
+            hd = e.decode_step(torch.cat([tok, torch.zeros(len(new), dtype=torch.long, device=DEV)]), st)[:nd]
+        outs.append([t.double().cpu() for t in (hp, hd)])
+    rel = lambda a, b: float((a - b).norm() / b.norm())
+    for m, s, r in zip(*outs):
+        em, es, d = rel(m, r), rel(s, r), rel(m, s)
+        print(f"{case} {tuple(m.shape)}: mixed {em:.4f} and separate {es:.4f} from fp32, {d:.4f} from each other")
+        assert em < 1.5 * es and d < 1.5 * (2 ** 0.5) * es, (em, es, d)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_mixed_rollout_of_a_16bit_engine_whose_attention_leaves_its_epilogue(dtype):
+    """The same through Rollout(mixed=True): greedy streams against the rollout that admits in passes of its own.  Streams may part
+    at a near-tie, and do on random weights; up to there the log-probs of a stream are two roundings of one number (bars: three
+    times what the two rollouts differ by on three prompt sets with the fused epilogue, 0.017 bf16 / 0.004 fp16)."""
+    from ultraviolet_amd.engine.rollout import Rollout
+    cfg, _, eng, _ = _setup(dtype=dtype, window=64, xsa=False)
+    prompts = _prompts(cfg, np.random.default_rng(3).integers(3, 32, size=24), seed=9)
+    runs = []
+    for mixed in (False, True):
+        g = Rollout(eng, slots=6, max_prompt=32, max_new=20, temperature=0.0, check_every=3, bucket=4, mixed=mixed)
+        for i, p in enumerate(prompts):
+            g.add(p, i, limit=4 + 5 * (i % 4))
+        runs.append({m: (row, lp) for m, row, lp, _ in g.run()})
+        assert (g.n_mixed_steps > 0) == mixed
+    gap, same = 0.0, 0
+    for i in range(len(prompts)):
+        (ta, la), (tb, lb) = runs[0][i], runs[1][i]
+        k = next((j for j, (x, y) in enumerate(zip(ta, tb)) if x != y), len(ta))
+        same += k == len(ta)
+        gap = max(gap, float(np.abs(la[:k] - lb[:k]).max(initial=0.0)))
+    print(f"{same} of {len(prompts)} streams the same, log-probs within {gap:.4f} up to where they part")
+    assert same >= 0.7 * len(prompts) and gap < (0.05 if dtype == torch.bfloat16 else 0.012), (same, gap)

@@ -297,6 +297,15 @@ class UVEngine:
                                     cfg.n_kv_heads, cfg.head_dim, cfg.d_model, cfg.gate_ch, b["zg"][off:].data_ptr(), L.stream_ptr(z))
         L.check(rc, "uvmi_attn_post")
 
+    def _finish_attn(self, l: int, z, h: Tensor | None = None):
+        """What an attention (the attn of _trunk) left undone: XSA + gate of the rows it returned.  The gate is a product of the
+        block's normalised input, buf xn; h: the block's input, where a plan has not written its norm there."""
+        parts = [(off, z) for off, z in (z if isinstance(z, list) else [(0, z)]) if z is not None and z.size(0)]
+        if parts and h is not None and self.w.layers[l]["attn_gate"] is not None:
+            self._add_norm(h, h, 1.0, 0.0, h.size(0), None, self.buf["xn"])
+        for off, z in parts:
+            self._attn_post(l, z, z.size(0), off)
+
     def _swiglu(self, n: int):
         b = self.buf
         rc = L.lib().uvmi_swiglu(b["gu"].data_ptr(), self.dt_code, n, self.cfg.d_ff, b["act"].data_ptr(), L.stream_ptr(b["gu"]))
@@ -415,10 +424,10 @@ class UVEngine:
 
     def _trunk(self, tok: Tensor, pos: Tensor, n: int, attn, rows=None, last_pos=None, st: KVState | None = None,
                fused_attn=None, defer_final_norm: bool = False, advance: bool = False, final_norm: bool = True) -> Tensor:
-        """n token rows through all layers; attn(l, q (n, H, hd)) -> z (n, H, hd) (or None when it wrote the post-processed
-        result to buf zg itself) runs after K/V of the layer have been appended to the cache and written unquantized to
-        buf k / v.  Returns the final normed hidden (n, d) (a buffer).  defer_final_norm: a plan whose last block leaves the
-        hidden un-normalised returns it as it is and sets self.hidden_is_raw - the caller's head GEMM then carries the final
+        """n token rows through all layers; attn(l, q (n, H, hd)) -> z (n, H, hd), or None when it wrote the post-processed
+        result to buf zg itself, or a list of (first row, z) of the parts that it left to _attn_post; it runs after K/V of the
+        layer have been appended to the cache and written unquantized to buf k / v.  Returns the final normed hidden (n, d) (a
+        buffer).  defer_final_norm: a plan whose last block leaves the hidden un-normalised returns it as it is and sets self.hidden_is_raw - the caller's head GEMM then carries the final
         norm as the row scale of its product (head_of), and the norm launch goes away; final_norm False: likewise at any row
         count, for a caller that norms the few rows it needs itself (_normed).  advance: the final norm's launch counts pos up
         by one."""
@@ -536,8 +545,8 @@ class UVEngine:
         """Prompts, mixed passes and the unfused attention of a 16-bit engine: the extended projection with the pre-norm in it,
         the post-processing kernel (which takes the gates' logits from the projection and appends to the cache), the
         attention launches, output and down projections with the residual update in place, gate-up with the pre-norm and
-        the SwiGLU.  The normalised hidden is not written between blocks (it is formed on demand for a layer whose attention
-        leaves its epilogue to _attn_post)."""
+        the SwiGLU.  The normalised hidden is not written between blocks (_finish_attn forms it for a layer whose attention
+        leaves its epilogue to _attn_post; layer 0 has the embedding's)."""
         cfg, b = self.cfg, self.buf
         x, zg, act = b["x"][:n], b["zg"][:n], b["act"][:n]
         gc = self.gemm_config
@@ -545,11 +554,7 @@ class UVEngine:
         for l, W in enumerate(self.w.layers):
             self._project_qkv(l, n, n <= self.fold_qkv_rows, config=gc)
             self._qkv_post(l, tok, pos, rows, last_pos, st, n, ext=True)
-            z = attn(l, b["q"][:n])
-            if z is not None:
-                if l > 0:
-                    self._add_norm(x, x, 1.0, 0.0, n, None, b["xn"])
-                self._attn_post(l, z, n)
+            self._finish_attn(l, attn(l, b["q"][:n]), x if l > 0 else None)
             self._gemm(zg, W["wo"], x, RESID, resid=x, ca=W["resid_attn"], cb=W["post_attn"], config=gc)
             self._gemm(x, W["gu_il"], act, SWIGLU, norm_eps=self.eps, config=gc)
             self._down(l, n, own_down)
@@ -574,9 +579,7 @@ class UVEngine:
             else:
                 mm(xn, W["wqkv"], b["qkv"][:n])
                 self._qkv_post(l, tok, pos, rows, last_pos, st, n)
-                z = attn(l, b["q"][:n])
-                if z is not None:   # None: the attention kernel already applied XSA + gate and wrote buf zg
-                    self._attn_post(l, z, n)
+                self._finish_attn(l, attn(l, b["q"][:n]))
             if skinny and "gu_il" in W:
                 # the residual update rides on the output projection (h = resid_attn * x + post_attn * a) and the MLP's
                 # pre-norm on the gate-up projection (a row scale of the product), whose epilogue is the SwiGLU
@@ -834,13 +837,8 @@ class UVEngine:
         pos_d, rows_d = pos[Np:N], rows[Np:N]
 
         def attn(l, q):
-            zp = self.prompt_attention(l, q[:Np], Np, cu)
-            if zp is not None:
-                self._attn_post(l, zp, Np)
-            zd = self.cache_attention(l, q[Np:N], st, pos_d, starts_d, nd, rows=rows_d, off=Np)
-            if zd is not None:
-                self._attn_post(l, zd, nd, off=Np)
-            return None
+            return [(0, self.prompt_attention(l, q[:Np], Np, cu)),
+                    (Np, self.cache_attention(l, q[Np:N], st, pos_d, starts_d, nd, rows=rows_d, off=Np))]
 
         run = lambda: self._trunk(tok[:N], pos[:N], N, attn, rows=rows[:N], last_pos=last[:N], st=st, final_norm=final_norm)
         if (Np > 0 and nd > 0 and self._pass_kind(N, False, st) == "packed" and self.prompt_attention_plannable() and self._append_fused(st)
