@@ -910,3 +910,41 @@ def test_mixed_rollout_of_a_16bit_engine_whose_attention_leaves_its_epilogue(dty
         gap = max(gap, float(np.abs(la[:k] - lb[:k]).max(initial=0.0)))
     print(f"{same} of {len(prompts)} streams the same, log-probs within {gap:.4f} up to where they part")
     assert same >= 0.7 * len(prompts) and gap < (0.05 if dtype == torch.bfloat16 else 0.012), (same, gap)
+
+
+@pytest.mark.parametrize("what", ["replaced", "moved", "scalar"])
+def test_recorded_passes_see_weights_that_changed_under_the_engine(what):
+    """A weight tensor replaced in the engine's layers, one whose storage moved, a residual scalar written there: the next pass on
+    a state with recorded launch lists gives what a state without any gives, bit for bit.  (The old storage stays alive: a
+    list that still reads it reads the old values.)"""
+    from ultraviolet_amd.engine import KVState
+    cfg, _, eng, _ = _setup(dtype=torch.bfloat16, window=64)
+    names = [k for k, v in eng.w.layers[1].items() if (isinstance(v, float) if what == "scalar" else isinstance(v, torch.Tensor))]
+    tok, alive = torch.tensor([5, 9, 2], device=DEV), []
+    old = KVState(cfg, 5, 96, DEV)
+
+    def passes(st):
+        hs = [eng.prefill([[3, 4, 5], [6] * 9, [7]], [0, 1, 2], st), eng.decode_step(tok, st)]
+        pk = eng.pack_prompts([[8, 9], [1, 2, 3]], [3, 4], 96)
+        return [h.clone() for h in (*hs, *eng.mixed_step(pk, tok, st.pos[:3].clone(), st.starts[:3].clone(), torch.arange(3, device=DEV), st))]
+
+    tables = [(eng.w, "embed"), (eng.w, "value_embed")] if what == "moved" else []
+    first = passes(old)
+    seen = 0
+    for W, name in [(eng.w.layers[1], n) for n in names] + tables:
+        get, put = (W.__getitem__, W.__setitem__) if isinstance(W, dict) else (lambda n: getattr(W, n), None)
+        v = get(name)
+        alive.append(v)
+        if what == "scalar":
+            put(name, v * 1.5)
+        elif what == "replaced":
+            put(name, v * 1.5)
+        else:
+            alive[-1] = v.data
+            v.data = v.data * 1.5
+        new = KVState(cfg, 5, 96, DEV)
+        a, b = passes(old), passes(new)
+        assert all(torch.equal(x, y) for x, y in zip(a, b)), name
+        seen += not all(torch.equal(x, y) for x, y in zip(a, first))
+        first = a
+    assert seen >= 4   # (some weights are read by the other plans only)

@@ -10,6 +10,7 @@ model.py:1099-1100)."""
 from __future__ import annotations
 
 import ctypes as C
+from itertools import chain
 
 import numpy as np
 import torch
@@ -22,7 +23,7 @@ from ..kernels.kv_quant import kv_write
 from ..kernels.varlen_attn import packed_attention, packed_attention_args
 from ..kernels.fused_sample import fused_sample_seeded, greedy_sample
 from .config import UVConfig
-from .plan import PassPlan, launch
+from .plan import Guard, PassPlan, launch
 from .weights import UVWeights
 
 
@@ -611,25 +612,24 @@ class UVEngine:
         """Run the pass that record() makes, from its recorded launch list: recorded on the state the first time a pass of this
         shape class runs on it (launched as it is recorded, so that a state's first pass waits for nothing), then only re-bound to
         the call's row counts and addresses (values).  The list is recorded again when an object it rests on is another one or
-        elsewhere (weights, cache tensors, a switch of the launch plans)."""
+        elsewhere (weights and residual scalars, cache tensors, a switch of the launch plans)."""
         own_down = n <= self.skinny_rows or n >= self.big_rows or self.fold_down_rows[0] <= n <= self.fold_down_rows[1]
         key = (id(self), what, kind, n <= self.fold_qkv_rows, n <= self.fold_o_rows, n <= self.fold_gu_rows, own_down,
                self.fold_down_rows[0] <= n <= self.fold_down_rows[1], self.gemm_config, getattr(self.w, "scalar_epoch", 0))
-        caches = [t for t in (*st.k, *st.v, *st.k_scale, *st.v_scale) if t is not None]
-        guard = (self.w, *caches)
+        w = self.w
+        rests_on = (w.embed, w.value_embed, w.inv_freq, *chain.from_iterable(map(dict.values, w.layers)), *st.k, *st.v, *st.k_scale, *st.v_scale)
         plans = st.__dict__.setdefault("_pass_plans", {})
         plan = plans.get(key)
-        at = tuple(map(Tensor.data_ptr, caches))   # (a cache may keep its object and move, as with `.data = `)
-        if plan is None or len(plan.guard) != len(guard) or any(a is not b for a, b in zip(plan.guard, guard)) or plan.at != at:
+        if plan is None or not plan.guard.holds(rests_on):
             if len(plans) >= 16:
                 plans.clear()
             plan = PassPlan()
+            plan.guard = Guard(rests_on)
             self._rec = plan
             try:
                 record()
             finally:
                 self._rec = None
-            plan.guard, plan.at = guard, at
             plan.engine = self          # (keeps id(self) from being reused while the plan lives)
             plan.raw = self.hidden_is_raw
             plans[key] = plan.close()

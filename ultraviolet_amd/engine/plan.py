@@ -7,8 +7,25 @@ results: every launch runs on every call."""
 from __future__ import annotations
 
 import ctypes as C
+from operator import is_
+
+from torch import Tensor
 
 from .. import _lib as L
+
+
+class Guard:
+    """The objects that recorded launches took addresses and numbers from - weights, residual scalars, cache tensors - and where the
+    tensors among them were: one may be replaced, or keep its object and move (`.data = `)."""
+
+    def __init__(self, objects):
+        self.objects = tuple(objects)
+        self.tensors = [t for t in self.objects if isinstance(t, Tensor)]
+        self.at = list(map(Tensor.data_ptr, self.tensors))
+
+    def holds(self, objects) -> bool:
+        objects = tuple(objects)
+        return len(objects) == len(self.objects) and all(map(is_, self.objects, objects)) and list(map(Tensor.data_ptr, self.tensors)) == self.at
 
 
 class PassPlan:
@@ -17,8 +34,7 @@ class PassPlan:
         self.keep = []      # what the argument blocks point into
         self.fields = {}    # name of a per-call value -> [(struct, field)] that hold it
         self.bound = {}     # the values they hold now
-        self.guard = ()     # objects whose identity the recorded addresses rest on
-        self.at = ()        # the addresses of those that a caller could move
+        self.guard = None   # Guard of what the recorded arguments were taken from
 
     def op(self, kind: int, args, keep=(), **per_call):
         """A launch; per_call: field of args (or (struct, field)) = name of the per-call value it holds."""
