@@ -948,3 +948,43 @@ def test_recorded_passes_see_weights_that_changed_under_the_engine(what):
         seen += not all(torch.equal(x, y) for x, y in zip(a, first))
         first = a
     assert seen >= 4   # (some weights are read by the other plans only)
+
+
+@pytest.mark.parametrize("plan", ["small", "large-library"])
+def test_states_and_engines_are_copied_pickled_and_freed_after_use(plan):
+    """A state that passes have run on: copy.copy, copy.deepcopy and pickle give states that go on as it does, bit for bit; so does a
+    deep copy of the engine.  Recorded passes keep neither alive: a state's caches go with it, the engine's buffers with the
+    engine, also while the other lives."""
+    import copy
+    import gc
+    import pickle
+    import weakref
+    from ultraviolet_amd.engine import KVState
+    cfg, _, eng, _ = _setup(dtype=torch.bfloat16, window=64)
+    _force_plan(eng, plan)
+    st = KVState(cfg, 3, 96, DEV)
+    tok = torch.tensor([5, 9, 2], device=DEV)
+    eng.prefill([[3, 4, 5], [6] * 9, [7]], [0, 1, 2], st)
+    eng.decode_step(tok, st)
+    eng2, states = copy.deepcopy(eng), [copy.deepcopy(st), pickle.loads(pickle.dumps(st))]
+    h = eng.decode_step(tok, st).clone()
+    for i, other in enumerate(states):
+        assert other.k[0].data_ptr() != st.k[0].data_ptr()
+        same = torch.equal((eng, eng2)[i].decode_step(tok, other), h) and torch.equal(other.pos, st.pos)
+        assert same, i
+        assert all(torch.equal(a, b) for a, b in zip(other.k + other.v, st.k + st.v))
+    twin = copy.copy(st)                       # (shares the caches)
+    h = eng.decode_step(tok, st).clone()
+    twin.pos.sub_(1)
+    same = torch.equal(eng.decode_step(tok, twin), h)
+    assert same
+    torch.cuda.synchronize()
+    gc.collect()
+    gc.disable()
+    try:
+        dead_state, dead_engine = weakref.ref(states[1].k[0]), weakref.ref(eng2.buf["x"])
+        del other, states[1], eng2
+        assert dead_state() is None and dead_engine() is None
+    finally:
+        gc.enable()
+    assert torch.isfinite(eng.decode_step(tok, states[0]).float()).all()

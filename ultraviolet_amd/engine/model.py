@@ -10,6 +10,7 @@ model.py:1099-1100)."""
 from __future__ import annotations
 
 import ctypes as C
+import weakref
 from itertools import chain
 
 import numpy as np
@@ -125,6 +126,12 @@ class _Stage:
             pass
 
 
+def _swiglu_norm(b: dict, h: Tensor, n: int, dt_code: int, cfg: UVConfig, eps: float):
+    """UVEngine._swiglu_norm on the engine's buffers b."""
+    rc = L.lib().uvmi_swiglu_norm(b["gu"].data_ptr(), h.data_ptr(), dt_code, n, cfg.d_ff, cfg.d_model, eps, b["act"].data_ptr(), L.stream_ptr(h))
+    L.check(rc, "uvmi_swiglu_norm")
+
+
 class UVEngine:
     def __init__(self, weights: UVWeights, max_tokens: int, skinny_rows: int = 192, fold_qkv_rows: int = 1 << 30, fold_o_rows: int = 1 << 30,
                  fold_gu_rows: int = 1 << 30, lean: bool = True, fold: bool = True, gemm_config: int = 0,
@@ -176,12 +183,24 @@ class UVEngine:
         self.fold_down_rows = (int(fold_down_rows[0]), int(fold_down_rows[1]))
         self.head_own_rows = 288       # decode steps of at most this many rows run the head GEMM on this library's kernel (own_head_ok)
         self.hidden_is_raw = False
-        self._stage, self._stage_at = [_Stage() for _ in range(2)], 0   # (_staging)
-        self._rec = None               # the PassPlan being recorded (None: operations are launched as they come)
+        self._new_scratch()
         self._rope_tabs: dict[int, Tensor] = {}  # rotation tables by position count, kept for the engine's life (graphs hold them)
         if self.fuse_qkv:
             self.buf["qkvx"] = e(n, UVWeights.qkv_ext_rows(cfg))
         self.pf_ws = torch.empty(L.lib().uvmi_prefill_attn_workspace_bytes(n), dtype=torch.uint8, device=dev)  # fails now if the library is missing
+
+    def _new_scratch(self):
+        """What belongs to this object and this process, and no copy takes along: staging memory and recorded passes."""
+        self._stage, self._stage_at = [_Stage() for _ in range(2)], 0   # (_staging)
+        self._plans = weakref.WeakKeyDictionary()   # per state its recorded passes (_planned), for as long as it lives
+        self._rec = None               # the PassPlan being recorded (None: operations are launched as they come)
+
+    def __getstate__(self):
+        return {k: v for k, v in self.__dict__.items() if k not in ("_stage", "_stage_at", "_plans", "_rec")}
+
+    def __setstate__(self, d):
+        self.__dict__.update(d)
+        self._new_scratch()
 
     # ------------------------------------------------------------------------------------------------ kernels
     # An operation is launched at once and, while a plan is being recorded (_planned), appended to it, where the names given for its
@@ -193,7 +212,8 @@ class UVEngine:
             self._rec.op(kind, args, keep, **per_call)
 
     def _lib_gemm(self, n: int, fn):
-        """A GEMM of the vendor library on the first n rows of the engine's buffers: fn(n)."""
+        """A GEMM of the vendor library on the first n rows of the engine's buffers: fn(n), which does not hold the engine (a
+        recorded list keeps it, and the engine keeps the lists)."""
         fn(n)
         if self._rec is not None:
             self._rec.call(lambda values: fn(values["n"]))
@@ -314,10 +334,7 @@ class UVEngine:
 
     def _swiglu_norm(self, h: Tensor, n: int):
         """buf act = SwiGLU of rmsnorm(h) @ gu.T, from buf gu = h @ gu.T (the norm as a row scale of the product)."""
-        b = self.buf
-        rc = L.lib().uvmi_swiglu_norm(b["gu"].data_ptr(), h.data_ptr(), self.dt_code, n, self.cfg.d_ff, self.cfg.d_model, self.eps,
-                                      b["act"].data_ptr(), L.stream_ptr(h))
-        L.check(rc, "uvmi_swiglu_norm")
+        _swiglu_norm(self.buf, h, n, self.dt_code, self.cfg, self.eps)
 
     # ------------------------------------------------------------------------------------------------ trunk
     def cache_attention_plannable(self, l: int, st: KVState) -> bool:
@@ -512,7 +529,7 @@ class UVEngine:
         residual update (the vendor library's C = alpha A B + beta C outside fold_down_rows)."""
         cfg, b = self.cfg, self.buf
         x, zg, act = b["x"][:n], b["zg"][:n], b["act"][:n]
-        gc = self.gemm_config
+        gc, dt_code, eps = self.gemm_config, self.dt_code, self.eps
         sk_ok = cfg.d_model % 64 == 0 and (cfg.n_heads * cfg.head_dim) % 64 == 0
         sk_qkv, sk_o = sk_ok and n <= self.fold_qkv_rows, sk_ok and n <= self.fold_o_rows
         for l, W in enumerate(self.w.layers):
@@ -529,7 +546,7 @@ class UVEngine:
             else:
                 def gate_up(n, W=W):
                     torch.mm(b["x"][:n], W["gu"].t(), out=b["gu"][:n])
-                    self._swiglu_norm(b["x"][:n], n)
+                    _swiglu_norm(b, b["x"][:n], n, dt_code, cfg, eps)
                 self._lib_gemm(n, gate_up)
             # x <- resid_mlp * x + post_mlp * (act @ down.T)
             self._down(l, n, sk_ok and self.fold_down_rows[0] <= n <= self.fold_down_rows[1] and cfg.d_ff % 64 == 0)
@@ -609,16 +626,16 @@ class UVEngine:
 
     # ---- recorded passes
     def _planned(self, what: str, st: KVState, kind: str, n: int, values: dict, record) -> Tensor:
-        """Run the pass that record() makes, from its recorded launch list: recorded on the state the first time a pass of this
-        shape class runs on it (launched as it is recorded, so that a state's first pass waits for nothing), then only re-bound to
+        """Run the pass that record() makes, from its recorded launch list: recorded the first time a pass of this
+        shape class runs on the state (launched as it is recorded, so that a state's first pass waits for nothing), then only re-bound to
         the call's row counts and addresses (values).  The list is recorded again when an object it rests on is another one or
         elsewhere (weights and residual scalars, cache tensors, a switch of the launch plans)."""
         own_down = n <= self.skinny_rows or n >= self.big_rows or self.fold_down_rows[0] <= n <= self.fold_down_rows[1]
-        key = (id(self), what, kind, n <= self.fold_qkv_rows, n <= self.fold_o_rows, n <= self.fold_gu_rows, own_down,
+        key = (what, kind, n <= self.fold_qkv_rows, n <= self.fold_o_rows, n <= self.fold_gu_rows, own_down,
                self.fold_down_rows[0] <= n <= self.fold_down_rows[1], self.gemm_config, getattr(self.w, "scalar_epoch", 0))
         w = self.w
         rests_on = (w.embed, w.value_embed, w.inv_freq, *chain.from_iterable(map(dict.values, w.layers)), *st.k, *st.v, *st.k_scale, *st.v_scale)
-        plans = st.__dict__.setdefault("_pass_plans", {})
+        plans = self._plans.setdefault(st, {})
         plan = plans.get(key)
         if plan is None or not plan.guard.holds(rests_on):
             if len(plans) >= 16:
@@ -630,7 +647,6 @@ class UVEngine:
                 record()
             finally:
                 self._rec = None
-            plan.engine = self          # (keeps id(self) from being reused while the plan lives)
             plan.raw = self.hidden_is_raw
             plans[key] = plan.close()
         else:
