@@ -41,7 +41,7 @@ extern "C" {
 #define UVMI_I64 5
 
 /* Revision of the argument structs below (uvmi_version() returns the value the library was built with). */
-#define UVMI_ABI_VERSION 5
+#define UVMI_ABI_VERSION 6
 int uvmi_version(void);
 const char* uvmi_last_error(void);
 /* Number of compute units of the current device (used by the split heuristics); <0 on error. */
@@ -490,7 +490,9 @@ int uvmi_sched_expand(const uvmi_sched_state* s, int n_adm, int n_tokens, const 
  * tok_d, pos_d, rows_d, and pos_d once more as their last position.  last_idx[a] = cu[a + 1] - 1.  Optional outputs (NULL: not
  * written): pos_t with tok_t, row_t and last_t, last_idx, the state's st_pos / st_starts of the rows, device copies of cu, row,
  * start and of the prompts' end positions, and check_out = check_in[0 .. n).  cu, row, start, tok and check_out may be pinned host
- * memory (n <= 2047 then): the launch reads a small table where the host wrote it, and a copy of its own would cost more. */
+ * memory (n <= 2047 then): the launch reads a small table where the host wrote it, and a copy of its own would cost more.
+ * check_zero: prompts whose check_in is not zero are refused: st_pos and st_starts of their rows stay, and their row_t is -1,
+ * which no launch of the pass appends to (the host learns of it from check_out, while the pass runs). */
 struct uvmi_prompt_tables_args {
   int n, n_tokens, nd; int64_t idx_ld;
   const int64_t* cu; const int64_t* row; const int64_t* start; const int64_t* tok;
@@ -498,7 +500,7 @@ struct uvmi_prompt_tables_args {
   int64_t* tok_t; int64_t* pos_t; int64_t* row_t; int64_t* last_t; int64_t* last_idx;
   int64_t* st_pos; int64_t* st_starts;
   int64_t* cu_out; int64_t* row_out; int64_t* start_out; int64_t* end_out;
-  const int64_t* check_in; int64_t* check_out;
+  const int64_t* check_in; int64_t* check_out; int check_zero;
 };
 int uvmi_prompt_tables(const struct uvmi_prompt_tables_args* a, void* stream);
 

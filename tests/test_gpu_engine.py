@@ -988,3 +988,25 @@ def test_states_and_engines_are_copied_pickled_and_freed_after_use(plan):
     finally:
         gc.enable()
     assert torch.isfinite(eng.decode_step(tok, states[0]).float()).all()
+
+
+@pytest.mark.parametrize("dtype,kv", [(torch.bfloat16, "int8"), (torch.bfloat16, "fp16"), (torch.float32, "int8")])
+def test_a_refused_single_prompt_leaves_the_state_alone(dtype, kv):
+    """prefill of one prompt that does not fill its row raises, whichever way its start is off, and cache row, scales, pos, starts and
+    host_pos stay; the same call with a good start goes on."""
+    from ultraviolet_amd.kernels import fast_decode as fd
+    cfg, params, _, _ = _setup(window=32)
+    m = fd.patch_model(_StubModel(cfg, params), kv_dtype=kv, dtype=dtype, max_tokens=512)
+    st = m.new_state(3, 48)
+    m.prefill(torch.arange(1, 31, device=DEV).view(3, 10), torch.zeros(3, dtype=torch.long, device=DEV), st)
+    m.decode_step(torch.tensor([3, 4, 5], device=DEV), st)
+    tensors = [t for t in st.k + st.v + st.k_scale + st.v_scale if t is not None] + [st.pos, st.starts]
+    before, host = [t.clone() for t in tensors], st.host_pos.copy()
+    idx, rows = torch.arange(40, 61, device=DEV)[None], torch.tensor([1], device=DEV)
+    for bad in (3, -2):
+        with pytest.raises(AssertionError, match="must fill all T columns"):
+            m.prefill(idx, torch.tensor([bad], device=DEV), st, rows=rows)
+        torch.cuda.synchronize()
+        assert all([torch.equal(a, b) for a, b in zip(before, tensors)]) and np.array_equal(st.host_pos, host)
+    m.prefill(idx, torch.zeros(1, dtype=torch.long, device=DEV), st, rows=rows)
+    assert st.pos.tolist() == [11, 21, 11] and st.host_pos.tolist() == [11, 21, 11] and not torch.equal(before[0][1], st.k[0][1])

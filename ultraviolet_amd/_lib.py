@@ -135,13 +135,13 @@ class PromptTablesArgs(C.Structure):   # struct uvmi_prompt_tables_args
                 ("tok_t", C.c_void_p), ("pos_t", C.c_void_p), ("row_t", C.c_void_p), ("last_t", C.c_void_p), ("last_idx", C.c_void_p),
                 ("st_pos", C.c_void_p), ("st_starts", C.c_void_p),
                 ("cu_out", C.c_void_p), ("row_out", C.c_void_p), ("start_out", C.c_void_p), ("end_out", C.c_void_p),
-                ("check_in", C.c_void_p), ("check_out", C.c_void_p)]
+                ("check_in", C.c_void_p), ("check_out", C.c_void_p), ("check_zero", C.c_int)]
 
 
 OP_GEMM, OP_DECODE_ATTN, OP_QKV_POST, OP_PREFILL_ATTN, OP_NORM = range(5)   # UVMI_OP_*
 
 _lib = None
-ABI_VERSION = 5   # UVMI_ABI_VERSION of include/uvmi.h
+ABI_VERSION = 6   # UVMI_ABI_VERSION of include/uvmi.h
 
 
 def lib() -> C.CDLL:

@@ -355,10 +355,11 @@ __global__ __launch_bounds__(256) void prompt_tables_kernel(uvmi_prompt_tables_a
   auto cu = [&](int a) -> int64_t { return lds ? scu[a] : A.cu[a]; };
   auto row = [&](int a) -> int64_t { return lds ? srow[a] : A.row[a]; };
   auto start = [&](int a) -> int64_t { return lds ? sst[a] : A.start[a]; };
+  auto refused = [&](int a) -> bool { return A.check_zero && A.check_in[a] != 0; };
   if (i < A.n) {
     const int64_t b = cu(i), e = cu(i + 1), r = row(i), s = start(i);
     if (A.last_idx) A.last_idx[i] = e - 1;
-    if (A.st_pos) {
+    if (A.st_pos && !refused(i)) {
       A.st_starts[r] = s;
       A.st_pos[r] = s + e - b;
     }
@@ -383,7 +384,7 @@ __global__ __launch_bounds__(256) void prompt_tables_kernel(uvmi_prompt_tables_a
   }
   const int64_t b = cu(lo), e = cu(lo + 1), s = start(lo);
   A.tok_t[i] = A.idx_ld > 0 ? A.tok[lo * A.idx_ld + A.idx_ld - (e - i)] : t_own;
-  A.pos_t[i] = s + i - b; A.row_t[i] = row(lo); A.last_t[i] = s + e - b - 1;
+  A.pos_t[i] = s + i - b; A.row_t[i] = refused(lo) ? -1 : row(lo); A.last_t[i] = s + e - b - 1;
 }
 
 }  // namespace uvmi
@@ -497,6 +498,7 @@ extern "C" int uvmi_prompt_tables(const uvmi_prompt_tables_args* a, void* stream
   UVMI_REQUIRE(!a->st_pos == !a->st_starts, UVMI_EINVAL, "uvmi_prompt_tables: st_pos and st_starts go together");
   UVMI_REQUIRE(!a->cu_out || (a->row_out && a->start_out && a->end_out), UVMI_EINVAL, "uvmi_prompt_tables: incomplete copies of the prompt table");
   UVMI_REQUIRE(!a->check_out || a->check_in, UVMI_EINVAL, "uvmi_prompt_tables: check_out without check_in");
+  UVMI_REQUIRE(!a->check_zero || a->check_in, UVMI_EINVAL, "uvmi_prompt_tables: check_zero without check_in");
   if (a->pos_t) {
     UVMI_REQUIRE(a->tok_t && a->row_t && a->last_t && (a->n_tokens == 0 || a->tok), UVMI_EINVAL, "uvmi_prompt_tables: null token table");
     UVMI_REQUIRE(a->nd == 0 || (a->tok_d && a->pos_d && a->rows_d), UVMI_EINVAL, "uvmi_prompt_tables: null decode rows");

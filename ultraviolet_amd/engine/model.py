@@ -749,10 +749,10 @@ class UVEngine:
         return st.buf, st.event
 
     def _pack(self, prompts, rows, max_len: int, left_pad: bool, st: KVState | None = None, idx: Tensor | None = None, lens=None,
-              check: Tensor | None = None) -> dict:
+              check: Tensor | None = None, check_zero: bool = False) -> dict:
         """pack_prompts; st: also bind its rows to the prompts; idx (n, T) with lens instead of prompts: right-aligned prompts
         already on the device; check: n int64 of the device that the caller wants to see: pk["check"]() waits for this launch
-        and gives them.  The launch reads the host's tables in pinned memory: a copy to the device would make the host wait
+        and gives them; check_zero: prompts whose entry is not zero leave the state as it is.  The launch reads the host's tables in pinned memory: a copy to the device would make the host wait
         for the passes still running (pageable memory) or cost the GPU 20 us (pinned memory)."""
         if idx is None:
             lens = np.fromiter((len(p) for p in prompts), dtype=np.int64, count=len(prompts))
@@ -789,7 +789,7 @@ class UVEngine:
             a.st_pos, a.st_starts = st.pos.data_ptr(), st.starts.data_ptr()
         if check is not None:
             assert pinned and check.dtype == torch.int64 and check.is_contiguous() and check.numel() == n
-            a.check_in, a.check_out = check.data_ptr(), src + 8 * (3 * n + 1)
+            a.check_in, a.check_out, a.check_zero = check.data_ptr(), src + 8 * (3 * n + 1), int(check_zero)
 
             def seen():
                 ev.synchronize()
@@ -880,10 +880,11 @@ class UVEngine:
     @torch.no_grad()
     def prefill_matrix(self, idx: Tensor, lens, rows, st: KVState, check: Tensor | None = None):
         """prefill(left_pad=True) of the prompts that stand right-aligned in idx (n, T), an int64 matrix on the engine's device: the
-        last lens[a] (host) tokens of row a.  The token ids never visit the host.  check: also returns a function that gives
-        these n int64 of the device without waiting for the pass."""
+        last lens[a] (host) tokens of row a.  The token ids never visit the host.  check: n int64 of the device that have to be
+        zero; also returns a function that gives them without waiting for the pass.  A prompt whose entry is not zero leaves
+        the state as it is - cache row, pos and starts -, so the caller may raise when it sees that."""
         assert idx.dtype == torch.int64 and idx.is_contiguous() and idx.size(0) == len(lens) and idx.size(1) >= int(lens.max())
-        pk = self._pack(None, rows, st.max_len, True, st, idx, lens, check)
+        pk = self._pack(None, rows, st.max_len, True, st, idx, lens, check, check_zero=check is not None)
         h = self._prefill(pk, st)
         return h if check is None else (h, pk["check"])
 

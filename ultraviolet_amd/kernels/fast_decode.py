@@ -138,7 +138,8 @@ def prefill_fast(self, idx: Tensor, starts: Tensor, st: KVState, rows: Tensor | 
     idx = idx.to(eng.device, torch.int64).contiguous()
     if n == 1 and starts.is_cuda and starts.dtype == torch.int64 and starts.is_contiguous():
         # One prompt has to fill its row, so its length needs no word from the device: the pass is launched first, and `starts`,
-        # which the pass's first launch leaves in host memory, is checked behind it.  (Waiting for it first leaves the GPU idle
+        # which the pass's first launch leaves in host memory, is checked behind it (where it is not zero, that launch keeps the pass
+        # away from the state).  (Waiting for it first leaves the GPU idle
         # for 90 us of a 93-token prefill's 460.)
         h, seen = eng.prefill_matrix(idx, np.array([T]), rows_l, st, check=starts)
         lg = eng.logits(h)
