@@ -41,7 +41,7 @@ extern "C" {
 #define UVMI_I64 5
 
 /* Revision of the argument structs below (uvmi_version() returns the value the library was built with). */
-#define UVMI_ABI_VERSION 6
+#define UVMI_ABI_VERSION 7
 int uvmi_version(void);
 const char* uvmi_last_error(void);
 /* Number of compute units of the current device (used by the split heuristics); <0 on error. */
@@ -125,6 +125,8 @@ typedef struct uvmi_attn_args {
   const float* post_xsa;                   /* (H,) tanh(alpha) fp32, or NULL */
   int post_round_dtype;                    /* activation dtype whose rounding the epilogue follows (F16 / BF16 / F32) */
   const struct uvmi_attn_qkv_fuse* fuse;   /* optional: take q and the row's own key from the projection output (below) */
+  int any_ring;                            /* the fused epilogue and the fused post-processing take a ring of any S >= 32 (else S % 32
+                                              must be 0), with products, probabilities and sums of 32 bits; needs out_dtype == q_dtype */
 } uvmi_attn_args;
 
 /* Fused QKV post-processing for decode rows (uvmi_attn_args.fuse).  The attention kernel then does what uvmi_qkv_post

@@ -812,36 +812,58 @@ def test_packed_prompt_tables_match_their_definition(n, hi, left_pad):
 
 @pytest.mark.parametrize("kv_dtype", ["int8", "fp16"])
 def test_ring_of_a_short_cache_keeps_its_length(kv_dtype):
-    """A ring that a short max_len cuts below the window has max_len slots for its user (their fills and copies see no other
-    shape) and runs on whole tiles: prefill, steps and row copies give what a state of whole tiles gives bit for bit, and a
-    state whose tensors are replaced runs on those."""
-    from ultraviolet_amd.engine import KVState
-    cfg, _, eng, _ = _setup(dtype=torch.bfloat16, window=64)
+    """A ring that a short max_len cuts below the window has max_len slots, in tensors like every other cache's: contiguous (they
+    can be viewed and kv_written through flat indices), counted by nbytes, and all there is - a state rebuilt from its tensors goes on
+    bit for bit, also at positions between max_len and the global caches' rounded length.  Prefill, steps and row copies write
+    the bytes that a state of whole tiles gets in layer 0, and are as far from an fp32 engine as that state's are."""
+    from ultraviolet_amd.engine import KVState, UVEngine, UVWeights
+    from ultraviolet_amd.kernels import kv_write
+    cfg, params, eng, _ = _setup(dtype=torch.bfloat16, window=64)
+    e32 = UVEngine(UVWeights(cfg, params, torch.float32, DEV), 256)
     prompts, B = _prompts(cfg, (40, 3, 33), seed=4), 5
-    a, b = (KVState(cfg, B, n, DEV, kv_dtype=kv_dtype, dtype=torch.bfloat16) for n in (50, 64))
+    a, b, r = (KVState(cfg, B, n, DEV, kv_dtype=kv_dtype, dtype=torch.bfloat16) for n in (50, 64, 64))
     l = [i for i in range(cfg.n_layers) if not cfg.is_global(i)][0]
-    assert a.k[l].size(2) == a.v[l].size(2) == a.local_len == 50 and a.slots(l) == 64 and b.slots(l) == 64 and a.max_len == 64
-    for st in (a, b):
+    assert a.k[l].size(2) == a.v[l].size(2) == a.local_len == a.slots(l) == 50 and b.slots(l) == 64 and a.max_len == 64
+    tensors = lambda st: [t for t in st.k + st.v + st.k_scale + st.v_scale if t is not None]
+    assert all(t.is_contiguous() for t in tensors(a)) and a.nbytes() == sum(t.numel() * t.element_size() for t in tensors(a))
+    kv_write(a.k[l], a.k_scale[l], torch.tensor([4 * 50 + 49], device=DEV), torch.full((1, 64), 3.0, dtype=torch.bfloat16, device=DEV))
+    assert bool((a.k[l].view(-1, 64)[4 * 50 + 49] != 0).all()) and int((a.k[l] != 0).sum()) == 64
+    for st in (a, b, r):
         g = torch.Generator(device=DEV).manual_seed(7)
         st.k[l][:, :, :50] = torch.randint(-5, 6, st.k[l][:, :, :50].shape, generator=g, device=DEV).to(st.k[l].dtype)
+    rel = lambda x, y: float((x.float() - y.float()).norm() / y.float().norm())
+    tok = torch.arange(B, device=DEV) + 9
     for step in range(4):
         if step == 0:
-            outs = [eng.prefill(prompts, [2, 0, 1], st, left_pad=False).clone() for st in (a, b)]
+            outs = [e.prefill(prompts, [2, 0, 1], st, left_pad=False).clone() for e, st in ((eng, a), (eng, b), (e32, r))]
         elif step == 2:
-            for st in (a, b):
+            for st in (a, b, r):
                 st.copy_rows(torch.tensor([2, 0], device=DEV), torch.tensor([3, 4], device=DEV), 41)
-        tok = torch.arange(B, device=DEV) + 9
-        outs = [eng.decode_step(tok, st).clone() for st in (a, b)]
-        assert torch.equal(*outs)
-    for i in range(cfg.n_layers):
-        n = a.k[i].size(2)
-        assert torch.equal(a.k[i], b.k[i][:, :, :n]) and torch.equal(a.v[i], b.v[i][:, :, :n])
-    a.k[l], a.v[l] = a.k[l].clone(), a.v[l].clone()
-    if kv_dtype == "int8":
-        a.k_scale[l], a.v_scale[l] = a.k_scale[l].clone(), a.v_scale[l].clone()
-    assert a.slots(l) == 50
-    outs = [eng.decode_step(tok, st).float() for st in (a, b)]
-    assert float((outs[0] - outs[1]).norm() / outs[1].norm()) < 0.05   # (the generic kernel: bf16 roundings of four layers)
+        outs = [e.decode_step(tok, st).clone() for e, st in ((eng, a), (eng, b), (e32, r))]
+        assert rel(outs[0], outs[2]) < 1.2 * rel(outs[1], outs[2]) < 0.05, (rel(outs[0], outs[2]), rel(outs[1], outs[2]))
+    assert not cfg.is_global(0) and torch.equal(a.k[0], b.k[0][:, :, :50]) and torch.equal(a.v[0], b.v[0][:, :, :50])
+    for _ in range(12):                    # (row 2 goes from position 44 to 56: past the ring's 50 slots, within 64)
+        eng.decode_step(tok, a)
+    assert 50 < int(a.pos.max()) <= 60
+    c = KVState(cfg, B, 50, DEV, kv_dtype=kv_dtype, dtype=torch.bfloat16)
+    for x, y in zip(tensors(c) + [c.pos, c.starts], tensors(a) + [a.pos, a.starts]):
+        x.copy_(y)
+    for _ in range(3):
+        x, y = eng.decode_step(tok, a).clone(), eng.decode_step(tok, c).clone()
+        same = torch.equal(x, y)
+        assert same
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("kv_dtype", ["int8", "fp16"])
+def test_fused_qkv_single_layer_is_exact_on_a_short_ring(kv_dtype, dtype):
+    """The fused launch against the separate ones on rings that max_len cut below the window - to 75 slots, of which the rows use 74,
+    and to 50, which they go past - and on a ring of a few slots, which the generic kernel takes."""
+    ulp = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10
+    for max_len, steps, lens in ((75, 34, (5, 40, 17, 33, 1, 26)), (50, 24, (5, 40, 17, 33, 1, 26)), (20, 10, (5, 9, 1))):
+        cfg, params, eng, _ = _setup("uv-test", dtype=dtype, perturb=0.05, window=128, n_layers=1, global_every=0, ve_every=1)
+        hdiff, agree, cmax, cfrac, sfrac = _fused_vs_unfused(cfg, eng, steps=steps, lens=lens, max_len=max_len, kv_dtype=kv_dtype)
+        assert cmax.max() == 0 and sfrac.max() == 0 and max(hdiff) <= 4 * 2 * ulp, (max_len, cmax, max(hdiff))
 
 
 _LEFT_TO_POST = {   # configurations whose attention leaves XSA and gate to the separate launch: what is not the default
@@ -962,7 +984,7 @@ def test_states_and_engines_are_copied_pickled_and_freed_after_use(plan):
     from ultraviolet_amd.engine import KVState
     cfg, _, eng, _ = _setup(dtype=torch.bfloat16, window=64)
     _force_plan(eng, plan)
-    st = KVState(cfg, 3, 96, DEV)
+    st = KVState(cfg, 3, 50, DEV)
     tok = torch.tensor([5, 9, 2], device=DEV)
     eng.prefill([[3, 4, 5], [6] * 9, [7]], [0, 1, 2], st)
     eng.decode_step(tok, st)

@@ -39,7 +39,7 @@ class AttnArgs(C.Structure):
                 ("scale", C.c_float), ("window", C.c_int), ("ring", C.c_int), ("num_splits", C.c_int),
                 ("chunk_keys", C.c_int), ("workspace", C.c_void_p), ("workspace_bytes", C.c_size_t),
                 ("post_vhat", C.c_void_p), ("post_gate", C.c_void_p), ("post_xsa", C.c_void_p), ("post_round_dtype", C.c_int),
-                ("fuse", C.c_void_p)]
+                ("fuse", C.c_void_p), ("any_ring", C.c_int)]
 
 
 class AttnQkvFuse(C.Structure):
@@ -141,7 +141,7 @@ class PromptTablesArgs(C.Structure):   # struct uvmi_prompt_tables_args
 OP_GEMM, OP_DECODE_ATTN, OP_QKV_POST, OP_PREFILL_ATTN, OP_NORM = range(5)   # UVMI_OP_*
 
 _lib = None
-ABI_VERSION = 6   # UVMI_ABI_VERSION of include/uvmi.h
+ABI_VERSION = 7   # UVMI_ABI_VERSION of include/uvmi.h
 
 
 def lib() -> C.CDLL:

@@ -178,15 +178,24 @@ struct AttnState {
 // FAST: the shape of the engine's decode step as compile-time constants - one kv head, 8 query heads, uncut rows, 64-bit
 // indices - so that the item arithmetic, the head masks, the split bookkeeping and the partial-result path fold away
 // (the fixed part of a wave's life is as long as its streaming loop on rows of a few hundred keys).
+// ANYRING (uvmi_attn_args.any_ring): rings of any length from 32 slots, at the precision of the generic kernel, which takes 133 us
+// on 16 rows of up to 128 keys for the attention alone where this one takes 5.2 with the fused post-processing.  A tile's keys are addressed one by
+// one, since it may wrap and its scales may start on any 2 bytes; K codes go into the MFMA without a bias (fp16, exact), V codes as
+// bf16 (exact, and with fp32's exponents for what multiplies them), and a probability - with its V scale, in fp32 - as three 16-bit
+// terms that hold all its bits.  Latency-bound like every launch on so few keys, the arithmetic costs little: a ring of whole tiles
+// at 16-bit probabilities takes 4.9 us there, 64 rows of up to 107 keys 5.3 / 4.9, 1000 rows of up to 249 keys 10.2 / 8.0; on a 16-bit
+// cache 5.0 / 5.1, 5.2 / 5.1 and 11.1 / 11.2.
 // PROBE (uvmi_decode_attn_probe; measurement only, the output is meaningless): 1 - the kernel's memory stream without its
 // arithmetic: every tile is loaded exactly as in the real kernel and folded into the state with a few xors; 2 - its
 // arithmetic without the stream: tiles are made up in registers, nothing is loaded from the cache.
-template <int QDT, int ODT, int WPR, bool FUSE, bool KV16 = false, bool FAST = false, int PROBE = 0, bool BYSLOT = false>
+template <int QDT, int ODT, int WPR, bool FUSE, bool KV16 = false, bool FAST = false, int PROBE = 0, bool BYSLOT = false, bool ANYRING = false>
 __global__ __launch_bounds__(WPR > 4 ? 64 * WPR : 256) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_rows, const void* a_q, const void* a_tok, int a_items,
                        int a_idx64, int a_splits, int a_kh, AttnParams P) {
   P.pos = a_pos; P.starts = a_starts; P.rows = a_rows; P.n_items = a_items; P.idx64 = a_idx64; P.splits = a_splits; P.KH = a_kh;
-  if constexpr (BYSLOT) P.ring = 1;
+  if constexpr (BYSLOT || ANYRING) P.ring = 1;
+  if constexpr (ANYRING) P.splits = 1;
+  constexpr bool BIASED = !KV16 && !ANYRING;   // int8 codes enter the MFMAs with the biases of the cheap conversion
   if constexpr (FAST) { P.idx64 = 1; P.splits = 1; P.KH = 1; P.G = 8; P.H = 8; P.hd = 64; P.chunk_keys = 0; }
   if (FUSE) P.f_qkv = a_q; else P.q = a_q;
   constexpr int BW = WPR > 4 ? WPR : 4, IPB = BW / WPR;  // waves and items per block
@@ -262,7 +271,7 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
   const float* pg_src = !FUSE && has_post && P.post_gate ? P.post_gate + (int64_t)b * P.H + hsafe : anyf;
   const float* px_src = has_post && P.post_xsa ? P.post_xsa + hsafe : anyf;
   const float pv_val = *pv_src, pg_val = *pg_src, px_val = *px_src;
-  const RowPlan rp = plan_row(P, ri, b, FUSE, FAST);
+  const RowPlan rp = plan_row(P, ri, b, FUSE, FAST || ANYRING);
   // FUSE: the row of the rotation table (cos / sin of the row's position per frequency, already rounded to the activation
   // type): prep_q reads its 32 values as scalars, the lane that owns dim d of the own key reads its own pair
   const int rope_row = rp.pc < 0 ? 0 : (rp.pc < P.f_rope_n ? rp.pc : P.f_rope_n - 1);
@@ -297,7 +306,7 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
   auto set_q = [&]() {
     QA0 = as_h8(qr[0] & mA, qr[1] & mA, qr[2] & mA, qr[3] & mA); QA1 = as_h8(qr[4] & mA, qr[5] & mA, qr[6] & mA, qr[7] & mA);
     QB0 = as_h8(qr[0] & mB, qr[1] & mB, qr[2] & mB, qr[3] & mB); QB1 = as_h8(qr[4] & mB, qr[5] & mB, qr[6] & mB, qr[7] & mB);
-    cinit = !KV16 && qmask ? -1152.0f * qsum : 0.f;
+    cinit = BIASED && qmask ? -1152.0f * qsum : 0.f;
   };
   // unfused: q arrives normalised and rotated, 16 dims per lane in the operand layout
   auto prep_q = [&]() {
@@ -491,7 +500,42 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
   auto load_tile = [&](int slot_in, TileX& T) {
     const int slot0 = __builtin_amdgcn_readfirstlane(slot_in);  // wave-uniform by construction
     const uint32_t ok = (uint32_t)slot0 * usks, ov = (uint32_t)slot0 * usvs, os = (uint32_t)slot0 * 2;
-    if constexpr (KV16) {
+    if constexpr (ANYRING) {
+      auto at = [&](uint32_t off) -> uint32_t {   // slot of the tile's key off < 32: one turn at most (S >= 32, host-checked)
+        const uint32_t s = (uint32_t)slot0 + off;
+        return s >= (uint32_t)S ? s - (uint32_t)S : s;
+      };
+      const uint32_t ka = at(m) * sks + 16 * ES * g, kb = at(16 + m) * sks + 16 * ES * g;
+      uint32_t va[4], vb[4];
+#pragma unroll
+      for (int j = 0; j < 4; j++) { va[j] = at(4 * g + j) * svs + 4 * ES * m; vb[j] = at(16 + 4 * g + j) * svs + 4 * ES * m; }
+      if constexpr (KV16) {
+        T.kA[0] = __builtin_amdgcn_raw_buffer_load_b128(rK, ka, 0, 0);
+        T.kA[1] = __builtin_amdgcn_raw_buffer_load_b128(rK, ka + 16, 0, 0);
+        T.kB[0] = __builtin_amdgcn_raw_buffer_load_b128(rK, kb, 0, 0);
+        T.kB[1] = __builtin_amdgcn_raw_buffer_load_b128(rK, kb + 16, 0, 0);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          T.vA[j] = __builtin_amdgcn_raw_buffer_load_b64(rV, va[j], 0, 0);
+          T.vB[j] = __builtin_amdgcn_raw_buffer_load_b64(rV, vb[j], 0, 0);
+        }
+      } else {
+        const u4 a = __builtin_amdgcn_raw_buffer_load_b128(rK, ka, 0, 0), b4 = __builtin_amdgcn_raw_buffer_load_b128(rK, kb, 0, 0);
+        T.kA = uint4{a.x, a.y, a.z, a.w};
+        T.kB = uint4{b4.x, b4.y, b4.z, b4.w};
+        uint32_t ks[4], vs[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          T.vA[j] = __builtin_amdgcn_raw_buffer_load_b32(rV, va[j], 0, 0);
+          T.vB[j] = __builtin_amdgcn_raw_buffer_load_b32(rV, vb[j], 0, 0);
+          const uint32_t sc = at(so + j) * 2;
+          ks[j] = __builtin_amdgcn_raw_buffer_load_b16(rKS, sc, 0, 0);
+          vs[j] = __builtin_amdgcn_raw_buffer_load_b16(rVS, sc, 0, 0);
+        }
+        T.ksc = uint2{ks[0] | (ks[1] << 16), ks[2] | (ks[3] << 16)};
+        T.vsc = uint2{vs[0] | (vs[1] << 16), vs[2] | (vs[3] << 16)};
+      }
+    } else if constexpr (KV16) {
       T.kA[0] = __builtin_amdgcn_raw_buffer_load_b128(rK, koA, ok, 0);
       T.kA[1] = __builtin_amdgcn_raw_buffer_load_b128(rK, koA + 16, ok, 0);
       T.kB[0] = __builtin_amdgcn_raw_buffer_load_b128(rK, koB, ok, 0);
@@ -578,10 +622,26 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
       const uint32_t a0 = T.kA.x ^ 0x80808080u, a1 = T.kA.y ^ 0x80808080u, a2 = T.kA.z ^ 0x80808080u, a3 = T.kA.w ^ 0x80808080u;
       const uint32_t b0 = T.kB.x ^ 0x80808080u, b1 = T.kB.y ^ 0x80808080u, b2 = T.kB.z ^ 0x80808080u, b3 = T.kB.w ^ 0x80808080u;
       constexpr uint32_t C64 = 0x64646464u, LO = 0x04010400u, HI = 0x04030402u;
+      if constexpr (ANYRING) {   // the code itself: (1024 + u) - 1152, exact
+        auto code = [&](uint32_t x, uint32_t sel) -> uint32_t {
+          const uint32_t w = perm(C64, x, sel);
+          h2 v;
+          __builtin_memcpy(&v, &w, 4);
+          v = v - h2{(_Float16)1152.0f, (_Float16)1152.0f};
+          uint32_t r;
+          __builtin_memcpy(&r, &v, 4);
+          return r;
+        };
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_h8(code(a0, LO), code(a0, HI), code(a1, LO), code(a1, HI)), QA0, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_h8(code(a2, LO), code(a2, HI), code(a3, LO), code(a3, HI)), QA1, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_h8(code(b0, LO), code(b0, HI), code(b1, LO), code(b1, HI)), QB0, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_h8(code(b2, LO), code(b2, HI), code(b3, LO), code(b3, HI)), QB1, acc, 0, 0, 0);
+      } else {
       acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_h8(perm(C64, a0, LO), perm(C64, a0, HI), perm(C64, a1, LO), perm(C64, a1, HI)), QA0, acc, 0, 0, 0);
       acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_h8(perm(C64, a2, LO), perm(C64, a2, HI), perm(C64, a3, LO), perm(C64, a3, HI)), QA1, acc, 0, 0, 0);
       acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_h8(perm(C64, b0, LO), perm(C64, b0, HI), perm(C64, b1, LO), perm(C64, b1, HI)), QB0, acc, 0, 0, 0);
       acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_h8(perm(C64, b2, LO), perm(C64, b2, HI), perm(C64, b3, LO), perm(C64, b3, HI)), QB1, acc, 0, 0, 0);
+      }
     }
     // ---- t_i = (q.k_int) * kscale_i for the lane's keys 4g+i of its stream (softmax scale applied inside exp2)
     float t[4], vsf[4];
@@ -625,7 +685,23 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
     // contraction slots
     uint32_t u01, u23;
     [[maybe_unused]] uint32_t l01 = 0, l23 = 0;
-    if constexpr (KV16 && QDT == UVMI_BF16) {
+    [[maybe_unused]] uint32_t e01[3], e23[3];   // ANYRING: the three terms
+    constexpr int PDT = KV16 ? QDT : UVMI_BF16; // and their type
+    if constexpr (ANYRING) {
+      using pt = std::conditional_t<PDT == UVMI_BF16, __bf16, _Float16>;
+      typedef pt pt2 __attribute__((ext_vector_type(2)));
+      float r[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) r[i] = p[i] * vsf[i];
+#pragma unroll
+      for (int e = 0; e < 3; e++) {
+        const pt2 x = pt2{(pt)r[0], (pt)r[1]}, y = pt2{(pt)r[2], (pt)r[3]};
+        __builtin_memcpy(&e01[e], &x, 4);
+        __builtin_memcpy(&e23[e], &y, 4);
+        r[0] -= (float)x[0]; r[1] -= (float)x[1]; r[2] -= (float)y[0]; r[3] -= (float)y[1];
+      }
+      u01 = u23 = 0;
+    } else if constexpr (KV16 && QDT == UVMI_BF16) {
       // a bf16 cache: p goes in as two bf16 terms, p = hi + lo (16 significant bits, where a single bf16 has 8), and P V is
       // two MFMAs per operand - the matrix pipe has the room, and the result stays within the fp16 path's error
       typedef __bf16 b2 __attribute__((ext_vector_type(2)));
@@ -669,8 +745,24 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
         const uint32_t sel = (tt & 1) ? HI : LO;
         const int e = tt >> 1;
         const h8 va = as_h8(perm(va_[1][e], va_[0][e], sel), perm(va_[3][e], va_[2][e], sel), perm(vb_[1][e], vb_[0][e], sel), perm(vb_[3][e], vb_[2][e], sel));
+        if constexpr (ANYRING) {
+#pragma unroll
+          for (int x = 2; x >= 0; x--) st.O[tt] = mfma_kv<QDT>(va, as_h8(e01[x] & mA, e23[x] & mA, e01[x] & mB, e23[x] & mB), st.O[tt]);
+          continue;
+        }
         st.O[tt] = mfma_kv<QDT>(va, PB, st.O[tt]);
         if constexpr (QDT == UVMI_BF16) st.O[tt] = mfma_kv<QDT>(va, as_h8(l01 & mA, l23 & mA, l01 & mB, l23 & mB), st.O[tt]);
+      }
+    } else if constexpr (ANYRING) {
+      auto pair = [&](uint32_t k1, uint32_t k0, int tt) -> uint32_t {   // byte tt of two keys as bf16
+        const float f1 = (float)((int)(k1 << (24 - 8 * tt)) >> 24), f0 = (float)((int)(k0 << (24 - 8 * tt)) >> 24);
+        return perm(__float_as_uint(f1), __float_as_uint(f0), 0x07060302u);
+      };
+#pragma unroll
+      for (int tt = 0; tt < 4; tt++) {
+        const h8 va = as_h8(pair(T.vA[1], T.vA[0], tt), pair(T.vA[3], T.vA[2], tt), pair(T.vB[1], T.vB[0], tt), pair(T.vB[3], T.vB[2], tt));
+#pragma unroll
+        for (int x = 2; x >= 0; x--) st.O[tt] = mfma_kv<UVMI_BF16>(va, as_h8(e01[x] & mA, e23[x] & mA, e01[x] & mB, e23[x] & mB), st.O[tt]);
       }
     } else {
       uint32_t xa[4], xb[4];
@@ -768,7 +860,7 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
   // ---- reduce l and sum P' over the 4 lane groups of a column
   const float lsum = xsum32(xsum16(st.lrun)), ps = xsum32(xsum16(st.psum));
   const float m2 = st.mrun == -INFINITY ? -INFINITY : st.mrun * c;  // exp2 domain
-  if (!FAST && rp.nsplit > 1) {
+  if (!FAST && !ANYRING && rp.nsplit > 1) {
     // ---- a chunk of a cut row: stream B is merged into stream A (lanes n and n ^ 8: a rotation by 8 inside a row of 16
     // lanes, a DPP move), the WPR waves of the item through LDS, and the item's first wave writes the partial state
     const float m_o = dpp_mov<0x128>(m2), l_o = dpp_mov<0x128>(lsum), ps_o = dpp_mov<0x128>(ps);
@@ -871,7 +963,7 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
         o[0] += ww * x.x; o[1] += ww * x.y;
       }
     }
-  if constexpr (!KV16) {  // undo the 2^-24 of the subnormal V operand and its +128 bias
+  if constexpr (BIASED) {  // undo the 2^-24 of the subnormal V operand and its +128 bias
     const float pm = 128.0f * psf;
 #pragma unroll
     for (int j = 0; j < NV; j++) o[j] = o[j] * 16777216.0f - pm;
@@ -1127,20 +1219,25 @@ static int check_common(const uvmi_attn_args* a) {
   return UVMI_OK;
 }
 
+// A ring that the MFMA kernel takes whatever its length (ANYRING); other calls go by the rules below.
+static bool any_ring(const uvmi_attn_args* a) {
+  return a->any_ring && a->ring && a->S >= 32 && a->num_splits == 1 && a->out_dtype == a->q_dtype && (a->fuse || a->post_vhat);
+}
+
 static bool mfma_ok(const uvmi_attn_args* a) {
   const int G = a->H / a->KH;
   if (a->hd != 64 || a->kv_dtype != UVMI_I8 || G > 8) return false;
   if (a->q_dtype == UVMI_F32) return false;  // fp32 queries keep every product and probability in fp32: the generic kernel
   if (!(a->scale > 0.f)) return false;  // the running maximum is tracked before the (positive) softmax scale
-  if (a->ring && (a->S % 32 != 0)) return false;
+  if (a->ring && a->S % 32 != 0 && !any_ring(a)) return false;
   if (a->sks > (1 << 20) || a->svs > (1 << 20) || a->sks < 0 || a->svs < 0) return false;  // 32-bit tile offsets
-  if (a->S % 4 != 0 || a->S < 32) return false;  // 8-byte scale loads; a whole 32-key tile at slot 0 must exist
+  if ((a->S % 4 != 0 && !any_ring(a)) || a->S < 32) return false;  // 8-byte scale loads; a whole 32-key tile at slot 0 must exist
   auto al = [](const void* p, int n) { return ((uintptr_t)p % n) == 0; };
   if (!al(a->q, 16) || a->sqb % 8 || a->sqh % 8) return false;
   if (!al(a->k_cache, 16) || a->skb % 16 || a->skh % 16 || a->sks % 16) return false;
   if (!al(a->v_cache, 4) || a->svb % 4 || a->svh % 4 || a->svs % 4) return false;
-  if (!al(a->k_scale, 8) || a->ssb % 4 || a->ssh % 4) return false;
-  if (!al(a->v_scale, 8) || a->stb % 4 || a->sth % 4) return false;
+  if (!any_ring(a) && (!al(a->k_scale, 8) || a->ssb % 4 || a->ssh % 4)) return false;
+  if (!any_ring(a) && (!al(a->v_scale, 8) || a->stb % 4 || a->sth % 4)) return false;
   const int ob = a->out_dtype == UVMI_F32 ? 4 : 2;
   if (!al(a->out, 16) || (a->sob * ob) % 16 || (a->soh * ob) % 16) return false;
   return true;
@@ -1151,7 +1248,7 @@ static bool mfma16_ok(const uvmi_attn_args* a) {
   const int G = a->H / a->KH;
   if (a->hd != 64 || G > 8 || a->kv_dtype != a->q_dtype || (a->q_dtype != UVMI_F16 && a->q_dtype != UVMI_BF16)) return false;
   if (!(a->scale > 0.f)) return false;
-  if (a->ring && (a->S % 32 != 0)) return false;
+  if (a->ring && a->S % 32 != 0 && !any_ring(a)) return false;
   if (a->S < 32) return false;  // a whole 32-key tile at slot 0 must exist
   if (a->sks > (1 << 19) || a->svs > (1 << 19) || a->sks < 0 || a->svs < 0) return false;  // 32-bit tile offsets in bytes
   auto al = [](const void* p, int n) { return ((uintptr_t)p % n) == 0; };
@@ -1269,7 +1366,7 @@ static int decode_attn_launch(const uvmi_attn_args* a, void* ws, size_t ws_bytes
       // 1024 keys 10.1 / 9.4); of 256 keys a wave has two tiles with four waves already (5.6 / 5.7).
       if (P.n_items <= cus) {
         if (wpr < 4) wpr = 4;
-        if (ctx >= 512 && !kv16 && a->num_splits == 1 && !probe) wpr = 8;
+        if (ctx >= 512 && !kv16 && a->num_splits == 1 && !probe && !any_ring(a)) wpr = 8;
       }
       // Rows of a known, short length - a window or ring of at most 512 keys, 16 tiles - are a chain of latencies rather than
       // a stream: they run fastest with about one wave per SIMD (measured on 256-key rings: 4 waves per row up to ~300 rows,
@@ -1335,7 +1432,16 @@ static int decode_attn_launch(const uvmi_attn_args* a, void* ws, size_t ws_bytes
     // rings that are streamed by slot once they have wrapped (BYSLOT): the window is the ring, S a power of two
     const bool by_slot = a->ring && a->window == a->S && (a->S & (a->S - 1)) == 0 && a->num_splits == 1 && !probe;
     const bool fast = !kv16 && a->num_splits == 1 && a->KH == 1 && a->H == 8 && a->idx_dtype == UVMI_I64;
-    if (probe) {
+    if (any_ring(a) && !probe) {
+#define UVMI_LR(QD, W, FU, K16) hipLaunchKernelGGL((attn_mfma_i8_hd64<QD, QD, W, FU, K16, false, 0, false, true>), grid, blk, 0, st, UVMI_LEAD, P)
+#define UVMI_LRW(QD, FU, K16) do { if (wpr == 4) UVMI_LR(QD, 4, FU, K16); else if (wpr == 2) UVMI_LR(QD, 2, FU, K16); else UVMI_LR(QD, 1, FU, K16); } while (0)
+#define UVMI_LRF(QD) do { if (a->fuse) { if (kv16) UVMI_LRW(QD, true, true); else UVMI_LRW(QD, true, false); } \
+                          else { if (kv16) UVMI_LRW(QD, false, true); else UVMI_LRW(QD, false, false); } } while (0)
+      if (a->q_dtype == UVMI_F16) UVMI_LRF(UVMI_F16); else UVMI_LRF(UVMI_BF16);
+#undef UVMI_LR
+#undef UVMI_LRW
+#undef UVMI_LRF
+    } else if (probe) {
       UVMI_REQUIRE(fast && !a->fuse && od == a->q_dtype && a->q_dtype == UVMI_BF16, UVMI_EUNSUPPORTED,
                    "uvmi_decode_attn_probe: only the engine's decode shape (int8 cache, bf16 q and output, 8 heads on 1 kv head, 64-bit indices, one split, no fused QKV)");
 #define UVMI_LP(PR)                                                                                                                   \

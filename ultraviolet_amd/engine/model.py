@@ -30,50 +30,51 @@ from .weights import UVWeights
 
 class KVState:
     """Slot-indexed KV cache (reference: KernelDecodeState, fast_decode.py:21-57): per layer k, v (B, K, S, hd) int8
-    and k_scale, v_scale (B, K, S) fp16 with S = max_len on global layers and min(window, max_len) on local (ring)
-    layers, max_len rounded up to a multiple of 32; pos / starts (B,) int64 on the device.  pos is the next position to write.  kv_dtype "fp16" (the
-    reference's name for "unquantized") keeps k, v in `dtype`, the activation type, with no scales."""
+    and k_scale, v_scale (B, K, S) fp16 with S = max_len, rounded up to a multiple of 32, on global layers and min(window, max_len)
+    on local (ring) layers; pos / starts (B,) int64 on the device.  pos is the next position to write.  kv_dtype "fp16" (the
+    reference's name for "unquantized") keeps k, v in `dtype`, the activation type, with no scales.  These tensors are all there
+    is: a ring holds the last S positions, also where the global caches have room for a few more."""
 
     def __init__(self, cfg: UVConfig, B: int, max_len: int, device="cuda", kv_dtype: str = "int8", dtype=torch.bfloat16):
         # Global caches have S rounded up to 32 slots: the MFMA attention kernel streams 32-key tiles and needs S % 4 == 0 for its
-        # 8-byte scale loads (other S fall back to the generic kernel).  A ring of a full window keeps its length; one that a short
-        # max_len cuts below the window never wraps: it keeps its length too, but as the front of an allocation of whole
-        # tiles, on which the kernels run (cache(); the generic kernel takes 123 us where the MFMA kernel takes 5.6 on 16 rows of
-        # up to 128 keys).
+        # 8-byte scale loads (other S fall back to the generic kernel).  Rings keep their length: a window, or what a short max_len
+        # cuts it to (short_ring).
         self.local_len = min(cfg.window, max_len)
         max_len = (max_len + 31) // 32 * 32
-        ring = min(cfg.window, max_len)
         self.cfg, self.B, self.max_len = cfg, B, max_len
         assert kv_dtype in ("int8", "fp16") and (kv_dtype == "int8" or dtype in (torch.float16, torch.bfloat16))
         self.kv_dtype, self.quantized = kv_dtype, kv_dtype == "int8"
         cdt = torch.int8 if self.quantized else dtype
         dev = torch.device(device)
         self.k, self.v, self.k_scale, self.v_scale = [], [], [], []
-        self._whole = []   # per layer the whole allocations where k, v and the scales are the front of them, else None
         for l in range(cfg.n_layers):
-            S, front = (max_len, max_len) if cfg.is_global(l) else (ring, self.local_len)
+            S = max_len if cfg.is_global(l) else self.local_len
             shp = (B, cfg.n_kv_heads, S, cfg.head_dim)
-            whole = [torch.zeros(shp, dtype=cdt, device=dev) for _ in range(2)]
-            whole += [torch.zeros(shp[:3], dtype=torch.float16, device=dev) if self.quantized else None for _ in range(2)]
-            self._whole.append(whole if front < S else None)
-            for ts, t in zip((self.k, self.v, self.k_scale, self.v_scale), whole):
-                ts.append(t if t is None or front == S else t[:, :, :front])
+            self.k.append(torch.zeros(shp, dtype=cdt, device=dev))
+            self.v.append(torch.zeros(shp, dtype=cdt, device=dev))
+            self.k_scale.append(torch.zeros(shp[:3], dtype=torch.float16, device=dev) if self.quantized else None)
+            self.v_scale.append(torch.zeros(shp[:3], dtype=torch.float16, device=dev) if self.quantized else None)
         self.pos = torch.zeros(B, dtype=torch.long, device=dev)
         self.starts = torch.zeros(B, dtype=torch.long, device=dev)
 
     def cache(self, l: int) -> tuple:
-        """k, v, k_scale, v_scale of layer l as the kernels take them: the whole allocations, as long as the layer's tensors are
-        still the front of them, else the tensors."""
-        ts = (self.k[l], self.v[l], self.k_scale[l], self.v_scale[l])
-        whole = self._whole[l]
-        if whole is None or any(t is not None and (t.data_ptr() != w.data_ptr() or t.stride() != w.stride()) for t, w in zip(ts, whole)):
-            return ts
-        return tuple(whole)
+        """k, v, k_scale, v_scale of layer l."""
+        return self.k[l], self.v[l], self.k_scale[l], self.v_scale[l]
 
     def slots(self, l: int) -> int:
-        """Slots of cache(l)'s rows (of its k; the launch checks the rest)."""
-        k, whole = self.k[l], self._whole[l]
-        return k.size(2) if whole is None or k.data_ptr() != whole[0].data_ptr() else whole[0].size(2)
+        """Slots of layer l's rows (of its k; the launch checks the rest)."""
+        return self.k[l].size(2)
+
+    def short_ring(self, l: int) -> bool:
+        """Whether layer l's cache is a ring that max_len cut below the window to a length of no whole tiles.  The engine runs those
+        as any_ring launches: the generic kernel, which takes such lengths too, needs 133 us where they need 5.2 on 16 rows of
+        up to 128 keys, and they keep its precision.  (Windows of such a length stay on the generic kernel.)"""
+        S = self.slots(l)
+        return not self.cfg.is_global(l) and 32 <= S < self.cfg.window and S % 32 != 0
+
+    def window(self, l: int) -> int:
+        """Keys that layer l attends (0: all): no more than its ring holds."""
+        return 0 if self.cfg.is_global(l) else min(self.cfg.window, self.slots(l)) if self.short_ring(l) else self.cfg.window
 
     def nbytes(self) -> int:
         return sum(t.numel() * t.element_size() for t in self.k + self.v + self.k_scale + self.v_scale if t is not None)
@@ -339,10 +340,12 @@ class UVEngine:
     # ------------------------------------------------------------------------------------------------ trunk
     def cache_attention_plannable(self, l: int, st: KVState) -> bool:
         """Whether layer l's attention over the cache is one launch with the fused XSA + gate epilogue: the MFMA kernel streams
-        32-key tiles (rings need S % 32 == 0, linear int8 caches S % 4 == 0) and serves int8 caches and caches in the q dtype."""
+        32-key tiles (rings need S % 32 == 0 or to be short ones, linear int8 caches S % 4 == 0) and serves
+        int8 caches and caches in the q dtype."""
         cfg, S = self.cfg, st.slots(l)
         mfma_cache = self.q_dtype != torch.float32 and (st.quantized or st.k[l].dtype == self.q_dtype)
-        return (mfma_cache and cfg.xsa and cfg.n_heads // cfg.n_kv_heads <= 8 and S % (4 if cfg.is_global(l) else 32) == 0 and S >= 32)
+        return (mfma_cache and cfg.xsa and cfg.n_heads // cfg.n_kv_heads <= 8 and S >= 32
+                and (S % (4 if cfg.is_global(l) else 32) == 0 or st.short_ring(l)))
 
     def cache_attention(self, l: int, q: Tensor, st: KVState, pos: Tensor, starts: Tensor, n: int, rows: Tensor | None = None,
                         off: int = 0):
@@ -350,15 +353,15 @@ class UVEngine:
         off..off+n of the call's buffers (q is already that slice); writes buf zg[off:off+n] and returns None, or, where
         the fused epilogue does not apply, returns the plain attention output for _attn_post."""
         cfg, b, W = self.cfg, self.buf, self.w.layers[l]
-        glob = cfg.is_global(l)
-        window = 0 if glob else cfg.window
+        glob, window = cfg.is_global(l), st.window(l)
         if self.cache_attention_plannable(l, st) and q.dtype == self.q_dtype:
             if rows is not None:
                 rows = rows.to(pos.dtype).contiguous()
             out = b["zg"][off:off + n].view(n, cfg.n_heads, cfg.head_dim)
             gate = None if W["attn_gate"] is None else b["gate"][off:off + n]
             k, v, ks, vs = st.cache(l)
-            a, keep = build_attn_args(q, k, v, pos.contiguous(), starts.contiguous(), cfg.attn_scale, window, not glob, ks, vs, 1, out, 0, rows, (b["vhat"][off:off + n], gate, W["xsa"], out.dtype))
+            a, keep = build_attn_args(q, k, v, pos.contiguous(), starts.contiguous(), cfg.attn_scale, window, not glob, ks, vs, 1, out, 0, rows,
+                                      (b["vhat"][off:off + n], gate, W["xsa"], out.dtype), any_ring=st.short_ring(l))
             self._op(L.OP_DECODE_ATTN, a, (keep, q, pos, starts), B="nd", q="q_d", post_vhat="vhat_d", out="zg_d", pos="pos_d", starts="starts_d",
                      **({} if gate is None else {"post_gate": "gate_d"}), **({} if rows is None else {"rows": "rows_d"}))
             return None
@@ -391,7 +394,7 @@ class UVEngine:
     def fused_layer_ok(self, l: int, st: KVState) -> bool:
         """Whether layer l's decode attention can take the fused path: the MFMA kernel streams 32-key tiles."""
         S = st.slots(l)
-        return self.fuse_qkv and (st.quantized or st.k[l].dtype == self.dtype) and S % 32 == 0 and S >= 32
+        return self.fuse_qkv and (st.quantized or st.k[l].dtype == self.dtype) and S >= 32 and (S % 32 == 0 or st.short_ring(l))
 
     def rope_table(self, n_positions: int) -> Tensor:
         """cos / sin of every position below n_positions in the activation type's rounding, built once per size."""
@@ -428,7 +431,8 @@ class UVEngine:
         glob = cfg.is_global(l)
         out = b["zg"][:n].view(n, cfg.n_heads, cfg.head_dim)
         k, v, ks, vs = st.cache(l)
-        return build_fused_args(qkvx[:n], cfg.n_heads, k, v, pos, starts, cfg.attn_scale, 0 if glob else cfg.window, not glob, ks, vs, W["xsa"], out, self._fuse_dict(l, tok, st), rows)
+        return build_fused_args(qkvx[:n], cfg.n_heads, k, v, pos, starts, cfg.attn_scale, st.window(l), not glob, ks, vs, W["xsa"], out,
+                                self._fuse_dict(l, tok, st), rows, any_ring=st.short_ring(l))
 
     def cache_attention_args(self, l: int, st: KVState, pos: Tensor, starts: Tensor, n: int, rows: Tensor | None = None):
         """The uvmi_attn_args struct cache_attention would launch for layer l on the engine's buffers (fused path only):
@@ -437,8 +441,8 @@ class UVEngine:
         glob = cfg.is_global(l)
         out = b["zg"][:n].view(n, cfg.n_heads, cfg.head_dim)
         k, v, ks, vs = st.cache(l)
-        return build_attn_args(b["q"][:n], k, v, pos, starts, cfg.attn_scale, 0 if glob else cfg.window, not glob, ks, vs, 1, out, 0, rows,
-                               (b["vhat"][:n], None if W["attn_gate"] is None else b["gate"][:n], W["xsa"], out.dtype))
+        return build_attn_args(b["q"][:n], k, v, pos, starts, cfg.attn_scale, st.window(l), not glob, ks, vs, 1, out, 0, rows,
+                               (b["vhat"][:n], None if W["attn_gate"] is None else b["gate"][:n], W["xsa"], out.dtype), any_ring=st.short_ring(l))
 
     def _trunk(self, tok: Tensor, pos: Tensor, n: int, attn, rows=None, last_pos=None, st: KVState | None = None,
                fused_attn=None, defer_final_norm: bool = False, advance: bool = False, final_norm: bool = True) -> Tensor:
@@ -730,7 +734,7 @@ class UVEngine:
                 return self.cache_attention(l, q, st, pos, starts, B)
             glob = cfg.is_global(l)
             k, v, ks, vs = st.cache(l)
-            return decode_attention(q, k, v, pos, starts, cfg.attn_scale, window=0 if glob else cfg.window, ring=not glob,
+            return decode_attention(q, k, v, pos, starts, cfg.attn_scale, window=st.window(l), ring=not glob,
                                     k_scale=ks, v_scale=vs, num_splits=ns[key])
 
         h = self._trunk(tok, pos, B, attn, st=st, fused_attn=fused)

@@ -69,8 +69,8 @@ def supported(q: Tensor, k_cache: Tensor) -> bool:
 
 
 def build_attn_args(q, k_cache, v_cache, pos, starts, scale, window, ring, k_scale, v_scale, num_splits, out, chunk_keys=0,
-                    rows=None, post=None, fuse=None):
-    """Fill a uvmi_attn_args struct for these tensors.  Returns (args, keepalive): the struct holds raw pointers, so the
+                    rows=None, post=None, fuse=None, any_ring=False):
+    """Fill a uvmi_attn_args struct for these tensors (any_ring: as in the header, for post and fuse).  Returns (args, keepalive): the struct holds raw pointers, so the
     caller keeps `keepalive` (and the tensors) alive until the launch has been enqueued."""
     B, H, hd = q.shape
     KH, S = k_cache.shape[1], k_cache.shape[2]
@@ -92,6 +92,7 @@ def build_attn_args(q, k_cache, v_cache, pos, starts, scale, window, ring, k_sca
                                             (None, None, 0, 0, 0, 0)),
                    pos.data_ptr(), starts.data_ptr(), dt(pos.dtype), None if rows is None else rows.data_ptr(), out.data_ptr(), dt(out.dtype),
                    *out.stride()[:2], B, H, KH, S, hd, scale, window, ring, num_splits, chunk_keys, None if ws is None else ws.data_ptr(), ws_bytes)
+    a.any_ring = int(any_ring)
     if post is not None:
         vhat, gate, xsa, round_dtype = post
         assert vhat.dtype == torch.float32 and vhat.is_contiguous()
@@ -243,20 +244,21 @@ def rope_table(inv_freq: Tensor, n_positions: int, round_dtype: torch.dtype) -> 
 
 def decode_attention_fused(qkv: Tensor, H: int, k_cache: Tensor, v_cache: Tensor, pos: Tensor, starts: Tensor, scale: float, *,
                            window: int, ring: bool, k_scale: Tensor, v_scale: Tensor, xsa: Tensor | None, out: Tensor,
-                           fuse: dict, rows: Tensor | None = None) -> Tensor:
+                           fuse: dict, rows: Tensor | None = None, any_ring: bool = False) -> Tensor:
     """A decode step's attention straight from the projection output: the kernel normalises and rotates q and k of each
     row's token, adds the value embedding to v, appends k and v to the cache at pos (int8 codes and scales, or the values
     themselves on a cache of the activation type), attends lo..pos and applies
     the XSA / gate epilogue (ultraviolet/model.py:302-333, kernels/fast_decode.py:291-325 of the reference in one launch).
     qkv (B, row) holds H*64 q, K*64 k, K*64 v and, from column fuse["ext_col"], the H gate logits and K value-embedding
-    gate logits; see uvmi_attn_qkv_fuse in include/uvmi.h for the other entries of `fuse`.  The caches are written."""
-    a, keep = build_fused_args(qkv, H, k_cache, v_cache, pos, starts, scale, window, ring, k_scale, v_scale, xsa, out, fuse, rows)
+    gate logits; see uvmi_attn_qkv_fuse in include/uvmi.h for the other entries of `fuse`.  any_ring: also rings of no whole
+    32-slot tiles.  The caches are written."""
+    a, keep = build_fused_args(qkv, H, k_cache, v_cache, pos, starts, scale, window, ring, k_scale, v_scale, xsa, out, fuse, rows, any_ring)
     L.check(L.lib().uvmi_decode_attn(C.byref(a), L.stream_ptr(qkv)), "uvmi_decode_attn")
     del keep
     return out
 
 
-def build_fused_args(qkv, H, k_cache, v_cache, pos, starts, scale, window, ring, k_scale, v_scale, xsa, out, fuse, rows=None):
+def build_fused_args(qkv, H, k_cache, v_cache, pos, starts, scale, window, ring, k_scale, v_scale, xsa, out, fuse, rows=None, any_ring=False):
     """The uvmi_attn_args struct (and what must stay alive with it) of decode_attention_fused."""
     L.require_cuda(qkv, k_cache, pos)
     B = qkv.size(0)
@@ -264,7 +266,7 @@ def build_fused_args(qkv, H, k_cache, v_cache, pos, starts, scale, window, ring,
     if rows is not None:
         rows = rows.to(pos.dtype).contiguous()
     a, keep = build_attn_args(q, k_cache, v_cache, pos.contiguous(), starts.contiguous(), float(scale), int(window), bool(ring), k_scale,
-                              v_scale, 1, out, 0, rows, None, dict(fuse, qkv=qkv))
+                              v_scale, 1, out, 0, rows, None, dict(fuse, qkv=qkv), any_ring)
     a.post_round_dtype = L.dtype_code(out.dtype)
     if xsa is not None:
         assert xsa.dtype == torch.float32 and xsa.is_contiguous()
