@@ -217,20 +217,6 @@ def decode_attention(q: Tensor, k_cache: Tensor, v_cache: Tensor, pos: Tensor, s
                            bool(ring), k_scale, v_scale, int(num_splits), bool(out_fp32), int(chunk_keys), rows)
 
 
-def decode_attention_post(q: Tensor, k_cache: Tensor, v_cache: Tensor, pos: Tensor, starts: Tensor, scale: float, *,
-                          window: int, ring: bool, k_scale: Tensor, v_scale: Tensor, vhat: Tensor, gate: Tensor | None,
-                          xsa: Tensor | None, out: Tensor, rows: Tensor | None = None) -> Tensor:
-    """decode_attention followed by the reference's Attention.post up to the output projection (XSA with the
-    unquantized current v, per-head sigmoid gate; ultraviolet/model.py:321-333) in the same kernel.  vhat (B, K, hd) fp32
-    is v / max(|v|, eps) and gate (B, H) fp32 the gate values, both produced by the qkv_post kernel; out (B, H, hd) in
-    the activation dtype is written in place.  int8 cache or a cache in the q dtype, head_dim 64, one chunk per row."""
-    L.require_cuda(q, k_cache, pos)
-    if rows is not None:
-        rows = rows.to(pos.dtype).contiguous()
-    return _launch(q, k_cache, v_cache, pos.contiguous(), starts.contiguous(), float(scale), int(window), bool(ring), k_scale,
-                   v_scale, 1, out, 0, rows, (vhat, gate, xsa, out.dtype))
-
-
 def rope_table(inv_freq: Tensor, n_positions: int, round_dtype: torch.dtype) -> Tensor:
     """(n_positions, 2 * n_pairs) fp32: cos(p * inv_freq) then sin(p * inv_freq), each rounded to round_dtype - the
     rotation table the fused decode path reads (the reference's Rotary buffers, ultraviolet/model.py:198-226)."""
