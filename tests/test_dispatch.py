@@ -58,3 +58,34 @@ def test_modes_and_transforms_reach_the_op(route):
     q, k, v = _qkv()
     torch.func.vmap(lambda a: (seen.append(route(a, k, v)), a)[1])(q[None])
     assert seen == ["op"]
+
+
+def test_guard_of_recorded_passes_sees_what_changes():
+    """Everything that launches took an address or a number from: a tensor replaced, moved under its object, a scalar, an entry that
+    comes or goes - in the weights and in the state; by torch's comparison of addresses and by the list of them."""
+    from types import SimpleNamespace as N
+    from ultraviolet_amd.engine import plan
+    t = lambda: torch.zeros(4)
+    w = N(embed=t(), value_embed=None, inv_freq=t(), layers=[{"wo": t(), "wqkv": t(), "xsa": None, "resid_attn": 1.5} for _ in range(2)])
+    st = N(k=[t(), t()], v=[t(), t()], k_scale=[None, None], v_scale=[None, None])
+
+    def moved(x):
+        x.data = x.data.clone()
+    changes = [lambda: setattr(w, "embed", t()), lambda: moved(w.embed), lambda: moved(w.inv_freq), lambda: setattr(w, "value_embed", t()),
+               lambda: w.layers[1].__setitem__("wo", t()), lambda: moved(w.layers[0]["wo"]), lambda: w.layers[0].__setitem__("resid_attn", 2.5),
+               lambda: w.layers[0].__setitem__("xsa", t()), lambda: w.layers[1].__setitem__("new", t()), lambda: w.layers[1].pop("new"),
+               lambda: w.layers[0].__setitem__("wqkv", t()), lambda: st.k.__setitem__(1, t()), lambda: moved(st.v[0]), lambda: st.v.pop()]
+    same = plan._same_addresses
+    try:
+        for f in (same, lambda ts, at, _: list(map(torch.Tensor.data_ptr, ts)) == at):
+            plan._same_addresses = f
+            for change in changes if f is same else changes[:9]:
+                g = plan.Guard(w, st)
+                assert g.holds(w, st)
+                change()
+                assert not g.holds(w, st)
+            if f is same:
+                st.v.append(t())
+                w.value_embed = None
+    finally:
+        plan._same_addresses = same

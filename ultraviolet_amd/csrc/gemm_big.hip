@@ -78,7 +78,7 @@ template <int DT> __device__ __forceinline__ void unpack2(uint32_t w, float& lo,
 // for its RMS-normalised rows.
 // FI: 16-row fragments per wave along M: 8 - the 256 x 256 tile on 8 waves (2 x 4); 4 - a 128 x 128 tile on 4 waves (2 x 2,
 // 64 x 64 per wave, two workgroups per compute unit) for passes whose 256 x 256 tiles would not fill the device.  (A
-// 64 x 64 tile on 2 waves was measured too: no faster than the tiled kernel's 64 x 64 form at 2 k rows.)
+// 64 x 64 tile on 2 waves was measured too: no faster at 2 k rows than 64 x 64 tiles staged through registers.)
 template <int DT, int EPI, bool NORM, int FI>
 __global__ __launch_bounds__(64 * FI) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_big_kernel(BigParams P) {

@@ -7,8 +7,10 @@ results: every launch runs on every call."""
 from __future__ import annotations
 
 import ctypes as C
+from itertools import chain
 from operator import is_
 
+import torch
 from torch import Tensor
 
 from .. import _lib as L
@@ -16,16 +18,27 @@ from .. import _lib as L
 
 class Guard:
     """The objects that recorded launches took addresses and numbers from - weights, residual scalars, cache tensors - and where the
-    tensors among them were: one may be replaced, or keep its object and move (`.data = `)."""
+    tensors among them were: one may be replaced, or keep its object and move (`.data = `).  Every pass asks, so it is two walks in C
+    over ~170 objects (10 us; the launches of one layer take 15)."""
 
-    def __init__(self, objects):
-        self.objects = tuple(objects)
-        self.tensors = [t for t in self.objects if isinstance(t, Tensor)]
+    _END = object()
+
+    def __init__(self, weights, state):
+        self.objects = tuple(self._of(weights, state))
+        live = {id(W[k]) for W in weights.layers for k in ("wqkv", "gu") if k in W}   # (no launch of this library in a list reads these)
+        self.tensors = [t for t in self.objects if isinstance(t, Tensor) and id(t) not in live]
         self.at = list(map(Tensor.data_ptr, self.tensors))
+        self.every = list(range(len(self.tensors)))
 
-    def holds(self, objects) -> bool:
-        objects = tuple(objects)
-        return len(objects) == len(self.objects) and all(map(is_, self.objects, objects)) and list(map(Tensor.data_ptr, self.tensors)) == self.at
+    def _of(self, w, st):
+        return chain((w.embed, w.value_embed, w.inv_freq), *map(dict.values, w.layers), st.k, st.v, st.k_scale, st.v_scale, (self._END,))
+
+    def holds(self, weights, state) -> bool:
+        return all(map(is_, self.objects, self._of(weights, state))) and _same_addresses(self.tensors, self.at, self.every)
+
+
+# (what torch's graph trees compare their static inputs with: half the time of a list of data_ptr() calls)
+_same_addresses = getattr(torch._C, "_tensors_data_ptrs_at_indices_equal", None) or (lambda ts, at, _: list(map(Tensor.data_ptr, ts)) == at)
 
 
 class PassPlan:
