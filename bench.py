@@ -404,8 +404,8 @@ def bench_attn_ceiling(args):
 
 def bench_gemm(args):
     """The projections of UV-50M as single launches, back to back in a graph on four rotating weight copies: this library's
-    GEMM forms (config 0 = what the dispatcher picks for the shape; 4 / 3 = 64 x 64 / 128 x 128 tiles staged through registers;
-    6 / 5 = 128 x 128 / 256 x 256 tiles loaded straight into LDS; 1 = the skinny form) beside the vendor library's (torch.mm /
+    GEMM forms (config 0 = what the dispatcher picks for the shape; 1 / 4 = the streaming form's 32 x 64 / 64 x 64 tiles; 3 = 128 x 128
+    tiles staged through registers; 6 / 5 = 128 x 128 / 256 x 256 tiles loaded straight into LDS) beside the vendor library's (torch.mm /
     addmm, without the norm or SwiGLU launch it needs around it), at a full decode step's 2048 rows and a mixed pass's 33 216."""
     from ultraviolet_amd.kernels.gemm import RESID, STORE, SWIGLU, gemm_tn, interleave_gate_up
     dev, dt = "cuda:0", torch.bfloat16

@@ -72,7 +72,7 @@ def test_guard_of_recorded_passes_sees_what_changes():
     def moved(x):
         x.data = x.data.clone()
     changes = [lambda: setattr(w, "embed", t()), lambda: moved(w.embed), lambda: moved(w.inv_freq), lambda: setattr(w, "value_embed", t()),
-               lambda: w.layers[1].__setitem__("wo", t()), lambda: moved(w.layers[0]["wo"]), lambda: w.layers[0].__setitem__("resid_attn", 2.5),
+               lambda: w.layers[1].__setitem__("wo", t()), lambda: moved(w.layers[0]["wo"]), lambda: w.layers[0].__setitem__("resid_attn", w.layers[0]["resid_attn"] + 1.0),
                lambda: w.layers[0].__setitem__("xsa", t()), lambda: w.layers[1].__setitem__("new", t()), lambda: w.layers[1].pop("new"),
                lambda: w.layers[0].__setitem__("wqkv", t()), lambda: st.k.__setitem__(1, t()), lambda: moved(st.v[0]), lambda: st.v.pop()]
     same = plan._same_addresses

@@ -120,7 +120,8 @@ def test_greedy_64_tokens_identical_fp32(name, over):
 
 
 # the decode pass's launch plans by row count, forced here at a few rows:
-# (skinny_rows, fold_qkv_rows, fold_o_rows, fold_gu_rows, form of the hand-written GEMM)
+# (skinny_rows, fold_qkv_rows, fold_o_rows, fold_gu_rows, form of the hand-written GEMM: 4 the streaming one's 64 x 64 tiles, 3 the
+# 128 x 128 tiles through registers)
 _TRUNK_PLANS = {"small": None, "large-skinny-attn-block": (0, 1 << 30, 1 << 30, 0, 0), "large-library": (0, 0, 0, 0, 0),
                 "large-tiled-64": (0, 1 << 30, 1 << 30, 1 << 30, 4), "large-tiled-128": (0, 1 << 30, 1 << 30, 1 << 30, 3),
                 "large-tiled-64-own-down": (0, 1 << 30, 1 << 30, 1 << 30, 4, (0, 1 << 30))}
@@ -129,7 +130,7 @@ _TRUNK_PLANS = {"small": None, "large-skinny-attn-block": (0, 1 << 30, 1 << 30, 
 def _force_plan(eng, plan):
     if _TRUNK_PLANS[plan] is not None:
         eng.skinny_rows, eng.fold_qkv_rows, eng.fold_o_rows, eng.fold_gu_rows, eng.gemm_config = _TRUNK_PLANS[plan][:5]
-        eng.general_skinny_rows = eng.skinny_rows   # the unfused path the plans are compared with runs the library's GEMMs too
+        eng.general_skinny_rows = eng.skinny_rows
         if len(_TRUNK_PLANS[plan]) > 5:   # the down projection on this library's tiled GEMM too
             eng.fold_down_rows = _TRUNK_PLANS[plan][5]
 
@@ -156,13 +157,32 @@ def test_16bit_engine_close_to_oracle(plan, dtype, max_bar, mean_bar):
 
 
 @pytest.mark.parametrize("dtype,max_bar,mean_bar", [(torch.bfloat16, 0.15, 0.02), (torch.float16, 0.04, 0.005)])
+@pytest.mark.parametrize("general_skinny_rows", [384, 0])
+def test_plain_plan_of_a_16bit_engine_close_to_oracle(general_skinny_rows, dtype, max_bar, mean_bar):
+    """A configuration that the other plans refuse (8 rotated pairs): prompts of 663 tokens on the vendor library's GEMMs and steps
+    on this library's, or both on the vendor library's, to the bars of the other plans."""
+    cfg, params, eng, OracleModel = _setup(dtype=dtype, window=128, rope_frac=0.25)
+    eng.general_skinny_rows = general_skinny_rows
+    if not general_skinny_rows:
+        eng.skinny_rows = 0
+    assert not eng.fuse_qkv and eng._pass_kind(663, False, None) == eng._pass_kind(6, False, None) == "plain"
+    prompts = _prompts(cfg, (100, 130, 90, 150, 129, 64))
+    cont = np.random.default_rng(2).integers(1, cfg.vocab_size, size=(6, 6))
+    got, _ = _teacher_forced(eng, prompts, cont, 192)
+    ref, _ = _oracle_teacher_forced(OracleModel(cfg, params, dtype), prompts, cont, 192)
+    d = np.abs(got - ref)
+    assert np.isfinite(got).all() and d.max() < max_bar and d.mean() < mean_bar, (d.max(), d.mean())
+    assert (got.argmax(-1) == ref.argmax(-1)).mean() > 0.98
+
+
+@pytest.mark.parametrize("dtype,max_bar,mean_bar", [(torch.bfloat16, 0.15, 0.02), (torch.float16, 0.04, 0.005)])
 def test_prefill_pass_on_own_gemms_close_to_oracle(dtype, max_bar, mean_bar):
-    """The plans of general-path passes with many rows (here 663 packed prompt tokens): from 448 rows the QKV, output and
-    gate-up projections on this library's GEMM with the residual update in place, the extended QKV projection with the
-    block's pre-norm as its row scale, and the post-processing taking the gates' logits from the projection instead of from
-    the normalised hidden; from big_rows rows (forced to 1 here) the down projection too - each against the oracle in the
-    same 16-bit arithmetic, to the bars of the other plans, and against the same engine on the vendor library's GEMMs with
-    a norm launch per block (same positions, first-layer keys equal up to last-place flips of the projection)."""
+    """The plan of prompts (here 663 packed tokens): QKV, output, gate-up and down projections on this library's GEMM with the
+    residual updates in place, the extended QKV projection with the block's pre-norm as its row scale, and the
+    post-processing taking the gates' logits from the projection instead of from the normalised hidden; with the down
+    projection left to the vendor library (as between fold_down_rows and big_rows) and back - each against the oracle in the
+    same 16-bit arithmetic, to the bars of the other plans, and against the same engine on the plain plan: the vendor library's
+    GEMMs with a norm launch per block (same positions, first-layer keys equal up to last-place flips of the projection)."""
     cfg, params, eng, OracleModel = _setup(dtype=dtype, window=128)
     prompts = _prompts(cfg, (100, 130, 90, 150, 129, 64))
     cont = np.random.default_rng(2).integers(1, cfg.vocab_size, size=(6, 6))
@@ -171,6 +191,8 @@ def test_prefill_pass_on_own_gemms_close_to_oracle(dtype, max_bar, mean_bar):
     base, st0 = _teacher_forced(eng, prompts, cont, 192)
     eng.tiled_prefill = True
     runs = [(base, st0), _teacher_forced(eng, prompts, cont, 192)]
+    eng.fold_down_rows = (0, 600)
+    runs.append(_teacher_forced(eng, prompts, cont, 192))
     eng.big_rows = 1
     runs.append(_teacher_forced(eng, prompts, cont, 192))
     for got, st in runs:
@@ -219,8 +241,9 @@ def test_prefill_left_pad_vs_zero_start_positions():
 def test_mixed_step_matches_separate_prefill_and_decode(window):
     """A mixed batch (two new prompts prefilled into free cache rows while three running rows decode, one pass over all
     token rows) against the oracle's separate prefill and decode step: logits close, positions exact, the new rows'
-    layer-0 cache bytes equal, the running rows' appended keys equal.  window 16 takes the unfused attention epilogue,
-    window 32 the fused one."""
+    layer-0 cache bytes equal, the running rows' appended keys equal.  (An fp32 engine: the plain plan on the generic attention
+    kernel, rings of 16 and 32 slots.  16-bit engines, whose mixed passes take another plan:
+    test_c4_full_size_mixed_pass_equals_its_halves, test_mixed_step_of_a_16bit_engine_whose_attention_leaves_its_epilogue.)"""
     from oracle.model import OracleState
     from ultraviolet_amd.engine import KVState
     cfg, params, eng, OracleModel = _setup(window=window)

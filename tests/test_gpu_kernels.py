@@ -497,8 +497,7 @@ def test_rope_table_matches_rounded_cos_sin(dtype):
 def test_skinny_gemm_matches_fp32_reference(dtype, M, K, N):
     """uvmi_gemm_tn against a float64 product of the same 16-bit inputs: the result is the fp32-accumulated product rounded
     once to the activation type (tolerance: half a unit in the last place of the largest magnitude plus the accumulation
-    error of K terms), on ragged M (rows past M cut off), N that is not a multiple of the strip, both strip widths (K
-    below / above 960) and padded row pitches."""
+    error of K terms), on ragged M (rows past M cut off), N that is not a multiple of the tile, and padded row pitches."""
     from ultraviolet_amd.kernels.gemm import gemm_tn, gemm_supported
     g = torch.Generator(device="cuda").manual_seed(M * 7 + N)
     a_full = torch.randn(M, K + 8, device="cuda", generator=g).to(dtype)
@@ -508,8 +507,8 @@ def test_skinny_gemm_matches_fp32_reference(dtype, M, K, N):
     ref = a.double() @ w.double().t()
     ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
     tol = ulp * ref.abs().clamp_min(1.0) + 1e-5 * K ** 0.5
-    # 64-row workgroups; 16-row workgroups whose waves split K (the latter when K % 128 == 0); the tiled kernel with 128 x 128
-    # and 64 x 64 tiles (any K); the library's own choice
+    # the streaming form's 32 x 64 and 16 x 16 tiles; the tiled kernel with 128 x 128 tiles and the streaming form's 64 x 64 (any K);
+    # the library's own choice
     for config in ((1, 2) if K <= 1984 else ()) + (3, 4, 0):
         out_full = torch.full((M, N + 4), 7.0, device="cuda", dtype=dtype)
         out = out_full[:, :N]
@@ -573,7 +572,7 @@ def test_skinny_gemm_rejects_what_it_cannot_do():
     from ultraviolet_amd.kernels.gemm import SWIGLU, gemm_supported, gemm_tn
     a = torch.zeros(4, 2048, device="cuda", dtype=torch.bfloat16)
     w = torch.zeros(32, 2048, device="cuda", dtype=torch.bfloat16)
-    assert gemm_supported(a, w)                # K above 1984: the tiled kernel only
+    assert gemm_supported(a, w)                # K above 1984: not by configs 1 and 2
     gemm_tn(a, w)
     for config in (1, 2):
         with pytest.raises(L.UvmiError):
@@ -581,7 +580,7 @@ def test_skinny_gemm_rejects_what_it_cannot_do():
     with pytest.raises(L.UvmiError):
         gemm_tn(a[:, :1000], w[:, :1000])      # K % 64 != 0
     with pytest.raises(L.UvmiError):
-        gemm_tn(a[:, :1024], w[:, :1024], epilogue=SWIGLU, config=1)   # the skinny SwiGLU strip needs K <= 960
+        gemm_tn(a[:, :1024], w[:, :1024], epilogue=SWIGLU, config=1)   # (config 1 takes K <= 960 with the SwiGLU)
     gemm_tn(a[:, :1024], w[:, :1024], epilogue=SWIGLU)
     assert not gemm_supported(a.float(), w.float())
 
