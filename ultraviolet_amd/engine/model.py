@@ -2,8 +2,9 @@
 
 Mirrors ultraviolet/kernels/fast_decode.py of the reference (KernelDecodeState :21-57, decode_step_fast :272-334,
 _prefill_packed / prefill_packed_host :117-269) and the layer math of ultraviolet/model.py (Attention.qkv / post
-:302-335, Block.finish :567-571, MathLM.logits :824-827).  The GEMMs are torch (hipBLASLt) calls on preallocated
-buffers; everything between them is one fused HIP kernel per stage, and K/V go straight into the int8 cache.
+:302-335, Block.finish :567-571, MathLM.logits :824-827).  The projections of a 16-bit engine run on this
+library's GEMMs with the norms, residual updates and the SwiGLU in them (_pass_kind), an fp32 engine's on the vendor library's; what lies
+between them is one fused HIP kernel per stage, and K/V go straight into the cache.
 One decode step is a fixed launch sequence with no host synchronisation: it reads per-row positions on the device, so
 a single captured graph serves every context length (the reference needs one graph per 1024-token bucket,
 model.py:1099-1100)."""
