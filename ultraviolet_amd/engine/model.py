@@ -643,7 +643,9 @@ class UVEngine:
         own_down = n <= self.skinny_rows or n >= self.big_rows or self.fold_down_rows[0] <= n <= self.fold_down_rows[1]
         key = (what, kind, n <= self.fold_qkv_rows, n <= self.fold_o_rows, n <= self.fold_gu_rows, own_down,
                self.fold_down_rows[0] <= n <= self.fold_down_rows[1], self.gemm_config, getattr(self.w, "scalar_epoch", 0))
-        plans = self._plans.setdefault(st, {})
+        plans = self._plans.get(st)
+        if plans is None:
+            plans = self._plans[st] = {}
         plan = plans.get(key)
         if plan is None or not plan.guard.holds(self.w, st):
             if len(plans) >= 16:
