@@ -89,3 +89,38 @@ def test_guard_of_recorded_passes_sees_what_changes():
                 w.value_embed = None
     finally:
         plan._same_addresses = same
+
+
+def test_native_path_sees_what_plain_eager_sees():
+    """csrc/eager.cpp asks plain_eager's questions itself, but for the two that decode_attention asks before it."""
+    native = D.L.eager().plain
+    q, k, v = _qkv()
+    ks = vs = torch.ones(2, 1, 32).half()
+    calls = [(q, k, v, None, None), (q, k, v, ks, vs), (q, k, v, None, vs), (q.clone().requires_grad_(), k, v, ks, vs), (q, k, v, ks.clone().requires_grad_(), vs),
+             (q, k.as_subclass(_Subclass), v, ks, vs), (q, k, v, ks, vs.as_subclass(_Subclass)), (q, torch.nn.Parameter(k), v, None, None),
+             (q, torch.nn.Parameter(k, requires_grad=False), v, None, None)]
+
+    def same():
+        return [native(*c) for c in calls] == [D.plain_eager(*c) for c in calls]
+    assert native(*calls[0]) and native(*calls[1]) and not any(native(*c) for c in calls[3:])
+    assert same()
+    with torch.inference_mode():
+        assert native(*calls[1]) and same()
+    with torch.no_grad():
+        assert native(*calls[1]) and same()
+    with _Passing():
+        assert not native(*calls[1]) and same()
+    with torch.overrides.BaseTorchFunctionMode():
+        assert not native(*calls[1]) and same()
+    seen = []
+    torch.func.vmap(lambda a: (seen.append((native(a, k, v, ks, vs), D.plain_eager(a, k, v, ks, vs))), a)[1])(q[None])
+    torch.func.grad(lambda a: (seen.append((native(a, k, v, ks, vs), D.plain_eager(a, k, v, ks, vs))), a.sum())[1])(q.float())
+    assert seen == [(False, False)] * 2
+
+
+def test_native_path_leaves_other_calls_to_the_general_one():
+    """None for what is not on a device, and nothing raised: the general path has its own words for it."""
+    q, k, v = _qkv()
+    idx = torch.zeros(2, dtype=torch.long)
+    assert D.L.eager().decode_attention(q, k, v, None, None, idx, idx, None, 0.1, 0, None, None, 1, False, 0) is None
+    assert D.L.eager().decode_attention(q, k, 3, None, None, idx, None, None, 0.1, 0, None, None, 1, False, 0) is None

@@ -983,3 +983,70 @@ def test_gemm_softcap_epilogue(dtype, M, N, K, norm, config):
     assert bool(((got >= lo) & (got <= hi)).all())
     exact = 23.0 * torch.sigmoid((x.to(dtype).double() + 5.0) / 7.5)
     assert float(((got - exact).abs() < 1e-5).double().mean()) > 0.97
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("int8", [False, True])
+@pytest.mark.parametrize("form", ["plain", "indices32", "mixed indices", "rows", "views", "q4", "ring", "splits", "chunks", "fp32 out", "scale int", "inference"])
+def test_native_call_equals_the_general_one(monkeypatch, dtype, int8, form):
+    """decode_attention's native path (csrc/eager.cpp) and the general one launch the same kernel on the same arguments: equal bits
+    over the forms a call may take, those that the native path hands on among them."""
+    from ultraviolet_amd.kernels import decode_attn as D
+    B, H, S = 9, 8, 320
+    q, k, v, ks, vs = (None if t is None else t.to(DEV) for t in attn_case(B, 1, H, 64, S, int8, dtype=torch.float16))
+    q = q.to(dtype)
+    if not int8:
+        k, v = k.to(dtype), v.to(dtype)
+    pos = torch.arange(B, device=DEV) * 30 + 5
+    starts = torch.arange(B, device=DEV) % 4
+    kw, scale = dict(k_scale=ks, v_scale=vs), 0.14
+    if form == "indices32":
+        pos, starts = pos.int(), starts.int()
+    elif form == "mixed indices":
+        starts = starts.int()
+    elif form == "rows":
+        kw["rows"] = torch.tensor([3, -1, 0, 8, 8, 1, -1, 2, 5], device=DEV)
+    elif form == "views":
+        q = torch.randn(B, 2 * H, 128, device=DEV).to(dtype)[:, ::2, :64]
+        k, v = torch.cat([k, k], 2)[:, :, :S], torch.cat([v, v], 2)[:, :, :S]
+        if int8:
+            kw = dict(k_scale=torch.cat([ks, ks], 2)[:, :, :S], v_scale=torch.cat([vs, vs], 2)[:, :, :S])
+    elif form == "q4":
+        q = q[:, None]
+    elif form == "ring":
+        kw.update(window=S, ctx_hint=S)
+        pos = pos * 7
+    elif form == "splits":
+        kw.update(num_splits=3)
+    elif form == "chunks":
+        kw.update(num_splits=4, chunk_keys=96)
+    elif form == "fp32 out":
+        kw.update(out_fp32=True)
+    elif form == "scale int":
+        scale = 1
+    with torch.inference_mode(form == "inference"):
+        got = D.decode_attention(q, k, v, pos, starts, scale, **kw)
+        monkeypatch.setattr(D, "_native", lambda: lambda *a: None)
+        want = D.decode_attention(q, k, v, pos, starts, scale, **kw)
+    assert got.dtype == want.dtype and got.shape == want.shape and torch.equal(got, want)
+
+
+def test_native_call_refuses_what_the_general_one_refuses(monkeypatch):
+    """The library's refusals come back as the same exception; nothing is launched."""
+    from ultraviolet_amd import _lib as L
+    from ultraviolet_amd.kernels import decode_attn as D
+    q, k, v, ks, vs = (t.to(DEV) for t in attn_case(3, 1, 8, 64, 64, True))
+    pos, starts = torch.full((3,), 5, device=DEV), torch.zeros(3, dtype=torch.long, device=DEV)
+    bad = [(dict(q=q[:, :, :63]), dict()), (dict(q=torch.cat([q] * 3, 1)[:, :17]), dict()), (dict(), dict(num_splits=0)), (dict(), dict(window=-1))]
+
+    def says(over, kw):
+        t = dict(q=q, k=k, v=v, **{})
+        t.update(over)
+        try:
+            D.decode_attention(t["q"], t["k"], t["v"], pos, starts, 0.1, k_scale=ks, v_scale=vs, **kw)
+            return "taken"
+        except L.UvmiError as e:
+            return str(e)
+    native = [says(*b) for b in bad]
+    monkeypatch.setattr(D, "_native", lambda: lambda *a: None)
+    assert native == [says(*b) for b in bad] and native[1] != "taken"

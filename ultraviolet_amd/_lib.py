@@ -3,6 +3,7 @@ been built, or a call fails, an exception is raised."""
 from __future__ import annotations
 
 import ctypes as C
+import importlib.util
 import os
 
 import torch
@@ -208,6 +209,24 @@ def lib() -> C.CDLL:
                                    C.c_int64, C.c_int, C.c_void_p]
         _lib = L
     return _lib
+
+
+_eager = None
+
+
+def eager():
+    """The extension module of csrc/eager.cpp, loaded once, behind libuvmi.so (which it calls).  Raises UvmiError when it is missing."""
+    global _eager
+    if _eager is None:
+        lib()
+        path = os.path.join(_HERE, "csrc", "uvmi_eager.so")
+        if not os.path.exists(path):
+            raise UvmiError(f"{path} not found: run `python -m ultraviolet_amd.csrc.build` (no CPU fallback)")
+        spec = importlib.util.spec_from_file_location("uvmi_eager", path)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        _eager = mod
+    return _eager
 
 
 def check(rc: int, what: str) -> None:

@@ -1,4 +1,4 @@
-"""Build libuvmi.so (the C-ABI HIP library) for gfx950 in-tree.
+"""Build libuvmi.so (the C-ABI HIP library) for gfx950 in-tree, and uvmi_eager.so, the native path of small eager calls from Python.
 
     python -m ultraviolet_amd.csrc.build            # rebuild what is out of date
     python -m ultraviolet_amd.csrc.build --force    # recompile every source
@@ -17,6 +17,7 @@ SOURCES = ["common.hip", "kv_quant.hip", "decode_attn.hip", "fused_sample.hip", 
            "prefill_attn.hip", "prefill_attn_bwd.hip", "gemm.hip", "gemm_tile.hip", "gemm_big.hip", "gemm_stream.hip",
            "op_list.hip"]
 LIB = os.path.join(HERE, "libuvmi.so")
+EAGER = os.path.join(HERE, "uvmi_eager.so")   # the Python extension of eager.cpp
 ARCH = "gfx950"
 FLAGS = ["-O3", "-fPIC", "-std=c++17", f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang",
          "-packed-fp32-ops", "-Wno-unused-result", "-Wno-unknown-warning-option",
@@ -39,6 +40,24 @@ def _stale(obj: str, src: str) -> bool:
         return True
     deps = [src, os.path.join(HERE, "common.h"), os.path.join(HERE, "sched_commit.h"), os.path.join(HERE, "gemm_util.h"), os.path.join(HERE, "attn_mfma_util.h"), os.path.join(HERE, "..", "..", "include", "uvmi.h"), __file__]
     return any(os.path.getmtime(d) > os.path.getmtime(obj) for d in deps)
+
+
+def _build_eager(run, force: bool, verbose: bool) -> None:
+    """eager.cpp against the installed torch's headers (host code only), next to libuvmi.so, which it finds by its own place."""
+    src = os.path.join(HERE, "eager.cpp")
+    deps = (src, os.path.join(HERE, "..", "..", "include", "uvmi.h"), __file__)
+    if not force and os.path.exists(EAGER) and all(os.path.getmtime(d) <= os.path.getmtime(EAGER) for d in deps):
+        return
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+    run([os.environ.get("CXX", "g++"), "-O2", "-fPIC", "-std=c++17", "-shared", src, *(x for d in include_paths() for x in ("-isystem", d)),
+         "-I" + sysconfig.get_paths()["include"], f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+         *("-L" + d for d in library_paths()), "-ltorch_python", "-ltorch_cpu", "-lc10", "-L" + HERE, "-l:libuvmi.so", "-Wl,-rpath,$ORIGIN",
+         "-o", EAGER])
+    if verbose:
+        print("linked", os.path.relpath(EAGER, HERE), flush=True)
 
 
 def build(force: bool = False, verbose: bool = True) -> str:
@@ -68,6 +87,7 @@ def build(force: bool = False, verbose: bool = True) -> str:
         run([hipcc, "-shared", "-fPIC", f"--offload-arch={ARCH}", "-o", LIB, *objs])
         if verbose:
             print("linked", os.path.relpath(LIB, HERE), flush=True)
+    _build_eager(run, force, verbose)
     return LIB
 
 

@@ -48,6 +48,14 @@ def plain_eager(q: Tensor, k: Tensor, v: Tensor, k_scale: Tensor | None, v_scale
     return type(k_scale) is Tensor and type(v_scale) is Tensor and not (k_scale.requires_grad or v_scale.requires_grad or k.requires_grad or v.requires_grad)
 
 
+@functools.lru_cache(maxsize=None)
+def _native():
+    """decode_attention of csrc/eager.cpp."""
+    mod = L.eager()
+    mod.bind(_device_cus)
+    return mod.decode_attention
+
+
 def default_splits(n_bk: int, ctx: int, device=None, min_chunk: int = 256, waves: int = 1) -> int:
     """Splits per (row, kv head) (reference: decode_attn.py:121-129, re-derived for MI355X).  Each (row, kv head,
     split) is one workgroup whose 4 waves stream interleaved key tiles, so a row is only cut when there are fewer rows
@@ -190,6 +198,13 @@ def decode_attention(q: Tensor, k_cache: Tensor, v_cache: Tensor, pos: Tensor, s
     chunk_keys  0: every row is cut into num_splits equal chunks (the reference's rule); > 0: chunks of at least this
              many keys and at most num_splits of them per row, so short rows take fewer work items.
     Returns (B, H, hd) in q.dtype.  Graph-capturable; registered as a torch custom op (opaque to torch.compile)."""
+    if not torch.compiler.is_compiling() and forward_ad._current_level < 0 and q.is_cuda:
+        # plain eager calls, checked, allocated and launched natively (None: not such a call)
+        out = _native()(q, k_cache, v_cache, k_scale, v_scale, pos, starts, rows, scale, window, ring, ctx_hint, num_splits, out_fp32, chunk_keys)
+        if type(out) is int:
+            L.check(out, "uvmi_decode_attn")
+        if out is not None:
+            return out
     if q.dim() == 4:
         q = q.reshape(q.size(0), q.size(-2), q.size(-1))
     L.require_cuda(q, k_cache, v_cache, pos, starts)
