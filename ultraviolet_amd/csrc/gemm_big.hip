@@ -11,8 +11,9 @@
 //     fragments from LDS for 32 MFMAs (the 64 x 64 wave tile of the smaller kernels reads 8 for 16), and the tile takes
 //     half the L2 bytes per flop of a 128 x 128 tile;
 //   * K is walked in slabs of 64: a row's share of a slab is one whole 128-byte line;
-//   * slabs go from global memory straight into LDS (global_load_lds, 16 bytes per lane): no staging registers, no LDS
-//     store instructions.  A wave-load lands as 1 KB of consecutive LDS - 8 rows of 128 bytes - so the xor swizzle that
+//   * slabs go from global memory straight into LDS (buffer loads, 16 bytes per lane): no staging registers, no LDS
+//     store instructions, and 32-bit offsets where global loads keep eight 64-bit addresses per lane (33 216-row gate-up without the
+//     norm 152 -> 149 us).  A wave-load lands as 1 KB of consecutive LDS - 8 rows of 128 bytes - so the xor swizzle that
 //     keeps the operand reads conflict-free (16-byte chunk index ^ (row / 2) % 8) is applied on the global side: lane l
 //     of a load fetches the chunk that belongs at physical position l % 8 of its row;
 //   * two LDS stages of 64 KB (A and W slab each 256 rows x 128 B).  An iteration multiplies slab k out of one stage while
@@ -23,6 +24,11 @@
 //     lanes so that the 4 lane groups of a row store 64 consecutive bytes (RESID: 16 columns per lane).  fp32 logits are
 //     stored as they lie: 4 columns are 16 bytes (512 x 32768 with the softcap 52.8 us behind the 4 x 4 transpose, 47.7 so,
 //     33.7 on 256 x 256 tiles; 128 rows 17.8 / 14.2; 256 rows 24.2 / 18.0);
+//   * the residual of the whole tile is requested at once behind the main loop, ahead of the first store (in place it may not be
+//     moved across one by the compiler, and was requested row block by row block: 18 432 x 640 x 512 27.9 -> 23.8 us, x 1664 53.8 ->
+//     50.8; 33 216 rows in 128 x 128 tiles 47.7 -> 45.3, 98.4 -> 96.7);
+//   * the pre-norm's sums of squares go between the matrix instructions (gate-up at 33 216 rows 170 -> 160 us, at 18 432 105 -> 98;
+//     without the norm 148 and 87);
 //   * no loads are made past the last slab (they were, to keep the loop free of branches: the epilogue then waited for them;
 //     1 - 3 % of a launch);
 //   * tiles are dealt to the XCDs in contiguous runs, as in the tiled kernel.
@@ -43,7 +49,6 @@ struct BigParams {
 };
 
 #define UVMI_LDSP(p) ((__attribute__((address_space(3))) void*)(p))
-#define UVMI_GLBP(p) ((const __attribute__((address_space(1))) void*)(p))
 
 // Two dwords x, y per lane in lane groups g = lane / 16 (x0 .. x3, y0 .. y3) -> x = (x0, x2, y0, y2), y = (x1, x3, y1, y3).
 // (permlane32_swap exchanges the upper 32 lanes of its first operand with the lower 32 of its second, permlane16_swap does the
@@ -67,10 +72,6 @@ __device__ __forceinline__ void xpose4(uint32_t (&x)[4]) {
 __device__ __forceinline__ void xpose2(uint32_t& x0, uint32_t& x1) {
   auto t = __builtin_amdgcn_permlane16_swap(x0, x1, false, false);
   x0 = t[0]; x1 = t[1];
-}
-template <int DT> __device__ __forceinline__ void unpack2(uint32_t w, float& lo, float& hi) {
-  if (DT == UVMI_BF16) { lo = __uint_as_float(w << 16); hi = __uint_as_float(w & 0xffff0000u); }
-  else { lo = half_bits_to_float((uint16_t)(w & 0xffff)); hi = half_bits_to_float((uint16_t)(w >> 16)); }
 }
 
 // EPI 0: C = A W^T (M, N).  EPI 1: W rows are [gate 16 | up 16] slabs; C = silu(gate) * up, (M, N / 2).
@@ -115,29 +116,34 @@ void gemm_big_kernel(BigParams P) {
     row = row < P.N ? row : P.N - 1;
     offB[i] = (uint32_t)row * P.ldw2 + 16 * ch;
   }
-  const unsigned char* ga = (const unsigned char*)P.a;
-  const unsigned char* gw = (const unsigned char*)P.w;
+  // (buffer loads: 32-bit offsets and the slab as a scalar, where global ones keep eight 64-bit addresses)
+  const __amdgpu_buffer_rsrc_t rA = __builtin_amdgcn_make_buffer_rsrc((void*)P.a, 0, (int)((uint32_t)(P.M - 1) * P.lda2 + (uint32_t)P.K * 2), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rW = __builtin_amdgcn_make_buffer_rsrc((void*)P.w, 0, (int)((uint32_t)(P.N - 1) * P.ldw2 + (uint32_t)P.K * 2), 0x00020000);
   auto issue = [&](unsigned char* sa, unsigned char* sb, int kt) {
-    const uint32_t ko = (uint32_t)kt * 128;
 #pragma unroll
     for (int i = 0; i < 4; i++)
-      __builtin_amdgcn_global_load_lds(UVMI_GLBP(ga + offA[i] + ko), UVMI_LDSP(sa + (4 * wave + i) * 1024), 16, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, UVMI_LDSP(sa + (4 * wave + i) * 1024), 16, offA[i], kt * 128, 0, 0);
 #pragma unroll
     for (int i = 0; i < 4; i++)
-      __builtin_amdgcn_global_load_lds(UVMI_GLBP(gw + offB[i] + ko), UVMI_LDSP(sb + (4 * wave + i) * 1024), 16, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, UVMI_LDSP(sb + (4 * wave + i) * 1024), 16, offB[i], kt * 128, 0, 0);
   };
 
   // ---- reader: wave (wm, wn) owns rows 16 FI wm .., columns 64 wn ..; lane (r, g) reads chunk (4 s + g) ^ ((r / 2) % 8) of
   // row r of a 16-row fragment for K-step s
   const int wm = wave / WN, wn = wave % WN;
   const int r = lane & 15, g = lane >> 4;
-  uint32_t a_off[2], b_off[2];
+  // The wave's pairs of row fragments are walked from pair wn on (NORM; accumulator rows 2 p, 2 p + 1 belong to pair (p + wn) mod
+  // FI / 2), so that the rows whose squares a wave sums are the same in the code of every wave.
+  constexpr int NP = FI / 2;
+  uint32_t a_off[2], b_off[2], pair_at[NP];
 #pragma unroll
   for (int s = 0; s < 2; s++) {
     const uint32_t lo = (uint32_t)r * 128 + (uint32_t)((((4 * s + g) ^ ((r >> 1) & 7))) << 4);
     a_off[s] = (uint32_t)wm * (16 * FI * 128) + lo;
     b_off[s] = (uint32_t)wn * 8192 + lo;
   }
+#pragma unroll
+  for (int p = 0; p < NP; p++) pair_at[p] = (uint32_t)(NORM ? ((p + wn) & (NP - 1)) : p) * 4096;
   gf4 acc[FI][4];
 #pragma unroll
   for (int i = 0; i < FI; i++)
@@ -150,8 +156,11 @@ void gemm_big_kernel(BigParams P) {
     for (int j = 0; j < 4; j++) w[j] = *(const gu4*)(sb + b_off[s] + j * 2048);
   };
   auto read_a = [&](const unsigned char* sa, int s, int i, gu4* f) {
-    f[0] = *(const gu4*)(sa + a_off[s] + i * 2048);
-    f[1] = *(const gu4*)(sa + a_off[s] + (i + 1) * 2048);
+    uint32_t o;
+    if constexpr (NORM) asm volatile("v_add_u32 %0, %1, %2" : "=v"(o) : "s"(pair_at[i / 2]), "v"(a_off[s]));   // (kept out of registers between uses)
+    else o = a_off[s] + pair_at[i / 2];
+    f[0] = *(const gu4*)(sa + o);
+    f[1] = *(const gu4*)(sa + o + 2048);
   };
   // (the MFMA's A input is the weight fragment, its B input the activation fragment: the accumulator holds C^T)
   auto mm1 = [&](int i, const gu4* f, const gu4* w) { acc[i][0] = gmfma<DT>(w[0], f[0], acc[i][0]); };
@@ -162,21 +171,30 @@ void gemm_big_kernel(BigParams P) {
     for (int j = 0; j < 4; j++) acc[i + 1][j] = gmfma<DT>(w[j], f[1], acc[i + 1][j]);
   };
   // NORM: the squares of the rows are summed from the operand fragments as they pass: wave (wm, wn) takes row pair wn of
-  // each K-step (rows 16 FI wm + 32 wn + 16 u + r, u = 0, 1; lane (r, g) sees 8 of a row's 32 values)
+  // each K-step (rows 16 FI wm + 32 wn + 16 u + r, u = 0, 1; lane (r, g) sees 8 of a row's 32 values), which is its first pair.  The
+  // sums' instructions go between the group's matrix instructions, a few behind each: behind all of them they left the matrix
+  // pipe idle (and a branch on wn around them kept them there).
   float ss[2] = {0.f, 0.f};
   auto sumsq = [&](int pair, const gu4* f) {
-    if (NORM && wn == pair) {
+    if (NORM && pair == 0) {
 #pragma unroll
-      for (int u = 0; u < 2; u++)
+      for (int e = 0; e < 4; e++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
+        for (int u = 0; u < 2; u++) {
           float lo, hi;
-          unpack2<DT>(f[u][e], lo, hi);
+          gunpack<DT>(f[u][e], lo, hi);
           ss[u] = fmaf(lo, lo, ss[u]);
           ss[u] = fmaf(hi, hi, ss[u]);
         }
+      asm volatile("" : "+v"(ss[0]), "+v"(ss[1]));   // (here, not where the loop ends)
+#pragma unroll
+      for (int q = 0; q < 7; q++) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // a matrix instruction,
+        __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);   // five vector ones
+      }
     }
   };
+  auto frow = [&](int i) { return 16 * FI * wm + 16 * (NORM ? ((i + 2 * wn) & (FI - 1)) : i) + r; };   // tile row of accumulator row fragment i
 #define UVMI_SB() __builtin_amdgcn_sched_barrier(0)
 
   issue(sA0, sB0, 0);
@@ -252,27 +270,36 @@ void gemm_big_kernel(BigParams P) {
     }
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < FI; i++) rn[i] = sRS[16 * FI * wm + 16 * i + r];
+    for (int i = 0; i < FI; i++) rn[i] = sRS[frow(i)];
   }
 
   // ---- epilogue: accumulator (i, j): lane (r, g) holds C[m0 + 16 FI wm + 16 i + r][n0 + 64 wn + 16 j + 4 g + t], t = 0..3
+  uint4 res[EPI == 2 ? FI : 1][2];
+  if constexpr (EPI == 2) {
+    const int n = n0 + 64 * wn + 16 * g;
+#pragma unroll
+    for (int i = 0; i < FI; i++) {
+      const int row = m0 + frow(i);
+      res[i][0] = res[i][1] = uint4{0u, 0u, 0u, 0u};
+      if (row < P.M && n < P.N) {
+        const uint16_t* rp = (const uint16_t*)P.r + (int64_t)row * P.ldr + n;
+        res[i][0] = *(const uint4*)rp;
+        res[i][1] = *(const uint4*)(rp + 8);
+      }
+    }
+  }
 #pragma unroll
   for (int i = 0; i < FI; i++) {
-    const int row = m0 + 16 * FI * wm + 16 * i + r;
+    const int row = m0 + frow(i);
     if (EPI == 1) {
       // gate slab j, up slab j + 1 -> 4 outputs per slab pair; after the 2 x 2 transpose lane (r, g) holds the 8 consecutive
       // output columns 16 (g % 2) + 8 (g / 2) .. of the wave's 32
       uint32_t x0[2], x1[2];
 #pragma unroll
       for (int jp = 0; jp < 2; jp++) {
-        float o[4];
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-          const float gv = ground<DT>(acc[i][2 * jp][t] * rn[i]), uv = ground<DT>(acc[i][2 * jp + 1][t] * rn[i]);
-          o[t] = silu_round<DT>(gv) * uv;
-        }
-        (jp == 0 ? x0 : x1)[0] = gpack<DT>(o[0], o[1]);
-        (jp == 0 ? x0 : x1)[1] = gpack<DT>(o[2], o[3]);
+        const gf4 gv = acc[i][2 * jp] * rn[i], uv = acc[i][2 * jp + 1] * rn[i];
+        (jp == 0 ? x0 : x1)[0] = gswiglu2<DT>(gv[0], gv[1], uv[0], uv[1]);
+        (jp == 0 ? x0 : x1)[1] = gswiglu2<DT>(gv[2], gv[3], uv[2], uv[3]);
       }
       xpose2(x0[0], x1[0]);
       xpose2(x0[1], x1[1]);
@@ -311,7 +338,7 @@ void gemm_big_kernel(BigParams P) {
       }
     } else {
       // (with the stores of EPI 0 here the residual's loads come in the same pieces: 0 - 3 % slower; requested in the last iteration
-      // but one, the residual costs 56 registers and 10 % of the K = 1664 product)
+      // but one instead of behind the loop, the residual costs 56 registers and 10 % of the K = 1664 product)
       uint32_t lo[4], hi[4];
 #pragma unroll
       for (int j = 0; j < 4; j++) {
@@ -324,14 +351,13 @@ void gemm_big_kernel(BigParams P) {
       const int n = n0 + 64 * wn + 16 * g;
       if (row < P.M && n < P.N) {
         uint32_t wds[8] = {lo[0], hi[0], lo[1], hi[1], lo[2], hi[2], lo[3], hi[3]};
-        const uint16_t* rp = (const uint16_t*)P.r + (int64_t)row * P.ldr + n;
-        const uint4 q0 = *(const uint4*)rp, q1 = *(const uint4*)(rp + 8);
+        const uint4 q0 = res[i][0], q1 = res[i][1];
         const uint32_t rw[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
 #pragma unroll
         for (int e = 0; e < 8; e++) {
           float p0, p1, x0, x1;
-          unpack2<DT>(wds[e], p0, p1);   // the product, already rounded to the activation type
-          unpack2<DT>(rw[e], x0, x1);
+          gunpack<DT>(wds[e], p0, p1);   // the product, already rounded to the activation type
+          gunpack<DT>(rw[e], x0, x1);
           wds[e] = gpack<DT>(P.ca * x0 + P.cb * p0, P.ca * x1 + P.cb * p1);
         }
         uint16_t* cp = (uint16_t*)P.c + (int64_t)row * P.ldc + n;

@@ -37,9 +37,25 @@ template <int DT> __device__ __forceinline__ float silu_round(float gv) {
   else return ground<DT>(gv / (1.0f + __expf(-gv)));
 }
 template <int DT> __device__ __forceinline__ uint32_t gpack(float a, float b) {
-  const uint32_t lo = DT == UVMI_BF16 ? float_to_bf16(a) : float_to_half_bits(a);
-  const uint32_t hi = DT == UVMI_BF16 ? float_to_bf16(b) : float_to_half_bits(b);
-  return lo | (hi << 16);
+  if constexpr (DT == UVMI_BF16) return float2_to_bf16x2(a, b);   // one conversion for the two
+  else return (uint32_t)float_to_half_bits(a) | ((uint32_t)float_to_half_bits(b) << 16);
+}
+template <int DT> __device__ __forceinline__ void gunpack(uint32_t w, float& lo, float& hi) {
+  if (DT == UVMI_BF16) { lo = __uint_as_float(w << 16); hi = __uint_as_float(w & 0xffff0000u); }
+  else { lo = half_bits_to_float((uint16_t)(w & 0xffff)); hi = half_bits_to_float((uint16_t)(w >> 16)); }
+}
+// silu(gate) * up for two outputs: everything is rounded to the activation type in pairs (a third fewer instructions than one by one)
+template <int DT> __device__ __forceinline__ uint32_t gswiglu2(float g0, float g1, float u0, float u1) {
+  float a, b, c, d;
+  gunpack<DT>(gpack<DT>(g0, g1), a, b);
+  gunpack<DT>(gpack<DT>(u0, u1), c, d);
+  if constexpr (DT == UVMI_BF16) {   // (silu_round for two)
+    float sa, sb;
+    gunpack<DT>(gpack<DT>(a * __builtin_amdgcn_rcpf(1.0f + __expf(-a)), b * __builtin_amdgcn_rcpf(1.0f + __expf(-b))), sa, sb);
+    return gpack<DT>(sa * c, sb * d);
+  } else {
+    return gpack<DT>(silu_round<DT>(a) * c, silu_round<DT>(b) * d);
+  }
 }
 
 }  // namespace uvmi
