@@ -1050,3 +1050,31 @@ def test_native_call_refuses_what_the_general_one_refuses(monkeypatch):
     native = [says(*b) for b in bad]
     monkeypatch.setattr(D, "_native", lambda: lambda *a: None)
     assert native == [says(*b) for b in bad] and native[1] != "taken"
+
+
+@pytest.mark.parametrize("M,K,N,epi,tile", [(5000, 640, 3328, "swiglu", 128), (8192, 640, 3328, "swiglu", 256), (14000, 512, 640, "resid", 128),
+                                            (14000, 1664, 640, "resid", 256), (20000, 512, 640, "resid", 256), (33216, 1664, 640, "resid", 128),
+                                            (24576, 640, 656, "store", 128), (33216, 640, 656, "store", 256), (4096, 640, 96, "swiglu", 128)])
+def test_tile_of_passes_of_many_rows(M, K, N, epi, tile):
+    """The built-in choice between 256 x 256 and 128 x 128 tiles by their rounds of the device, on both sides of its lines: the bits of
+    the form that the rule names (the two sum K alike but take the pre-norm's squares in another order), and near the float64
+    product on rows at the tiles' edges."""
+    from ultraviolet_amd.kernels.gemm import RESID, STORE, SWIGLU, gemm_tn
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    a, w = (torch.randn(s, K, device="cuda", generator=g).bfloat16() for s in (M, N))
+    w = (w.float() / K ** 0.5).bfloat16()
+    kw = {"store": dict(norm_eps=1e-6), "swiglu": dict(norm_eps=1e-6, epilogue=SWIGLU),
+          "resid": dict(epilogue=RESID, resid=torch.randn(M, N, device="cuda", generator=g).bfloat16(), ca=0.75, cb=1.25)}[epi]
+    got = gemm_tn(a, w, **kw)
+    assert torch.equal(got, gemm_tn(a, w, config=5 if tile == 256 else 6, **kw))
+    rows = torch.tensor([0, 127, 128, 255, 256, M - 1], device="cuda")
+    x = a[rows].double()
+    if "norm_eps" in kw:
+        x = x * torch.rsqrt((x * x).mean(1, keepdim=True) + 1e-6)
+    p = (x @ w.double().t()).bfloat16().double()
+    if epi == "swiglu":
+        p = p.view(len(rows), N // 32, 2, 16)
+        p = (torch.nn.functional.silu(p[:, :, 0]).bfloat16().double() * p[:, :, 1]).reshape(len(rows), N // 2)
+    elif epi == "resid":
+        p = 0.75 * kw["resid"][rows].double() + 1.25 * p
+    assert bool(((got[rows].double() - p).abs() <= 8 * 2.0 ** -8 * p.abs().clamp_min(1.0)).all())

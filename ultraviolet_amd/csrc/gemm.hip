@@ -12,9 +12,8 @@ int gemm_stream_form(const uvmi_gemm_args* a, int cus);                         
 void gemm_stream_launch(const uvmi_gemm_args* a, int form, int cus, hipStream_t st);
 }
 
-// Rows from which the 256 x 256 tile of gemm_big.hip takes over (one workgroup per compute unit: it needs several rounds of
-// tiles to pay; measured on UV-50M's projections at 2 k - 33 k rows: from ~12 k rows it is the fastest form for every
-// projection, for the wide gate-up projection with its SwiGLU epilogue already from 4 k).
+// Rows from which a product may take the 256 x 256 tile of gemm_big.hip (one workgroup per compute unit) by big_tiles_pay; below, its
+// rounds of the device are too few and too empty on UV-50M's projections.
 constexpr int64_t BIG_MIN_ROWS = 12288, BIG_MIN_ROWS_SWIGLU = 4096;
 
 // what the 256 x 256 kernel assumes beyond uvmi_gemm_tn_supported: two slabs at least, 16-byte stores and residual loads
@@ -22,6 +21,19 @@ static bool big_ok(const uvmi_gemm_args* a) {
   if (a->K < 128 || ((uintptr_t)a->c % 16) != 0 || a->ldc % 8 != 0) return false;
   if (a->epilogue == UVMI_GEMM_RESID && (((uintptr_t)a->resid % 16) != 0 || a->ldr % 8 != 0)) return false;
   return true;
+}
+
+// Whether a pass of many rows takes 256 x 256 tiles rather than 128 x 128 ones.  A launch lasts as long as its rounds of the device: of
+// one 256 x 256 tile per compute unit, or of two 128 x 128 ones, which take about 0.6 of that.  us, 256 against 128, activations in
+// the last-level cache as a pass leaves them: gate-up with norm and SwiGLU 5000 rows, 2 rounds against 3, 43.0 / 33.2; 8192 rows, 2
+// against 4, 43.1 / 46.9; 10 000 rows, 3 against 5, 66.1 / 58.6; 18 432 rows, 4 against 8, 90.3 / 97.2; 20 000 rows, 5 against 8, 110.9 /
+// 105.6.  640 columns, K 1664: 18 432 rows, 1 against 2, 45.0 / 46.1 (50.8 / 62.9 with activations from memory); 24 576 rows, 2 against 2,
+// 81.7 / 53.3; 40 000 rows, 2 against 4, 88.7 / 95.3.  With a short K a last round of 128 x 128 tiles that fills a quarter of the device or
+// less takes half a round (K 512: 16 384 rows 22.9 / 20.4, 18 432 rows, 0.4 of a round, 22.8 / 24.1).
+static bool big_tiles_pay(const uvmi_gemm_args* a, int64_t t128, int64_t t256, int cus) {
+  const int64_t r256 = (t256 + cus - 1) / cus, slots = 2 * (int64_t)cus, rest = t128 % slots;
+  const int64_t halves128 = 2 * (t128 / slots) + (rest == 0 ? 0 : (a->K <= 768 && 4 * rest <= slots ? 1 : 2));
+  return 17 * r256 <= 5 * halves128;
 }
 
 extern "C" int uvmi_gemm_tn_supported(int dtype, int64_t M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc, int epilogue) {
@@ -62,15 +74,14 @@ extern "C" int uvmi_gemm_tn_ex(const uvmi_gemm_args* a, void* stream) {
   const int64_t t128 = ((a->M + 127) / 128) * (((int64_t)a->N + 127) / 128), t256 = ((a->M + 255) / 256) * (((int64_t)a->N + 255) / 256);
   const bool one_round = a->N % 256 == 0 && a->M >= (a->epilogue == UVMI_GEMM_SOFTCAP ? 384 : 512) && t256 <= cus && 8 * t256 >= 7 * (int64_t)cus && t128 > 2 * (int64_t)cus;
   const bool many_big_tiles = one_round || (a->M >= 1024 && t256 >= 2 * (int64_t)cus);
-  if (a->config == 5 || (a->config == 0 && (many_big_tiles || a->M >= (a->epilogue == UVMI_GEMM_SWIGLU ? BIG_MIN_ROWS_SWIGLU : BIG_MIN_ROWS)) && big_ok(a))) {
+  const bool rows_ok = a->M >= (a->epilogue == UVMI_GEMM_SWIGLU ? BIG_MIN_ROWS_SWIGLU : BIG_MIN_ROWS);
+  if (a->config == 5 || (a->config == 0 && (many_big_tiles || rows_ok) && big_ok(a))) {
     UVMI_REQUIRE(big_ok(a), UVMI_EUNSUPPORTED,
                  "uvmi_gemm_tn: config 5 (256 x 256 tiles) needs K >= 128, C (and the residual) 16-byte aligned, ldc (ldr) %% 8 == 0");
-    // An output whose width fills 128-wide tiles much better than 256-wide ones (N = 640: 5 tiles of 128 against 3 of 256, a
-    // sixth of which would be computed for nothing) runs on the 128 x 128 form of the same kernel (measured at 33 216 rows:
-    // the output projection 37.5 us against 40.8, the down projection 79.8 against 84.8).
+    // (a product of fewer rows whose many 256-wide tiles would be more than a tenth emptier than 128-wide ones takes those)
     const int64_t pad128 = ((int64_t)a->N + 127) / 128 * 128, pad256 = ((int64_t)a->N + 255) / 256 * 256;
-    const int tile = a->config == 0 && pad128 * 10 < pad256 * 9 ? 128 : 256;
-    gemm_big_launch(a, tile, (hipStream_t)stream);
+    const bool small = rows_ok ? !big_tiles_pay(a, t128, t256, cus) : pad128 * 10 < pad256 * 9;
+    gemm_big_launch(a, a->config == 0 && small ? 128 : 256, (hipStream_t)stream);
     UVMI_CHECK_LAUNCH("uvmi_gemm_tn(direct to LDS)");
     return UVMI_OK;
   }
