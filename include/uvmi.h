@@ -41,7 +41,7 @@ extern "C" {
 #define UVMI_I64 5
 
 /* Revision of the argument structs below (uvmi_version() returns the value the library was built with). */
-#define UVMI_ABI_VERSION 7
+#define UVMI_ABI_VERSION 8
 int uvmi_version(void);
 const char* uvmi_last_error(void);
 /* Number of compute units of the current device (used by the split heuristics); <0 on error. */
@@ -139,6 +139,7 @@ typedef struct uvmi_attn_args {
  * gate epilogue is always applied (post_vhat and post_gate are ignored: the kernel forms them; post_xsa may be NULL).
  * Needs the MFMA path (head_dim 64, an int8 cache or one in the q dtype), num_splits == 1, q dtype = activation dtype,
  * n_pairs 16 when rope. */
+struct uvmi_attn_oproj;
 typedef struct uvmi_attn_qkv_fuse {
   const void* qkv; int64_t row_stride;     /* elements */
   int ext_col;                             /* first gate-logit column */
@@ -150,7 +151,24 @@ typedef struct uvmi_attn_qkv_fuse {
                                                  every pos[b] must be below it */
   int n_pairs; int rope;
   float eps, xsa_eps;
+  const struct uvmi_attn_oproj* oproj;     /* optional: the output projection and the block's residual update in the same launch (below) */
 } uvmi_attn_qkv_fuse;
+
+/* The output projection behind the fused attention of a few rows (uvmi_attn_qkv_fuse.oproj): with z the row's (H * 64) result that
+ * uvmi_attn_args.out would hold, rounded to the q dtype (`out` is not written),
+ *   out[b] = ca * resid[b] + cb * round(z . w^T)
+ * - the attention half of the block's residual update (ultraviolet/model.py:321-335, 567-571), UVMI_GEMM_RESID's arithmetic.  A row's
+ * attention is computed by every workgroup that forms a part of its outputs, so the rows are few: uvmi_attn_oproj_rows(N) at most.
+ * Needs 8 query heads on 1 kv head, I64 indices, 16-byte aligned w with ldw % 8 == 0, N % 32 == 0 or N % 80 == 0. */
+struct uvmi_attn_oproj {
+  const void* w; int64_t ldw;              /* (N, 512) in the q dtype */
+  const void* resid; int64_t ldr;          /* (B, N); may be out itself */
+  void* out; int64_t ldo;                  /* (B, N) */
+  int N;
+  float ca, cb;
+};
+/* Most rows that uvmi_attn_oproj serves for N output columns on the current device; 0: none. */
+int uvmi_attn_oproj_rows(int N);
 /* The rotation table of the fused path: out (n_positions, 2 * n_pairs) fp32, row p = cos(p * inv_freq[j]) for j <
  * n_pairs, then sin, each rounded to round_dtype - the values uvmi_qkv_post forms per token (the reference keeps the same
  * table as a buffer of the model, ultraviolet/model.py:198-226). */

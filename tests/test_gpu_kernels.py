@@ -1078,3 +1078,77 @@ def test_tile_of_passes_of_many_rows(M, K, N, epi, tile):
     elif epi == "resid":
         p = 0.75 * kw["resid"][rows].double() + 1.25 * p
     assert bool(((got[rows].double() - p).abs() <= 8 * 2.0 ** -8 * p.abs().clamp_min(1.0)).all())
+
+
+def _fused_case(B, S, ring, kv, dtype, seed, any_ring=False):
+    """A fused decode launch on random data: (launch(out, caches, oproj), caches, extras)."""
+    from ultraviolet_amd.kernels.decode_attn import decode_attention_fused, rope_table
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    rn = lambda *s: torch.randn(*s, device=DEV, generator=g)
+    slots = B + 3
+    if kv == "int8":
+        k, v = (torch.randint(-127, 128, (slots, 1, S, 64), device=DEV, generator=g, dtype=torch.int8) for _ in range(2))
+        ks, vs = (torch.rand(slots, 1, S, device=DEV, generator=g).mul_(0.02).add_(0.005).half() for _ in range(2))
+    else:
+        k, v, ks, vs = rn(slots, 1, S, 64).to(dtype), rn(slots, 1, S, 64).to(dtype), None, None
+    qkv = rn(B, 656).to(dtype)
+    pos = torch.randint(0, 3 * S if ring else S, (B,), device=DEV, generator=g)
+    pos[0] = 3 * S - 1 if ring else S - 1
+    starts = torch.randint(0, 40, (B,), device=DEV, generator=g).clamp(max=pos)
+    rows = torch.randperm(slots, device=DEV, generator=g)[:B]
+    if B > 4:
+        rows[3] = -1
+    tok = torch.randint(0, 100, (B,), device=DEV, generator=g)
+    ve = rn(100, 1, 64).to(dtype)
+    table = rope_table(torch.rand(16, device=DEV, generator=g), 3 * S + 8, dtype)
+    xsa = torch.rand(8, device=DEV, generator=g)
+    fuse = dict(ext_col=640, has_gate=True, tok=tok, ve_table=ve, vocab=100, rope_table=table, n_pairs=16, rope=True, eps=1e-6, xsa_eps=1e-6)
+
+    def launch(out, oproj=None):
+        c = [None if t is None else t.clone() for t in (k, v, ks, vs)]
+        decode_attention_fused(qkv, 8, c[0], c[1], pos, starts, 0.14, window=S if ring else 0, ring=ring, k_scale=c[2], v_scale=c[3], xsa=xsa, out=out,
+                               fuse=dict(fuse, oproj=oproj), rows=rows, any_ring=any_ring)
+        return c
+    return launch, rn
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("kv", ["int8", "unquantized"])
+@pytest.mark.parametrize("S,ring", [(128, False), (1056, False), (256, True), (1024, True), (100, True)])
+@pytest.mark.parametrize("B,N", [(1, 640), (8, 640), (9, 640), (24, 640), (25, 640), (32, 640), (6, 160), (40, 256), (64, 256)])
+def test_output_projection_in_the_attention_launch(B, N, S, ring, kv, dtype):
+    """uvmi_attn_oproj against the two launches it stands for - the fused attention, then the GEMM with the residual update: the
+    same cache words and the same bits of the output, at 4 and 8 waves per row, on linear caches, rings that have wrapped and
+    short rings, with every size of a workgroup's part and rows on both sides of its lines, and a padding row."""
+    from ultraviolet_amd.kernels.gemm import RESID, gemm_tn
+    launch, rn = _fused_case(B, S, ring, kv, dtype, seed=B * 7 + S + N, any_ring=S == 100)
+    w, x = (rn(N, 512) / 512 ** 0.5).to(dtype), rn(B, N + 8).to(dtype)[:, :N]
+    z = torch.empty(B, 8, 64, device=DEV, dtype=dtype)
+    want_cache = launch(z)
+    want = gemm_tn(z.view(B, 512), w, epilogue=RESID, resid=x, ca=0.75, cb=1.25)
+    zn = torch.full_like(z, 7.0)
+    full = torch.full((B, N + 8), 7.0, device=DEV, dtype=dtype)
+    got_cache = launch(zn, dict(w=w, resid=x, out=full[:, :N], ca=0.75, cb=1.25))
+    for a, b in zip(got_cache, want_cache):
+        assert a is None and b is None or torch.equal(a, b)
+    assert bool((full[:, N:] == 7.0).all()) and bool((zn == 7.0).all())
+    d = (full[:, :N].double() - want.double()).abs()
+    assert torch.equal(full[:, :N], want), (int((d > 0).sum()), float(d.max()))
+    again = torch.empty_like(full)
+    launch(zn, dict(w=w, resid=x, out=again[:, :N], ca=0.75, cb=1.25))
+    assert torch.equal(again[:, :N], full[:, :N])
+    inplace = x.clone()
+    launch(zn, dict(w=w, resid=inplace, out=inplace, ca=0.75, cb=1.25))
+    assert torch.equal(inplace, want)
+
+
+def test_output_projection_in_the_attention_launch_refuses():
+    """Too many rows, widths no part divides, other indices: refused before anything is launched."""
+    from ultraviolet_amd import _lib as L
+    assert L.lib().uvmi_attn_oproj_rows(640) == 32 and L.lib().uvmi_attn_oproj_rows(48) == 0
+    for B, N in ((33, 640), (4, 48)):
+        launch, rn = _fused_case(B, 128, False, "int8", torch.bfloat16, 1)
+        h = torch.full((B, N), 7.0, device=DEV, dtype=torch.bfloat16)
+        with pytest.raises(L.UvmiError):
+            launch(torch.empty(B, 8, 64, device=DEV, dtype=torch.bfloat16), dict(w=rn(N, 512).bfloat16(), resid=h, out=h, ca=1.0, cb=1.0))
+        assert bool((h == 7.0).all())

@@ -46,7 +46,12 @@ class AttnArgs(C.Structure):
 class AttnQkvFuse(C.Structure):
     _fields_ = [("qkv", C.c_void_p), ("row_stride", C.c_int64), ("ext_col", C.c_int), ("has_gate", C.c_int), ("tok", C.c_void_p),
                 ("ve_table", C.c_void_p), ("vocab", C.c_int64), ("has_ve", C.c_int), ("rope_table", C.c_void_p), ("rope_positions", C.c_int),
-                ("n_pairs", C.c_int), ("rope", C.c_int), ("eps", C.c_float), ("xsa_eps", C.c_float)]
+                ("n_pairs", C.c_int), ("rope", C.c_int), ("eps", C.c_float), ("xsa_eps", C.c_float), ("oproj", C.c_void_p)]
+
+
+class AttnOproj(C.Structure):
+    _fields_ = [("w", C.c_void_p), ("ldw", C.c_int64), ("resid", C.c_void_p), ("ldr", C.c_int64), ("out", C.c_void_p), ("ldo", C.c_int64),
+                ("N", C.c_int), ("ca", C.c_float), ("cb", C.c_float)]
 
 
 class GemmArgs(C.Structure):
@@ -142,7 +147,7 @@ class PromptTablesArgs(C.Structure):   # struct uvmi_prompt_tables_args
 OP_GEMM, OP_DECODE_ATTN, OP_QKV_POST, OP_PREFILL_ATTN, OP_NORM = range(5)   # UVMI_OP_*
 
 _lib = None
-ABI_VERSION = 7   # UVMI_ABI_VERSION of include/uvmi.h
+ABI_VERSION = 8   # UVMI_ABI_VERSION of include/uvmi.h
 
 
 def lib() -> C.CDLL:
@@ -249,7 +254,7 @@ def require_cuda(*ts: torch.Tensor) -> None:
 
 EXPORTS = ["uvmi_version", "uvmi_last_error", "uvmi_device_cus", "uvmi_quantize_rows", "uvmi_dequantize_rows",
            "uvmi_kv_write", "uvmi_kv_append", "uvmi_decode_attn", "uvmi_decode_attn_workspace_bytes",
-           "uvmi_default_splits", "uvmi_decode_attn_path", "uvmi_decode_attn_noalloc", "uvmi_decode_attn_probe", "uvmi_prefill_attn", "uvmi_prefill_attn_workspace_bytes",
+           "uvmi_default_splits", "uvmi_decode_attn_path", "uvmi_attn_oproj_rows", "uvmi_decode_attn_noalloc", "uvmi_decode_attn_probe", "uvmi_prefill_attn", "uvmi_prefill_attn_workspace_bytes",
            "uvmi_prefill_attn_path", "uvmi_fused_sample", "uvmi_philox4x32_10",
            "uvmi_embed_norm", "uvmi_add_norm", "uvmi_qkv_post", "uvmi_attn_post", "uvmi_swiglu", "uvmi_swiglu_norm",
            "uvmi_prefill_attn_bwd", "uvmi_prefill_attn_bwd_workspace_bytes", "uvmi_sched_compact", "uvmi_sched_commit", "uvmi_sched_commit_dense", "uvmi_sched_admit", "uvmi_sched_expand", "uvmi_sched_harvest", "uvmi_sched_plan_admit", "uvmi_sched_step_plan", "uvmi_run_ops", "uvmi_prompt_tables", "uvmi_rope_table", "uvmi_gemm_tn_supported", "uvmi_gemm_tn", "uvmi_gemm_tn_ex"]

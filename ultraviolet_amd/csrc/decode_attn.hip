@@ -58,6 +58,10 @@ struct AttnParams {
   int64_t f_sqkv, f_vocab;
   int f_ext, f_rope, f_rope_n, f_has_ve, f_has_gate;
   float f_eps, f_xsa_eps;
+  // optional output projection of the row in the same launch (uvmi_attn_oproj)
+  const void* o_w; const void* o_r; void* o_out;
+  int64_t o_ldw, o_ldr, o_ldo;
+  float o_ca, o_cb;
 };
 
 // Key range of a row and how it is cut.  The span starts at lo rounded down to 32 so tiles stay aligned to the
@@ -185,34 +189,46 @@ struct AttnState {
 // terms that hold all its bits.  Latency-bound like every launch on so few keys, the arithmetic costs little: a ring of whole tiles
 // at 16-bit probabilities takes 4.9 us there, 64 rows of up to 107 keys 5.3 / 4.9, 1000 rows of up to 249 keys 10.2 / 8.0; on a 16-bit
 // cache 5.0 / 5.1, 5.2 / 5.1 and 11.1 / 11.2.
+// OPF (with FUSE): the output projection and the residual update in the same launch, for a few rows (uvmi_attn_oproj).  A launch of
+// one lasts 2.5 us on a row, nearly all of it the start of a launch and a trip for 655 KB of weights, in the middle of a chain of
+// launches that do little more.  Here blockIdx.y is a part of OPF 16-column fragments of the outputs: every part's workgroup computes
+// the row's attention for itself (the device is idle otherwise, and the parts of a row sit on one XCD, whose L2 gives them its keys),
+// while its 16 OPF rows of the weight (32 .. 80 KB) go from memory straight into LDS behind the first tile's request; part 0 writes the
+// cache.  The waves then split the 512 of the contraction and meet in LDS once more.  The bits are those of the two launches.  LDS rows are 1 KB: the 16-byte chunks are
+// xor-ed with the row, so the operand reads (lane (r, g): chunk 4 s + g of row r) spread over the banks.
 // PROBE (uvmi_decode_attn_probe; measurement only, the output is meaningless): 1 - the kernel's memory stream without its
 // arithmetic: every tile is loaded exactly as in the real kernel and folded into the state with a few xors; 2 - its
 // arithmetic without the stream: tiles are made up in registers, nothing is loaded from the cache.
-template <int QDT, int ODT, int WPR, bool FUSE, bool KV16 = false, bool FAST = false, int PROBE = 0, bool BYSLOT = false, bool ANYRING = false>
-__global__ __launch_bounds__(WPR > 4 ? 64 * WPR : 256) __attribute__((amdgpu_waves_per_eu(4, 4)))
+template <int QDT, int ODT, int WPR, bool FUSE, bool KV16 = false, bool FAST = false, int PROBE = 0, bool BYSLOT = false, bool ANYRING = false, int OPF = 0>
+__global__ __launch_bounds__(WPR > 4 ? 64 * WPR : 256) __attribute__((amdgpu_waves_per_eu(OPF == 0 ? 4 : WPR / 4, OPF == 0 ? 4 : WPR / 4)))
 void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_rows, const void* a_q, const void* a_tok, int a_items,
                        int a_idx64, int a_splits, int a_kh, AttnParams P) {
   P.pos = a_pos; P.starts = a_starts; P.rows = a_rows; P.n_items = a_items; P.idx64 = a_idx64; P.splits = a_splits; P.KH = a_kh;
   if constexpr (BYSLOT || ANYRING) P.ring = 1;
-  if constexpr (ANYRING) P.splits = 1;
+  if constexpr (ANYRING || OPF != 0) P.splits = 1;
   constexpr bool BIASED = !KV16 && !ANYRING;   // int8 codes enter the MFMAs with the biases of the cheap conversion
   if constexpr (FAST) { P.idx64 = 1; P.splits = 1; P.KH = 1; P.G = 8; P.H = 8; P.hd = 64; P.chunk_keys = 0; }
   if (FUSE) P.f_qkv = a_q; else P.q = a_q;
   constexpr int BW = WPR > 4 ? WPR : 4, IPB = BW / WPR;  // waves and items per block
   __shared__ __attribute__((aligned(16))) float sh_o[BW][16][68];
   __shared__ __attribute__((aligned(16))) float sh_ml[BW][16][4];
-  __shared__ float sh_post[4][80];  // epilogue operands of the item whose first wave this is: v_hat[64], gate[8], xsa[8]
-  __shared__ float sh_cur[FUSE ? 4 : 1][72];  // own key of that item: score per head [8], dequantised v [64]
-  __shared__ __attribute__((aligned(16))) uint16_t sh_q[FUSE ? 4 : 1][8][64];  // the item's q as fp16 operand words
-  __shared__ float sh_qs[FUSE ? 4 : 1][8];                                      // and their sum per head
-  __shared__ float sh_kq[FUSE ? 4 : 1][64];   // the own key's int8 codes (as floats), for its score against every head
+  static_assert(OPF == 0 || (FUSE && WPR >= 4 && QDT == ODT), "one row per workgroup");
+  constexpr int NIW = BW - WPR + 1;                      // an item's operands are at the index of its first wave
+  __shared__ float sh_post[NIW][80];  // epilogue operands of the item whose first wave this is: v_hat[64], gate[8], xsa[8]
+  __shared__ float sh_cur[FUSE ? NIW : 1][72];  // own key of that item: score per head [8], dequantised v [64]
+  __shared__ __attribute__((aligned(16))) uint16_t sh_q[FUSE ? NIW : 1][8][64];  // the item's q as fp16 operand words
+  __shared__ float sh_qs[FUSE ? NIW : 1][8];                                      // and their sum per head
+  __shared__ float sh_kq[FUSE ? NIW : 1][64];   // the own key's int8 codes (as floats), for its score against every head
+  __shared__ __attribute__((aligned(1024))) unsigned char sh_w[OPF ? OPF * 16 * 1024 : 16];   // OPF: the part's rows of the weight
+  __shared__ __attribute__((aligned(16))) uint16_t sh_z[OPF ? 512 : 8];                       // the row's attention output
+  __shared__ __attribute__((aligned(16))) float sh_part[OPF ? 8 : 1][OPF ? OPF * 16 : 4];     // and its products by 64 of the contraction
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wsub = wave % WPR;
   int64_t item = (int64_t)blockIdx.x * IPB + wave / WPR;  // wave-uniform
   const bool live_item = item < P.n_items;
   if (!live_item) {
-    if (WPR == 1) return;
+    if (WPR == 1 || OPF != 0) return;   // (OPF: the whole workgroup)
     item = P.n_items - 1;  // keep the wave for the barrier below; it does no work
   }
   // (items fit 31 bits, host-checked; one split and one kv head - the engine's shape - need no division)
@@ -271,7 +287,7 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
   const float* pg_src = !FUSE && has_post && P.post_gate ? P.post_gate + (int64_t)b * P.H + hsafe : anyf;
   const float* px_src = has_post && P.post_xsa ? P.post_xsa + hsafe : anyf;
   const float pv_val = *pv_src, pg_val = *pg_src, px_val = *px_src;
-  const RowPlan rp = plan_row(P, ri, b, FUSE, FAST || ANYRING);
+  const RowPlan rp = plan_row(P, ri, b, FUSE, FAST || ANYRING || OPF != 0);
   // FUSE: the row of the rotation table (cos / sin of the row's position per frequency, already rounded to the activation
   // type): prep_q reads its 32 values as scalars, the lane that owns dim d of the own key reads its own pair
   const int rope_row = rp.pc < 0 ? 0 : (rp.pc < P.f_rope_n ? rp.pc : P.f_rope_n - 1);
@@ -392,6 +408,11 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
     const float sf = fmaxf(half_bits_to_float(sb), 1e-30f);
     return fminf(fmaxf(__builtin_rintf(__fdiv_rn(x, sf)), -127.0f), 127.0f);
   };
+  // OPF: this thread's output column and its residual
+  const int col = OPF == 0 ? 0 : (int)(blockIdx.y * (OPF * 16) + threadIdx.x);
+  const bool mine = (int)threadIdx.x < OPF * 16;
+  uint16_t rraw = 0;
+  const bool writer = OPF == 0 || blockIdx.y == 0;   // of the row's cache entry
   auto own_k = [&](uint16_t raw, float kcs, float ksn) {
     float k = cvt_in(raw);
     const float rs = rsqrtf(bfly_sum(k * k) * (1.0f / 64.0f) + P.f_eps);
@@ -402,7 +423,7 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
     }
     uint16_t sbk = 0;
     float kq;   // what the cache holds for this lane's dim: the int8 code, or (16-bit cache) k itself
-    const int slot = ring_slot(P, rp.pc);
+    const int slot = writer ? ring_slot(P, rp.pc) : P.S;
     if constexpr (KV16) {
       kq = k;   // on the cache type's grid already
       if (slot < P.S)
@@ -443,7 +464,7 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
       v = ve_add(v, gv, cvt_in(raw_ve), rq);
     }
     const float nv = fmaxf(sqrtf(bfly_sum(v * v)), P.f_xsa_eps);
-    const int slot = ring_slot(P, rp.pc);
+    const int slot = writer ? ring_slot(P, rp.pc) : P.S;
     if constexpr (KV16) {
       if (slot < P.S)
         ((uint16_t*)P.vc)[(int64_t)rp.cb * P.svb + (int64_t)h * P.svh + (int64_t)slot * P.svs + lane] =
@@ -815,6 +836,19 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
     // one burst of more than half the launch's bytes.)
     TileX TA, TB;
     load_tile(slot, TA);
+    if constexpr (OPF != 0) {
+      rraw = ((const uint16_t*)P.o_r)[(int64_t)b * P.o_ldr + (mine ? col : 0)];
+      // wave w fetches rows w, w + BW, .. of the part: one load is one row
+      // (buffer loads: behind a global load into LDS the compiler waits for every load before it uses one)
+      const uint32_t ldw2 = (uint32_t)P.o_ldw * 2;
+      const __amdgpu_buffer_rsrc_t rOW = __builtin_amdgcn_make_buffer_rsrc((void*)((const uint16_t*)P.o_w + (int64_t)(blockIdx.y * (OPF * 16)) * P.o_ldw), 0,
+                                                                           (int)((OPF * 16 - 1) * ldw2 + 1024), 0x00020000);
+#pragma unroll
+      for (int i = 0; i < OPF * 16 / BW; i++) {
+        const int r = wave + BW * i;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rOW, (__attribute__((address_space(3))) void*)(sh_w + r * 1024), 16, 16 * (lane ^ (r & 7)), r * ldw2, 0, 0);
+      }
+    }
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (!FUSE) {
       prep_q();
@@ -826,7 +860,9 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
       const bool own = live && rp.pc >= 0;
       if (wsub == 0) prep_q_item(rc0, rc1, rs0, rs1);
       else if (WPR > 1 && wsub == VW && own) own_v(raw_a, raw_ve);  // needs no q: done while the first wave prepares it
-      if (WPR > 1) __syncthreads(); else __builtin_amdgcn_wave_barrier();
+      if (OPF != 0) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // (not for the weight's rows, as __syncthreads would)
+      else if (WPR > 1) __syncthreads();
+      else __builtin_amdgcn_wave_barrier();
       fetch_q();
       if (own && wsub == 0) {
         own_k(raw_a, kcs, ksn);
@@ -860,7 +896,7 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
   // ---- reduce l and sum P' over the 4 lane groups of a column
   const float lsum = xsum32(xsum16(st.lrun)), ps = xsum32(xsum16(st.psum));
   const float m2 = st.mrun == -INFINITY ? -INFINITY : st.mrun * c;  // exp2 domain
-  if (!FAST && !ANYRING && rp.nsplit > 1) {
+  if (!FAST && !ANYRING && OPF == 0 && rp.nsplit > 1) {
     // ---- a chunk of a cut row: stream B is merged into stream A (lanes n and n ^ 8: a rotation by 8 inside a row of 16
     // lanes, a DPP move), the WPR waves of the item through LDS, and the item's first wave writes the partial state
     const float m_o = dpp_mov<0x128>(m2), l_o = dpp_mov<0x128>(lsum), ps_o = dpp_mov<0x128>(ps);
@@ -929,9 +965,12 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
 #pragma unroll
   for (int i = 0; i < 4; i++) *(float4*)&sh_o[wave][m][16 * g + 4 * i] = float4{st.O[0][i], st.O[1][i], st.O[2][i], st.O[3][i]};
   if (g == 0) *(float4*)&sh_ml[wave][m][0] = float4{m2, lsum, ps, 0.f};
-  if (WPR > 1) __syncthreads(); else __builtin_amdgcn_wave_barrier();
+  if (OPF != 0) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  else if (WPR > 1) __syncthreads();
+  else __builtin_amdgcn_wave_barrier();
   if (!live) return;
-  if (WPR > 4 && wsub >= 4) return;                // (four waves cover the item's 512 outputs, 2 each)
+  if (WPR > 4 && wsub >= 4 && OPF == 0) return;    // (four waves cover the item's 512 outputs, 2 each)
+  if (WPR <= 4 || wsub < 4) {
   constexpr int NV = 8 / (WPR > 4 ? 4 : WPR), TPH = 64 / NV;   // values per thread, threads per head
   const int ti = wsub * 64 + lane;
   const int eh = ti / TPH, d0 = (ti % TPH) * NV;   // head and first dim of this thread
@@ -1012,7 +1051,17 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
 #pragma unroll
     for (int j = 0; j < NV; j++) o[j] *= inv;
   }
-  if (eh < G) {
+  if constexpr (OPF != 0) {
+    uint32_t w[NV / 2];
+#pragma unroll
+    for (int j = 0; j < NV / 2; j++) {
+      const uint32_t l16 = ODT == UVMI_BF16 ? float_to_bf16(o[2 * j]) : float_to_half_bits(o[2 * j]);
+      const uint32_t h16 = ODT == UVMI_BF16 ? float_to_bf16(o[2 * j + 1]) : float_to_half_bits(o[2 * j + 1]);
+      w[j] = l16 | (h16 << 16);
+    }
+    static_assert(OPF == 0 || NV == 2, "");
+    *(uint32_t*)&sh_z[eh * 64 + d0] = w[0];
+  } else if (eh < G) {
     const int64_t off = (int64_t)b * P.sob + (int64_t)(h * G + eh) * P.soh + d0;
     if constexpr (ODT == UVMI_F32) {
       float* op = (float*)P.out + off;
@@ -1032,6 +1081,45 @@ void attn_mfma_i8_hd64(const void* a_pos, const void* a_starts, const void* a_ro
       if constexpr (NV == 8) *(uint4*)op = uint4{w[0], w[1], w[2], w[3]};
       else if constexpr (NV == 4) *(uint2*)op = uint2{w[0], w[1]};
       else *(uint32_t*)op = w[0];
+    }
+  }
+  }
+  if constexpr (OPF != 0) {
+    // ---- out = ca resid + cb round(z . w^T) for the part's columns, with the sums of the streaming GEMM's smallest tile, which is what
+    // so few rows would take: eight slabs of 64, each summed by itself, then added in order - the same bits.  The weight fragment
+    // is the MFMA's first operand, z (in every column) its second: lane (0, g) holds columns 4 g .. of each fragment
+    __builtin_amdgcn_s_waitcnt(0x0f70);   // this wave's rows of the weight have landed
+    __syncthreads();
+    constexpr int SW = 8 / BW;            // slabs per wave
+#pragma unroll
+    for (int i = 0; i < SW; i++) {
+      const int slab = wave * SW + i;
+      f4 pr[OPF];
+#pragma unroll
+      for (int f = 0; f < OPF; f++) pr[f] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < 2; s++) {
+        const int ch = 8 * slab + 4 * s + g;   // chunk of 8 of the contraction
+        const u4 zw = *(const u4*)&sh_z[8 * ch];
+        const h8 z = as_h8(zw.x, zw.y, zw.z, zw.w);
+#pragma unroll
+        for (int f = 0; f < OPF; f++) {
+          const u4 x = *(const u4*)(sh_w + (16 * f + m) * 1024 + 16 * (ch ^ (m & 7)));
+          pr[f] = mfma_kv<QDT>(as_h8(x.x, x.y, x.z, x.w), z, pr[f]);
+        }
+      }
+      if (m == 0) {
+#pragma unroll
+        for (int f = 0; f < OPF; f++) *(f4*)&sh_part[slab][16 * f + 4 * g] = pr[f];
+      }
+    }
+    __syncthreads();
+    if (mine) {
+      float p = sh_part[0][threadIdx.x];
+#pragma unroll
+      for (int w = 1; w < 8; w++) p += sh_part[w][threadIdx.x];
+      const float y = P.o_ca * cvt_in(rraw) + P.o_cb * rq(p);
+      ((uint16_t*)P.o_out)[(int64_t)b * P.o_ldo + col] = QDT == UVMI_BF16 ? float_to_bf16(y) : float_to_half_bits(y);
     }
   }
 }
@@ -1260,6 +1348,20 @@ static bool mfma16_ok(const uvmi_attn_args* a) {
   return true;
 }
 
+// Fragments per workgroup for an output projection of N columns behind the attention of `rows` rows: the smallest part with which every
+// workgroup has a compute unit of its own, since the part's rows of the weight are most of what the projection adds to the launch (N 640,
+// two steps of ten layers: 1 row 346 us with 2 fragments, 368 with 5; 8 rows 371 / 384, with 4 375; 16 rows 376 with 4, 383 with 5; as two launches
+// 382, 409, 406; 32 rows 401 with 5, 427; 48 rows with 8 fragments, 128 KB, 419 against 428, and no room for the states of eight waves: not
+// built).  0: too many rows.
+static int oproj_fragments(int N, int64_t rows) {
+  int cus = uvmi_device_cus();
+  if (cus <= 0) cus = 256;
+  const int64_t pad = rows < 8 ? rows : (rows + 7) / 8 * 8;
+  for (int f : {2, 4, 5})
+    if (N > 0 && N % (16 * f) == 0 && pad * (N / (16 * f)) <= cus) return f;
+  return 0;
+}
+
 }  // namespace uvmi
 
 using namespace uvmi;
@@ -1284,6 +1386,18 @@ extern "C" int uvmi_default_splits(int64_t n_bk, int ctx, int n_cus) {
   if (s > 64) s = 64;
   if (s < 1) s = 1;
   return (int)s;
+}
+
+extern "C" int uvmi_attn_oproj_rows(int N) {
+  int cus = uvmi_device_cus();
+  if (cus <= 0) cus = 256;
+  int rows = 0;
+  for (int f : {2, 4, 5})
+    if (N > 0 && N % (16 * f) == 0) {
+      const int most = cus / (N / (16 * f));
+      rows = rows > most ? rows : most;
+    }
+  return rows < 8 ? rows : rows / 8 * 8;
 }
 
 extern "C" int uvmi_decode_attn_path(const uvmi_attn_args* a) {
@@ -1313,6 +1427,8 @@ static int decode_attn_launch(const uvmi_attn_args* a, void* ws, size_t ws_bytes
   P.ws_o = P.ws_m = P.ws_l = nullptr;
   P.post_vhat = a->post_vhat; P.post_gate = a->post_gate; P.post_xsa = a->post_xsa; P.post_dt = a->post_round_dtype;
   P.f_qkv = nullptr; P.f_rope_tab = nullptr; P.f_rope_n = 1; P.f_rope = 0;
+  P.o_w = P.o_r = nullptr; P.o_out = nullptr; P.o_ldw = P.o_ldr = P.o_ldo = 0; P.o_ca = P.o_cb = 0.f;
+  int opf = 0;   // 16-column fragments of the output projection per workgroup
   if (const uvmi_attn_qkv_fuse* f = a->fuse) {
     UVMI_REQUIRE((mfma_ok(a) || mfma16_ok(a)) && a->num_splits == 1, UVMI_EUNSUPPORTED,
                  "uvmi_decode_attn: fused QKV post-processing needs the MFMA kernel (head_dim 64, int8 cache or one of the q dtype, aligned rows) and num_splits == 1");
@@ -1327,6 +1443,16 @@ static int decode_attn_launch(const uvmi_attn_args* a, void* ws, size_t ws_bytes
     P.f_tok = f->tok; P.f_ve = f->ve_table; P.f_vocab = f->vocab; P.f_has_ve = f->has_ve ? 1 : 0;
     P.f_rope_tab = f->rope_table; P.f_rope_n = f->rope ? f->rope_positions : 1; P.f_rope = f->rope ? 1 : 0; P.f_eps = f->eps; P.f_xsa_eps = f->xsa_eps;
     P.post_vhat = nullptr; P.post_gate = nullptr;
+    if (const struct uvmi_attn_oproj* o = f->oproj) {
+      opf = oproj_fragments(o->N, a->B);
+      UVMI_REQUIRE(opf != 0 && a->KH == 1 && a->H == 8 && a->idx_dtype == UVMI_I64 && !probe, UVMI_EUNSUPPORTED,
+                   "uvmi_decode_attn: the output projection in the launch needs 8 query heads on 1 kv head, I64 indices, N %% 32 == 0 or N %% 80 == 0 "
+                   "and at most uvmi_attn_oproj_rows(N) rows (N %d, %d rows)", o->N, a->B);
+      UVMI_REQUIRE(o->w && o->resid && o->out && ((uintptr_t)o->w % 16) == 0 && ((uintptr_t)o->resid % 2) == 0 && ((uintptr_t)o->out % 2) == 0 &&
+                       o->ldw >= 512 && o->ldw % 8 == 0 && o->ldr >= o->N && o->ldo >= o->N && (int64_t)o->N * o->ldw * 2 < (1LL << 31), UVMI_EINVAL,
+                   "uvmi_decode_attn: bad output projection layout");
+      P.o_w = o->w; P.o_ldw = o->ldw; P.o_r = o->resid; P.o_ldr = o->ldr; P.o_out = o->out; P.o_ldo = o->ldo; P.o_ca = o->ca; P.o_cb = o->cb;
+    }
   }
   if (a->post_vhat && !a->fuse) {
     UVMI_REQUIRE((mfma_ok(a) || mfma16_ok(a)) && a->num_splits == 1, UVMI_EUNSUPPORTED,
@@ -1378,6 +1504,7 @@ static int decode_attn_launch(const uvmi_attn_args* a, void* ws, size_t ws_bytes
         if (wpr == 2 && !a->fuse && P.n_items * 2 > (int64_t)cus * 5) wpr = 1;
       }
     }
+    if (opf && wpr < 4) wpr = 4;
     P.gran = 32 * wpr;
     if (P.chunk_keys) P.chunk_keys = (P.chunk_keys + P.gran - 1) / P.gran * P.gran;
     const int ipb = wpr > 4 ? 1 : 4 / wpr;
@@ -1432,7 +1559,28 @@ static int decode_attn_launch(const uvmi_attn_args* a, void* ws, size_t ws_bytes
     // rings that are streamed by slot once they have wrapped (BYSLOT): the window is the ring, S a power of two
     const bool by_slot = a->ring && a->window == a->S && (a->S & (a->S - 1)) == 0 && a->num_splits == 1 && !probe;
     const bool fast = !kv16 && a->num_splits == 1 && a->KH == 1 && a->H == 8 && a->idx_dtype == UVMI_I64;
-    if (any_ring(a) && !probe) {
+    if (opf) {
+      // (the parts of a row on one XCD: workgroup ids go round-robin over the eight, and a part's ids begin at a multiple of eight)
+      const dim3 og((unsigned)(a->B < 8 ? a->B : (a->B + 7) / 8 * 8), (unsigned)(a->fuse->oproj->N / (16 * opf)));
+#define UVMI_LO(QD, W, K16, FA, BS, AR, F) hipLaunchKernelGGL((attn_mfma_i8_hd64<QD, QD, W, true, K16, FA, 0, BS, AR, F>), og, blk, 0, st, UVMI_LEAD, P)
+#define UVMI_LOF(QD, F)                                                                                                       \
+  do {                                                                                                                        \
+    if (any_ring(a)) { if (kv16) UVMI_LO(QD, 4, true, false, false, true, F); else UVMI_LO(QD, 4, false, false, false, true, F); } \
+    else if (by_slot) { if (kv16) UVMI_LO(QD, 4, true, false, true, false, F); else UVMI_LO(QD, 4, false, true, true, false, F); } \
+    else if (kv16) UVMI_LO(QD, 4, true, false, false, false, F);                                                              \
+    else UVMI_LO(QD, 4, false, true, false, false, F);                                                                        \
+  } while (0)
+#define UVMI_LOT(F)                                                                                                           \
+  do {                                                                                                                        \
+    if (wpr == 8) {   /* (int8 caches of 512 slots or more, rings among them) */                                              \
+      if (a->q_dtype == UVMI_F16) UVMI_LO(UVMI_F16, 8, false, true, false, false, F); else UVMI_LO(UVMI_BF16, 8, false, true, false, false, F); \
+    } else if (a->q_dtype == UVMI_F16) UVMI_LOF(UVMI_F16, F); else UVMI_LOF(UVMI_BF16, F);                                    \
+  } while (0)
+      if (opf == 2) UVMI_LOT(2); else if (opf == 4) UVMI_LOT(4); else UVMI_LOT(5);
+#undef UVMI_LOT
+#undef UVMI_LO
+#undef UVMI_LOF
+    } else if (any_ring(a) && !probe) {
 #define UVMI_LR(QD, W, FU, K16) hipLaunchKernelGGL((attn_mfma_i8_hd64<QD, QD, W, FU, K16, false, 0, false, true>), grid, blk, 0, st, UVMI_LEAD, P)
 #define UVMI_LRW(QD, FU, K16) do { if (wpr == 4) UVMI_LR(QD, 4, FU, K16); else if (wpr == 2) UVMI_LR(QD, 2, FU, K16); else UVMI_LR(QD, 1, FU, K16); } while (0)
 #define UVMI_LRF(QD) do { if (a->fuse) { if (kv16) UVMI_LRW(QD, true, true); else UVMI_LRW(QD, true, false); } \

@@ -136,7 +136,7 @@ def _swiglu_norm(b: dict, h: Tensor, n: int, dt_code: int, cfg: UVConfig, eps: f
 class UVEngine:
     def __init__(self, weights: UVWeights, max_tokens: int, skinny_rows: int = 192, fold_qkv_rows: int = 1 << 30, fold_o_rows: int = 1 << 30,
                  fold_gu_rows: int = 1 << 30, lean: bool = True, fold: bool = True, gemm_config: int = 0,
-                 tiled_prefill: bool = True, big_rows: int = 12288, fold_down_rows: tuple = (0, 5120), general_skinny_rows: int = 384):
+                 tiled_prefill: bool = True, big_rows: int = 12288, fold_down_rows: tuple = (0, 5120), general_skinny_rows: int = 384, oproj_rows: int | None = None):
         """max_tokens: largest number of token rows one forward call processes (decode rows + packed prefill tokens).
         skinny_rows: decode passes of at most this many rows run every projection on this library's GEMM, the residual updates out of
         place (general_skinny_rows: the same for passes of the plain path); fold_qkv_rows, fold_o_rows,
@@ -147,7 +147,8 @@ class UVEngine:
         choice by size; tests force the tiled forms at a few rows); big_rows: passes of the general path with at least this
         many rows (a packed prefill, a mixed pass) run the down projection too on this library's GEMM, whose 256 x 256 tile
         form is as fast as the vendor library there; fold_down_rows: (first, last) row count of passes whose down projection runs
-        on this library's GEMM.  The defaults are the measured
+        on this library's GEMM; oproj_rows: decode passes of at most this many rows leave the output projection and its residual
+        update to the attention launch (None: as many as it takes, 0: none).  The defaults are the measured
         optimum on UV-50M."""
         self.w, self.cfg = weights, weights.cfg
         cfg, dt, dev = self.cfg, weights.dtype, weights.device
@@ -170,6 +171,11 @@ class UVEngine:
         # Decode passes of at most this many rows keep the block's two hiddens apart (h and x); above it the folded plan updates
         # one in place.
         self.skinny_rows = int(skinny_rows) if dt in (torch.bfloat16, torch.float16) else 0
+        # Of those, passes of at most this many rows have the output projection in the attention launch (one launch of five less a layer:
+        # a step of 1 row 191 -> 173 us, of 8 204 -> 186, of 16 203 -> 188, of 32 214 -> 201, to the same bits).
+        one_kv = cfg.n_heads == 8 and cfg.n_kv_heads == 1 and self.skinny_rows > 0
+        most = L.lib().uvmi_attn_oproj_rows(cfg.d_model) if one_kv else 0
+        self.oproj_rows = most if oproj_rows is None else min(int(oproj_rows), most)
         # passes of the plain path run on this library's GEMM up to this many rows: their alternative is the vendor library with
         # separate SwiGLU and norm launches
         self.general_skinny_rows = int(general_skinny_rows) if dt in (torch.bfloat16, torch.float16) else 0
@@ -420,16 +426,18 @@ class UVEngine:
                     ve_table=self.w.value_embed if has_ve else None, vocab=cfg.vocab_size, rope_table=self.rope_table(st.max_len) if rope else None,
                     n_pairs=cfg.n_pairs, rope=rope, eps=self.eps, xsa_eps=cfg.xsa_eps)
 
-    def fused_cache_attention(self, l: int, tok: Tensor, st: KVState, pos: Tensor, starts: Tensor, n: int, rows: Tensor | None = None):
+    def fused_cache_attention(self, l: int, tok: Tensor, st: KVState, pos: Tensor, starts: Tensor, n: int, rows: Tensor | None = None,
+                              oproj: bool = False):
         """Decode attention of layer l straight from buf qkvx (the extended projection of the n rows): QK-norm, rotation,
-        value embedding, int8 append, attention over lo..pos, XSA and gate in one launch; writes buf zg."""
-        a, keep = self.fused_attention_args(l, self.buf["qkvx"], tok, st, pos, starts, n, rows)
+        value embedding, int8 append, attention over lo..pos, XSA and gate in one launch; writes buf zg.  oproj: also the output
+        projection and the block's first residual update; writes buf h instead."""
+        a, keep = self.fused_attention_args(l, self.buf["qkvx"], tok, st, pos, starts, n, rows, oproj)
         if self._rec is not None and self.cfg.has_ve(l):
             self._rec.field(keep[0][2], "tok", "tok")
         self._op(L.OP_DECODE_ATTN, a, (keep, pos, starts), B="n", pos="pos", starts="starts", **({} if rows is None else {"rows": "rows"}))
 
     def fused_attention_args(self, l: int, qkvx: Tensor, tok: Tensor, st: KVState, pos: Tensor, starts: Tensor, n: int,
-                             rows: Tensor | None = None):
+                             rows: Tensor | None = None, oproj: bool = False):
         """The uvmi_attn_args struct fused_cache_attention launches for layer l, on a given copy of that layer's extended
         projection (qkvx_keep): lets a benchmark re-issue exactly the step's launches through the C ABI.  Re-issuing it
         on the step's own positions rewrites the same K/V bytes."""
@@ -437,8 +445,11 @@ class UVEngine:
         glob = cfg.is_global(l)
         out = b["zg"][:n].view(n, cfg.n_heads, cfg.head_dim)
         k, v, ks, vs = st.cache(l)
+        fuse = self._fuse_dict(l, tok, st)
+        if oproj:
+            fuse["oproj"] = dict(w=W["wo"], resid=b["x"][:n], out=b["h"][:n], ca=W["resid_attn"], cb=W["post_attn"])
         return build_fused_args(qkvx[:n], cfg.n_heads, k, v, pos, starts, cfg.attn_scale, st.window(l), not glob, ks, vs, W["xsa"], out,
-                                self._fuse_dict(l, tok, st), rows, any_ring=st.short_ring(l))
+                                fuse, rows, any_ring=st.short_ring(l))
 
     def cache_attention_args(self, l: int, st: KVState, pos: Tensor, starts: Tensor, n: int, rows: Tensor | None = None):
         """The uvmi_attn_args struct cache_attention would launch for layer l on the engine's buffers (fused path only):
@@ -467,8 +478,8 @@ class UVEngine:
         self.hidden_is_raw = False
         raw = True          # the last block leaves buf x un-normalised
         kind = self._pass_kind(n, fused_attn is not None, st)
-        if kind == "lean":
-            self._layers_lean(n, fused_attn)
+        if kind in ("lean", "lean-o"):
+            self._layers_lean(n, fused_attn, kind == "lean-o")
         elif kind == "folded":
             self._layers_folded(n, fused_attn)
         elif kind == "packed":
@@ -485,7 +496,7 @@ class UVEngine:
         return xn
 
     def _pass_kind(self, n: int, fused: bool, st: KVState | None) -> str:
-        """The launch plan of a pass of n rows: "lean" and "folded" for decode rows whose every layer takes the fused
+        """The launch plan of a pass of n rows: "lean" ("lean-o": with the output projection in the attention launch) and "folded" for decode rows whose every layer takes the fused
         attention, "packed" for prompts, mixed passes and the unfused attention of a 16-bit engine, "plain" for the rest
         (fp32, widths the GEMMs do not take, plans switched off)."""
         cfg = self.cfg
@@ -495,7 +506,7 @@ class UVEngine:
         if fused and ok16 and self._fused_layers_ok(st):
             skinny = n <= self.skinny_rows and div
             if skinny and self.lean and il and cfg.d_ff % 64 == 0:
-                return "lean"
+                return "lean-o" if n <= self.oproj_rows else "lean"
             if self.fold and not skinny and cfg.d_ff % 8 == 0:
                 return "folded"
         if not fused and ok16 and self.fold and self.tiled_prefill and self.fuse_qkv and il and div and cfg.d_ff % 64 == 0:
@@ -519,16 +530,20 @@ class UVEngine:
         else:
             self._gemm(b["x"][:n], W["wqkv_ext"], b["qkvx"][:n], norm_eps=self.eps, **kw)
 
-    def _layers_lean(self, n: int, fused_attn):
+    def _layers_lean(self, n: int, fused_attn, oproj: bool):
         """Decode passes of few rows: every projection on this library's GEMM, the residual updates in the epilogues of the output
-        and down projections, both pre-norms as row scales of the products that read them.  Five launches per layer."""
+        and down projections, both pre-norms as row scales of the products that read them.  Five launches per layer; four where
+        the attention launch does the output projection and its residual update (oproj)."""
         b = self.buf
         x, h, zg, act = b["x"][:n], b["h"][:n], b["zg"][:n], b["act"][:n]
         for l, W in enumerate(self.w.layers):
             self._project_qkv(l, n)
             self._keep_projection(l, n)
-            fused_attn(l)
-            self._gemm(zg, W["wo"], h, RESID, resid=x, ca=W["resid_attn"], cb=W["post_attn"])
+            if oproj:
+                fused_attn(l, oproj=True)
+            else:
+                fused_attn(l)
+                self._gemm(zg, W["wo"], h, RESID, resid=x, ca=W["resid_attn"], cb=W["post_attn"])
             self._gemm(h, W["gu_il"], act, SWIGLU, norm_eps=self.eps)
             self._gemm(act, W["down"], x, RESID, resid=h, ca=W["resid_mlp"], cb=W["post_mlp"])
 
@@ -720,9 +735,9 @@ class UVEngine:
         ns = num_splits or {}
         fused = None
         if self.fuse_qkv and not num_splits and fuse:
-            fused = lambda l: self.fused_cache_attention(l, tok, st, pos, starts, B)
+            fused = lambda l, oproj=False: self.fused_cache_attention(l, tok, st, pos, starts, B, oproj=oproj)
             kind = self._pass_kind(B, True, st)
-            if kind in ("lean", "folded") and self.qkvx_keep is None:
+            if kind in ("lean", "lean-o", "folded") and self.qkvx_keep is None:
                 assert B <= self.max_tokens and B <= st.B
                 # (a recorded list takes addresses only, so what its launches assume of the arrays is checked on every call)
                 assert all(t.dtype == torch.int64 and t.is_contiguous() and t.numel() >= B for t in (tok, pos, starts))

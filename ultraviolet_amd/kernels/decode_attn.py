@@ -128,8 +128,16 @@ def build_attn_args(q, k_cache, v_cache, pos, starts, scale, window, ring, k_sca
             assert tab.dtype == torch.float32 and tab.is_contiguous() and tab.dim() == 2 and tab.size(1) == 2 * f.n_pairs
             f.rope_table, f.rope_positions = tab.data_ptr(), tab.size(0)
         f.eps, f.xsa_eps = float(fuse["eps"]), float(fuse["xsa_eps"])
+        proj = fuse.get("oproj")
+        if proj is not None:
+            # oproj: dict(w (N, H * hd), resid (B, N), out (B, N), ca, cb): the output projection and the residual update, out = ca resid + cb z w^T
+            w, resid, h = proj["w"], proj["resid"], proj["out"]
+            assert w.dim() == 2 and w.size(1) == H * hd and w.stride(1) == 1 and resid.shape == h.shape == (B, w.size(0))
+            assert resid.stride(1) == h.stride(1) == 1 and w.dtype == resid.dtype == h.dtype == q.dtype
+            o = L.AttnOproj(w.data_ptr(), w.stride(0), resid.data_ptr(), resid.stride(0), h.data_ptr(), h.stride(0), w.size(0), proj["ca"], proj["cb"])
+            f.oproj, post = C.addressof(o), (o, w, resid, h)
         a.fuse = C.addressof(f)
-    return a, (ws, rows, f)
+    return a, (ws, rows, f, post)
 
 
 def _launch(q, k_cache, v_cache, pos, starts, scale, window, ring, k_scale, v_scale, num_splits, out, chunk_keys=0, rows=None,
