@@ -5,7 +5,7 @@
 // i - window < j <= i.
 //
 // prefill_attn_mfma_hd64 (head_dim 64, 16-bit q/k/v of one dtype, up to 8 query heads per kv head):
-//   * a wave owns 16 consecutive packed tokens x 4 query heads of one kv head, and walks the keys in 32-key
+//   * a wave owns 16 consecutive packed tokens x 2 query heads of one kv head, and walks the keys in 32-key
 //     super-tiles.  Query blocks are aligned to the packed index, not to the sequences: a block that straddles a
 //     boundary walks the union of its rows' key ranges and masks per (row, key), so the grid is ceil(N / 16) blocks
 //     with no search for "which sequence is block i in";
@@ -13,18 +13,21 @@
 //     holds 4 consecutive keys of one query row, for two 16-key tiles A and B.  Exactly these 8 values, rounded to
 //     the 16-bit input type, are the lane's slice of the B operand of O^T = V^T . P^T when contraction slot 8g+j is
 //     key 4g+j of tile A (j < 4) or of tile B (j >= 4): probabilities never move between lanes;
-//   * V^T operands come from 8-byte loads (lane = dims 4m..4m+3 of 8 keys) regrouped with v_perm_b32 into four
-//     operands whose row m is head dim 4m + t; they are built once per super-tile and shared by the wave's 4 heads,
-//     as are the K operands (16-byte reads, lane = key m, dims 8g..8g+7 of each half);
-//   * the 4 waves of a workgroup are 2 consecutive query blocks x 2 head groups (4 blocks x 1 group for up to 4 query
-//     heads per kv head) of one kv head and walk the same keys, so a super-tile of K and V is fetched once per workgroup:
-//     each thread requests 16 bytes of K and of V two tiles ahead into registers, parks them in one of two LDS halves
-//     (K rows chunk-swizzled, so the 16-byte operand reads are conflict-free) and the waves take their operands from
-//     there, one barrier per tile; a wave skips the tiles outside its own block's key range;
+//   * V^T operands come out of LDS through the transposing read (ds_read_b64_tr_b16), once per super-tile for the wave's heads, as
+//     do the K operands (16-byte reads, lane = key m, dims 8g..8g+7 of each half);
+//   * the 4 waves of a workgroup are the 4 head pairs of a query block (2 blocks x 2 pairs for up to 4 query heads per kv head, 4
+//     blocks for up to 2) of one kv head and walk the same keys, so a super-tile of K and V is fetched once per workgroup, from
+//     global memory straight into one of three LDS stages, two tiles ahead; one barrier per tile; a wave skips the tiles outside
+//     its own block's key range;
 //   * online softmax per (row, head) in the exp2 domain; tiles that every row of the block sees completely skip the
-//     mask arithmetic (one branch per tile, so the four heads of a tile form one block the scheduler interleaves);
+//     mask arithmetic (one branch per tile, so the heads of a tile form one block the scheduler interleaves);
 //   * workgroup ids are remapped so that each XCD (one L2 each) owns a contiguous range of query blocks and therefore
-//     whole sequences.
+//     whole sequences, the last blocks first: they see the most keys.
+// What bounds it: vector instructions (79 % of the cycles that a compute unit is busy; the matrix cores 18 %), ~155 a tile and head
+// pair of which 36 are exponentials, at three waves per SIMD.  With four heads per wave it held 255 registers, two waves per SIMD, staged
+// K and V through registers, and made eight trips to memory one after the other for its epilogue.  us, before -> now, with the
+// epilogue: 93 tokens 9.4 -> 5.8; 400 16.6 -> 9.6; 64 x 64 .. 512 tokens 41.2 -> 33.1, window 256 34.2 -> 27.4; 64 x 512 62.2 -> 47.7 and
+// 46.3 -> 39.0; 4 x 2048 without 77.6 -> 48.4; 61 x 16 .. 1024, window 256, 42.1 -> 38.3.
 //
 // Everything else (fp32 K/V, other head dims) goes token by token through the decode kernel's generic path with the
 // packed K/V as a batch-stride-0 "cache".
@@ -40,7 +43,7 @@ struct PrefillParams {
   const void* q; const void* k; const void* v; void* out;
   const int32_t* seg_start;  // (N,) packed index of the first token of each token's sequence
   int64_t sqn, sqh, skn, skh, svn, svh, son, soh;
-  int N, H, KH, G, window, n_hg;   // n_hg: head groups of 4 query heads per kv head, 1 or 2
+  int N, H, KH, G, window, n_hg;   // n_hg: waves that share a query block of a kv head, HPW query heads each: 1, 2 or 4
   int n_wg;                        // workgroups with work: ceil(query blocks / (4 / n_hg)) * KH
   float scale_log2;
   const float* post_vhat; const float* post_gate; const float* post_xsa;  // fused Attention.post epilogue when post_vhat != null
@@ -60,69 +63,105 @@ __global__ __launch_bounds__(256) void prefill_segments(const void* cu, int idx6
   pidx[i] = i;
 }
 
-struct PTile {   // one 32-key super-tile as loaded (32 dwords per lane)
-  pu4 k[4];      // [tile A dims 0..31, tile A dims 32..63, tile B dims 0..31, tile B dims 32..63]: key m, dims 8g..8g+7
-  pu2 v[8];      // keys 4g+j of tile A (j < 4) / tile B (j >= 4), dims 4m..4m+3
-};
+constexpr int HPW = 2;  // query heads per wave
 
-constexpr int HPW = 4;  // query heads per wave
-
-constexpr int RING = 2;  // super-tiles requested ahead of the one being parked in LDS
+// Transposing LDS read (ds_read_b64_tr_b16): of 16 lanes, lane 4 t + q names 4 consecutive 16-bit elements of row t from column 4 q on;
+// lane i gets column i of rows 0 .. 3.
+__device__ __forceinline__ pu2 ld_tr16(const unsigned char* p) {
+  typedef short s4 __attribute__((ext_vector_type(4)));
+  const s4 r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4*)p);
+  pu2 v;
+  __builtin_memcpy(&v, &r, 8);
+  return v;
+}
+// maximum over lanes l, l ^ 16, l ^ 32, l ^ 48
+__device__ __forceinline__ float xmaximum(float v) {
+  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __builtin_elementwise_maximum(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __builtin_elementwise_maximum(__uint_as_float(q[0]), __uint_as_float(q[1]));
+}
+__device__ __forceinline__ float max3(float a, float b, float c) { return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c); }
 
 template <int DT, int ODT>
-__global__ __launch_bounds__(256) void prefill_attn_mfma_hd64(PrefillParams P) {
-  __shared__ __attribute__((aligned(16))) unsigned char smem[2][2][4096];  // [half][K, V][32 keys x 128 B]
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void prefill_attn_mfma_hd64(PrefillParams P) {
+  // one object per stage: the compiler can then tell that reads of one do not touch the one a load is filling
+  __shared__ __attribute__((aligned(1024))) unsigned char s0[2][4096], s1[2][4096], s2[2][4096];  // [K, V][32 keys x 128 B]
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // gridDim.x is a multiple of 8; ids congruent mod 8 run on one XCD and get a contiguous range of work
   const int per = gridDim.x >> 3;
-  const int bid = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  // from its end: a sequence's last blocks, which see the most keys, start first
+  const int bid = (blockIdx.x & 7) * per + per - 1 - (blockIdx.x >> 3);
   if (bid >= P.n_wg) return;   // (the whole workgroup: no barrier is left waiting)
   const int kvh = bid % P.KH;
   const int qg = bid / P.KH;               // group of 4 / n_hg consecutive query blocks
-  const int hsh = P.n_hg - 1;              // n_hg is 1 or 2
+  const int hsh = P.n_hg >> 1;             // n_hg is 1, 2 or 4
   const int qbw = 4 >> hsh;
-  const int hg = wave & hsh;
+  const int hg = wave & (P.n_hg - 1);
   const int qb = qg * qbw + (wave >> hsh);
   const int m = lane & 15, g = lane >> 4;
   const int G = P.G;
   const float c = P.scale_log2;
 
-  // ---- this lane's query row (accumulator column m) and its key range; a wave whose block starts past the last token
-  // (the tail of the last group) has an empty range and only helps with the loads
+  // ---- this lane's query row (accumulator column m); a wave whose block starts past the last token (the tail of the last
+  // group) has an empty key range and only helps with the loads
   const int r0 = qb * 16;
   const bool wave_ok = r0 < P.N;
   const int row = r0 + m;
   const bool row_ok = row < P.N;
   const int rowc = row_ok ? row : P.N - 1;
+  const int row0 = qg * qbw * 16;          // < N
+  // ---- what depends on the row alone goes out first: Q^T operands (lane (row m, group g) holds q[row][head][32 s + 8 g .. + 8] for
+  // s = 0, 1; absent heads read the last one and are not stored), the row's segment, the epilogue's gates
+  pu4 Q[HPW][2];
+  float gate[HPW], xsa[HPW];
+  const bool has_post = P.post_vhat != nullptr;
+#pragma unroll
+  for (int hh = 0; hh < HPW; hh++) {
+    const int head = kvh * G + min(hg * HPW + hh, G - 1);
+    const uint16_t* qp = (const uint16_t*)P.q + (int64_t)rowc * P.sqn + (int64_t)head * P.sqh + 8 * g;
+    Q[hh][0] = *(const pu4*)qp;
+    Q[hh][1] = *(const pu4*)(qp + 32);
+    gate[hh] = 1.0f;
+    xsa[hh] = 0.f;
+    if (has_post && P.post_gate) gate[hh] = P.post_gate[(int64_t)rowc * P.H + head];
+    if (has_post && P.post_xsa) xsa[hh] = P.post_xsa[head];
+  }
   int lo_n = P.seg_start[rowc];
+  int lo0 = P.seg_start[row0];
+  __builtin_amdgcn_sched_barrier(0);
+  // ---- key ranges: the row's, the block's, and the workgroup's from its first row's lower bound (the smallest) to its last row
   if (P.window > 0 && row - P.window + 1 > lo_n) lo_n = row - P.window + 1;
   if (!row_ok) lo_n = INT_MAX;
+  if (P.window > 0 && row0 - P.window + 1 > lo0) lo0 = row0 - P.window + 1;
   const int rl = min(r0 + 15, P.N - 1);                                       // last real row of the block
   const int lo_first = __builtin_amdgcn_readfirstlane(lo_n);                  // lo is non-decreasing in the row
   const int lo_last = __builtin_amdgcn_readfirstlane(__shfl(lo_n, wave_ok ? rl - r0 : 0, 64));
   const int kbeg = wave_ok ? lo_first & ~31 : 0, kend = wave_ok ? rl + 1 : 0;
-  // ---- the workgroup's key range: from the first row's lower bound (the smallest of the group) to its last row
-  const int row0 = qg * qbw * 16;          // < N
-  int lo0 = P.seg_start[row0];
-  if (P.window > 0 && row0 - P.window + 1 > lo0) lo0 = row0 - P.window + 1;
   const int kbeg_wg = __builtin_amdgcn_readfirstlane(lo0) & ~31;
   const int kend_wg = min(row0 + qbw * 16, P.N);
   const int nk = (kend_wg - kbeg_wg + 31) >> 5;   // >= 1
 
-  // ---- Q^T operands: lane (row m, group g) holds q[row][head][32 s + 8 g .. + 8] for s = 0, 1
-  pu4 Q[HPW][2];
-#pragma unroll
-  for (int hh = 0; hh < HPW; hh++) {
-    const int hq = hg * HPW + hh;
-    Q[hh][0] = Q[hh][1] = pu4{0u, 0u, 0u, 0u};
-    if (hq < G) {
-      const uint16_t* qp = (const uint16_t*)P.q + (int64_t)rowc * P.sqn + (int64_t)(kvh * G + hq) * P.sqh + 8 * g;
-      Q[hh][0] = *(const pu4*)qp;
-      Q[hh][1] = *(const pu4*)(qp + 32);
-    }
-  }
+  // ---- K / V super-tiles go from global memory straight into one of three LDS stages, two tiles ahead: wave w moves keys 8 w .. 8 w + 7
+  // of K and of V, 16 bytes per lane.  Keys are clamped to N - 1 (a clamped key is masked).  K rows keep their 16-byte chunks
+  // xor-ed with (key / 2) % 8, V rows theirs with 2 (key % 4), which makes the operand reads (lane = key m, chunk 4 s + g; four keys'
+  // 32 bytes per 16 lanes) free of bank conflicts.
+  const uint16_t* kbase = (const uint16_t*)P.k + (int64_t)kvh * P.skh;
+  const uint16_t* vbase = (const uint16_t*)P.v + (int64_t)kvh * P.svh;
+  const uint32_t skn2 = (uint32_t)P.skn * 2, svn2 = (uint32_t)P.svn * 2;  // row strides in bytes
+  const __amdgpu_buffer_rsrc_t rK = __builtin_amdgcn_make_buffer_rsrc((void*)kbase, 0, (int)((uint32_t)(P.N - 1) * skn2 + 128), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rV = __builtin_amdgcn_make_buffer_rsrc((void*)vbase, 0, (int)((uint32_t)(P.N - 1) * svn2 + 128), 0x00020000);
+  const int lkey = 8 * wave + (lane >> 3), lch = lane & 7;
+  const uint32_t kch = (uint32_t)((lch ^ ((lkey >> 1) & 7)) << 4), vch = (uint32_t)((lch ^ ((lkey & 3) << 1)) << 4);
+  auto issue = [&](unsigned char (*S)[4096], int k) {
+    const uint32_t r = (uint32_t)min(kbeg_wg + 32 * k + lkey, P.N - 1);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rK, (__attribute__((address_space(3))) void*)(S[0] + 1024 * wave), 16, r * skn2 + kch, 0, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rV, (__attribute__((address_space(3))) void*)(S[1] + 1024 * wave), 16, r * svn2 + vch, 0, 0, 0);
+  };
+  issue(s0, 0);
+  if (nk > 1) issue(s1, 1);
 
   pf4 O[HPW][4];
   float mrun[HPW], lrun[HPW];
@@ -133,70 +172,33 @@ __global__ __launch_bounds__(256) void prefill_attn_mfma_hd64(PrefillParams P) {
     mrun[hh] = -INFINITY;
     lrun[hh] = 0.f;
   }
-
-  // ---- addressing: one descriptor per stream, per-lane byte offsets
-  const uint16_t* kbase = (const uint16_t*)P.k + (int64_t)kvh * P.skh;
-  const uint16_t* vbase = (const uint16_t*)P.v + (int64_t)kvh * P.svh;
-  const uint32_t skn2 = (uint32_t)P.skn * 2, svn2 = (uint32_t)P.svn * 2;  // row strides in bytes
-  const __amdgpu_buffer_rsrc_t rK = __builtin_amdgcn_make_buffer_rsrc((void*)kbase, 0, (int)((uint32_t)(P.N - 1) * skn2 + 128), 0x00020000);
-  const __amdgpu_buffer_rsrc_t rV = __builtin_amdgcn_make_buffer_rsrc((void*)vbase, 0, (int)((uint32_t)(P.N - 1) * svn2 + 128), 0x00020000);
-
-  // ---- K / V super-tiles go global -> registers (RING tiles ahead) -> LDS (two halves) -> MFMA operands.  Thread t moves
-  // 16 bytes of K and of V per tile: key t / 8, chunk t % 8 of the 128-byte row.  Rows are clamped to N - 1 (the keys of a
-  // clamped row are masked); tiles past the group's last are re-reads of the last one.  K rows are stored with their
-  // 16-byte chunks XOR-swizzled by (key / 2) % 8, which makes both the stores and the operand reads (lane = key m, chunk
-  // 4 s + g) free of bank conflicts; V rows are stored as they are (an operand read takes whole 128-byte rows).
-  pu4 rk[RING], rv[RING];
-  const int lkey = tid >> 3, lch = tid & 7;
-  const uint32_t kst = (uint32_t)lkey * 128 + (uint32_t)((lch ^ ((lkey >> 1) & 7)) << 4), vst = (uint32_t)lkey * 128 + (uint32_t)lch * 16;
-  auto fetch = [&](int k, int slot) {
-    const int tb = kbeg_wg + 32 * min(k, nk - 1);
-    const uint32_t r = (uint32_t)min(tb + lkey, P.N - 1);
-    rk[slot] = __builtin_amdgcn_raw_buffer_load_b128(rK, r * skn2 + 16 * lch, 0, 0);
-    rv[slot] = __builtin_amdgcn_raw_buffer_load_b128(rV, r * svn2 + 16 * lch, 0, 0);
-  };
-  auto park = [&](int slot, int half) {
-    *(pu4*)(&smem[half][0][kst]) = rk[slot];
-    *(pu4*)(&smem[half][1][vst]) = rv[slot];
-  };
   const uint32_t kld0 = (uint32_t)m * 128 + (uint32_t)((g ^ ((m >> 1) & 7)) << 4), kld1 = (uint32_t)m * 128 + (uint32_t)(((4 + g) ^ ((m >> 1) & 7)) << 4);
-  const uint32_t vld = (uint32_t)(4 * g) * 128 + 8 * m;
-  auto read_tile = [&](int half, PTile& T) {
-    const unsigned char* sk = smem[half][0];
-    const unsigned char* sv = smem[half][1];
-    T.k[0] = *(const pu4*)(sk + kld0);
-    T.k[1] = *(const pu4*)(sk + kld1);
-    T.k[2] = *(const pu4*)(sk + 2048 + kld0);
-    T.k[3] = *(const pu4*)(sk + 2048 + kld1);
+  // V^T operand t: lane m of group g names key 4 g + m / 4, dims 16 t + 4 (m % 4) ..; the transposing read hands it dim 16 t + m of keys
+  // 4 g .. 4 g + 3
+  uint32_t vld[4];
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      T.v[j] = *(const pu2*)(sv + vld + 128 * j);
-      T.v[4 + j] = *(const pu2*)(sv + 2048 + vld + 128 * j);
-    }
-  };
+  for (int t = 0; t < 4; t++) vld[t] = (uint32_t)(4 * g + (m >> 2)) * 128 + (uint32_t)(((2 * t + ((m & 3) >> 1)) ^ ((m >> 2) << 1)) << 4) + 8 * (m & 1);
 
-  auto step_t = [&](const PTile& T, int tb, auto EDGE) {
+  auto step_t = [&](const unsigned char (*S)[4096], int tb, auto EDGE) {
     constexpr bool edge = decltype(EDGE)::value;
-    // V^T operands: operand t, row m is head dim 4m + t; dword p of an operand holds contraction slots 2p, 2p+1
-    pu4 VA[4];
-    {
-      constexpr uint32_t LO = 0x05040100u, HI = 0x07060302u;
-#pragma unroll
-      for (int p = 0; p < 4; p++) {
-        VA[0][p] = __builtin_amdgcn_perm(T.v[2 * p + 1].x, T.v[2 * p].x, LO);
-        VA[1][p] = __builtin_amdgcn_perm(T.v[2 * p + 1].x, T.v[2 * p].x, HI);
-        VA[2][p] = __builtin_amdgcn_perm(T.v[2 * p + 1].y, T.v[2 * p].y, LO);
-        VA[3][p] = __builtin_amdgcn_perm(T.v[2 * p + 1].y, T.v[2 * p].y, HI);
-      }
-    }
+    pu4 K[4];      // [tile A dims 0..31, tile A dims 32..63, tile B dims 0..31, tile B dims 32..63]: key m, dims 8g..8g+7
+    K[0] = *(const pu4*)(S[0] + kld0);
+    K[1] = *(const pu4*)(S[0] + kld1);
+    K[2] = *(const pu4*)(S[0] + 2048 + kld0);
+    K[3] = *(const pu4*)(S[0] + 2048 + kld1);
     const int kA = tb + 4 * g, kB = kA + 16;  // first of this lane's 4 keys in tile A / B
+    pu4 VA[4];     // V^T operands: row m is head dim 16 t + m; slots 0..3 are keys 4g+j of tile A, 4..7 of tile B
+#pragma unroll
+    for (int tt = 0; tt < 4; tt++) {
+      const pu2 a = ld_tr16(S[1] + vld[tt]), b = ld_tr16(S[1] + 2048 + vld[tt]);
+      VA[tt] = pu4{a.x, a.y, b.x, b.y};
+    }
 #pragma unroll
     for (int hh = 0; hh < HPW; hh++) {
-      pf4 sA = pf4{0.f, 0.f, 0.f, 0.f}, sB = pf4{0.f, 0.f, 0.f, 0.f};
-      sA = mfma16<DT>(T.k[0], Q[hh][0], sA);
-      sB = mfma16<DT>(T.k[2], Q[hh][0], sB);
-      sA = mfma16<DT>(T.k[1], Q[hh][1], sA);
-      sB = mfma16<DT>(T.k[3], Q[hh][1], sB);
+      pf4 sA = mfma16<DT>(K[0], Q[hh][0], pf4{0.f, 0.f, 0.f, 0.f});
+      pf4 sB = mfma16<DT>(K[2], Q[hh][0], pf4{0.f, 0.f, 0.f, 0.f});
+      sA = mfma16<DT>(K[1], Q[hh][1], sA);
+      sB = mfma16<DT>(K[3], Q[hh][1], sB);
       float t[8] = {sA[0], sA[1], sA[2], sA[3], sB[0], sB[1], sB[2], sB[3]};
       if (edge) {
 #pragma unroll
@@ -205,12 +207,14 @@ __global__ __launch_bounds__(256) void prefill_attn_mfma_hd64(PrefillParams P) {
           if (kB + i < lo_n || kB + i > row) t[4 + i] = -INFINITY;
         }
       }
-      float mx = fmaxf(fmaxf(fmaxf(t[0], t[1]), fmaxf(t[2], t[3])), fmaxf(fmaxf(t[4], t[5]), fmaxf(t[6], t[7])));
-      mx = pmax32(pmax16(mx));
+      // (the maximum that hands NaN on: one instruction for three values, where the one that ignores it needs each made quiet first; a
+      // score that is NaN makes its row NaN either way)
+      const float mx = max3(max3(max3(t[0], t[1], t[2]), t[3], t[4]), max3(t[5], t[6], t[7]), mrun[hh]);
       {  // rescale by alpha = exp2((m_old - m_new) c), 1 where the row's maximum did not grow.  Unconditional: a branch
-         // here would split the four heads into separate blocks and stop the scheduler from overlapping one head's
-         // softmax arithmetic with the next head's MFMAs
-        const float mnew = fmaxf(mrun[hh], mx);
+         // here would split the heads into separate blocks and stop the scheduler from overlapping one head's
+         // softmax arithmetic with the next head's MFMAs.  (A reference point that may lag behind the maximum, as the decode
+         // kernel's, costs precision here: the largest probability is then no longer 1, which is exact in 16 bits.)
+        const float mnew = xmaximum(mx);
         const float alpha = mnew == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f((mrun[hh] - mnew) * c);
 #pragma unroll
         for (int tt = 0; tt < 4; tt++) O[hh][tt] *= alpha;
@@ -227,55 +231,40 @@ __global__ __launch_bounds__(256) void prefill_attn_mfma_hd64(PrefillParams P) {
       for (int tt = 0; tt < 4; tt++) O[hh][tt] = mfma16<DT>(VA[tt], PB, O[hh][tt]);
     }
   };
-
-  // the mask test is hoisted out of the head loop (one branch per tile, two straight-line bodies), so that the four
-  // heads of a tile form one block the scheduler can interleave
-  auto step = [&](const PTile& T, int tb, bool edge) {
-    if (edge) step_t(T, tb, std::true_type{}); else step_t(T, tb, std::false_type{});
+  // a tile needs no mask when every row of the block sees all of it: it starts at or after the last row's lower bound and ends at or
+  // before the first row (the test is hoisted out of the head loop, so that the heads of a tile form one block the scheduler can
+  // interleave); a wave skips the tiles outside its own block's range
+  auto step = [&](const unsigned char (*S)[4096], int k) {
+    const int tb = kbeg_wg + 32 * k;
+    if (tb < kbeg || tb >= kend) return;   // (wave-uniform)
+    if (tb >= lo_last && tb + 31 <= r0) step_t(S, tb, std::false_type{}); else step_t(S, tb, std::true_type{});
   };
-
-  {
-    // a tile needs no mask when every row of the block sees all of it: it starts at or after the last row's lower
-    // bound and ends at or before the first row
-    auto edge_of = [&](int tb) { return !(tb >= lo_last && tb + 31 <= r0); };
-    // iteration k: this wave's operands of tile k come out of LDS half k % 2 (when the tile lies in the wave's own range),
-    // tile k + 1 is parked in the other half, tile k + 1 + RING is requested into the ring slot that frees, then the
-    // arithmetic of tile k runs; the barrier lets the next iteration overwrite the half just read
-    auto iteration = [&](int k, int d) {
-      const int tb = kbeg_wg + 32 * k;
-      const bool act = tb >= kbeg && tb < kend;   // wave-uniform
-      PTile T;
-      if (act) read_tile(k & 1, T);
-      park((d + 1) % RING, (k + 1) & 1);
-      fetch(k + 1 + RING, (d + 1) % RING);
-      if (act) step(T, tb, edge_of(tb));
-      __syncthreads();
-    };
-#pragma unroll
-    for (int d = 0; d < RING; d++) fetch(d, d);
-    park(0, 0);
-    fetch(RING, 0);
-    __syncthreads();
-    int k = 0;
-    for (; k + RING <= nk; k += RING) {
-#pragma unroll
-      for (int d = 0; d < RING; d++) iteration(k + d, d);
-    }
-#pragma unroll
-    for (int d = 0; d < RING - 1; d++)
-      if (k + d < nk) iteration(k + d, d);   // workgroup-uniform
+  // iteration k: tile k has landed (own loads: the wait, which leaves tile k + 1's in flight; the other waves': the barrier) and every
+  // wave is done with tile k - 1, whose stage takes tile k + 2
+  auto iteration = [&](unsigned char (*S)[4096], unsigned char (*SN)[4096], int k) {
+    if (k + 1 < nk) __builtin_amdgcn_s_waitcnt(0x0f72); else __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(2) / (0)
+    asm volatile("s_barrier" ::: "memory");
+    if (k + 2 < nk) issue(SN, k + 2);
+    step(S, k);
+  };
+  int k = 0;
+  for (; k + 3 <= nk; k += 3) {
+    iteration(s0, s2, k);
+    iteration(s1, s0, k + 1);
+    iteration(s2, s1, k + 2);
   }
+  if (k < nk) iteration(s0, s2, k);
+  if (k + 1 < nk) iteration(s1, s0, k + 1);
 
-  // ---- normalise and store: lane (row m, group g) holds head dims 16g .. 16g+15 (O[t][i] is dim 16g + 4i + t)
+  // ---- normalise and store: lane (row m, group g) holds head dims 16 t + 4 g + i, t, i = 0 .. 3
   // Optional epilogue, as in the decode kernel: z (rounded to the activation type, as the attention output tensor would be)
   // -> XSA with the token's normalised v -> per-head gate; the 4 lane groups of a row reduce z . v_hat between them.
-  const bool has_post = P.post_vhat != nullptr;
   float vv[16];
   if (has_post) {
-    const float* vp = P.post_vhat + ((int64_t)rowc * P.KH + kvh) * 64 + 16 * g;
+    const float* vp = P.post_vhat + ((int64_t)rowc * P.KH + kvh) * 64 + 4 * g;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      const float4 x = *(const float4*)(vp + 4 * i);
+      const float4 x = *(const float4*)(vp + 16 * i);
       vv[4 * i] = x.x; vv[4 * i + 1] = x.y; vv[4 * i + 2] = x.z; vv[4 * i + 3] = x.w;
     }
   }
@@ -292,9 +281,8 @@ __global__ __launch_bounds__(256) void prefill_attn_mfma_hd64(PrefillParams P) {
 #pragma unroll
     for (int t = 0; t < 4; t++)
 #pragma unroll
-      for (int i = 0; i < 4; i++) o[4 * i + t] = O[hh][t][i] * inv;
+      for (int i = 0; i < 4; i++) o[4 * t + i] = O[hh][t][i] * inv;
     if (has_post) {  // (every lane takes part in the reduction; lanes of absent heads / rows compute on clamped operands)
-      const int head = kvh * G + (hq < G ? hq : G - 1);
       float proj = 0.f;
 #pragma unroll
       for (int i = 0; i < 16; i++) {
@@ -303,27 +291,26 @@ __global__ __launch_bounds__(256) void prefill_attn_mfma_hd64(PrefillParams P) {
       }
       if (P.post_xsa) {
         proj = psum32(psum16(proj));
-        const float ah = P.post_xsa[head] * proj;
+        const float ah = xsa[hh] * proj;
 #pragma unroll
         for (int i = 0; i < 16; i++) o[i] = rnd(o[i] - ah * vv[i]);
       }
-      const float gate = P.post_gate ? P.post_gate[(int64_t)rowc * P.H + head] : 1.0f;
 #pragma unroll
-      for (int i = 0; i < 16; i++) o[i] *= gate;
+      for (int i = 0; i < 16; i++) o[i] *= gate[hh];
     }
     if (hq >= G || !row_ok) continue;
-    const int64_t off = (int64_t)row * P.son + (int64_t)(kvh * G + hq) * P.soh + 16 * g;
+    const int64_t off = (int64_t)row * P.son + (int64_t)(kvh * G + hq) * P.soh + 4 * g;
     if (ODT == UVMI_F32) {
       float* op = (float*)P.out + off;
 #pragma unroll
-      for (int i = 0; i < 4; i++) *(float4*)(op + 4 * i) = float4{o[4 * i], o[4 * i + 1], o[4 * i + 2], o[4 * i + 3]};
+      for (int i = 0; i < 4; i++) *(float4*)(op + 16 * i) = float4{o[4 * i], o[4 * i + 1], o[4 * i + 2], o[4 * i + 3]};
     } else {
       uint32_t w[8];
 #pragma unroll
       for (int i = 0; i < 8; i++) w[i] = ODT == UVMI_BF16 ? pack2<UVMI_BF16>(o[2 * i], o[2 * i + 1]) : pack2<UVMI_F16>(o[2 * i], o[2 * i + 1]);
       uint16_t* op = (uint16_t*)P.out + off;
-      *(uint4*)op = uint4{w[0], w[1], w[2], w[3]};
-      *(uint4*)(op + 8) = uint4{w[4], w[5], w[6], w[7]};
+#pragma unroll
+      for (int i = 0; i < 4; i++) *(uint2*)(op + 16 * i) = uint2{w[2 * i], w[2 * i + 1]};
     }
   }
 }
@@ -381,7 +368,7 @@ static int launch_mfma(const uvmi_prefill_attn_args* a, const int32_t* seg_start
   P.q = a->q; P.k = a->k; P.v = a->v; P.out = a->out; P.seg_start = seg_start;
   P.sqn = a->sqn; P.sqh = a->sqh; P.skn = a->skn; P.skh = a->skh; P.svn = a->svn; P.svh = a->svh; P.son = a->son; P.soh = a->soh;
   P.N = a->N; P.H = a->H; P.KH = a->KH; P.G = a->H / a->KH; P.window = a->window;
-  P.n_hg = (P.G + HPW - 1) / HPW;   // 1 or 2 (G <= 8)
+  P.n_hg = P.G <= HPW ? 1 : (P.G <= 2 * HPW ? 2 : 4);   // (G <= 8)
   const int64_t n_qb = (a->N + 15) / 16, qbw = 4 / P.n_hg;
   const int64_t n_wg = (n_qb + qbw - 1) / qbw * a->KH;
   P.scale_log2 = a->scale * 1.4426950408889634f;
