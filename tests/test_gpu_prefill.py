@@ -259,6 +259,24 @@ def test_backward_odd_head_groups_at_block_edges(H, K, n):
             assert np.abs(a - b).max() <= 2 * 2.0 ** -7 * np.abs(b).max() + 1e-6, (lens, np.abs(a - b).max(), np.abs(b).max())
 
 
+@pytest.mark.parametrize("window", [2, 31, 32, 33, 64, 65, 96, 97, 330, 331, 332, 2 ** 31 - 1])
+def test_attention_and_backward_at_the_mask_rules(window):
+    """Windows around the places where a 32-key tile stops needing a mask, or a wave of 32 keys stops seeing a 32-query tile: both
+    depend on the window modulo the tile and on the sequence's start and end inside one; and windows that hide one key and none.
+    Tolerance: one rounding of the largest value for the forward, two for the gradients (as above)."""
+    from oracle.varlen_attn import varlen_attention_ref
+    from ultraviolet_amd.kernels import varlen_attention
+    lens, ulp = [331, 37, 130], 2.0 ** -10
+    q, k, v, cu = _case(lens, 8, 1, 64, torch.float16, seed=5)
+    o = varlen_attention(q[None].to(DEV), k[None].to(DEV), v[None].to(DEV), cu.to(DEV), max(lens), SC, window)
+    ref = varlen_attention_ref(to_np(q), to_np(k), to_np(v), to_np(cu), SC, window)
+    assert np.abs(to_np(o[0]).astype(np.float64) - ref).max() <= ulp * np.abs(ref).max()
+    got, ref = _grad_case(lens, 8, 1, torch.float16, window, seed=5)
+    for a, b in zip(got, ref):
+        assert np.isfinite(a).all()
+        assert np.abs(a - b).max() <= 2 * ulp * np.abs(b).max() + 1e-6, (np.abs(a - b).max(), np.abs(b).max())
+
+
 def test_backward_rejects_what_it_cannot_do():
     from ultraviolet_amd import _lib as L
     from ultraviolet_amd.kernels.varlen_attn import packed_attention_backward

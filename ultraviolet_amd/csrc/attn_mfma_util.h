@@ -57,9 +57,15 @@ __device__ __forceinline__ float psum32(float v) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// K / V (or Q / dO) tiles parked in LDS as 32 rows of 128 bytes: the 16-byte chunk c of row r sits at chunk c ^ ((r / 2) % 8),
-// which keeps 16-byte stores (8 threads per row) and the operand reads below free of bank conflicts.
-__device__ __forceinline__ uint32_t lds_chunk_off(int row, int chunk) { return (uint32_t)row * 128 + (uint32_t)((chunk ^ ((row >> 1) & 7)) << 4); }
+// Transposing LDS read (ds_read_b64_tr_b16): of 16 lanes, lane 4 t + q names 4 consecutive 16-bit elements of row t from column 4 q on;
+// lane i gets column i of rows 0 .. 3.
+__device__ __forceinline__ pu2 ld_tr16(const unsigned char* p) {
+  typedef short s4 __attribute__((ext_vector_type(4)));
+  const s4 r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4*)p);
+  pu2 v;
+  __builtin_memcpy(&v, &r, 8);
+  return v;
+}
 
 // prefill_attn.hip: the segment table of a->cu_seqlens into seg_start (N ints; pidx: N ints of scratch) and the rows' softmax
 // statistics - log2 of sum_j exp2(scale log2(e) q_i . k_j) - into lse (H, lse_stride) from a forward pass that stores no output.

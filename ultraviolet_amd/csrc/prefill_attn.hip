@@ -20,14 +20,15 @@
 //     global memory straight into one of three LDS stages, two tiles ahead; one barrier per tile; a wave skips the tiles outside
 //     its own block's key range;
 //   * online softmax per (row, head) in the exp2 domain; tiles that every row of the block sees completely skip the
-//     mask arithmetic (one branch per tile, so the heads of a tile form one block the scheduler interleaves);
+//     mask arithmetic: one branch per tile, around the mask alone (as two versions of the whole tile, the accumulators of the two met
+//     in copies, 40 registers a tile, and it took 153 registers instead of 118, three waves per SIMD instead of four);
 //   * workgroup ids are remapped so that each XCD (one L2 each) owns a contiguous range of query blocks and therefore
 //     whole sequences, the last blocks first: they see the most keys.
-// What bounds it: vector instructions (79 % of the cycles that a compute unit is busy; the matrix cores 18 %), ~155 a tile and head
-// pair of which 36 are exponentials, at three waves per SIMD.  With four heads per wave it held 255 registers, two waves per SIMD, staged
+// What bounds it: vector instructions (79 % of the cycles that a compute unit is busy; the matrix cores 18 %), ~135 a tile and head
+// pair of which 36 are exponentials, at four waves per SIMD.  With four heads per wave it held 255 registers, two waves per SIMD, staged
 // K and V through registers, and made eight trips to memory one after the other for its epilogue.  us, before -> now, with the
-// epilogue: 93 tokens 9.4 -> 5.8; 400 16.6 -> 9.6; 64 x 64 .. 512 tokens 41.2 -> 33.1, window 256 34.2 -> 27.4; 64 x 512 62.2 -> 47.7 and
-// 46.3 -> 39.0; 4 x 2048 without 77.6 -> 48.4; 61 x 16 .. 1024, window 256, 42.1 -> 38.3.
+// epilogue: 93 tokens 9.4 -> 5.3; 400 16.6 -> 8.6; 64 x 64 .. 512 tokens 41.2 -> 30.8, window 256 34.2 -> 25.2; 64 x 512 62.2 -> 43.4 and
+// 46.3 -> 34.8; 4 x 2048 without 77.6 -> 43.5; 61 x 16 .. 1024, window 256, 42.1 -> 34.6.
 //
 // Everything else (fp32 K/V, other head dims) goes token by token through the decode kernel's generic path with the
 // packed K/V as a batch-stride-0 "cache".
@@ -35,7 +36,6 @@
 #include "attn_mfma_util.h"
 
 #include <climits>
-#include <type_traits>
 
 namespace uvmi {
 
@@ -65,15 +65,6 @@ __global__ __launch_bounds__(256) void prefill_segments(const void* cu, int idx6
 
 constexpr int HPW = 2;  // query heads per wave
 
-// Transposing LDS read (ds_read_b64_tr_b16): of 16 lanes, lane 4 t + q names 4 consecutive 16-bit elements of row t from column 4 q on;
-// lane i gets column i of rows 0 .. 3.
-__device__ __forceinline__ pu2 ld_tr16(const unsigned char* p) {
-  typedef short s4 __attribute__((ext_vector_type(4)));
-  const s4 r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4*)p);
-  pu2 v;
-  __builtin_memcpy(&v, &r, 8);
-  return v;
-}
 // maximum over lanes l, l ^ 16, l ^ 32, l ^ 48
 __device__ __forceinline__ float xmaximum(float v) {
   auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
@@ -84,7 +75,7 @@ __device__ __forceinline__ float xmaximum(float v) {
 __device__ __forceinline__ float max3(float a, float b, float c) { return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c); }
 
 template <int DT, int ODT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void prefill_attn_mfma_hd64(PrefillParams P) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void prefill_attn_mfma_hd64(PrefillParams P) {
   // one object per stage: the compiler can then tell that reads of one do not touch the one a load is filling
   __shared__ __attribute__((aligned(1024))) unsigned char s0[2][4096], s1[2][4096], s2[2][4096];  // [K, V][32 keys x 128 B]
   const int tid = threadIdx.x;
@@ -136,6 +127,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void p
   if (P.window > 0 && row - P.window + 1 > lo_n) lo_n = row - P.window + 1;
   if (!row_ok) lo_n = INT_MAX;
   if (P.window > 0 && row0 - P.window + 1 > lo0) lo0 = row0 - P.window + 1;
+  const uint32_t n_keys = row_ok ? (uint32_t)(row - lo_n + 1) : 0u;           // the row sees keys lo_n .. lo_n + n_keys - 1
   const int rl = min(r0 + 15, P.N - 1);                                       // last real row of the block
   const int lo_first = __builtin_amdgcn_readfirstlane(lo_n);                  // lo is non-decreasing in the row
   const int lo_last = __builtin_amdgcn_readfirstlane(__shfl(lo_n, wave_ok ? rl - r0 : 0, 64));
@@ -146,15 +138,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void p
 
   // ---- K / V super-tiles go from global memory straight into one of three LDS stages, two tiles ahead: wave w moves keys 8 w .. 8 w + 7
   // of K and of V, 16 bytes per lane.  Keys are clamped to N - 1 (a clamped key is masked).  K rows keep their 16-byte chunks
-  // xor-ed with (key / 2) % 8, V rows theirs with 2 (key % 4), which makes the operand reads (lane = key m, chunk 4 s + g; four keys'
-  // 32 bytes per 16 lanes) free of bank conflicts.
+  // xor-ed with (key / 2) % 8, V rows theirs with 2 (key / 2 % 4), which makes the operand reads (lane = key m, chunk 4 s + g;
+  // eight keys' 32 bytes per 32 lanes) free of bank conflicts.
   const uint16_t* kbase = (const uint16_t*)P.k + (int64_t)kvh * P.skh;
   const uint16_t* vbase = (const uint16_t*)P.v + (int64_t)kvh * P.svh;
   const uint32_t skn2 = (uint32_t)P.skn * 2, svn2 = (uint32_t)P.svn * 2;  // row strides in bytes
   const __amdgpu_buffer_rsrc_t rK = __builtin_amdgcn_make_buffer_rsrc((void*)kbase, 0, (int)((uint32_t)(P.N - 1) * skn2 + 128), 0x00020000);
   const __amdgpu_buffer_rsrc_t rV = __builtin_amdgcn_make_buffer_rsrc((void*)vbase, 0, (int)((uint32_t)(P.N - 1) * svn2 + 128), 0x00020000);
   const int lkey = 8 * wave + (lane >> 3), lch = lane & 7;
-  const uint32_t kch = (uint32_t)((lch ^ ((lkey >> 1) & 7)) << 4), vch = (uint32_t)((lch ^ ((lkey & 3) << 1)) << 4);
+  const uint32_t kch = (uint32_t)((lch ^ ((lkey >> 1) & 7)) << 4), vch = (uint32_t)((lch ^ (lkey & 6)) << 4);
   auto issue = [&](unsigned char (*S)[4096], int k) {
     const uint32_t r = (uint32_t)min(kbeg_wg + 32 * k + lkey, P.N - 1);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rK, (__attribute__((address_space(3))) void*)(S[0] + 1024 * wave), 16, r * skn2 + kch, 0, 0, 0);
@@ -177,39 +169,47 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void p
   // 4 g .. 4 g + 3
   uint32_t vld[4];
 #pragma unroll
-  for (int t = 0; t < 4; t++) vld[t] = (uint32_t)(4 * g + (m >> 2)) * 128 + (uint32_t)(((2 * t + ((m & 3) >> 1)) ^ ((m >> 2) << 1)) << 4) + 8 * (m & 1);
+  for (int t = 0; t < 4; t++) vld[t] = (uint32_t)(4 * g + (m >> 2)) * 128 + (uint32_t)(((2 * t + ((m & 3) >> 1)) ^ ((4 * g + (m >> 2)) & 6)) << 4) + 8 * (m & 1);
 
-  auto step_t = [&](const unsigned char (*S)[4096], int tb, auto EDGE) {
-    constexpr bool edge = decltype(EDGE)::value;
+  auto step = [&](const unsigned char (*S)[4096], int k) __attribute__((always_inline)) {
+    const int tb = kbeg_wg + 32 * k;
+    if (tb < kbeg || tb >= kend) return;   // (wave-uniform)
     pu4 K[4];      // [tile A dims 0..31, tile A dims 32..63, tile B dims 0..31, tile B dims 32..63]: key m, dims 8g..8g+7
     K[0] = *(const pu4*)(S[0] + kld0);
     K[1] = *(const pu4*)(S[0] + kld1);
     K[2] = *(const pu4*)(S[0] + 2048 + kld0);
     K[3] = *(const pu4*)(S[0] + 2048 + kld1);
-    const int kA = tb + 4 * g, kB = kA + 16;  // first of this lane's 4 keys in tile A / B
     pu4 VA[4];     // V^T operands: row m is head dim 16 t + m; slots 0..3 are keys 4g+j of tile A, 4..7 of tile B
 #pragma unroll
     for (int tt = 0; tt < 4; tt++) {
       const pu2 a = ld_tr16(S[1] + vld[tt]), b = ld_tr16(S[1] + 2048 + vld[tt]);
       VA[tt] = pu4{a.x, a.y, b.x, b.y};
     }
+    float t[HPW][8];
 #pragma unroll
     for (int hh = 0; hh < HPW; hh++) {
       pf4 sA = mfma16<DT>(K[0], Q[hh][0], pf4{0.f, 0.f, 0.f, 0.f});
       pf4 sB = mfma16<DT>(K[2], Q[hh][0], pf4{0.f, 0.f, 0.f, 0.f});
       sA = mfma16<DT>(K[1], Q[hh][1], sA);
       sB = mfma16<DT>(K[3], Q[hh][1], sB);
-      float t[8] = {sA[0], sA[1], sA[2], sA[3], sB[0], sB[1], sB[2], sB[3]};
-      if (edge) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-          if (kA + i < lo_n || kA + i > row) t[i] = -INFINITY;
-          if (kB + i < lo_n || kB + i > row) t[4 + i] = -INFINITY;
-        }
+      for (int i = 0; i < 4; i++) { t[hh][i] = sA[i]; t[hh][4 + i] = sB[i]; }
+    }
+    if (tb < lo_last || tb + 31 > r0) {   // some row of the block does not see all of the tile
+      const uint32_t kA = (uint32_t)(tb + 4 * g - lo_n);
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        const bool out = kA + (i & 3) + 16 * (i >> 2) >= n_keys;
+#pragma unroll
+        for (int hh = 0; hh < HPW; hh++)
+          if (out) t[hh][i] = -INFINITY;
       }
+    }
+#pragma unroll
+    for (int hh = 0; hh < HPW; hh++) {
       // (the maximum that hands NaN on: one instruction for three values, where the one that ignores it needs each made quiet first; a
       // score that is NaN makes its row NaN either way)
-      const float mx = max3(max3(max3(t[0], t[1], t[2]), t[3], t[4]), max3(t[5], t[6], t[7]), mrun[hh]);
+      const float mx = max3(max3(max3(t[hh][0], t[hh][1], t[hh][2]), t[hh][3], t[hh][4]), max3(t[hh][5], t[hh][6], t[hh][7]), mrun[hh]);
       {  // rescale by alpha = exp2((m_old - m_new) c), 1 where the row's maximum did not grow.  Unconditional: a branch
          // here would split the heads into separate blocks and stop the scheduler from overlapping one head's
          // softmax arithmetic with the next head's MFMAs.  (A reference point that may lag behind the maximum, as the decode
@@ -224,26 +224,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void p
       const float mc = mrun[hh] == -INFINITY ? 0.f : mrun[hh] * c;
       float p[8];
 #pragma unroll
-      for (int i = 0; i < 8; i++) p[i] = __builtin_amdgcn_exp2f(fmaf(t[i], c, -mc));
+      for (int i = 0; i < 8; i++) p[i] = __builtin_amdgcn_exp2f(fmaf(t[hh][i], c, -mc));
       lrun[hh] += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
       const pu4 PB = pu4{pack2<DT>(p[0], p[1]), pack2<DT>(p[2], p[3]), pack2<DT>(p[4], p[5]), pack2<DT>(p[6], p[7])};
 #pragma unroll
       for (int tt = 0; tt < 4; tt++) O[hh][tt] = mfma16<DT>(VA[tt], PB, O[hh][tt]);
     }
   };
-  // a tile needs no mask when every row of the block sees all of it: it starts at or after the last row's lower bound and ends at or
-  // before the first row (the test is hoisted out of the head loop, so that the heads of a tile form one block the scheduler can
-  // interleave); a wave skips the tiles outside its own block's range
-  auto step = [&](const unsigned char (*S)[4096], int k) {
-    const int tb = kbeg_wg + 32 * k;
-    if (tb < kbeg || tb >= kend) return;   // (wave-uniform)
-    if (tb >= lo_last && tb + 31 <= r0) step_t(S, tb, std::false_type{}); else step_t(S, tb, std::true_type{});
-  };
   // iteration k: tile k has landed (own loads: the wait, which leaves tile k + 1's in flight; the other waves': the barrier) and every
   // wave is done with tile k - 1, whose stage takes tile k + 2
   auto iteration = [&](unsigned char (*S)[4096], unsigned char (*SN)[4096], int k) {
     if (k + 1 < nk) __builtin_amdgcn_s_waitcnt(0x0f72); else __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(2) / (0)
-    asm volatile("s_barrier" ::: "memory");
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if (k + 2 < nk) issue(SN, k + 2);
     step(S, k);
   };

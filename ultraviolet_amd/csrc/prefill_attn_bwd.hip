@@ -234,20 +234,26 @@ __global__ __launch_bounds__(64) void bwd_dkv_kernel(BwdParams P) {
 // Same mathematics on the matrix cores, on the forward kernel's operand layouts (prefill_attn.hip):
 //   * the rows' log-sum-exp (log2 domain) is the forward's, or comes from one more run of the forward kernel without output;
 //   * bwd_dq_mfma: a workgroup owns 16 query rows of one kv head, wave w the query heads 2w, 2w+1 of the group.  K and V
-//     super-tiles (32 keys) are staged once per workgroup in LDS.  S^T = K Q^T and dP^T = V dO^T have the same shape: a lane
+//     super-tiles (32 keys) are staged once per workgroup in LDS, as in the forward.  S^T = K Q^T and dP^T = V dO^T have the same shape: a lane
 //     of either accumulator holds 4 consecutive keys of one query row for two 16-key tiles, so p = exp2(c s - lse) and
 //     ds = p (dp - D) are lane-local, and the 8 values of ds, rounded to the input type, are the lane's slice of the B
-//     operand of dQ^T += K^T dS^T (K^T operands from 8-byte LDS reads regrouped with v_perm_b32, as V^T in the forward);
+//     operand of dQ^T += K^T dS^T (K^T operands from the transposing LDS read, as V^T in the
+//     forward);
 //   * bwd_dkv_mfma: the transposed problem.  A workgroup owns 64 keys of one kv head and walks (query tile of 32, pair of query
 //     heads): the tile's Q and dO rows are staged in LDS; S = Q K^T and dP = dO V^T leave 4 consecutive queries
 //     of one key in a lane for two 16-query tiles, exactly the B-operand slices of dV^T += dO^T P and dK^T += Q^T dS, which
 //     accumulate over the tiles and over the heads of the group in registers.
-// Probabilities and ds are rounded to the input type for their second products; everything else is fp32.
+// The accumulators of dP start at -D.  Probabilities and ds are rounded to the input type for their second products; everything else is
+// fp32.  Both kernels keep a tile's mask in a branch of its own, with the products on both sides of it outside: as two versions of the
+// whole tile the accumulators of the two met in copies, 32 and 64 registers of them a tile.
+//
+// us, forward's statistics at hand: 61 x 16 .. 1024 tokens, window 256: 122 -> 98 (dq 49 -> 42, dk / dv 73 -> 56); without a window 252 -> 189;
+// 20 x 512, window 256, 65 -> 52; 4 x 2048 300 -> 225; 400 67 -> 51; 93 24.0 -> 19.6.
 struct BwdMParams {
   const void* q; const void* k; const void* v; const void* o; const void* go;
   void* dq; void* dk; void* dv;
   const float* lse; int64_t lse_ld;            // (H, lse_ld): log2-domain log-sum-exp of a row
-  float* dsum; int64_t ls;                      // (H, ls): D = go . o
+  float* dsum; int64_t ls;                      // (H, ls): -D = -(go . o)
   const int32_t* seg_start;                     // (ls,) first token of each token's sequence (entries >= N unused)
   const void* cu; int idx64, n_seg;
   int N, H, KH, G, window, n_wg;
@@ -266,55 +272,46 @@ __device__ __forceinline__ float dot2w(uint32_t a, uint32_t b, float acc) {  // 
   return fmaf(a1, b1, fmaf(a0, b0, acc));
 }
 
-// Four transposed operands from eight 8-byte reads: r[j] holds dims 4m..4m+3 of contraction slot j's row; operand t, row m is
-// dim 4m + t, dword p of an operand holds slots 2p, 2p+1.
-__device__ __forceinline__ void transpose_ops(const pu2* r, pu4* op) {
-  constexpr uint32_t LO = 0x05040100u, HI = 0x07060302u;
-#pragma unroll
-  for (int p = 0; p < 4; p++) {
-    op[0][p] = __builtin_amdgcn_perm(r[2 * p + 1].x, r[2 * p].x, LO);
-    op[1][p] = __builtin_amdgcn_perm(r[2 * p + 1].x, r[2 * p].x, HI);
-    op[2][p] = __builtin_amdgcn_perm(r[2 * p + 1].y, r[2 * p].y, LO);
-    op[3][p] = __builtin_amdgcn_perm(r[2 * p + 1].y, r[2 * p].y, HI);
-  }
-}
+// A staged tile of 32 rows of 128 bytes: row r keeps its 16-byte chunks xor-ed with the bits 1, 2 and then 3 of r / 2 rotated to the left.
+// Rows r and r + 1 share a 256-byte line of banks, so both reads of a tile are free of conflicts: 16 lanes' 16 bytes of one chunk of 16
+// rows (eight different places per half line), and 32 lanes' transposing reads of two neighbouring chunks of 8 rows (four pairs of places).
+__device__ __forceinline__ int tile_swizzle(int row) { return ((row & 6) | ((row >> 3) & 1)); }
 
-// LDS reads of a staged 32-row tile (rows of 128 bytes, chunk-swizzled): the A-operand form (lane = row m of tile A / B,
-// dims 8g.. of each half) and the rows for the transposed form (rows 4g+j of tile A / B, dims 4m..4m+3).
-__device__ __forceinline__ void read_rows_a(const unsigned char* s, int m, int g, pu4* a) {
-  const uint32_t o0 = lds_chunk_off(m, g), o1 = lds_chunk_off(m, 4 + g);   // (rows m and 16 + m swizzle alike)
-  a[0] = *(const pu4*)(s + o0);
-  a[1] = *(const pu4*)(s + o1);
-  a[2] = *(const pu4*)(s + 2048 + o0);
-  a[3] = *(const pu4*)(s + 2048 + o1);
-}
-__device__ __forceinline__ void read_rows_t(const unsigned char* s, int m, int g, pu2* r) {
+// Operands of a staged tile.  Rows: [tile A dims 0..31, A dims 32..63, B dims 0..31, B dims 32..63], lane = row m, dims 8 g .. ;
+// transposed: operand t is dim 16 t + m, slots 0..3 are rows 4 g + j of tile A, 4..7 of tile B.
+struct TileReads {
+  uint32_t row[2], col[4];
+  __device__ __forceinline__ TileReads(int m, int g) {
 #pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const uint32_t o = lds_chunk_off(4 * g + j, m >> 1) + 8 * (m & 1);
-    r[j] = *(const pu2*)(s + o);
-    r[4 + j] = *(const pu2*)(s + 2048 + o);
+    for (int s = 0; s < 2; s++) row[s] = (uint32_t)(m * 128 + (((4 * s + g) ^ tile_swizzle(m)) << 4));
+    const int r = 4 * g + (m >> 2);   // the row that this lane names to the transposing read, 4 dims from 4 (m % 4)
+#pragma unroll
+    for (int t = 0; t < 4; t++) col[t] = (uint32_t)(r * 128 + (((2 * t + ((m & 3) >> 1)) ^ tile_swizzle(r)) << 4) + 8 * (m & 1));
   }
-}
+  __device__ __forceinline__ void rows(const unsigned char* s, pu4* a) const {
+    a[0] = *(const pu4*)(s + row[0]);
+    a[1] = *(const pu4*)(s + row[1]);
+    a[2] = *(const pu4*)(s + 2048 + row[0]);
+    a[3] = *(const pu4*)(s + 2048 + row[1]);
+  }
+  __device__ __forceinline__ pu4 cols(const unsigned char* s, int t) const {
+    const pu2 a = ld_tr16(s + col[t]), b = ld_tr16(s + 2048 + col[t]);
+    return pu4{a.x, a.y, b.x, b.y};
+  }
+};
 
 template <int DT>
-__device__ __forceinline__ void store_dims16(void* base, int64_t off, const pf4* acc, float mul) {  // acc[t][i] is dim 4 i + t of the lane's 16
-  float o[16];
+__device__ __forceinline__ void store_dims16(void* base, int64_t off, const pf4* acc, float mul) {  // acc[t][i] is dim 16 t + i from `off` on
+  uint16_t* p = (uint16_t*)base + off;
 #pragma unroll
   for (int t = 0; t < 4; t++)
-#pragma unroll
-    for (int i = 0; i < 4; i++) o[4 * i + t] = acc[t][i] * mul;
-  uint32_t w[8];
-#pragma unroll
-  for (int i = 0; i < 8; i++) w[i] = pack2<DT>(o[2 * i], o[2 * i + 1]);
-  uint16_t* p = (uint16_t*)base + off;
-  *(uint4*)p = uint4{w[0], w[1], w[2], w[3]};
-  *(uint4*)(p + 8) = uint4{w[4], w[5], w[6], w[7]};
+    *(uint2*)(p + 16 * t) = uint2{pack2<DT>(acc[t][0] * mul, acc[t][1] * mul), pack2<DT>(acc[t][2] * mul, acc[t][3] * mul)};
 }
 
 template <int DT>
-__global__ __launch_bounds__(256) void bwd_dq_mfma(BwdMParams P) {
-  __shared__ __attribute__((aligned(16))) unsigned char smem[2][2][4096];  // [half][K, V][32 keys x 128 B]
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void bwd_dq_mfma(BwdMParams P) {
+  // one object per stage: the compiler can then tell that reads of one do not touch the one a load is filling
+  __shared__ __attribute__((aligned(1024))) unsigned char s0[2][4096], s1[2][4096], s2[2][4096];  // [K, V][32 keys x 128 B]
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int per = gridDim.x >> 3;
   const int bid = (blockIdx.x & 7) * per + (blockIdx.x >> 3);   // an XCD (ids congruent mod 8) gets a contiguous range
@@ -323,26 +320,14 @@ __global__ __launch_bounds__(256) void bwd_dq_mfma(BwdMParams P) {
   const int m = lane & 15, g = lane >> 4;
   const int G = P.G;
   const float c = P.scale_log2;
-  int n_end = (int)load_index(P.cu, P.idx64, P.n_seg);   // tokens at or after it are padding
-  n_end = n_end < 0 ? 0 : (n_end > P.N ? P.N : n_end);
   const int r0 = qb * 16, row = r0 + m;
-  const bool row_ok = row < n_end;
   const int rowc = row < P.N ? row : P.N - 1;
-  int lo_n = P.seg_start[rowc];
-  if (P.window > 0 && row - P.window + 1 > lo_n) lo_n = row - P.window + 1;
-  if (!row_ok) lo_n = INT_MAX;
-  // the block's key range: from its first live row's lower bound to its last live row (none: no tile)
-  const int rl = min(r0 + 15, n_end - 1);
-  const bool any = r0 < n_end;
-  const int lo_first = __builtin_amdgcn_readfirstlane(lo_n);
-  const int lo_last = __builtin_amdgcn_readfirstlane(__shfl(lo_n, any ? rl - r0 : 0, 64));
-  const int kbeg = any ? lo_first & ~31 : 0, kend = any ? rl + 1 : 0;
-  const int nk = (kend - kbeg + 31) >> 5;
-
-  // ---- Q^T and dO^T operands (lane = row m, dims 32 s + 8 g ..), D = dO . O, the row's log-sum-exp
-  pu4 Q[2][2], GO[2][2];
-  float lse2[2], Dr[2];
+  // ---- what depends on the row alone goes out first: Q^T, dO^T and O operands (lane = row m, dims 32 s + 8 g ..), the row's statistics
+  pu4 Q[2][2], GO[2][2], Ov[2][2];
+  float lse2[2];
   bool hok[2];
+  int lo_n = P.seg_start[rowc];
+  int n_end = (int)load_index(P.cu, P.idx64, P.n_seg);   // tokens at or after it are padding
 #pragma unroll
   for (int hh = 0; hh < 2; hh++) {
     const int hq = 2 * wave + hh;
@@ -353,106 +338,136 @@ __global__ __launch_bounds__(256) void bwd_dq_mfma(BwdMParams P) {
     Q[hh][1] = *(const pu4*)((const uint16_t*)P.q + base + 32);
     GO[hh][0] = *(const pu4*)((const uint16_t*)P.go + base);
     GO[hh][1] = *(const pu4*)((const uint16_t*)P.go + base + 32);
-    const pu4 o0 = *(const pu4*)((const uint16_t*)P.o + base), o1 = *(const pu4*)((const uint16_t*)P.o + base + 32);
+    Ov[hh][0] = *(const pu4*)((const uint16_t*)P.o + base);
+    Ov[hh][1] = *(const pu4*)((const uint16_t*)P.o + base + 32);
+    lse2[hh] = P.lse[(int64_t)head * P.lse_ld + rowc];
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  n_end = n_end < 0 ? 0 : (n_end > P.N ? P.N : n_end);
+  const bool row_ok = row < n_end;
+  if (P.window > 0 && row - P.window + 1 > lo_n) lo_n = row - P.window + 1;
+  if (!row_ok) lo_n = INT_MAX;
+  // the block's key range: from its first live row's lower bound to its last live row (none: no tile)
+  const int rl = min(r0 + 15, n_end - 1);
+  const bool any = r0 < n_end;
+  const int lo_first = __builtin_amdgcn_readfirstlane(lo_n);
+  const int lo_last = __builtin_amdgcn_readfirstlane(__shfl(lo_n, any ? rl - r0 : 0, 64));
+  const int kbeg = any ? lo_first & ~31 : 0, kend = any ? rl + 1 : 0;
+  const int nk = __builtin_amdgcn_readfirstlane((kend - kbeg + 31) >> 5);
+  const uint32_t n_keys = row_ok ? (uint32_t)(row - lo_n + 1) : 0u;   // the row sees keys lo_n .. lo_n + n_keys - 1
+
+  // ---- K / V tiles go from global memory straight into one of three LDS stages, two tiles ahead: wave w moves rows 8 w .. 8 w + 7
+  const uint32_t rstride = (uint32_t)P.KH * 128;
+  const int kv_bytes = (int)((uint32_t)P.N * rstride - (uint32_t)kvh * 128);
+  const __amdgpu_buffer_rsrc_t rK = __builtin_amdgcn_make_buffer_rsrc((void*)((const uint16_t*)P.k + (int64_t)kvh * 64), 0, kv_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rV = __builtin_amdgcn_make_buffer_rsrc((void*)((const uint16_t*)P.v + (int64_t)kvh * 64), 0, kv_bytes, 0x00020000);
+  const int lkey = 8 * wave + (lane >> 3);
+  const uint32_t lch = (uint32_t)(((lane & 7) ^ tile_swizzle(lkey)) << 4);
+  auto issue = [&](unsigned char (*S)[4096], int k) {   // (keys are clamped: a clamped key is masked)
+    const uint32_t off = (uint32_t)min(kbeg + 32 * k + lkey, P.N - 1) * rstride + lch;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rK, (__attribute__((address_space(3))) void*)(S[0] + 1024 * wave), 16, off, 0, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rV, (__attribute__((address_space(3))) void*)(S[1] + 1024 * wave), 16, off, 0, 0, 0);
+  };
+  if (nk > 0) issue(s0, 0);
+  if (nk > 1) issue(s1, 1);
+
+  // ---- D = dO . O; -D is where the accumulators of dP^T start
+  pf4 nD[2], dQ[2][4];
+#pragma unroll
+  for (int hh = 0; hh < 2; hh++) {
     float d = 0.f;
 #pragma unroll
-    for (int i = 0; i < 4; i++) d = dot2w<DT>(GO[hh][1][i], o1[i], dot2w<DT>(GO[hh][0][i], o0[i], d));
-    d = psum32(psum16(d));
-    Dr[hh] = d;
-    lse2[hh] = row_ok ? P.lse[(int64_t)head * P.lse_ld + row] : INFINITY;
-    if (hok[hh] && g == 0 && row < P.N) P.dsum[(int64_t)head * P.ls + row] = row_ok ? d : 0.f;
-  }
-  pf4 dQ[2][4];
-#pragma unroll
-  for (int hh = 0; hh < 2; hh++)
+    for (int i = 0; i < 4; i++) d = dot2w<DT>(GO[hh][1][i], Ov[hh][1][i], dot2w<DT>(GO[hh][0][i], Ov[hh][0][i], d));
+    d = -psum32(psum16(d));
+    nD[hh] = pf4{d, d, d, d};
+    if (!row_ok) lse2[hh] = INFINITY;
 #pragma unroll
     for (int t = 0; t < 4; t++) dQ[hh][t] = pf4{0.f, 0.f, 0.f, 0.f};
-
-  // ---- K / V tiles: global -> registers -> LDS, one tile ahead of the arithmetic
-  const uint16_t* kbase = (const uint16_t*)P.k + (int64_t)kvh * 64;
-  const uint16_t* vbase = (const uint16_t*)P.v + (int64_t)kvh * 64;
-  const int64_t rstride = (int64_t)P.KH * 64;
-  const int lkey = tid >> 3, lch = tid & 7;
-  const uint32_t st_off = lds_chunk_off(lkey, lch);
-  pu4 rk, rv;
-  auto fetch = [&](int kt) {
-    const int tb = kbeg + 32 * min(kt, max(nk - 1, 0));
-    const int64_t r = (int64_t)min(tb + lkey, P.N - 1) * rstride + 8 * lch;
-    rk = *(const pu4*)(kbase + r);
-    rv = *(const pu4*)(vbase + r);
-  };
-  auto park = [&](int half) {
-    *(pu4*)(&smem[half][0][st_off]) = rk;
-    *(pu4*)(&smem[half][1][st_off]) = rv;
-  };
-  const bool work = hok[0];   // (wave-uniform: a wave without a head only helps with the loads)
-  auto step = [&](int half, int tb) {
+  }
+  const TileReads at(m, g);
+  auto step = [&](const unsigned char (*S)[4096], int tb) __attribute__((always_inline)) {
     pu4 KA[4], VA[4], KT[4];
-    pu2 kt[8];
-    read_rows_a(smem[half][0], m, g, KA);
-    read_rows_a(smem[half][1], m, g, VA);
-    read_rows_t(smem[half][0], m, g, kt);
-    transpose_ops(kt, KT);
-    const bool edge = !(tb >= lo_last && tb + 31 <= r0);
-    const int kA = tb + 4 * g, kB = kA + 16;
+    at.rows(S[0], KA);
+    at.rows(S[1], VA);
+#pragma unroll
+    for (int t = 0; t < 4; t++) KT[t] = at.cols(S[0], t);
+    float p[2][8];
+    pf4 dP[2][2];
 #pragma unroll
     for (int hh = 0; hh < 2; hh++) {
-      if (!hok[hh]) continue;
-      pf4 sA = pf4{0.f, 0.f, 0.f, 0.f}, sB = sA, pA = sA, pB = sA;
+      pf4 sA = pf4{0.f, 0.f, 0.f, 0.f}, sB = sA, pA = nD[hh], pB = pA;
       sA = mfma16<DT>(KA[0], Q[hh][0], sA);
       sB = mfma16<DT>(KA[2], Q[hh][0], sB);
       pA = mfma16<DT>(VA[0], GO[hh][0], pA);
       pB = mfma16<DT>(VA[2], GO[hh][0], pB);
       sA = mfma16<DT>(KA[1], Q[hh][1], sA);
       sB = mfma16<DT>(KA[3], Q[hh][1], sB);
-      pA = mfma16<DT>(VA[1], GO[hh][1], pA);
-      pB = mfma16<DT>(VA[3], GO[hh][1], pB);
-      float ds[8];
+      dP[hh][0] = mfma16<DT>(VA[1], GO[hh][1], pA);
+      dP[hh][1] = mfma16<DT>(VA[3], GO[hh][1], pB);
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        float p0 = __builtin_amdgcn_exp2f(fmaf(sA[i], c, -lse2[hh])), p1 = __builtin_amdgcn_exp2f(fmaf(sB[i], c, -lse2[hh]));
-        if (edge) {
-          if (kA + i < lo_n || kA + i > row) p0 = 0.f;
-          if (kB + i < lo_n || kB + i > row) p1 = 0.f;
-        }
-        ds[i] = p0 * (pA[i] - Dr[hh]);
-        ds[4 + i] = p1 * (pB[i] - Dr[hh]);
+        p[hh][i] = __builtin_amdgcn_exp2f(fmaf(sA[i], c, -lse2[hh]));
+        p[hh][4 + i] = __builtin_amdgcn_exp2f(fmaf(sB[i], c, -lse2[hh]));
       }
+    }
+    if (!(tb >= lo_last && tb + 31 <= r0)) {   // some row of the block does not see all keys of the tile
+      const uint32_t kA = (uint32_t)(tb + 4 * g - lo_n);
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        const bool out = kA + (i & 3) + 16 * (i >> 2) >= n_keys;
+        if (out) p[0][i] = 0.f;
+        if (out) p[1][i] = 0.f;
+      }
+    }
+#pragma unroll
+    for (int hh = 0; hh < 2; hh++) {
+      float ds[8];
+#pragma unroll
+      for (int i = 0; i < 8; i++) ds[i] = p[hh][i] * dP[hh][i >> 2][i & 3];
       const pu4 dsB = pu4{pack2<DT>(ds[0], ds[1]), pack2<DT>(ds[2], ds[3]), pack2<DT>(ds[4], ds[5]), pack2<DT>(ds[6], ds[7])};
 #pragma unroll
       for (int t = 0; t < 4; t++) dQ[hh][t] = mfma16<DT>(KT[t], dsB, dQ[hh][t]);
     }
   };
-  if (nk > 0) {
-    fetch(0);
-    park(0);
-    __syncthreads();
-    for (int kt = 0; kt < nk; kt++) {
-      fetch(kt + 1);
-      if (work) step(kt & 1, kbeg + 32 * kt);
-      park((kt + 1) & 1);
-      __syncthreads();
-    }
+  const bool work = hok[0];   // (wave-uniform: a wave without a head only helps with the loads)
+  // iteration k: tile k has landed (own loads: the wait, which leaves tile k + 1's in flight; the other waves': the barrier) and every
+  // wave is done with tile k - 1, whose stage takes tile k + 2
+  auto iteration = [&](unsigned char (*S)[4096], unsigned char (*SN)[4096], int k) {
+    if (k + 1 < nk) __builtin_amdgcn_s_waitcnt(0x0f72); else __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(2) / (0)
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (k + 2 < nk) issue(SN, k + 2);
+    if (work) step(S, kbeg + 32 * k);
+  };
+  int k = 0;
+  for (; k + 3 <= nk; k += 3) {
+    iteration(s0, s2, k);
+    iteration(s1, s0, k + 1);
+    iteration(s2, s1, k + 2);
   }
-  // ---- dq = scale dQ; lane (row m, group g) holds head dims 16g .. 16g+15 (zeros for padding rows)
+  if (k < nk) iteration(s0, s2, k);
+  if (k + 1 < nk) iteration(s1, s0, k + 1);
+  // ---- dq = scale dQ; lane (row m, group g) holds head dims 16 t + 4 g + i (zeros for padding rows)
   if (row < P.N) {
 #pragma unroll
     for (int hh = 0; hh < 2; hh++) {
       if (!hok[hh]) continue;
       const int head = kvh * G + 2 * wave + hh;
-      store_dims16<DT>(P.dq, ((int64_t)row * P.H + head) * 64 + 16 * g, dQ[hh], P.scale);
+      if (g == 0) P.dsum[(int64_t)head * P.ls + row] = row_ok ? nD[hh][0] : 0.f;
+      store_dims16<DT>(P.dq, ((int64_t)row * P.H + head) * 64 + 4 * g, dQ[hh], P.scale);
     }
   }
 }
 
-// dk / dv.  What bounds it is the vector work per (query, key) pair (an exponential and ~8 instructions) and, before it was
-// pipelined, the round trips of the staged tiles: 31 700 tokens, window 256, took 130 us with 16 keys per wave, one tile in flight and
-// the statistics read from global memory inside the arithmetic; 72 us as it is now:
-//   * a wave owns 32 keys, so the operands of a query tile (16 KB of LDS reads, 32 permutes) serve two 16-key columns; the
-//     workgroup's waves are 2 key groups x 2 heads of a pair, which add their sums through LDS at the end;
+// dk / dv.  What bounds it is a tile's chain (LDS reads, products, exponentials, products) at two waves per SIMD: 512 cycles of matrix
+// instructions and about as many of vector instructions of the ~1 700 that a wave takes a tile.  Three waves per SIMD would need 168
+// registers; it takes 240, and with fewer it spills.
+//   * a wave owns 32 keys, so the operands of a query tile (16 KB of LDS reads, all requested at the tile's start) serve two 16-key
+//     columns; the workgroup's waves are 2 key groups x 2 heads of a pair, which add their sums through LDS at the end.  A wave skips
+//     the query tiles that see none of its keys and masks those that see some: 9 of the 10 tiles of a window of 256, two masked;
 //   * the pair's Q and dO tiles and their statistics go from global memory straight into one of three LDS stages, two
 //     iterations ahead of their use (no staging registers; a wave's 1 KB load is 8 rows, the chunk swizzle is applied to the
-//     global address); an iteration waits for the loads of the one before last only;
+//     global address); an iteration waits for the loads of the one before last only.  The first two are requested before the search
+//     for the sequences;
 //   * the queries a key sees are an index range, key .. min(end of its sequence, key + window), found once per lane: the loop
 //     reads no tables.
 struct DkvStage { unsigned char t[4][4096]; float st[4][64]; };   // Q of head 0, 1, dO of head 0, 1; lse of head 0, 1, D of head 0, 1
@@ -473,7 +488,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   int n_end = (int)load_index(P.cu, P.idx64, P.n_seg);
   n_end = n_end < 0 ? 0 : (n_end > P.N ? P.N : n_end);
   const int jw0 = kb * 64, jw_last = min(jw0 + 63, n_end - 1);
-  const int key0 = jw0 + 32 * kg + n;       // column block b: key0 + 16 b
+  const int jw = jw0 + 32 * kg;             // the wave's first key
+  const int key0 = jw + n;                  // column block b: key0 + 16 b
   // ---- K^T / V^T operands (B side: lane = key, dims 32 s + 8 g ..)
   pu4 Kb[2][2], Vb[2][2];
 #pragma unroll
@@ -489,6 +505,33 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   for (int b = 0; b < 2; b++)
 #pragma unroll
     for (int t = 0; t < 4; t++) dK[b][t] = dV[b][t] = pf4{0.f, 0.f, 0.f, 0.f};
+  // ---- loader: wave w fills tile w and statistics row w of a stage: Q / dO of head w % 2, four loads of 8 rows
+  const int lrow = lane >> 3;
+  const uint32_t rstride = (uint32_t)P.H * 128;
+  const int64_t st_ld = wave < 2 ? P.lse_ld : P.ls;
+  const __amdgpu_buffer_rsrc_t rT = __builtin_amdgcn_make_buffer_rsrc((void*)(wave < 2 ? P.q : P.go), 0, (int)((uint32_t)P.N * rstride), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rS = __builtin_amdgcn_make_buffer_rsrc((void*)(wave < 2 ? P.lse : P.dsum), 0, (int)((st_ld * (P.H - 1) + P.N + 32) * 4), 0x00020000);
+  uint32_t l_off[4], l_st = (uint32_t)(jw0 + (lane & 31)) * 4;   // offsets of the next tile's rows (head 0) and statistics
+#pragma unroll
+  for (int i = 0; i < 4; i++) l_off[i] = (uint32_t)(jw0 + 8 * i + lrow) * rstride + (uint32_t)(((lane & 7) ^ tile_swizzle(8 * i + lrow)) << 4);
+  int f_p = 0;   // head pair of the next request
+  auto issue = [&](DkvStage& S) {   // (rows past the last token come out as zeros: the descriptor's bound)
+    const int head = kvh * G + min(2 * f_p + (wave & 1), G - 1);
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rT, (__attribute__((address_space(3))) void*)(S.t[wave] + 1024 * i), 16, l_off[i] + (uint32_t)head * 128, 0, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rS, (__attribute__((address_space(3))) void*)S.st[wave], 4, l_st + (uint32_t)(head * st_ld) * 4, 0, 0, 0);
+    if (++f_p == GP) {
+      f_p = 0;
+#pragma unroll
+      for (int i = 0; i < 4; i++) l_off[i] += 32 * rstride;
+      l_st += 128;
+    }
+  };
+  if (jw0 < n_end) {   // (at least one tile: the keys' own)
+    issue(s0);
+    issue(s1);
+  }
   // ---- sequences of the first and the last key (the last s with cu[s] <= key), 64 probes at a time
   auto seq_of = [&](int j) {
     int lo = 0, hi = P.n_seg;   // cu[lo] <= j, and hi == n_seg or cu[hi] > j
@@ -500,65 +543,60 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
     return lo;
   };
-  int first_end = 0, last_end = 0, hi_q[2] = {0, 0};   // ends of those sequences; key block b is seen by queries key .. hi_q[b] - 1
+  // key block b is seen by the n_q[b] queries from the key on
+  int first_end = 0, qend = 0, qend_w = 0;   // end of the sequence of the wave's first key; of the workgroup's and of the wave's queries
+  uint32_t n_q[2] = {0, 0};
   if (jw0 < n_end) {
     const int sf = seq_of(jw0), sl = seq_of(jw_last);
-    first_end = min((int)load_index(P.cu, P.idx64, sf + 1), n_end);
-    last_end = min((int)load_index(P.cu, P.idx64, sl + 1), n_end);
-    hi_q[0] = hi_q[1] = last_end;
+    const int last_end = min((int)load_index(P.cu, P.idx64, sl + 1), n_end);
+    int hi_q[2] = {last_end, last_end};
     for (int s = sl - 1; s >= sf; s--) {
       const int e = (int)load_index(P.cu, P.idx64, s + 1);
 #pragma unroll
       for (int b = 0; b < 2; b++)
         if (key0 + 16 * b < e) hi_q[b] = e;
     }
+    first_end = __builtin_amdgcn_readfirstlane(hi_q[0]);
+    qend = qend_w = last_end;
+    if (P.window > 0) {
+      qend = min(qend, jw_last + P.window);
+      qend_w = min(qend_w, min(jw + 31, n_end - 1) + P.window);
+    }
+    if (jw >= n_end) qend_w = 0;
 #pragma unroll
     for (int b = 0; b < 2; b++) {
       if (P.window > 0) hi_q[b] = min(hi_q[b], key0 + 16 * b + P.window);
-      if (key0 + 16 * b >= n_end) hi_q[b] = 0;
+      if (key0 + 16 * b < n_end) n_q[b] = (uint32_t)(hi_q[b] - key0 - 16 * b);
     }
   }
-  const int qend = P.window > 0 ? min(last_end, jw_last + P.window) : last_end;
+  // no mask in a query tile that starts in full_from .. full_to: every query follows every key of the wave, in the first key's sequence and window
+  const int full_from = jw + 31, full_to = (P.window > 0 ? min(first_end, jw + P.window) : first_end) - 32;
   const int n_it = jw0 < n_end ? ((qend - jw0 + 31) >> 5) * GP : 0;
-
-  // ---- loader: wave w fills tile w and statistics row w of a stage: Q / dO of head w % 2, four loads of 8 rows
-  const int lrow = lane >> 3, lch = lane & 7;
-  const uint16_t* lsrc = (const uint16_t*)(wave < 2 ? P.q : P.go);
-  const float* lst = wave < 2 ? P.lse : P.dsum;
-  const int64_t lst_ld = wave < 2 ? P.lse_ld : P.ls;
-  int f_t = 0, f_p = 0;   // tile and head pair of the next request
-  auto issue = [&](DkvStage& S) {
-    const int tq = jw0 + 32 * f_t, head = kvh * G + min(2 * f_p + (wave & 1), G - 1);
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int r = 8 * i + lrow;
-      const uint16_t* src = lsrc + ((int64_t)min(tq + r, P.N - 1) * P.H + head) * 64 + 8 * (lch ^ ((r >> 1) & 7));
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)(S.t[wave] + 1024 * i), 16, 0, 0);
-    }
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(lst + head * lst_ld + min(tq + (lane & 31), P.N - 1)),
-                                     (__attribute__((address_space(3))) void*)S.st[wave], 4, 0, 0);
-    if (++f_p == GP) { f_p = 0; f_t = min(f_t + 1, max((qend - jw0 - 1) >> 5, 0)); }   // (past the last tile: re-reads of it, into a stage nobody uses)
-  };
   int c_t = 0, c_p = 0;   // tile and head pair of the next arithmetic
-  auto step = [&](const DkvStage& S) {
+  const TileReads at(n, g);
+  auto step = [&](const DkvStage& S) __attribute__((always_inline)) {
     const int tq = jw0 + 32 * c_t;
     const bool live = 2 * c_p + hg < G;   // (an odd last head has no partner)
-    // no mask needed when every query of the tile follows every key, in the first key's sequence and window
-    const bool interior = tq >= jw0 + 63 && tq + 31 < first_end && (P.window == 0 || tq + 31 - jw0 < P.window);
     if (++c_p == GP) { c_p = 0; c_t++; }
-    if (!live) return;
+    if (!live || tq + 31 < jw || tq >= qend_w) return;   // (no query of the tile sees a key of the wave)
     const unsigned char* sq = S.t[hg];
     const unsigned char* sg = S.t[2 + hg];
     pu4 QA[4], GA[4];
-    read_rows_a(sq, n, g, QA);
-    read_rows_a(sg, n, g, GA);
+    at.rows(sq, QA);
+    at.rows(sg, GA);
     // statistics of this lane's queries tq + 4g + i (tile A) and tq + 16 + 4g + i (tile B)
     const pf4 lA = *(const pf4*)(S.st[hg] + 4 * g), lB = *(const pf4*)(S.st[hg] + 16 + 4 * g);
     const pf4 dA = *(const pf4*)(S.st[2 + hg] + 4 * g), dB = *(const pf4*)(S.st[2 + hg] + 16 + 4 * g);
-    pu4 PB[2], SB[2];
+    pu4 TG[4], TQ[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) TG[t] = at.cols(sg, t);
+#pragma unroll
+    for (int t = 0; t < 4; t++) TQ[t] = at.cols(sq, t);
+    __builtin_amdgcn_sched_barrier(0);
+    float p[2][8], ds[2][8];
 #pragma unroll
     for (int b = 0; b < 2; b++) {
-      pf4 sA = pf4{0.f, 0.f, 0.f, 0.f}, sB = sA, pA = sA, pB = sA;
+      pf4 sA = pf4{0.f, 0.f, 0.f, 0.f}, sB = sA, pA = dA, pB = dB;   // (dP starts at -D)
       sA = mfma16<DT>(QA[0], Kb[b][0], sA);
       sB = mfma16<DT>(QA[2], Kb[b][0], sB);
       pA = mfma16<DT>(GA[0], Vb[b][0], pA);
@@ -567,47 +605,46 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       sB = mfma16<DT>(QA[3], Kb[b][1], sB);
       pA = mfma16<DT>(GA[1], Vb[b][1], pA);
       pB = mfma16<DT>(GA[3], Vb[b][1], pB);
-      float p[8], ds[8];
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        p[i] = __builtin_amdgcn_exp2f(fmaf(sA[i], c, -lA[i]));
-        p[4 + i] = __builtin_amdgcn_exp2f(fmaf(sB[i], c, -lB[i]));
-        ds[i] = p[i] * (pA[i] - dA[i]);
-        ds[4 + i] = p[4 + i] * (pB[i] - dB[i]);
+        p[b][i] = __builtin_amdgcn_exp2f(fmaf(sA[i], c, -lA[i]));
+        p[b][4 + i] = __builtin_amdgcn_exp2f(fmaf(sB[i], c, -lB[i]));
+        ds[b][i] = p[b][i] * pA[i];
+        ds[b][4 + i] = p[b][4 + i] * pB[i];
       }
-      if (!interior) {   // (selects, not products: the statistics of a query past the last token are whatever the workspace held)
-        const int key = key0 + 16 * b;
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-          const int iq = tq + 4 * g + (i & 3) + 16 * (i >> 2);
-          if (iq < key || iq >= hi_q[b]) { p[i] = 0.f; ds[i] = 0.f; }
-        }
-      }
-      PB[b] = pu4{pack2<DT>(p[0], p[1]), pack2<DT>(p[2], p[3]), pack2<DT>(p[4], p[5]), pack2<DT>(p[6], p[7])};
-      SB[b] = pu4{pack2<DT>(ds[0], ds[1]), pack2<DT>(ds[2], ds[3]), pack2<DT>(ds[4], ds[5]), pack2<DT>(ds[6], ds[7])};
     }
-    pu2 rt[8];
-    pu4 T[4];
-    read_rows_t(sg, n, g, rt);
-    transpose_ops(rt, T);
+    if (tq < full_from || tq > full_to) {
+      // (selects, not products: the statistics of a query past the last token are whatever the workspace held)
 #pragma unroll
-    for (int t = 0; t < 4; t++)
+      for (int b = 0; b < 2; b++) {
+        const uint32_t from = (uint32_t)(tq + 4 * g - key0 - 16 * b);
 #pragma unroll
-      for (int b = 0; b < 2; b++) dV[b][t] = mfma16<DT>(T[t], PB[b], dV[b][t]);
-    read_rows_t(sq, n, g, rt);
-    transpose_ops(rt, T);
+        for (int i = 0; i < 8; i++)
+          if (from + (i & 3) + 16 * (i >> 2) >= n_q[b]) { p[b][i] = 0.f; ds[b][i] = 0.f; }
+      }
+    }
+    pu4 PB[2], SB[2];
 #pragma unroll
-    for (int t = 0; t < 4; t++)
+    for (int b = 0; b < 2; b++) {
+      PB[b] = pu4{pack2<DT>(p[b][0], p[b][1]), pack2<DT>(p[b][2], p[b][3]), pack2<DT>(p[b][4], p[b][5]), pack2<DT>(p[b][6], p[b][7])};
+      SB[b] = pu4{pack2<DT>(ds[b][0], ds[b][1]), pack2<DT>(ds[b][2], ds[b][3]), pack2<DT>(ds[b][4], ds[b][5]), pack2<DT>(ds[b][6], ds[b][7])};
+    }
 #pragma unroll
-      for (int b = 0; b < 2; b++) dK[b][t] = mfma16<DT>(T[t], SB[b], dK[b][t]);
+    for (int t = 0; t < 4; t++) {
+#pragma unroll
+      for (int b = 0; b < 2; b++) dV[b][t] = mfma16<DT>(TG[t], PB[b], dV[b][t]);
+    }
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+#pragma unroll
+      for (int b = 0; b < 2; b++) dK[b][t] = mfma16<DT>(TQ[t], SB[b], dK[b][t]);
+    }
   };
   if (n_it > 0) {
     // iteration i: request i + 2 into the stage that i - 1 used (every wave is done with it: the barrier), multiply i, wait
     // until i + 1 has landed (its 5 loads are all but the newest 5)
-    issue(s0);
-    issue(s1);
     __builtin_amdgcn_s_waitcnt(0x0f75);   // vmcnt(5)
-    __syncthreads();
+    asm volatile("s_barrier" ::: "memory");
 #define UVMI_DKV(CUR, NEXT2)                                             \
   do {                                                                   \
     issue(NEXT2);                                                        \
@@ -646,7 +683,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       for (int i = 0; i < 4; i++) acc[t][i] = (hg ? dV[b][t][i] : dK[b][t][i]) + theirs[((b * 4 + t) * 4 + i) * 64];
     const int key = key0 + 16 * b;
     if (key < P.N)   // (zeros for padding tokens)
-      store_dims16<DT>(hg ? P.dv : P.dk, ((int64_t)key * P.KH + kvh) * 64 + 16 * g, acc, hg ? 1.0f : P.scale);
+      store_dims16<DT>(hg ? P.dv : P.dk, ((int64_t)key * P.KH + kvh) * 64 + 4 * g, acc, hg ? 1.0f : P.scale);
   }
 }
 
@@ -706,7 +743,8 @@ extern "C" int uvmi_prefill_attn_bwd(const uvmi_prefill_attn_bwd_args* a, void* 
     M.q = a->q; M.k = a->k; M.v = a->v; M.o = a->o; M.go = a->go; M.dq = a->dq; M.dk = a->dk; M.dv = a->dv;
     M.lse = stats; M.lse_ld = stats_ld; M.dsum = dsum; M.ls = ls; M.seg_start = seg_start;
     M.cu = a->cu_seqlens; M.idx64 = a->idx_dtype == UVMI_I64 ? 1 : 0; M.n_seg = a->n_seg;
-    M.N = a->N; M.H = a->H; M.KH = a->KH; M.G = G; M.window = a->window;
+    M.N = a->N; M.H = a->H; M.KH = a->KH; M.G = G; M.window = a->window < a->N ? a->window : 0;   // (a window of all tokens hides none)
+   
     M.scale = a->scale; M.scale_log2 = a->scale * 1.4426950408889634f;
     M.n_wg = ((a->N + 15) / 16) * a->KH;
     const dim3 blk4(256), gq((unsigned)((M.n_wg + 7) / 8 * 8));
