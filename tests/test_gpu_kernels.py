@@ -1080,6 +1080,38 @@ def test_tile_of_passes_of_many_rows(M, K, N, epi, tile):
     assert bool(((got[rows].double() - p).abs() <= 8 * 2.0 ** -8 * p.abs().clamp_min(1.0)).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("K", [128, 192, 640])
+@pytest.mark.parametrize("config", [5, 6])
+def test_big_tiles_in_several_rounds(dtype, K, config):
+    """A workgroup that takes several tiles has the next one's first slabs on their way during a tile's last two (K = 128: all of its
+    slabs; K = 192, an odd number, a workgroup per tile): bit for bit the product of row slices that are one round of the device each,
+    for every epilogue, with the pre-norm, the residual in place and ragged edges; and near the float64 product at the slices' edges."""
+    from ultraviolet_amd.kernels.gemm import RESID, SOFTCAP, STORE, SWIGLU, gemm_tn
+    M, N, step = 7697, 3312, 1024
+    g = torch.Generator(device="cuda").manual_seed(K + config)
+    a, w = (torch.randn(s, K, device="cuda", generator=g).to(dtype) for s in (M, N))
+    w = (w.float() / K ** 0.5).to(dtype)
+    r = torch.randn(M, N, device="cuda", generator=g).to(dtype)
+    for kw in (dict(norm_eps=1e-6), dict(), dict(epilogue=SWIGLU, norm_eps=1e-6), dict(epilogue=RESID, ca=0.75, cb=1.25), dict(epilogue=SOFTCAP, ca=23.0, cb=5.0, cap_c=7.5)):
+        n = N // 32 * 32 if kw.get("epilogue") == SWIGLU else N
+        res = lambda lo, hi: dict(resid=r[lo:hi]) if kw.get("epilogue") == RESID else {}
+        got = gemm_tn(a, w[:n], config=config, **res(0, M), **kw)
+        want = torch.cat([gemm_tn(a[lo:lo + step], w[:n], config=config, **res(lo, lo + step), **kw) for lo in range(0, M, step)])
+        assert torch.equal(got, want), kw
+        if kw.get("epilogue") == RESID:
+            c = r.clone()
+            gemm_tn(a, w[:n], config=config, resid=c, out=c, **kw)
+            assert torch.equal(c, want)
+        elif kw.get("epilogue", STORE) == STORE:
+            rows = torch.tensor([0, 255, 256, step - 1, step, M - 1], device="cuda")
+            x = a[rows].double()
+            if "norm_eps" in kw:
+                x = x * torch.rsqrt((x * x).mean(1, keepdim=True) + 1e-6)
+            p = x @ w[:n].double().t()
+            assert bool(((got[rows].double() - p).abs() <= (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11) * p.abs().clamp_min(1.0)).all())
+
+
 def _fused_case(B, S, ring, kv, dtype, seed, any_ring=False):
     """A fused decode launch on random data: (launch(out, caches, oproj), caches, extras)."""
     from ultraviolet_amd.kernels.decode_attn import decode_attention_fused, rope_table

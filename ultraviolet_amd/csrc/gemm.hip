@@ -7,7 +7,7 @@ using namespace uvmi;
 
 namespace uvmi {
 void gemm_tile_launch(const uvmi_gemm_args* a, hipStream_t st);                     // gemm_tile.hip
-void gemm_big_launch(const uvmi_gemm_args* a, int tile, hipStream_t st);            // gemm_big.hip
+void gemm_big_launch(const uvmi_gemm_args* a, int tile, int cus, hipStream_t st);   // gemm_big.hip
 int gemm_stream_form(const uvmi_gemm_args* a, int cus);                             // gemm_stream.hip
 void gemm_stream_launch(const uvmi_gemm_args* a, int form, int cus, hipStream_t st);
 }
@@ -25,11 +25,11 @@ static bool big_ok(const uvmi_gemm_args* a) {
 
 // Whether a pass of many rows takes 256 x 256 tiles rather than 128 x 128 ones.  A launch lasts as long as its rounds of the device: of
 // one 256 x 256 tile per compute unit, or of two 128 x 128 ones, which take about 0.6 of that.  us, 256 against 128, activations in
-// the last-level cache as a pass leaves them: gate-up with norm and SwiGLU 5000 rows, 2 rounds against 3, 43.0 / 33.2; 8192 rows, 2
-// against 4, 43.1 / 46.9; 10 000 rows, 3 against 5, 66.1 / 58.6; 18 432 rows, 4 against 8, 90.3 / 97.2; 20 000 rows, 5 against 8, 110.9 /
-// 105.6.  640 columns, K 1664: 18 432 rows, 1 against 2, 45.0 / 46.1 (50.8 / 62.9 with activations from memory); 24 576 rows, 2 against 2,
-// 81.7 / 53.3; 40 000 rows, 2 against 4, 88.7 / 95.3.  With a short K a last round of 128 x 128 tiles that fills a quarter of the device or
-// less takes half a round (K 512: 16 384 rows 22.9 / 20.4, 18 432 rows, 0.4 of a round, 22.8 / 24.1).
+// the last-level cache as a pass leaves them: gate-up with norm and SwiGLU 5000 rows, 2 rounds against 3, 41.0 / 31.1; 8192 rows, 2
+// against 4, 42.0 / 41.5; 10 000 rows, 3 against 5, 62.6 / 51.4; 18 432 rows, 4 against 8, 88.6 / 96.0; 20 000 rows, 5 against 8, 100.3 /
+// 104.9; 33 216 rows, 7 against 14, 150 / 171.  640 columns, K 1664: 18 432 rows, 1 against 2, 51.2 / 59.4; 24 576 rows, 2 against 2, 97.1 /
+// 66.4; 40 000 rows, 2 against 4, 103 / 112.  With a short K a last round of 128 x 128 tiles that fills a quarter of the device or
+// less takes half a round (K 512: 16 384 rows 21.9 / 20.4, 18 432 rows, 0.4 of a round, 23.4 / 26.0).
 static bool big_tiles_pay(const uvmi_gemm_args* a, int64_t t128, int64_t t256, int cus) {
   const int64_t r256 = (t256 + cus - 1) / cus, slots = 2 * (int64_t)cus, rest = t128 % slots;
   const int64_t halves128 = 2 * (t128 / slots) + (rest == 0 ? 0 : (a->K <= 768 && 4 * rest <= slots ? 1 : 2));
@@ -81,14 +81,14 @@ extern "C" int uvmi_gemm_tn_ex(const uvmi_gemm_args* a, void* stream) {
     // (a product of fewer rows whose many 256-wide tiles would be more than a tenth emptier than 128-wide ones takes those)
     const int64_t pad128 = ((int64_t)a->N + 127) / 128 * 128, pad256 = ((int64_t)a->N + 255) / 256 * 256;
     const bool small = rows_ok ? !big_tiles_pay(a, t128, t256, cus) : pad128 * 10 < pad256 * 9;
-    gemm_big_launch(a, a->config == 0 && small ? 128 : 256, (hipStream_t)stream);
+    gemm_big_launch(a, a->config == 0 && small ? 128 : 256, cus, (hipStream_t)stream);
     UVMI_CHECK_LAUNCH("uvmi_gemm_tn(direct to LDS)");
     return UVMI_OK;
   }
   if (a->config == 6 || a->epilogue == UVMI_GEMM_SOFTCAP) {
     UVMI_REQUIRE(big_ok(a), UVMI_EUNSUPPORTED,
                  "uvmi_gemm_tn: config %d (tiles loaded straight into LDS) needs K >= 128, C (and the residual) 16-byte aligned, ldc (ldr) %% 8 == 0", a->config);
-    gemm_big_launch(a, 128, (hipStream_t)stream);
+    gemm_big_launch(a, 128, cus, (hipStream_t)stream);
     UVMI_CHECK_LAUNCH("uvmi_gemm_tn(128 x 128, direct)");
     return UVMI_OK;
   }
@@ -102,7 +102,7 @@ extern "C" int uvmi_gemm_tn_ex(const uvmi_gemm_args* a, void* stream) {
     gemm_stream_launch(a, form, cus, (hipStream_t)stream);
     UVMI_CHECK_LAUNCH("uvmi_gemm_tn(streaming)");
   } else if (a->config == 0 && big_ok(a)) {
-    gemm_big_launch(a, 128, (hipStream_t)stream);
+    gemm_big_launch(a, 128, cus, (hipStream_t)stream);
     UVMI_CHECK_LAUNCH("uvmi_gemm_tn(128 x 128, direct)");
   } else {
     gemm_tile_launch(a, (hipStream_t)stream);

@@ -27,11 +27,16 @@
 //   * the residual of the whole tile is requested at once behind the main loop, ahead of the first store (in place it may not be
 //     moved across one by the compiler, and was requested row block by row block: 18 432 x 640 x 512 27.9 -> 23.8 us, x 1664 53.8 ->
 //     50.8; 33 216 rows in 128 x 128 tiles 47.7 -> 45.3, 98.4 -> 96.7);
-//   * the pre-norm's sums of squares go between the matrix instructions (gate-up at 33 216 rows 170 -> 160 us, at 18 432 105 -> 98;
-//     without the norm 148 and 87);
+//   * a pass of more tiles than run at a time (K a multiple of 128) has a workgroup take several: the next tile's first two slabs are
+//     requested in a tile's last two iterations, so they land under its epilogue (33 216-row gate-up 165 -> 160 us, without the norm 150 ->
+//     142; 128 x 128 tiles 174 -> 161; 640 columns, K 1664, 97 -> 94).  Per-tile constants of the lane are computed anew between
+//     tiles: there is no register for them in the main loop, and a spilled one is reloaded behind the loads in flight;
+//   * the pre-norm's sums of squares are matrix instructions too, one for 16 rows and 32 columns, a sixteenth of the product's
+//     (gate-up at 33 216 rows 160 -> 154 us, at 18 432 rows 96 -> 90; as vector instructions between the matrix ones they cost 12 % of
+//     a launch, in 128 x 128 tiles 14 %: 177 -> 169).  The results' distance from 64 bits is the same to seven digits, K 512 .. 2560;
 //   * no loads are made past the last slab (they were, to keep the loop free of branches: the epilogue then waited for them;
 //     1 - 3 % of a launch);
-//   * tiles are dealt to the XCDs in contiguous runs, as in the tiled kernel.
+//   * tiles are dealt to the XCDs in contiguous runs, as in the tiled kernel; a workgroup's tiles are a stride apart in its XCD's run.
 // One workgroup per compute unit (128 KB of LDS, 2 waves per SIMD).  K >= 128; C and the residual 16-byte aligned with
 // pitches that are multiples of 8 elements (the caller checks).
 #include "common.h"
@@ -74,13 +79,21 @@ __device__ __forceinline__ void xpose2(uint32_t& x0, uint32_t& x1) {
   x0 = t[0]; x1 = t[1];
 }
 
+// The lane, computed anew: what is derived from it does not stay in registers across a tile's main loop, which has none to spare.
+__device__ __forceinline__ int fresh_lane() {
+  int l;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+  return l;
+}
+
 // EPI 0: C = A W^T (M, N).  EPI 1: W rows are [gate 16 | up 16] slabs; C = silu(gate) * up, (M, N / 2).
 // EPI 2: C = ca * R + cb * (A W^T).  EPI 3: C fp32 = ca * sigmoid((x + cb) / cap_c) of the rounded product x.  NORM: A stands
 // for its RMS-normalised rows.
 // FI: 16-row fragments per wave along M: 8 - the 256 x 256 tile on 8 waves (2 x 4); 4 - a 128 x 128 tile on 4 waves (2 x 2,
 // 64 x 64 per wave, two workgroups per compute unit) for passes whose 256 x 256 tiles would not fill the device.  (A
 // 64 x 64 tile on 2 waves was measured too: no faster at 2 k rows than 64 x 64 tiles staged through registers.)
-template <int DT, int EPI, bool NORM, int FI>
+// MANY: a workgroup takes several tiles (an even number of slabs: a tile ends on the stage that it does not begin on).
+template <int DT, int EPI, bool NORM, int FI, bool MANY>
 __global__ __launch_bounds__(64 * FI) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_big_kernel(BigParams P) {
   constexpr int WN = FI / 2;                   // waves along N (2 along M)
@@ -91,31 +104,39 @@ void gemm_big_kernel(BigParams P) {
   __shared__ __attribute__((aligned(1024))) unsigned char sA1[BM * 128];
   __shared__ __attribute__((aligned(1024))) unsigned char sB0[BN * 128];
   __shared__ __attribute__((aligned(1024))) unsigned char sB1[BN * 128];
+  __shared__ float sRS[NORM ? BM : 1];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int T = P.tiles_m * P.tiles_n;
   const int per = (T + 7) / 8;
-  const int L = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
-  if (L >= T) return;
-  const int bn = P.rowsplit ? L % P.tiles_n : L / P.tiles_m, bm = P.rowsplit ? L / P.tiles_n : L % P.tiles_m;
-  const int m0 = bm * BM, n0 = bn * BN;
+  // the workgroup's tiles: every gridDim.x / 8 th of its XCD's run
+  const int step = (int)(gridDim.x / 8), last = min((int)(blockIdx.x % 8 + 1) * per, T);
+  int L = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+  if (L >= last) return;
   const int nk = P.K / 64;
+  int m0, n0;
+  auto tile_at = [&](int l) {
+    const int bn = P.rowsplit ? l % P.tiles_n : l / P.tiles_m, bm = P.rowsplit ? l / P.tiles_n : l % P.tiles_m;
+    m0 = bm * BM;
+    n0 = bn * BN;
+  };
+  tile_at(L);
 
   // ---- loader: wave w fills blocks 4 w .. 4 w + 3 (8 rows each) of A and of W (BM = BN = 32 x the number of waves).  Rows
   // past M / N repeat the last row: what they produce is never stored.
   uint32_t offA[4], offB[4];
+  auto offsets = [&]() {
+    const int ln = fresh_lane();
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int rl = 8 * (4 * wave + i) + (lane >> 3);   // row inside the tile
-    const int ch = (lane & 7) ^ ((rl >> 1) & 7);
-    int row = m0 + rl;
-    row = row < P.M ? row : P.M - 1;
-    offA[i] = (uint32_t)row * P.lda2 + 16 * ch;
-    row = n0 + rl;
-    row = row < P.N ? row : P.N - 1;
-    offB[i] = (uint32_t)row * P.ldw2 + 16 * ch;
-  }
+    for (int i = 0; i < 4; i++) {
+      const int rl = 8 * (4 * wave + i) + (ln >> 3);   // row inside the tile
+      const int ch = (ln & 7) ^ ((rl >> 1) & 7);
+      offA[i] = (uint32_t)min(m0 + rl, P.M - 1) * P.lda2 + 16 * ch;
+      offB[i] = (uint32_t)min(n0 + rl, P.N - 1) * P.ldw2 + 16 * ch;
+    }
+  };
+  offsets();
   // (buffer loads: 32-bit offsets and the slab as a scalar, where global ones keep eight 64-bit addresses)
   const __amdgpu_buffer_rsrc_t rA = __builtin_amdgcn_make_buffer_rsrc((void*)P.a, 0, (int)((uint32_t)(P.M - 1) * P.lda2 + (uint32_t)P.K * 2), 0x00020000);
   const __amdgpu_buffer_rsrc_t rW = __builtin_amdgcn_make_buffer_rsrc((void*)P.w, 0, (int)((uint32_t)(P.N - 1) * P.ldw2 + (uint32_t)P.K * 2), 0x00020000);
@@ -131,24 +152,19 @@ void gemm_big_kernel(BigParams P) {
   // ---- reader: wave (wm, wn) owns rows 16 FI wm .., columns 64 wn ..; lane (r, g) reads chunk (4 s + g) ^ ((r / 2) % 8) of
   // row r of a 16-row fragment for K-step s
   const int wm = wave / WN, wn = wave % WN;
-  const int r = lane & 15, g = lane >> 4;
   // The wave's pairs of row fragments are walked from pair wn on (NORM; accumulator rows 2 p, 2 p + 1 belong to pair (p + wn) mod
   // FI / 2), so that the rows whose squares a wave sums are the same in the code of every wave.
   constexpr int NP = FI / 2;
   uint32_t a_off[2], b_off[2], pair_at[NP];
 #pragma unroll
   for (int s = 0; s < 2; s++) {
-    const uint32_t lo = (uint32_t)r * 128 + (uint32_t)((((4 * s + g) ^ ((r >> 1) & 7))) << 4);
+    const uint32_t lo = (uint32_t)(lane & 15) * 128 + (uint32_t)((((4 * s + (lane >> 4)) ^ ((lane >> 1) & 7))) << 4);
     a_off[s] = (uint32_t)wm * (16 * FI * 128) + lo;
     b_off[s] = (uint32_t)wn * 8192 + lo;
   }
 #pragma unroll
   for (int p = 0; p < NP; p++) pair_at[p] = (uint32_t)(NORM ? ((p + wn) & (NP - 1)) : p) * 4096;
   gf4 acc[FI][4];
-#pragma unroll
-  for (int i = 0; i < FI; i++)
-#pragma unroll
-    for (int j = 0; j < 4; j++) acc[i][j] = gf4{0.f, 0.f, 0.f, 0.f};
 
   gu4 w0[4], w1[4], f0[2], f1[2], f2[2];
   auto read_b = [&](const unsigned char* sb, int s, gu4* w) {
@@ -170,37 +186,44 @@ void gemm_big_kernel(BigParams P) {
 #pragma unroll
     for (int j = 0; j < 4; j++) acc[i + 1][j] = gmfma<DT>(w[j], f[1], acc[i + 1][j]);
   };
-  // NORM: the squares of the rows are summed from the operand fragments as they pass: wave (wm, wn) takes row pair wn of
-  // each K-step (rows 16 FI wm + 32 wn + 16 u + r, u = 0, 1; lane (r, g) sees 8 of a row's 32 values), which is its first pair.  The
-  // sums' instructions go between the group's matrix instructions, a few behind each: behind all of them they left the matrix
-  // pipe idle (and a branch on wn around them kept them there).
-  float ss[2] = {0.f, 0.f};
+  // NORM: the squares of a row are the diagonal of X X^T: one more matrix instruction on an operand fragment with itself per 16 rows and
+  // K-step.  Wave (wm, wn) takes row pair wn (rows 16 FI wm + 32 wn + 16 u + r, u = 0, 1),
+  // which is its first pair (as a branch on wn it costs 4 us of 157).
+  gf4 sq[2];
   auto sumsq = [&](int pair, const gu4* f) {
     if (NORM && pair == 0) {
 #pragma unroll
-      for (int e = 0; e < 4; e++)
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-          float lo, hi;
-          gunpack<DT>(f[u][e], lo, hi);
-          ss[u] = fmaf(lo, lo, ss[u]);
-          ss[u] = fmaf(hi, hi, ss[u]);
-        }
-      asm volatile("" : "+v"(ss[0]), "+v"(ss[1]));   // (here, not where the loop ends)
-#pragma unroll
-      for (int q = 0; q < 7; q++) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // a matrix instruction,
-        __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);   // five vector ones
-      }
+      for (int u = 0; u < 2; u++) sq[u] = gmfma<DT>(f[u], f[u], sq[u]);
     }
   };
-  auto frow = [&](int i) { return 16 * FI * wm + 16 * (NORM ? ((i + 2 * wn) & (FI - 1)) : i) + r; };   // tile row of accumulator row fragment i
+  auto frow = [&](int i) { return 16 * FI * wm + 16 * (NORM ? ((i + 2 * wn) & (FI - 1)) : i); };   // first tile row of accumulator row fragment i
 #define UVMI_SB() __builtin_amdgcn_sched_barrier(0)
 
+  auto clear = [&]() {
+#pragma unroll
+    for (int i = 0; i < FI; i++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) acc[i][j] = gf4{0.f, 0.f, 0.f, 0.f};
+    sq[0] = sq[1] = gf4{0.f, 0.f, 0.f, 0.f};
+  };
   issue(sA0, sB0, 0);
+  clear();
+#pragma unroll
+  for (int i = 0; i < FI; i++) asm volatile("" : "+v"(acc[i][0]), "+v"(acc[i][1]), "+v"(acc[i][2]), "+v"(acc[i][3]));   // (while the loads are on their way)
   __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
   asm volatile("s_barrier" ::: "memory");
   issue(sA1, sB1, 1);
+  for (;;) {   // tiles
+  const int cm0 = m0, cn0 = n0;
+  const bool more = MANY && L + step < last;
+  // slab k of this tile or, past its last one, slab k - nk of the next
+  auto request = [&](unsigned char* sa, unsigned char* sb, int k) {
+    if (k < nk) issue(sa, sb, k);
+    else if (more) {
+      if (k == nk) { tile_at(L + step); offsets(); }
+      issue(sa, sb, k - nk);
+    }
+  };
   read_b(sB0, 0, w0);
   read_a(sA0, 0, 0, f0);
   // Iteration k multiplies slab k out of stage S: 8 groups of 8 MFMAs (K-step s, row pair p); the operands of a group are
@@ -219,7 +242,7 @@ void gemm_big_kernel(BigParams P) {
     mm1(4, f0, w1); UVMI_SB(); read_a(SA, 1, 6, f1); UVMI_SB(); mm7(4, f0, w1); sumsq(2, f0); UVMI_SB();                 \
     __builtin_amdgcn_s_waitcnt(0x0f70);                                                                                  \
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");                                                      \
-    if ((k) + 2 < nk) issue(SA, SB_, (k) + 2);                                                                           \
+    request(SA, SB_, (k) + 2);                                                                                           \
     read_b(SBN, 0, w0); read_a(SAN, 0, 0, f0); UVMI_SB();                                                                \
     mm1(6, f1, w1); mm7(6, f1, w1); sumsq(3, f1); UVMI_SB();                                                             \
   } while (0)
@@ -232,7 +255,7 @@ void gemm_big_kernel(BigParams P) {
     mm1(0, f2, w1); UVMI_SB(); read_a(SA, 1, 2, X); UVMI_SB(); mm7(0, f2, w1); sumsq(0, f2); UVMI_SB();                  \
     __builtin_amdgcn_s_waitcnt(0x0f70);                                                                                  \
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");                                                      \
-    if ((k) + 2 < nk) issue(SA, SB_, (k) + 2);                                                                           \
+    request(SA, SB_, (k) + 2);                                                                                           \
     read_b(SBN, 0, w0); read_a(SAN, 0, 0, Y); UVMI_SB();                                                                 \
     mm1(2, X, w1); mm7(2, X, w1); sumsq(1, X); UVMI_SB();                                                                \
   } while (0)
@@ -242,44 +265,43 @@ void gemm_big_kernel(BigParams P) {
       UVMI_ITER(sA0, sB0, sA1, sB1, k);
       UVMI_ITER(sA1, sB1, sA0, sB0, k + 1);
     }
-    if (k < nk) UVMI_ITER(sA0, sB0, sA1, sB1, k);
+    if (!MANY && k < nk) UVMI_ITER(sA0, sB0, sA1, sB1, k);
   } else {
     for (; k + 2 <= nk; k += 2) {
       UVMI_ITER4(sA0, sB0, sA1, sB1, k, f0, f1);
       UVMI_ITER4(sA1, sB1, sA0, sB0, k + 1, f1, f0);
     }
-    if (k < nk) UVMI_ITER4(sA0, sB0, sA1, sB1, k, f0, f1);
+    if (!MANY && k < nk) UVMI_ITER4(sA0, sB0, sA1, sB1, k, f0, f1);
   }
 #undef UVMI_ITER4
 #undef UVMI_ITER
 #undef UVMI_SB
 
+  const int el = fresh_lane(), r = el & 15, g = el >> 4;
   // ---- row scales of the pre-norm: the 4 lane groups of a row add their sums; LDS carries the scales to every wave
   float rn[FI];
 #pragma unroll
   for (int i = 0; i < FI; i++) rn[i] = 1.0f;
   if (NORM) {
-    float* sRS = (float*)sA0;
-    __syncthreads();   // every wave's loads have landed and its operand reads are done
+    int kd = P.K;
+    asm volatile("" : "+s"(kd));   // (not a register of its own through the main loop)
 #pragma unroll
-    for (int u = 0; u < 2; u++) {
-      float v = ss[u];
-      v += lane_xor16(v);
-      v = xsum32(v);
-      if (g == 0) sRS[16 * FI * wm + 32 * wn + 16 * u + r] = rsqrtf(v / (float)P.K + P.eps);
+    for (int u = 0; u < 2; u++) {   // (lane (r, g) holds elements (4 g + t, r) of X X^T)
+      const float v = r & 2 ? (r & 1 ? sq[u][3] : sq[u][2]) : (r & 1 ? sq[u][1] : sq[u][0]);
+      if (g == r >> 2) sRS[16 * FI * wm + 32 * wn + 16 * u + r] = rsqrtf(v / (float)kd + P.eps);
     }
-    __syncthreads();
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
-    for (int i = 0; i < FI; i++) rn[i] = sRS[frow(i)];
+    for (int i = 0; i < FI; i++) rn[i] = sRS[frow(i) + r];
   }
 
   // ---- epilogue: accumulator (i, j): lane (r, g) holds C[m0 + 16 FI wm + 16 i + r][n0 + 64 wn + 16 j + 4 g + t], t = 0..3
   uint4 res[EPI == 2 ? FI : 1][2];
   if constexpr (EPI == 2) {
-    const int n = n0 + 64 * wn + 16 * g;
+    const int n = cn0 + 64 * wn + 16 * g;
 #pragma unroll
     for (int i = 0; i < FI; i++) {
-      const int row = m0 + frow(i);
+      const int row = cm0 + frow(i) + r;
       res[i][0] = res[i][1] = uint4{0u, 0u, 0u, 0u};
       if (row < P.M && n < P.N) {
         const uint16_t* rp = (const uint16_t*)P.r + (int64_t)row * P.ldr + n;
@@ -290,7 +312,7 @@ void gemm_big_kernel(BigParams P) {
   }
 #pragma unroll
   for (int i = 0; i < FI; i++) {
-    const int row = m0 + frow(i);
+    const int row = cm0 + frow(i) + r;
     if (EPI == 1) {
       // gate slab j, up slab j + 1 -> 4 outputs per slab pair; after the 2 x 2 transpose lane (r, g) holds the 8 consecutive
       // output columns 16 (g % 2) + 8 (g / 2) .. of the wave's 32
@@ -303,7 +325,7 @@ void gemm_big_kernel(BigParams P) {
       }
       xpose2(x0[0], x1[0]);
       xpose2(x0[1], x1[1]);
-      const int n = (n0 >> 1) + 32 * wn + 16 * (g & 1) + 8 * (g >> 1);   // output column
+      const int n = (cn0 >> 1) + 32 * wn + 16 * (g & 1) + 8 * (g >> 1);   // output column
       if (row < P.M && 2 * n < P.N) {
         uint16_t* cp = (uint16_t*)P.c + (int64_t)row * P.ldc + n;
         *(uint4*)cp = uint4{x0[0], x0[1], x1[0], x1[1]};
@@ -315,7 +337,7 @@ void gemm_big_kernel(BigParams P) {
       auto cap = [&](float x) { return P.ca * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f((ground<DT>(x * rn[i]) + P.cb) * k2)); };
 #pragma unroll
       for (int j = 0; j < 4; j++) {
-        const int n = n0 + 64 * wn + 16 * j + 4 * g;
+        const int n = cn0 + 64 * wn + 16 * j + 4 * g;
         if (row < P.M && n < P.N)
           *(float4*)((float*)P.c + (int64_t)row * P.ldc + n) = float4{cap(acc[i][j][0]), cap(acc[i][j][1]), cap(acc[i][j][2]), cap(acc[i][j][3])};
       }
@@ -333,7 +355,7 @@ void gemm_big_kernel(BigParams P) {
         }
         xpose_pair(x[0][0], x[1][0]);
         xpose_pair(x[0][1], x[1][1]);
-        const int n = n0 + 64 * wn + 32 * s + 8 * g;
+        const int n = cn0 + 64 * wn + 32 * s + 8 * g;
         if (row < P.M && n < P.N) *(uint4*)((uint16_t*)P.c + (int64_t)row * P.ldc + n) = uint4{x[0][0], x[0][1], x[1][0], x[1][1]};
       }
     } else {
@@ -348,7 +370,7 @@ void gemm_big_kernel(BigParams P) {
       xpose4(lo);
       xpose4(hi);
       // lane (r, g) now holds columns 16 g .. 16 g + 15 of the wave's 64: words lo[0] hi[0] lo[1] hi[1] ...
-      const int n = n0 + 64 * wn + 16 * g;
+      const int n = cn0 + 64 * wn + 16 * g;
       if (row < P.M && n < P.N) {
         uint32_t wds[8] = {lo[0], hi[0], lo[1], hi[1], lo[2], hi[2], lo[3], hi[3]};
         const uint4 q0 = res[i][0], q1 = res[i][1];
@@ -366,13 +388,24 @@ void gemm_big_kernel(BigParams P) {
       }
     }
   }
+  if (!more) break;
+  L += step;
+  clear();
+  }
 }
 
 template <int DT, int FI>
-static void launch_big(const uvmi_gemm_args* a, const BigParams& P, hipStream_t st) {
+static void launch_big(const uvmi_gemm_args* a, const BigParams& P, int cus, hipStream_t st) {
   const int T = P.tiles_m * P.tiles_n;
-  const dim3 grid((unsigned)(((T + 7) / 8) * 8)), blk(64 * FI);
-#define UVMI_GO(EPI, NORM) hipLaunchKernelGGL((gemm_big_kernel<DT, EPI, NORM, FI>), grid, blk, 0, st, P)
+  const int slots = (FI == 8 ? cus : 2 * cus) / 8 * 8;   // workgroups that run at a time
+  // (a launch of one round keeps the shorter code: it lost 0.5 us of 9 to the other's)
+  const bool many = P.K % 128 == 0 && slots > 0 && T > slots;
+  const dim3 grid((unsigned)(many ? slots : ((T + 7) / 8) * 8)), blk(64 * FI);
+#define UVMI_GO(EPI, NORM)                                                                              \
+  do {                                                                                                  \
+    if (many) hipLaunchKernelGGL((gemm_big_kernel<DT, EPI, NORM, FI, true>), grid, blk, 0, st, P);      \
+    else hipLaunchKernelGGL((gemm_big_kernel<DT, EPI, NORM, FI, false>), grid, blk, 0, st, P);          \
+  } while (0)
   const bool norm = a->norm_a != 0;
   if (a->epilogue == UVMI_GEMM_RESID) { if (norm) UVMI_GO(2, true); else UVMI_GO(2, false); }
   else if (a->epilogue == UVMI_GEMM_SWIGLU) { if (norm) UVMI_GO(1, true); else UVMI_GO(1, false); }
@@ -382,7 +415,7 @@ static void launch_big(const uvmi_gemm_args* a, const BigParams& P, hipStream_t 
 }
 
 // Arguments are validated by the caller (uvmi_gemm_tn_ex), which also checks K >= 128.  tile: 256 or 128.
-void gemm_big_launch(const uvmi_gemm_args* a, int tile, hipStream_t st) {
+void gemm_big_launch(const uvmi_gemm_args* a, int tile, int cus, hipStream_t st) {
   BigParams P;
   P.a = a->a; P.w = a->w; P.c = a->c; P.r = a->resid;
   P.lda2 = (uint32_t)a->lda * 2; P.ldw2 = (uint32_t)a->ldw * 2; P.ldc = a->ldc; P.ldr = a->ldr;
@@ -392,8 +425,8 @@ void gemm_big_launch(const uvmi_gemm_args* a, int tile, hipStream_t st) {
   P.eps = a->eps; P.ca = a->ca; P.cb = a->cb; P.cap_c = a->cap_c;
   const double bytes_a = (double)a->M * a->K, bytes_w = (double)a->N * a->K;
   P.rowsplit = bytes_a / 8 + bytes_w < bytes_a + bytes_w / 8;
-  if (a->dtype == UVMI_F16) { if (tile == 256) launch_big<UVMI_F16, 8>(a, P, st); else launch_big<UVMI_F16, 4>(a, P, st); }
-  else { if (tile == 256) launch_big<UVMI_BF16, 8>(a, P, st); else launch_big<UVMI_BF16, 4>(a, P, st); }
+  if (a->dtype == UVMI_F16) { if (tile == 256) launch_big<UVMI_F16, 8>(a, P, cus, st); else launch_big<UVMI_F16, 4>(a, P, cus, st); }
+  else { if (tile == 256) launch_big<UVMI_BF16, 8>(a, P, cus, st); else launch_big<UVMI_BF16, 4>(a, P, cus, st); }
 }
 
 }  // namespace uvmi

@@ -17,16 +17,17 @@
 //   * the MFMA's A input is the weight fragment and its B input the activation fragment, so an accumulator holds C^T: a lane
 //     has 4 consecutive columns of one row and stores them as one 8-byte write;
 //   * the partial sums meet in LDS (the slabs' space) behind the kernel's only barrier; a wave adds and finishes its share of the
-//     fragments.  The residual of that share is requested before anything else, the squares of NORM are summed from the
-//     operand fragments as they pass;
+//     fragments.  The residual of that share is requested before anything else; the squares of NORM are the diagonal of an
+//     activation fragment's product with itself, one more matrix instruction for it (32 vector ones before: twice the time of the 64 x
+//     64 tile's own products);
 //   * rows past M or N are clamped to the last one (computed, not stored);
 //   * individual scalar arguments rather than a parameter block: they arrive in SGPRs with the wave.
 // us per launch in a stream of launches with 20 layers' weights in turn (N x K: 656 x 640 with NORM | 640 x 512 RESID | 3328 x 640
 // NORM, SWIGLU | 640 x 1664 RESID), and in brackets what the forms took that it replaced (a whole weight strip parked in LDS
 // behind a barrier below 448 rows, 64 x 64 tiles through registers from there on):
-//      1 row   2.7 [3.9] | 2.5 [3.8] | 3.4 [4.7] | 2.9 [4.3]        64 rows   2.8 [4.4] | 2.5 [4.3] | 3.9 [6.0] | 3.2 [5.3]
-//    256 rows  3.6 [5.6] | 3.0 [5.4] | 5.8 [6.5] | 4.6 [9.2]       512 rows   4.4 [6.2] | 3.7 [5.2] | 8.1 [8.7] | 5.9 [8.9]
-//   2048 rows  7.9 [8.4] | 6.7 [7.4] |     -     | 12.1 [13.7]
+//      1 row   2.7 [3.9] | 2.5 [3.8] | 3.4 [4.7] | 2.9 [4.3]        64 rows   2.8 [4.4] | 2.5 [4.3] | 3.7 [6.0] | 3.2 [5.3]
+//    256 rows  3.5 [5.6] | 3.0 [5.4] | 5.4 [6.5] | 4.6 [9.2]       512 rows   4.1 [6.2] | 3.7 [5.2] | 7.6 [8.7] | 5.9 [8.9]
+//   2048 rows  7.4 [8.4] | 6.7 [7.4] |     -     | 12.1 [13.7]
 #include "common.h"
 #include "gemm_util.h"
 
@@ -42,20 +43,6 @@ struct StreamParams {
 
 #define UVMI_GLBP(p) ((const __attribute__((address_space(1))) void*)(p))
 #define UVMI_LDSP(p) ((__attribute__((address_space(3))) void*)(p))
-
-// s + the squares of the 8 values of an operand word
-template <int DT>
-__device__ __forceinline__ float sumsq8(gu4 v, float s) {
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    float lo, hi;
-    if (DT == UVMI_BF16) { lo = __uint_as_float(v[i] << 16); hi = __uint_as_float(v[i] & 0xffff0000u); }
-    else { lo = half_bits_to_float((uint16_t)(v[i] & 0xffff)); hi = half_bits_to_float((uint16_t)(v[i] >> 16)); }
-    s = fmaf(lo, lo, s);
-    s = fmaf(hi, hi, s);
-  }
-  return s;
-}
 
 template <int N> __device__ __forceinline__ void wait_vm() {   // all but the newest N loads have landed
   static_assert(N >= 0 && N < 64, "vmcnt has six bits");
@@ -128,10 +115,10 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(const void* a_a, c
   if (R > 1 && nw > 1) issue(s1, 1);
 
   gf4 acc[FM][FN];
-  float ss[FM];
+  gf4 sq[FM];   // NORM: the squares of a row are the diagonal of X X^T, one more matrix instruction per fragment
 #pragma unroll
   for (int i = 0; i < FM; i++) {
-    ss[i] = 0.f;
+    sq[i] = gf4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < FN; j++) acc[i][j] = gf4{0.f, 0.f, 0.f, 0.f};
   }
@@ -159,7 +146,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(const void* a_a, c
       for (int f = 0; f < FM; f++) {
 #pragma unroll
         for (int j = 0; j < FN; j++) acc[f][j] = gmfma<DT>(wf[s][j], af[s][f], acc[f][j]);
-        if (NORM) ss[f] = sumsq8<DT>(af[s][f], ss[f]);
+        if (NORM) sq[f] = gmfma<DT>(af[s][f], af[s][f], sq[f]);
       }
     }
   };
@@ -174,11 +161,9 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(const void* a_a, c
   // ---- the waves' partial sums meet in LDS
   if (NORM) {
 #pragma unroll
-    for (int f = 0; f < FM; f++) {
-      float v = ss[f];
-      v += __shfl_xor(v, 16, 64);
-      v += __shfl_xor(v, 32, 64);
-      if (g == 0) sSS[wave * BM + 16 * f + r] = v;
+    for (int f = 0; f < FM; f++) {   // (lane (r, g) holds elements (4 g + t, r) of X X^T)
+      const float v = r & 2 ? (r & 1 ? sq[f][3] : sq[f][2]) : (r & 1 ? sq[f][1] : sq[f][0]);
+      if (g == r >> 2) sSS[wave * BM + 16 * f + r] = v;
     }
   }
   auto part = [&](int w, int f) { return (gf4*)(s0 + w * (ROWS * 128) + 1024 * f) + lane; };   // fragment f of wave w's sums
