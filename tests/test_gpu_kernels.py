@@ -929,6 +929,61 @@ def test_qkv_post_engine_shape_kernel_equals_the_general_kernel(dtype, rope, rin
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n", [6144, 6145, 6151])
+@pytest.mark.parametrize("cache,rope,ring,has_ve,gate", [("int8", 1, 1, 1, 1), ("int8", 0, 0, 0, 0), ("16 bit", 1, 1, 0, 1), ("none", 1, 0, 1, 1), ("int8, odd pitch", 1, 0, 1, 1)])
+def test_qkv_post_of_many_rows_equals_that_of_few(dtype, n, cache, rope, ring, has_ve, gate):
+    """From 6144 rows on a wave takes 8 rows and wide accesses: bit for bit what calls of 1000 rows each write, on rows past the
+    rotation table, without a cache row, with the last wave partly empty; a cache whose rows are not 8-byte aligned keeps the other kernel."""
+    import ctypes as C
+    from ultraviolet_amd import _lib as L
+    from ultraviolet_amd.kernels.decode_attn import rope_table
+    g = torch.Generator(device="cuda").manual_seed(n + rope + 2 * ring + 4 * has_ve)
+    H, S, vocab, ld = 8, 64, 500, 656
+    B = n // 32 + 1
+    qkv = (torch.randn(n, ld, device="cuda", generator=g) * 1.5).to(dtype)
+    at = torch.arange(n, device="cuda")
+    pos, rows = at % 32 + (at // 32) % 3 * 32, at // 32                       # positions 80 .. 95 lie past the table; no two rows share a slot
+    rows[::7] = -1
+    last = pos + torch.randint(0, 100, (n,), device="cuda", generator=g)
+    tok = torch.randint(-3, vocab + 3, (n,), device="cuda", generator=g)
+    ve = torch.randn(vocab, 64, device="cuda", generator=g).to(dtype)
+    inv_freq = (1.0 / (1024.0 ** (torch.arange(16, device="cuda").float() / 16))).contiguous()
+    tab = rope_table(inv_freq, 80, dtype)
+    outs = []
+    for step in (n, 1000):
+        q, k, v = torch.zeros(n, H, 64, device="cuda", dtype=dtype), *(torch.zeros(n, 64, device="cuda", dtype=dtype) for _ in range(2))
+        vhat, gt = torch.zeros(n, 64, device="cuda"), torch.zeros(n, H, device="cuda")
+        kc, vc = (torch.zeros(B, 1, S, 65 if "odd" in cache else 64, device="cuda", dtype=torch.int8 if "int8" in cache else dtype) for _ in range(2))
+        ks, vs = (torch.zeros(B, 1, S, device="cuda", dtype=torch.float16) for _ in range(2))
+        for lo in range(0, n, step):
+            a = L.QkvPostArgs()
+            a.qkv, a.dtype, a.qkv_ld, a.ext_logits = qkv[lo:].data_ptr(), L.dtype_code(dtype), ld, 1
+            a.pos, a.rows, a.last_pos, a.inv_freq = pos[lo:].data_ptr(), rows[lo:].data_ptr(), last[lo:].data_ptr() if ring else None, inv_freq.data_ptr()
+            if has_ve:
+                a.ve_table, a.tok = ve.data_ptr(), tok[lo:].data_ptr()
+            a.q_out, a.q_dtype, a.k_out, a.v_out = q[lo:].data_ptr(), L.dtype_code(dtype), k[lo:].data_ptr(), v[lo:].data_ptr()
+            if cache != "none":
+                a.k_cache, a.v_cache = kc.data_ptr(), vc.data_ptr()
+                if "int8" in cache:
+                    a.k_scale, a.v_scale = ks.data_ptr(), vs.data_ptr()
+            a.scb, a.sch, a.scs, a.ssb, a.ssh, a.S = kc.stride(0), kc.stride(1), kc.stride(2), ks.stride(0), ks.stride(1), S
+            a.n, a.vocab, a.H, a.KH, a.hd, a.d, a.n_pairs = min(step, n - lo), vocab, H, 1, 64, 640, 16
+            a.ring, a.has_ve, a.rope, a.eps, a.xsa_eps = ring, has_ve, rope, 1e-6, 1e-4
+            if rope:
+                a.rope_table, a.rope_positions = tab.data_ptr(), tab.size(0)
+            a.vhat_out = vhat[lo:].data_ptr()
+            if gate:
+                a.gate_out = gt[lo:].data_ptr()
+            L.check(L.lib().uvmi_qkv_post(C.byref(a), L.stream_ptr(qkv)), "uvmi_qkv_post")
+        torch.cuda.synchronize()
+        outs.append((q, k, v, vhat, gt, kc, vc, ks, vs))
+    for nm, x, y in zip(("q", "k", "v", "v_hat", "gate", "k cache", "v cache", "k scale", "v scale"), *outs):
+        assert torch.equal(x, y), nm
+    assert cache == "none" or float(outs[0][5].float().abs().sum()) > 0
+
+
+@pytest.mark.gpu
 def test_attention_probe_runs_the_engine_shape_and_refuses_the_rest():
     """uvmi_decode_attn_probe (a measurement aid: the kernel's memory stream without its arithmetic, or the reverse)
     launches for the engine's decode shape, leaves the caches untouched, returns, and refuses other shapes and modes with an

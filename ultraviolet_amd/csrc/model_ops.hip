@@ -429,6 +429,190 @@ __global__ __launch_bounds__(256) void qkv_post_fast_kernel(QkvArgs A) {
   }
 }
 
+// The same again for passes of many rows: a wave owns 8 rows, lane (i, c) dims 8 c .. 8 c + 7 of row i, for the keys and values too, and
+// walks the query heads.  What bounded the kernel above there was its vector instructions (the key and value of a row, an element per lane:
+// six-step reductions, divisions and rounding for one row at a time) and the rotation table's row read per head; here a reduction serves 8
+// rows, the table's row all heads and the key, every access is 16 bytes per lane, and all rows of a pass of 33 000 are in flight at once.
+// wave_sum's order of additions (dims d ^ 32, 16, 8, 4, 2, 1) is kept, so the three kernels agree bit for bit.  us, one row per wave -> 8:
+// 33 216 rows 34.2 -> 26.5, with a value embedding 42.6 -> 28.1; 18 432 rows 18.3 -> 16.7 and 20.4 -> 17.3 (100 MB at 33 216 rows: what bounds it
+// is memory now, behind ~4 us of latencies; with the queries before the keys the stores come in a burst, 30 us).
+__device__ __forceinline__ float row_sum(const float (&e)[8], int c) {   // of 8 lanes x 8 elements, in wave_sum's order
+  float a[4], b[2];
+#pragma unroll
+  for (int j = 0; j < 4; j++) a[j] = add_sep(c & 4 ? e[4 + j] : e[j], lane_xor4(c & 4 ? e[j] : e[4 + j]));
+#pragma unroll
+  for (int j = 0; j < 2; j++) b[j] = add_sep(c & 2 ? a[2 + j] : a[j], lane_xor2(c & 2 ? a[j] : a[2 + j]));
+  float u = add_sep(c & 1 ? b[1] : b[0], lane_xor1(c & 1 ? b[0] : b[1]));   // sum over the lanes of element c
+  u = add_sep(u, lane_xor4(u));
+  u = add_sep(u, lane_xor2(u));
+  return add_sep(u, lane_xor1(u));
+}
+template <int DT>
+__device__ __forceinline__ void unpack8(uint4 w, float (&o)[8]) {
+  const uint32_t r[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    if (DT == UVMI_BF16) { o[2 * j] = __uint_as_float(r[j] << 16); o[2 * j + 1] = __uint_as_float(r[j] & 0xffff0000u); }
+    else { o[2 * j] = half_bits_to_float(r[j] & 0xffff); o[2 * j + 1] = half_bits_to_float(r[j] >> 16); }
+  }
+}
+template <int DT>
+__global__ __launch_bounds__(64) void qkv_post_rows_kernel(QkvArgs A) {
+  const int lane = threadIdx.x & 63, c = lane & 7;
+  const int64_t r0 = (int64_t)blockIdx.x * 8, r1 = r0 + (lane >> 3);
+  if (r0 >= A.n) return;
+  const bool live = r1 < A.n;
+  const int64_t r = live ? r1 : A.n - 1;   // (a lane past the last row computes it again and stores nothing)
+  auto rnd = [](float f) { return round_t<DT>(f); };
+  const uint16_t* src = (const uint16_t*)A.qkv + r * A.ld + 8 * c;
+  // ---- requests that depend on the row index alone
+  const int64_t p = A.pos[r];
+  const int64_t row = A.rows ? A.rows[r] : r;
+  const int64_t lastp = A.last_pos ? A.last_pos[r] : 0;
+  int64_t t = A.has_ve ? A.tok[r] : 0;
+  const uint4 kw = *(const uint4*)(src + 512), vw = *(const uint4*)(src + 576);
+  const float glog = A.gate_out ? elem<DT>::ld(A.qkv, r * A.ld + 640 + c) : 0.f;   // head c
+  const float vlog = A.has_ve ? elem<DT>::ld(A.qkv, r * A.ld + 648) : 0.f;
+  uint4 qw[8];
+#pragma unroll
+  for (int h = 0; h < 8; h++) qw[h] = *(const uint4*)(src + 64 * h);
+  // ---- requests that depend on the position and the token
+  const bool in_tab = p >= 0 && p < A.rope_n;
+  float cs[8], sn[8];   // dim 8 c + j turns by frequency (8 c + j) % 16
+  if (A.rope) {
+    const float* tq = A.rope_tab + (in_tab ? p : 0) * 32 + 8 * (c & 1);
+    const float4 c0 = *(const float4*)tq, c1 = *(const float4*)(tq + 4), s0 = *(const float4*)(tq + 16), s1 = *(const float4*)(tq + 20);
+    cs[0] = c0.x; cs[1] = c0.y; cs[2] = c0.z; cs[3] = c0.w; cs[4] = c1.x; cs[5] = c1.y; cs[6] = c1.z; cs[7] = c1.w;
+    sn[0] = s0.x; sn[1] = s0.y; sn[2] = s0.z; sn[3] = s0.w; sn[4] = s1.x; sn[5] = s1.y; sn[6] = s1.z; sn[7] = s1.w;
+  }
+  if (t < 0) t = 0;
+  if (t >= A.vocab) t = A.vocab - 1;
+  uint4 ew = uint4{0u, 0u, 0u, 0u};
+  if (A.has_ve) ew = *(const uint4*)((const uint16_t*)A.ve_table + t * 64 + 8 * c);
+  if (A.rope && __any(!in_tab)) {   // a position outside the table: the angles are formed here (one at a time: there are few, and cosf is long)
+#pragma unroll 1
+    for (int j = 0; j < 8; j++) {
+      const float th = (float)p * A.inv_freq[8 * (c & 1) + j];
+      const float cj = rnd(cosf(th)), sj = rnd(sinf(th));
+#pragma unroll
+      for (int q = 0; q < 8; q++)
+        if (!in_tab && q == j) { cs[q] = cj; sn[q] = sj; }
+    }
+  }
+  if (A.rope && c < 2) {
+#pragma unroll
+    for (int j = 0; j < 8; j++) sn[j] = -sn[j];
+  }
+  auto round8 = [&](float (&x)[8]) {   // (in pairs: three instructions for two bf16 values)
+#pragma unroll
+    for (int j = 0; j < 8; j += 2) {
+      if constexpr (DT == UVMI_BF16) {
+        const uint32_t w = float2_to_bf16x2(x[j], x[j + 1]);
+        x[j] = __uint_as_float(w << 16);
+        x[j + 1] = __uint_as_float(w & 0xffff0000u);
+      } else {
+        x[j] = rnd(x[j]);
+        x[j + 1] = rnd(x[j + 1]);
+      }
+    }
+  };
+  auto rotate = [&](float (&x)[8]) {   // (rope_rot)
+    float y[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) y[j] = lane_xor2(x[j]);   // partner chunk: c <-> c ^ 2 inside the head
+    if (c < 4) {
+#pragma unroll
+      for (int j = 0; j < 8; j++) { x[j] = mul_sep(x[j], cs[j]); y[j] = mul_sep(y[j], sn[j]); }
+      round8(x);
+      round8(y);
+#pragma unroll
+      for (int j = 0; j < 8; j++) x[j] = add_sep(x[j], y[j]);
+      round8(x);
+    }
+  };
+  // ---- key and value
+  float k[8], v[8];
+  unpack8<DT>(kw, k);
+  unpack8<DT>(vw, v);
+  {
+    float e[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) e[j] = mul_sep(k[j], k[j]);
+    const float rs = rsqrtf(row_sum(e, c) * (1.0f / 64.0f) + A.eps);
+#pragma unroll
+    for (int j = 0; j < 8; j++) k[j] = k[j] * rs;
+    round8(k);
+    if (A.rope) rotate(k);
+  }
+  if (A.has_ve) {
+    const float g = rnd(2.0f * rnd(1.0f / (1.0f + __expf(-vlog))));
+    float e[8];
+    unpack8<DT>(ew, e);
+#pragma unroll
+    for (int j = 0; j < 8; j++) v[j] = ve_add(v[j], g, e[j], rnd);
+  }
+  if (live && A.k_out) st8<DT>(A.k_out, r * 64 + 8 * c, k);
+  if (live && A.v_out) st8<DT>(A.v_out, r * 64 + 8 * c, v);
+  if (A.vhat_out) {
+    float e[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) e[j] = mul_sep(v[j], v[j]);
+    const float nv = fmaxf(sqrtf(row_sum(e, c)), A.xsa_eps);
+#pragma unroll
+    for (int j = 0; j < 8; j++) e[j] = v[j] / nv;
+    if (live) st8<UVMI_F32>(A.vhat_out, r * 64 + 8 * c, e);
+  }
+  const int64_t slot = A.ring ? (p % A.S) : p;
+  bool wr = live && A.k_cache && row >= 0 && p >= 0 && slot < A.S;
+  if (A.ring && A.last_pos && p <= lastp - A.S) wr = false;   // only the last S positions of a prompt survive in a ring
+  if (A.k_cache && !A.k_scale) {
+    if (wr) {
+      st8<DT>(A.k_cache, row * A.scb + slot * A.scs + 8 * c, k);
+      st8<DT>(A.v_cache, row * A.scb + slot * A.scs + 8 * c, v);
+    }
+  } else if (A.k_cache) {
+    int8_t* caches[2] = {A.k_cache, A.v_cache};
+    uint16_t* scales[2] = {A.k_scale, A.v_scale};
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      float am = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; j++) am = fmaxf(am, fabsf(u ? v[j] : k[j]));
+      am = fmaxf(am, lane_xor4(am));
+      am = fmaxf(am, lane_xor2(am));
+      am = fmaxf(am, lane_xor1(am));
+      const uint16_t sb = float_to_half_bits(__fdiv_rn(am, 127.0f));
+      const float sf = fmaxf(half_bits_to_float(sb), 1e-30f);
+      uint32_t b[2] = {0u, 0u};
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const float qv = fminf(fmaxf(__builtin_rintf(__fdiv_rn(u ? v[j] : k[j], sf)), -127.0f), 127.0f);
+        b[j / 4] |= (uint32_t)(uint8_t)(int8_t)(int)qv << (8 * (j % 4));
+      }
+      if (wr) {
+        *(uint2*)(caches[u] + row * A.scb + slot * A.scs + 8 * c) = uint2{b[0], b[1]};
+        if (c == 0) scales[u][row * A.ssb + slot] = sb;
+      }
+    }
+  }
+  // ---- queries
+  if (live && A.gate_out) A.gate_out[r * 8 + c] = rnd(2.0f * rnd(1.0f / (1.0f + __expf(-glog))));
+#pragma unroll
+  for (int h = 0; h < 8; h++) {
+    float x[8], ss = 0.f;
+    unpack8<DT>(qw[h], x);
+#pragma unroll
+    for (int j = 0; j < 8; j++) ss += x[j] * x[j];
+    ss += lane_xor1(ss); ss += lane_xor2(ss); ss += lane_xor4(ss);
+    const float rs = rsqrtf(ss * (1.0f / 64.0f) + A.eps);
+#pragma unroll
+    for (int j = 0; j < 8; j++) x[j] = x[j] * rs;
+    round8(x);
+    if (A.rope) rotate(x);
+    if (live) st8<DT>(A.q_out, (r * 8 + h) * 64 + 8 * c, x);
+  }
+}
+
 // ------------------------------------------------------------------------------------------------ attn_post (hd = 64)
 struct PostArgs {
   const void* z; const void* v; const void* xn; const float* gate_w; const float* xsa;
@@ -612,7 +796,16 @@ extern "C" int uvmi_qkv_post(const uvmi_qkv_post_args* a, void* stream) {
   const dim3 grid((unsigned)((a->n + 3) / 4)), blk(256);
   const bool fast = (a->dtype == UVMI_F16 || a->dtype == UVMI_BF16) && a->q_dtype == a->dtype && a->H == 8 && a->KH == 1 && A.ext &&
                     (!a->rope || (a->n_pairs == 16 && A.rope_tab && ((uintptr_t)A.rope_tab % 16) == 0));
-  if (fast) {
+  // passes of many rows: 8 per wave, with wide accesses to everything that a row reads or writes.  A wave of 8 rows has the longer chain (2048
+  // rows 7.1 us against 4.7, 4096 7.8 against 6.8, 6144 8.9 against 9.1, 8192 9.9 against 11.2)
+  const uintptr_t wide = (uintptr_t)a->k_out | (uintptr_t)a->v_out | (uintptr_t)a->vhat_out | (a->has_ve ? (uintptr_t)a->ve_table : 0) |
+                         (a->k_cache ? (uintptr_t)a->k_cache | (uintptr_t)a->v_cache : 0) * (a->k_scale ? 2 : 1);
+  const bool cache_ok = !a->k_cache || (a->scb % 8 == 0 && a->scs % 8 == 0);
+  if (fast && a->n >= 6144 && wide % 16 == 0 && cache_ok) {
+    const dim3 g8((unsigned)((a->n + 7) / 8)), blk(64);
+    if (a->dtype == UVMI_F16) hipLaunchKernelGGL((qkv_post_rows_kernel<UVMI_F16>), g8, blk, 0, (hipStream_t)stream, A);
+    else hipLaunchKernelGGL((qkv_post_rows_kernel<UVMI_BF16>), g8, blk, 0, (hipStream_t)stream, A);
+  } else if (fast) {
     if (a->dtype == UVMI_F16) hipLaunchKernelGGL((qkv_post_fast_kernel<UVMI_F16>), grid, blk, 0, (hipStream_t)stream, A);
     else hipLaunchKernelGGL((qkv_post_fast_kernel<UVMI_BF16>), grid, blk, 0, (hipStream_t)stream, A);
   } else {
