@@ -1239,3 +1239,37 @@ def test_output_projection_in_the_attention_launch_refuses():
         with pytest.raises(L.UvmiError):
             launch(torch.empty(B, 8, 64, device=DEV, dtype=torch.bfloat16), dict(w=rn(N, 512).bfloat16(), resid=h, out=h, ca=1.0, cb=1.0))
         assert bool((h == 7.0).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K,epi", [(400, 640, 1664, "resid"), (512, 640, 1664, "resid"), (513, 640, 512, "resid"), (832, 640, 1664, "resid"), (1009, 640, 512, "resid"),
+                                       (1152, 640, 1664, "resid"), (1280, 640, 512, "resid"), (1601, 640, 1664, "resid"), (2048, 640, 1664, "resid"), (2049, 640, 1664, "resid"),
+                                       (450, 656, 640, "norm"), (900, 656, 640, "norm"), (1790, 656, 640, "norm"), (260, 3328, 640, "swiglu"), (448, 3328, 640, "swiglu"),
+                                       (449, 3328, 640, "swiglu"), (300, 3232, 192, "swiglu"), (1792, 336, 64, "store"), (577, 624, 128, "store")])
+def test_streaming_tiles_of_few_hundred_to_two_thousand_rows(dtype, M, N, K, epi):
+    """The built-in choice at the row counts where the tile changes (32 x 48, 48 x 64, 64 x 80 and, with SWIGLU, 64 x 96 among them), whole
+    tiles and ragged ones in both directions, K down to a slab that most waves have no share of: every element within two roundings of
+    the float64 product."""
+    from ultraviolet_amd.kernels.gemm import RESID, SWIGLU, gemm_tn
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a, w = (torch.randn(s, K, device="cuda", generator=g).to(dtype) for s in (M, N))
+    w = (w.float() / K ** 0.5).to(dtype)
+    r = torch.randn(M, N, device="cuda", generator=g).to(dtype)
+    kw = {"resid": dict(epilogue=RESID, resid=r, ca=0.75, cb=1.25), "norm": dict(norm_eps=1e-6), "swiglu": dict(epilogue=SWIGLU, norm_eps=1e-6), "store": {}}[epi]
+    got = gemm_tn(a, w, **kw).double()
+    x = a.double()
+    if "norm_eps" in kw:
+        x = x * torch.rsqrt((x * x).mean(1, keepdim=True) + 1e-6)
+    p = x @ w.double().t()
+    ulp = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    if epi == "swiglu":   # gate, up and silu(gate) are rounded before their product
+        p = p.view(M, N // 32, 2, 16)
+        gate, up = p[:, :, 0].reshape(M, -1), p[:, :, 1].reshape(M, -1)
+        p = torch.nn.functional.silu(gate) * up
+        bound = ulp * (2 * p.abs() + (gate.abs() * 1.1).clamp_min(0.3) * up.abs() * 1.5) + 1e-3 * ulp
+    elif epi == "resid":
+        p, bound = 0.75 * r.double() + 1.25 * p, ulp * (1.25 * p.abs() + (0.75 * r.double() + 1.25 * p).abs()) + 1e-3 * ulp
+    else:
+        bound = ulp * p.abs() + 1e-3 * ulp
+    assert bool(((got - p).abs() <= bound + 1e-5).all()), float(((got - p).abs() - bound).max())

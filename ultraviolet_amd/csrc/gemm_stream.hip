@@ -60,10 +60,10 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(const void* a_a, c
   constexpr int ROWS = BM + BN, LOADS = ROWS / 8;          // a load instruction moves 8 rows of 128 bytes
   constexpr int FW = (F + NW - 1) / NW;                    // fragments per wave in the epilogue
   static_assert(R == 1 || R == 2, "slabs of a wave in flight");
-  static_assert(F * 1024 <= ROWS * 128, "a wave's partial sums fit its slab's space");
+  constexpr int SLAB = ROWS * 128 > F * 1024 ? ROWS * 128 : F * 1024;   // a wave's slab, later its partial sums
   // (one object per stage: the compiler can then tell that reads of one do not touch the one a load is filling)
-  __shared__ __attribute__((aligned(1024))) unsigned char s0[NW * ROWS * 128];
-  __shared__ __attribute__((aligned(1024))) unsigned char s1[R > 1 ? NW * ROWS * 128 : 16];
+  __shared__ __attribute__((aligned(1024))) unsigned char s0[NW * SLAB];
+  __shared__ __attribute__((aligned(1024))) unsigned char s1[R > 1 ? (NW - 1) * SLAB + ROWS * 128 : 16];
   __shared__ float sSS[NORM ? NW * BM : 1];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -90,7 +90,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(const void* a_a, c
   }
   const int nk = P.K / 64;
   const int nw = (nk - wave + NW - 1) / NW;                // slabs of this wave: wave, wave + NW, ..
-  const int lds0 = wave * (ROWS * 128);
+  const int lds0 = wave * SLAB;
   auto issue = [&](unsigned char* S, int i) {
     const int ko = (wave + NW * i) * 128;
 #pragma unroll
@@ -166,7 +166,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(const void* a_a, c
       if (g == r >> 2) sSS[wave * BM + 16 * f + r] = v;
     }
   }
-  auto part = [&](int w, int f) { return (gf4*)(s0 + w * (ROWS * 128) + 1024 * f) + lane; };   // fragment f of wave w's sums
+  auto part = [&](int w, int f) { return (gf4*)(s0 + w * SLAB + 1024 * f) + lane; };   // fragment f of wave w's sums
 #pragma unroll
   for (int fi = 0; fi < FM; fi++)
 #pragma unroll
@@ -262,6 +262,9 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(const void* a_a, c
   }
 }
 
+// (a gate and an up fragment beside each other in every wave's share)
+constexpr bool swiglu_tile(int bm, int bn) { return bn == 16 || (bn % 32 == 0 && bm != 48); }
+
 template <int DT, int BM, int BN, int NW, int R>
 static void launch_stream(const uvmi_gemm_args* a, StreamParams& P, hipStream_t st) {
   P.tiles_m = (int)((a->M + BM - 1) / BM);
@@ -270,43 +273,64 @@ static void launch_stream(const uvmi_gemm_args* a, StreamParams& P, hipStream_t 
   const dim3 grid((unsigned)(((T + 7) / 8) * 8)), blk(64 * NW);
 #define UVMI_GO(EPI, NORM) hipLaunchKernelGGL((gemm_stream_kernel<DT, BM, BN, NW, R, EPI, NORM>), grid, blk, 0, st, P.a, P.w, P.lda2, P.ldw2, P.M, P.N, P.K, P.tiles_m, P.tiles_n, P.rowsplit, P.r, P.c, P.ldc, P.ldr, P.eps, P.ca, P.cb)
   const bool norm = a->norm_a != 0;
-  if (a->epilogue == UVMI_GEMM_RESID) { if (norm) UVMI_GO(2, true); else UVMI_GO(2, false); }
-  else if (a->epilogue == UVMI_GEMM_SWIGLU) {
-    if (norm) UVMI_GO(1, true); else UVMI_GO(1, false);
-  } else { if (norm) UVMI_GO(0, true); else UVMI_GO(0, false); }
+  if (a->epilogue == UVMI_GEMM_SWIGLU) {
+    if constexpr (swiglu_tile(BM, BN)) { if (norm) UVMI_GO(1, true); else UVMI_GO(1, false); }
+  } else if constexpr (BN != 96) {   // (which serves SWIGLU alone)
+    if (a->epilogue == UVMI_GEMM_RESID) { if (norm) UVMI_GO(2, true); else UVMI_GO(2, false); }
+    else { if (norm) UVMI_GO(0, true); else UVMI_GO(0, false); }
+  }
 #undef UVMI_GO
 }
 
-// The tiles, from the smallest: (BM, BN, NW, R).  LDS: 64, 48, 64, 96 / 48, 64 KB.  The smallest tile takes 8 waves (K of 512 or
-// 640: one or two slabs each, all in flight at once).
+// The tiles, by the rows of A and W that they load: (BM, BN, NW, R).  LDS: 64, 48, 64, 80, 96 / 48, 112, 64, 152, 96 KB.  The smallest
+// tile takes 8 waves (K of 512 or 640: one or two slabs each, all in flight at once).
+constexpr int TILE_M[9] = {16, 16, 32, 32, 32, 48, 64, 64, 64}, TILE_N[9] = {16, 32, 32, 48, 64, 64, 64, 80, 96};
+constexpr int FORM_64 = 6, FORM_96 = 8;
 template <int DT>
 static void launch_form(const uvmi_gemm_args* a, int form, bool single_round, StreamParams& P, hipStream_t st) {
   switch (form) {
     case 0: launch_stream<DT, 16, 16, 8, 2>(a, P, st); break;
     case 1: launch_stream<DT, 16, 32, 4, 2>(a, P, st); break;
     case 2: launch_stream<DT, 32, 32, 4, 2>(a, P, st); break;
-    case 3:   // two slabs per wave ahead where a compute unit has one workgroup; else one, and three workgroups fit (384 rows, N 3328: 7.3 against 11.3 us)
+    case 3: launch_stream<DT, 32, 48, 4, 2>(a, P, st); break;
+    case 4:   // two slabs per wave ahead where a compute unit has one workgroup; else one, and three workgroups fit (384 rows, N 3328: 7.3 against 11.3 us)
       if (single_round) launch_stream<DT, 32, 64, 4, 2>(a, P, st);
       else launch_stream<DT, 32, 64, 4, 1>(a, P, st);
       break;
+    case 5: launch_stream<DT, 48, 64, 4, 2>(a, P, st); break;
+    case 7: launch_stream<DT, 64, 80, 4, 2>(a, P, st); break;
+    case FORM_96: launch_stream<DT, 64, 96, 4, 1>(a, P, st); break;
     default: launch_stream<DT, 64, 64, 4, 1>(a, P, st); break;
   }
 }
 
 static int64_t stream_tiles(const uvmi_gemm_args* a, int form) {
-  static const int bm[5] = {16, 16, 32, 32, 64}, bn[5] = {16, 32, 32, 64, 64};
-  return ((a->M + bm[form] - 1) / bm[form]) * ((a->N + bn[form] - 1) / bn[form]);
+  return ((a->M + TILE_M[form] - 1) / TILE_M[form]) * ((a->N + TILE_N[form] - 1) / TILE_N[form]);
 }
 
-// The smallest tile that leaves a compute unit about one workgroup: smaller ones re-read the operands more often, larger ones
-// leave compute units idle and a longer chain of slabs per wave (640 columns, K 1664, 128 rows: 16 x 16 4.0 us, 16 x 32 3.7, 32 x 32
-// 4.5; 512 rows: 16 x 32 6.7, 32 x 32 6.8, 32 x 64 5.9, 64 x 64 7.9).  A short K ends before a second workgroup on the unit
-// hurts: 7 / 4 per unit up to K = 768 (640 columns, K 512, 256 rows: 16 x 32, 320 tiles, 3.0 us; 32 x 32, 160 tiles, 3.1).
-// -1: more than that even of 64 x 64 tiles.
+// The smallest tile that leaves a compute unit one workgroup: a launch lasts as long as a unit takes to load its tiles' rows, about 0.055 us
+// a row at K 1664, and larger tiles leave units idle.  (640 columns, K 1664: 384 rows, 32 x 32, 64 rows of operands a unit, 5.4 us; 512 rows,
+// where those come to 320 tiles, 7.4, 32 x 48, 80 rows, 6.0, 32 x 64 6.8; 1024 rows 48 x 64 7.7, 64 x 64 8.8; 2048 rows 64 x 80 9.8, two rounds of 64 x 64
+// 12.4.  K 512: 512 rows 32 x 32 4.4, 32 x 48 4.0; 2048 rows 64 x 80 6.1, 64 x 64 6.9.)  Of the two smallest a short K ends before a second
+// workgroup on the unit hurts: 7 / 4 per unit up to K = 768 (K 512, 256 rows: 16 x 32, 320 tiles, 3.0 us; 32 x 32, 160 tiles, 3.1); nor does it with
+// 32 x 64 ones where 48 x 64 come to more than one (1280 rows 5.3, 64 x 64 5.5).  So with SWIGLU,
+// whose tiles are multiples of 32 wide (N 3328, 256 rows: 32 x 64, 416 tiles, 5.9, 64 x 64 6.0), unless 64 x 96 ones fill one round where
+// 64 x 64 ones begin a second (448 rows 7.2, 64 x 64 7.7; 320 rows 7.1 and 7.4).
+// -1: more than that of every tile.
 int gemm_stream_form(const uvmi_gemm_args* a, int cus) {
   const int64_t most = a->K <= 768 ? (int64_t)cus * 7 / 4 : cus;
-  for (int f = 0; f < 5; f++)
-    if (stream_tiles(a, f) <= most) return f;
+  if (a->epilogue == UVMI_GEMM_SWIGLU) {
+    for (int f = 0; f < FORM_64; f++)
+      if (swiglu_tile(TILE_M[f], TILE_N[f]) && stream_tiles(a, f) <= most) return f;
+    const int64_t t = stream_tiles(a, FORM_64);
+    if (t > cus && stream_tiles(a, FORM_96) <= cus) return FORM_96;
+    return t <= most ? FORM_64 : -1;
+  }
+  for (int f = 0; f < FORM_64; f++)
+    if (stream_tiles(a, f) <= (f < 2 ? most : cus)) return f;
+  if (stream_tiles(a, 4) <= most) return 4;
+  for (int f = FORM_64; f < FORM_96; f++)
+    if (stream_tiles(a, f) <= cus) return f;
   return -1;
 }
 
