@@ -1273,3 +1273,29 @@ def test_streaming_tiles_of_few_hundred_to_two_thousand_rows(dtype, M, N, K, epi
     else:
         bound = ulp * p.abs() + 1e-3 * ulp
     assert bool(((got - p).abs() <= bound + 1e-5).all()), float(((got - p).abs() - bound).max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("B,V", [(1, 512), (3, 1536), (256, 32768), (257, 32768), (255, 8704), (300, 512)])
+def test_greedy_at_both_widths(dtype, B, V):
+    """1024 threads per row up to a row per compute unit, 256 beyond: the first maximal index (ties inside a vector, across threads and
+    waves; values that are not numbers never win), the float64 log-prob to the sum's 32-bit rounding, and an uncommitted
+    row's results alone touched."""
+    from ultraviolet_amd.kernels.fused_sample import greedy_sample
+    g = torch.Generator(device="cuda").manual_seed(B + V)
+    x = (torch.randn(B, V, device="cuda", generator=g) * 2 - 4).to(dtype)
+    top = torch.tensor(9.0, device="cuda").to(dtype)
+    x[0, V - 1] = x[0, V // 2] = top                                   # a tie far apart
+    if B > 2:
+        x[1] = 1.0                                                     # all alike
+        x[2, 5:9] = top
+    tok, lp = greedy_sample(x, (23.0, 5.0, 7.5))
+    want = x.float().argmax(-1)
+    first = (x == x.max(-1, keepdim=True).values).float().argmax(-1)   # torch's argmax may return any of a tie's
+    assert torch.equal(tok, first) and bool((x.gather(1, want[:, None]) == x.gather(1, tok[:, None])).all())
+    z = 23.0 * torch.sigmoid((x.double() + 5.0) / 7.5)
+    ref = torch.log_softmax(z, -1).gather(1, tok[:, None])[:, 0]
+    assert float((lp.double() - ref).abs().max()) < 5e-6
+    x[0, 3] = float("nan")
+    assert int(greedy_sample(x, (23.0, 5.0, 7.5))[0][0]) == int(tok[0])

@@ -47,11 +47,27 @@ struct SampleParams {
   int commit; float retire_p; uint64_t commit_seed; uvmi_sched_state S; DenseArrays D;
 };
 
-// The row's result; with P.commit also what uvmi_sched_commit_dense does for the row (one thread per row calls this).
-__device__ __forceinline__ void emit(const SampleParams P, int row, int tok, float logp) {
+// The row's result; with P.commit also what uvmi_sched_commit_dense does for the row (one thread per row calls this; r: its commit_ahead).
+__device__ __forceinline__ void emit(const SampleParams& P, int row, int tok, float logp, const CommitRow& r) {
   P.tok[row] = tok;
   P.logp[row] = logp;
-  if (P.commit) commit_row<true>(P.S, P.D, row, tok, logp, P.retire_p, P.commit_seed);
+  if (P.commit) commit_store<true>(P.S, P.D, row, r, tok, logp);
+}
+// what emit's commit reads, for thread 0, which emits: behind the requests for the row's logits
+__device__ __forceinline__ CommitRow commit_ahead(const SampleParams& P, int row) {
+  CommitRow r = {};
+  if (P.commit && threadIdx.x == 0) r = commit_load<true>(P.S, P.D, row, P.retire_p, P.commit_seed);
+  return r;
+}
+// the row's uniform (every thread of the wave that draws)
+__device__ __forceinline__ float uniform_of(const SampleParams& P, int row) {
+  if (P.u) return P.u[row];
+  const uint64_t rid = (uint64_t)P.req_id[row], ti = (uint64_t)P.tok_idx[row];
+  const uint32_t ctr[4] = {(uint32_t)ti, (uint32_t)rid, (uint32_t)(rid >> 32), DOMAIN_SAMPLE};
+  const uint32_t key[2] = {(uint32_t)P.seed, (uint32_t)(P.seed >> 32)};
+  uint32_t o[4];
+  philox4x32_10(ctr, key, o);
+  return (float)(o[0] >> 8) * 5.9604644775390625e-08f;  // 2^-24
 }
 
 template <int DT>
@@ -94,6 +110,8 @@ __global__ __launch_bounds__(NT) void sample_kernel(const void* a_x, int64_t a_s
   const int row = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const char* xr = (const char*)P.x + (int64_t)row * P.stride * (DT == UVMI_F32 ? 4 : 2);
   const int nchunks = P.V / CHUNK;  // host guarantees V % 512 == 0 and nchunks <= 64
+  const float u = wave == 0 ? uniform_of(P, row) : 0.f;
+  const CommitRow cr = commit_ahead(P, row);
   for (int c = wave; c < nchunks; c += NT / 64) {
     float v[8];
     load8<DT>(xr, c * 64 + lane, v);
@@ -114,17 +132,6 @@ __global__ __launch_bounds__(NT) void sample_kernel(const void* a_x, int64_t a_s
     if (lane >= o) incl += t;
   }
   const float S = __shfl(incl, 63, 64);
-  float u;
-  if (P.u) {
-    u = P.u[row];
-  } else {
-    const uint64_t rid = (uint64_t)P.req_id[row], ti = (uint64_t)P.tok_idx[row];
-    const uint32_t ctr[4] = {(uint32_t)ti, (uint32_t)rid, (uint32_t)(rid >> 32), DOMAIN_SAMPLE};
-    const uint32_t key[2] = {(uint32_t)P.seed, (uint32_t)(P.seed >> 32)};
-    uint32_t o[4];
-    philox4x32_10(ctr, key, o);
-    u = (float)(o[0] >> 8) * 5.9604644775390625e-08f;  // 2^-24
-  }
   const float target = (1.0f - u) * S;
   const unsigned long long below = __ballot(lane < nchunks && incl < target);
   int ck = __popcll(below);  // first chunk whose inclusive sum reaches target
@@ -165,7 +172,7 @@ __global__ __launch_bounds__(NT) void sample_kernel(const void* a_x, int64_t a_s
     // logp = (z_tok - a)/T - log S, with (z - a)/T = -(a/T) / (1 + exp(t))
     const float E = __builtin_amdgcn_exp2f(fmaf(xsel, P.inv_c_l2, P.b_over_c_l2));
     if (P.u_out) P.u_out[row] = u;
-    emit(P, row, tok, P.neg_a_over_t * __builtin_amdgcn_rcpf(1.0f + E) - __logf(S));
+    emit(P, row, tok, P.neg_a_over_t * __builtin_amdgcn_rcpf(1.0f + E) - __logf(S), cr);
   }
 }
 
@@ -271,19 +278,9 @@ __global__ __launch_bounds__(1024) void sample_filtered_kernel(SampleParams P) {
     const int c = wave + 16 * q;
     if (c < nchunks) load8<DT>(xr, c * 64 + lane, e[q]);
   }
-  float u = 0.f;   // (requested with the row: the draw at the end of the chain needs it at once)
-  if (wave == 0) {
-    if (P.u) {
-      u = P.u[row];
-    } else {
-      const uint64_t rid = (uint64_t)P.req_id[row], ti = (uint64_t)P.tok_idx[row];
-      const uint32_t ctr[4] = {(uint32_t)ti, (uint32_t)rid, (uint32_t)(rid >> 32), DOMAIN_SAMPLE};
-      const uint32_t key[2] = {(uint32_t)P.seed, (uint32_t)(P.seed >> 32)};
-      uint32_t o[4];
-      philox4x32_10(ctr, key, o);
-      u = (float)(o[0] >> 8) * 5.9604644775390625e-08f;  // 2^-24
-    }
-  }
+  // (requested with the row: the end of the chain needs them at once)
+  const float u = wave == 0 ? uniform_of(P, row) : 0.f;
+  const CommitRow cr = commit_ahead(P, row);
   for (int i = tid; i < 4096; i += 1024) h1[i] = 0;
   h2[tid] = 0;
   h3[tid] = 0;
@@ -531,31 +528,52 @@ __global__ __launch_bounds__(1024) void sample_filtered_kernel(SampleParams P) {
     const float E = __builtin_amdgcn_exp2f(fmaf(xsel, P.inv_c_l2, P.b_over_c_l2));
     if (P.u_out) P.u_out[row] = u;
     if (P.thr_out) P.thr_out[row] = __uint_as_float(thr);
-    emit(P, row, ck * CHUNK + sel, P.neg_a_over_t * __builtin_amdgcn_rcpf(1.0f + E) - __logf(S));
+    emit(P, row, ck * CHUNK + sel, P.neg_a_over_t * __builtin_amdgcn_rcpf(1.0f + E) - __logf(S), cr);
   }
 }
 
 // Greedy: argmax of the raw head output (the softcap is strictly increasing, so argmax z = argmax x), first maximal
 // index; logp = log softmax(z)[tok] at T = 1.
-template <int DT>
-__global__ __launch_bounds__(256) void argmax_kernel(SampleParams P) {
-  __shared__ float smax[4];
-  __shared__ int sidx[4];
-  __shared__ float ssum[4];
+// What bounds it: three quarter-rate instructions an element (exp2, reciprocal, exp2) on the compute unit that has the row, behind the
+// launch and a load; with a commit, what that reads.  us with a commit, its reads at the end -> ahead and 1024 threads up to a row per
+// compute unit: 1 row 8.3 -> 7.4, 16 rows 9.2 -> 8.0, 256 rows 10.4 -> 8.9; 640 rows 17.8 -> 16.5, 1024 rows 21.0 -> 19.8.
+// (The last bits of the log-prob's sum of exponentials go with the width; the token does not.)
+template <int DT, int NT>
+__global__ __launch_bounds__(NT) void argmax_kernel(SampleParams P) {
+  constexpr int NW = NT / 64;
+  __shared__ float smax[NW];
+  __shared__ int sidx[NW];
+  __shared__ float ssum[NW];
   const int row = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const char* xr = (const char*)P.x + (int64_t)row * P.stride * (DT == UVMI_F32 ? 4 : 2);
   const int nvec = P.V / 8;
   float best = -INFINITY, esum = 0.f;
   int bi = 0x7fffffff;
-  for (int i = threadIdx.x; i < nvec; i += 256) {
-    float v[8];
-    load8<DT>(xr, i, v);
+  CommitRow cr = {};
+  if constexpr (NT == 256) cr = commit_ahead(P, row);
+  auto take = [&](const float (&v)[8], int i) {
 #pragma unroll
     for (int j = 0; j < 8; j++) {
       if (v[j] > best) { best = v[j]; bi = i * 8 + j; }
       // softmax(z) with T = 1: e = exp(z - a)
       const float E = __builtin_amdgcn_exp2f(fmaf(v[j], P.inv_c_l2, P.b_over_c_l2));
       esum += __builtin_amdgcn_exp2f(-P.cap_a * 1.4426950408889634f * __builtin_amdgcn_rcpf(1.0f + E));
+    }
+  };
+  if constexpr (NT == 1024) {   // (at most four vectors a thread: all requested at once)
+    float v[4][8];
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+      if (threadIdx.x + 1024 * q < nvec) load8<DT>(xr, threadIdx.x + 1024 * q, v[q]);
+    cr = commit_ahead(P, row);
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+      if (threadIdx.x + 1024 * q < nvec) take(v[q], threadIdx.x + 1024 * q);
+  } else {
+    for (int i = threadIdx.x; i < nvec; i += NT) {
+      float v[8];
+      load8<DT>(xr, i, v);
+      take(v, i);
     }
   }
   for (int o = 32; o > 0; o >>= 1) {
@@ -568,13 +586,13 @@ __global__ __launch_bounds__(256) void argmax_kernel(SampleParams P) {
   __syncthreads();
   if (threadIdx.x == 0) {
     float tot = 0.f;
-    for (int w = 0; w < 4; w++) {
+    for (int w = 0; w < NW; w++) {
       tot += ssum[w];
       if (smax[w] > best || (smax[w] == best && sidx[w] < bi)) { best = smax[w]; bi = sidx[w]; }
     }
     const float E = __builtin_amdgcn_exp2f(fmaf(best, P.inv_c_l2, P.b_over_c_l2));
     if (P.u_out) P.u_out[row] = 0.f;
-    emit(P, row, bi, -P.cap_a * __builtin_amdgcn_rcpf(1.0f + E) - __logf(tot));
+    emit(P, row, bi, -P.cap_a * __builtin_amdgcn_rcpf(1.0f + E) - __logf(tot), cr);
   }
 }
 
@@ -631,26 +649,27 @@ extern "C" int uvmi_fused_sample(const uvmi_sample_args* a, void* stream) {
   }
   const bool filtered = !greedy && (P.top_k > 0 || P.top_p < 1.0f);
   hipStream_t st = (hipStream_t)stream;
-  const dim3 grid(a->B), blk(filtered ? 1024 : 256);
-#define UVMI_S(K)                                                                          \
-  do {                                                                                     \
-    if (a->x_dtype == UVMI_F16) hipLaunchKernelGGL((K<UVMI_F16>), grid, blk, 0, st, P);    \
-    else if (a->x_dtype == UVMI_BF16) hipLaunchKernelGGL((K<UVMI_BF16>), grid, blk, 0, st, P); \
-    else hipLaunchKernelGGL((K<UVMI_F32>), grid, blk, 0, st, P);                           \
-  } while (0)
-  if (greedy) UVMI_S(argmax_kernel);
-  else if (filtered) UVMI_S(sample_filtered_kernel);
-  else {
+  // Drawing, 1024 threads per row are faster up to ~640 rows (12.0 against 14.5 us at 384 rows), slower from 1024 on; its sums are formed per
+  // chunk whatever the width, so the draw does not depend on it.  Greedy, up to a row per compute unit (256 rows 8.4 against 8.7,
+  // 300 rows 12.9 against 10.8).
+  int cus = uvmi_device_cus();
+  if (cus <= 0) cus = 256;
+  const bool wide = filtered || a->B <= (greedy ? cus : 640);
+  const dim3 grid(a->B), blk(wide ? 1024 : 256);
+#define UVMI_S(...) hipLaunchKernelGGL((__VA_ARGS__), grid, blk, 0, st, P)
 #define UVMI_SK(DT, NT) \
-  hipLaunchKernelGGL((sample_kernel<DT, NT>), grid, dim3(NT), 0, st, P.x, P.stride, P.V, P.inv_c_l2, P.b_over_c_l2, P.neg_a_over_t_l2, P)
-    // 1024 threads per row are faster up to ~640 rows (measured: 12.0 against 14.5 us at 384 rows), slower from 1024 on; the
-    // chunk sums are formed per chunk whatever the width, so the draw does not depend on it
-    const bool wide = a->B <= 640;
-    if (a->x_dtype == UVMI_F16) { if (wide) UVMI_SK(UVMI_F16, 1024); else UVMI_SK(UVMI_F16, 256); }
-    else if (a->x_dtype == UVMI_BF16) { if (wide) UVMI_SK(UVMI_BF16, 1024); else UVMI_SK(UVMI_BF16, 256); }
-    else { if (wide) UVMI_SK(UVMI_F32, 1024); else UVMI_SK(UVMI_F32, 256); }
+  hipLaunchKernelGGL((sample_kernel<DT, NT>), grid, blk, 0, st, P.x, P.stride, P.V, P.inv_c_l2, P.b_over_c_l2, P.neg_a_over_t_l2, P)
+#define UVMI_DT(DT)                                                                                      \
+  do {                                                                                                   \
+    if (filtered) UVMI_S(sample_filtered_kernel<DT>);                                                    \
+    else if (greedy) { if (wide) UVMI_S(argmax_kernel<DT, 1024>); else UVMI_S(argmax_kernel<DT, 256>); } \
+    else { if (wide) UVMI_SK(DT, 1024); else UVMI_SK(DT, 256); }                                         \
+  } while (0)
+  if (a->x_dtype == UVMI_F16) UVMI_DT(UVMI_F16);
+  else if (a->x_dtype == UVMI_BF16) UVMI_DT(UVMI_BF16);
+  else UVMI_DT(UVMI_F32);
+#undef UVMI_DT
 #undef UVMI_SK
-  }
 #undef UVMI_S
   UVMI_CHECK_LAUNCH("uvmi_fused_sample");
   return UVMI_OK;

@@ -71,13 +71,14 @@ __global__ __launch_bounds__(1024) void sched_compact_kernel(uvmi_sched_state S,
   compact_phase(S, n_bucket, act_slot, tok_c, pos_c, starts_c, req_c, cnt_c, wsum, base_sh);
 }
 
-// One thread per dense row (see commit_row).
+// One thread per dense row (see commit_store).
 template <bool DENSE>
 __global__ __launch_bounds__(256) void sched_commit_kernel(uvmi_sched_state S, int n_bucket, DenseArrays D, const int64_t* new_tok,
                                                            const float* new_lp, float retire_p, uint64_t seed) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= n_bucket) return;
-  commit_row<DENSE>(S, D, i, new_tok[i], new_lp ? new_lp[i] : 0.f, retire_p, seed);
+  const CommitRow r = commit_load<DENSE>(S, D, i, retire_p, seed);
+  commit_store<DENSE>(S, D, i, r, new_tok[i], new_lp ? new_lp[i] : 0.f);
 }
 
 // Admission after a prefill: bind request ids to slots and record the first sampled token (it counts as token 0 of
