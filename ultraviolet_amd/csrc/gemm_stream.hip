@@ -20,14 +20,14 @@
 //     fragments.  The residual of that share is requested before anything else; the squares of NORM are the diagonal of an
 //     activation fragment's product with itself, one more matrix instruction for it (32 vector ones before: twice the time of the 64 x
 //     64 tile's own products);
-//   * rows past M or N are clamped to the last one (computed, not stored);
+//   * rows past M or N are zeros (computed, not stored);
 //   * individual scalar arguments rather than a parameter block: they arrive in SGPRs with the wave.
 // us per launch in a stream of launches with 20 layers' weights in turn (N x K: 656 x 640 with NORM | 640 x 512 RESID | 3328 x 640
 // NORM, SWIGLU | 640 x 1664 RESID), and in brackets what the forms took that it replaced (a whole weight strip parked in LDS
 // behind a barrier below 448 rows, 64 x 64 tiles through registers from there on):
-//      1 row   2.7 [3.9] | 2.5 [3.8] | 3.4 [4.7] | 2.9 [4.3]        64 rows   2.8 [4.4] | 2.5 [4.3] | 3.7 [6.0] | 3.2 [5.3]
-//    256 rows  3.5 [5.6] | 3.0 [5.4] | 5.4 [6.5] | 4.6 [9.2]       512 rows   4.1 [6.2] | 3.7 [5.2] | 7.6 [8.7] | 5.9 [8.9]
-//   2048 rows  7.4 [8.4] | 6.7 [7.4] |     -     | 12.1 [13.7]
+//      1 row   2.7 [3.9] | 2.5 [3.8] | 3.4 [4.7] | 2.9 [4.3]        64 rows   2.7 [4.4] | 2.5 [4.3] | 3.7 [6.0] | 3.2 [5.3]
+//    256 rows  3.5 [5.6] | 3.0 [5.4] | 5.4 [6.5] | 4.6 [9.2]       512 rows   4.0 [6.2] | 3.4 [5.2] | 7.4 [8.7] | 5.3 [8.9]
+//   2048 rows  7.3 [8.4] | 5.9 [7.4] |     -     | 9.5 [13.7]
 #include "common.h"
 #include "gemm_util.h"
 
@@ -41,8 +41,12 @@ struct StreamParams {
   float eps, ca, cb;
 };
 
-#define UVMI_GLBP(p) ((const __attribute__((address_space(1))) void*)(p))
 #define UVMI_LDSP(p) ((__attribute__((address_space(3))) void*)(p))
+
+// 16 bytes per lane from byte off + at of a buffer to 1 KB of LDS (a template's own code cannot hold the builtin: the host's pass checks it)
+__device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t r, unsigned char* lds, uint32_t off, int at) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, UVMI_LDSP(lds), 16, off, at, 0, 0);
+}
 
 template <int N> __device__ __forceinline__ void wait_vm() {   // all but the newest N loads have landed
   static_assert(N >= 0 && N < 64, "vmcnt has six bits");
@@ -74,27 +78,33 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(const void* a_a, c
   const int m0 = bm * BM, n0 = bn * BN;
   const int r = lane & 15, g = lane >> 4;
 
-  // ---- loader: load i of a slab moves its rows 8 i .. 8 i + 7 (the tile's rows of A, then of W)
+  // ---- loader: load i of a slab moves its rows 8 i .. 8 i + 7 (the tile's rows of A, then of W).  Rows past the last one come out as zeros:
+  // the descriptors' bounds.  (One multiplication and an addition per load: 64-bit addresses of clamped rows took ~60 cycles a load
+  // before the first one left, and twice the registers; 2 - 3 % of a launch of 400 to 2500 rows, 512 x 3328 x 640 7.76 -> 7.57 us.)
   const int lr = lane >> 3;
-  const unsigned char* gp[LOADS];
+  uint32_t off[LOADS];
+  {
+    const uint32_t c0 = (uint32_t)(((lane & 7) ^ (lr >> 1)) << 4), c1 = c0 ^ 64;   // chunk of an even, an odd load
+    const uint32_t ra = (uint32_t)(m0 + lr) * P.lda2;
 #pragma unroll
-  for (int i = 0; i < LOADS; i++) {
-    const int row = 8 * i + lr;
-    const int sw = (lane & 7) ^ ((row >> 1) & 7);
-    if (8 * i < BM) gp[i] = (const unsigned char*)P.a + (uint32_t)min(m0 + row, P.M - 1) * (size_t)P.lda2 + 16 * sw;
-    else {
-      const int j = row - BM;
-      const int wr = EPI == 1 && BN == 16 ? (n0 & ~31) + ((n0 & 16) >> 1) + (j & 7) + ((j & 8) << 1) : n0 + j;
-      gp[i] = (const unsigned char*)P.w + (uint32_t)min(wr, P.N - 1) * (size_t)P.ldw2 + 16 * sw;
-    }
+    for (int i = 0; i < BM / 8; i++) off[i] = ra + (i & 1 ? c1 : c0) + (uint32_t)(8 * i) * P.lda2;
+    // (EPI 1, 16 columns: 8 gate rows and, 16 rows on, their 8 up rows)
+    constexpr bool SPLIT = EPI == 1 && BN == 16;
+    const uint32_t rw = (uint32_t)((SPLIT ? (n0 & ~31) + ((n0 & 16) >> 1) : n0) + lr) * P.ldw2;
+#pragma unroll
+    for (int i = 0; i < BN / 8; i++) off[BM / 8 + i] = rw + (i & 1 ? c1 : c0) + (uint32_t)((SPLIT ? 16 : 8) * i) * P.ldw2;
   }
+  const __amdgpu_buffer_rsrc_t rA = __builtin_amdgcn_make_buffer_rsrc((void*)P.a, 0, (int)((uint32_t)(P.M - 1) * P.lda2 + (uint32_t)P.K * 2), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rW = __builtin_amdgcn_make_buffer_rsrc((void*)P.w, 0, (int)((uint32_t)(P.N - 1) * P.ldw2 + (uint32_t)P.K * 2), 0x00020000);
   const int nk = P.K / 64;
   const int nw = (nk - wave + NW - 1) / NW;                // slabs of this wave: wave, wave + NW, ..
   const int lds0 = wave * SLAB;
   auto issue = [&](unsigned char* S, int i) {
     const int ko = (wave + NW * i) * 128;
 #pragma unroll
-    for (int l = 0; l < LOADS; l++) __builtin_amdgcn_global_load_lds(UVMI_GLBP(gp[l] + ko), UVMI_LDSP(S + lds0 + 1024 * l), 16, 0, 0);
+    for (int l = 0; l < BM / 8; l++) load_lds16(rA, S + lds0 + 1024 * l, off[l], ko);
+#pragma unroll
+    for (int l = BM / 8; l < LOADS; l++) load_lds16(rW, S + lds0 + 1024 * l, off[l], ko);
   };
 
   // ---- this wave's share of the output, and its residual
