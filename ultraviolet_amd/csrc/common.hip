@@ -11,6 +11,8 @@ void set_error(const char* fmt, ...) {
   vsnprintf(g_err, sizeof(g_err), fmt, ap);
   va_end(ap);
 }
+static thread_local volatile char g_touched = 0;
+void touch_thread() { g_touched = 1; }
 }  // namespace uvmi
 
 extern "C" int uvmi_version(void) { return UVMI_ABI_VERSION; }
