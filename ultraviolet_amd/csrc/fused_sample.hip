@@ -278,9 +278,8 @@ __global__ __launch_bounds__(1024) void sample_filtered_kernel(SampleParams P) {
     const int c = wave + 16 * q;
     if (c < nchunks) load8<DT>(xr, c * 64 + lane, e[q]);
   }
-  // (requested with the row: the end of the chain needs them at once)
+  // (requested with the row: the draw at the end of the chain needs it at once)
   const float u = wave == 0 ? uniform_of(P, row) : 0.f;
-  const CommitRow cr = commit_ahead(P, row);
   for (int i = tid; i < 4096; i += 1024) h1[i] = 0;
   h2[tid] = 0;
   h3[tid] = 0;
@@ -299,6 +298,7 @@ __global__ __launch_bounds__(1024) void sample_filtered_kernel(SampleParams P) {
       if (lane == 0) csum_all[c] = s;
     }
   }
+  const CommitRow cr = commit_ahead(P, row);
   __syncthreads();
 
   unsigned int thr = 0;   // keep keys >= thr
