@@ -1246,7 +1246,8 @@ def test_output_projection_in_the_attention_launch_refuses():
 @pytest.mark.parametrize("M,N,K,epi", [(400, 640, 1664, "resid"), (512, 640, 1664, "resid"), (513, 640, 512, "resid"), (832, 640, 1664, "resid"), (1009, 640, 512, "resid"),
                                        (1152, 640, 1664, "resid"), (1280, 640, 512, "resid"), (1601, 640, 1664, "resid"), (2048, 640, 1664, "resid"), (2049, 640, 1664, "resid"),
                                        (450, 656, 640, "norm"), (900, 656, 640, "norm"), (1790, 656, 640, "norm"), (260, 3328, 640, "swiglu"), (448, 3328, 640, "swiglu"),
-                                       (449, 3328, 640, "swiglu"), (300, 3232, 192, "swiglu"), (1792, 336, 64, "store"), (577, 624, 128, "store")])
+                                       (449, 3328, 640, "swiglu"), (300, 3232, 192, "swiglu"), (576, 3328, 640, "swiglu"), (577, 3328, 640, "swiglu"), (3264, 640, 512, "resid"), (3265, 640, 512, "resid"),
+                                       (4864, 640, 1664, "resid"), (4865, 640, 1664, "resid"), (1792, 336, 64, "store"), (577, 624, 128, "store")])
 def test_streaming_tiles_of_few_hundred_to_two_thousand_rows(dtype, M, N, K, epi):
     """The built-in choice at the row counts where the tile changes (32 x 48, 48 x 64, 64 x 80 and, with SWIGLU, 64 x 96 among them), whole
     tiles and ragged ones in both directions, K down to a slab that most waves have no share of: every element within two roundings of

@@ -92,12 +92,14 @@ extern "C" int uvmi_gemm_tn_ex(const uvmi_gemm_args* a, void* stream) {
     UVMI_CHECK_LAUNCH("uvmi_gemm_tn(128 x 128, direct)");
     return UVMI_OK;
   }
-  // The streaming form while one of its tiles leaves a compute unit about one workgroup (gemm_stream_form) and, on 64 x 64 tiles,
-  // until 128 x 128 tiles fill enough of the device: 9/16 of it (N 656, K 640: 10.2 against 11.2 us at 3072 rows), with a longer
-  // K, where a tile's chain of slabs is longer, 4/5 (640 columns, K 1664: at 4608 rows 21.0 against 19.3, at 6144 21.6 against 24.5).
+  // The streaming form while one of its tiles leaves a compute unit about one workgroup (gemm_stream_form) and, on 64 x 64 tiles, while
+  // they are at most two to a unit, which run at the same time (N 640, K 512: 3072 rows, 480 tiles, 7.7 us against 9.2 in 128 x 128 tiles; 3328
+  // rows, 520 tiles, 10.6 / 9.3; gate-up 576 rows, 468 tiles, 7.9 / 9.5, 640 rows, 520 tiles, 11.0 / 9.9).  With a longer K, where rounds of
+  // the small tiles overlap, until 128 x 128 tiles fill 3/4 of the device (640 columns, K 1664: 4608 rows 19.3 / 20.5, 5120 rows 23.3 / 20.5).
   static const int of_config[9] = {-1, 4, 0, -1, 6, -1, -1, 1, 2};
   int form = a->config == 0 ? gemm_stream_form(a, cus) : of_config[a->config];
-  if (a->config == 0 && form < 0 && (a->K <= 768 ? 16 * t128 < 9 * (int64_t)cus : 5 * t128 < 4 * (int64_t)cus)) form = 6;
+  const int64_t t64 = ((a->M + 63) / 64) * (((int64_t)a->N + 63) / 64);
+  if (a->config == 0 && form < 0 && (a->K <= 768 ? t64 <= 2 * (int64_t)cus : 4 * t128 < 3 * (int64_t)cus)) form = 6;
   if (form >= 0) {
     gemm_stream_launch(a, form, cus, (hipStream_t)stream);
     UVMI_CHECK_LAUNCH("uvmi_gemm_tn(streaming)");
