@@ -45,18 +45,21 @@ __device__ __forceinline__ void st2(void* p, int64_t i, float a, float b) {
 }
 
 template <int DT>
+__device__ __forceinline__ void unpack8(uint4 w, float (&o)[8]) {  // 8 elements of a 16-bit type
+  const uint32_t r[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    if (DT == UVMI_BF16) { o[2 * j] = __uint_as_float(r[j] << 16); o[2 * j + 1] = __uint_as_float(r[j] & 0xffff0000u); }
+    else { o[2 * j] = half_bits_to_float(r[j] & 0xffff); o[2 * j + 1] = half_bits_to_float(r[j] >> 16); }
+  }
+}
+template <int DT>
 __device__ __forceinline__ void ld8(const void* p, int64_t i, float (&o)[8]) {  // 8 consecutive elements starting at i
   if (DT == UVMI_F32) {
     const float4 a = *(const float4*)((const float*)p + i), b = *(const float4*)((const float*)p + i + 4);
     o[0] = a.x; o[1] = a.y; o[2] = a.z; o[3] = a.w; o[4] = b.x; o[5] = b.y; o[6] = b.z; o[7] = b.w;
   } else {
-    const uint4 w = *(const uint4*)((const uint16_t*)p + i);
-    const uint32_t r[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      if (DT == UVMI_BF16) { o[2 * j] = __uint_as_float(r[j] << 16); o[2 * j + 1] = __uint_as_float(r[j] & 0xffff0000u); }
-      else { o[2 * j] = half_bits_to_float(r[j] & 0xffff); o[2 * j + 1] = half_bits_to_float(r[j] >> 16); }
-    }
+    unpack8<DT>(*(const uint4*)((const uint16_t*)p + i), o);
   }
 }
 template <int DT>
@@ -446,15 +449,6 @@ __device__ __forceinline__ float row_sum(const float (&e)[8], int c) {   // of 8
   u = add_sep(u, lane_xor4(u));
   u = add_sep(u, lane_xor2(u));
   return add_sep(u, lane_xor1(u));
-}
-template <int DT>
-__device__ __forceinline__ void unpack8(uint4 w, float (&o)[8]) {
-  const uint32_t r[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    if (DT == UVMI_BF16) { o[2 * j] = __uint_as_float(r[j] << 16); o[2 * j + 1] = __uint_as_float(r[j] & 0xffff0000u); }
-    else { o[2 * j] = half_bits_to_float(r[j] & 0xffff); o[2 * j + 1] = half_bits_to_float(r[j] >> 16); }
-  }
 }
 template <int DT>
 __global__ __launch_bounds__(64) void qkv_post_rows_kernel(QkvArgs A) {
