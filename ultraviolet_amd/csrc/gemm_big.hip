@@ -214,23 +214,23 @@ void gemm_big_kernel(BigParams P) {
   asm volatile("s_barrier" ::: "memory");
   issue(sA1, sB1, 1);
   for (;;) {   // tiles
-  const int cm0 = m0, cn0 = n0;
-  const bool more = MANY && L + step < last;
-  // slab k of this tile or, past its last one, slab k - nk of the next
-  auto request = [&](unsigned char* sa, unsigned char* sb, int k) {
-    if (k < nk) issue(sa, sb, k);
-    else if (more) {
-      if (k == nk) { tile_at(L + step); offsets(); }
-      issue(sa, sb, k - nk);
-    }
-  };
-  read_b(sB0, 0, w0);
-  read_a(sA0, 0, 0, f0);
-  // Iteration k multiplies slab k out of stage S: 8 groups of 8 MFMAs (K-step s, row pair p); the operands of a group are
-  // requested behind the first MFMA of the group before it, so a wait for them comes seven MFMAs after their request.
-  // Before the last group: slab k + 1 has landed in the other stage (own loads: the wait; the other waves': the barrier)
-  // and every read of stage S is complete, so S is refilled with slab k + 2 and the first operands of slab k + 1 are
-  // requested.
+    const int cm0 = m0, cn0 = n0;
+    const bool more = MANY && L + step < last;
+    // slab k of this tile or, past its last one, slab k - nk of the next
+    auto request = [&](unsigned char* sa, unsigned char* sb, int k) {
+      if (k < nk) issue(sa, sb, k);
+      else if (more) {
+        if (k == nk) { tile_at(L + step); offsets(); }
+        issue(sa, sb, k - nk);
+      }
+    };
+    read_b(sB0, 0, w0);
+    read_a(sA0, 0, 0, f0);
+    // Iteration k multiplies slab k out of stage S: 8 groups of 8 MFMAs (K-step s, row pair p); the operands of a group are
+    // requested behind the first MFMA of the group before it, so a wait for them comes seven MFMAs after their request.
+    // Before the last group: slab k + 1 has landed in the other stage (own loads: the wait; the other waves': the barrier)
+    // and every read of stage S is complete, so S is refilled with slab k + 2 and the first operands of slab k + 1 are
+    // requested.
 #define UVMI_ITER(SA, SB_, SAN, SBN, k)                                                                                  \
   do {                                                                                                                   \
     mm1(0, f0, w0); UVMI_SB(); read_a(SA, 0, 2, f1); UVMI_SB(); mm7(0, f0, w0); sumsq(0, f0); UVMI_SB();                 \
@@ -246,8 +246,8 @@ void gemm_big_kernel(BigParams P) {
     read_b(SBN, 0, w0); read_a(SAN, 0, 0, f0); UVMI_SB();                                                                \
     mm1(6, f1, w1); mm7(6, f1, w1); sumsq(3, f1); UVMI_SB();                                                             \
   } while (0)
-  // FI = 4: 4 groups per slab; the first operands of the next slab arrive in the buffer the iteration's second group used,
-  // so two iterations alternate the roles of f0 and f1
+    // FI = 4: 4 groups per slab; the first operands of the next slab arrive in the buffer the iteration's second group used,
+    // so two iterations alternate the roles of f0 and f1
 #define UVMI_ITER4(SA, SB_, SAN, SBN, k, X, Y)                                                                           \
   do {                                                                                                                   \
     mm1(0, X, w0); UVMI_SB(); read_a(SA, 0, 2, Y); UVMI_SB(); mm7(0, X, w0); sumsq(0, X); UVMI_SB();                     \
@@ -259,138 +259,138 @@ void gemm_big_kernel(BigParams P) {
     read_b(SBN, 0, w0); read_a(SAN, 0, 0, Y); UVMI_SB();                                                                 \
     mm1(2, X, w1); mm7(2, X, w1); sumsq(1, X); UVMI_SB();                                                                \
   } while (0)
-  int k = 0;
-  if constexpr (FI == 8) {
-    for (; k + 2 <= nk; k += 2) {
-      UVMI_ITER(sA0, sB0, sA1, sB1, k);
-      UVMI_ITER(sA1, sB1, sA0, sB0, k + 1);
+    int k = 0;
+    if constexpr (FI == 8) {
+      for (; k + 2 <= nk; k += 2) {
+        UVMI_ITER(sA0, sB0, sA1, sB1, k);
+        UVMI_ITER(sA1, sB1, sA0, sB0, k + 1);
+      }
+      if (!MANY && k < nk) UVMI_ITER(sA0, sB0, sA1, sB1, k);
+    } else {
+      for (; k + 2 <= nk; k += 2) {
+        UVMI_ITER4(sA0, sB0, sA1, sB1, k, f0, f1);
+        UVMI_ITER4(sA1, sB1, sA0, sB0, k + 1, f1, f0);
+      }
+      if (!MANY && k < nk) UVMI_ITER4(sA0, sB0, sA1, sB1, k, f0, f1);
     }
-    if (!MANY && k < nk) UVMI_ITER(sA0, sB0, sA1, sB1, k);
-  } else {
-    for (; k + 2 <= nk; k += 2) {
-      UVMI_ITER4(sA0, sB0, sA1, sB1, k, f0, f1);
-      UVMI_ITER4(sA1, sB1, sA0, sB0, k + 1, f1, f0);
-    }
-    if (!MANY && k < nk) UVMI_ITER4(sA0, sB0, sA1, sB1, k, f0, f1);
-  }
 #undef UVMI_ITER4
 #undef UVMI_ITER
 #undef UVMI_SB
 
-  const int el = fresh_lane(), r = el & 15, g = el >> 4;
-  // ---- row scales of the pre-norm: the 4 lane groups of a row add their sums; LDS carries the scales to every wave
-  float rn[FI];
+    const int el = fresh_lane(), r = el & 15, g = el >> 4;
+    // ---- row scales of the pre-norm: the 4 lane groups of a row add their sums; LDS carries the scales to every wave
+    float rn[FI];
 #pragma unroll
-  for (int i = 0; i < FI; i++) rn[i] = 1.0f;
-  if (NORM) {
-    int kd = P.K;
-    asm volatile("" : "+s"(kd));   // (not a register of its own through the main loop)
+    for (int i = 0; i < FI; i++) rn[i] = 1.0f;
+    if (NORM) {
+      int kd = P.K;
+      asm volatile("" : "+s"(kd));   // (not a register of its own through the main loop)
 #pragma unroll
-    for (int u = 0; u < 2; u++) {   // (lane (r, g) holds elements (4 g + t, r) of X X^T)
-      const float v = r & 2 ? (r & 1 ? sq[u][3] : sq[u][2]) : (r & 1 ? sq[u][1] : sq[u][0]);
-      if (g == r >> 2) sRS[16 * FI * wm + 32 * wn + 16 * u + r] = rsqrtf(v / (float)kd + P.eps);
+      for (int u = 0; u < 2; u++) {   // (lane (r, g) holds elements (4 g + t, r) of X X^T)
+        const float v = r & 2 ? (r & 1 ? sq[u][3] : sq[u][2]) : (r & 1 ? sq[u][1] : sq[u][0]);
+        if (g == r >> 2) sRS[16 * FI * wm + 32 * wn + 16 * u + r] = rsqrtf(v / (float)kd + P.eps);
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+      for (int i = 0; i < FI; i++) rn[i] = sRS[frow(i) + r];
     }
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-#pragma unroll
-    for (int i = 0; i < FI; i++) rn[i] = sRS[frow(i) + r];
-  }
 
-  // ---- epilogue: accumulator (i, j): lane (r, g) holds C[m0 + 16 FI wm + 16 i + r][n0 + 64 wn + 16 j + 4 g + t], t = 0..3
-  uint4 res[EPI == 2 ? FI : 1][2];
-  if constexpr (EPI == 2) {
-    const int n = cn0 + 64 * wn + 16 * g;
+    // ---- epilogue: accumulator (i, j): lane (r, g) holds C[m0 + 16 FI wm + 16 i + r][n0 + 64 wn + 16 j + 4 g + t], t = 0..3
+    uint4 res[EPI == 2 ? FI : 1][2];
+    if constexpr (EPI == 2) {
+      const int n = cn0 + 64 * wn + 16 * g;
+#pragma unroll
+      for (int i = 0; i < FI; i++) {
+        const int row = cm0 + frow(i) + r;
+        res[i][0] = res[i][1] = uint4{0u, 0u, 0u, 0u};
+        if (row < P.M && n < P.N) {
+          const uint16_t* rp = (const uint16_t*)P.r + (int64_t)row * P.ldr + n;
+          res[i][0] = *(const uint4*)rp;
+          res[i][1] = *(const uint4*)(rp + 8);
+        }
+      }
+    }
 #pragma unroll
     for (int i = 0; i < FI; i++) {
       const int row = cm0 + frow(i) + r;
-      res[i][0] = res[i][1] = uint4{0u, 0u, 0u, 0u};
-      if (row < P.M && n < P.N) {
-        const uint16_t* rp = (const uint16_t*)P.r + (int64_t)row * P.ldr + n;
-        res[i][0] = *(const uint4*)rp;
-        res[i][1] = *(const uint4*)(rp + 8);
+      if (EPI == 1) {
+        // gate slab j, up slab j + 1 -> 4 outputs per slab pair; after the 2 x 2 transpose lane (r, g) holds the 8 consecutive
+        // output columns 16 (g % 2) + 8 (g / 2) .. of the wave's 32
+        uint32_t x0[2], x1[2];
+#pragma unroll
+        for (int jp = 0; jp < 2; jp++) {
+          const gf4 gv = acc[i][2 * jp] * rn[i], uv = acc[i][2 * jp + 1] * rn[i];
+          (jp == 0 ? x0 : x1)[0] = gswiglu2<DT>(gv[0], gv[1], uv[0], uv[1]);
+          (jp == 0 ? x0 : x1)[1] = gswiglu2<DT>(gv[2], gv[3], uv[2], uv[3]);
+        }
+        xpose2(x0[0], x1[0]);
+        xpose2(x0[1], x1[1]);
+        const int n = (cn0 >> 1) + 32 * wn + 16 * (g & 1) + 8 * (g >> 1);   // output column
+        if (row < P.M && 2 * n < P.N) {
+          uint16_t* cp = (uint16_t*)P.c + (int64_t)row * P.ldc + n;
+          *(uint4*)cp = uint4{x0[0], x0[1], x1[0], x1[1]};
+        }
+      } else if (EPI == 3) {   // fp32: 4 columns are 16 bytes, the 4 lane groups of a row store 64 consecutive ones
+        // (the hardware's exponential and reciprocal, with one scale for -x log2(e) / c: over every 16-bit x of the softcap's range 2.40e-8
+        // from 64 bits in the 2-norm and 5.5e-7 at most; an exact quotient, expf and a division, as torch's expression has, 2.42e-8 and 6.4e-7)
+        const float k2 = -1.4426950408889634f / P.cap_c;
+        auto cap = [&](float x) { return P.ca * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f((ground<DT>(x * rn[i]) + P.cb) * k2)); };
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          const int n = cn0 + 64 * wn + 16 * j + 4 * g;
+          if (row < P.M && n < P.N)
+            *(float4*)((float*)P.c + (int64_t)row * P.ldc + n) = float4{cap(acc[i][j][0]), cap(acc[i][j][1]), cap(acc[i][j][2]), cap(acc[i][j][3])};
+        }
+      } else if (EPI == 0) {
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+          // columns 16 (2 s + j) + 4 g .. of fragments j = 0, 1 -> the 8 consecutive columns 32 s + 8 g ..: the 4 lane groups of a row
+          // store 64 consecutive bytes (pieces of 16 bytes 32 apart: 33 216 x 656 x 640 51.9 us, so 49.2)
+          uint32_t x[2][2];
+#pragma unroll
+          for (int j = 0; j < 2; j++) {
+            const gf4 v = acc[i][2 * s + j] * rn[i];
+            x[j][0] = gpack<DT>(v[0], v[1]);
+            x[j][1] = gpack<DT>(v[2], v[3]);
+          }
+          xpose_pair(x[0][0], x[1][0]);
+          xpose_pair(x[0][1], x[1][1]);
+          const int n = cn0 + 64 * wn + 32 * s + 8 * g;
+          if (row < P.M && n < P.N) *(uint4*)((uint16_t*)P.c + (int64_t)row * P.ldc + n) = uint4{x[0][0], x[0][1], x[1][0], x[1][1]};
+        }
+      } else {
+        // (with the stores of EPI 0 here the residual's loads come in the same pieces: 0 - 3 % slower; requested in the last iteration
+        // but one instead of behind the loop, the residual costs 56 registers and 10 % of the K = 1664 product)
+        uint32_t lo[4], hi[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          lo[j] = gpack<DT>(acc[i][j][0] * rn[i], acc[i][j][1] * rn[i]);
+          hi[j] = gpack<DT>(acc[i][j][2] * rn[i], acc[i][j][3] * rn[i]);
+        }
+        xpose4(lo);
+        xpose4(hi);
+        // lane (r, g) now holds columns 16 g .. 16 g + 15 of the wave's 64: words lo[0] hi[0] lo[1] hi[1] ...
+        const int n = cn0 + 64 * wn + 16 * g;
+        if (row < P.M && n < P.N) {
+          uint32_t wds[8] = {lo[0], hi[0], lo[1], hi[1], lo[2], hi[2], lo[3], hi[3]};
+          const uint4 q0 = res[i][0], q1 = res[i][1];
+          const uint32_t rw[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+#pragma unroll
+          for (int e = 0; e < 8; e++) {
+            float p0, p1, x0, x1;
+            gunpack<DT>(wds[e], p0, p1);   // the product, already rounded to the activation type
+            gunpack<DT>(rw[e], x0, x1);
+            wds[e] = gpack<DT>(P.ca * x0 + P.cb * p0, P.ca * x1 + P.cb * p1);
+          }
+          uint16_t* cp = (uint16_t*)P.c + (int64_t)row * P.ldc + n;
+          *(uint4*)cp = uint4{wds[0], wds[1], wds[2], wds[3]};
+          *(uint4*)(cp + 8) = uint4{wds[4], wds[5], wds[6], wds[7]};
+        }
       }
     }
-  }
-#pragma unroll
-  for (int i = 0; i < FI; i++) {
-    const int row = cm0 + frow(i) + r;
-    if (EPI == 1) {
-      // gate slab j, up slab j + 1 -> 4 outputs per slab pair; after the 2 x 2 transpose lane (r, g) holds the 8 consecutive
-      // output columns 16 (g % 2) + 8 (g / 2) .. of the wave's 32
-      uint32_t x0[2], x1[2];
-#pragma unroll
-      for (int jp = 0; jp < 2; jp++) {
-        const gf4 gv = acc[i][2 * jp] * rn[i], uv = acc[i][2 * jp + 1] * rn[i];
-        (jp == 0 ? x0 : x1)[0] = gswiglu2<DT>(gv[0], gv[1], uv[0], uv[1]);
-        (jp == 0 ? x0 : x1)[1] = gswiglu2<DT>(gv[2], gv[3], uv[2], uv[3]);
-      }
-      xpose2(x0[0], x1[0]);
-      xpose2(x0[1], x1[1]);
-      const int n = (cn0 >> 1) + 32 * wn + 16 * (g & 1) + 8 * (g >> 1);   // output column
-      if (row < P.M && 2 * n < P.N) {
-        uint16_t* cp = (uint16_t*)P.c + (int64_t)row * P.ldc + n;
-        *(uint4*)cp = uint4{x0[0], x0[1], x1[0], x1[1]};
-      }
-    } else if (EPI == 3) {   // fp32: 4 columns are 16 bytes, the 4 lane groups of a row store 64 consecutive ones
-      // (the hardware's exponential and reciprocal, with one scale for -x log2(e) / c: over every 16-bit x of the softcap's range 2.40e-8
-      // from 64 bits in the 2-norm and 5.5e-7 at most; an exact quotient, expf and a division, as torch's expression has, 2.42e-8 and 6.4e-7)
-      const float k2 = -1.4426950408889634f / P.cap_c;
-      auto cap = [&](float x) { return P.ca * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f((ground<DT>(x * rn[i]) + P.cb) * k2)); };
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const int n = cn0 + 64 * wn + 16 * j + 4 * g;
-        if (row < P.M && n < P.N)
-          *(float4*)((float*)P.c + (int64_t)row * P.ldc + n) = float4{cap(acc[i][j][0]), cap(acc[i][j][1]), cap(acc[i][j][2]), cap(acc[i][j][3])};
-      }
-    } else if (EPI == 0) {
-#pragma unroll
-      for (int s = 0; s < 2; s++) {
-        // columns 16 (2 s + j) + 4 g .. of fragments j = 0, 1 -> the 8 consecutive columns 32 s + 8 g ..: the 4 lane groups of a row
-        // store 64 consecutive bytes (pieces of 16 bytes 32 apart: 33 216 x 656 x 640 51.9 us, so 49.2)
-        uint32_t x[2][2];
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-          const gf4 v = acc[i][2 * s + j] * rn[i];
-          x[j][0] = gpack<DT>(v[0], v[1]);
-          x[j][1] = gpack<DT>(v[2], v[3]);
-        }
-        xpose_pair(x[0][0], x[1][0]);
-        xpose_pair(x[0][1], x[1][1]);
-        const int n = cn0 + 64 * wn + 32 * s + 8 * g;
-        if (row < P.M && n < P.N) *(uint4*)((uint16_t*)P.c + (int64_t)row * P.ldc + n) = uint4{x[0][0], x[0][1], x[1][0], x[1][1]};
-      }
-    } else {
-      // (with the stores of EPI 0 here the residual's loads come in the same pieces: 0 - 3 % slower; requested in the last iteration
-      // but one instead of behind the loop, the residual costs 56 registers and 10 % of the K = 1664 product)
-      uint32_t lo[4], hi[4];
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        lo[j] = gpack<DT>(acc[i][j][0] * rn[i], acc[i][j][1] * rn[i]);
-        hi[j] = gpack<DT>(acc[i][j][2] * rn[i], acc[i][j][3] * rn[i]);
-      }
-      xpose4(lo);
-      xpose4(hi);
-      // lane (r, g) now holds columns 16 g .. 16 g + 15 of the wave's 64: words lo[0] hi[0] lo[1] hi[1] ...
-      const int n = cn0 + 64 * wn + 16 * g;
-      if (row < P.M && n < P.N) {
-        uint32_t wds[8] = {lo[0], hi[0], lo[1], hi[1], lo[2], hi[2], lo[3], hi[3]};
-        const uint4 q0 = res[i][0], q1 = res[i][1];
-        const uint32_t rw[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-          float p0, p1, x0, x1;
-          gunpack<DT>(wds[e], p0, p1);   // the product, already rounded to the activation type
-          gunpack<DT>(rw[e], x0, x1);
-          wds[e] = gpack<DT>(P.ca * x0 + P.cb * p0, P.ca * x1 + P.cb * p1);
-        }
-        uint16_t* cp = (uint16_t*)P.c + (int64_t)row * P.ldc + n;
-        *(uint4*)cp = uint4{wds[0], wds[1], wds[2], wds[3]};
-        *(uint4*)(cp + 8) = uint4{wds[4], wds[5], wds[6], wds[7]};
-      }
-    }
-  }
-  if (!more) break;
-  L += step;
-  clear();
+    if (!more) break;
+    L += step;
+    clear();
   }
 }
 
