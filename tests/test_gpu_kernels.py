@@ -1300,3 +1300,17 @@ def test_greedy_at_both_widths(dtype, B, V):
     assert float((lp.double() - ref).abs().max()) < 5e-6
     x[0, 3] = float("nan")
     assert int(greedy_sample(x, (23.0, 5.0, 7.5))[0][0]) == int(tok[0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("V", [512, 1536, 8192, 8704, 32768])
+def test_a_greedy_row_does_not_depend_on_the_rows_beside_it(dtype, V):
+    """Token and log-prob of a row, bit for bit, in calls on either side of the width's line and by itself."""
+    from ultraviolet_amd.kernels.fused_sample import greedy_sample
+    g = torch.Generator(device="cuda").manual_seed(V)
+    x = (torch.randn(600, V, device="cuda", generator=g) * 2 - 4).to(dtype)
+    tok, lp = greedy_sample(x, (23.0, 5.0, 7.5))
+    for lo, hi in ((0, 1), (1, 256), (255, 511), (300, 557), (599, 600)):
+        t, p = greedy_sample(x[lo:hi], (23.0, 5.0, 7.5))
+        assert torch.equal(t, tok[lo:hi]) and torch.equal(p, lp[lo:hi]), (lo, hi)

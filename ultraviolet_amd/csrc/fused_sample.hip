@@ -537,27 +537,29 @@ __global__ __launch_bounds__(1024) void sample_filtered_kernel(SampleParams P) {
 // What bounds it: three quarter-rate instructions an element (exp2, reciprocal, exp2) on the compute unit that has the row, behind the
 // launch and a load; with a commit, what that reads.  us with a commit, its reads at the end -> ahead and 1024 threads up to a row per
 // compute unit: 1 row 8.3 -> 7.4, 16 rows 9.2 -> 8.0, 256 rows 10.4 -> 8.9; 640 rows 17.8 -> 16.5, 1024 rows 21.0 -> 19.8.
-// (The last bits of the log-prob's sum of exponentials go with the width; the token does not.)
+// The sum of exponentials is formed in 16 parts - a wave's of 1024 threads - at either width, so a row's log-prob does not depend on how many rows are in the
+// call: 256 threads keep four sums each and add up each part as wave_sum does.  us so at 256 threads, one sum -> four: bf16 300 rows 10.7 -> 10.4, 1024 rows
+// 19.5 -> 18.5, 2048 rows 32.3 -> 31.6; fp32 12.4 -> 12.6, 22.8 -> 23.0, 45.1 -> 45.5.
 template <int DT, int NT>
 __global__ __launch_bounds__(NT) void argmax_kernel(SampleParams P) {
-  constexpr int NW = NT / 64;
+  constexpr int NW = NT / 64, NP = 1024 / NT;
   __shared__ float smax[NW];
   __shared__ int sidx[NW];
-  __shared__ float ssum[NW];
+  __shared__ __attribute__((aligned(16))) float ssum[16];
   const int row = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const char* xr = (const char*)P.x + (int64_t)row * P.stride * (DT == UVMI_F32 ? 4 : 2);
   const int nvec = P.V / 8;
-  float best = -INFINITY, esum = 0.f;
+  float best = -INFINITY, esum[NP] = {};   // esum[p]: vectors threadIdx.x + NT p of every 1024
   int bi = 0x7fffffff;
   CommitRow cr = {};
   if constexpr (NT == 256) cr = commit_ahead(P, row);
-  auto take = [&](const float (&v)[8], int i) {
+  auto take = [&](const float (&v)[8], int i, float& sum) {
 #pragma unroll
     for (int j = 0; j < 8; j++) {
       if (v[j] > best) { best = v[j]; bi = i * 8 + j; }
       // softmax(z) with T = 1: e = exp(z - a)
       const float E = __builtin_amdgcn_exp2f(fmaf(v[j], P.inv_c_l2, P.b_over_c_l2));
-      esum += __builtin_amdgcn_exp2f(-P.cap_a * 1.4426950408889634f * __builtin_amdgcn_rcpf(1.0f + E));
+      sum += __builtin_amdgcn_exp2f(-P.cap_a * 1.4426950408889634f * __builtin_amdgcn_rcpf(1.0f + E));
     }
   };
   if constexpr (NT == 1024) {   // (at most four vectors a thread: all requested at once)
@@ -568,26 +570,55 @@ __global__ __launch_bounds__(NT) void argmax_kernel(SampleParams P) {
     cr = commit_ahead(P, row);
 #pragma unroll
     for (int q = 0; q < 4; q++)
-      if (threadIdx.x + 1024 * q < nvec) take(v[q], threadIdx.x + 1024 * q);
+      if (threadIdx.x + 1024 * q < nvec) take(v[q], threadIdx.x + 1024 * q, esum[0]);
   } else {
-    for (int i = threadIdx.x; i < nvec; i += NT) {
+    auto one = [&](int i, float& sum) {
       float v[8];
       load8<DT>(xr, i, v);
-      take(v, i);
+      take(v, i, sum);
+    };
+    int i0 = 0;
+    for (; i0 + 1024 <= nvec; i0 += 1024) {
+#pragma unroll
+      for (int p = 0; p < NP; p++) {
+        one(i0 + NT * p + threadIdx.x, esum[p]);
+        // (16-bit rows request all four at once: 640 rows 16.0 -> 14.5 us; fp32 ones lose by it, 800 rows 19.6 -> 22.1)
+        if (DT == UVMI_F32) __builtin_amdgcn_sched_barrier(0);
+      }
     }
+#pragma unroll
+    for (int p = 0; p < NP; p++)
+      if (i0 + NT * p + (int)threadIdx.x < nvec) one(i0 + NT * p + threadIdx.x, esum[p]);
   }
   for (int o = 32; o > 0; o >>= 1) {
     const float ob = __shfl_xor(best, o, 64);
     const int oi = __shfl_xor(bi, o, 64);
     if (ob > best || (ob == best && oi < bi)) { best = ob; bi = oi; }
   }
-  esum = wave_sum(esum);
-  if (lane == 0) { smax[wave] = best; sidx[wave] = bi; ssum[wave] = esum; }
+  if constexpr (NP == 1) {
+    esum[0] = wave_sum(esum[0]);
+    if (lane == 0) ssum[wave] = esum[0];
+  } else {   // wave_sum of the four at once: a swap adds the halves of two sums; rows 0 .. 3 of 16 lanes end with those of p = 0, 2, 1, 3
+    auto fold = [](auto r) { return __uint_as_float(r[0]) + __uint_as_float(r[1]); };
+    const float a = fold(__builtin_amdgcn_permlane32_swap(__float_as_uint(esum[0]), __float_as_uint(esum[1]), false, false));
+    const float b = fold(__builtin_amdgcn_permlane32_swap(__float_as_uint(esum[2]), __float_as_uint(esum[3]), false, false));
+    float e = fold(__builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false));
+    e += lane_xor8(e);
+    e += lane_xor4(e);
+    e += lane_xor2(e);
+    e += lane_xor1(e);
+    if (lane % 16 == 0) ssum[wave + NW * ((lane >> 5) + 2 * ((lane >> 4) & 1))] = e;
+  }
+  if (lane == 0) { smax[wave] = best; sidx[wave] = bi; }
   __syncthreads();
   if (threadIdx.x == 0) {
     float tot = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+      const float4 x = ((const float4*)ssum)[w];
+      tot = tot + x.x + x.y + x.z + x.w;
+    }
     for (int w = 0; w < NW; w++) {
-      tot += ssum[w];
       if (smax[w] > best || (smax[w] == best && sidx[w] < bi)) { best = smax[w]; bi = sidx[w]; }
     }
     const float E = __builtin_amdgcn_exp2f(fmaf(best, P.inv_c_l2, P.b_over_c_l2));
@@ -650,8 +681,8 @@ extern "C" int uvmi_fused_sample(const uvmi_sample_args* a, void* stream) {
   const bool filtered = !greedy && (P.top_k > 0 || P.top_p < 1.0f);
   hipStream_t st = (hipStream_t)stream;
   // Drawing, 1024 threads per row are faster up to ~640 rows (12.0 against 14.5 us at 384 rows), slower from 1024 on; its sums are formed per
-  // chunk whatever the width, so the draw does not depend on it.  Greedy, up to a row per compute unit (256 rows 8.4 against 8.7,
-  // 300 rows 12.9 against 10.8).
+  // chunk whatever the width, so the draw does not depend on it.  Greedy, whose sums do not either, up to a row per compute unit (256
+  // rows 8.4 against 8.7, 300 rows 12.9 against 10.8).
   int cus = uvmi_device_cus();
   if (cus <= 0) cus = 256;
   const bool wide = filtered || a->B <= (greedy ? cus : 640);
