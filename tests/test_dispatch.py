@@ -1,5 +1,8 @@
 """Which calls of decode_attention may launch past the dispatcher: those that no transform, mode, tracer or gradient sees.
 No GPU: the launch and the registered op are replaced by recorders."""
+import ctypes
+import subprocess
+
 import pytest
 import torch
 from torch.utils._python_dispatch import TorchDispatchMode
@@ -124,3 +127,54 @@ def test_native_path_leaves_other_calls_to_the_general_one():
     idx = torch.zeros(2, dtype=torch.long)
     assert D.L.eager().decode_attention(q, k, v, None, None, idx, idx, None, 0.1, 0, None, None, 1, False, 0) is None
     assert D.L.eager().decode_attention(q, k, 3, None, None, idx, None, None, 0.1, 0, None, None, 1, False, 0) is None
+
+
+def test_native_path_of_another_build_is_not_loaded(monkeypatch, tmp_path):
+    """The extension is looked for under the interpreter's and torch's versions, refused when it was built for another revision of the
+    argument structs or calls a library of one, and where there is none the general path takes every call."""
+    import sysconfig
+    L = D.L
+    q, k, v = _qkv()
+    idx = torch.zeros(2, dtype=torch.long)
+    assert sysconfig.get_config_var("SOABI") in L.EAGER_PATH and torch.__version__ in L.EAGER_PATH
+    mod = L.eager()
+    assert mod.revision == mod.library_revision == L.ABI_VERSION and mod.attn_args_bytes == ctypes.sizeof(L.AttnArgs)
+
+    def none_of_it(words):
+        monkeypatch.setattr(L, "_eager", None)
+        with pytest.raises(L.UvmiError, match=words):
+            L.eager()
+        D._native.cache_clear()
+        with pytest.warns(UserWarning, match=words):
+            native = D._native()
+        D._native.cache_clear()
+        assert native(q, k, v, None, None, idx, idx, None, 0.1, 0, None, None, 1, False, 0) is None
+    with monkeypatch.context() as m:
+        m.setattr(L, "ABI_VERSION", L.ABI_VERSION + 1)
+        none_of_it("revision")
+    with monkeypatch.context() as m:
+        m.setattr(L, "AttnArgs", L.SampleArgs)
+        none_of_it("revision")
+    with monkeypatch.context() as m:
+        m.setattr(L, "EAGER_PATH", str(tmp_path / "none.so"))
+        none_of_it("not found")
+    with monkeypatch.context() as m:
+        (tmp_path / "other.so").write_bytes(b"not a library")
+        m.setattr(L, "EAGER_PATH", str(tmp_path / "other.so"))
+        none_of_it("does not load")
+
+
+def test_library_is_built_where_the_extension_cannot_be(monkeypatch, tmp_path, capsys):
+    """A compiler or headers that are missing cost the extension only, and an older one does not stay."""
+    from ultraviolet_amd.csrc import build as B
+    old = tmp_path / "eager.so"
+    old.write_bytes(b"older")
+    monkeypatch.setattr(D.L, "EAGER_PATH", str(old))
+
+    def run(cmd):
+        raise RuntimeError("no such header")
+    B._build_eager(run, True, True)
+    assert not old.exists() and "no such header" in capsys.readouterr().err
+    monkeypatch.setenv("CXX", str(tmp_path / "no-compiler"))
+    B._build_eager(lambda cmd: subprocess.run(cmd, check=True), True, True)
+    assert "no-compiler" in capsys.readouterr().err

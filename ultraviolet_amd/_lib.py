@@ -5,6 +5,7 @@ from __future__ import annotations
 import ctypes as C
 import importlib.util
 import os
+import sysconfig
 
 import torch
 
@@ -217,19 +218,28 @@ def lib() -> C.CDLL:
 
 
 _eager = None
+# (named after the interpreter and the torch that it is built for: it uses the structs of both)
+EAGER_PATH = os.path.join(_HERE, "csrc", f"uvmi_eager.{sysconfig.get_config_var('SOABI')}.torch-{torch.__version__}.so")
 
 
 def eager():
-    """The extension module of csrc/eager.cpp, loaded once, behind libuvmi.so (which it calls).  Raises UvmiError when it is missing."""
+    """The extension module of csrc/eager.cpp, loaded once, behind libuvmi.so (which it calls).  Raises UvmiError where there is none for this
+    interpreter and torch, or one of another revision of include/uvmi.h."""
     global _eager
     if _eager is None:
         lib()
-        path = os.path.join(_HERE, "csrc", "uvmi_eager.so")
-        if not os.path.exists(path):
-            raise UvmiError(f"{path} not found: run `python -m ultraviolet_amd.csrc.build` (no CPU fallback)")
-        spec = importlib.util.spec_from_file_location("uvmi_eager", path)
-        mod = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(mod)
+        if not os.path.exists(EAGER_PATH):
+            raise UvmiError(f"{EAGER_PATH} not found: run `python -m ultraviolet_amd.csrc.build`")
+        spec = importlib.util.spec_from_file_location("uvmi_eager", EAGER_PATH)
+        try:
+            mod = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(mod)
+        except ImportError as e:
+            raise UvmiError(f"{EAGER_PATH} does not load: {e}") from e
+        # (it fills the argument structs itself, and calls whichever libuvmi.so the loader found for it)
+        if not (mod.revision == mod.library_revision == ABI_VERSION and mod.attn_args_bytes == C.sizeof(AttnArgs)):
+            raise UvmiError(f"{EAGER_PATH} was built for revision {mod.revision} of include/uvmi.h and calls a library of revision {mod.library_revision}, these "
+                            f"bindings are for {ABI_VERSION}: rebuild it with `python -m ultraviolet_amd.csrc.build`")
         _eager = mod
     return _eager
 

@@ -184,5 +184,10 @@ PyMODINIT_FUNC PyInit_uvmi_eager() {
   if (!c) return nullptr;
   raw_stream_fn = PyObject_GetAttrString(c, "_cuda_getCurrentRawStream");
   if (!raw_stream_fn) return nullptr;
-  return PyModule_Create(&module);
+  THPObjectPtr m(PyModule_Create(&module));
+  // what the loader compares with its own: the revision and layout this was built for, and the revision of the library it calls
+  if (!m || PyModule_AddIntConstant(m.get(), "revision", UVMI_ABI_VERSION) || PyModule_AddIntConstant(m.get(), "library_revision", uvmi_version()) ||
+      PyModule_AddIntConstant(m.get(), "attn_args_bytes", sizeof(uvmi_attn_args)))
+    return nullptr;
+  return m.release();
 }

@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import ctypes as C
 import functools
+import warnings
 
 import torch
 from torch import Tensor
@@ -50,8 +51,13 @@ def plain_eager(q: Tensor, k: Tensor, v: Tensor, k_scale: Tensor | None, v_scale
 
 @functools.lru_cache(maxsize=None)
 def _native():
-    """decode_attention of csrc/eager.cpp."""
-    mod = L.eager()
+    """decode_attention of csrc/eager.cpp; where that was not built for this interpreter, torch and library, what hands every call on to
+    the general path below, which launches the same kernels."""
+    try:
+        mod = L.eager()
+    except L.UvmiError as e:
+        warnings.warn(f"decode_attention: eager calls are prepared in Python, which takes longer than a small launch ({e})", stacklevel=3)
+        return lambda *call: None
     mod.bind(_device_cus)
     return mod.decode_attention
 
