@@ -1045,7 +1045,7 @@ def test_gemm_softcap_epilogue(dtype, M, N, K, norm, config):
 @pytest.mark.parametrize("form", ["plain", "indices32", "mixed indices", "rows", "views", "q4", "ring", "splits", "chunks", "fp32 out", "scale int", "inference"])
 def test_native_call_equals_the_general_one(monkeypatch, dtype, int8, form):
     """decode_attention's native path (csrc/eager.cpp) and the general one launch the same kernel on the same arguments: equal bits
-    over the forms a call may take, those that the native path hands on among them."""
+    over the forms a call may take.  Three of them the native path hands on; the others it serves itself."""
     from ultraviolet_amd.kernels import decode_attn as D
     B, H, S = 9, 8, 320
     q, k, v, ks, vs = (None if t is None else t.to(DEV) for t in attn_case(B, 1, H, 64, S, int8, dtype=torch.float16))
@@ -1079,11 +1079,35 @@ def test_native_call_equals_the_general_one(monkeypatch, dtype, int8, form):
         kw.update(out_fp32=True)
     elif form == "scale int":
         scale = 1
+    o = dict(dict(rows=None, window=0, ring=None, ctx_hint=None, num_splits=None, out_fp32=False, chunk_keys=0, k_scale=None, v_scale=None), **kw)
     with torch.inference_mode(form == "inference"):
+        native = D._native()(q, k, v, o["k_scale"], o["v_scale"], pos, starts, o["rows"], scale, o["window"], o["ring"], o["ctx_hint"], o["num_splits"], o["out_fp32"], o["chunk_keys"])
         got = D.decode_attention(q, k, v, pos, starts, scale, **kw)
         monkeypatch.setattr(D, "_native", lambda: lambda *a: None)
         want = D.decode_attention(q, k, v, pos, starts, scale, **kw)
     assert got.dtype == want.dtype and got.shape == want.shape and torch.equal(got, want)
+    if form in ("mixed indices", "q4", "scale int"):
+        assert native is None
+    else:
+        assert type(native) is torch.Tensor and native.dtype == want.dtype and torch.equal(native, want)
+
+
+@pytest.mark.parametrize("kw", [dict(), dict(num_splits=3), dict(out_fp32=True)])
+def test_eager_calls_go_through_the_native_path(monkeypatch, kw):
+    """Of decode_attention's two ways a plain call takes the native one: with the other taken away it is served, with either gone not."""
+    from ultraviolet_amd.kernels import decode_attn as D
+    q, k, v, ks, vs = (t.to(DEV) for t in attn_case(3, 1, 8, 64, 64, True))
+    pos, starts = torch.full((3,), 5, device=DEV), torch.zeros(3, dtype=torch.long, device=DEV)
+    want = D.decode_attention(q, k, v, pos, starts, 0.1, k_scale=ks, v_scale=vs, **kw)
+
+    def unreached(*a, **k):
+        raise AssertionError("the general path was taken")
+    monkeypatch.setattr(D, "_launch", unreached)
+    monkeypatch.setattr(D, "_decode_attn_op", unreached)
+    assert torch.equal(D.decode_attention(q, k, v, pos, starts, 0.1, k_scale=ks, v_scale=vs, **kw), want)
+    monkeypatch.setattr(D, "_native", lambda: lambda *a: None)
+    with pytest.raises(AssertionError, match="general path"):
+        D.decode_attention(q, k, v, pos, starts, 0.1, k_scale=ks, v_scale=vs, **kw)
 
 
 def test_native_call_refuses_what_the_general_one_refuses(monkeypatch):
