@@ -277,6 +277,15 @@ def test_attention_and_backward_at_the_mask_rules(window):
         assert np.abs(a - b).max() <= 2 * ulp * np.abs(b).max() + 1e-6, (np.abs(a - b).max(), np.abs(b).max())
 
 
+@pytest.mark.parametrize("window", [33, 167, 168, 2 ** 31 - 1])
+def test_plain_backward_with_windows_that_hide_few_keys_and_none(window):
+    """16 query heads on a kv head, which the plain kernels serve: windows up to the largest that an int holds.  Tolerance as above."""
+    got, ref = _grad_case([131, 37], 16, 1, torch.float16, window, seed=6)
+    for a, b in zip(got, ref):
+        assert np.isfinite(a).all()
+        assert np.abs(a - b).max() <= 2 * 2.0 ** -10 * np.abs(b).max() + 1e-6, (np.abs(a - b).max(), np.abs(b).max())
+
+
 def test_backward_rejects_what_it_cannot_do():
     from ultraviolet_amd import _lib as L
     from ultraviolet_amd.kernels.varlen_attn import packed_attention_backward

@@ -711,6 +711,7 @@ extern "C" int uvmi_prefill_attn_bwd(const uvmi_prefill_attn_bwd_args* a, void* 
   for (const void* p : ptrs) UVMI_REQUIRE(((uintptr_t)p % 16) == 0, UVMI_EINVAL, "uvmi_prefill_attn_bwd: tensors must be 16-byte aligned");
   UVMI_REQUIRE(a->workspace && ((uintptr_t)a->workspace % 16) == 0 && a->workspace_bytes >= uvmi_prefill_attn_bwd_workspace_bytes(a->N, a->H),
                UVMI_EWORKSPACE, "uvmi_prefill_attn_bwd: workspace of %zu bytes needed", uvmi_prefill_attn_bwd_workspace_bytes(a->N, a->H));
+  const int window = a->window < a->N ? a->window : 0;   // (a window of all tokens hides none; the kernels add it to an index)
   hipStream_t st = (hipStream_t)stream;
   const int64_t ls = bwd_row_stride(a->N);
   float* lse = (float*)a->workspace;
@@ -724,7 +725,7 @@ extern "C" int uvmi_prefill_attn_bwd(const uvmi_prefill_attn_bwd_args* a, void* 
     f.q = a->q; f.q_dtype = a->dtype; f.sqn = (int64_t)a->H * 64; f.sqh = 64;
     f.k = a->k; f.v = a->v; f.kv_dtype = a->dtype; f.skn = f.svn = (int64_t)a->KH * 64; f.skh = f.svh = 64;
     f.cu_seqlens = a->cu_seqlens; f.idx_dtype = a->idx_dtype; f.n_seg = a->n_seg;
-    f.N = a->N; f.H = a->H; f.KH = a->KH; f.hd = a->hd; f.scale = a->scale; f.window = a->window;
+    f.N = a->N; f.H = a->H; f.KH = a->KH; f.hd = a->hd; f.scale = a->scale; f.window = window;
     UVMI_REQUIRE(a->scale > 0.f, UVMI_EUNSUPPORTED, "uvmi_prefill_attn_bwd: scale must be positive");
     const float* stats = lse;
     int64_t stats_ld = ls;
@@ -743,8 +744,7 @@ extern "C" int uvmi_prefill_attn_bwd(const uvmi_prefill_attn_bwd_args* a, void* 
     M.q = a->q; M.k = a->k; M.v = a->v; M.o = a->o; M.go = a->go; M.dq = a->dq; M.dk = a->dk; M.dv = a->dv;
     M.lse = stats; M.lse_ld = stats_ld; M.dsum = dsum; M.ls = ls; M.seg_start = seg_start;
     M.cu = a->cu_seqlens; M.idx64 = a->idx_dtype == UVMI_I64 ? 1 : 0; M.n_seg = a->n_seg;
-    M.N = a->N; M.H = a->H; M.KH = a->KH; M.G = G; M.window = a->window < a->N ? a->window : 0;   // (a window of all tokens hides none)
-   
+    M.N = a->N; M.H = a->H; M.KH = a->KH; M.G = G; M.window = window;
     M.scale = a->scale; M.scale_log2 = a->scale * 1.4426950408889634f;
     M.n_wg = ((a->N + 15) / 16) * a->KH;
     const dim3 blk4(256), gq((unsigned)((M.n_wg + 7) / 8 * 8));
@@ -764,7 +764,7 @@ extern "C" int uvmi_prefill_attn_bwd(const uvmi_prefill_attn_bwd_args* a, void* 
   P.lse = lse;
   P.dsum = P.lse + (size_t)a->N * a->H;
   P.cu = a->cu_seqlens; P.idx64 = a->idx_dtype == UVMI_I64 ? 1 : 0; P.n_seg = a->n_seg; P.N = a->N; P.H = a->H; P.KH = a->KH; P.G = a->H / a->KH;
-  P.window = a->window; P.scale = a->scale;
+  P.window = window; P.scale = a->scale;
   const dim3 blk(64), g1((unsigned)((a->N + 63) / 64), (unsigned)a->H), g2((unsigned)((a->N + 31) / 32), (unsigned)a->KH);
   if (a->dtype == UVMI_F16) hipLaunchKernelGGL((bwd_dq_kernel<UVMI_F16>), g1, blk, 0, st, P);
   else hipLaunchKernelGGL((bwd_dq_kernel<UVMI_BF16>), g1, blk, 0, st, P);
