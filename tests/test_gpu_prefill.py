@@ -286,6 +286,23 @@ def test_plain_backward_with_windows_that_hide_few_keys_and_none(window):
         assert np.abs(a - b).max() <= 2 * 2.0 ** -10 * np.abs(b).max() + 1e-6, (np.abs(a - b).max(), np.abs(b).max())
 
 
+def test_backward_from_statistics_of_a_wide_pitch():
+    """The forward's statistics as rows of a larger array, 8 of them within 32-bit byte offsets and beyond: the bits of the call whose rows are
+    close together."""
+    from ultraviolet_amd.kernels.varlen_attn import packed_attention, packed_attention_backward, statistics_pitch
+    from ultraviolet_amd import _lib as L
+    q, k, v, cu = (t.to(DEV) for t in _case([131, 37], 8, 1, 64, torch.bfloat16, seed=7))
+    go = torch.randn(q.shape, device=DEV, generator=torch.Generator(device=DEV).manual_seed(8)).to(q.dtype)
+    N, grads = q.size(0), []
+    ws = torch.empty(L.lib().uvmi_prefill_attn_workspace_bytes(N), dtype=torch.uint8, device=DEV)
+    for pitch in (statistics_pitch(N), 1 << 20, 160_000_000):
+        lse = torch.empty(7 * pitch + statistics_pitch(N), device=DEV).as_strided((8, statistics_pitch(N)), (pitch, 1))
+        o = packed_attention(q, k, v, cu, SC, 100, workspace=ws, lse_out=lse)
+        grads.append(packed_attention_backward(go, q, k, v, o, cu, SC, 100, saved=(lse, ws)))
+    for other in grads[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(grads[0], other))
+
+
 def test_backward_rejects_what_it_cannot_do():
     from ultraviolet_amd import _lib as L
     from ultraviolet_amd.kernels.varlen_attn import packed_attention_backward

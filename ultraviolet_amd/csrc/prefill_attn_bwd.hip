@@ -733,6 +733,9 @@ extern "C" int uvmi_prefill_attn_bwd(const uvmi_prefill_attn_bwd_args* a, void* 
     if (a->lse) {   // the forward kept them: no pass of its own (43 us of 290 for forward and backward of 31 700 tokens)
       UVMI_REQUIRE(a->fwd_workspace && ((uintptr_t)a->lse % 16) == 0 && a->lse_stride >= a->N + 32 && a->lse_stride % 4 == 0, UVMI_EINVAL,
                    "uvmi_prefill_attn_bwd: lse must be 16-byte aligned with a pitch of at least N + 32 that is a multiple of 4, beside fwd_workspace");
+    }
+    // (bwd_dkv_mfma reaches the statistics by 32-bit offsets: those of a wider pitch are formed again)
+    if (a->lse && a->lse_stride < (1LL << 29) / a->H) {
       stats = a->lse;
       stats_ld = a->lse_stride;
       seg_start = (const int32_t*)a->fwd_workspace;
