@@ -171,7 +171,7 @@ __global__ __launch_bounds__(64) void bwd_dkv_kernel(BwdParams P) {
   const int j = blockIdx.x * 32 + jj;
   int n_end = (int)load_index(P.cu, P.idx64, P.n_seg);
   n_end = n_end < 0 ? 0 : (n_end > P.N ? P.N : n_end);
-  const bool live = j < n_end;
+  const bool live = j < n_end && j >= (int)load_index(P.cu, P.idx64, 0);   // (in a sequence)
   int lo = 0x7fffffff, hi = 0;   // queries lo .. hi - 1 see key j
   if (live) {
     int se = (int)load_index(P.cu, P.idx64, segment_of(P, j) + 1);
@@ -487,6 +487,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const float c = P.scale_log2;
   int n_end = (int)load_index(P.cu, P.idx64, P.n_seg);
   n_end = n_end < 0 ? 0 : (n_end > P.N ? P.N : n_end);
+  const int n_beg = (int)load_index(P.cu, P.idx64, 0);   // no query sees a key ahead of it
   const int jw0 = kb * 64, jw_last = min(jw0 + 63, n_end - 1);
   const int jw = jw0 + 32 * kg;             // the wave's first key
   const int key0 = jw + n;                  // column block b: key0 + 16 b
@@ -566,11 +567,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int b = 0; b < 2; b++) {
       if (P.window > 0) hi_q[b] = min(hi_q[b], key0 + 16 * b + P.window);
-      if (key0 + 16 * b < n_end) n_q[b] = (uint32_t)(hi_q[b] - key0 - 16 * b);
+      if (key0 + 16 * b < n_end && key0 + 16 * b >= n_beg) n_q[b] = (uint32_t)(hi_q[b] - key0 - 16 * b);
     }
   }
   // no mask in a query tile that starts in full_from .. full_to: every query follows every key of the wave, in the first key's sequence and window
-  const int full_from = jw + 31, full_to = (P.window > 0 ? min(first_end, jw + P.window) : first_end) - 32;
+  // (nowhere for a wave whose first keys lie ahead of the first sequence)
+  const int full_from = jw + 31, full_to = jw < n_beg ? -1 : (P.window > 0 ? min(first_end, jw + P.window) : first_end) - 32;
   const int n_it = jw0 < n_end ? ((qend - jw0 + 31) >> 5) * GP : 0;
   int c_t = 0, c_p = 0;   // tile and head pair of the next arithmetic
   const TileReads at(n, g);
