@@ -1035,6 +1035,20 @@ def test_states_and_engines_are_copied_pickled_and_freed_after_use(plan):
     assert torch.isfinite(eng.decode_step(tok, states[0]).float()).all()
 
 
+def test_an_engine_saved_before_a_setting_existed_goes_on():
+    """Without the row count of the projection that rides in the attention launch, the engine takes the launches it took."""
+    from ultraviolet_amd.engine import KVState, UVEngine
+    cfg, _, eng, _ = _setup(dtype=torch.bfloat16, window=64)
+    saved = eng.__getstate__()
+    del saved["oproj_rows"]
+    old = UVEngine.__new__(UVEngine)
+    old.__setstate__(saved)
+    st, tok = [KVState(cfg, 3, 50, DEV) for _ in range(2)], torch.tensor([5, 9, 2], device=DEV)
+    assert old._pass_kind(3, True, st[0]) == "lean" and eng._pass_kind(3, True, st[0]) == "lean-o"
+    a, b = (e.decode_step(tok, s).clone() for e, s in zip((old, eng), st))
+    assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("dtype,kv", [(torch.bfloat16, "int8"), (torch.bfloat16, "fp16"), (torch.float32, "int8")])
 def test_a_refused_single_prompt_leaves_the_state_alone(dtype, kv):
     """prefill of one prompt that does not fill its row raises, whichever way its start is off, and cache row, scales, pos, starts and

@@ -206,7 +206,7 @@ class UVEngine:
         return {k: v for k, v in self.__dict__.items() if k not in ("_stage", "_stage_at", "_plans", "_rec")}
 
     def __setstate__(self, d):
-        self.__dict__.update(d)
+        self.__dict__.update({"oproj_rows": 0, **d})   # (an engine saved before it had them: five launches a layer, as it ran then)
         self._new_scratch()
 
     # ------------------------------------------------------------------------------------------------ kernels
