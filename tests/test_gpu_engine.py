@@ -121,8 +121,8 @@ def test_greedy_64_tokens_identical_fp32(name, over):
 
 # the decode pass's launch plans by row count, forced here at a few rows:
 # (skinny_rows, fold_qkv_rows, fold_o_rows, fold_gu_rows, form of the hand-written GEMM: 4 the streaming one's 64 x 64 tiles, 3 the
-# 128 x 128 tiles through registers)
-_TRUNK_PLANS = {"small": None, "large-skinny-attn-block": (0, 1 << 30, 1 << 30, 0, 0), "large-library": (0, 0, 0, 0, 0),
+# 128 x 128 tiles through registers); "small" has the output projection in the attention launch, "small-five-launches" has one of its own
+_TRUNK_PLANS = {"small": None, "small-five-launches": (192, 1 << 30, 1 << 30, 1 << 30, 0, (0, 5120), 0), "large-skinny-attn-block": (0, 1 << 30, 1 << 30, 0, 0), "large-library": (0, 0, 0, 0, 0),
                 "large-tiled-64": (0, 1 << 30, 1 << 30, 1 << 30, 4), "large-tiled-128": (0, 1 << 30, 1 << 30, 1 << 30, 3),
                 "large-tiled-64-own-down": (0, 1 << 30, 1 << 30, 1 << 30, 4, (0, 1 << 30))}
 
@@ -133,22 +133,30 @@ def _force_plan(eng, plan):
         eng.general_skinny_rows = eng.skinny_rows
         if len(_TRUNK_PLANS[plan]) > 5:   # the down projection on this library's tiled GEMM too
             eng.fold_down_rows = _TRUNK_PLANS[plan][5]
+        if len(_TRUNK_PLANS[plan]) > 6:
+            eng.oproj_rows = _TRUNK_PLANS[plan][6]
+
+
+_KINDS = {"small": "lean-o", "small-five-launches": "lean"}   # (the others: "folded")
 
 
 @pytest.mark.parametrize("dtype,max_bar,mean_bar", [(torch.bfloat16, 0.15, 0.02), (torch.float16, 0.04, 0.005)])
 @pytest.mark.parametrize("plan", list(_TRUNK_PLANS))
-def test_16bit_engine_close_to_oracle(plan, dtype, max_bar, mean_bar):
+@pytest.mark.parametrize("window", [16, 32])
+def test_16bit_engine_close_to_oracle(window, plan, dtype, max_bar, mean_bar):
     """The 16-bit engine against the oracle run in the same 16-bit arithmetic (both sides use the int8 cache and round at
     the same points), for each of the decode pass's launch plans (the one for few rows, and the two for many rows:
     residual updates inside the projections, the MLP's pre-norm inside the SwiGLU launch).  Bars: twice the measured gap -
     bf16 max 0.062-0.077 / mean 0.0099, fp16 max 0.016-0.020 / mean 0.0026 on logits in (0, 23), i.e. one or two units in
     the last place of the tied head's 16-bit output; every argmax agrees.  (The reference's bar for its int8 kernel path
-    against its unquantized SDPA path is 0.25 / 0.9, tests/test_math_kernels.py:170-172.)"""
-    cfg, params, eng, OracleModel = _setup(dtype=dtype, window=16)
+    against its unquantized SDPA path is 0.25 / 0.9, tests/test_math_kernels.py:170-172.)  On rings of 16 slots, too short for the
+    fused attention, the settings reach the plain plan's projections."""
+    cfg, params, eng, OracleModel = _setup(dtype=dtype, window=window)
     _force_plan(eng, plan)
     prompts = _prompts(cfg, (5, 12, 9, 20, 3, 17))
     cont = np.random.default_rng(1).integers(1, cfg.vocab_size, size=(6, 30))
-    lg, _ = _teacher_forced(eng, prompts, cont, 64)
+    lg, st = _teacher_forced(eng, prompts, cont, 64)
+    assert eng._pass_kind(len(prompts), True, st) == ("plain" if window == 16 else _KINDS.get(plan, "folded"))
     ref, _ = _oracle_teacher_forced(OracleModel(cfg, params, dtype), prompts, cont, 64)
     assert np.isfinite(lg).all()
     d = np.abs(lg - ref)
@@ -434,9 +442,9 @@ def test_fused_qkv_decode_matches_unfused(dtype, name, over):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("plan", ["large-skinny-attn-block", "large-library", "large-tiled-64", "large-tiled-128", "large-tiled-64-own-down"])
+@pytest.mark.parametrize("plan", ["large-skinny-attn-block", "large-library", "large-tiled-64", "large-tiled-128", "large-tiled-64-own-down", "small-five-launches"])
 def test_large_pass_plans_match_unfused(dtype, plan):
-    """The launch plans of passes with many rows (forced here at 6 rows) against the unfused general path, to the same
+    """The launch plans of passes with more rows (forced here at 6 rows) against the unfused general path, to the same
     bounds as the small-pass plan above."""
     cfg, params, eng, _ = _setup("uv-50m-alpha", dtype=dtype, perturb=0.05)
     _force_plan(eng, plan)
@@ -1033,6 +1041,35 @@ def test_states_and_engines_are_copied_pickled_and_freed_after_use(plan):
     finally:
         gc.enable()
     assert torch.isfinite(eng.decode_step(tok, states[0]).float()).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("kv_dtype", ["int8", "fp16"])
+def test_steps_with_the_output_projection_in_the_attention_launch_equal_those_without(kv_dtype, dtype):
+    """decode_step of up to 32 rows leaves the output projection to the attention launch; with oproj_rows=0 it is a launch of its own.  Equal
+    hiddens and caches, bit for bit, step after step on one state each: recorded passes bound to other row counts, steps
+    on either side of the line, and the sampled steps of a rollout, padding rows among them."""
+    from ultraviolet_amd.engine import KVState, UVEngine
+    cfg, _, eng, _ = _setup("uv-50m-alpha", dtype=dtype, perturb=0.05)
+    two = UVEngine(eng.w, max_tokens=2048, oproj_rows=0)
+    B = 40
+    sts = [KVState(cfg, B, 320, DEV, kv_dtype=kv_dtype, dtype=dtype) for _ in range(2)]
+    prompts = _prompts(cfg, [3, 290, 31, 32, 33, 260] + [7] * (B - 6), seed=2)
+    for e, st in zip((eng, two), sts):
+        e.prefill(prompts, list(range(B)), st)
+    rng = np.random.default_rng(3)
+    for n in (1, 32, 33, 8, 9, 25, 32, 40, 1, 32):
+        assert [e._pass_kind(n, True, sts[0]) for e in (eng, two)] == ["lean-o" if n <= 32 else "lean", "lean"]
+        tok = torch.from_numpy(rng.integers(1, cfg.vocab_size, size=n)).to(DEV)
+        a, b = (e.decode_step(tok, st).clone() for e, st in zip((eng, two), sts))
+        assert torch.equal(a, b) and bool(torch.isfinite(a.float()).all()), n
+        assert all(torch.equal(x, y) for x, y in zip(sts[0].k + sts[0].v + [sts[0].pos], sts[1].k + sts[1].v + [sts[1].pos])), n
+    rows = torch.tensor([4, -1, 0, 39, 17, -1], device=DEV)
+    pos, starts = (t[rows.clamp(min=0)].clone() for t in (sts[0].pos, sts[0].starts))
+    tok = torch.arange(6, device=DEV) + 3
+    a, b = (e._trunk(tok, pos, 6, None, rows=rows, st=st, fused_attn=lambda l, oproj=False, e=e, st=st: e.fused_cache_attention(l, tok, st, pos, starts, 6, rows=rows, oproj=oproj)).clone()
+            for e, st in zip((eng, two), sts))
+    assert torch.equal(a, b) and all(torch.equal(x, y) for x, y in zip(sts[0].k + sts[0].v, sts[1].k + sts[1].v))
 
 
 def test_an_engine_saved_before_a_setting_existed_goes_on():
