@@ -214,7 +214,7 @@ int uvmi_decode_attn_noalloc(const uvmi_attn_args* a, void* stream);
  * fused inference path (ultraviolet/model.py:302-335 attention projections, 388-391 MLP).  K % 64 == 0, K <= 8192;
  * N % 16 == 0.  Three kernel families behind one entry point:
  *   - a streaming form for steps of up to a few thousand rows, where round trips to memory are the time: tiles of 16 x 16 to
- *     64 x 64, the workgroup's waves split K and pull their slabs straight into LDS without a barrier between them;
+ *     64 x 96, the workgroup's waves split K and pull their slabs straight into LDS without a barrier between them;
  *   - a form whose slabs go from global memory straight into LDS, with operand reads pipelined ahead of the MFMAs and
  *     whole-line stores: 256 x 256 tiles (128 x 64 per wave) for the passes of many thousand rows - a packed prefill, a
  *     mixed prefill + decode pass - where L2 and LDS bandwidth per flop decide, and 128 x 128 tiles in between;
@@ -253,6 +253,12 @@ typedef struct uvmi_gemm_args {
   float cap_c;                             /* SOFTCAP: the cap is ca * sigmoid((x + cb) / cap_c) */
 } uvmi_gemm_args;
 int uvmi_gemm_tn_ex(const uvmi_gemm_args* a, void* stream);
+/* Which kernel uvmi_gemm_tn_ex takes for these arguments (UVMI_GEMM_PATH_*; negative: its refusal) and, where not NULL, its tile's rows and
+ * columns of the product.  Nothing is launched. */
+#define UVMI_GEMM_PATH_TILED 0  /* through registers */
+#define UVMI_GEMM_PATH_STREAM 1
+#define UVMI_GEMM_PATH_BIG 2    /* slabs straight into LDS */
+int uvmi_gemm_tn_path(const uvmi_gemm_args* a, int* tile_rows, int* tile_cols);
 
 /* ------------------------------------------------------------------------------------------------------------
  * Packed (cu_seqlens) causal self-attention with an optional sliding window over unquantized K/V: the attention of

@@ -80,6 +80,40 @@ def test_gemm_capability_predicate_and_argument_checks():
     assert lib.uvmi_gemm_tn_ex(None, None) == -1
 
 
+def test_gemm_path_names_every_tile_and_no_other():
+    """The choice of a kernel and tile by size is host logic.  Over UV-50M's projections, and widths and depths around them, every tile of
+    the streaming form is taken somewhere (by SWIGLU those that hold a gate column beside its up column), none that
+    the library has no kernel for, and the other kernels where the rows or the alignment ask for them."""
+    from ultraviolet_amd import _lib
+    from ultraviolet_amd.kernels.gemm import BIG, RESID, SOFTCAP, STORE, STREAM, SWIGLU, TILED, gemm_path
+    stream = {(16, 16), (16, 32), (32, 32), (32, 48), (32, 64), (48, 64), (64, 64), (64, 80)}
+    swiglu = {(16, 16), (16, 32), (32, 32), (32, 64), (64, 64), (64, 96)}
+
+    def path(M, N, K, epi, config=0, norm=0, at=1 << 20):
+        n = N // 2 if epi == SWIGLU else N
+        return gemm_path(_lib.GemmArgs(1 << 20, 1 << 20, at, 1, M, N, K, K, K, n, epi, norm, 1e-6, (1 << 20) if epi == RESID else None, n, 1.0, 1.0, config, 7.5))
+    rows = sorted({int(1.07 ** i) for i in range(163)})
+    seen = {STORE: set(), SWIGLU: set(), RESID: set()}
+    for N, K, epi in ((656, 640, STORE), (640, 512, RESID), (640, 1664, RESID), (3328, 640, SWIGLU), (336, 64, STORE), (1280, 2560, RESID), (96, 128, SWIGLU), (6656, 1280, SWIGLU)):
+        done = False
+        for M in rows:
+            kind, r, c = path(M, N, K, epi)
+            assert kind == (TILED if K < 128 else BIG) and (r, c) in ((128, 128), (256, 256)) or kind == STREAM and (r, c) in (swiglu if epi == SWIGLU else stream), (M, N, K, kind, r, c)
+            if kind == STREAM:
+                assert not done, (M, N, K, r, c)      # (no streaming tile behind another kernel's)
+                seen[epi].add((r, c))
+            done = kind != STREAM
+    assert seen[STORE] | seen[RESID] == stream and seen[SWIGLU] == swiglu
+    assert path(512, 32768, 640, SOFTCAP) == (BIG, 256, 256) and path(128, 32768, 640, SOFTCAP) == (BIG, 128, 128)
+    assert path(5000, 656, 640, STORE, at=(1 << 20) + 8)[0] == TILED and path(5000, 656, 640, STORE) == (BIG, 128, 128)
+    assert [path(100, 640, 640, STORE, config=f) for f in range(1, 9)] == [(STREAM, 32, 64), (STREAM, 16, 16), (TILED, 128, 128), (STREAM, 64, 64), (BIG, 256, 256),
+                                                                        (BIG, 128, 128), (STREAM, 16, 32), (STREAM, 32, 32)]
+    for bad in (dict(config=9), dict(config=5, at=(1 << 20) + 8), dict(config=6, at=(1 << 20) + 8)):
+        with pytest.raises(_lib.UvmiError):
+            path(100, 640, 640, STORE, **bad)
+    assert path(0, 640, 640, STORE, config=5, at=(1 << 20) + 8)[0] == BIG      # (nothing to compute: taken, as ever)
+
+
 def test_no_cpu_fallback():
     import torch
     from ultraviolet_amd import _lib

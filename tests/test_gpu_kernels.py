@@ -1267,22 +1267,28 @@ def test_output_projection_in_the_attention_launch_refuses():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("M,N,K,epi", [(400, 640, 1664, "resid"), (512, 640, 1664, "resid"), (513, 640, 512, "resid"), (832, 640, 1664, "resid"), (1009, 640, 512, "resid"),
-                                       (1152, 640, 1664, "resid"), (1280, 640, 512, "resid"), (1601, 640, 1664, "resid"), (2048, 640, 1664, "resid"), (2049, 640, 1664, "resid"),
-                                       (450, 656, 640, "norm"), (900, 656, 640, "norm"), (1790, 656, 640, "norm"), (260, 3328, 640, "swiglu"), (448, 3328, 640, "swiglu"),
-                                       (449, 3328, 640, "swiglu"), (300, 3232, 192, "swiglu"), (576, 3328, 640, "swiglu"), (577, 3328, 640, "swiglu"), (3264, 640, 512, "resid"), (3265, 640, 512, "resid"),
-                                       (4864, 640, 1664, "resid"), (4865, 640, 1664, "resid"), (1792, 336, 64, "store"), (577, 624, 128, "store")])
-def test_streaming_tiles_of_few_hundred_to_two_thousand_rows(dtype, M, N, K, epi):
+@pytest.mark.parametrize("M,N,K,epi,tile", [(400, 640, 1664, "resid", "32x48"), (512, 640, 1664, "resid", "32x48"), (513, 640, 512, "resid", "32x48"),
+                                       (832, 640, 1664, "resid", "48x64"), (1009, 640, 512, "resid", "48x64"), (1152, 640, 1664, "resid", "48x64"),
+                                       (1280, 640, 512, "resid", "32x64"), (1601, 640, 1664, "resid", "64x80"), (2048, 640, 1664, "resid", "64x80"),
+                                       (2049, 640, 1664, "resid", "64x64"), (450, 656, 640, "norm", "32x48"), (900, 656, 640, "norm", "48x64"),
+                                       (1790, 656, 640, "norm", "64x80"), (260, 3328, 640, "swiglu", "64x96"), (448, 3328, 640, "swiglu", "64x96"),
+                                       (449, 3328, 640, "swiglu", "64x64"), (300, 3232, 192, "swiglu", "64x64"), (576, 3328, 640, "swiglu", "64x64"),
+                                       (577, 3328, 640, "swiglu", "128x128"), (3264, 640, 512, "resid", "64x64"), (3265, 640, 512, "resid", "128x128"),
+                                       (4864, 640, 1664, "resid", "64x64"), (4865, 640, 1664, "resid", "128x128"), (1792, 336, 64, "store", "48x64"),
+                                       (577, 624, 128, "store", "32x48")])
+def test_streaming_tiles_of_few_hundred_to_two_thousand_rows(dtype, M, N, K, epi, tile):
     """The built-in choice at the row counts where the tile changes (32 x 48, 48 x 64, 64 x 80 and, with SWIGLU, 64 x 96 among them), whole
-    tiles and ragged ones in both directions, K down to a slab that most waves have no share of: every element within two roundings of
-    the float64 product."""
-    from ultraviolet_amd.kernels.gemm import RESID, SWIGLU, gemm_tn
+    tiles and ragged ones in both directions, K down to a slab that most waves have no share of: the tile that is named, and every
+    element within two roundings of the float64 product."""
+    from ultraviolet_amd.kernels.gemm import RESID, SWIGLU, gemm_args, gemm_path, gemm_tn
     g = torch.Generator(device="cuda").manual_seed(M + N + K)
     a, w = (torch.randn(s, K, device="cuda", generator=g).to(dtype) for s in (M, N))
     w = (w.float() / K ** 0.5).to(dtype)
     r = torch.randn(M, N, device="cuda", generator=g).to(dtype)
     kw = {"resid": dict(epilogue=RESID, resid=r, ca=0.75, cb=1.25), "norm": dict(norm_eps=1e-6), "swiglu": dict(epilogue=SWIGLU, norm_eps=1e-6), "store": {}}[epi]
-    got = gemm_tn(a, w, **kw).double()
+    got = gemm_tn(a, w, **kw)
+    assert "%dx%d" % gemm_path(gemm_args(a, w, got, **kw))[1:] == tile
+    got = got.double()
     x = a.double()
     if "norm_eps" in kw:
         x = x * torch.rsqrt((x * x).mean(1, keepdim=True) + 1e-6)

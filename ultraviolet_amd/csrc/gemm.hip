@@ -9,6 +9,7 @@ namespace uvmi {
 void gemm_tile_launch(const uvmi_gemm_args* a, hipStream_t st);                     // gemm_tile.hip
 void gemm_big_launch(const uvmi_gemm_args* a, int tile, int cus, hipStream_t st);   // gemm_big.hip
 int gemm_stream_form(const uvmi_gemm_args* a, int cus);                             // gemm_stream.hip
+void gemm_stream_tile(int form, int* rows, int* cols);
 void gemm_stream_launch(const uvmi_gemm_args* a, int form, int cus, hipStream_t st);
 }
 
@@ -47,7 +48,7 @@ extern "C" int uvmi_gemm_tn_supported(int dtype, int64_t M, int N, int K, int64_
   return 1;
 }
 
-extern "C" int uvmi_gemm_tn_ex(const uvmi_gemm_args* a, void* stream) {
+static int check_gemm(const uvmi_gemm_args* a) {
   UVMI_REQUIRE(a && a->a && a->w && a->c, UVMI_EINVAL, "uvmi_gemm_tn: null pointer");
   UVMI_REQUIRE(uvmi_gemm_tn_supported(a->dtype, a->M, a->N, a->K, a->lda, a->ldw, a->ldc, a->epilogue), UVMI_EUNSUPPORTED,
                "uvmi_gemm_tn: unsupported problem (dtype %d, M %lld, N %d, K %d, lda %lld, ldw %lld, ldc %lld, epilogue %d): needs F16 / BF16, "
@@ -64,34 +65,35 @@ extern "C" int uvmi_gemm_tn_ex(const uvmi_gemm_args* a, void* stream) {
   UVMI_REQUIRE(a->config >= 0 && a->config <= 8, UVMI_EINVAL, "uvmi_gemm_tn: config %d", a->config);
   UVMI_REQUIRE((a->config != 1 && a->config != 2) || a->K <= (a->epilogue == UVMI_GEMM_SWIGLU ? 960 : 1984), UVMI_EUNSUPPORTED,
                "uvmi_gemm_tn: K = %d is beyond config 1, 2 (1984; 960 with SWIGLU)", a->K);
-  if (a->M == 0) return UVMI_OK;
+  UVMI_REQUIRE(a->config != 5 || a->M == 0 || big_ok(a), UVMI_EUNSUPPORTED,
+               "uvmi_gemm_tn: config 5 (256 x 256 tiles) needs K >= 128, C (and the residual) 16-byte aligned, ldc (ldr) %% 8 == 0");
+  UVMI_REQUIRE(a->config != 6 || a->M == 0 || big_ok(a), UVMI_EUNSUPPORTED,
+               "uvmi_gemm_tn: config 6 (tiles loaded straight into LDS) needs K >= 128, C (and the residual) 16-byte aligned, ldc (ldr) %% 8 == 0");
+  return UVMI_OK;
+}
+
+// The kernel that takes the problem: through registers (a 128 x 128 tile), streaming (the tile of `form`) or direct to LDS (128 x 128 or 256 x 256).
+struct Path {
+  int kind;   // UVMI_GEMM_PATH_*
+  int form;   // STREAM: gemm_stream.hip's form; BIG: 128 or 256
+};
+static Path gemm_path(const uvmi_gemm_args* a, int cus) {
   // (also a product of fewer rows whose 256 x 256 tiles still come to two rounds of the device or more - the tied head,
   // 2048 x 32768: 104 us against 129 us on 128 x 128 tiles - or, none of their columns padding, to one full round where 128 x 128
   // tiles, two to a compute unit, take a second one: 512 x 32768 26.6 us against 29.9, with the softcap 33.7 against 47.7 and
   // from 384 rows on 28.3 against 35.6; 288 rows 27.9 against 26.4, 384 without the softcap 26.6 against 24.1)
-  int cus = uvmi_device_cus();
-  if (cus <= 0) cus = 256;
   const int64_t t128 = ((a->M + 127) / 128) * (((int64_t)a->N + 127) / 128), t256 = ((a->M + 255) / 256) * (((int64_t)a->N + 255) / 256);
   const bool one_round = a->N % 256 == 0 && a->M >= (a->epilogue == UVMI_GEMM_SOFTCAP ? 384 : 512) && t256 <= cus && 8 * t256 >= 7 * (int64_t)cus && t128 > 2 * (int64_t)cus;
   const bool many_big_tiles = one_round || (a->M >= 1024 && t256 >= 2 * (int64_t)cus);
   const bool rows_ok = a->M >= (a->epilogue == UVMI_GEMM_SWIGLU ? BIG_MIN_ROWS_SWIGLU : BIG_MIN_ROWS);
-  if (a->config == 5 || (a->config == 0 && (many_big_tiles || rows_ok) && big_ok(a))) {
-    UVMI_REQUIRE(big_ok(a), UVMI_EUNSUPPORTED,
-                 "uvmi_gemm_tn: config 5 (256 x 256 tiles) needs K >= 128, C (and the residual) 16-byte aligned, ldc (ldr) %% 8 == 0");
+  if (a->config == 5) return {UVMI_GEMM_PATH_BIG, 256};
+  if (a->config == 0 && (many_big_tiles || rows_ok) && big_ok(a)) {
     // (a product of fewer rows whose many 256-wide tiles would be more than a tenth emptier than 128-wide ones takes those)
     const int64_t pad128 = ((int64_t)a->N + 127) / 128 * 128, pad256 = ((int64_t)a->N + 255) / 256 * 256;
     const bool small = rows_ok ? !big_tiles_pay(a, t128, t256, cus) : pad128 * 10 < pad256 * 9;
-    gemm_big_launch(a, a->config == 0 && small ? 128 : 256, cus, (hipStream_t)stream);
-    UVMI_CHECK_LAUNCH("uvmi_gemm_tn(direct to LDS)");
-    return UVMI_OK;
+    return {UVMI_GEMM_PATH_BIG, small ? 128 : 256};
   }
-  if (a->config == 6 || a->epilogue == UVMI_GEMM_SOFTCAP) {
-    UVMI_REQUIRE(big_ok(a), UVMI_EUNSUPPORTED,
-                 "uvmi_gemm_tn: config %d (tiles loaded straight into LDS) needs K >= 128, C (and the residual) 16-byte aligned, ldc (ldr) %% 8 == 0", a->config);
-    gemm_big_launch(a, 128, cus, (hipStream_t)stream);
-    UVMI_CHECK_LAUNCH("uvmi_gemm_tn(128 x 128, direct)");
-    return UVMI_OK;
-  }
+  if (a->config == 6 || a->epilogue == UVMI_GEMM_SOFTCAP) return {UVMI_GEMM_PATH_BIG, 128};
   // The streaming form while one of its tiles leaves a compute unit about one workgroup (gemm_stream_form) and, on 64 x 64 tiles, while
   // they are at most two to a unit, which run at the same time (N 640, K 512: 3072 rows, 480 tiles, 7.7 us against 9.2 in 128 x 128 tiles; 3328
   // rows, 520 tiles, 10.6 / 9.3; gate-up 576 rows, 468 tiles, 7.9 / 9.5, 640 rows, 520 tiles, 11.0 / 9.9).  With a longer K, where rounds of
@@ -100,16 +102,38 @@ extern "C" int uvmi_gemm_tn_ex(const uvmi_gemm_args* a, void* stream) {
   int form = a->config == 0 ? gemm_stream_form(a, cus) : of_config[a->config];
   const int64_t t64 = ((a->M + 63) / 64) * (((int64_t)a->N + 63) / 64);
   if (a->config == 0 && form < 0 && (a->K <= 768 ? t64 <= 2 * (int64_t)cus : 4 * t128 < 3 * (int64_t)cus)) form = 6;
-  if (form >= 0) {
-    gemm_stream_launch(a, form, cus, (hipStream_t)stream);
-    UVMI_CHECK_LAUNCH("uvmi_gemm_tn(streaming)");
-  } else if (a->config == 0 && big_ok(a)) {
-    gemm_big_launch(a, 128, cus, (hipStream_t)stream);
-    UVMI_CHECK_LAUNCH("uvmi_gemm_tn(128 x 128, direct)");
-  } else {
-    gemm_tile_launch(a, (hipStream_t)stream);
-    UVMI_CHECK_LAUNCH("uvmi_gemm_tn(tiled)");
-  }
+  if (form >= 0) return {UVMI_GEMM_PATH_STREAM, form};
+  if (a->config == 0 && big_ok(a)) return {UVMI_GEMM_PATH_BIG, 128};
+  return {UVMI_GEMM_PATH_TILED, 0};
+}
+
+static int compute_units() {
+  const int cus = uvmi_device_cus();
+  return cus > 0 ? cus : 256;
+}
+
+extern "C" int uvmi_gemm_tn_path(const uvmi_gemm_args* a, int* tile_rows, int* tile_cols) {
+  const int rc = check_gemm(a);
+  if (rc) return rc;
+  const Path p = gemm_path(a, compute_units());
+  int rows = 128, cols = 128;
+  if (p.kind == UVMI_GEMM_PATH_BIG) rows = cols = p.form;
+  else if (p.kind == UVMI_GEMM_PATH_STREAM) gemm_stream_tile(p.form, &rows, &cols);
+  if (tile_rows) *tile_rows = rows;
+  if (tile_cols) *tile_cols = cols;
+  return p.kind;
+}
+
+extern "C" int uvmi_gemm_tn_ex(const uvmi_gemm_args* a, void* stream) {
+  const int rc = check_gemm(a);
+  if (rc) return rc;
+  if (a->M == 0) return UVMI_OK;
+  const int cus = compute_units();
+  const Path p = gemm_path(a, cus);
+  if (p.kind == UVMI_GEMM_PATH_STREAM) gemm_stream_launch(a, p.form, cus, (hipStream_t)stream);
+  else if (p.kind == UVMI_GEMM_PATH_BIG) gemm_big_launch(a, p.form, cus, (hipStream_t)stream);
+  else gemm_tile_launch(a, (hipStream_t)stream);
+  UVMI_CHECK_LAUNCH("uvmi_gemm_tn");
   return UVMI_OK;
 }
 

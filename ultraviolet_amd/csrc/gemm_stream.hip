@@ -344,6 +344,8 @@ int gemm_stream_form(const uvmi_gemm_args* a, int cus) {
   return -1;
 }
 
+void gemm_stream_tile(int form, int* rows, int* cols) { *rows = TILE_M[form]; *cols = TILE_N[form]; }
+
 // Arguments are validated by the caller (uvmi_gemm_tn_ex).
 void gemm_stream_launch(const uvmi_gemm_args* a, int form, int cus, hipStream_t st) {
   StreamParams P;

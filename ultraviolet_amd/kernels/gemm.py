@@ -38,6 +38,18 @@ def gemm_args(a: Tensor, w: Tensor, out: Tensor, epilogue: int = STORE, *, norm_
                       epilogue, norm_eps is not None, norm_eps or 0.0, rp, ldr, ca, cb, config, cap_c)
 
 
+TILED, STREAM, BIG = range(3)   # UVMI_GEMM_PATH_*
+
+
+def gemm_path(g) -> tuple[int, int, int]:
+    """Which kernel takes a gemm_args block (TILED, STREAM or BIG), and its tile's rows and columns."""
+    rows, cols = C.c_int(), C.c_int()
+    kind = L.lib().uvmi_gemm_tn_path(C.byref(g), C.byref(rows), C.byref(cols))
+    if kind < 0:
+        L.check(kind, "uvmi_gemm_tn")
+    return kind, rows.value, cols.value
+
+
 def gemm_tn(a: Tensor, w: Tensor, out: Tensor | None = None, epilogue: int = STORE, *, norm_eps: float | None = None,
             resid: Tensor | None = None, ca: float = 1.0, cb: float = 1.0, cap_c: float = 0.0, config: int = 0) -> Tensor:
     """a (M, K) @ w (N, K).T -> (M, N); with epilogue=SWIGLU w is interleave_gate_up(w_gate, w_up) and the result is
