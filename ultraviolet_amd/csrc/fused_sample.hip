@@ -53,7 +53,8 @@ __device__ __forceinline__ void emit(const SampleParams& P, int row, int tok, fl
   P.logp[row] = logp;
   if (P.commit) commit_store<true>(P.S, P.D, row, r, tok, logp);
 }
-// what emit's commit reads, for thread 0, which emits: behind the requests for the row's logits
+// what emit's commit reads, for thread 0, which emits: ahead of the draw, so that it is there by then (the kernels of 1024 threads that hold a row
+// in registers request its logits first)
 __device__ __forceinline__ CommitRow commit_ahead(const SampleParams& P, int row) {
   CommitRow r = {};
   if (P.commit && threadIdx.x == 0) r = commit_load<true>(P.S, P.D, row, P.retire_p, P.commit_seed);

@@ -69,6 +69,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_stream_kernel(const void* a_a, c
   __shared__ __attribute__((aligned(1024))) unsigned char s0[NW * SLAB];
   __shared__ __attribute__((aligned(1024))) unsigned char s1[R > 1 ? (NW - 1) * SLAB + ROWS * 128 : 16];
   __shared__ float sSS[NORM ? NW * BM : 1];
+  static_assert(sizeof(s0) + (R > 1 ? sizeof(s1) : 0) + (NORM ? sizeof(sSS) : 0) <= 160 * 1024, "a compute unit's LDS");
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int T = P.tiles_m * P.tiles_n, per = (T + 7) / 8;
@@ -292,7 +293,7 @@ static void launch_stream(const uvmi_gemm_args* a, StreamParams& P, hipStream_t 
 #undef UVMI_GO
 }
 
-// The tiles, by the rows of A and W that they load: (BM, BN, NW, R).  LDS: 64, 48, 64, 80, 96 / 48, 112, 64, 152, 96 KB.  The smallest
+// The tiles, by the rows of A and W that they load: (BM, BN, NW, R).  LDS: 64, 48, 64, 80, 96 / 48, 112, 64, 158 (159 with NORM, of 160), 96 KB.  The smallest
 // tile takes 8 waves (K of 512 or 640: one or two slabs each, all in flight at once).
 constexpr int TILE_M[9] = {16, 16, 32, 32, 32, 48, 64, 64, 64}, TILE_N[9] = {16, 32, 32, 48, 64, 64, 64, 80, 96};
 constexpr int FORM_64 = 6, FORM_96 = 8;

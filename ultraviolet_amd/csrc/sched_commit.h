@@ -24,9 +24,9 @@ struct DenseArrays {
   int64_t* act_slot; int64_t* tok; int64_t* pos; int64_t* starts; int64_t* req; int64_t* cnt;
 };
 
-// What committing dense row i reads, none of which depends on the token: loaded ahead of it (by a sampler kernel while the row of logits
-// is on its way; one load behind the other and behind the stores between them they took 3 us of a launch of 11).  No other row of
-// a step has the row's slot.
+// What committing dense row i reads, none of which depends on the token: loaded ahead of it (by a sampler kernel at its start or behind its
+// requests for the row of logits; one load behind the other and behind the stores between them they took 3 us of a launch of 11).  No other
+// row of a step has the row's slot.
 struct CommitRow {
   int64_t slot, cnt, req, pos, dense_pos;
   bool ends;   // its length limit or the seeded Bernoulli(retire_p) draw keyed by (seed, request, token index) retires it
