@@ -59,7 +59,8 @@ __global__ __launch_bounds__(256) void prefill_segments(const void* cu, int idx6
     const int mid = (lo + hi) >> 1;
     if (load_index(cu, idx64, mid) <= i) lo = mid; else hi = mid;
   }
-  seg_start[i] = (int32_t)load_index(cu, idx64, lo);
+  const int first = (int)load_index(cu, idx64, lo);
+  seg_start[i] = first <= i ? first : i + 1;   // (ahead of the first sequence: behind the token itself, so that it sees no key)
   pidx[i] = i;
 }
 
@@ -127,14 +128,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void p
   if (P.window > 0 && row - P.window + 1 > lo_n) lo_n = row - P.window + 1;
   if (!row_ok) lo_n = INT_MAX;
   if (P.window > 0 && row0 - P.window + 1 > lo0) lo0 = row0 - P.window + 1;
-  const uint32_t n_keys = row_ok && row >= lo_n ? (uint32_t)(row - lo_n + 1) : 0u;   // the row sees keys lo_n .. lo_n + n_keys - 1 (none ahead of the first sequence)
+  const uint32_t n_keys = row_ok ? (uint32_t)(row - lo_n + 1) : 0u;           // the row sees keys lo_n .. lo_n + n_keys - 1
   const int rl = min(r0 + 15, P.N - 1);                                       // last real row of the block
   const int lo_first = __builtin_amdgcn_readfirstlane(lo_n);                  // lo is non-decreasing in the row
   const int lo_last = __builtin_amdgcn_readfirstlane(__shfl(lo_n, wave_ok ? rl - r0 : 0, 64));
   const int kbeg = wave_ok ? lo_first & ~31 : 0, kend = wave_ok ? rl + 1 : 0;
   const int kbeg_wg = __builtin_amdgcn_readfirstlane(lo0) & ~31;
   const int kend_wg = min(row0 + qbw * 16, P.N);
-  const int nk = (kend_wg - kbeg_wg + 31) >> 5;   // (none: every row lies ahead of the first sequence)
+  const int nk = (kend_wg - kbeg_wg + 31) >> 5;   // >= 1
 
   // ---- K / V super-tiles go from global memory straight into one of three LDS stages, two tiles ahead: wave w moves keys 8 w .. 8 w + 7
   // of K and of V, 16 bytes per lane.  Keys are clamped to N - 1 (a clamped key is masked).  K rows keep their 16-byte chunks
@@ -152,7 +153,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void p
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rK, (__attribute__((address_space(3))) void*)(S[0] + 1024 * wave), 16, r * skn2 + kch, 0, 0, 0);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rV, (__attribute__((address_space(3))) void*)(S[1] + 1024 * wave), 16, r * svn2 + vch, 0, 0, 0);
   };
-  if (nk > 0) issue(s0, 0);
+  issue(s0, 0);
   if (nk > 1) issue(s1, 1);
 
   pf4 O[HPW][4];

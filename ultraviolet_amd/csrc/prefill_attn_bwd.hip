@@ -354,7 +354,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void b
   const int lo_last = __builtin_amdgcn_readfirstlane(__shfl(lo_n, any ? rl - r0 : 0, 64));
   const int kbeg = any ? lo_first & ~31 : 0, kend = any ? rl + 1 : 0;
   const int nk = __builtin_amdgcn_readfirstlane((kend - kbeg + 31) >> 5);
-  const uint32_t n_keys = row_ok && row >= lo_n ? (uint32_t)(row - lo_n + 1) : 0u;   // the row sees keys lo_n .. lo_n + n_keys - 1 (none ahead of the first sequence)
+  const uint32_t n_keys = row_ok ? (uint32_t)(row - lo_n + 1) : 0u;   // the row sees keys lo_n .. lo_n + n_keys - 1 (none ahead of the first sequence)
 
   // ---- K / V tiles go from global memory straight into one of three LDS stages, two tiles ahead: wave w moves rows 8 w .. 8 w + 7
   const uint32_t rstride = (uint32_t)P.KH * 128;
