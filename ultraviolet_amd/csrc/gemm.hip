@@ -27,7 +27,8 @@ static bool big_ok(const uvmi_gemm_args* a) {
 // Whether a pass of many rows takes 256 x 256 tiles rather than 128 x 128 ones.  A launch lasts as long as its rounds of the device: of
 // one 256 x 256 tile per compute unit, or of two 128 x 128 ones, which take about 0.6 of that.  us, 256 against 128, activations in
 // the last-level cache as a pass leaves them: gate-up with norm and SwiGLU 5000 rows, 2 rounds against 3, 41.0 / 31.1; 8192 rows, 2
-// against 4, 42.0 / 41.5; 10 000 rows, 3 against 5, 62.6 / 51.4; 18 432 rows, 4 against 8, 88.6 / 96.0; 20 000 rows, 5 against 8, 100.3 /
+// against 3 and a quarter, 42.0 / 41.5 and again 43.9 / 42.3 (the one size measured where the choice is not the faster, by 1 - 4 %; 7168 rows
+// 47.1 / 37.9, 9216 rows 45.1 / 49.0); 10 000 rows, 3 against 5, 62.6 / 51.4; 18 432 rows, 4 against 8, 88.6 / 96.0; 20 000 rows, 5 against 8, 100.3 /
 // 104.9; 33 216 rows, 7 against 14, 150 / 171.  640 columns, K 1664: 18 432 rows, 1 against 2, 51.2 / 59.4; 24 576 rows, 2 against 2, 97.1 /
 // 66.4; 40 000 rows, 2 against 4, 103 / 112.  With a short K a last round of 128 x 128 tiles that fills a quarter of the device or
 // less takes half a round (K 512: 16 384 rows 21.9 / 20.4, 18 432 rows, 0.4 of a round, 23.4 / 26.0).

@@ -24,8 +24,8 @@
 //     in copies, 40 registers a tile, and it took 153 registers instead of 118, three waves per SIMD instead of four);
 //   * workgroup ids are remapped so that each XCD (one L2 each) owns a contiguous range of query blocks and therefore
 //     whole sequences, the last blocks first: they see the most keys.
-// What bounds it: vector instructions (79 % of the cycles that a compute unit is busy; the matrix cores 18 %), ~135 a tile and head
-// pair of which 36 are exponentials, at four waves per SIMD.  With four heads per wave it held 255 registers, two waves per SIMD, staged
+// What bounds it: vector instructions (74 % of the cycles that a SIMD is busy; the matrix cores 22 %; 64 x 512 tokens, both windows), ~135 a
+// tile and head pair of which 36 are exponentials, at 3.3 of the four waves per SIMD that it has room for.  With four heads per wave it held 255 registers, two waves per SIMD, staged
 // K and V through registers, and made eight trips to memory one after the other for its epilogue.  us, before -> now, with the
 // epilogue: 93 tokens 9.4 -> 5.3; 400 16.6 -> 8.6; 64 x 64 .. 512 tokens 41.2 -> 30.8, window 256 34.2 -> 25.2; 64 x 512 62.2 -> 43.4 and
 // 46.3 -> 34.8; 4 x 2048 without 77.6 -> 43.5; 61 x 16 .. 1024, window 256, 42.1 -> 34.6.

@@ -273,8 +273,9 @@ __device__ __forceinline__ float dot2w(uint32_t a, uint32_t b, float acc) {  // 
 }
 
 // A staged tile of 32 rows of 128 bytes: row r keeps its 16-byte chunks xor-ed with the bits 1, 2 and then 3 of r / 2 rotated to the left.
-// Rows r and r + 1 share a 256-byte line of banks, so both reads of a tile are free of conflicts: 16 lanes' 16 bytes of one chunk of 16
-// rows (eight different places per half line), and 32 lanes' transposing reads of two neighbouring chunks of 8 rows (four pairs of places).
+// Rows r and r + 1 share a 256-byte line of banks.  The transposing reads, 32 lanes on two neighbouring chunks of 8 rows (four pairs of
+// places), are free of conflicts; those of rows are not, 4 cycles for each 16-byte read (32 a tile of 32 keys x 16 rows x 2 heads): the sixteen lanes of a pass
+// are rows of two chunks g and g + 1, and rows 8 apart differ in the bit that those do.
 __device__ __forceinline__ int tile_swizzle(int row) { return ((row & 6) | ((row >> 3) & 1)); }
 
 // Operands of a staged tile.  Rows: [tile A dims 0..31, A dims 32..63, B dims 0..31, B dims 32..63], lane = row m, dims 8 g .. ;
