@@ -60,6 +60,17 @@ def test_global_ragged(dtype, int8, B, KH, G, hd, splits):
     _attn_check(q, k, v, ks, vs, pos, starts, 1.13 / hd ** 0.5, splits=splits)
 
 
+@pytest.mark.parametrize("B,KH,G,hd,S,splits", [(3, 1, 8, 64, 2304, 2), (2, 2, 4, 64, 2304, 17), (1, 1, 8, 64, 8448, 65), (3, 2, 3, 128, 2112, 65),
+                                                (2, 1, 2, 256, 700, 5), (2, 1, 16, 64, 544, 16), (1, 1, 1, 16, 96, 1024)])
+def test_rows_cut_into_many_splits(B, KH, G, hd, S, splits):
+    """The combine pass around the splits whose partials it has in flight at a time (16; 4 beyond 64 dims) and around a wave's 64 of them: full rows,
+    a row of one chunk and a row whose last chunks are empty."""
+    q, k, v, ks, vs = attn_case(B, KH, G, hd, S, True, dtype=torch.bfloat16)
+    pos = torch.tensor([S - 1, S // 2 + 3, 5][:B])
+    starts = torch.tensor([0, S // 2 - 60, 0][:B])
+    _attn_check(q, k, v, ks, vs, pos, starts, 1.13 / hd ** 0.5, splits=splits)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("B,S,ring", [(3, 1056, False), (200, 1056, False), (300, 2080, False), (500, 1024, False), (40, 1024, True)])
 def test_few_and_many_rows_on_long_caches(dtype, B, S, ring):
