@@ -63,6 +63,24 @@ def test_modes_and_transforms_reach_the_op(route):
     assert seen == ["op"]
 
 
+@pytest.mark.parametrize("q_dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("kv_dtype", [torch.int8, torch.float16, torch.bfloat16])
+def test_splits_of_a_call_that_names_none(monkeypatch, q_dtype, kv_dtype):
+    """The native call and the general path cut a row alike, and never into chunks beyond one per compute unit or under 128 keys where the
+    matrix-core kernel serves; the generic kernel's geometries are cut as default_splits has it."""
+    monkeypatch.setattr(D, "_device_cus", lambda index: 256)
+    native = D.L.lib().uvmi_decode_attn_splits
+    for G, hd, S, ring in [(8, 64, 4096, False), (8, 64, 4098, False), (1, 64, 31, False), (4, 64, 250, True), (4, 64, 256, True), (9, 64, 4096, False), (8, 128, 4096, False)]:
+        for n in (0, 1, 3, 32, 64, 65, 128, 129, 256, 257, 5000):
+            for ctx in (0, 1, 127, 800, 1023, 1024, 2048, 2400, 4096, 100000):
+                s = D._own_splits(q_dtype, kv_dtype, n, G, hd, S, ring, ctx, torch.device("cuda", 0))
+                assert s == native(D.L.dtype_code(q_dtype), D.L.dtype_code(kv_dtype), n, G, hd, S, ring, ctx, 256)
+                if hd == 128 or G == 9 or S == 31 or q_dtype == torch.float32:
+                    assert s == D.default_splits(n, ctx, torch.device("cuda", 0))
+                elif s > 1 and S % 32 == 0 and kv_dtype in (torch.int8, q_dtype):
+                    assert s * n <= 256 and ctx // s >= 128
+
+
 def test_guard_of_recorded_passes_sees_what_changes():
     """Everything that launches took an address or a number from: a tensor replaced, moved under its object, a scalar, an entry that
     comes or goes - in the weights and in the state; by torch's comparison of addresses and by the list of them."""

@@ -1415,6 +1415,30 @@ extern "C" int uvmi_default_splits(int64_t n_bk, int ctx, int n_cus) {
   return (int)s;
 }
 
+// The splits that a call which names none is given.  A launch without splits lasts as long as its longest row; with them it is followed by
+// the combine pass (2.6 us on the GPU, and 9.3 us a call is what the host needs for the two launches and the workspace, 4.5 for one launch), and what
+// it saves depends on how fast one workgroup streams a row: an int8 cache 1024 keys in 2.0 us (eight waves), a 16-bit one in 4.9 (four).  So
+// splits pay where they take about 2900 and 1000 keys off the longest row, and only with a compute unit for every chunk; chunks of less
+// than 128 keys gain nothing.  us on the GPU, rows up to that many keys without / with splits: int8 4 rows of 4096 11.0 / 7.9, of 2048 7.4 / 7.5; 64 rows of
+// 4096 12.2 / 10.2, of 2048 8.1 / 8.6; 100 rows of 4096 in two 12.5 / 13.1; 178 rows of 2048 8.6 / 12.4; 16-bit 16 rows of 1024
+// 8.7 / 7.7, of 2048 13.6 / 7.9; 64 rows of 2048 13.7 / 9.6; 128 rows of 2048 14.7 / 13.4, of 4096 24.9 / 20.5; 178 rows of 4096 25.4 / 32.1.
+// The generic kernel, a wave to an item, keeps uvmi_default_splits.
+extern "C" int uvmi_decode_attn_splits(int q_dtype, int kv_dtype, int64_t n_bk, int G, int hd, int S, int ring, int ctx, int n_cus) {
+  const bool kv16 = kv_dtype == q_dtype;
+  const bool mfma = hd == 64 && G <= 8 && (q_dtype == UVMI_F16 || q_dtype == UVMI_BF16) && (kv16 || kv_dtype == UVMI_I8) && S >= 32 &&
+                    (!ring || S % 32 == 0) && (kv16 || S % 4 == 0);
+  if (!mfma) return uvmi_default_splits(n_bk, ctx, n_cus);
+  if (n_cus <= 0) n_cus = uvmi_device_cus();
+  if (n_cus <= 0) n_cus = 256;
+  if (n_bk < 1) n_bk = 1;
+  int64_t s = n_cus / n_bk;
+  if (s > ctx / 128) s = ctx / 128;
+  if (s > 64) s = 64;
+  if (s < 2) return 1;
+  const int64_t saved = ctx - ctx / s;
+  return saved >= (kv16 ? 1000 : 2900) ? (int)s : 1;
+}
+
 extern "C" int uvmi_attn_oproj_rows(int N) {
   int cus = uvmi_device_cus();
   if (cus <= 0) cus = 256;

@@ -120,7 +120,7 @@ PyObject* py_decode_attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
   else Py_RETURN_NONE;
   if (args[12] != Py_None) {
     if (!as_int(args[12], a.num_splits)) Py_RETURN_NONE;
-  } else {   // default_splits
+  } else {
     int ctx = 0;
     if (args[11] != Py_None && !as_int(args[11], ctx)) Py_RETURN_NONE;
     if (ctx == 0) ctx = a.S;
@@ -134,10 +134,7 @@ PyObject* py_decode_attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
       if (!r || !as_int(r, cus)) return nullptr;
       device_cus[dev].store(cus, std::memory_order_relaxed);
     }
-    const int64_t work = static_cast<int64_t>(a.B) * a.KH, per = work > 1 ? work : 1;
-    const int64_t want = (cus + per - 1) / per, most = ctx / 256 > 1 ? ctx / 256 : 1;
-    const int64_t s = want < most ? want : most;
-    a.num_splits = static_cast<int>(s < 1 ? 1 : (s > 64 ? 64 : s));
+    a.num_splits = uvmi_decode_attn_splits(qd, kd, static_cast<int64_t>(a.B) * a.KH, a.KH > 0 ? a.H / a.KH : 0, a.hd, a.S, a.ring, ctx, cus);
   }
   const int fp32 = PyObject_IsTrue(args[13]);
   if (fp32 < 0) return nullptr;

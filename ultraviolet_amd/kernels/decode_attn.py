@@ -72,6 +72,21 @@ def default_splits(n_bk: int, ctx: int, device=None, min_chunk: int = 256, waves
     return int(max(1, min(want, max(1, int(ctx) // min_chunk), 64)))
 
 
+def _own_splits(q_dtype, kv_dtype, n_bk: int, G: int, hd: int, S: int, ring: bool, ctx: int, device=None) -> int:
+    """uvmi_decode_attn_splits (its reasons stand there), for calls that are traced: the splits of a call that names none."""
+    kv16 = kv_dtype == q_dtype
+    if not (hd == 64 and G <= 8 and q_dtype in (torch.float16, torch.bfloat16) and (kv16 or kv_dtype == torch.int8) and S >= 32
+            and (not ring or S % 32 == 0) and (kv16 or S % 4 == 0)):
+        return default_splits(n_bk, ctx, device)
+    index = None if device is None else torch.device(device).index
+    cus = _device_cus(torch.cuda.current_device() if index is None else index)
+    s = min(cus // max(int(n_bk), 1), ctx // 128, 64)
+    if s < 2:
+        return 1
+    saved = ctx - ctx // s
+    return s if saved >= (1000 if kv16 else 2900) else 1
+
+
 def supported(q: Tensor, k_cache: Tensor) -> bool:
     """True when the MFMA kernel serves this geometry (reference: decode_attn_cuda.supported,
     decode_attn_cuda.py:265-270): head_dim 64, up to 8 query heads per kv head, an int8 cache or one in the q dtype.  Other
@@ -232,7 +247,7 @@ def decode_attention(q: Tensor, k_cache: Tensor, v_cache: Tensor, pos: Tensor, s
         ctx = ctx_hint or S
         if window > 0:
             ctx = min(ctx, window)
-        num_splits = default_splits(B * KH, ctx, q.device)
+        num_splits = _own_splits(q.dtype, k_cache.dtype, B * KH, H // KH if KH else 0, hd, S, bool(ring), int(ctx), q.device)
     q = q.contiguous() if q.stride(-1) != 1 else q
     if pos.dtype != starts.dtype:
         starts = starts.to(pos.dtype)
