@@ -331,3 +331,65 @@ def test_backward_rejects_what_it_cannot_do():
     with pytest.raises(L.UvmiError):   # fp32 tensors
         packed_attention_backward(*(z(4, 2, 64, dt=torch.float32) for _ in range(2)), *(z(4, 1, 64, dt=torch.float32) for _ in range(2)),
                                   z(4, 2, 64, dt=torch.float32), cu, 1.0)
+
+
+@pytest.mark.parametrize("form", ["plain", "fp16", "indices64", "views", "padding", "k alone", "no gradient", "no grad mode", "inference", "hooks",
+                                  "parameter", "generic", "scale int", "fp32"])
+def test_native_varlen_call_equals_the_general_one(monkeypatch, form):
+    """varlen_attention's native path (csrc/eager.cpp) and the general one make the same launches on the same arguments: equal bits, output and
+    gradients, over the forms a call may take; the last four the native path hands on.  A hook on saved tensors sees the same ones."""
+    from ultraviolet_amd.kernels import varlen_attn as A
+    dtype = torch.float16 if form == "fp16" else torch.float32 if form == "fp32" else torch.bfloat16
+    q, k, v, cu = (t.to(DEV) for t in _case([131, 0, 37, 64], 16 if form == "generic" else 8, 1, 64, dtype, seed=3))
+    q, k, v = (t[None] for t in (q, k, v))
+    go = torch.randn(q.shape, device=DEV, generator=torch.Generator(device=DEV).manual_seed(4)).to(dtype)
+    scale = 1 if form == "scale int" else 0.14
+    if form == "indices64":
+        cu = cu.long()
+    elif form == "views":
+        qkv = torch.cat([q, k, v], 2)
+        q, k, v, go = qkv[:, :, :8], qkv[:, :, 8:9], qkv[:, :, 9:], go.transpose(1, 2).contiguous().transpose(1, 2)
+    elif form == "padding":
+        cu = cu[:3].contiguous()
+    elif form == "parameter":
+        q = torch.nn.Parameter(q)
+    grads = form not in ("no gradient", "no grad mode", "inference", "generic", "fp32")
+    wrt = [k] if form == "k alone" else [q, k, v]
+    if form != "no gradient" and form != "generic" and form != "fp32":
+        wrt = [t.detach().requires_grad_() if form != "parameter" or t is not q else t for t in wrt]
+        q, k, v = (q, wrt[0], v) if form == "k alone" else wrt
+    seen = []
+
+    def call():
+        seen.append([])
+        keep = lambda t: seen[-1].append((t.shape, t.dtype)) or t
+        with torch.autograd.graph.saved_tensors_hooks(keep, lambda t: t) if form == "hooks" else torch.inference_mode(form == "inference"):
+            with torch.set_grad_enabled(form != "no grad mode" and form != "inference"):
+                o = A.varlen_attention(q, k, v, cu, 131, scale, 100)
+        return (o.detach(), *torch.autograd.grad(o, wrt, go)) if grads else (o,)
+    used = []
+    native = A._native()
+    monkeypatch.setattr(A, "_native", lambda: lambda *a: used.append(native(*a)) or used[-1])
+    got = call()
+    monkeypatch.setattr(A, "_native", lambda: lambda *a: None)
+    want = call()
+    assert (used[0] is None) == (form in ("parameter", "generic", "scale int", "fp32"))
+    assert len(got) == len(want) and all(a.dtype == b.dtype and a.shape == b.shape and torch.equal(a, b) for a, b in zip(got, want))
+    assert seen[0] == seen[1] and (form != "hooks" or len(seen[0]) == 7)
+
+
+def test_native_varlen_gradient_of_a_changed_input_is_refused():
+    """A saved operand changed in place before the backward: the error of a graph, not gradients of other values."""
+    from ultraviolet_amd.kernels import varlen_attention
+    q, k, v, cu = (t.to(DEV) for t in _case([64, 7], 8, 1, 64, torch.bfloat16, seed=3))
+    q, k, v = (t[None] for t in (q, k, v))
+    q.requires_grad_()
+    o = varlen_attention(q, k, v, cu, 64, 0.14)
+    k.add_(1)
+    with pytest.raises(RuntimeError, match="inplace"):
+        o.sum().backward()
+    o = varlen_attention(q, k, v, cu, 64, 0.14)
+    o.sum().backward(retain_graph=True)
+    first, q.grad = q.grad, None
+    o.backward(torch.ones_like(o))
+    assert torch.equal(first, q.grad)

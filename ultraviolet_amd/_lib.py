@@ -239,7 +239,8 @@ def eager():
         except ImportError as e:
             raise UvmiError(f"{EAGER_PATH} does not load: {e}") from e
         # (it fills the argument structs itself, and calls whichever libuvmi.so the loader found for it)
-        if not (mod.revision == mod.library_revision == ABI_VERSION and mod.attn_args_bytes == C.sizeof(AttnArgs)):
+        sizes = (mod.attn_args_bytes, mod.prefill_attn_args_bytes, mod.prefill_attn_bwd_args_bytes)
+        if not (mod.revision == mod.library_revision == ABI_VERSION and sizes == tuple(C.sizeof(t) for t in (AttnArgs, PrefillAttnArgs, PrefillAttnBwdArgs))):
             raise UvmiError(f"{EAGER_PATH} was built for revision {mod.revision} of include/uvmi.h and calls a library of revision {mod.library_revision}, these "
                             f"bindings are for {ABI_VERSION}: rebuild it with `python -m ultraviolet_amd.csrc.build`")
         _eager = mod

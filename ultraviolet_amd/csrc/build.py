@@ -57,9 +57,9 @@ def _build_eager(run, force: bool, verbose: bool) -> None:
             return
         os.remove(out)   # (one of other sources is worse than none)
     try:
-        run([os.environ.get("CXX", "g++"), "-O2", "-fPIC", "-std=c++17", "-shared", src, *(x for d in include_paths() for x in ("-isystem", d)),
+        run([os.environ.get("CXX", "g++"), "-O2", "-fPIC", "-std=c++17", "-shared", src, *(x for d in include_paths("cuda") for x in ("-isystem", d)), "-D__HIP_PLATFORM_AMD__=1",
              "-I" + sysconfig.get_paths()["include"], f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-             *("-L" + d for d in library_paths()), "-ltorch_python", "-ltorch_cpu", "-lc10", "-L" + HERE, "-l:libuvmi.so", "-Wl,-rpath,$ORIGIN",
+             *("-L" + d for d in library_paths()), "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", "-L" + HERE, "-l:libuvmi.so", "-Wl,-rpath,$ORIGIN",
              "-o", out])
     except (OSError, RuntimeError) as e:
         print(f"not built: {os.path.relpath(out, HERE)}; eager calls of decode_attention will be slower.\n{e}", file=sys.stderr, flush=True)

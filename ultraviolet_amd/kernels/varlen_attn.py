@@ -6,9 +6,12 @@ q / k / v must be device tensors; there is no CPU path."""
 from __future__ import annotations
 
 import ctypes as C
+import functools
+import warnings
 
 import torch
 from torch import Tensor
+from torch.autograd import forward_ad
 
 from .. import _lib as L
 
@@ -121,6 +124,17 @@ def statistics_pitch(N: int) -> int:
     return (N + 31) // 32 * 32 + 32
 
 
+@functools.lru_cache(maxsize=None)
+def _native():
+    """varlen_attention of csrc/eager.cpp; where that was not built for this interpreter, torch and library, what hands every call on to
+    the general path below, which launches the same kernels."""
+    try:
+        return L.eager().varlen_attention
+    except L.UvmiError as e:
+        warnings.warn(f"varlen_attention: eager calls and their gradients are prepared in Python, which takes longer than small launches ({e})", stacklevel=3)
+        return lambda *call: None
+
+
 class _PackedAttention(torch.autograd.Function):
     """packed_attention with the backward above (the reference registers its pair of custom ops with autograd the same
     way, varlen_attn.py:69-84), on the (1, N, ..) tensors themselves: a select in front of it would cost a zero fill and a copy
@@ -152,6 +166,13 @@ def varlen_attention(q: Tensor, k: Tensor, v: Tensor, cu_seqlens: Tensor, max_se
     """The reference's signature: q (1, N, H, hd), k / v (1, N, K, hd) packed along N, cu_seqlens (S+1,) with cu[0] = 0
     and cu[-1] = N; returns (1, N, H, hd).  max_seqlen is accepted for compatibility (the kernel does not need it).
     Differentiable in q, k, v (16-bit inputs, head_dim 64)."""
+    if not torch.compiler.is_compiling() and forward_ad._current_level < 0 and q.is_cuda:
+        # plain eager calls, checked, allocated, launched and differentiated natively (None: not such a call)
+        out = _native()(q, k, v, cu_seqlens, scale, window)
+        if type(out) is int:
+            L.check(out, "uvmi_prefill_attn")
+        if out is not None:
+            return out
     assert q.dim() == 4 and q.size(0) == 1 and k.size(0) == 1 and v.size(0) == 1
     if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
         return _PackedAttention.apply(q, k, v, cu_seqlens, float(scale), int(window or 0))
