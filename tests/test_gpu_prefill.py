@@ -277,6 +277,17 @@ def test_attention_and_backward_at_the_mask_rules(window):
         assert np.abs(a - b).max() <= 2 * ulp * np.abs(b).max() + 1e-6, (np.abs(a - b).max(), np.abs(b).max())
 
 
+@pytest.mark.parametrize("G", [1, 2, 3, 8])
+@pytest.mark.parametrize("K,lens,window", [(40, [330, 5, 200], None), (20, [330, 5, 200], 70), (20, [330, 5, 200], None), (1, [3] * 64 + [40], None), (2, [2, 0, 5] * 50, 4)])
+def test_backward_of_keys_by_heads_and_strides(G, K, lens, window):
+    """dk / dv with more workgroups than the 8-wave form takes (with and without a window) and fewer, for every padding of the head group; around and
+    beyond the 64 sequences whose ends a wave holds.  Tolerance as above."""
+    got, ref = _grad_case(lens, G * K, K, torch.float16, window, seed=7)
+    for a, b in zip(got, ref):
+        assert np.isfinite(a).all()
+        assert np.abs(a - b).max() <= 2 * 2.0 ** -10 * np.abs(b).max() + 1e-6, (np.abs(a - b).max(), np.abs(b).max())
+
+
 @pytest.mark.parametrize("window", [33, 167, 168, 2 ** 31 - 1])
 def test_plain_backward_with_windows_that_hide_few_keys_and_none(window):
     """16 query heads on a kv head, which the plain kernels serve: windows up to the largest that an int holds.  Tolerance as above."""

@@ -6,7 +6,7 @@
 // D_i = go_i . o_i:   dv_j = sum_i p_ij go_i,   ds_ij = p_ij (go_i . v_j - D_i),   dq_i = scale sum_j ds_ij k_j,
 // dk_j = scale sum_i ds_ij q_i  (dk, dv also summed over the query heads of the group).
 //
-// Two forms.  The matrix-core form (bwd_dq_mfma, bwd_dkv_mfma, described where they are defined) serves up to 8 query heads
+// Two forms.  The matrix-core form (bwd_dq_mfma, bwd_dkv_heads, described where they are defined) serves up to 8 query heads
 // per kv head.  The plain form below it serves the rest: fp32 arithmetic on the vector units, no atomics, no
 // cross-workgroup state.
 //   bwd_dq_kernel   lane = query token (64 per wave), one query head per workgroup: the wave walks the union of its
@@ -239,16 +239,13 @@ __global__ __launch_bounds__(64) void bwd_dkv_kernel(BwdParams P) {
 //     ds = p (dp - D) are lane-local, and the 8 values of ds, rounded to the input type, are the lane's slice of the B
 //     operand of dQ^T += K^T dS^T (K^T operands from the transposing LDS read, as V^T in the
 //     forward);
-//   * bwd_dkv_mfma: the transposed problem.  A workgroup owns 64 keys of one kv head and walks (query tile of 32, pair of query
-//     heads): the tile's Q and dO rows are staged in LDS; S = Q K^T and dP = dO V^T leave 4 consecutive queries
-//     of one key in a lane for two 16-query tiles, exactly the B-operand slices of dV^T += dO^T P and dK^T += Q^T dS, which
-//     accumulate over the tiles and over the heads of the group in registers.
+//   * bwd_dkv_heads: the transposed problem.  A workgroup owns 32 keys of one kv head and walks the 32-query tiles of the heads, a head to a wave:
+//     S = Q K^T and dP = dO V^T leave 4 consecutive queries of one key in a lane for two 16-query tiles, exactly the B-operand slices
+//     of dV^T += dO^T P and dK^T += Q^T dS, which accumulate over the tiles in registers and over the heads in LDS at the end.
 // The accumulators of dP start at -D.  Probabilities and ds are rounded to the input type for their second products; everything else is
 // fp32.  Both kernels keep a tile's mask in a branch of its own, with the products on both sides of it outside: as two versions of the
 // whole tile the accumulators of the two met in copies, 32 and 64 registers of them a tile.
 //
-// us, forward's statistics at hand: 61 x 16 .. 1024 tokens, window 256: 122 -> 98 (dq 49 -> 42, dk / dv 73 -> 56); without a window 252 -> 189;
-// 20 x 512, window 256, 65 -> 52; 4 x 2048 300 -> 225; 400 67 -> 51; 93 24.0 -> 19.6.
 struct BwdMParams {
   const void* q; const void* k; const void* v; const void* o; const void* go;
   void* dq; void* dk; void* dv;
@@ -272,11 +269,11 @@ __device__ __forceinline__ float dot2w(uint32_t a, uint32_t b, float acc) {  // 
   return fmaf(a1, b1, fmaf(a0, b0, acc));
 }
 
-// A staged tile of 32 rows of 128 bytes: row r keeps its 16-byte chunks xor-ed with the bits 1, 2 and then 3 of r / 2 rotated to the left.
-// Rows r and r + 1 share a 256-byte line of banks.  The transposing reads, 32 lanes on two neighbouring chunks of 8 rows (four pairs of
-// places), are free of conflicts; those of rows are not, 4 cycles for each 16-byte read (32 a tile of 32 keys x 16 rows x 2 heads): the sixteen lanes of a pass
-// are rows of two chunks g and g + 1, and rows 8 apart differ in the bit that those do.
-__device__ __forceinline__ int tile_swizzle(int row) { return ((row & 6) | ((row >> 3) & 1)); }
+// A staged tile of 32 rows of 128 bytes: row r keeps its 16-byte chunks xor-ed with r & 6.  Rows r and r + 1 share a 256-byte line of banks.  Both
+// kinds of read are free of conflicts so: the transposing one takes 32 lanes on two neighbouring chunks of 8 rows at a time, that of rows
+// 16 lanes, rows 0 .. 3 and 12 .. 15 of an even chunk with rows 4 .. 11 of the odd one beside it, or the other way about.  (With bit 3 of the row as
+// the lowest one of the pattern the latter met: 4 cycles for each 16-byte read.)
+__device__ __forceinline__ int tile_swizzle(int row) { return row & 6; }
 
 // Operands of a staged tile.  Rows: [tile A dims 0..31, A dims 32..63, B dims 0..31, B dims 32..63], lane = row m, dims 8 g .. ;
 // transposed: operand t is dim 16 t + m, slots 0..3 are rows 4 g + j of tile A, 4..7 of tile B.
@@ -459,40 +456,40 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void b
   }
 }
 
-// dk / dv.  What bounds it is a tile's chain (LDS reads, products, exponentials, products) at two waves per SIMD: 512 cycles of matrix
-// instructions and about as many of vector instructions of the ~1 700 that a wave takes a tile.  Three waves per SIMD would need 168
-// registers; it takes 240, and with fewer it spills.
-//   * a wave owns 32 keys, so the operands of a query tile (16 KB of LDS reads, all requested at the tile's start) serve two 16-key
-//     columns; the workgroup's waves are 2 key groups x 2 heads of a pair, which add their sums through LDS at the end.  A wave skips
-//     the query tiles that see none of its keys and masks those that see some: 9 of the 10 tiles of a window of 256, two masked;
-//   * the pair's Q and dO tiles and their statistics go from global memory straight into one of three LDS stages, two
-//     iterations ahead of their use (no staging registers; a wave's 1 KB load is 8 rows, the chunk swizzle is applied to the
-//     global address); an iteration waits for the loads of the one before last only.  The first two are requested before the search
-//     for the sequences;
+// dk / dv.  A workgroup owns 32 keys of one kv head, and its NW waves are the heads of the group (GP: 1, 2, 4 or 8, the group padded; two
+// passes over 8 heads with 4 waves) times strides of query tiles:
+//   * a wave multiplies the Q and dO tiles of its own head, which nothing else in the workgroup reads, so it loads them straight into two LDS
+//     stages of its own and waits for its own loads only: no barrier until the sums of the waves meet in LDS behind the loop.  A tile's
+//     operands are all in registers before its products begin, so its stage is filled again, two tiles ahead, while they run;
+//   * whatever the start needs is requested at once - the ends of the sequences (a lane each, up to 64 of them), the keys' own rows, the
+//     first two tiles, which are made again or dropped where a head has fewer;
 //   * the queries a key sees are an index range, key .. min(end of its sequence, key + window), found once per lane: the loop
-//     reads no tables.
-struct DkvStage { unsigned char t[4][4096]; float st[4][64]; };   // Q of head 0, 1, dO of head 0, 1; lse of head 0, 1, D of head 0, 1
-
-template <int DT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void bwd_dkv_mfma(BwdMParams P) {
-  // (one object per stage: the compiler can then tell that reads of one stage do not touch the stage a load is filling)
-  __shared__ __attribute__((aligned(1024))) DkvStage s0, s1, s2;
+//     reads no tables, and only the tiles at the ends of the range are masked.
+// What bounds it: issue (vector instructions 41 % and matrix ones 33 % of the cycles of a SIMD, 70 % of them with some instruction; two waves per
+// SIMD, for three it would have to hold 168 registers instead of 230), and for few keys the launch and its first trip, ~8 us.
+// Before, four waves - two groups of 32 keys, two heads of a pair - shared the tiles behind a barrier per pair of heads and a workgroup
+// of 64 keys walked its queries four times: 1.3 us a step, so a launch lasted as long as its longest row of steps.  us: 2 sequences of up to 778
+// tokens 64.7 -> 25.1; 12 of up to 80 20.3 -> 10.6; 39 of up to 933 105 -> 56; 61 of up to 1024, window 256, 55.3 -> 52.6.
+template <int DT, int GP, int NW>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void bwd_dkv_heads(BwdMParams P) {
+  struct Stage { unsigned char q[4096], g[4096]; float lse[64], nd[64]; };   // 32 rows of 128 B of Q and dO; statistics of 32 (64 loaded)
+  __shared__ __attribute__((aligned(1024))) Stage s0[NW], s1[NW];            // (an object per stage: the compiler can then tell that reads of one do not touch the one a load is filling)
+  constexpr int LOADS = 10;                                                  // of a tile
+  constexpr int HP = GP < NW ? GP : NW, TS = NW / HP;                        // heads at a time, tile strides
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int per = gridDim.x >> 3;
   const int bid = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
   if (bid >= P.n_wg) return;
   const int kvh = bid % P.KH, kb = bid / P.KH;
-  const int n = lane & 15, g = lane >> 4;   // accumulator column n = key, group g = queries 4g .. 4g+3 of a 16-query tile
-  const int kg = wave & 1, hg = wave >> 1;
-  const int G = P.G, GP = (G + 1) >> 1;     // head pairs
+  const int n = lane & 15, g = lane >> 4;
+  const int hq = wave % HP, t0 = wave / HP, G = P.G;
   const float c = P.scale_log2;
+  const int jw = kb * 32, key0 = jw + n;
+  // ---- requested together: the ends of the sequences (lane s: of sequence s, where there are at most 64), K^T / V^T operands, the first two tiles
+  const bool few = P.n_seg <= 64;
+  const int end_l = few ? (int)load_index(P.cu, P.idx64, min(lane + 1, P.n_seg)) : 0;
   int n_end = (int)load_index(P.cu, P.idx64, P.n_seg);
-  n_end = n_end < 0 ? 0 : (n_end > P.N ? P.N : n_end);
-  const int n_beg = (int)load_index(P.cu, P.idx64, 0);   // no query sees a key ahead of it
-  const int jw0 = kb * 64, jw_last = min(jw0 + 63, n_end - 1);
-  const int jw = jw0 + 32 * kg;             // the wave's first key
-  const int key0 = jw + n;                  // column block b: key0 + 16 b
-  // ---- K^T / V^T operands (B side: lane = key, dims 32 s + 8 g ..)
+  const int n_beg = (int)load_index(P.cu, P.idx64, 0);
   pu4 Kb[2][2], Vb[2][2];
 #pragma unroll
   for (int b = 0; b < 2; b++) {
@@ -502,100 +499,113 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     Vb[b][0] = *(const pu4*)((const uint16_t*)P.v + base);
     Vb[b][1] = *(const pu4*)((const uint16_t*)P.v + base + 32);
   }
-  pf4 dK[2][4], dV[2][4];
-#pragma unroll
-  for (int b = 0; b < 2; b++)
-#pragma unroll
-    for (int t = 0; t < 4; t++) dK[b][t] = dV[b][t] = pf4{0.f, 0.f, 0.f, 0.f};
-  // ---- loader: wave w fills tile w and statistics row w of a stage: Q / dO of head w % 2, four loads of 8 rows
-  const int lrow = lane >> 3;
+  // loader: tile t of the wave is rows jw + 32 (t0 + TS t) ..
   const uint32_t rstride = (uint32_t)P.H * 128;
-  const int64_t st_ld = wave < 2 ? P.lse_ld : P.ls;
-  const __amdgpu_buffer_rsrc_t rT = __builtin_amdgcn_make_buffer_rsrc((void*)(wave < 2 ? P.q : P.go), 0, (int)((uint32_t)P.N * rstride), 0x00020000);
-  const __amdgpu_buffer_rsrc_t rS = __builtin_amdgcn_make_buffer_rsrc((void*)(wave < 2 ? P.lse : P.dsum), 0, (int)((st_ld * (P.H - 1) + P.N + 32) * 4), 0x00020000);
-  uint32_t l_off[4], l_st = (uint32_t)(jw0 + (lane & 31)) * 4;   // offsets of the next tile's rows (head 0) and statistics
+  const __amdgpu_buffer_rsrc_t rQ = __builtin_amdgcn_make_buffer_rsrc((void*)P.q, 0, (int)((uint32_t)P.N * rstride), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rG = __builtin_amdgcn_make_buffer_rsrc((void*)P.go, 0, (int)((uint32_t)P.N * rstride), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rL = __builtin_amdgcn_make_buffer_rsrc((void*)P.lse, 0, (int)((P.lse_ld * (P.H - 1) + P.N + 32) * 4), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rD = __builtin_amdgcn_make_buffer_rsrc((void*)P.dsum, 0, (int)((P.ls * (P.H - 1) + P.N + 32) * 4), 0x00020000);
+  uint32_t l_off[4];
+  const uint32_t l_st = (uint32_t)(jw + 32 * t0 + (lane & 31)) * 4;
 #pragma unroll
-  for (int i = 0; i < 4; i++) l_off[i] = (uint32_t)(jw0 + 8 * i + lrow) * rstride + (uint32_t)(((lane & 7) ^ tile_swizzle(8 * i + lrow)) << 4);
-  int f_p = 0;   // head pair of the next request
-  auto issue = [&](DkvStage& S) {   // (rows past the last token come out as zeros: the descriptor's bound)
-    const int head = kvh * G + min(2 * f_p + (wave & 1), G - 1);
+  for (int i = 0; i < 4; i++) {
+    const int r = 8 * i + (lane >> 3);
+    l_off[i] = (uint32_t)(jw + 32 * t0 + r) * rstride + (uint32_t)(((lane & 7) ^ tile_swizzle(r)) << 4);
+  }
+  int f_t = 0, f_h = kvh * G + min(hq, G - 1);   // tile and head of the next request
+  auto issue = [&](Stage* S) {                   // (rows past the last token come out as zeros: the descriptors' bounds)
+    const uint32_t row = (uint32_t)(32 * TS * f_t), at = row * rstride + (uint32_t)f_h * 128;
 #pragma unroll
     for (int i = 0; i < 4; i++)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rT, (__attribute__((address_space(3))) void*)(S.t[wave] + 1024 * i), 16, l_off[i] + (uint32_t)head * 128, 0, 0, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rS, (__attribute__((address_space(3))) void*)S.st[wave], 4, l_st + (uint32_t)(head * st_ld) * 4, 0, 0, 0);
-    if (++f_p == GP) {
-      f_p = 0;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rQ, (__attribute__((address_space(3))) void*)(S[wave].q + 1024 * i), 16, l_off[i] + at, 0, 0, 0);
 #pragma unroll
-      for (int i = 0; i < 4; i++) l_off[i] += 32 * rstride;
-      l_st += 128;
-    }
+    for (int i = 0; i < 4; i++)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rG, (__attribute__((address_space(3))) void*)(S[wave].g + 1024 * i), 16, l_off[i] + at, 0, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rL, (__attribute__((address_space(3))) void*)S[wave].lse, 4, l_st + (row + (uint32_t)(f_h * P.lse_ld)) * 4, 0, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rD, (__attribute__((address_space(3))) void*)S[wave].nd, 4, l_st + (row + (uint32_t)(f_h * P.ls)) * 4, 0, 0, 0);
   };
-  if (jw0 < n_end) {   // (at least one tile: the keys' own)
+  if (hq < G) {   // (whether the keys are seen by these tiles is not known yet: the ends are on their way)
     issue(s0);
+    f_t = 1;
     issue(s1);
   }
-  // ---- sequences of the first and the last key (the last s with cu[s] <= key), 64 probes at a time
-  auto seq_of = [&](int j) {
-    int lo = 0, hi = P.n_seg;   // cu[lo] <= j, and hi == n_seg or cu[hi] > j
-    while (hi - lo > 1) {
-      const int step = (hi - lo + 63) >> 6, at = lo + (lane + 1) * step;
-      const bool below = at < hi && load_index(P.cu, P.idx64, at) <= j;
-      lo += __popcll(__ballot(below)) * step;
-      hi = min(hi, lo + step);
-    }
-    return lo;
-  };
-  // key block b is seen by the n_q[b] queries from the key on
-  int first_end = 0, qend = 0, qend_w = 0;   // end of the sequence of the wave's first key; of the workgroup's and of the wave's queries
+  // ---- the queries that see a key: n_q from the key on
+  n_end = n_end < 0 ? 0 : (n_end > P.N ? P.N : n_end);
+  int first_end = 0, qend = 0;
   uint32_t n_q[2] = {0, 0};
-  if (jw0 < n_end) {
-    const int sf = seq_of(jw0), sl = seq_of(jw_last);
-    const int last_end = min((int)load_index(P.cu, P.idx64, sl + 1), n_end);
-    int hi_q[2] = {last_end, last_end};
+  if (jw < n_end) {
+    const int j_last = min(jw + 31, n_end - 1);
+    auto seq_of = [&](int j) {   // the last sequence s with cu[s] <= j
+      if (few) return (int)__popcll(__ballot(lane + 1 < P.n_seg && end_l <= j));
+      int lo = 0, hi = P.n_seg;
+      while (hi - lo > 1) {      // 64 probes at a time
+        const int step = (hi - lo + 63) >> 6, at = lo + (lane + 1) * step;
+        const bool below = at < hi && load_index(P.cu, P.idx64, at) <= j;
+        lo += __popcll(__ballot(below)) * step;
+        hi = min(hi, lo + step);
+      }
+      return lo;
+    };
+    auto end_of = [&](int s) { return few ? __builtin_amdgcn_readlane(end_l, s) : (int)load_index(P.cu, P.idx64, s + 1); };
+    const int sf = __builtin_amdgcn_readfirstlane(seq_of(jw)), sl = __builtin_amdgcn_readfirstlane(seq_of(j_last));
+    qend = min(end_of(sl), n_end);
+    int hi_q[2] = {qend, qend};
     for (int s = sl - 1; s >= sf; s--) {
-      const int e = (int)load_index(P.cu, P.idx64, s + 1);
+      const int e = end_of(s);
 #pragma unroll
       for (int b = 0; b < 2; b++)
         if (key0 + 16 * b < e) hi_q[b] = e;
     }
     first_end = __builtin_amdgcn_readfirstlane(hi_q[0]);
-    qend = qend_w = last_end;
-    if (P.window > 0) {
-      qend = min(qend, jw_last + P.window);
-      qend_w = min(qend_w, min(jw + 31, n_end - 1) + P.window);
-    }
-    if (jw >= n_end) qend_w = 0;
+    if (P.window > 0) qend = min(qend, j_last + P.window);
 #pragma unroll
     for (int b = 0; b < 2; b++) {
       if (P.window > 0) hi_q[b] = min(hi_q[b], key0 + 16 * b + P.window);
       if (key0 + 16 * b < n_end && key0 + 16 * b >= n_beg) n_q[b] = (uint32_t)(hi_q[b] - key0 - 16 * b);
     }
   }
-  // no mask in a query tile that starts in full_from .. full_to: every query follows every key of the wave, in the first key's sequence and window
-  // (nowhere for a wave whose first keys lie ahead of the first sequence)
+  // no mask in a query tile that starts in full_from .. full_to: every query follows every key, in the first key's sequence and window (nowhere
+  // for first keys that lie ahead of the first sequence)
   const int full_from = jw + 31, full_to = jw < n_beg ? -1 : (P.window > 0 ? min(first_end, jw + P.window) : first_end) - 32;
-  const int n_it = jw0 < n_end ? ((qend - jw0 + 31) >> 5) * GP : 0;
-  int c_t = 0, c_p = 0;   // tile and head pair of the next arithmetic
+  const int nt = qend > jw ? (qend - jw + 31) >> 5 : 0;                                            // query tiles that see some key,
+  const int mine = __builtin_amdgcn_readfirstlane(nt > t0 ? (nt - t0 + TS - 1) / TS : 0);          // this wave's of them
+  const int total = mine * __builtin_amdgcn_readfirstlane(hq < G ? (G - hq + HP - 1) / HP : 0);    // and for all its heads
+  // (the second request was tile 1 of the first head; where there is no such tile it is made again)
+  bool again = false;
+  if (total > 1 && mine == 1) { f_t = 0; f_h += HP; again = true; }
+  auto advance = [&]() {
+    if (++f_t == mine) { f_t = 0; f_h += HP; }
+  };
+  if (again) {
+    __builtin_amdgcn_s_waitcnt(0x0f70);   // (the one that it replaces has landed)
+    issue(s1);
+  }
+  pf4 dK[2][4], dV[2][4];
+#pragma unroll
+  for (int b = 0; b < 2; b++)
+#pragma unroll
+    for (int t = 0; t < 4; t++) dK[b][t] = dV[b][t] = pf4{0.f, 0.f, 0.f, 0.f};
   const TileReads at(n, g);
-  auto step = [&](const DkvStage& S) __attribute__((always_inline)) {
-    const int tq = jw0 + 32 * c_t;
-    const bool live = 2 * c_p + hg < G;   // (an odd last head has no partner)
-    if (++c_p == GP) { c_p = 0; c_t++; }
-    if (!live || tq + 31 < jw || tq >= qend_w) return;   // (no query of the tile sees a key of the wave)
-    const unsigned char* sq = S.t[hg];
-    const unsigned char* sg = S.t[2 + hg];
-    pu4 QA[4], GA[4];
-    at.rows(sq, QA);
-    at.rows(sg, GA);
-    // statistics of this lane's queries tq + 4g + i (tile A) and tq + 16 + 4g + i (tile B)
-    const pf4 lA = *(const pf4*)(S.st[hg] + 4 * g), lB = *(const pf4*)(S.st[hg] + 16 + 4 * g);
-    const pf4 dA = *(const pf4*)(S.st[2 + hg] + 4 * g), dB = *(const pf4*)(S.st[2 + hg] + 16 + 4 * g);
-    pu4 TG[4], TQ[4];
+  int c_t = 0;   // tile of the next arithmetic
+  auto step = [&](Stage* SS, int i) __attribute__((always_inline)) {
+    const int tq = jw + 32 * (t0 + TS * c_t);
+    if (++c_t == mine) c_t = 0;
+    if (i + 1 < total) __builtin_amdgcn_s_waitcnt(0x0f70 | LOADS); else __builtin_amdgcn_s_waitcnt(0x0f70);   // (the next tile's may be on their way)
+    asm volatile("" ::: "memory");
+    const Stage& S = SS[wave];
+    pu4 QA[4], GA[4], TG[4], TQ[4];
+    at.rows(S.q, QA);
+    at.rows(S.g, GA);
+    // statistics of this lane's queries tq + 4g + j (tile A) and tq + 16 + 4g + j (tile B)
+    const pf4 lA = *(const pf4*)(S.lse + 4 * g), lB = *(const pf4*)(S.lse + 16 + 4 * g);
+    const pf4 dA = *(const pf4*)(S.nd + 4 * g), dB = *(const pf4*)(S.nd + 16 + 4 * g);
 #pragma unroll
-    for (int t = 0; t < 4; t++) TG[t] = at.cols(sg, t);
+    for (int t = 0; t < 4; t++) TG[t] = at.cols(S.g, t);
 #pragma unroll
-    for (int t = 0; t < 4; t++) TQ[t] = at.cols(sq, t);
+    for (int t = 0; t < 4; t++) TQ[t] = at.cols(S.q, t);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
+    if (i + 2 < total) { advance(); issue(SS); }
     float p[2][8], ds[2][8];
 #pragma unroll
     for (int b = 0; b < 2; b++) {
@@ -609,11 +619,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       pA = mfma16<DT>(GA[1], Vb[b][1], pA);
       pB = mfma16<DT>(GA[3], Vb[b][1], pB);
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        p[b][i] = __builtin_amdgcn_exp2f(fmaf(sA[i], c, -lA[i]));
-        p[b][4 + i] = __builtin_amdgcn_exp2f(fmaf(sB[i], c, -lB[i]));
-        ds[b][i] = p[b][i] * pA[i];
-        ds[b][4 + i] = p[b][4 + i] * pB[i];
+      for (int j = 0; j < 4; j++) {
+        p[b][j] = __builtin_amdgcn_exp2f(fmaf(sA[j], c, -lA[j]));
+        p[b][4 + j] = __builtin_amdgcn_exp2f(fmaf(sB[j], c, -lB[j]));
+        ds[b][j] = p[b][j] * pA[j];
+        ds[b][4 + j] = p[b][4 + j] * pB[j];
       }
     }
     if (tq < full_from || tq > full_to) {
@@ -622,8 +632,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       for (int b = 0; b < 2; b++) {
         const uint32_t from = (uint32_t)(tq + 4 * g - key0 - 16 * b);
 #pragma unroll
-        for (int i = 0; i < 8; i++)
-          if (from + (i & 3) + 16 * (i >> 2) >= n_q[b]) { p[b][i] = 0.f; ds[b][i] = 0.f; }
+        for (int j = 0; j < 8; j++)
+          if (from + (j & 3) + 16 * (j >> 2) >= n_q[b]) { p[b][j] = 0.f; ds[b][j] = 0.f; }
       }
     }
     pu4 PB[2], SB[2];
@@ -643,50 +653,42 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       for (int b = 0; b < 2; b++) dK[b][t] = mfma16<DT>(TQ[t], SB[b], dK[b][t]);
     }
   };
-  if (n_it > 0) {
-    // iteration i: request i + 2 into the stage that i - 1 used (every wave is done with it: the barrier), multiply i, wait
-    // until i + 1 has landed (its 5 loads are all but the newest 5)
-    __builtin_amdgcn_s_waitcnt(0x0f75);   // vmcnt(5)
-    asm volatile("s_barrier" ::: "memory");
-#define UVMI_DKV(CUR, NEXT2)                                             \
-  do {                                                                   \
-    issue(NEXT2);                                                        \
-    step(CUR);                                                           \
-    __builtin_amdgcn_s_waitcnt(0x0f75);                                  \
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      \
-  } while (0)
-    int it = 0;
-    for (; it + 3 <= n_it; it += 3) {
-      UVMI_DKV(s0, s2);
-      UVMI_DKV(s1, s0);
-      UVMI_DKV(s2, s1);
-    }
-    if (it < n_it) UVMI_DKV(s0, s2);
-    if (it + 1 < n_it) UVMI_DKV(s1, s0);
-#undef UVMI_DKV
-    __builtin_amdgcn_s_waitcnt(0x0f70);   // the requests past the last iteration have landed before LDS is used again
-    __syncthreads();
+  for (int i = 0; i < total; i += 2) {
+    step(s0, i);
+    if (i + 1 < total) step(s1, i + 1);
   }
-  // ---- the two heads of a pair meet in LDS: head 0's wave finishes dk of its keys, head 1's dv
-  float* mine = (float*)(kg ? &s1 : &s0) + (hg ? 0 : 2048) + lane;        // what the partner takes: [register][lane]
-  const float* theirs = (const float*)(kg ? &s1 : &s0) + (hg ? 2048 : 0) + lane;
+  // ---- the waves' sums meet in LDS, [register][lane], 16 KB a wave: wave w finishes registers 64 / NW w .. (dk: 0 .. 31, 16 of a key block)
+  __builtin_amdgcn_s_waitcnt(0x0f70);   // (requests without a tile)
+  __syncthreads();                      // (every wave has read its last tile)
+  auto part = [&](int w) { return (float*)(w < NW / 2 ? (unsigned char*)s0 : (unsigned char*)s1) + (w & (NW / 2 - 1)) * 4096 + lane; };
+  {
+    float* o = part(wave);
 #pragma unroll
-  for (int b = 0; b < 2; b++)
+    for (int b = 0; b < 2; b++)
 #pragma unroll
-    for (int t = 0; t < 4; t++)
+      for (int t = 0; t < 4; t++)
 #pragma unroll
-      for (int i = 0; i < 4; i++) mine[((b * 4 + t) * 4 + i) * 64] = hg ? dK[b][t][i] : dV[b][t][i];
+        for (int j = 0; j < 4; j++) {
+          o[((b * 4 + t) * 4 + j) * 64] = dK[b][t][j];
+          o[(32 + (b * 4 + t) * 4 + j) * 64] = dV[b][t][j];
+        }
+  }
   __syncthreads();
 #pragma unroll
-  for (int b = 0; b < 2; b++) {
-    pf4 acc[4];
+  for (int u = 0; u < 16 / NW; u++) {
+    const int r = 64 / NW * wave + 4 * u, key = key0 + (r & 16);
+    const bool is_v = r >= 32;
+    float acc[4];
 #pragma unroll
-    for (int t = 0; t < 4; t++)
+    for (int j = 0; j < 4; j++) {
+      float v = part(0)[(r + j) * 64];
 #pragma unroll
-      for (int i = 0; i < 4; i++) acc[t][i] = (hg ? dV[b][t][i] : dK[b][t][i]) + theirs[((b * 4 + t) * 4 + i) * 64];
-    const int key = key0 + 16 * b;
+      for (int w = 1; w < NW; w++) v += part(w)[(r + j) * 64];
+      acc[j] = is_v ? v : v * P.scale;
+    }
     if (key < P.N)   // (zeros for padding tokens)
-      store_dims16<DT>(hg ? P.dv : P.dk, ((int64_t)key * P.KH + kvh) * 64 + 4 * g, acc, hg ? 1.0f : P.scale);
+      *(uint2*)((uint16_t*)(is_v ? P.dv : P.dk) + ((int64_t)key * P.KH + kvh) * 64 + 4 * (r & 12) + 4 * g) =
+          uint2{pack2<DT>(acc[0], acc[1]), pack2<DT>(acc[2], acc[3])};
   }
 }
 
@@ -737,7 +739,7 @@ extern "C" int uvmi_prefill_attn_bwd(const uvmi_prefill_attn_bwd_args* a, void* 
       UVMI_REQUIRE(a->fwd_workspace && ((uintptr_t)a->lse % 16) == 0 && a->lse_stride >= a->N + 32 && a->lse_stride % 4 == 0, UVMI_EINVAL,
                    "uvmi_prefill_attn_bwd: lse must be 16-byte aligned with a pitch of at least N + 32 that is a multiple of 4, beside fwd_workspace");
     }
-    // (bwd_dkv_mfma reaches the statistics by 32-bit offsets: those of a wider pitch are formed again)
+    // (bwd_dkv_heads reaches the statistics by 32-bit offsets: those of a wider pitch are formed again)
     if (a->lse && a->lse_stride < (1LL << 29) / a->H) {
       stats = a->lse;
       stats_ld = a->lse_stride;
@@ -757,10 +759,24 @@ extern "C" int uvmi_prefill_attn_bwd(const uvmi_prefill_attn_bwd_args* a, void* 
     if (a->dtype == UVMI_F16) hipLaunchKernelGGL((bwd_dq_mfma<UVMI_F16>), gq, blk4, 0, st, M);
     else hipLaunchKernelGGL((bwd_dq_mfma<UVMI_BF16>), gq, blk4, 0, st, M);
     UVMI_CHECK_LAUNCH("uvmi_prefill_attn_bwd(dq)");
-    M.n_wg = ((a->N + 63) / 64) * a->KH;
+    int cus = uvmi_device_cus();
+    if (cus <= 0) cus = 256;
+    M.n_wg = ((a->N + 31) / 32) * a->KH;
+    // A wave for each of 8 heads where workgroups have compute units of their own, or where there is no window: a launch lasts as long as the keys
+    // that the most queries see, whose row of tiles is then half as long (forward and backward, 16 sequences of up to 1024 tokens, 260
+    // workgroups, 96.7 us against 107.7; 24, 390, 114.5 / 117.4; 39 of up to 933, 582, 139.1 / 142.3; 61, 991, 213.0 / 212.1).  A window
+    // makes the rows short, and two workgroups on a unit cover each other's ends (24 sequences 70.9 / 68.2, 61 138.4 / 129.0).
+    const bool wide = M.n_wg <= cus || (window == 0 && 2 * M.n_wg <= 5 * cus);
     const dim3 gk((unsigned)((M.n_wg + 7) / 8 * 8));
-    if (a->dtype == UVMI_F16) hipLaunchKernelGGL((bwd_dkv_mfma<UVMI_F16>), gk, blk4, 0, st, M);
-    else hipLaunchKernelGGL((bwd_dkv_mfma<UVMI_BF16>), gk, blk4, 0, st, M);
+#define UVMI_DKV_W(DT, GP)                                                                   \
+  do {                                                                                       \
+    if (wide) hipLaunchKernelGGL((bwd_dkv_heads<DT, GP, 8>), gk, dim3(512), 0, st, M);       \
+    else hipLaunchKernelGGL((bwd_dkv_heads<DT, GP, 4>), gk, dim3(256), 0, st, M);            \
+  } while (0)
+#define UVMI_DKV(DT) do { if (G > 4) UVMI_DKV_W(DT, 8); else if (G > 2) UVMI_DKV_W(DT, 4); else if (G > 1) UVMI_DKV_W(DT, 2); else UVMI_DKV_W(DT, 1); } while (0)
+    if (a->dtype == UVMI_F16) UVMI_DKV(UVMI_F16); else UVMI_DKV(UVMI_BF16);
+#undef UVMI_DKV
+#undef UVMI_DKV_W
     UVMI_CHECK_LAUNCH("uvmi_prefill_attn_bwd(dkv)");
     return UVMI_OK;
   }
