@@ -434,6 +434,12 @@ struct uvmi_norm_args {
   void* h_out; void* n_out; int64_t* advance;
 };
 
+/* The extended QKV projection (uvmi_gemm_tn_ex) and the post-processing of its rows (uvmi_qkv_post), which reads gemm->c at post->qkv with the
+ * gates' logits behind q, k, v: as one launch for a few hundred rows of 8 query heads on 1 kv head, else as the two.  What becomes of
+ * gemm->c is unspecified: the one launch does not write it. */
+struct uvmi_qkv_proj_args { const struct uvmi_gemm_args* gemm; const uvmi_qkv_post_args* post; };
+int uvmi_qkv_proj(const struct uvmi_qkv_proj_args* a, void* stream);
+
 /* A sequence of launches in one call: the layers of a pass without a host language between them.  kinds[i] says which
  * entry point args[i] is for; the launches go to `stream` in order, and the first one that fails ends the call with its
  * code and message.  The argument blocks are read before the call returns. */
@@ -442,6 +448,7 @@ struct uvmi_norm_args {
 #define UVMI_OP_QKV_POST 2      /* uvmi_qkv_post_args */
 #define UVMI_OP_PREFILL_ATTN 3  /* uvmi_prefill_attn_args */
 #define UVMI_OP_NORM 4          /* struct uvmi_norm_args */
+#define UVMI_OP_QKV_PROJ 5      /* struct uvmi_qkv_proj_args */
 int uvmi_run_ops(const int* kinds, const void* const* args, int n_ops, void* stream);
 
 /* ------------------------------------------------------------------------------------------------------------

@@ -994,6 +994,73 @@ def test_qkv_post_of_many_rows_equals_that_of_few(dtype, n, cache, rope, ring, h
     assert cache == "none" or float(outs[0][5].float().abs().sum()) > 0
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,cache,norm,rope,ring,has_ve,gate", [
+    (1, "int8", 1, 1, 1, 1, 1), (15, "int8", 0, 1, 0, 1, 1), (17, "16 bit", 1, 1, 1, 0, 1), (93, "int8", 1, 0, 1, 1, 0), (400, "none", 1, 1, 0, 1, 1),
+    (401, "int8", 1, 1, 1, 1, 1), (799, "16 bit", 0, 1, 0, 0, 0), (801, "int8", 1, 1, 1, 1, 1), (1599, "int8", 0, 1, 1, 1, 1), (1601, "int8", 1, 1, 1, 1, 1),
+    (33, "int8, odd pitch", 1, 1, 0, 1, 1)])
+def test_qkv_projection_with_its_post_processing_equals_the_two_launches(dtype, n, cache, norm, rope, ring, has_ve, gate):
+    """uvmi_qkv_proj at the edges of its tiles (16, 32 and 64 rows) and beyond them, where it makes the two launches: everything that is written, bit for
+    bit.  The operands are integers whose products, squares and row scales are exact, so the order of a sum is not seen; where the value
+    embedding has rounded v, |v| may differ in its last places: 64 terms, 64 half units in the last place of 24 bits at most."""
+    import ctypes as C
+    from ultraviolet_amd import _lib as L
+    from ultraviolet_amd.kernels.decode_attn import rope_table
+    from ultraviolet_amd.kernels.gemm import gemm_args
+    g = torch.Generator(device="cuda").manual_seed(n + rope + 2 * ring + 4 * has_ve)
+    H, S, vocab, B = 8, 64, 500, n // 32 + 1
+    sign = lambda *s: (torch.randint(0, 2, s, device="cuda", generator=g) * 2 - 1).float()
+    a = (sign(n, 640) * 2.0 ** (torch.arange(n, device="cuda") % 3)[:, None]).to(dtype)
+    w = (torch.randint(-1, 2, (656, 640), device="cuda", generator=g).float() / 8).to(dtype)
+    at = torch.arange(n, device="cuda")
+    pos, rows = at % 32 + (at // 32) % 3 * 32, at // 32                       # positions 80 .. 95 lie past the table; no two rows share a slot
+    rows[::7] = -1
+    last = pos + torch.randint(0, 100, (n,), device="cuda", generator=g)
+    tok = torch.randint(-3, vocab + 3, (n,), device="cuda", generator=g)
+    ve = torch.randn(vocab, 64, device="cuda", generator=g).to(dtype)
+    inv_freq = (1.0 / (1024.0 ** (torch.arange(16, device="cuda").float() / 16))).contiguous()
+    tab = rope_table(inv_freq, 80, dtype)
+    outs, wrote = [], []
+    for one in (False, True):
+        c = torch.full((n, 656), 77.0, device="cuda", dtype=dtype)
+        q, k, v = torch.zeros(n, H, 64, device="cuda", dtype=dtype), *(torch.zeros(n, 64, device="cuda", dtype=dtype) for _ in range(2))
+        vhat, gt = torch.zeros(n, 64, device="cuda"), torch.zeros(n, H, device="cuda")
+        kc, vc = (torch.zeros(B, 1, S, 65 if "odd" in cache else 64, device="cuda", dtype=torch.int8 if "int8" in cache else dtype) for _ in range(2))
+        ks, vs = (torch.zeros(B, 1, S, device="cuda", dtype=torch.float16) for _ in range(2))
+        p = L.QkvPostArgs()
+        p.qkv, p.dtype, p.qkv_ld, p.ext_logits = c.data_ptr(), L.dtype_code(dtype), 656, 1
+        p.pos, p.rows, p.last_pos, p.inv_freq = pos.data_ptr(), rows.data_ptr(), last.data_ptr() if ring else None, inv_freq.data_ptr()
+        if has_ve:
+            p.ve_table, p.tok = ve.data_ptr(), tok.data_ptr()
+        p.q_out, p.q_dtype, p.k_out, p.v_out = q.data_ptr(), L.dtype_code(dtype), k.data_ptr(), v.data_ptr()
+        if cache != "none":
+            p.k_cache, p.v_cache = kc.data_ptr(), vc.data_ptr()
+            if "int8" in cache:
+                p.k_scale, p.v_scale = ks.data_ptr(), vs.data_ptr()
+        p.scb, p.sch, p.scs, p.ssb, p.ssh, p.S = kc.stride(0), kc.stride(1), kc.stride(2), ks.stride(0), ks.stride(1), S
+        p.n, p.vocab, p.H, p.KH, p.hd, p.d, p.n_pairs = n, vocab, H, 1, 64, 640, 16
+        p.ring, p.has_ve, p.rope, p.eps, p.xsa_eps = ring, has_ve, rope, 1e-6, 1e-4
+        if rope:
+            p.rope_table, p.rope_positions = tab.data_ptr(), tab.size(0)
+        p.vhat_out = vhat.data_ptr()
+        if gate:
+            p.gate_out = gt.data_ptr()
+        ga = gemm_args(a, w, c, norm_eps=0.0 if norm else None)
+        if one:
+            L.check(L.lib().uvmi_qkv_proj(C.byref(L.QkvProjArgs(C.addressof(ga), C.addressof(p))), L.stream_ptr(a)), "uvmi_qkv_proj")
+        else:
+            L.check(L.lib().uvmi_gemm_tn_ex(C.byref(ga), L.stream_ptr(a)), "uvmi_gemm_tn")
+            L.check(L.lib().uvmi_qkv_post(C.byref(p), L.stream_ptr(a)), "uvmi_qkv_post")
+        torch.cuda.synchronize()
+        wrote.append(not bool((c == 77.0).all()))
+        outs.append((q, k, v, gt, kc, vc, ks, vs, vhat))
+    assert wrote == [True, n > 1600 or "odd" in cache]
+    for nm, x, y in zip(("q", "k", "v", "gate", "k cache", "v cache", "k scale", "v scale"), *outs):
+        assert torch.equal(x, y), nm
+    assert float((outs[0][8] - outs[1][8]).abs().max()) <= (64 * 2.0 ** -24 if has_ve else 0.0)
+    assert cache == "none" or n == 1 or float(outs[0][4].float().abs().sum()) > 0
+
+
 @pytest.mark.gpu
 def test_attention_probe_runs_the_engine_shape_and_refuses_the_rest():
     """uvmi_decode_attn_probe (a measurement aid: the kernel's memory stream without its arithmetic, or the reverse)

@@ -145,7 +145,11 @@ class PromptTablesArgs(C.Structure):   # struct uvmi_prompt_tables_args
                 ("check_in", C.c_void_p), ("check_out", C.c_void_p), ("check_zero", C.c_int)]
 
 
-OP_GEMM, OP_DECODE_ATTN, OP_QKV_POST, OP_PREFILL_ATTN, OP_NORM = range(5)   # UVMI_OP_*
+class QkvProjArgs(C.Structure):   # struct uvmi_qkv_proj_args: addresses of a GemmArgs and a QkvPostArgs
+    _fields_ = [("gemm", C.c_void_p), ("post", C.c_void_p)]
+
+
+OP_GEMM, OP_DECODE_ATTN, OP_QKV_POST, OP_PREFILL_ATTN, OP_NORM, OP_QKV_PROJ = range(6)   # UVMI_OP_*
 
 _lib = None
 ABI_VERSION = 8   # UVMI_ABI_VERSION of include/uvmi.h
@@ -192,6 +196,7 @@ def lib() -> C.CDLL:
         L.uvmi_add_norm.argtypes = [C.c_void_p, C.c_void_p, C.c_int, C.c_float, C.c_float, C.c_int64, C.c_int, C.c_float,
                                     C.c_void_p, C.c_void_p, C.c_void_p]
         L.uvmi_qkv_post.argtypes = [C.POINTER(QkvPostArgs), C.c_void_p]
+        L.uvmi_qkv_proj.argtypes = [C.POINTER(QkvProjArgs), C.c_void_p]
         L.uvmi_attn_post.argtypes = [C.c_void_p, C.c_int, C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_void_p, C.c_float,
                                      C.c_int64, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_void_p]
         L.uvmi_swiglu.argtypes = [C.c_void_p, C.c_int, C.c_int64, C.c_int, C.c_void_p, C.c_void_p]
@@ -269,5 +274,5 @@ EXPORTS = ["uvmi_version", "uvmi_last_error", "uvmi_device_cus", "uvmi_quantize_
            "uvmi_kv_write", "uvmi_kv_append", "uvmi_decode_attn", "uvmi_decode_attn_workspace_bytes",
            "uvmi_default_splits", "uvmi_decode_attn_splits", "uvmi_decode_attn_path", "uvmi_attn_oproj_rows", "uvmi_decode_attn_noalloc", "uvmi_decode_attn_probe", "uvmi_prefill_attn", "uvmi_prefill_attn_workspace_bytes",
            "uvmi_prefill_attn_path", "uvmi_fused_sample", "uvmi_philox4x32_10",
-           "uvmi_embed_norm", "uvmi_add_norm", "uvmi_qkv_post", "uvmi_attn_post", "uvmi_swiglu", "uvmi_swiglu_norm",
+           "uvmi_embed_norm", "uvmi_add_norm", "uvmi_qkv_post", "uvmi_qkv_proj", "uvmi_attn_post", "uvmi_swiglu", "uvmi_swiglu_norm",
            "uvmi_prefill_attn_bwd", "uvmi_prefill_attn_bwd_workspace_bytes", "uvmi_sched_compact", "uvmi_sched_commit", "uvmi_sched_commit_dense", "uvmi_sched_admit", "uvmi_sched_expand", "uvmi_sched_harvest", "uvmi_sched_plan_admit", "uvmi_sched_step_plan", "uvmi_run_ops", "uvmi_prompt_tables", "uvmi_rope_table", "uvmi_gemm_tn_supported", "uvmi_gemm_tn", "uvmi_gemm_tn_ex", "uvmi_gemm_tn_path"]

@@ -53,8 +53,6 @@ struct BigParams {
   float eps, ca, cb, cap_c;
 };
 
-#define UVMI_LDSP(p) ((__attribute__((address_space(3))) void*)(p))
-
 // Two dwords x, y per lane in lane groups g = lane / 16 (x0 .. x3, y0 .. y3) -> x = (x0, x2, y0, y2), y = (x1, x3, y1, y3).
 // (permlane32_swap exchanges the upper 32 lanes of its first operand with the lower 32 of its second, permlane16_swap does the
 // same inside each half.)

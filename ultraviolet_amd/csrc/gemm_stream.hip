@@ -41,18 +41,6 @@ struct StreamParams {
   float eps, ca, cb;
 };
 
-#define UVMI_LDSP(p) ((__attribute__((address_space(3))) void*)(p))
-
-// 16 bytes per lane from byte off + at of a buffer to 1 KB of LDS (a template's own code cannot hold the builtin: the host's pass checks it)
-__device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t r, unsigned char* lds, uint32_t off, int at) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, UVMI_LDSP(lds), 16, off, at, 0, 0);
-}
-
-template <int N> __device__ __forceinline__ void wait_vm() {   // all but the newest N loads have landed
-  static_assert(N >= 0 && N < 64, "vmcnt has six bits");
-  __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N >> 4) << 14));
-}
-
 // EPI 0: C = A W^T (M, N).  EPI 1: W rows are [gate 16 | up 16] slabs; C = silu(gate) * up, (M, N / 2); a tile of 16 columns
 // takes 8 gate rows and their 8 up rows.  EPI 2: C = ca * R + cb * (A W^T).  NORM: A stands for its RMS-normalised rows.
 template <int DT, int BM, int BN, int NW, int R, int EPI, bool NORM>

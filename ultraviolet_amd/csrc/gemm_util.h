@@ -10,6 +10,18 @@ typedef __bf16 gb8 __attribute__((ext_vector_type(8)));
 typedef float gf4 __attribute__((ext_vector_type(4)));
 typedef unsigned int gu4 __attribute__((ext_vector_type(4)));
 
+#define UVMI_LDSP(p) ((__attribute__((address_space(3))) void*)(p))
+
+// 16 bytes per lane from byte off + at of a buffer to 1 KB of LDS (a template's own code cannot hold the builtin: the host's pass checks it)
+__device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t r, unsigned char* lds, uint32_t off, int at) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, UVMI_LDSP(lds), 16, off, at, 0, 0);
+}
+
+template <int N> __device__ __forceinline__ void wait_vm() {   // all but the newest N loads have landed
+  static_assert(N >= 0 && N < 64, "vmcnt has six bits");
+  __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N >> 4) << 14));
+}
+
 template <int DT>
 __device__ __forceinline__ gf4 gmfma(gu4 a, gu4 b, gf4 c) {
   if constexpr (DT == UVMI_F16) {

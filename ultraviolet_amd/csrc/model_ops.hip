@@ -15,6 +15,7 @@
 // All of them are HBM/launch-bound and tiny next to the GEMMs and attention; they exist to keep the step at a handful
 // of launches per layer and to write K/V straight into the int8 cache without a round trip through HBM.
 #include "common.h"
+#include "qkv_post.h"
 
 #include <type_traits>
 
@@ -138,20 +139,6 @@ __global__ __launch_bounds__(256) void norm_kernel(const void* __restrict__ xin,
 }
 
 // ------------------------------------------------------------------------------------------------ qkv_post (hd = 64)
-struct QkvArgs {
-  const void* qkv; const void* xn; const void* ve_table; const float* ve_gate; const int64_t* tok;
-  const int64_t* pos; const int64_t* rows; const int64_t* last_pos; const float* inv_freq;
-  void* q_out; void* k_out; void* v_out;
-  int8_t* k_cache; int8_t* v_cache; uint16_t* k_scale; uint16_t* v_scale;
-  const float* gate_w; float* gate_out; float* vhat_out;
-  int64_t scb, sch, scs, ssb, ssh;
-  int64_t n, vocab;
-  int H, KH, d, ve_ch, n_pairs, S, ring, has_ve, rope, q_dt, gate_ch;
-  float eps, xsa_eps;
-  const float* rope_tab; int rope_n;   // optional table of the rounded cos / sin per position (row: cos[n_pairs], sin[n_pairs])
-  int64_t ld; int ext;                 // row pitch of qkv; gate logits read from columns W .. of the row instead of formed from xn
-};
-
 template <int DT>
 __global__ __launch_bounds__(256) void qkv_post_kernel(QkvArgs A) {
   const int lane = threadIdx.x & 63;
@@ -754,7 +741,8 @@ extern "C" int uvmi_add_norm(const void* x, const void* y, int dtype, float a, f
   return norm_run(&n, stream);
 }
 
-extern "C" int uvmi_qkv_post(const uvmi_qkv_post_args* a, void* stream) {
+namespace uvmi {
+int qkv_post_prepare(const uvmi_qkv_post_args* a, QkvArgs* out) {
   UVMI_REQUIRE(a, UVMI_EINVAL, "uvmi_qkv_post: null args");
   UVMI_REQUIRE(a->qkv && a->pos && a->q_out, UVMI_EINVAL, "uvmi_qkv_post: null pointer");
   UVMI_REQUIRE(a->hd == 64, UVMI_EUNSUPPORTED, "uvmi_qkv_post: head_dim %d (only 64)", a->hd);
@@ -774,8 +762,7 @@ extern "C" int uvmi_qkv_post(const uvmi_qkv_post_args* a, void* stream) {
                "uvmi_qkv_post: value-embedding inputs missing");
   UVMI_REQUIRE(!a->k_cache || (a->v_cache && !a->k_scale == !a->v_scale && (a->k_scale || a->dtype != UVMI_F32) && a->S > 0), UVMI_EINVAL,
                "uvmi_qkv_post: incomplete cache arguments");
-  if (a->n == 0) return UVMI_OK;
-  QkvArgs A;
+  QkvArgs& A = *out;
   A.qkv = a->qkv; A.xn = a->xn; A.ve_table = a->ve_table; A.ve_gate = a->ve_gate; A.tok = a->tok; A.pos = a->pos; A.rows = a->rows;
   A.last_pos = a->last_pos; A.inv_freq = a->inv_freq; A.q_out = a->q_out; A.k_out = a->k_out; A.v_out = a->v_out;
   A.k_cache = a->k_cache; A.v_cache = a->v_cache; A.k_scale = a->k_scale; A.v_scale = a->v_scale;
@@ -787,9 +774,21 @@ extern "C" int uvmi_qkv_post(const uvmi_qkv_post_args* a, void* stream) {
   A.rope_n = a->rope_positions;
   A.ld = a->qkv_ld ? a->qkv_ld : qkv_w;
   A.ext = a->ext_logits != 0;
+  return UVMI_OK;
+}
+bool qkv_post_engine_shape(const uvmi_qkv_post_args* a, const QkvArgs& A) {
+  return (a->dtype == UVMI_F16 || a->dtype == UVMI_BF16) && a->q_dtype == a->dtype && a->H == 8 && a->KH == 1 && A.ext &&
+         (!a->rope || (a->n_pairs == 16 && A.rope_tab && ((uintptr_t)A.rope_tab % 16) == 0));
+}
+}  // namespace uvmi
+
+extern "C" int uvmi_qkv_post(const uvmi_qkv_post_args* a, void* stream) {
+  QkvArgs A;
+  const int rc = qkv_post_prepare(a, &A);
+  if (rc) return rc;
+  if (a->n == 0) return UVMI_OK;
   const dim3 grid((unsigned)((a->n + 3) / 4)), blk(256);
-  const bool fast = (a->dtype == UVMI_F16 || a->dtype == UVMI_BF16) && a->q_dtype == a->dtype && a->H == 8 && a->KH == 1 && A.ext &&
-                    (!a->rope || (a->n_pairs == 16 && A.rope_tab && ((uintptr_t)A.rope_tab % 16) == 0));
+  const bool fast = qkv_post_engine_shape(a, A);
   // passes of many rows: 8 per wave, with wide accesses to everything that a row reads or writes.  A wave of 8 rows has the longer chain (2048
   // rows 7.1 us against 4.7, 4096 7.8 against 6.8, 6144 8.9 against 9.1, 8192 9.9 against 11.2)
   const uintptr_t wide = (uintptr_t)a->k_out | (uintptr_t)a->v_out | (uintptr_t)a->vhat_out | (a->has_ve ? (uintptr_t)a->ve_table : 0) |

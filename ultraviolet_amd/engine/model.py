@@ -244,9 +244,10 @@ class UVEngine:
         self._op(L.OP_NORM, args, (), rows="n", **({} if advance is None else {"advance": "pos"}))
 
     def _qkv_post(self, l: int, tok: Tensor, pos: Tensor, rows: Tensor | None, last_pos: Tensor | None, st: KVState | None,
-                  n: int, write_cache: bool = True, ext: bool = False):
+                  n: int, write_cache: bool = True, ext: bool = False, gemm=None):
         """ext: the rows come from the extended projection (buf qkvx), whose last columns are the gates' logits: the
-        normalised block input is then not read."""
+        normalised block input is then not read.  gemm: the argument block of that projection, which has yet to be made: the two
+        are one operation."""
         cfg, b, W = self.cfg, self.buf, self.w.layers[l]
         glob = cfg.is_global(l)
         a = L.QkvPostArgs()
@@ -288,7 +289,15 @@ class UVEngine:
             a.vhat_out, a.xsa_eps = b["vhat"].data_ptr(), float(cfg.xsa_eps)
         if W["attn_gate"] is not None:
             a.gate_w, a.gate_ch, a.gate_out = W["attn_gate"].data_ptr(), cfg.gate_ch, b["gate"].data_ptr()
-        self._op(L.OP_QKV_POST, a, (tok, pos, rows, last_pos), **per_call)
+        keep = (tok, pos, rows, last_pos)
+        if gemm is None:
+            self._op(L.OP_QKV_POST, a, keep, **per_call)
+        else:
+            self._op(L.OP_QKV_PROJ, L.QkvProjArgs(C.addressof(gemm), C.addressof(a)), (gemm, a, keep))
+            if self._rec is not None:
+                self._rec.field(gemm, "M", "n")
+                for field, name in per_call.items():
+                    self._rec.field(a, field, name)
         if write_cache and not fused_write:
             self._write_kv_cast(l, pos, rows, last_pos, st, n)
 
@@ -596,8 +605,12 @@ class UVEngine:
         gc = self.gemm_config
         own_down = n <= self.skinny_rows or n >= self.big_rows or self.fold_down_rows[0] <= n <= self.fold_down_rows[1]
         for l, W in enumerate(self.w.layers):
-            self._project_qkv(l, n, n <= self.fold_qkv_rows, config=gc)
-            self._qkv_post(l, tok, pos, rows, last_pos, st, n, ext=True)
+            gemm = None
+            if n <= self.fold_qkv_rows and last_pos is not None:   # (decode rows alone: the projection of the fused attention's plans, to the same bits)
+                gemm = gemm_args(b["xn" if l == 0 else "x"][:n], W["wqkv_ext"], b["qkvx"][:n], norm_eps=None if l == 0 else self.eps, config=gc)
+            else:
+                self._project_qkv(l, n, n <= self.fold_qkv_rows, config=gc)
+            self._qkv_post(l, tok, pos, rows, last_pos, st, n, ext=True, gemm=gemm)
             self._finish_attn(l, attn(l, b["q"][:n]), x if l > 0 else None)
             self._gemm(zg, W["wo"], x, RESID, resid=x, ca=W["resid_attn"], cb=W["post_attn"], config=gc)
             self._gemm(x, W["gu_il"], act, SWIGLU, norm_eps=self.eps, config=gc)
