@@ -440,6 +440,12 @@ struct uvmi_norm_args {
 struct uvmi_qkv_proj_args { const struct uvmi_gemm_args* gemm; const uvmi_qkv_post_args* post; };
 int uvmi_qkv_proj(const struct uvmi_qkv_proj_args* a, void* stream);
 
+/* Packed attention (uvmi_prefill_attn) and the output projection with its residual update of the rows that it writes (gemm->a is attn->out; RESID): as
+ * one launch for a few hundred tokens of 8 query heads on 1 kv head, else as the two.  What becomes of attn->out is unspecified: the
+ * one launch does not write it. */
+struct uvmi_prefill_attn_o_args { const uvmi_prefill_attn_args* attn; const uvmi_gemm_args* gemm; };
+int uvmi_prefill_attn_o(const struct uvmi_prefill_attn_o_args* a, void* stream);
+
 /* A sequence of launches in one call: the layers of a pass without a host language between them.  kinds[i] says which
  * entry point args[i] is for; the launches go to `stream` in order, and the first one that fails ends the call with its
  * code and message.  The argument blocks are read before the call returns. */
@@ -449,6 +455,7 @@ int uvmi_qkv_proj(const struct uvmi_qkv_proj_args* a, void* stream);
 #define UVMI_OP_PREFILL_ATTN 3  /* uvmi_prefill_attn_args */
 #define UVMI_OP_NORM 4          /* struct uvmi_norm_args */
 #define UVMI_OP_QKV_PROJ 5      /* struct uvmi_qkv_proj_args */
+#define UVMI_OP_PREFILL_ATTN_O 6 /* struct uvmi_prefill_attn_o_args */
 int uvmi_run_ops(const int* kinds, const void* const* args, int n_ops, void* stream);
 
 /* ------------------------------------------------------------------------------------------------------------

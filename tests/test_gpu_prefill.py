@@ -404,3 +404,34 @@ def test_native_varlen_gradient_of_a_changed_input_is_refused():
     first, q.grad = q.grad, None
     o.backward(torch.ones_like(o))
     assert torch.equal(first, q.grad)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("lens,window,post", [([1], 0, True), ([15], 0, True), ([17, 2], 256, True), ([93], 256, True), ([33, 1, 95], 40, False), ([384], 256, True),
+                                              ([330, 54], 0, True), ([385], 256, True), ([500, 268], 0, True), ([769], 256, True)])
+def test_attention_with_the_output_projection_in_its_launch(dtype, lens, window, post):
+    """uvmi_prefill_attn_o at the edges of its 16-token blocks and key tiles, around the 384 and 768 tokens up to which every block's every
+    part of 64 and 128 columns has a compute unit, in place, against the attention and a float64 product of what it writes.  Tolerance: the product's rounding to the type, the
+    update's, and 512 terms in fp32."""
+    import ctypes as C
+    from ultraviolet_amd import _lib as L
+    from ultraviolet_amd.kernels.gemm import RESID, gemm_args
+    from ultraviolet_amd.kernels.varlen_attn import packed_attention, packed_attention_args
+    q, k, v, cu = (t.to(DEV) for t in _case(lens, 8, 1, 64, dtype, seed=sum(lens)))
+    g = torch.Generator(device=DEV).manual_seed(2)
+    N = q.size(0)
+    rnd = lambda *s_: torch.randn(*s_, device=DEV, generator=g)
+    extra = (torch.nn.functional.normalize(v.float(), dim=-1).contiguous(), rnd(N, 8).sigmoid().contiguous(), rnd(8).tanh().contiguous()) if post else None
+    w, x = (rnd(640, 512) / 512 ** 0.5).to(dtype), rnd(N, 640).to(dtype)
+    ws = torch.empty(L.lib().uvmi_prefill_attn_workspace_bytes(N), dtype=torch.uint8, device=DEV)
+    zg = torch.full((N, 512), 77.0, device=DEV, dtype=dtype)
+    y = x.clone()
+    a = packed_attention_args(q, k, v, cu, SC, window, zg.view(N, 8, 64), ws, post=extra)
+    ga = gemm_args(zg, w, y, RESID, resid=y, ca=0.75, cb=1.25)
+    L.check(L.lib().uvmi_prefill_attn_o(C.byref(L.PrefillAttnOArgs(C.addressof(a), C.addressof(ga))), L.stream_ptr(q)), "uvmi_prefill_attn_o")
+    assert bool((zg == 77.0).all()) == (N <= 768)
+    z = packed_attention(q, k, v, cu, SC, window, post=extra).reshape(N, 512)
+    prod = z.double() @ w.double().t()
+    want, ulp = 0.75 * x.double() + 1.25 * prod, 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    bound = ulp * (1.25 * prod.abs() + want.abs()) * 1.01 + 512 * 2.0 ** -24 * (z.double().abs() @ w.double().abs().t())
+    assert bool(((y.double() - want).abs() <= bound).all()), float(((y.double() - want).abs() / bound).max())

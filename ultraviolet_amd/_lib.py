@@ -149,7 +149,11 @@ class QkvProjArgs(C.Structure):   # struct uvmi_qkv_proj_args: addresses of a Ge
     _fields_ = [("gemm", C.c_void_p), ("post", C.c_void_p)]
 
 
-OP_GEMM, OP_DECODE_ATTN, OP_QKV_POST, OP_PREFILL_ATTN, OP_NORM, OP_QKV_PROJ = range(6)   # UVMI_OP_*
+class PrefillAttnOArgs(C.Structure):   # struct uvmi_prefill_attn_o_args: addresses of a PrefillAttnArgs and a GemmArgs
+    _fields_ = [("attn", C.c_void_p), ("gemm", C.c_void_p)]
+
+
+OP_GEMM, OP_DECODE_ATTN, OP_QKV_POST, OP_PREFILL_ATTN, OP_NORM, OP_QKV_PROJ, OP_PREFILL_ATTN_O = range(7)   # UVMI_OP_*
 
 _lib = None
 ABI_VERSION = 8   # UVMI_ABI_VERSION of include/uvmi.h
@@ -176,6 +180,7 @@ def lib() -> C.CDLL:
         L.uvmi_decode_attn_noalloc.argtypes = [C.POINTER(AttnArgs), C.c_void_p]
         L.uvmi_decode_attn_probe.argtypes = [C.POINTER(AttnArgs), C.c_int, C.c_void_p]
         L.uvmi_prefill_attn.argtypes = [C.POINTER(PrefillAttnArgs), C.c_void_p]
+        L.uvmi_prefill_attn_o.argtypes = [C.POINTER(PrefillAttnOArgs), C.c_void_p]
         L.uvmi_prefill_attn_path.argtypes = [C.POINTER(PrefillAttnArgs)]
         L.uvmi_prefill_attn_workspace_bytes.restype = C.c_size_t
         L.uvmi_prefill_attn_workspace_bytes.argtypes = [C.c_int]
@@ -272,7 +277,7 @@ def require_cuda(*ts: torch.Tensor) -> None:
 
 EXPORTS = ["uvmi_version", "uvmi_last_error", "uvmi_device_cus", "uvmi_quantize_rows", "uvmi_dequantize_rows",
            "uvmi_kv_write", "uvmi_kv_append", "uvmi_decode_attn", "uvmi_decode_attn_workspace_bytes",
-           "uvmi_default_splits", "uvmi_decode_attn_splits", "uvmi_decode_attn_path", "uvmi_attn_oproj_rows", "uvmi_decode_attn_noalloc", "uvmi_decode_attn_probe", "uvmi_prefill_attn", "uvmi_prefill_attn_workspace_bytes",
+           "uvmi_default_splits", "uvmi_decode_attn_splits", "uvmi_decode_attn_path", "uvmi_attn_oproj_rows", "uvmi_decode_attn_noalloc", "uvmi_decode_attn_probe", "uvmi_prefill_attn", "uvmi_prefill_attn_o", "uvmi_prefill_attn_workspace_bytes",
            "uvmi_prefill_attn_path", "uvmi_fused_sample", "uvmi_philox4x32_10",
            "uvmi_embed_norm", "uvmi_add_norm", "uvmi_qkv_post", "uvmi_qkv_proj", "uvmi_attn_post", "uvmi_swiglu", "uvmi_swiglu_norm",
            "uvmi_prefill_attn_bwd", "uvmi_prefill_attn_bwd_workspace_bytes", "uvmi_sched_compact", "uvmi_sched_commit", "uvmi_sched_commit_dense", "uvmi_sched_admit", "uvmi_sched_expand", "uvmi_sched_harvest", "uvmi_sched_plan_admit", "uvmi_sched_step_plan", "uvmi_run_ops", "uvmi_prompt_tables", "uvmi_rope_table", "uvmi_gemm_tn_supported", "uvmi_gemm_tn", "uvmi_gemm_tn_ex", "uvmi_gemm_tn_path"]

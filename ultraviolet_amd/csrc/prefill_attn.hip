@@ -34,6 +34,7 @@
 // packed K/V as a batch-stride-0 "cache".
 #include "common.h"
 #include "attn_mfma_util.h"
+#include "gemm_util.h"
 
 #include <climits>
 
@@ -48,6 +49,11 @@ struct PrefillParams {
   float scale_log2;
   const float* post_vhat; const float* post_gate; const float* post_xsa;  // fused Attention.post epilogue when post_vhat != null
   float* lse_out; int64_t lse_stride;  // optional (H, lse_stride) fp32: log2 of each row's sum of exp2(scale_log2 s) (the backward's statistics)
+  // the output projection and residual update of the rows in the same launch (OP): y = o_ca r + o_cb (attention W^T), o_n columns
+  const void* o_w; const void* o_r; void* o_out;
+  int64_t o_ldw, o_ldr, o_ldo;
+  int o_n;
+  float o_ca, o_cb;
 };
 
 // seg_start[i] = cu[s] for the last s with cu[s] <= i (empty sequences are skipped); pidx[i] = i.
@@ -75,10 +81,18 @@ __device__ __forceinline__ float xmaximum(float v) {
 }
 __device__ __forceinline__ float max3(float a, float b, float c) { return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c); }
 
-template <int DT, int ODT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void prefill_attn_mfma_hd64(PrefillParams P) {
+// OP: blockIdx.y is a part of 64 OP columns of the output projection.  Every part's workgroup computes the block's attention for itself (8 heads on 1
+// kv head: a wave has two of them, a workgroup all) while its rows of the weight go straight into LDS behind the first two tiles; the
+// heads' outputs meet in LDS, and a wave forms 16 OP columns of the block's 16 rows from them.  For passes whose blocks leave most of
+// the device idle: what is repeated takes no time, and a launch of the projection alone lasts 3.4 us at 93 rows, nearly all of it its start
+// and a trip for the weights.  A whole prefill, us: 30 tokens 267 -> 245, 93 296 -> 274, 300 347 -> 323 (64 columns a part: up to 384 tokens),
+// 500 400 -> 377, 700 444 -> 422 (128: up to 768; 780 tokens, where an XCD has more workgroups than compute units, 469 -> 479).
+template <int DT, int ODT, int OP>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OP ? 1 : 4))) void prefill_attn_mfma_hd64(PrefillParams P) {
   // one object per stage: the compiler can then tell that reads of one do not touch the one a load is filling
   __shared__ __attribute__((aligned(1024))) unsigned char s0[2][4096], s1[2][4096], s2[2][4096];  // [K, V][32 keys x 128 B]
+  constexpr int OW = 16 * OP;   // weight rows of a wave, a load each
+  __shared__ __attribute__((aligned(1024))) unsigned char sw[OP ? 4 * OW * 1024 : 16];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -123,6 +137,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void p
   }
   int lo_n = P.seg_start[rowc];
   int lo0 = P.seg_start[row0];
+  const int on = OP * (64 * (int)blockIdx.y + 16 * wave);   // the wave's first output column
+  uint2 ores[OP ? OP : 1];
+#pragma unroll
+  for (int j = 0; j < OP; j++) ores[j] = *(const uint2*)((const uint16_t*)P.o_r + (int64_t)rowc * P.o_ldr + on + 16 * j + 4 * g);
   __builtin_amdgcn_sched_barrier(0);
   // ---- key ranges: the row's, the block's, and the workgroup's from its first row's lower bound (the smallest) to its last row
   if (P.window > 0 && row - P.window + 1 > lo_n) lo_n = row - P.window + 1;
@@ -155,6 +173,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void p
   };
   issue(s0, 0);
   if (nk > 1) issue(s1, 1);
+  if constexpr (OP > 0) {   // row i of the wave's weight rows, 1 KB, keeps its 16-byte chunks xor-ed with i % 16
+    const __amdgpu_buffer_rsrc_t rO = __builtin_amdgcn_make_buffer_rsrc((void*)P.o_w, 0, (int)((uint32_t)(P.o_n - 1) * (uint32_t)P.o_ldw * 2 + 1024u), 0x00020000);
+#pragma unroll
+    for (int i = 0; i < OW; i++) load_lds16(rO, sw + (wave * OW + i) * 1024, (uint32_t)(on + i) * (uint32_t)P.o_ldw * 2 + (uint32_t)((lane ^ (i & 15)) << 4), 0);
+  }
 
   pf4 O[HPW][4];
   float mrun[HPW], lrun[HPW];
@@ -235,7 +258,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void p
   // iteration k: tile k has landed (own loads: the wait, which leaves tile k + 1's in flight; the other waves': the barrier) and every
   // wave is done with tile k - 1, whose stage takes tile k + 2
   auto iteration = [&](unsigned char (*S)[4096], unsigned char (*SN)[4096], int k) {
-    if (k + 1 < nk) __builtin_amdgcn_s_waitcnt(0x0f72); else __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(2) / (0)
+    if (OP > 0 && k < 2) {   // (the weight rows were requested behind tile 1)
+      if (k + 1 < nk) wait_vm<2 + OW>(); else wait_vm<OW>();
+    } else {
+      if (k + 1 < nk) wait_vm<2>(); else wait_vm<0>();
+    }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if (k + 2 < nk) issue(SN, k + 2);
     step(S, k);
@@ -248,6 +275,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void p
   }
   if (k < nk) iteration(s0, s2, k);
   if (k + 1 < nk) iteration(s1, s0, k + 1);
+  if constexpr (OP > 0) __syncthreads();   // (the stages take the heads' outputs)
 
   // ---- normalise and store: lane (row m, group g) holds head dims 16 t + 4 g + i, t, i = 0 .. 3
   // Optional epilogue, as in the decode kernel: z (rounded to the activation type, as the attention output tensor would be)
@@ -291,6 +319,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void p
 #pragma unroll
       for (int i = 0; i < 16; i++) o[i] *= gate[hh];
     }
+    if constexpr (OP > 0) {   // into the tiles' first two stages, four heads each: 16 rows of 512 bytes, chunks xor-ed with the row
+      unsigned char* sz = (unsigned char*)(hg < 2 ? s0 : s1) + m * 512 + 8 * (g & 1);
+#pragma unroll
+      for (int t = 0; t < 4; t++)
+        *(uint2*)(sz + (((8 * (hq & 3) + 2 * t + (g >> 1)) ^ m) << 4)) = uint2{pack2<DT>(o[4 * t], o[4 * t + 1]), pack2<DT>(o[4 * t + 2], o[4 * t + 3])};
+      continue;
+    }
     if (hq >= G || !row_ok) continue;
     const int64_t off = (int64_t)row * P.son + (int64_t)(kvh * G + hq) * P.soh + 4 * g;
     if (ODT == UVMI_F32) {
@@ -304,6 +339,32 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void p
       uint16_t* op = (uint16_t*)P.out + off;
 #pragma unroll
       for (int i = 0; i < 4; i++) *(uint2*)(op + 16 * i) = uint2{w[2 * i], w[2 * i + 1]};
+    }
+  }
+  if constexpr (OP > 0) {
+    wait_vm<0>();   // (the wave's own weight rows)
+    __syncthreads();
+    gf4 y[OP][2];
+#pragma unroll
+    for (int j = 0; j < OP; j++) y[j][0] = y[j][1] = gf4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < 16; s++) {
+      const gu4 z = *(const gu4*)((const unsigned char*)(s < 8 ? s0 : s1) + m * 512 + (((4 * (s & 7) + g) ^ m) << 4));
+#pragma unroll
+      for (int j = 0; j < OP; j++) {
+        const gu4 w = *(const gu4*)(sw + (wave * OW + 16 * j + m) * 1024 + (((4 * s + g) ^ m) << 4));
+        y[j][s & 1] = gmfma<DT>(w, z, y[j][s & 1]);   // (C^T: the lane has columns 16 j + 4 g .. of row m)
+      }
+    }
+    if (!row_ok) return;
+#pragma unroll
+    for (int j = 0; j < OP; j++) {
+      float x[4], q[4];
+      gunpack<DT>(ores[j].x, x[0], x[1]);
+      gunpack<DT>(ores[j].y, x[2], x[3]);
+#pragma unroll
+      for (int t = 0; t < 4; t++) q[t] = P.o_ca * x[t] + P.o_cb * ground<DT>(y[j][0][t] + y[j][1][t]);
+      *(uint2*)((uint16_t*)P.o_out + (int64_t)row * P.o_ldo + on + 16 * j + 4 * g) = uint2{gpack<DT>(q[0], q[1]), gpack<DT>(q[2], q[3])};
     }
   }
 }
@@ -356,8 +417,23 @@ static bool prefill_mfma_ok(const uvmi_prefill_attn_args* a) {
   return true;
 }
 
-static int launch_mfma(const uvmi_prefill_attn_args* a, const int32_t* seg_start, float* lse_out, int64_t lse_stride, hipStream_t st) {
-  PrefillParams P;
+// 64-column pieces of an output projection's part that rides in the attention's launch, 0: a launch of its own.  8 heads on 1 kv head, the projection
+// of what the attention writes, and a compute unit for every block's every part, the smaller one if it can.
+static int oproj_pieces(const uvmi_prefill_attn_args* a, const uvmi_gemm_args* o) {
+  if (a->H != 8 || a->KH != 1 || a->out_dtype != a->q_dtype || a->lse_out || a->soh != 64) return 0;
+  if (!uvmi_gemm_tn_supported(o->dtype, o->M, o->N, o->K, o->lda, o->ldw, o->ldc, o->epilogue)) return 0;
+  if (o->epilogue != UVMI_GEMM_RESID || o->norm_a || o->config != 0 || o->dtype != a->q_dtype || o->M != a->N || o->K != 512 || o->N % 64 != 0) return 0;
+  if (o->a != a->out || o->lda != a->son || !o->w || !o->c || !o->resid) return 0;
+  if (((uintptr_t)o->w % 16) != 0 || ((uintptr_t)o->c % 8) != 0 || ((uintptr_t)o->resid % 8) != 0 || o->ldr % 4 != 0 || o->ldr < o->N) return 0;
+  int cus = uvmi_device_cus();
+  if (cus <= 0) cus = 256;
+  for (int pieces : {1, 2})
+    if (o->N % (64 * pieces) == 0 && (int64_t)((a->N + 127) / 128) * (o->N / (64 * pieces)) <= cus / 8) return pieces;   // (of an XCD's blocks)
+  return 0;
+}
+
+static int launch_mfma(const uvmi_prefill_attn_args* a, const int32_t* seg_start, float* lse_out, int64_t lse_stride, hipStream_t st, const uvmi_gemm_args* o = nullptr, int pieces = 0) {
+  PrefillParams P = {};
   P.q = a->q; P.k = a->k; P.v = a->v; P.out = a->out; P.seg_start = seg_start;
   P.sqn = a->sqn; P.sqh = a->sqh; P.skn = a->skn; P.skh = a->skh; P.svn = a->svn; P.svh = a->svh; P.son = a->son; P.soh = a->soh;
   P.N = a->N; P.H = a->H; P.KH = a->KH; P.G = a->H / a->KH; P.window = a->window;
@@ -372,11 +448,24 @@ static int launch_mfma(const uvmi_prefill_attn_args* a, const int32_t* seg_start
   const unsigned nblk = (unsigned)((n_wg + 7) / 8 * 8);
   const dim3 grid(nblk), blk(256);
   const int od = a->out_dtype;
-#define UVMI_L(QD)                                                                                                \
-  do {                                                                                                            \
-    if (od == UVMI_F16) hipLaunchKernelGGL((prefill_attn_mfma_hd64<QD, UVMI_F16>), grid, blk, 0, st, P);          \
-    else if (od == UVMI_BF16) hipLaunchKernelGGL((prefill_attn_mfma_hd64<QD, UVMI_BF16>), grid, blk, 0, st, P);   \
-    else hipLaunchKernelGGL((prefill_attn_mfma_hd64<QD, UVMI_F32>), grid, blk, 0, st, P);                         \
+  if (o) {
+    P.o_w = o->w; P.o_r = o->resid; P.o_out = o->c; P.o_ldw = o->ldw; P.o_ldr = o->ldr; P.o_ldo = o->ldc; P.o_n = o->N; P.o_ca = o->ca; P.o_cb = o->cb;
+    const dim3 parts(nblk, (unsigned)(o->N / (64 * pieces)));
+#define UVMI_LO(DT)                                                                                                       \
+  do {                                                                                                                    \
+    if (pieces == 1) hipLaunchKernelGGL((prefill_attn_mfma_hd64<DT, DT, 1>), parts, blk, 0, st, P);                       \
+    else hipLaunchKernelGGL((prefill_attn_mfma_hd64<DT, DT, 2>), parts, blk, 0, st, P);                                   \
+  } while (0)
+    if (a->q_dtype == UVMI_F16) UVMI_LO(UVMI_F16); else UVMI_LO(UVMI_BF16);
+#undef UVMI_LO
+    UVMI_CHECK_LAUNCH("uvmi_prefill_attn_o");
+    return UVMI_OK;
+  }
+#define UVMI_L(QD)                                                                                                       \
+  do {                                                                                                                   \
+    if (od == UVMI_F16) hipLaunchKernelGGL((prefill_attn_mfma_hd64<QD, UVMI_F16, 0>), grid, blk, 0, st, P);          \
+    else if (od == UVMI_BF16) hipLaunchKernelGGL((prefill_attn_mfma_hd64<QD, UVMI_BF16, 0>), grid, blk, 0, st, P);   \
+    else hipLaunchKernelGGL((prefill_attn_mfma_hd64<QD, UVMI_F32, 0>), grid, blk, 0, st, P);                         \
   } while (0)
   if (a->q_dtype == UVMI_F16) UVMI_L(UVMI_F16); else UVMI_L(UVMI_BF16);
 #undef UVMI_L
@@ -413,10 +502,11 @@ extern "C" int uvmi_prefill_attn_path(const uvmi_prefill_attn_args* a) {
   return prefill_mfma_ok(a) ? 1 : 0;
 }
 
-extern "C" int uvmi_prefill_attn(const uvmi_prefill_attn_args* a, void* stream) {
+// o: the output projection that follows (uvmi_prefill_attn_o)
+static int prefill_attn_run(const uvmi_prefill_attn_args* a, const uvmi_gemm_args* o, void* stream) {
   int rc = check_prefill(a);
   if (rc) return rc;
-  if (a->N == 0) return UVMI_OK;
+  if (a->N == 0) return o ? uvmi_gemm_tn_ex(o, stream) : UVMI_OK;
   hipStream_t st = (hipStream_t)stream;
   int32_t* seg_start = (int32_t*)a->workspace;
   int32_t* pidx = (int32_t*)((char*)a->workspace + ((size_t)a->N * 4 + 255) / 256 * 256);
@@ -440,8 +530,18 @@ extern "C" int uvmi_prefill_attn(const uvmi_prefill_attn_args* a, void* stream) 
     d.out = a->out; d.out_dtype = a->out_dtype; d.sob = a->son; d.soh = a->soh;
     d.B = a->N; d.H = a->H; d.KH = a->KH; d.S = a->N; d.hd = a->hd;
     d.scale = a->scale; d.window = a->window; d.ring = 0; d.num_splits = 1;
-    return uvmi_decode_attn(&d, stream);
+    rc = uvmi_decode_attn(&d, stream);
+    return rc || !o ? rc : uvmi_gemm_tn_ex(o, stream);
   }
-  return launch_mfma(a, seg_start, a->lse_out, a->lse_stride, st);
+  if (const int pieces = o ? oproj_pieces(a, o) : 0) return launch_mfma(a, seg_start, nullptr, 0, st, o, pieces);
+  rc = launch_mfma(a, seg_start, a->lse_out, a->lse_stride, st);
+  return rc || !o ? rc : uvmi_gemm_tn_ex(o, stream);
+}
+
+extern "C" int uvmi_prefill_attn(const uvmi_prefill_attn_args* a, void* stream) { return prefill_attn_run(a, nullptr, stream); }
+
+extern "C" int uvmi_prefill_attn_o(const struct uvmi_prefill_attn_o_args* a, void* stream) {
+  UVMI_REQUIRE(a && a->attn && a->gemm, UVMI_EINVAL, "uvmi_prefill_attn_o: null args");
+  return prefill_attn_run(a->attn, a->gemm, stream);
 }
 

@@ -390,11 +390,12 @@ class UVEngine:
         return (cfg.xsa and self.dtype in (torch.bfloat16, torch.float16) and self.q_dtype == self.dtype and cfg.head_dim == 64
                 and cfg.n_heads // cfg.n_kv_heads <= 8)
 
-    def prompt_attention(self, l: int, q: Tensor, N: int, cu: Tensor):
+    def prompt_attention(self, l: int, q: Tensor, N: int, cu: Tensor, gemm=None):
         """Causal (windowed on local layers) attention of the N packed prompt tokens at the head of the call's buffers over
         their own unquantized K / V (buf k, v).  Where the MFMA kernel runs (16-bit engine) XSA and the gate ride in its
         epilogue - it writes buf zg[:N] and None is returned; otherwise the plain attention output is returned for
-        _attn_post.  The segment table of cu is built by layer 0's call and reused by the other layers of the pass."""
+        _attn_post.  The segment table of cu is built by layer 0's call and reused by the other layers of the pass.  gemm: the argument
+        block of the output projection of buf zg (prompt_attention_plannable passes without decode rows): the two are one operation."""
         cfg, b, W = self.cfg, self.buf, self.w.layers[l]
         w = 0 if cfg.is_global(l) else cfg.window
         if self.prompt_attention_plannable():
@@ -403,7 +404,15 @@ class UVEngine:
             out = b["zg"][:N].view(N, cfg.n_heads, cfg.head_dim)
             a = packed_attention_args(q, b["k"][:N], b["v"][:N], cu, cfg.attn_scale, w, out, self.pf_ws, segments_ready=l > 0,
                                       post=(b["vhat"][:N], None if W["attn_gate"] is None else b["gate"][:N], W["xsa"]))
-            self._op(L.OP_PREFILL_ATTN, a, (q, out, cu), N="Np", cu_seqlens="cu", n_seg="n_seg")
+            per_call = dict(N="Np", cu_seqlens="cu", n_seg="n_seg")
+            if gemm is None:
+                self._op(L.OP_PREFILL_ATTN, a, (q, out, cu), **per_call)
+            else:
+                self._op(L.OP_PREFILL_ATTN_O, L.PrefillAttnOArgs(C.addressof(a), C.addressof(gemm)), (gemm, a, q, out, cu))
+                if self._rec is not None:
+                    self._rec.field(gemm, "M", "n")
+                    for field, name in per_call.items():
+                        self._rec.field(a, field, name)
             return None
         return packed_attention(q, b["k"][:N], b["v"][:N], cu, cfg.attn_scale, w, workspace=self.pf_ws, segments_ready=l > 0)
 
@@ -472,14 +481,14 @@ class UVEngine:
                                (b["vhat"][:n], None if W["attn_gate"] is None else b["gate"][:n], W["xsa"], out.dtype), any_ring=st.short_ring(l))
 
     def _trunk(self, tok: Tensor, pos: Tensor, n: int, attn, rows=None, last_pos=None, st: KVState | None = None,
-               fused_attn=None, defer_final_norm: bool = False, advance: bool = False, final_norm: bool = True) -> Tensor:
+               fused_attn=None, defer_final_norm: bool = False, advance: bool = False, final_norm: bool = True, oproj: bool = False) -> Tensor:
         """n token rows through all layers; attn(l, q (n, H, hd)) -> z (n, H, hd), or None when it wrote the post-processed
         result to buf zg itself, or a list of (first row, z) of the parts that it left to _attn_post; it runs after K/V of the
         layer have been appended to the cache and written unquantized to buf k / v.  Returns the final normed hidden (n, d) (a
         buffer).  defer_final_norm: a plan whose last block leaves the hidden un-normalised returns it as it is and sets self.hidden_is_raw - the caller's head GEMM then carries the final
         norm as the row scale of its product (head_of), and the norm launch goes away; final_norm False: likewise at any row
         count, for a caller that norms the few rows it needs itself (_normed).  advance: the final norm's launch counts pos up
-        by one."""
+        by one.  oproj: attn(l, q, gemm) makes the output projection of the rows too (_layers_packed)."""
         cfg, b = self.cfg, self.buf
         assert n <= self.max_tokens
         self._embed_norm(tok, n)
@@ -493,7 +502,7 @@ class UVEngine:
         elif kind == "folded":
             self._layers_folded(n, fused_attn)
         elif kind == "packed":
-            self._layers_packed(n, tok, pos, rows, last_pos, st, attn)
+            self._layers_packed(n, tok, pos, rows, last_pos, st, attn, oproj)
         else:
             raw = self._layers_plain(n, tok, pos, rows, last_pos, st, attn, fused_attn)
         if raw:
@@ -594,12 +603,12 @@ class UVEngine:
         else:
             self._lib_gemm(n, lambda n: torch.addmm(b["x"][:n], b["act"][:n], W["down"].t(), beta=W["resid_mlp"], alpha=W["post_mlp"], out=b["x"][:n]))
 
-    def _layers_packed(self, n: int, tok, pos, rows, last_pos, st, attn):
+    def _layers_packed(self, n: int, tok, pos, rows, last_pos, st, attn, oproj: bool = False):
         """Prompts, mixed passes and the unfused attention of a 16-bit engine: the extended projection with the pre-norm in it,
         the post-processing kernel (which takes the gates' logits from the projection and appends to the cache), the
         attention launches, output and down projections with the residual update in place, gate-up with the pre-norm and
         the SwiGLU.  The normalised hidden is not written between blocks (_finish_attn forms it for a layer whose attention
-        leaves its epilogue to _attn_post; layer 0 has the embedding's)."""
+        leaves its epilogue to _attn_post; layer 0 has the embedding's).  oproj: attn also takes the output projection (prompt_attention's gemm)."""
         cfg, b = self.cfg, self.buf
         x, zg, act = b["x"][:n], b["zg"][:n], b["act"][:n]
         gc = self.gemm_config
@@ -611,8 +620,11 @@ class UVEngine:
             else:
                 self._project_qkv(l, n, n <= self.fold_qkv_rows, config=gc)
             self._qkv_post(l, tok, pos, rows, last_pos, st, n, ext=True, gemm=gemm)
-            self._finish_attn(l, attn(l, b["q"][:n]), x if l > 0 else None)
-            self._gemm(zg, W["wo"], x, RESID, resid=x, ca=W["resid_attn"], cb=W["post_attn"], config=gc)
+            if oproj:   # (the attention's launch, or one behind it)
+                attn(l, b["q"][:n], gemm_args(zg, W["wo"], x, RESID, resid=x, ca=W["resid_attn"], cb=W["post_attn"], config=gc))
+            else:
+                self._finish_attn(l, attn(l, b["q"][:n]), x if l > 0 else None)
+                self._gemm(zg, W["wo"], x, RESID, resid=x, ca=W["resid_attn"], cb=W["post_attn"], config=gc)
             self._gemm(x, W["gu_il"], act, SWIGLU, norm_eps=self.eps, config=gc)
             self._down(l, n, own_down)
 
@@ -930,11 +942,11 @@ class UVEngine:
     def _prefill(self, pk: dict, st: KVState) -> Tensor:
         N = pk["N"]
 
-        def attn(l, q):
-            return self.prompt_attention(l, q, N, pk["cu"])
+        def attn(l, q, gemm=None):
+            return self.prompt_attention(l, q, N, pk["cu"], gemm)
 
         tok, pos, row, last, cu = pk["tok"], pk["pos"], pk["row"], pk["last"], pk["cu"]
-        run = lambda: self._trunk(tok, pos, N, attn, rows=row, last_pos=last, st=st, final_norm=False)
+        run = lambda: self._trunk(tok, pos, N, attn, rows=row, last_pos=last, st=st, final_norm=False, oproj=self.prompt_attention_plannable())
         if self._pass_kind(N, False, st) == "packed" and self.prompt_attention_plannable() and self._append_fused(st):
             h = self._planned("prefill", st, "packed", N, dict(n=N, Np=N, tok=tok.data_ptr(), pos=pos.data_ptr(), rows=row.data_ptr(), last=last.data_ptr(),
                                                                 cu=cu.data_ptr(), n_seg=cu.numel() - 1), run)
