@@ -191,11 +191,15 @@ __global__ __launch_bounds__(NT) void sample_kernel(const void* a_x, int64_t a_s
 // (48 bits, 32.32 fixed point: sums do not depend on the order of the additions) of its keys in one 64-bit word, so one
 // histogram serves both selects: the nucleus walk starts on the histograms that the top-k walk left and only builds new
 // ones for the bins in which it ends elsewhere.  200 rows x 32768, top_k 50 + top_p 0.95: 203 us for eleven sweeps of the
-// row with 8-bit digits, one thread walking each histogram; 13.6 us as it is now (top-k cuts of at most 256 through the
-// candidate list: the exponentials 2.8, the bound 2, collecting and ranking 2.5, the draw 2.5, launch and loads 4); 23 us for
-// top_p alone, which needs the histogram of the whole row (9 us: 512 wave-wide 64-bit LDS atomics of ~40 clocks each).
+// row with 8-bit digits, one thread walking each histogram; 13.9 us with a bound from 4096 64-bit bins that every thread scanned,
+// ranks and masses gathered by LDS atomics and the chosen chunk read again for the draw; 11.9 us as it is now, where the bound is
+// 256 bins that a wave scans in four words a lane, ranks are counted by ballots, one wave walks the sorted masses and the wave that
+// holds the chosen chunk draws from its registers (75 rows, top_k 50 alone: 13.2 -> 10.9).  What is left: launch and loads 4, the exponentials
+// 2.8, the selects and barriers behind them; 22 - 23 us for top_p alone, which needs the histogram of the whole row (9 us: 512
+// wave-wide 64-bit LDS atomics of ~40 clocks each).
 constexpr unsigned long long BIN_ONE = 1ull << 48, BIN_MASS = BIN_ONE - 1;
 constexpr unsigned int CAND = 512;   // most candidates of a top-k select that are ranked key by key
+constexpr unsigned int BOUND_BINS = 256, BOUND_SHIFT = 19;   // of the bound below them: sixteen bins an octave
 
 // floor(e * 2^32) for 0 <= e <= 1
 __device__ __forceinline__ unsigned long long fix32(float e) {
@@ -263,41 +267,65 @@ __device__ __forceinline__ BinPick pick_bin(const unsigned long long* h, unsigne
   return r;
 }
 
+// inclusive prefix sum of 32-bit counts over the lanes, as wave_scan
+template <int CTRL, int ROWS>
+__device__ __forceinline__ unsigned int count_step(unsigned int v) { return v + (unsigned int)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false); }
+__device__ __forceinline__ unsigned int wave_count(unsigned int v) {
+  return count_step<0x143, 0xc>(count_step<0x142, 0xa>(count_step<0x118, 0xf>(count_step<0x114, 0xf>(count_step<0x112, 0xf>(count_step<0x111, 0xf>(v))))));
+}
+
 template <int DT>
 __global__ __launch_bounds__(1024) void sample_filtered_kernel(SampleParams P) {
   __shared__ float csum[64 + 4], csum_all[64];
   __shared__ unsigned long long h1[4096], h2[1024], h3[1024], wtot[16];
   __shared__ BinPick sh;
-  __shared__ unsigned int cand[CAND], n_cand;
-  const int row = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, tid = threadIdx.x;
+  __shared__ __attribute__((aligned(16))) unsigned int bound[BOUND_BINS];
+  __shared__ unsigned int cand[CAND], sorted[CAND], n_cand, wmax[16], sh_thr;
+  __shared__ float sh_u, sh_lp;
+  __shared__ int sh_tok;
+  const int row = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), tid = threadIdx.x;
   const char* xr = (const char*)P.x + (int64_t)row * P.stride * (DT == UVMI_F32 ? 4 : 2);
   const int nchunks = P.V / CHUNK;   // <= 64: wave w holds chunks w, w + 16, w + 32, w + 48
 
+  // the thread's logits, 16-bit ones kept beside their exponentials for the draw
   float e[4][8];
-#pragma unroll
-  for (int q = 0; q < 4; q++) {
-    const int c = wave + 16 * q;
-    if (c < nchunks) load8<DT>(xr, c * 64 + lane, e[q]);
-  }
-  // (requested with the row: the draw at the end of the chain needs it at once)
-  const float u = wave == 0 ? uniform_of(P, row) : 0.f;
-  for (int i = tid; i < 4096; i += 1024) h1[i] = 0;
-  h2[tid] = 0;
-  h3[tid] = 0;
-  // ---- unfiltered chunk sums (for the log-prob), in the order of the unfiltered kernel
+  uint4 raw[DT == UVMI_F32 ? 1 : 4];
 #pragma unroll
   for (int q = 0; q < 4; q++) {
     const int c = wave + 16 * q;
     if (c < nchunks) {
+      if constexpr (DT == UVMI_F32) load8<DT>(xr, c * 64 + lane, e[q]);
+      else raw[q] = ((const uint4*)xr)[c * 64 + lane];
+    }
+  }
+  // (requested with the row: the draw at the end of the chain needs it at once)
+  if (wave == 0) {
+    const float u = uniform_of(P, row);
+    if (lane == 0) sh_u = u;
+  }
+  if (tid < BOUND_BINS) bound[tid] = 0;
+  if (tid == 0) n_cand = 0;
+  // ---- unfiltered chunk sums (for the log-prob), in the order of the unfiltered kernel, and the thread's largest key
+  unsigned int mx = 0;
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const int c = wave + 16 * q;
+    if (c < nchunks) {
+      if constexpr (DT != UVMI_F32) load8<DT>(&raw[q], 0, e[q]);
       float s = 0.f;
 #pragma unroll
       for (int j = 0; j < 8; j++) {
         e[q][j] = e_of(e[q][j], P);
         s += e[q][j];
+        mx = max(mx, __float_as_uint(e[q][j]));
       }
       s = wave_sum(s);
       if (lane == 0) csum_all[c] = s;
     }
+  }
+  {
+    const float wm = wave_max(__uint_as_float(mx));
+    if (lane == 0) wmax[wave] = __float_as_uint(wm);
   }
   const CommitRow cr = commit_ahead(P, row);
   __syncthreads();
@@ -305,35 +333,30 @@ __global__ __launch_bounds__(1024) void sample_filtered_kernel(SampleParams P) {
   unsigned int thr = 0;   // keep keys >= thr
   const bool by_count = P.top_k > 0 && P.top_k < P.V;
   const double share = P.top_p > 0.f ? (double)P.top_p : 0.0;
-  unsigned int mx = 0, top = 0;   // the thread's largest key, the row's
-#pragma unroll
-  for (int q = 0; q < 4; q++)
-    if (wave + 16 * q < nchunks) {
-#pragma unroll
-      for (int j = 0; j < 8; j++) mx = max(mx, __float_as_uint(e[q][j]));
-    }
-  {
-    const float wm = wave_max(__uint_as_float(mx));
-    if (lane == 0) wtot[wave] = __float_as_uint(wm);
-    if (tid == 0) n_cand = 0;
-    __syncthreads();
-#pragma unroll
-    for (int w = 0; w < 16; w++) top = max(top, (unsigned int)wtot[w]);
-    top >>= 16;
-    __syncthreads();
-  }
   // ---- top-k of at most 256: the threads' largest keys bound the k-th largest key from below (k of them are at least as
-  // large), so only keys from that bound's bin up can matter.  They are about a hundred of the 32 768 and are collected in LDS.
-  // There a key's rank and the mass above it are counted key by key, which gives both cuts at once; rows whose candidates
-  // are too many for that (long runs of equal logits) take the histograms.
+  // large), so only keys from that bound's bin up can matter: the bins are sixteenths of an octave below the row's largest key.  They are about a
+  // hundred of the 32 768 and are collected in LDS, and each is put in its place by its rank among them, which the waves count
+  // with ballots; one wave then walks the sorted keys' masses.  Rows whose candidates are too many for that (long runs of equal
+  // logits) take the histograms.
   bool ranked = false;
   if (by_count && P.top_k <= 256) {
-    atomicAdd(&h1[4095u - min(4095u, top - (mx >> 16))], BIN_ONE);
+    unsigned int top = 0;
+#pragma unroll
+    for (int w = 0; w < 16; w++) top = max(top, wmax[w]);
+    atomicAdd(&bound[min(BOUND_BINS - 1u, (top - mx) >> BOUND_SHIFT)], 1u);
     __syncthreads();
-    unsigned long long k_th = (unsigned long long)P.top_k;
-    const unsigned int digit = pick_bin<4, false>(h1, k_th, wtot, &sh).digit;
-    const unsigned int low = digit ? (top - (4095u - digit)) << 16 : 0u;
-    for (int i = tid; i < 4096; i += 1024) h1[i] = 0;
+    unsigned int low;
+    {   // (every wave for itself)
+      const uint4 c4 = ((const uint4*)bound)[lane];
+      const unsigned int incl = wave_count(c4.x + c4.y + c4.z + c4.w), k = (unsigned int)P.top_k;
+      const unsigned long long reach = __ballot(incl >= k);
+      const int at = __ffsll((long long)reach) - 1;   // (1024 keys in the bins, k <= 256)
+      unsigned int run = incl - (c4.x + c4.y + c4.z + c4.w), b = 4 * lane;
+      if (run + c4.x < k) { run += c4.x; b++; if (run + c4.y < k) { run += c4.y; b++; if (run + c4.z < k) b++; } }
+      b = (unsigned int)__builtin_amdgcn_readlane((int)b, at);
+      const unsigned int span = (b + 1) << BOUND_SHIFT;   // keys above top - span
+      low = b == BOUND_BINS - 1 || span > top ? 0u : top - span + 1;
+    }
 #pragma unroll
     for (int q = 0; q < 4; q++)
       if (wave + 16 * q < nchunks) {
@@ -350,40 +373,56 @@ __global__ __launch_bounds__(1024) void sample_filtered_kernel(SampleParams P) {
     ranked = n_cand <= CAND;
   }
   if (ranked) {
-    // every wave compares the candidates with a sixteenth of the list: h1 gathers their counts (larger keys in the low word,
-    // equal ones in the high word), h2 the mass of the larger keys
-    const unsigned int n = n_cand;
-    for (unsigned int i = lane; i < n; i += 64) {
-      const unsigned int mine = cand[i];
-      unsigned long long cnt = 0, mgt = 0;
-      for (unsigned int j = wave; j < n; j += 16) {
-        const unsigned int key = cand[j];
-        const unsigned long long m = fix32(__uint_as_float(key));
-        cnt += key > mine ? 1ull : (key == mine ? 1ull << 32 : 0ull);
-        mgt += key > mine ? m : 0ull;
+    const int n = (int)n_cand, R = (n + 63) >> 6;
+    unsigned int key[CAND / 64];
+#pragma unroll
+    for (int r = 0; r < (int)CAND / 64; r++) key[r] = 64 * r + lane < n ? cand[64 * r + lane] : 0u;
+    for (int c = wave; c < n; c += 16) {
+      const unsigned int mine = cand[c];
+      int rank = 0;
+#pragma unroll
+      for (int r = 0; r < (int)CAND / 64; r++) {
+        if (r >= R) break;
+        rank += __popcll(__ballot(key[r] > mine || (key[r] == mine && 64 * r + lane < c)));
       }
-      if (cnt) atomicAdd(&h1[i], cnt);
-      if (mgt) atomicAdd(&h2[i], mgt);
+      if (lane == 0) sorted[rank] = mine;
     }
     __syncthreads();
-    // (equal keys write the same words)
-    unsigned int mine = 0, gt = 0, eq = 0;
-    if (tid < (int)n) {
-      mine = cand[tid];
-      gt = (unsigned int)h1[tid];
-      eq = (unsigned int)(h1[tid] >> 32);
-      if (gt < (unsigned int)P.top_k && gt + eq >= (unsigned int)P.top_k) sh = BinPick{mine, gt, h2[tid], eq * fix32(__uint_as_float(mine))};
+    if (wave == 0) {   // lane l has the sorted keys R l .. R l + R - 1
+      unsigned int t = sorted[P.top_k - 1];
+      if (P.top_p < 1.0f) {
+        unsigned long long m[CAND / 64], mine = 0, kept = 0;
+#pragma unroll
+        for (int r = 0; r < (int)CAND / 64; r++) {
+          m[r] = 0;
+          if (r >= R) break;
+          key[r] = R * lane + r < n ? sorted[R * lane + r] : 0u;
+          m[r] = key[r] ? fix32(__uint_as_float(key[r])) : 0ull;
+          mine += m[r];
+          kept += key[r] >= t ? m[r] : 0ull;
+        }
+        const unsigned long long all = wave_scan(kept);
+        const unsigned long long mass = ((unsigned long long)(unsigned int)__builtin_amdgcn_readlane((int)(all >> 32), 63) << 32) |
+                                        (unsigned int)__builtin_amdgcn_readlane((int)(unsigned int)all, 63);
+        const unsigned long long want = (unsigned long long)(share * (double)mass);
+        // the first key whose mass of keys up to it reaches want (a run of equal keys is kept whole: the threshold is their value)
+        const unsigned long long incl = wave_scan(mine);
+        unsigned long long run = incl - mine;
+        unsigned int pick = 0;
+        bool found = false;
+#pragma unroll
+        for (int r = 0; r < (int)CAND / 64; r++) {
+          if (r >= R) break;
+          run += m[r];
+          if (!found && key[r] && run >= want) { pick = key[r]; found = true; }
+        }
+        const unsigned long long reach = __ballot(found);
+        if (reach) t = (unsigned int)__builtin_amdgcn_readlane((int)pick, __ffsll((long long)reach) - 1);
+      }
+      if (lane == 0) sh_thr = t;
     }
     __syncthreads();
-    const BinPick b = sh;
-    thr = b.digit;
-    __syncthreads();
-    if (P.top_p < 1.0f) {
-      const unsigned long long want = (unsigned long long)(share * (double)(b.mass_above + b.mass));
-      if (tid < (int)n && (want == 0 ? gt == 0 : h2[tid] < want && h2[tid] + eq * fix32(__uint_as_float(mine)) >= want)) sh.digit = mine;
-      __syncthreads();
-      thr = sh.digit;
-    }
+    thr = sh_thr;
   }
   // ---- the general form: radix selects over histograms of the whole row, by digits of 12 + 10 + 10 bits.  (Digits counted from
   // the row's largest key in 128 bins per octave were measured too: no faster - a wave's 64-bit LDS atomics take ~40 clocks
@@ -452,10 +491,6 @@ __global__ __launch_bounds__(1024) void sample_filtered_kernel(SampleParams P) {
       thr = (d1 << 20) | (d2 << 10) | b.digit;
     }
   }
-  auto e_kept = [&](float x) -> float {
-    const float e = e_of(x, P);
-    return __float_as_uint(e) >= thr ? e : 0.f;
-  };
 
   // ---- draw from the kept tokens: chunk sums, then the chunk, the lane, the element (as the unfiltered kernel)
 #pragma unroll
@@ -470,7 +505,6 @@ __global__ __launch_bounds__(1024) void sample_filtered_kernel(SampleParams P) {
     }
   }
   __syncthreads();
-  if (wave != 0) return;
   float incl = lane < nchunks ? csum[lane] : 0.f;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
@@ -478,58 +512,73 @@ __global__ __launch_bounds__(1024) void sample_filtered_kernel(SampleParams P) {
     if (lane >= o) incl += t;
   }
   const float Sk = __shfl(incl, 63, 64);
-  const float S = wave_sum(lane < nchunks ? csum_all[lane] : 0.f);
-  const float target = (1.0f - u) * Sk;
+  const float target = (1.0f - sh_u) * Sk;
   const unsigned long long below = __ballot(lane < nchunks && incl < target);
   int ck = __popcll(below);
   if (ck > nchunks - 1) ck = nchunks - 1;
   // (a chunk without kept tokens has the inclusive sum of its predecessor, which is < target whenever it is chosen over,
   // so the chosen chunk always holds a kept token unless rounding pushed target past the total: then walk back)
   while (ck > 0 && (ck > 0 ? __shfl(incl, ck - 1, 64) : 0.f) >= Sk) ck--;
-  const float before = ck > 0 ? __shfl(incl, ck - 1, 64) : 0.f;
-  float v[8], ek[8];
-  load8<DT>(xr, ck * 64 + lane, v);
-  float ls = 0.f;
+  ck = __builtin_amdgcn_readfirstlane(ck);
+  if (wave == (ck & 15)) {   // the wave that holds the chunk
+    const float before = ck > 0 ? __shfl(incl, ck - 1, 64) : 0.f;
+    float ek[8];
+    uint4 w = uint4{0u, 0u, 0u, 0u};
 #pragma unroll
-  for (int j = 0; j < 8; j++) {
-    ek[j] = e_kept(v[j]);
-    ls += ek[j];
-  }
-  float linc = ls;
+    for (int q = 0; q < 4; q++)
+      if (q == ck >> 4) {
 #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const float t = __shfl_up(linc, o, 64);
-    if (lane >= o) linc += t;
-  }
-  linc += before;
-  // the lane: the first one whose inclusive sum reaches target and that holds a kept token; when rounding pushed target
-  // past the chunk's total, the last lane that holds one
-  const unsigned long long has = __ballot(ls > 0.f);
-  int ln = __popcll(__ballot(linc < target));
-  {
-    const unsigned long long hi = ln < 64 ? has & ~((1ull << ln) - 1ull) : 0ull;
-    ln = hi ? __ffsll((long long)hi) - 1 : (has ? 63 - __clzll((long long)has) : 0);
-  }
-  // every lane recomputes that lane's walk from broadcast values: the first kept element whose running sum reaches
-  // target, else the lane's last kept element
-  float run = ln > 0 ? __shfl(linc, ln - 1, 64) : before;
-  int sel = ln * 8;
-  float xsel = __shfl(v[0], ln, 64);
-  bool found = false;
+        for (int j = 0; j < 8; j++) ek[j] = __float_as_uint(e[q][j]) >= thr ? e[q][j] : 0.f;
+        if constexpr (DT != UVMI_F32) w = raw[q];
+      }
+    float ls = 0.f;
 #pragma unroll
-  for (int j = 0; j < 8; j++) {
-    const float ej = __shfl(ek[j], ln, 64), xj = __shfl(v[j], ln, 64);
-    if (ej > 0.f && !found) {
-      run += ej;
-      sel = ln * 8 + j; xsel = xj;
-      if (run >= target) found = true;
+    for (int j = 0; j < 8; j++) ls += ek[j];
+    float linc = ls;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const float t = __shfl_up(linc, o, 64);
+      if (lane >= o) linc += t;
+    }
+    linc += before;
+    // the lane: the first one whose inclusive sum reaches target and that holds a kept token; when rounding pushed target
+    // past the chunk's total, the last lane that holds one
+    const unsigned long long has = __ballot(ls > 0.f);
+    int ln = __popcll(__ballot(linc < target));
+    {
+      const unsigned long long hi = ln < 64 ? has & ~((1ull << ln) - 1ull) : 0ull;
+      ln = hi ? __ffsll((long long)hi) - 1 : (has ? 63 - __clzll((long long)has) : 0);
+    }
+    // every lane walks its own elements from the sum ahead of it, for that one is among them: the first kept element whose running sum
+    // reaches target, else the lane's last kept element
+    const float prev = __shfl_up(linc, 1, 64);
+    float run = lane > 0 ? prev : before, xsel;
+    int sel = 0;
+    bool found = false;
+    float v[8];
+    if constexpr (DT == UVMI_F32) load8<DT>(xr, ck * 64 + lane, v);
+    else load8<DT>(&w, 0, v);
+    xsel = v[0];
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      if (ek[j] > 0.f && !found) {
+        run += ek[j];
+        sel = j; xsel = v[j];
+        if (run >= target) found = true;
+      }
+    }
+    if (lane == ln) {
+      const float E = __builtin_amdgcn_exp2f(fmaf(xsel, P.inv_c_l2, P.b_over_c_l2));
+      sh_tok = ck * CHUNK + ln * 8 + sel;
+      sh_lp = __builtin_amdgcn_rcpf(1.0f + E);
     }
   }
-  if (lane == 0) {
-    const float E = __builtin_amdgcn_exp2f(fmaf(xsel, P.inv_c_l2, P.b_over_c_l2));
-    if (P.u_out) P.u_out[row] = u;
+  const float S = wave == 0 ? wave_sum(lane < nchunks ? csum_all[lane] : 0.f) : 0.f;
+  __syncthreads();
+  if (tid == 0) {
+    if (P.u_out) P.u_out[row] = sh_u;
     if (P.thr_out) P.thr_out[row] = __uint_as_float(thr);
-    emit(P, row, ck * CHUNK + sel, P.neg_a_over_t * __builtin_amdgcn_rcpf(1.0f + E) - __logf(S), cr);
+    emit(P, row, sh_tok, P.neg_a_over_t * sh_lp - __logf(S), cr);
   }
 }
 
