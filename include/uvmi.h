@@ -262,6 +262,10 @@ int uvmi_gemm_tn_ex(const uvmi_gemm_args* a, void* stream);
 #define UVMI_GEMM_PATH_STREAM 1
 #define UVMI_GEMM_PATH_BIG 2    /* slabs straight into LDS */
 int uvmi_gemm_tn_path(const uvmi_gemm_args* a, int* tile_rows, int* tile_cols);
+/* uvmi_gemm_tn_ex for the residual update of a pass of any number of rows: where many rows fill the device better so, on 192 x 128 tiles, to the same
+ * bits.  uvmi_gemm_resid_tile: 192 where it takes those, else 0 (negative: its refusal). */
+int uvmi_gemm_resid(const uvmi_gemm_args* a, void* stream);
+int uvmi_gemm_resid_tile(const uvmi_gemm_args* a);
 
 /* ------------------------------------------------------------------------------------------------------------
  * Packed (cu_seqlens) causal self-attention with an optional sliding window over unquantized K/V: the attention of
@@ -456,6 +460,7 @@ int uvmi_prefill_attn_o(const struct uvmi_prefill_attn_o_args* a, void* stream);
 #define UVMI_OP_NORM 4          /* struct uvmi_norm_args */
 #define UVMI_OP_QKV_PROJ 5      /* struct uvmi_qkv_proj_args */
 #define UVMI_OP_PREFILL_ATTN_O 6 /* struct uvmi_prefill_attn_o_args */
+#define UVMI_OP_GEMM_RESID 7    /* uvmi_gemm_args, for uvmi_gemm_resid */
 int uvmi_run_ops(const int* kinds, const void* const* args, int n_ops, void* stream);
 
 /* ------------------------------------------------------------------------------------------------------------

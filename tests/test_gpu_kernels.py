@@ -1238,6 +1238,24 @@ def test_tile_of_passes_of_many_rows(M, K, N, epi, tile):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,K,N", [(13441, 128, 640), (18432, 192, 640), (13999, 512, 640), (18431, 1664, 640), (28001, 512, 640), (33216, 192, 640), (14000, 640, 608)])
+def test_residual_update_on_192_row_tiles(dtype, M, K, N):
+    """uvmi_gemm_resid where it takes 192 x 128 tiles - one round of the device and several, an even and an odd number of slabs, ragged edges, in
+    place - gives the bits of the 128 x 128 tiles, which sum K alike."""
+    import ctypes as C
+    from ultraviolet_amd import _lib as L
+    from ultraviolet_amd.kernels.gemm import RESID, gemm_args, gemm_tn
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    a, w = (torch.randn(s, K, device="cuda", generator=g).to(dtype) for s in (M, N))
+    x = torch.randn(M, N, device="cuda", generator=g).to(dtype)
+    want = gemm_tn(a, w, epilogue=RESID, resid=x, ca=0.75, cb=0.125, config=6)
+    ga = gemm_args(a, w, x, RESID, resid=x, ca=0.75, cb=0.125)
+    assert L.lib().uvmi_gemm_resid_tile(C.byref(ga)) == 192
+    L.check(L.lib().uvmi_gemm_resid(C.byref(ga), L.stream_ptr(a)), "uvmi_gemm_resid")
+    assert torch.equal(x, want)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("K", [128, 192, 640])
 @pytest.mark.parametrize("config", [5, 6])
 def test_big_tiles_in_several_rounds(dtype, K, config):

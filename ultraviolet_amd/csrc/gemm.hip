@@ -7,7 +7,7 @@ using namespace uvmi;
 
 namespace uvmi {
 void gemm_tile_launch(const uvmi_gemm_args* a, hipStream_t st);                     // gemm_tile.hip
-void gemm_big_launch(const uvmi_gemm_args* a, int tile, int cus, hipStream_t st);   // gemm_big.hip
+void gemm_big_launch(const uvmi_gemm_args* a, int tile, int cus, hipStream_t st);   // gemm_big.hip; tile: 128, 256, 192 (x 128: RESID)
 int gemm_stream_form(const uvmi_gemm_args* a, int cus);                             // gemm_stream.hip
 void gemm_stream_tile(int form, int* rows, int* cols);
 void gemm_stream_launch(const uvmi_gemm_args* a, int form, int cus, hipStream_t st);
@@ -144,4 +144,38 @@ extern "C" int uvmi_gemm_tn(const void* a, const void* w, void* c, int dtype, in
   g.a = a; g.w = w; g.c = c; g.dtype = dtype; g.M = M; g.N = N; g.K = K; g.lda = lda; g.ldw = ldw; g.ldc = ldc; g.epilogue = epilogue;
   UVMI_REQUIRE(epilogue != UVMI_GEMM_RESID, UVMI_EINVAL, "uvmi_gemm_tn: the RESID epilogue takes its residual through uvmi_gemm_tn_ex");
   return uvmi_gemm_tn_ex(&g, stream);
+}
+
+// The residual update of a pass of many rows also has 192 x 128 tiles, two to a compute unit, to choose from: between the rounds of the
+// device of the other two, and with two epilogues to overlap.  A launch lasts as long as its rounds, of which a last one that gives a unit one
+// workgroup takes about six tenths (128 x 128) and four (192 x 128) of a full one; a full one of 192 x 128 tiles 1.48 and one of 256 x 256
+// tiles 1.7 of one of 128 x 128 ones.  us, 128 / 192 / 256, 640 columns, K 1664 and 512: 12 288 rows 30.1 / 38.1 / 45.0 and 15.2 /
+// 18.5 / 22.1; 14 000 46.3 / 38.3 / 45.3 and 21.2 / 19.7 / 22.5; 18 432 47.3 / 41.6 / 48.6 and 22.6 / 21.5 / 23.8; 20 000 52.1 / 56.9 / 47.7 and
+// 26.2 / 28.1 / 24.3; 24 576 54.9 / 57.0 / 86.5 and 27.3 / 28.0 / 41.3; 28 000 71.6 / 61.6 / 88.9 and 32.7 / 29.6 / 41.8; 33 216 77.2 / 79.0 /
+// 90.6 and 37.6 / 36.5 / 43.8; 50 000 106.8 / 116.2 / 131.9 and 49.4 / 52.4 / 60.4.
+static bool resid_192(const uvmi_gemm_args* a, int cus) {
+  if (a->epilogue != UVMI_GEMM_RESID || a->norm_a || a->config != 0 || a->M < BIG_MIN_ROWS || !big_ok(a)) return false;
+  const int64_t slots = 2 * (int64_t)cus, n128 = ((int64_t)a->N + 127) / 128;
+  auto rounds = [&](int64_t tiles, int full, int part) {
+    const int64_t rest = tiles % slots;
+    return tiles / slots * full + (rest == 0 ? 0 : (rest <= cus ? part : full));
+  };
+  const int64_t t256 = ((a->M + 255) / 256) * (((int64_t)a->N + 255) / 256);
+  const int64_t c192 = rounds(((a->M + 191) / 192) * n128, 148, 59);
+  return c192 < rounds(((a->M + 127) / 128) * n128, 100, 64) && c192 < (t256 + cus - 1) / cus * 170;
+}
+
+extern "C" int uvmi_gemm_resid_tile(const uvmi_gemm_args* a) {
+  const int rc = check_gemm(a);
+  return rc ? rc : (resid_192(a, compute_units()) ? 192 : 0);
+}
+
+extern "C" int uvmi_gemm_resid(const uvmi_gemm_args* a, void* stream) {
+  const int rc = check_gemm(a);
+  if (rc) return rc;
+  const int cus = compute_units();
+  if (a->M == 0 || !resid_192(a, cus)) return uvmi_gemm_tn_ex(a, stream);
+  gemm_big_launch(a, 192, cus, (hipStream_t)stream);
+  UVMI_CHECK_LAUNCH("uvmi_gemm_resid");
+  return UVMI_OK;
 }

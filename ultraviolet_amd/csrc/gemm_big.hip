@@ -87,15 +87,17 @@ __device__ __forceinline__ int fresh_lane() {
 // EPI 0: C = A W^T (M, N).  EPI 1: W rows are [gate 16 | up 16] slabs; C = silu(gate) * up, (M, N / 2).
 // EPI 2: C = ca * R + cb * (A W^T).  EPI 3: C fp32 = ca * sigmoid((x + cb) / cap_c) of the rounded product x.  NORM: A stands
 // for its RMS-normalised rows.
-// FI: 16-row fragments per wave along M: 8 - the 256 x 256 tile on 8 waves (2 x 4); 4 - a 128 x 128 tile on 4 waves (2 x 2,
-// 64 x 64 per wave, two workgroups per compute unit) for passes whose 256 x 256 tiles would not fill the device.  (A
+// FI: 16-row fragments per wave along M: 8 - the 256 x 256 tile on 8 waves (2 x 4); 6 - 192 x 128 on 4 waves (2 x 2, 96 x 64 per wave, two
+// workgroups per compute unit; no pre-norm); 4 - a 128 x 128 tile on 4 waves (64 x 64 per wave, two workgroups per compute unit) for passes whose 256 x 256 tiles would not fill the device.  (A
 // 64 x 64 tile on 2 waves was measured too: no faster at 2 k rows than 64 x 64 tiles staged through registers.)
 // MANY: a workgroup takes several tiles (an even number of slabs: a tile ends on the stage that it does not begin on).
+template <int FI> constexpr int BIG_THREADS = FI == 8 ? 512 : 256;
 template <int DT, int EPI, bool NORM, int FI, bool MANY>
-__global__ __launch_bounds__(64 * FI) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ __launch_bounds__(BIG_THREADS<FI>) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_big_kernel(BigParams P) {
-  constexpr int WN = FI / 2;                   // waves along N (2 along M)
-  constexpr int BM = 32 * FI, BN = 64 * WN;
+  constexpr int WN = BIG_THREADS<FI> / 128;    // waves along N (2 along M)
+  constexpr int BM = 32 * FI, BN = 64 * WN, LA = BM / (16 * WN);   // LA: a wave's loads of A per slab (of W: 4)
+  static_assert(!NORM || FI / 2 == WN, "a wave along N for every pair of a wave's row fragments");
   // one array per stage and operand: the compiler can then tell that the operand reads of one stage do not touch the
   // stage a load in flight is writing, and does not wait for that load
   __shared__ __attribute__((aligned(1024))) unsigned char sA0[BM * 128];
@@ -121,17 +123,20 @@ void gemm_big_kernel(BigParams P) {
   };
   tile_at(L);
 
-  // ---- loader: wave w fills blocks 4 w .. 4 w + 3 (8 rows each) of A and of W (BM = BN = 32 x the number of waves).  Rows
-  // past M / N repeat the last row: what they produce is never stored.
-  uint32_t offA[4], offB[4];
+  // ---- loader: wave w fills blocks LA w .. of A and 4 w .. 4 w + 3 of W (8 rows each).  Rows past M / N repeat the last row: what they
+  // produce is never stored.
+  uint32_t offA[LA], offB[4];
   auto offsets = [&]() {
     const int ln = fresh_lane();
 #pragma unroll
+    for (int i = 0; i < LA; i++) {
+      const int rl = 8 * (LA * wave + i) + (ln >> 3);   // row inside the tile
+      offA[i] = (uint32_t)min(m0 + rl, P.M - 1) * P.lda2 + 16 * ((ln & 7) ^ ((rl >> 1) & 7));
+    }
+#pragma unroll
     for (int i = 0; i < 4; i++) {
-      const int rl = 8 * (4 * wave + i) + (ln >> 3);   // row inside the tile
-      const int ch = (ln & 7) ^ ((rl >> 1) & 7);
-      offA[i] = (uint32_t)min(m0 + rl, P.M - 1) * P.lda2 + 16 * ch;
-      offB[i] = (uint32_t)min(n0 + rl, P.N - 1) * P.ldw2 + 16 * ch;
+      const int rl = 8 * (4 * wave + i) + (ln >> 3);
+      offB[i] = (uint32_t)min(n0 + rl, P.N - 1) * P.ldw2 + 16 * ((ln & 7) ^ ((rl >> 1) & 7));
     }
   };
   offsets();
@@ -140,11 +145,11 @@ void gemm_big_kernel(BigParams P) {
   const __amdgpu_buffer_rsrc_t rW = __builtin_amdgcn_make_buffer_rsrc((void*)P.w, 0, (int)((uint32_t)(P.N - 1) * P.ldw2 + (uint32_t)P.K * 2), 0x00020000);
   auto issue = [&](unsigned char* sa, unsigned char* sb, int kt) {
 #pragma unroll
-    for (int i = 0; i < 4; i++)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, UVMI_LDSP(sa + (4 * wave + i) * 1024), 16, offA[i], kt * 128, 0, 0);
+    for (int i = 0; i < LA; i++)
+      load_lds16(rA, sa + (LA * wave + i) * 1024, offA[i], kt * 128);
 #pragma unroll
     for (int i = 0; i < 4; i++)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, UVMI_LDSP(sb + (4 * wave + i) * 1024), 16, offB[i], kt * 128, 0, 0);
+      load_lds16(rW, sb + (4 * wave + i) * 1024, offB[i], kt * 128);
   };
 
   // ---- reader: wave (wm, wn) owns rows 16 FI wm .., columns 64 wn ..; lane (r, g) reads chunk (4 s + g) ^ ((r / 2) % 8) of
@@ -257,8 +262,28 @@ void gemm_big_kernel(BigParams P) {
     read_b(SBN, 0, w0); read_a(SAN, 0, 0, Y); UVMI_SB();                                                                 \
     mm1(2, X, w1); mm7(2, X, w1); sumsq(1, X); UVMI_SB();                                                                \
   } while (0)
+    // FI = 6: 6 groups per slab, whose operands take the three buffers in turn
+#define UVMI_ITER6(SA, SB_, SAN, SBN, k)                                                                                 \
+  do {                                                                                                                   \
+    mm1(0, f0, w0); UVMI_SB(); read_a(SA, 0, 2, f1); UVMI_SB(); mm7(0, f0, w0); UVMI_SB();                               \
+    mm1(2, f1, w0); UVMI_SB(); read_a(SA, 0, 4, f2); UVMI_SB(); mm7(2, f1, w0); UVMI_SB();                               \
+    mm1(4, f2, w0); UVMI_SB(); read_b(SB_, 1, w1); read_a(SA, 1, 0, f0); UVMI_SB(); mm7(4, f2, w0); UVMI_SB();           \
+    mm1(0, f0, w1); UVMI_SB(); read_a(SA, 1, 2, f1); UVMI_SB(); mm7(0, f0, w1); UVMI_SB();                               \
+    mm1(2, f1, w1); UVMI_SB(); read_a(SA, 1, 4, f2); UVMI_SB(); mm7(2, f1, w1); UVMI_SB();                               \
+    __builtin_amdgcn_s_waitcnt(0x0f70);                                                                                  \
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");                                                      \
+    request(SA, SB_, (k) + 2);                                                                                           \
+    read_b(SBN, 0, w0); read_a(SAN, 0, 0, f0); UVMI_SB();                                                                \
+    mm1(4, f2, w1); mm7(4, f2, w1); UVMI_SB();                                                                           \
+  } while (0)
     int k = 0;
-    if constexpr (FI == 8) {
+    if constexpr (FI == 6) {
+      for (; k + 2 <= nk; k += 2) {
+        UVMI_ITER6(sA0, sB0, sA1, sB1, k);
+        UVMI_ITER6(sA1, sB1, sA0, sB0, k + 1);
+      }
+      if (!MANY && k < nk) UVMI_ITER6(sA0, sB0, sA1, sB1, k);
+    } else if constexpr (FI == 8) {
       for (; k + 2 <= nk; k += 2) {
         UVMI_ITER(sA0, sB0, sA1, sB1, k);
         UVMI_ITER(sA1, sB1, sA0, sB0, k + 1);
@@ -272,6 +297,7 @@ void gemm_big_kernel(BigParams P) {
       if (!MANY && k < nk) UVMI_ITER4(sA0, sB0, sA1, sB1, k, f0, f1);
     }
 #undef UVMI_ITER4
+#undef UVMI_ITER6
 #undef UVMI_ITER
 #undef UVMI_SB
 
@@ -398,33 +424,38 @@ static void launch_big(const uvmi_gemm_args* a, const BigParams& P, int cus, hip
   const int slots = (FI == 8 ? cus : 2 * cus) / 8 * 8;   // workgroups that run at a time
   // (a launch of one round keeps the shorter code: it lost 0.5 us of 9 to the other's)
   const bool many = P.K % 128 == 0 && slots > 0 && T > slots;
-  const dim3 grid((unsigned)(many ? slots : ((T + 7) / 8) * 8)), blk(64 * FI);
+  const dim3 grid((unsigned)(many ? slots : ((T + 7) / 8) * 8)), blk(BIG_THREADS<FI>);
 #define UVMI_GO(EPI, NORM)                                                                              \
   do {                                                                                                  \
     if (many) hipLaunchKernelGGL((gemm_big_kernel<DT, EPI, NORM, FI, true>), grid, blk, 0, st, P);      \
     else hipLaunchKernelGGL((gemm_big_kernel<DT, EPI, NORM, FI, false>), grid, blk, 0, st, P);          \
   } while (0)
   const bool norm = a->norm_a != 0;
-  if (a->epilogue == UVMI_GEMM_RESID) { if (norm) UVMI_GO(2, true); else UVMI_GO(2, false); }
+  if constexpr (FI == 6) {
+    UVMI_GO(2, false);
+  } else if (a->epilogue == UVMI_GEMM_RESID) { if (norm) UVMI_GO(2, true); else UVMI_GO(2, false); }
   else if (a->epilogue == UVMI_GEMM_SWIGLU) { if (norm) UVMI_GO(1, true); else UVMI_GO(1, false); }
   else if (a->epilogue == UVMI_GEMM_SOFTCAP) { if (norm) UVMI_GO(3, true); else UVMI_GO(3, false); }
   else { if (norm) UVMI_GO(0, true); else UVMI_GO(0, false); }
 #undef UVMI_GO
 }
 
-// Arguments are validated by the caller (uvmi_gemm_tn_ex), which also checks K >= 128.  tile: 256 or 128.
+// Arguments are validated by the caller (uvmi_gemm_tn_ex), which also checks K >= 128.  tile: 256, 128 or (RESID without
+// the pre-norm: uvmi_gemm_resid) 192 rows.
 void gemm_big_launch(const uvmi_gemm_args* a, int tile, int cus, hipStream_t st) {
   BigParams P;
   P.a = a->a; P.w = a->w; P.c = a->c; P.r = a->resid;
   P.lda2 = (uint32_t)a->lda * 2; P.ldw2 = (uint32_t)a->ldw * 2; P.ldc = a->ldc; P.ldr = a->ldr;
   P.M = (int)a->M; P.N = a->N; P.K = a->K;
+  const int cols = tile == 192 ? 128 : tile;
   P.tiles_m = (int)((a->M + tile - 1) / tile);
-  P.tiles_n = (a->N + tile - 1) / tile;
+  P.tiles_n = (a->N + cols - 1) / cols;
   P.eps = a->eps; P.ca = a->ca; P.cb = a->cb; P.cap_c = a->cap_c;
   const double bytes_a = (double)a->M * a->K, bytes_w = (double)a->N * a->K;
   P.rowsplit = bytes_a / 8 + bytes_w < bytes_a + bytes_w / 8;
-  if (a->dtype == UVMI_F16) { if (tile == 256) launch_big<UVMI_F16, 8>(a, P, cus, st); else launch_big<UVMI_F16, 4>(a, P, cus, st); }
-  else { if (tile == 256) launch_big<UVMI_BF16, 8>(a, P, cus, st); else launch_big<UVMI_BF16, 4>(a, P, cus, st); }
+#define UVMI_T(DT) do { if (tile == 256) launch_big<DT, 8>(a, P, cus, st); else if (tile == 192) launch_big<DT, 6>(a, P, cus, st); else launch_big<DT, 4>(a, P, cus, st); } while (0)
+  if (a->dtype == UVMI_F16) UVMI_T(UVMI_F16); else UVMI_T(UVMI_BF16);
+#undef UVMI_T
 }
 
 }  // namespace uvmi

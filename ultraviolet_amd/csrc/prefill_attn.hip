@@ -506,7 +506,7 @@ extern "C" int uvmi_prefill_attn_path(const uvmi_prefill_attn_args* a) {
 static int prefill_attn_run(const uvmi_prefill_attn_args* a, const uvmi_gemm_args* o, void* stream) {
   int rc = check_prefill(a);
   if (rc) return rc;
-  if (a->N == 0) return o ? uvmi_gemm_tn_ex(o, stream) : UVMI_OK;
+  if (a->N == 0) return o ? uvmi_gemm_resid(o, stream) : UVMI_OK;
   hipStream_t st = (hipStream_t)stream;
   int32_t* seg_start = (int32_t*)a->workspace;
   int32_t* pidx = (int32_t*)((char*)a->workspace + ((size_t)a->N * 4 + 255) / 256 * 256);
@@ -531,11 +531,11 @@ static int prefill_attn_run(const uvmi_prefill_attn_args* a, const uvmi_gemm_arg
     d.B = a->N; d.H = a->H; d.KH = a->KH; d.S = a->N; d.hd = a->hd;
     d.scale = a->scale; d.window = a->window; d.ring = 0; d.num_splits = 1;
     rc = uvmi_decode_attn(&d, stream);
-    return rc || !o ? rc : uvmi_gemm_tn_ex(o, stream);
+    return rc || !o ? rc : uvmi_gemm_resid(o, stream);
   }
   if (const int pieces = o ? oproj_pieces(a, o) : 0) return launch_mfma(a, seg_start, nullptr, 0, st, o, pieces);
   rc = launch_mfma(a, seg_start, a->lse_out, a->lse_stride, st);
-  return rc || !o ? rc : uvmi_gemm_tn_ex(o, stream);
+  return rc || !o ? rc : uvmi_gemm_resid(o, stream);
 }
 
 extern "C" int uvmi_prefill_attn(const uvmi_prefill_attn_args* a, void* stream) { return prefill_attn_run(a, nullptr, stream); }

@@ -228,7 +228,7 @@ class UVEngine:
 
     def _gemm(self, a: Tensor, w: Tensor, out: Tensor, epilogue: int = STORE, **kw):
         g = gemm_args(a, w, out, epilogue, **kw)
-        self._op(L.OP_GEMM, g, (a, w, out), M="n")
+        self._op(L.OP_GEMM_RESID if epilogue == RESID else L.OP_GEMM, g, (a, w, out), M="n")
 
     def _embed_norm(self, tok: Tensor, n: int):
         b = self.buf
