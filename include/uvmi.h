@@ -266,6 +266,11 @@ int uvmi_gemm_tn_path(const uvmi_gemm_args* a, int* tile_rows, int* tile_cols);
  * bits.  uvmi_gemm_resid_tile: 192 where it takes those, else 0 (negative: its refusal). */
 int uvmi_gemm_resid(const uvmi_gemm_args* a, void* stream);
 int uvmi_gemm_resid_tile(const uvmi_gemm_args* a);
+/* uvmi_gemm_resid (RESID without norm_a) that also leaves the sums of squares of C's rows, 64 columns at a time, in sums (ceil(N / 64), ld), and uvmi_gemm_tn_ex
+ * (STORE or SWIGLU with norm_a) that takes those of A's rows from there, (K / 64, ld).  256 (to take sums) to 1024 columns; 12 288 rows or more, or config 5 or 6;
+ * sums 16-byte aligned, ld a multiple of 4 and at least M. */
+struct uvmi_gemm_sums_args { const uvmi_gemm_args* gemm; float* sums; int64_t ld; };
+int uvmi_gemm_sums(const struct uvmi_gemm_sums_args* a, void* stream);
 
 /* ------------------------------------------------------------------------------------------------------------
  * Packed (cu_seqlens) causal self-attention with an optional sliding window over unquantized K/V: the attention of
@@ -461,6 +466,7 @@ int uvmi_prefill_attn_o(const struct uvmi_prefill_attn_o_args* a, void* stream);
 #define UVMI_OP_QKV_PROJ 5      /* struct uvmi_qkv_proj_args */
 #define UVMI_OP_PREFILL_ATTN_O 6 /* struct uvmi_prefill_attn_o_args */
 #define UVMI_OP_GEMM_RESID 7    /* uvmi_gemm_args, for uvmi_gemm_resid */
+#define UVMI_OP_GEMM_SUMS 8     /* struct uvmi_gemm_sums_args */
 int uvmi_run_ops(const int* kinds, const void* const* args, int n_ops, void* stream);
 
 /* ------------------------------------------------------------------------------------------------------------

@@ -1287,6 +1287,63 @@ def test_big_tiles_in_several_rounds(dtype, K, config):
             assert bool(((got[rows].double() - p).abs() <= (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11) * p.abs().clamp_min(1.0)).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,d,config", [(1, 640, 5), (257, 640, 5), (129, 640, 6), (300, 192, 6), (9001, 1024, 5), (2999, 576, 6), (7697, 256, 5), (14000, 640, 0), (18433, 640, 0)])
+def test_rows_squares_summed_where_they_are_written(dtype, M, d, config):
+    """uvmi_gemm_sums.  The residual update leaves the same C and, per row and 64 columns, the sum of C's squares (18 roundings of non-negative
+    terms).  Projections that take a norm from such sums equal, bit for bit, those that form it, on rows whose squares add up exactly."""
+    import ctypes as C
+    from ultraviolet_amd import _lib as L
+    from ultraviolet_amd.kernels.gemm import RESID, STORE, SWIGLU, gemm_args, gemm_tn
+    g = torch.Generator(device="cuda").manual_seed(M + d)
+    rn = lambda *s: torch.randn(*s, device="cuda", generator=g).to(dtype)
+    ld = (M + 3) // 4 * 4 + 8
+
+    def launch(ga, sums):
+        L.check(L.lib().uvmi_gemm_sums(C.byref(L.GemmSumsArgs(C.addressof(ga), sums.data_ptr(), ld)), L.stream_ptr(sums)), "uvmi_gemm_sums")
+
+    a, w, x = rn(M, 192), (rn(d, 192).float() / 14).to(dtype), rn(M, d)
+    want = gemm_tn(a, w, epilogue=RESID, resid=x, ca=0.75, cb=1.25, config=config)
+    sums = torch.full(((d + 63) // 64 + 1, ld), -1.0, device="cuda")
+    launch(gemm_args(a, w, x, RESID, resid=x, ca=0.75, cb=1.25, config=config), sums)
+    assert torch.equal(x, want)
+    exact = want.double().square().view(M, d // 64, 64).sum(2).t()
+    assert bool(((sums[:-1, :M].double() - exact).abs() <= 18 * 2.0 ** -24 * exact).all())
+    assert bool((sums[-1] == -1).all()) and bool((sums[:, M:] == -1).all())
+
+    if d < 256:
+        return
+    x = (torch.randint(-15, 16, (M, d), device="cuda", generator=g).float() / 8).to(dtype)
+    sums = torch.full((d // 64, ld), float("nan"), device="cuda")
+    sums[:, :M] = x.float().square().view(M, d // 64, 64).sum(2).t()
+    for N, epi in ((656, STORE), (3328, SWIGLU)):
+        w = (rn(N, d).float() / d ** 0.5).to(dtype)
+        want = gemm_tn(x, w, epilogue=epi, norm_eps=1e-6, config=config)
+        out = torch.empty_like(want)
+        launch(gemm_args(x, w, out, epi, norm_eps=1e-6, config=config), sums)
+        assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("change", [dict(config=3), dict(M=64), dict(ld=8), dict(ld=131), dict(epilogue=0), dict(norm_a=1), dict(K=2048)])
+def test_sums_of_squares_are_refused_elsewhere(change):
+    """Other forms of the GEMM, few rows, pitches that do not hold the rows, epilogues that neither write nor read sums: refused, nothing launched."""
+    import ctypes as C
+    from ultraviolet_amd import _lib as L
+    from ultraviolet_amd.kernels.gemm import RESID, gemm_args
+    x, w = torch.zeros(130, 128, device="cuda", dtype=torch.bfloat16), torch.zeros(128, 128, device="cuda", dtype=torch.bfloat16)
+    ga = gemm_args(x, w, x, RESID, resid=x, config=0 if "M" in change else 6)
+    sums = torch.full((2, 132), -1.0, device="cuda")
+    if change.get("K"):   # (the rows of a hidden of 2048 columns)
+        ga = gemm_args(torch.zeros(130, 2048, device="cuda", dtype=torch.bfloat16), torch.zeros(128, 2048, device="cuda", dtype=torch.bfloat16), x, norm_eps=1e-6, config=6)
+    else:
+        for k, v in change.items():
+            if k != "ld":
+                setattr(ga, k, v)
+    assert L.lib().uvmi_gemm_sums(C.byref(L.GemmSumsArgs(C.addressof(ga), sums.data_ptr(), change.get("ld", 132))), L.stream_ptr(sums)) < 0
+    torch.cuda.synchronize()
+    assert bool((sums == -1).all())
+
+
 def _fused_case(B, S, ring, kv, dtype, seed, any_ring=False):
     """A fused decode launch on random data: (launch(out, caches, oproj), caches, extras)."""
     from ultraviolet_amd.kernels.decode_attn import decode_attention_fused, rope_table

@@ -71,6 +71,26 @@ def test_c3_full_size_churn_properties_and_graph_equals_eager(device_admit):
     assert runs[0][0] == runs[1][0]
 
 
+def test_prefills_around_the_rows_whose_squares_are_summed_where_they_are_written():
+    """Prefills of 12 287, 12 289 and 14 003 tokens on one state, again in another order: the passes of 12 288 rows and more take the rows' norms
+    from sums that the residual updates leave, to within a few units in the last place of the passes that form them (16-bit
+    hidden, ten layers: as test_c4_full_size_mixed_pass_equals_its_halves), and every repetition to the same bits."""
+    from ultraviolet_amd.engine import KVState
+    cfg, params, eng = _uv50m(14003)
+    rng = np.random.default_rng(3)
+    st = KVState(cfg, 29, 512, DEV)
+    sets = [[rng.integers(1, cfg.vocab_size, size=k).tolist() for k in [500] * (n // 500) + [n % 500]] for n in (12287, 12289, 14003)]
+    run = lambda ps: eng.prefill(ps, list(range(len(ps))), st, left_pad=False).float().clone()
+    got = [run(ps) for ps in sets]
+    assert [eng._sums_ok(n) for n in (12287, 12288, 14003)] == [False, True, True]
+    assert all(torch.equal(run(sets[k]), got[k]) for k in (1, 0, 2, 1))
+    eng._sums_ok = lambda n: False
+    ulp = 2.0 ** -7
+    for k in (1, 2):
+        d = (run(sets[k]) - got[k]).abs()
+        assert float(d.max()) <= 16 * 2 * ulp and float(d.mean()) < 2 * ulp, (float(d.max()), float(d.mean()))
+
+
 def test_c4_full_size_mixed_pass_equals_its_halves():
     """BASELINE configs[3] at its size: one pass over 64 prompt chunks x 512 tokens packed with 448 decode rows on contexts
     U{256..2048}.  Its decode rows must agree with a decode-only pass over the same cache and its prompt rows with a

@@ -7,7 +7,7 @@ using namespace uvmi;
 
 namespace uvmi {
 void gemm_tile_launch(const uvmi_gemm_args* a, hipStream_t st);                     // gemm_tile.hip
-void gemm_big_launch(const uvmi_gemm_args* a, int tile, int cus, hipStream_t st);   // gemm_big.hip; tile: 128, 256, 192 (x 128: RESID)
+void gemm_big_launch(const uvmi_gemm_args* a, int tile, int cus, hipStream_t st, float* sums = nullptr, int64_t sums_ld = 0);   // gemm_big.hip; tile: 128, 256, 192 (x 128: RESID)
 int gemm_stream_form(const uvmi_gemm_args* a, int cus);                             // gemm_stream.hip
 void gemm_stream_tile(int form, int* rows, int* cols);
 void gemm_stream_launch(const uvmi_gemm_args* a, int form, int cus, hipStream_t st);
@@ -177,5 +177,24 @@ extern "C" int uvmi_gemm_resid(const uvmi_gemm_args* a, void* stream) {
   if (a->M == 0 || !resid_192(a, cus)) return uvmi_gemm_tn_ex(a, stream);
   gemm_big_launch(a, 192, cus, (hipStream_t)stream);
   UVMI_CHECK_LAUNCH("uvmi_gemm_resid");
+  return UVMI_OK;
+}
+
+// A pass of many rows takes the squares of a block's hidden where the residual updates write it, 64 columns at a time, not again in every
+// column of tiles that reads it.
+extern "C" int uvmi_gemm_sums(const struct uvmi_gemm_sums_args* s, void* stream) {
+  UVMI_REQUIRE(s && s->gemm && s->sums, UVMI_EINVAL, "uvmi_gemm_sums: null pointer");
+  const uvmi_gemm_args* a = s->gemm;
+  const int rc = check_gemm(a);
+  if (rc) return rc;
+  const bool writes = a->epilogue == UVMI_GEMM_RESID && !a->norm_a, reads = a->norm_a && (a->epilogue == UVMI_GEMM_STORE || a->epilogue == UVMI_GEMM_SWIGLU);
+  UVMI_REQUIRE((writes || reads) && (writes ? a->N : a->K) <= 1024 && (writes || a->K >= 256) && big_ok(a) && a->M > 0 &&
+               (a->config == 5 || a->config == 6 || (a->config == 0 && a->M >= BIG_MIN_ROWS)), UVMI_EUNSUPPORTED,
+               "uvmi_gemm_sums: RESID without a pre-norm or STORE / SWIGLU with one, of a hidden of 256 to 1024 columns, on tiles loaded straight into LDS");
+  UVMI_REQUIRE((uintptr_t)s->sums % 16 == 0 && s->ld % 4 == 0 && s->ld >= a->M && s->ld <= (1 << 24), UVMI_EINVAL,
+               "uvmi_gemm_sums: sums 16-byte aligned, with a pitch that is a multiple of 4, >= M");
+  const int cus = compute_units();
+  gemm_big_launch(a, resid_192(a, cus) ? 192 : gemm_path(a, cus).form, cus, (hipStream_t)stream, s->sums, s->ld);
+  UVMI_CHECK_LAUNCH("uvmi_gemm_sums");
   return UVMI_OK;
 }

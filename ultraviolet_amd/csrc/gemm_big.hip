@@ -34,6 +34,9 @@
 //   * the pre-norm's sums of squares are matrix instructions too, one for 16 rows and 32 columns, a sixteenth of the product's
 //     (gate-up at 33 216 rows 160 -> 154 us, at 18 432 rows 96 -> 90; as vector instructions between the matrix ones they cost 12 % of
 //     a launch, in 128 x 128 tiles 14 %: 177 -> 169).  The results' distance from 64 bits is the same to seven digits, K 512 .. 2560;
+//   * in a pass of many rows they are not formed here at all: the residual updates leave them where they write the hidden (uvmi_gemm_sums;
+//     gate-up at 33 216 rows 144 -> 133 us, at 18 432 rows 86 -> 79; without any norm 128 and 77).  Against 64 bits the products are as before
+//     (2-norms of the error over 12 288 .. 40 000 rows, K 256 .. 1024, equal to eight digits, fp16 to six, the smaller of the two);
 //   * no loads are made past the last slab (they were, to keep the loop free of branches: the epilogue then waited for them;
 //     1 - 3 % of a launch);
 //   * tiles are dealt to the XCDs in contiguous runs, as in the tiled kernel; a workgroup's tiles are a stride apart in its XCD's run.
@@ -51,7 +54,9 @@ struct BigParams {
   int M, N, K, tiles_m, tiles_n;
   int rowsplit;
   float eps, ca, cb, cap_c;
+  float* sums; uint32_t sums_ld4; int parts;   // NORM 2: read; EPI 2 (or null): written.  parts x sums_ld4 bytes
 };
+constexpr int SUM_PARTS = 16;
 
 // Two dwords x, y per lane in lane groups g = lane / 16 (x0 .. x3, y0 .. y3) -> x = (x0, x2, y0, y2), y = (x1, x3, y1, y3).
 // (permlane32_swap exchanges the upper 32 lanes of its first operand with the lower 32 of its second, permlane16_swap does the
@@ -86,18 +91,19 @@ __device__ __forceinline__ int fresh_lane() {
 
 // EPI 0: C = A W^T (M, N).  EPI 1: W rows are [gate 16 | up 16] slabs; C = silu(gate) * up, (M, N / 2).
 // EPI 2: C = ca * R + cb * (A W^T).  EPI 3: C fp32 = ca * sigmoid((x + cb) / cap_c) of the rounded product x.  NORM: A stands
-// for its RMS-normalised rows.
+// for its RMS-normalised rows, whose squares are summed here (1) or were by the launches that wrote them (2: a number per row and 64
+// columns, which an EPI 2 launch leaves).
 // FI: 16-row fragments per wave along M: 8 - the 256 x 256 tile on 8 waves (2 x 4); 6 - 192 x 128 on 4 waves (2 x 2, 96 x 64 per wave, two
 // workgroups per compute unit; no pre-norm); 4 - a 128 x 128 tile on 4 waves (64 x 64 per wave, two workgroups per compute unit) for passes whose 256 x 256 tiles would not fill the device.  (A
 // 64 x 64 tile on 2 waves was measured too: no faster at 2 k rows than 64 x 64 tiles staged through registers.)
 // MANY: a workgroup takes several tiles (an even number of slabs: a tile ends on the stage that it does not begin on).
 template <int FI> constexpr int BIG_THREADS = FI == 8 ? 512 : 256;
-template <int DT, int EPI, bool NORM, int FI, bool MANY>
+template <int DT, int EPI, int NORM, int FI, bool MANY>
 __global__ __launch_bounds__(BIG_THREADS<FI>) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_big_kernel(BigParams P) {
   constexpr int WN = BIG_THREADS<FI> / 128;    // waves along N (2 along M)
   constexpr int BM = 32 * FI, BN = 64 * WN, LA = BM / (16 * WN);   // LA: a wave's loads of A per slab (of W: 4)
-  static_assert(!NORM || FI / 2 == WN, "a wave along N for every pair of a wave's row fragments");
+  static_assert(NORM != 1 || FI / 2 == WN, "a wave along N for every pair of a wave's row fragments");
   // one array per stage and operand: the compiler can then tell that the operand reads of one stage do not touch the
   // stage a load in flight is writing, and does not wait for that load
   __shared__ __attribute__((aligned(1024))) unsigned char sA0[BM * 128];
@@ -105,6 +111,7 @@ void gemm_big_kernel(BigParams P) {
   __shared__ __attribute__((aligned(1024))) unsigned char sB0[BN * 128];
   __shared__ __attribute__((aligned(1024))) unsigned char sB1[BN * 128];
   __shared__ float sRS[NORM ? BM : 1];
+  __shared__ __attribute__((aligned(1024))) unsigned char sPart[NORM == 2 ? SUM_PARTS * BM * 4 : 4];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -166,7 +173,7 @@ void gemm_big_kernel(BigParams P) {
     b_off[s] = (uint32_t)wn * 8192 + lo;
   }
 #pragma unroll
-  for (int p = 0; p < NP; p++) pair_at[p] = (uint32_t)(NORM ? ((p + wn) & (NP - 1)) : p) * 4096;
+  for (int p = 0; p < NP; p++) pair_at[p] = (uint32_t)(NORM == 1 ? ((p + wn) & (NP - 1)) : p) * 4096;
   gf4 acc[FI][4];
 
   gu4 w0[4], w1[4], f0[2], f1[2], f2[2];
@@ -176,7 +183,7 @@ void gemm_big_kernel(BigParams P) {
   };
   auto read_a = [&](const unsigned char* sa, int s, int i, gu4* f) {
     uint32_t o;
-    if constexpr (NORM) asm volatile("v_add_u32 %0, %1, %2" : "=v"(o) : "s"(pair_at[i / 2]), "v"(a_off[s]));   // (kept out of registers between uses)
+    if constexpr (NORM == 1) asm volatile("v_add_u32 %0, %1, %2" : "=v"(o) : "s"(pair_at[i / 2]), "v"(a_off[s]));   // (kept out of registers between uses)
     else o = a_off[s] + pair_at[i / 2];
     f[0] = *(const gu4*)(sa + o);
     f[1] = *(const gu4*)(sa + o + 2048);
@@ -194,12 +201,12 @@ void gemm_big_kernel(BigParams P) {
   // which is its first pair (as a branch on wn it costs 4 us of 157).
   gf4 sq[2];
   auto sumsq = [&](int pair, const gu4* f) {
-    if (NORM && pair == 0) {
+    if (NORM == 1 && pair == 0) {
 #pragma unroll
       for (int u = 0; u < 2; u++) sq[u] = gmfma<DT>(f[u], f[u], sq[u]);
     }
   };
-  auto frow = [&](int i) { return 16 * FI * wm + 16 * (NORM ? ((i + 2 * wn) & (FI - 1)) : i); };   // first tile row of accumulator row fragment i
+  auto frow = [&](int i) { return 16 * FI * wm + 16 * (NORM == 1 ? ((i + 2 * wn) & (FI - 1)) : i); };   // first tile row of accumulator row fragment i
 #define UVMI_SB() __builtin_amdgcn_sched_barrier(0)
 
   auto clear = [&]() {
@@ -209,7 +216,29 @@ void gemm_big_kernel(BigParams P) {
       for (int j = 0; j < 4; j++) acc[i][j] = gf4{0.f, 0.f, 0.f, 0.f};
     sq[0] = sq[1] = gf4{0.f, 0.f, 0.f, 0.f};
   };
+  // NORM 2: the sums of the tile's rows, SUM_PARTS x BM, on their way with its first slab, and its scales, formed behind its first barrier, when all
+  // waves are past the epilogue before (requested there the sums were waited for, added up in the epilogue they held it: 4 - 7 us
+  // of 80 - 140)
+  auto issue_sums = [&]() {
+    if constexpr (NORM == 2) {
+      const __amdgpu_buffer_rsrc_t rS = __builtin_amdgcn_make_buffer_rsrc((void*)P.sums, 0, (int)(P.parts * P.sums_ld4), 0x00020000);
+      const int ln = fresh_lane();
+      for (int b = wave; b * 256 < P.parts * BM; b += 2 * WN)
+        load_lds16(rS, sPart + b * 1024, (uint32_t)((b * 256 + 4 * ln) / BM) * P.sums_ld4 + 4 * (m0 + (b * 256 + 4 * ln) % BM), 0);
+    }
+  };
+  auto scales = [&]() {
+    if constexpr (NORM == 2) {
+      if (wave < BM / 64) {   // (two lanes a row, for half of the numbers each, in batches: no faster)
+        const int row = 64 * wave + fresh_lane();
+        float v = 0.f;
+        for (int p = 0; p < P.parts; p++) v += ((const float*)sPart)[p * BM + row];
+        sRS[row] = rsqrtf(v / (float)P.K + P.eps);
+      }
+    }
+  };
   issue(sA0, sB0, 0);
+  issue_sums();
   clear();
 #pragma unroll
   for (int i = 0; i < FI; i++) asm volatile("" : "+v"(acc[i][0]), "+v"(acc[i][1]), "+v"(acc[i][2]), "+v"(acc[i][3]));   // (while the loads are on their way)
@@ -223,7 +252,7 @@ void gemm_big_kernel(BigParams P) {
     auto request = [&](unsigned char* sa, unsigned char* sb, int k) {
       if (k < nk) issue(sa, sb, k);
       else if (more) {
-        if (k == nk) { tile_at(L + step); offsets(); }
+        if (k == nk) { tile_at(L + step); offsets(); issue_sums(); }
         issue(sa, sb, k - nk);
       }
     };
@@ -286,12 +315,14 @@ void gemm_big_kernel(BigParams P) {
     } else if constexpr (FI == 8) {
       for (; k + 2 <= nk; k += 2) {
         UVMI_ITER(sA0, sB0, sA1, sB1, k);
+        if (k == 0) scales();
         UVMI_ITER(sA1, sB1, sA0, sB0, k + 1);
       }
       if (!MANY && k < nk) UVMI_ITER(sA0, sB0, sA1, sB1, k);
     } else {
       for (; k + 2 <= nk; k += 2) {
         UVMI_ITER4(sA0, sB0, sA1, sB1, k, f0, f1);
+        if (k == 0) scales();
         UVMI_ITER4(sA1, sB1, sA0, sB0, k + 1, f1, f0);
       }
       if (!MANY && k < nk) UVMI_ITER4(sA0, sB0, sA1, sB1, k, f0, f1);
@@ -306,7 +337,10 @@ void gemm_big_kernel(BigParams P) {
     float rn[FI];
 #pragma unroll
     for (int i = 0; i < FI; i++) rn[i] = 1.0f;
-    if (NORM) {
+    if constexpr (NORM == 2) {
+#pragma unroll
+      for (int i = 0; i < FI; i++) rn[i] = sRS[frow(i) + r];
+    } else if constexpr (NORM == 1) {
       int kd = P.K;
       asm volatile("" : "+s"(kd));   // (not a register of its own through the main loop)
 #pragma unroll
@@ -395,6 +429,7 @@ void gemm_big_kernel(BigParams P) {
         xpose4(hi);
         // lane (r, g) now holds columns 16 g .. 16 g + 15 of the wave's 64: words lo[0] hi[0] lo[1] hi[1] ...
         const int n = cn0 + 64 * wn + 16 * g;
+        float s = 0.f;
         if (row < P.M && n < P.N) {
           uint32_t wds[8] = {lo[0], hi[0], lo[1], hi[1], lo[2], hi[2], lo[3], hi[3]};
           const uint4 q0 = res[i][0], q1 = res[i][1];
@@ -409,6 +444,21 @@ void gemm_big_kernel(BigParams P) {
           uint16_t* cp = (uint16_t*)P.c + (int64_t)row * P.ldc + n;
           *(uint4*)cp = uint4{wds[0], wds[1], wds[2], wds[3]};
           *(uint4*)(cp + 8) = uint4{wds[4], wds[5], wds[6], wds[7]};
+          if (NORM == 0 && P.sums) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+              float x0, x1;
+              gunpack<DT>(wds[e], x0, x1);
+              s = fmaf(x1, x1, fmaf(x0, x0, s));
+            }
+          }
+        }
+        if (NORM == 0 && P.sums) {   // the squares of the row's 64 columns: its 4 lane groups
+          auto t = __builtin_amdgcn_permlane16_swap(__float_as_uint(s), __float_as_uint(s), false, false);
+          s = __uint_as_float(t[0]) + __uint_as_float(t[1]);
+          t = __builtin_amdgcn_permlane32_swap(__float_as_uint(s), __float_as_uint(s), false, false);
+          s = __uint_as_float(t[0]) + __uint_as_float(t[1]);
+          if (g == 0 && row < P.M && cn0 + 64 * wn < P.N) *(float*)((char*)P.sums + (uint32_t)(cn0 / 64 + wn) * P.sums_ld4 + 4 * (uint32_t)row) = s;
         }
       }
     }
@@ -430,19 +480,19 @@ static void launch_big(const uvmi_gemm_args* a, const BigParams& P, int cus, hip
     if (many) hipLaunchKernelGGL((gemm_big_kernel<DT, EPI, NORM, FI, true>), grid, blk, 0, st, P);      \
     else hipLaunchKernelGGL((gemm_big_kernel<DT, EPI, NORM, FI, false>), grid, blk, 0, st, P);          \
   } while (0)
-  const bool norm = a->norm_a != 0;
+  const int norm = a->norm_a ? (P.sums ? 2 : 1) : 0;
   if constexpr (FI == 6) {
-    UVMI_GO(2, false);
-  } else if (a->epilogue == UVMI_GEMM_RESID) { if (norm) UVMI_GO(2, true); else UVMI_GO(2, false); }
-  else if (a->epilogue == UVMI_GEMM_SWIGLU) { if (norm) UVMI_GO(1, true); else UVMI_GO(1, false); }
-  else if (a->epilogue == UVMI_GEMM_SOFTCAP) { if (norm) UVMI_GO(3, true); else UVMI_GO(3, false); }
-  else { if (norm) UVMI_GO(0, true); else UVMI_GO(0, false); }
+    UVMI_GO(2, 0);
+  } else if (a->epilogue == UVMI_GEMM_RESID) { if (norm) UVMI_GO(2, 1); else UVMI_GO(2, 0); }
+  else if (a->epilogue == UVMI_GEMM_SWIGLU) { if (norm == 2) UVMI_GO(1, 2); else if (norm) UVMI_GO(1, 1); else UVMI_GO(1, 0); }
+  else if (a->epilogue == UVMI_GEMM_SOFTCAP) { if (norm) UVMI_GO(3, 1); else UVMI_GO(3, 0); }
+  else { if (norm == 2) UVMI_GO(0, 2); else if (norm) UVMI_GO(0, 1); else UVMI_GO(0, 0); }
 #undef UVMI_GO
 }
 
 // Arguments are validated by the caller (uvmi_gemm_tn_ex), which also checks K >= 128.  tile: 256, 128 or (RESID without
-// the pre-norm: uvmi_gemm_resid) 192 rows.
-void gemm_big_launch(const uvmi_gemm_args* a, int tile, int cus, hipStream_t st) {
+// the pre-norm: uvmi_gemm_resid) 192 rows.  sums: as uvmi_gemm_sums has it, or null.
+void gemm_big_launch(const uvmi_gemm_args* a, int tile, int cus, hipStream_t st, float* sums, int64_t sums_ld) {
   BigParams P;
   P.a = a->a; P.w = a->w; P.c = a->c; P.r = a->resid;
   P.lda2 = (uint32_t)a->lda * 2; P.ldw2 = (uint32_t)a->ldw * 2; P.ldc = a->ldc; P.ldr = a->ldr;
@@ -450,6 +500,7 @@ void gemm_big_launch(const uvmi_gemm_args* a, int tile, int cus, hipStream_t st)
   const int cols = tile == 192 ? 128 : tile;
   P.tiles_m = (int)((a->M + tile - 1) / tile);
   P.tiles_n = (a->N + cols - 1) / cols;
+  P.sums = sums; P.sums_ld4 = (uint32_t)sums_ld * 4; P.parts = ((a->norm_a ? a->K : a->N) + 63) / 64;
   P.eps = a->eps; P.ca = a->ca; P.cb = a->cb; P.cap_c = a->cap_c;
   const double bytes_a = (double)a->M * a->K, bytes_w = (double)a->N * a->K;
   P.rowsplit = bytes_a / 8 + bytes_w < bytes_a + bytes_w / 8;

@@ -21,6 +21,7 @@ extern "C" int uvmi_run_ops(const int* kinds, const void* const* args, int n_ops
       case UVMI_OP_QKV_PROJ: rc = uvmi_qkv_proj((const struct uvmi_qkv_proj_args*)a, stream); break;
       case UVMI_OP_PREFILL_ATTN_O: rc = uvmi_prefill_attn_o((const struct uvmi_prefill_attn_o_args*)a, stream); break;
       case UVMI_OP_GEMM_RESID: rc = uvmi_gemm_resid((const uvmi_gemm_args*)a, stream); break;
+      case UVMI_OP_GEMM_SUMS: rc = uvmi_gemm_sums((const struct uvmi_gemm_sums_args*)a, stream); break;
       case UVMI_OP_NORM: rc = uvmi::norm_run((const uvmi_norm_args*)a, stream); break;
       default: UVMI_REQUIRE(false, UVMI_EINVAL, "uvmi_run_ops: operation %d has the unknown kind %d", i, kinds[i]);
     }

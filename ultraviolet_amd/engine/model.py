@@ -230,6 +230,21 @@ class UVEngine:
         g = gemm_args(a, w, out, epilogue, **kw)
         self._op(L.OP_GEMM_RESID if epilogue == RESID else L.OP_GEMM, g, (a, w, out), M="n")
 
+    def _gemm_sums(self, a: Tensor, w: Tensor, out: Tensor, epilogue: int = STORE, **kw):
+        """_gemm of a pass that keeps its hidden's sums of squares (_sums_ok), in what buf h is for other plans."""
+        h = self.buf["h"]
+        g = gemm_args(a, w, out, epilogue, **kw)
+        self._op(L.OP_GEMM_SUMS, L.GemmSumsArgs(C.addressof(g), h.data_ptr(), (self.max_tokens + 3) // 4 * 4), (g, a, w, out, h))
+        if self._rec is not None:
+            self._rec.field(g, "M", "n")
+
+    def _sums_ok(self, n: int) -> bool:
+        """Whether the residual updates of a packed pass sum the squares of the hidden they write for the projections that take its norm.
+        Formed again in every tile that reads it, it is a sixteenth of their matrix instructions: gate-up at 18 432 rows 86 us against 79 so, extended
+        projection 22.7 / 21.4; at 33 216 rows 144 / 133, 37.7 / 35.9; the updates pay 0.4 - 1 us each (a pass of 64 prompts 2252 -> 2200 us, a
+        mixed one 3901 -> 3824).  All four have to run on the kernels of many rows."""
+        return n >= max(self.big_rows, 12288) and n <= min(self.fold_qkv_rows, 1 << 16) and self.gemm_config == 0 and 256 <= self.cfg.d_model <= 1024
+
     def _embed_norm(self, tok: Tensor, n: int):
         b = self.buf
         self._op(L.OP_NORM, L.NormArgs(x=self.w.embed.data_ptr(), tok=tok.data_ptr(), vocab=self.cfg.vocab_size, dtype=self.dt_code, rows=n,
@@ -613,20 +628,27 @@ class UVEngine:
         x, zg, act = b["x"][:n], b["zg"][:n], b["act"][:n]
         gc = self.gemm_config
         own_down = n <= self.skinny_rows or n >= self.big_rows or self.fold_down_rows[0] <= n <= self.fold_down_rows[1]
+        sums = last_pos is not None and self._sums_ok(n)
+        project = self._gemm_sums if sums else self._gemm
         for l, W in enumerate(self.w.layers):
             gemm = None
-            if n <= self.fold_qkv_rows and last_pos is not None:   # (decode rows alone: the projection of the fused attention's plans, to the same bits)
+            if sums and l > 0:
+                self._gemm_sums(x, W["wqkv_ext"], b["qkvx"][:n], norm_eps=self.eps)
+            elif n <= self.fold_qkv_rows and last_pos is not None:   # (decode rows alone: the projection of the fused attention's plans, to the same bits)
                 gemm = gemm_args(b["xn" if l == 0 else "x"][:n], W["wqkv_ext"], b["qkvx"][:n], norm_eps=None if l == 0 else self.eps, config=gc)
             else:
                 self._project_qkv(l, n, n <= self.fold_qkv_rows, config=gc)
             self._qkv_post(l, tok, pos, rows, last_pos, st, n, ext=True, gemm=gemm)
-            if oproj:   # (the attention's launch, or one behind it)
+            if oproj and not sums:   # (the attention's launch, or one behind it)
                 attn(l, b["q"][:n], gemm_args(zg, W["wo"], x, RESID, resid=x, ca=W["resid_attn"], cb=W["post_attn"], config=gc))
             else:
                 self._finish_attn(l, attn(l, b["q"][:n]), x if l > 0 else None)
-                self._gemm(zg, W["wo"], x, RESID, resid=x, ca=W["resid_attn"], cb=W["post_attn"], config=gc)
-            self._gemm(x, W["gu_il"], act, SWIGLU, norm_eps=self.eps, config=gc)
-            self._down(l, n, own_down)
+                project(zg, W["wo"], x, RESID, resid=x, ca=W["resid_attn"], cb=W["post_attn"], config=gc)
+            project(x, W["gu_il"], act, SWIGLU, norm_eps=self.eps, config=gc)
+            if sums:
+                self._gemm_sums(act, W["down"], x, RESID, resid=x, ca=W["resid_mlp"], cb=W["post_mlp"])
+            else:
+                self._down(l, n, own_down)
 
     def _layers_plain(self, n: int, tok, pos, rows, last_pos, st, attn, fused_attn) -> bool:
         """The reference's order of operations on the vendor library's GEMMs (16-bit passes of few rows: on this one's),
@@ -683,7 +705,7 @@ class UVEngine:
         elsewhere (weights and residual scalars, cache tensors, a switch of the launch plans)."""
         own_down = n <= self.skinny_rows or n >= self.big_rows or self.fold_down_rows[0] <= n <= self.fold_down_rows[1]
         key = (what, kind, n <= self.fold_qkv_rows, n <= self.fold_o_rows, n <= self.fold_gu_rows, own_down,
-               self.fold_down_rows[0] <= n <= self.fold_down_rows[1], self.gemm_config, getattr(self.w, "scalar_epoch", 0))
+               self.fold_down_rows[0] <= n <= self.fold_down_rows[1], self._sums_ok(n), self.gemm_config, getattr(self.w, "scalar_epoch", 0))
         plans = self._plans.get(st)
         if plans is None:
             plans = self._plans[st] = {}

@@ -93,7 +93,8 @@ class PassPlan:
 
 
 _ENTRY = {L.OP_GEMM: "uvmi_gemm_tn_ex", L.OP_DECODE_ATTN: "uvmi_decode_attn", L.OP_QKV_POST: "uvmi_qkv_post", L.OP_PREFILL_ATTN: "uvmi_prefill_attn",
-          L.OP_QKV_PROJ: "uvmi_qkv_proj", L.OP_PREFILL_ATTN_O: "uvmi_prefill_attn_o", L.OP_GEMM_RESID: "uvmi_gemm_resid"}
+          L.OP_QKV_PROJ: "uvmi_qkv_proj", L.OP_PREFILL_ATTN_O: "uvmi_prefill_attn_o", L.OP_GEMM_RESID: "uvmi_gemm_resid",
+          L.OP_GEMM_SUMS: "uvmi_gemm_sums"}
 
 
 def launch(kind: int, args, stream: int):
