@@ -444,9 +444,9 @@ struct uvmi_norm_args {
 };
 
 /* The extended QKV projection (uvmi_gemm_tn_ex) and the post-processing of its rows (uvmi_qkv_post), which reads gemm->c at post->qkv with the
- * gates' logits behind q, k, v: as one launch for a few hundred rows of 8 query heads on 1 kv head, else as the two.  What becomes of
- * gemm->c is unspecified: the one launch does not write it. */
-struct uvmi_qkv_proj_args { const struct uvmi_gemm_args* gemm; const uvmi_qkv_post_args* post; };
+ * gates' logits behind q, k, v: as one launch for a few hundred rows of 8 query heads on 1 kv head, else as two, of which the first may have the query
+ * heads' part.  What becomes of gemm->c is unspecified.  sums (or NULL), sums_ld: the projection is uvmi_gemm_sums'. */
+struct uvmi_qkv_proj_args { const struct uvmi_gemm_args* gemm; const uvmi_qkv_post_args* post; float* sums; int64_t sums_ld; };
 int uvmi_qkv_proj(const struct uvmi_qkv_proj_args* a, void* stream);
 
 /* Packed attention (uvmi_prefill_attn) and the output projection with its residual update of the rows that it writes (gemm->a is attn->out; RESID): as

@@ -145,8 +145,8 @@ class PromptTablesArgs(C.Structure):   # struct uvmi_prompt_tables_args
                 ("check_in", C.c_void_p), ("check_out", C.c_void_p), ("check_zero", C.c_int)]
 
 
-class QkvProjArgs(C.Structure):   # struct uvmi_qkv_proj_args: addresses of a GemmArgs and a QkvPostArgs
-    _fields_ = [("gemm", C.c_void_p), ("post", C.c_void_p)]
+class QkvProjArgs(C.Structure):   # struct uvmi_qkv_proj_args: addresses of a GemmArgs, a QkvPostArgs and sums of squares
+    _fields_ = [("gemm", C.c_void_p), ("post", C.c_void_p), ("sums", C.c_void_p), ("sums_ld", C.c_int64)]
 
 
 class PrefillAttnOArgs(C.Structure):   # struct uvmi_prefill_attn_o_args: addresses of a PrefillAttnArgs and a GemmArgs

@@ -2,12 +2,13 @@
 // 256 x 256 tiles loaded straight into LDS), gemm_tile.hip (128 x 128 tiles through registers: outputs whose rows are not 16-byte
 // aligned).
 #include "common.h"
+#include "qkv_post.h"
 
 using namespace uvmi;
 
 namespace uvmi {
 void gemm_tile_launch(const uvmi_gemm_args* a, hipStream_t st);                     // gemm_tile.hip
-void gemm_big_launch(const uvmi_gemm_args* a, int tile, int cus, hipStream_t st, float* sums = nullptr, int64_t sums_ld = 0);   // gemm_big.hip; tile: 128, 256, 192 (x 128: RESID)
+void gemm_big_launch(const uvmi_gemm_args* a, int tile, int cus, hipStream_t st, float* sums = nullptr, int64_t sums_ld = 0, const QueryPost* q = nullptr);   // gemm_big.hip; tile: 128, 256, 192 (x 128: RESID)
 int gemm_stream_form(const uvmi_gemm_args* a, int cus);                             // gemm_stream.hip
 void gemm_stream_tile(int form, int* rows, int* cols);
 void gemm_stream_launch(const uvmi_gemm_args* a, int form, int cus, hipStream_t st);
@@ -32,10 +33,10 @@ static bool big_ok(const uvmi_gemm_args* a) {
 // 104.9; 33 216 rows, 7 against 14, 150 / 171.  640 columns, K 1664: 18 432 rows, 1 against 2, 51.2 / 59.4; 24 576 rows, 2 against 2, 97.1 /
 // 66.4; 40 000 rows, 2 against 4, 103 / 112.  With a short K a last round of 128 x 128 tiles that fills a quarter of the device or
 // less takes half a round (K 512: 16 384 rows 21.9 / 20.4, 18 432 rows, 0.4 of a round, 23.4 / 26.0).
-static bool big_tiles_pay(const uvmi_gemm_args* a, int64_t t128, int64_t t256, int cus) {
+static bool big_tiles_pay(const uvmi_gemm_args* a, int64_t t128, int64_t t256, int cus, int round256 = 17) {
   const int64_t r256 = (t256 + cus - 1) / cus, slots = 2 * (int64_t)cus, rest = t128 % slots;
   const int64_t halves128 = 2 * (t128 / slots) + (rest == 0 ? 0 : (a->K <= 768 && 4 * rest <= slots ? 1 : 2));
-  return 17 * r256 <= 5 * halves128;
+  return round256 * r256 <= 5 * halves128;
 }
 
 extern "C" int uvmi_gemm_tn_supported(int dtype, int64_t M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc, int epilogue) {
@@ -182,19 +183,38 @@ extern "C" int uvmi_gemm_resid(const uvmi_gemm_args* a, void* stream) {
 
 // A pass of many rows takes the squares of a block's hidden where the residual updates write it, 64 columns at a time, not again in every
 // column of tiles that reads it.
-extern "C" int uvmi_gemm_sums(const struct uvmi_gemm_sums_args* s, void* stream) {
-  UVMI_REQUIRE(s && s->gemm && s->sums, UVMI_EINVAL, "uvmi_gemm_sums: null pointer");
-  const uvmi_gemm_args* a = s->gemm;
-  const int rc = check_gemm(a);
-  if (rc) return rc;
+static int check_sums(const uvmi_gemm_args* a, const float* sums, int64_t ld) {
   const bool writes = a->epilogue == UVMI_GEMM_RESID && !a->norm_a, reads = a->norm_a && (a->epilogue == UVMI_GEMM_STORE || a->epilogue == UVMI_GEMM_SWIGLU);
   UVMI_REQUIRE((writes || reads) && (writes ? a->N : a->K) <= 1024 && (writes || a->K >= 256) && big_ok(a) && a->M > 0 &&
                (a->config == 5 || a->config == 6 || (a->config == 0 && a->M >= BIG_MIN_ROWS)), UVMI_EUNSUPPORTED,
                "uvmi_gemm_sums: RESID without a pre-norm or STORE / SWIGLU with one, of a hidden of 256 to 1024 columns, on tiles loaded straight into LDS");
-  UVMI_REQUIRE((uintptr_t)s->sums % 16 == 0 && s->ld % 4 == 0 && s->ld >= a->M && s->ld <= (1 << 24), UVMI_EINVAL,
+  UVMI_REQUIRE((uintptr_t)sums % 16 == 0 && ld % 4 == 0 && ld >= a->M && ld <= (1 << 24), UVMI_EINVAL,
                "uvmi_gemm_sums: sums 16-byte aligned, with a pitch that is a multiple of 4, >= M");
+  return UVMI_OK;
+}
+
+extern "C" int uvmi_gemm_sums(const struct uvmi_gemm_sums_args* s, void* stream) {
+  UVMI_REQUIRE(s && s->gemm && s->sums, UVMI_EINVAL, "uvmi_gemm_sums: null pointer");
+  const uvmi_gemm_args* a = s->gemm;
+  int rc = check_gemm(a);
+  if (!rc) rc = check_sums(a, s->sums, s->ld);
+  if (rc) return rc;
   const int cus = compute_units();
   gemm_big_launch(a, resid_192(a, cus) ? 192 : gemm_path(a, cus).form, cus, (hipStream_t)stream, s->sums, s->ld);
   UVMI_CHECK_LAUNCH("uvmi_gemm_sums");
   return UVMI_OK;
+}
+
+bool uvmi::gemm_query_post(const uvmi_gemm_args* a, const QueryPost& q, float* sums, int64_t sums_ld, hipStream_t st) {
+  const int cus = compute_units();
+  if (check_gemm(a) || a->M == 0 || a->epilogue != UVMI_GEMM_STORE || a->K < 256 || q.rope_n > (1 << 23)) return false;
+  if (sums && check_sums(a, sums, sums_ld)) return false;
+  Path p = gemm_path(a, cus);
+  if (p.kind != UVMI_GEMM_PATH_BIG) return false;
+  // (256 x 256 tiles come one to a workgroup here, a round costs more: 33 216 rows 49.7 us against 45.2 in 128 x 128 tiles; 40 000
+  // rows, two full rounds, 59.6 / 61.5 with the rest of the post-processing, 18 432 rows, one, 25.6 / 26.7)
+  const int64_t t256 = ((a->M + 255) / 256) * 3, t128 = ((a->M + 127) / 128) * 6;
+  if (a->config == 0 && p.form == 256 && t256 > cus && !big_tiles_pay(a, t128, t256, cus, 20)) p.form = 128;
+  gemm_big_launch(a, p.form, cus, st, sums, sums_ld, &q);
+  return true;
 }

@@ -44,6 +44,7 @@
 // pitches that are multiples of 8 elements (the caller checks).
 #include "common.h"
 #include "gemm_util.h"
+#include "qkv_post.h"
 
 namespace uvmi {
 
@@ -55,6 +56,7 @@ struct BigParams {
   int rowsplit;
   float eps, ca, cb, cap_c;
   float* sums; uint32_t sums_ld4; int parts;   // NORM 2: read; EPI 2 (or null): written.  parts x sums_ld4 bytes
+  QueryPost q;                                 // EPI 4
 };
 constexpr int SUM_PARTS = 16;
 
@@ -93,6 +95,9 @@ __device__ __forceinline__ int fresh_lane() {
 // EPI 2: C = ca * R + cb * (A W^T).  EPI 3: C fp32 = ca * sigmoid((x + cb) / cap_c) of the rounded product x.  NORM: A stands
 // for its RMS-normalised rows, whose squares are summed here (1) or were by the launches that wrote them (2: a number per row and 64
 // columns, which an EPI 2 launch leaves).
+// EPI 4: EPI 0 whose columns 0 .. 511, a wave's 64 of them a query head, are normed, rotated (QK-norm and RoPE, with the roundings of
+// qkv_post_rows_kernel) and go to q.out: 18 432 rows 21.7 -> 25.8 us on 256 x 256 tiles, 33 216 rows 39.2 -> 45.5 on 128 x 128 ones, where an epilogue
+// runs beside another workgroup's main loop.
 // FI: 16-row fragments per wave along M: 8 - the 256 x 256 tile on 8 waves (2 x 4); 6 - 192 x 128 on 4 waves (2 x 2, 96 x 64 per wave, two
 // workgroups per compute unit; no pre-norm); 4 - a 128 x 128 tile on 4 waves (64 x 64 per wave, two workgroups per compute unit) for passes whose 256 x 256 tiles would not fill the device.  (A
 // 64 x 64 tile on 2 waves was measured too: no faster at 2 k rows than 64 x 64 tiles staged through registers.)
@@ -112,6 +117,8 @@ void gemm_big_kernel(BigParams P) {
   __shared__ __attribute__((aligned(1024))) unsigned char sB1[BN * 128];
   __shared__ float sRS[NORM ? BM : 1];
   __shared__ __attribute__((aligned(1024))) unsigned char sPart[NORM == 2 ? SUM_PARTS * BM * 4 : 4];
+  __shared__ __attribute__((aligned(1024))) unsigned char sPos[EPI == 4 ? BM * 8 : 4];
+  __shared__ int sAt[EPI == 4 ? BM : 1];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -217,7 +224,7 @@ void gemm_big_kernel(BigParams P) {
     sq[0] = sq[1] = gf4{0.f, 0.f, 0.f, 0.f};
   };
   // NORM 2: the sums of the tile's rows, SUM_PARTS x BM, on their way with its first slab, and its scales, formed behind its first barrier, when all
-  // waves are past the epilogue before (requested there the sums were waited for, added up in the epilogue they held it: 4 - 7 us
+  // waves are past the epilogue before; EPI 4: likewise the rows' positions and what they point to in the table (requested there the sums were waited for, added up in the epilogue they held it: 4 - 7 us
   // of 80 - 140)
   auto issue_sums = [&]() {
     if constexpr (NORM == 2) {
@@ -225,6 +232,10 @@ void gemm_big_kernel(BigParams P) {
       const int ln = fresh_lane();
       for (int b = wave; b * 256 < P.parts * BM; b += 2 * WN)
         load_lds16(rS, sPart + b * 1024, (uint32_t)((b * 256 + 4 * ln) / BM) * P.sums_ld4 + 4 * (m0 + (b * 256 + 4 * ln) % BM), 0);
+    }
+    if constexpr (EPI == 4) {
+      const __amdgpu_buffer_rsrc_t rP = __builtin_amdgcn_make_buffer_rsrc((void*)P.q.pos, 0, P.M * 8, 0x00020000);
+      if (wave < BM / 128) load_lds16(rP, sPos + wave * 1024, (uint32_t)m0 * 8 + 1024 * wave + 16 * fresh_lane(), 0);
     }
   };
   auto scales = [&]() {
@@ -234,6 +245,13 @@ void gemm_big_kernel(BigParams P) {
         float v = 0.f;
         for (int p = 0; p < P.parts; p++) v += ((const float*)sPart)[p * BM + row];
         sRS[row] = rsqrtf(v / (float)P.K + P.eps);
+      }
+    }
+    if constexpr (EPI == 4) {
+      if (wave < BM / 64) {
+        const int row = 64 * wave + fresh_lane();
+        const int64_t p = ((const int64_t*)sPos)[row];
+        sAt[row] = P.q.tab && p >= 0 && p < P.q.rope_n ? (int)p * 128 : -1;   // (bytes)
       }
     }
   };
@@ -315,14 +333,14 @@ void gemm_big_kernel(BigParams P) {
     } else if constexpr (FI == 8) {
       for (; k + 2 <= nk; k += 2) {
         UVMI_ITER(sA0, sB0, sA1, sB1, k);
-        if (k == 0) scales();
+        if ((NORM == 2 || EPI == 4) && k == 0) scales();
         UVMI_ITER(sA1, sB1, sA0, sB0, k + 1);
       }
       if (!MANY && k < nk) UVMI_ITER(sA0, sB0, sA1, sB1, k);
     } else {
       for (; k + 2 <= nk; k += 2) {
         UVMI_ITER4(sA0, sB0, sA1, sB1, k, f0, f1);
-        if (k == 0) scales();
+        if ((NORM == 2 || EPI == 4) && k == 0) scales();
         UVMI_ITER4(sA1, sB1, sA0, sB0, k + 1, f1, f0);
       }
       if (!MANY && k < nk) UVMI_ITER4(sA0, sB0, sA1, sB1, k, f0, f1);
@@ -352,6 +370,19 @@ void gemm_big_kernel(BigParams P) {
 #pragma unroll
       for (int i = 0; i < FI; i++) rn[i] = sRS[frow(i) + r];
     }
+
+    // ---- EPI 4: rotations of row fragment i + 1 on their way while fragment i is finished
+    const bool head = EPI == 4 && cn0 + 64 * wn < 512;
+    int at[2];
+    float4 cs[2], sn[2];
+    auto rotation = [&](int i) {
+      at[i & 1] = sAt[EPI == 4 ? frow(i) + r : 0];
+      if (!P.q.tab) return;
+      const float* t = (const float*)((const char*)P.q.tab + (uint32_t)max(at[i & 1], 0)) + 4 * g;
+      cs[i & 1] = *(const float4*)t;
+      sn[i & 1] = *(const float4*)(t + 16);
+    };
+    if (EPI == 4 && head) rotation(0);
 
     // ---- epilogue: accumulator (i, j): lane (r, g) holds C[m0 + 16 FI wm + 16 i + r][n0 + 64 wn + 16 j + 4 g + t], t = 0..3
     uint4 res[EPI == 2 ? FI : 1][2];
@@ -399,22 +430,59 @@ void gemm_big_kernel(BigParams P) {
           if (row < P.M && n < P.N)
             *(float4*)((float*)P.c + (int64_t)row * P.ldc + n) = float4{cap(acc[i][j][0]), cap(acc[i][j][1]), cap(acc[i][j][2]), cap(acc[i][j][3])};
         }
-      } else if (EPI == 0) {
+      } else if (EPI == 0 || EPI == 4) {
+        uint32_t w[4][2];   // columns 16 j + 4 g ..
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          const gf4 v = acc[i][j] * rn[i];
+          w[j][0] = gpack<DT>(v[0], v[1]);
+          w[j][1] = gpack<DT>(v[2], v[3]);
+        }
+        if constexpr (EPI == 4) {
+          if (head) {
+            if (i + 1 < FI) rotation(i + 1);
+            auto round2 = [](float& a, float& b) { gunpack<DT>(gpack<DT>(a, b), a, b); };
+            float x[4][4], ss = 0.f;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+              gunpack<DT>(w[j][0], x[j][0], x[j][1]);
+              gunpack<DT>(w[j][1], x[j][2], x[j][3]);
+#pragma unroll
+              for (int t = 0; t < 4; t++) ss = fmaf(x[j][t], x[j][t], ss);
+            }
+            const float rs = rsqrtf(xsum32(xsum16(ss)) * (1.0f / 64.0f) + P.q.eps);
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+              w[j][0] = gpack<DT>(x[j][0] * rs, x[j][1] * rs);
+              w[j][1] = gpack<DT>(x[j][2] * rs, x[j][3] * rs);
+            }
+            if (at[i & 1] >= 0) {   // dims d and d + 16, columns of fragments 0 and 1 (rope_rot, two at a time)
+              const float c4[4] = {cs[i & 1].x, cs[i & 1].y, cs[i & 1].z, cs[i & 1].w}, s4[4] = {sn[i & 1].x, sn[i & 1].y, sn[i & 1].z, sn[i & 1].w};
+#pragma unroll
+              for (int t = 0; t < 4; t += 2) {
+                float a0, a1, b0, b1;
+                gunpack<DT>(w[0][t / 2], a0, a1);
+                gunpack<DT>(w[1][t / 2], b0, b1);
+                float ac0 = mul_sep(a0, c4[t]), ac1 = mul_sep(a1, c4[t + 1]), bs0 = mul_sep(b0, s4[t]), bs1 = mul_sep(b1, s4[t + 1]);
+                float bc0 = mul_sep(b0, c4[t]), bc1 = mul_sep(b1, c4[t + 1]), as0 = mul_sep(a0, s4[t]), as1 = mul_sep(a1, s4[t + 1]);
+                round2(ac0, ac1); round2(bs0, bs1); round2(bc0, bc1); round2(as0, as1);
+                w[0][t / 2] = gpack<DT>(add_sep(ac0, -bs0), add_sep(ac1, -bs1));
+                w[1][t / 2] = gpack<DT>(add_sep(bc0, as0), add_sep(bc1, as1));
+              }
+            }
+          }
+        }
+        uint16_t* const base = head ? (uint16_t*)P.q.out : (uint16_t*)P.c;
+        const int64_t pitch = head ? 512 : P.ldc;
 #pragma unroll
         for (int s = 0; s < 2; s++) {
           // columns 16 (2 s + j) + 4 g .. of fragments j = 0, 1 -> the 8 consecutive columns 32 s + 8 g ..: the 4 lane groups of a row
           // store 64 consecutive bytes (pieces of 16 bytes 32 apart: 33 216 x 656 x 640 51.9 us, so 49.2)
-          uint32_t x[2][2];
-#pragma unroll
-          for (int j = 0; j < 2; j++) {
-            const gf4 v = acc[i][2 * s + j] * rn[i];
-            x[j][0] = gpack<DT>(v[0], v[1]);
-            x[j][1] = gpack<DT>(v[2], v[3]);
-          }
-          xpose_pair(x[0][0], x[1][0]);
-          xpose_pair(x[0][1], x[1][1]);
+          uint32_t(&x0)[2] = w[2 * s], (&x1)[2] = w[2 * s + 1];
+          xpose_pair(x0[0], x1[0]);
+          xpose_pair(x0[1], x1[1]);
           const int n = cn0 + 64 * wn + 32 * s + 8 * g;
-          if (row < P.M && n < P.N) *(uint4*)((uint16_t*)P.c + (int64_t)row * P.ldc + n) = uint4{x[0][0], x[0][1], x[1][0], x[1][1]};
+          if (row < P.M && n < P.N) *(uint4*)(base + (int64_t)row * pitch + n) = uint4{x0[0], x0[1], x1[0], x1[1]};
         }
       } else {
         // (with the stores of EPI 0 here the residual's loads come in the same pieces: 0 - 3 % slower; requested in the last iteration
@@ -473,11 +541,12 @@ static void launch_big(const uvmi_gemm_args* a, const BigParams& P, int cus, hip
   const int T = P.tiles_m * P.tiles_n;
   const int slots = (FI == 8 ? cus : 2 * cus) / 8 * 8;   // workgroups that run at a time
   // (a launch of one round keeps the shorter code: it lost 0.5 us of 9 to the other's)
-  const bool many = P.K % 128 == 0 && slots > 0 && T > slots;
+  // (nor are there registers in a 256 x 256 tile for several and the query heads' epilogue)
+  const bool many = P.K % 128 == 0 && slots > 0 && T > slots && !(FI == 8 && P.q.out);
   const dim3 grid((unsigned)(many ? slots : ((T + 7) / 8) * 8)), blk(BIG_THREADS<FI>);
 #define UVMI_GO(EPI, NORM)                                                                              \
   do {                                                                                                  \
-    if (many) hipLaunchKernelGGL((gemm_big_kernel<DT, EPI, NORM, FI, true>), grid, blk, 0, st, P);      \
+    if (many) hipLaunchKernelGGL((gemm_big_kernel<DT, EPI, NORM, FI, FI != 8 || EPI != 4>), grid, blk, 0, st, P); \
     else hipLaunchKernelGGL((gemm_big_kernel<DT, EPI, NORM, FI, false>), grid, blk, 0, st, P);          \
   } while (0)
   const int norm = a->norm_a ? (P.sums ? 2 : 1) : 0;
@@ -486,13 +555,15 @@ static void launch_big(const uvmi_gemm_args* a, const BigParams& P, int cus, hip
   } else if (a->epilogue == UVMI_GEMM_RESID) { if (norm) UVMI_GO(2, 1); else UVMI_GO(2, 0); }
   else if (a->epilogue == UVMI_GEMM_SWIGLU) { if (norm == 2) UVMI_GO(1, 2); else if (norm) UVMI_GO(1, 1); else UVMI_GO(1, 0); }
   else if (a->epilogue == UVMI_GEMM_SOFTCAP) { if (norm) UVMI_GO(3, 1); else UVMI_GO(3, 0); }
+  else if (P.q.out) { if (norm == 2) UVMI_GO(4, 2); else if (norm) UVMI_GO(4, 1); else UVMI_GO(4, 0); }
   else { if (norm == 2) UVMI_GO(0, 2); else if (norm) UVMI_GO(0, 1); else UVMI_GO(0, 0); }
 #undef UVMI_GO
 }
 
 // Arguments are validated by the caller (uvmi_gemm_tn_ex), which also checks K >= 128.  tile: 256, 128 or (RESID without
-// the pre-norm: uvmi_gemm_resid) 192 rows.  sums: as uvmi_gemm_sums has it, or null.
-void gemm_big_launch(const uvmi_gemm_args* a, int tile, int cus, hipStream_t st, float* sums, int64_t sums_ld) {
+// the pre-norm: uvmi_gemm_resid) 192 rows.  sums: as uvmi_gemm_sums has it, q: STORE of K >= 256 and the
+// extended projection's columns; or null.
+void gemm_big_launch(const uvmi_gemm_args* a, int tile, int cus, hipStream_t st, float* sums, int64_t sums_ld, const QueryPost* q) {
   BigParams P;
   P.a = a->a; P.w = a->w; P.c = a->c; P.r = a->resid;
   P.lda2 = (uint32_t)a->lda * 2; P.ldw2 = (uint32_t)a->ldw * 2; P.ldc = a->ldc; P.ldr = a->ldr;
@@ -500,6 +571,7 @@ void gemm_big_launch(const uvmi_gemm_args* a, int tile, int cus, hipStream_t st,
   const int cols = tile == 192 ? 128 : tile;
   P.tiles_m = (int)((a->M + tile - 1) / tile);
   P.tiles_n = (a->N + cols - 1) / cols;
+  P.q = q ? *q : QueryPost{};
   P.sums = sums; P.sums_ld4 = (uint32_t)sums_ld * 4; P.parts = ((a->norm_a ? a->K : a->N) + 63) / 64;
   P.eps = a->eps; P.ca = a->ca; P.cb = a->cb; P.cap_c = a->cap_c;
   const double bytes_a = (double)a->M * a->K, bytes_w = (double)a->N * a->K;

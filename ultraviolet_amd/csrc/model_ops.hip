@@ -437,26 +437,33 @@ __device__ __forceinline__ float row_sum(const float (&e)[8], int c) {   // of 8
   u = add_sep(u, lane_xor2(u));
   return add_sep(u, lane_xor1(u));
 }
-template <int DT>
+// Q false: the projection's epilogue has the query heads (QueryPost); what is left of them here is the rotation of rows whose position the table does
+// not hold.  18 432 rows 16.1 us with the query heads, 8.5 without (a copy of what is left would take 4), 33 216 rows 24.7 / 11.9; with arguments and arrays
+// asked for one by one and divisions in the quantiser 9.3 and 13.6: it is bound by its chain of trips and, at many rows, by its instructions.
+template <int DT, bool Q>
 __global__ __launch_bounds__(64) void qkv_post_rows_kernel(QkvArgs A) {
   const int lane = threadIdx.x & 63, c = lane & 7;
   const int64_t r0 = (int64_t)blockIdx.x * 8, r1 = r0 + (lane >> 3);
+  // (the arguments that branches further down ask for, with the first ones: each was a trip of its own)
+  asm volatile("" :: "s"(A.k_out), "s"(A.v_out), "s"(A.vhat_out), "s"(A.gate_out), "s"(A.k_cache), "s"(A.v_cache), "s"(A.k_scale), "s"(A.v_scale), "s"(A.scb),
+               "s"(A.scs), "s"(A.ssb), "s"(A.S), "s"(A.ring), "s"(A.rope), "s"(A.rope_tab), "s"(A.rope_n), "s"(A.ve_table), "s"(A.vocab), "s"(A.eps), "s"(A.xsa_eps));
   if (r0 >= A.n) return;
   const bool live = r1 < A.n;
   const int64_t r = live ? r1 : A.n - 1;   // (a lane past the last row computes it again and stores nothing)
   auto rnd = [](float f) { return round_t<DT>(f); };
   const uint16_t* src = (const uint16_t*)A.qkv + r * A.ld + 8 * c;
   // ---- requests that depend on the row index alone
-  const int64_t p = A.pos[r];
-  const int64_t row = A.rows ? A.rows[r] : r;
-  const int64_t lastp = A.last_pos ? A.last_pos[r] : 0;
-  int64_t t = A.has_ve ? A.tok[r] : 0;
+  // (all at once, an array that is not there read as another: behind a branch each, they were waited for one by one)
+  const int64_t p = A.pos[r], rows_r = (A.rows ? A.rows : A.pos)[r], lastp = (A.last_pos ? A.last_pos : A.pos)[r];
+  int64_t t = (A.has_ve ? A.tok : A.pos)[r];
+  const int64_t row = A.rows ? rows_r : r;
   const uint4 kw = *(const uint4*)(src + 512), vw = *(const uint4*)(src + 576);
-  const float glog = A.gate_out ? elem<DT>::ld(A.qkv, r * A.ld + 640 + c) : 0.f;   // head c
-  const float vlog = A.has_ve ? elem<DT>::ld(A.qkv, r * A.ld + 648) : 0.f;
-  uint4 qw[8];
+  const uint16_t gw = ((const uint16_t*)A.qkv)[r * A.ld + 640 + c], tw = ((const uint16_t*)A.qkv)[r * A.ld + 648];   // head c's gate, the value embedding's
+  uint4 qw[Q ? 8 : 1];
+  if constexpr (Q) {
 #pragma unroll
-  for (int h = 0; h < 8; h++) qw[h] = *(const uint4*)(src + 64 * h);
+    for (int h = 0; h < 8; h++) qw[h] = *(const uint4*)(src + 64 * h);
+  }
   // ---- requests that depend on the position and the token
   const bool in_tab = p >= 0 && p < A.rope_n;
   float cs[8], sn[8];   // dim 8 c + j turns by frequency (8 c + j) % 16
@@ -466,6 +473,7 @@ __global__ __launch_bounds__(64) void qkv_post_rows_kernel(QkvArgs A) {
     cs[0] = c0.x; cs[1] = c0.y; cs[2] = c0.z; cs[3] = c0.w; cs[4] = c1.x; cs[5] = c1.y; cs[6] = c1.z; cs[7] = c1.w;
     sn[0] = s0.x; sn[1] = s0.y; sn[2] = s0.z; sn[3] = s0.w; sn[4] = s1.x; sn[5] = s1.y; sn[6] = s1.z; sn[7] = s1.w;
   }
+  const float glog = elem<DT>::ld(&gw, 0), vlog = elem<DT>::ld(&tw, 0);
   if (t < 0) t = 0;
   if (t >= A.vocab) t = A.vocab - 1;
   uint4 ew = uint4{0u, 0u, 0u, 0u};
@@ -564,10 +572,16 @@ __global__ __launch_bounds__(64) void qkv_post_rows_kernel(QkvArgs A) {
       am = fmaxf(am, lane_xor1(am));
       const uint16_t sb = float_to_half_bits(__fdiv_rn(am, 127.0f));
       const float sf = fmaxf(half_bits_to_float(sb), 1e-30f);
+      // 8 quotients by one divisor, rounded as a division rounds: the reciprocal rounded to nearest, the product and its remainder (Markstein).  An
+      // infinite divisor leaves the product as it is.
+      const float r0f = __builtin_amdgcn_rcpf(sf);
+      const bool fin = sf < __builtin_inff();
+      const float d = fin ? sf : 0.f, rc = fin ? fmaf(fmaf(-sf, r0f, 1.0f), r0f, r0f) : 0.f;
       uint32_t b[2] = {0u, 0u};
 #pragma unroll
       for (int j = 0; j < 8; j++) {
-        const float qv = fminf(fmaxf(__builtin_rintf(__fdiv_rn(u ? v[j] : k[j], sf)), -127.0f), 127.0f);
+        const float x = u ? v[j] : k[j], q0 = x * rc;
+        const float qv = fminf(fmaxf(__builtin_rintf(fmaf(fmaf(-q0, d, x), rc, q0)), -127.0f), 127.0f);
         b[j / 4] |= (uint32_t)(uint8_t)(int8_t)(int)qv << (8 * (j % 4));
       }
       if (wr) {
@@ -578,10 +592,21 @@ __global__ __launch_bounds__(64) void qkv_post_rows_kernel(QkvArgs A) {
   }
   // ---- queries
   if (live && A.gate_out) A.gate_out[r * 8 + c] = rnd(2.0f * rnd(1.0f / (1.0f + __expf(-glog))));
+  if constexpr (!Q) {
+    if (A.rope && __any(!in_tab)) {
+      for (int h = 0; h < 8; h++) {
+        float x[8];
+        unpack8<DT>(*(const uint4*)((const uint16_t*)A.q_out + (r * 8 + h) * 64 + 8 * c), x);
+        rotate(x);
+        if (live && !in_tab) st8<DT>(A.q_out, (r * 8 + h) * 64 + 8 * c, x);
+      }
+    }
+    return;
+  }
 #pragma unroll
   for (int h = 0; h < 8; h++) {
     float x[8], ss = 0.f;
-    unpack8<DT>(qw[h], x);
+    unpack8<DT>(qw[Q ? h : 0], x);
 #pragma unroll
     for (int j = 0; j < 8; j++) ss += x[j] * x[j];
     ss += lane_xor1(ss); ss += lane_xor2(ss); ss += lane_xor4(ss);
@@ -780,6 +805,16 @@ bool qkv_post_engine_shape(const uvmi_qkv_post_args* a, const QkvArgs& A) {
   return (a->dtype == UVMI_F16 || a->dtype == UVMI_BF16) && a->q_dtype == a->dtype && a->H == 8 && a->KH == 1 && A.ext &&
          (!a->rope || (a->n_pairs == 16 && A.rope_tab && ((uintptr_t)A.rope_tab % 16) == 0));
 }
+bool qkv_post_rows_ok(const uvmi_qkv_post_args* a) {
+  const uintptr_t wide = (uintptr_t)a->k_out | (uintptr_t)a->v_out | (uintptr_t)a->vhat_out | (a->has_ve ? (uintptr_t)a->ve_table : 0) |
+                         (a->k_cache ? (uintptr_t)a->k_cache | (uintptr_t)a->v_cache : 0) * (a->k_scale ? 2 : 1);
+  return wide % 16 == 0 && (!a->k_cache || (a->scb % 8 == 0 && a->scs % 8 == 0));
+}
+void qkv_post_kv_launch(int dtype, const QkvArgs& A, hipStream_t st) {
+  const dim3 grid((unsigned)((A.n + 7) / 8)), blk(64);
+  if (dtype == UVMI_F16) hipLaunchKernelGGL((qkv_post_rows_kernel<UVMI_F16, false>), grid, blk, 0, st, A);
+  else hipLaunchKernelGGL((qkv_post_rows_kernel<UVMI_BF16, false>), grid, blk, 0, st, A);
+}
 }  // namespace uvmi
 
 extern "C" int uvmi_qkv_post(const uvmi_qkv_post_args* a, void* stream) {
@@ -791,13 +826,10 @@ extern "C" int uvmi_qkv_post(const uvmi_qkv_post_args* a, void* stream) {
   const bool fast = qkv_post_engine_shape(a, A);
   // passes of many rows: 8 per wave, with wide accesses to everything that a row reads or writes.  A wave of 8 rows has the longer chain (2048
   // rows 7.1 us against 4.7, 4096 7.8 against 6.8, 6144 8.9 against 9.1, 8192 9.9 against 11.2)
-  const uintptr_t wide = (uintptr_t)a->k_out | (uintptr_t)a->v_out | (uintptr_t)a->vhat_out | (a->has_ve ? (uintptr_t)a->ve_table : 0) |
-                         (a->k_cache ? (uintptr_t)a->k_cache | (uintptr_t)a->v_cache : 0) * (a->k_scale ? 2 : 1);
-  const bool cache_ok = !a->k_cache || (a->scb % 8 == 0 && a->scs % 8 == 0);
-  if (fast && a->n >= 6144 && wide % 16 == 0 && cache_ok) {
+  if (fast && a->n >= 6144 && qkv_post_rows_ok(a)) {
     const dim3 g8((unsigned)((a->n + 7) / 8)), blk(64);
-    if (a->dtype == UVMI_F16) hipLaunchKernelGGL((qkv_post_rows_kernel<UVMI_F16>), g8, blk, 0, (hipStream_t)stream, A);
-    else hipLaunchKernelGGL((qkv_post_rows_kernel<UVMI_BF16>), g8, blk, 0, (hipStream_t)stream, A);
+    if (a->dtype == UVMI_F16) hipLaunchKernelGGL((qkv_post_rows_kernel<UVMI_F16, true>), g8, blk, 0, (hipStream_t)stream, A);
+    else hipLaunchKernelGGL((qkv_post_rows_kernel<UVMI_BF16, true>), g8, blk, 0, (hipStream_t)stream, A);
   } else if (fast) {
     if (a->dtype == UVMI_F16) hipLaunchKernelGGL((qkv_post_fast_kernel<UVMI_F16>), grid, blk, 0, (hipStream_t)stream, A);
     else hipLaunchKernelGGL((qkv_post_fast_kernel<UVMI_BF16>), grid, blk, 0, (hipStream_t)stream, A);

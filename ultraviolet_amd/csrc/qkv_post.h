@@ -18,9 +18,19 @@ struct QkvArgs {
   int64_t ld; int ext;                 // row pitch of qkv; gate logits read from columns W .. of the row instead of formed from xn
 };
 
+// The query heads' part of it, as an epilogue of the projection takes it: columns 0 .. 511 are 8 heads, whose normed and rotated rows go to out
+// (n, 512); a row whose position the table does not hold is normed only.
+struct QueryPost { void* out; const int64_t* pos; const float* tab; int rope_n; float eps; };   // tab: null without a rotation
+
 // model_ops.hip: uvmi_qkv_post's checks and the kernels' arguments.
 int qkv_post_prepare(const uvmi_qkv_post_args* a, QkvArgs* out);
 // 16-bit rows of 8 query heads on 1 kv head with the gates' logits behind them and a rotation of 16 pairs by table
 bool qkv_post_engine_shape(const uvmi_qkv_post_args* a, const QkvArgs& A);
+// alignment that the rows' keys, values and caches need for 16-byte accesses
+bool qkv_post_rows_ok(const uvmi_qkv_post_args* a);
+// the rest of the post-processing behind such an epilogue (engine shape, qkv_post_rows_ok)
+void qkv_post_kv_launch(int dtype, const QkvArgs& A, hipStream_t st);
+// gemm.hip: the projection with that epilogue (sums: as uvmi_gemm_sums reads them, or null), if its tiles are loaded straight into LDS: whether it was launched
+bool gemm_query_post(const uvmi_gemm_args* a, const QueryPost& q, float* sums, int64_t sums_ld, hipStream_t st);
 
 }  // namespace uvmi

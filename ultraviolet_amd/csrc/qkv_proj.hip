@@ -284,12 +284,17 @@ static void launch_qkv(const uvmi_gemm_args* g, const QkvArgs& A, hipStream_t st
   else hipLaunchKernelGGL((qkv_proj_kernel<DT, FM, R, false>), grid, blk, 0, st, g->a, g->w, lda2, ldw2, (int)g->M, g->K, tiles, g->eps, A);
 }
 
+// The extended projection of the engine's shape, of the rows that the post-processing reads.
+static bool proj_shape(const uvmi_gemm_args* g, const uvmi_qkv_post_args* p, const QkvArgs& A) {
+  if (!g->a || !g->w || !g->c || !uvmi_gemm_tn_supported(g->dtype, g->M, g->N, g->K, g->lda, g->ldw, g->ldc, g->epilogue)) return false;
+  if (g->N != 656 || g->epilogue != UVMI_GEMM_STORE || g->M == 0 || g->M != p->n || g->dtype != p->dtype) return false;
+  if (((uintptr_t)g->a | (uintptr_t)g->w) % 16 != 0 || (g->norm_a && g->eps < 0.f)) return false;
+  return qkv_post_engine_shape(p, A) && A.ld == g->ldc && p->qkv == g->c;
+}
+
 // Rows of the tile that takes the projection with its post-processing in one launch; 0: two launches.
 static int proj_rows(const uvmi_gemm_args* g, const uvmi_qkv_post_args* p, const QkvArgs& A) {
-  if (!uvmi_gemm_tn_supported(g->dtype, g->M, g->N, g->K, g->lda, g->ldw, g->ldc, g->epilogue)) return 0;
-  if (g->N != 656 || g->epilogue != UVMI_GEMM_STORE || g->config != 0 || g->M == 0 || g->M != p->n || g->dtype != p->dtype) return 0;
-  if (((uintptr_t)g->a | (uintptr_t)g->w) % 16 != 0 || (g->norm_a && g->eps < 0.f)) return 0;
-  if (!qkv_post_engine_shape(p, A) || A.ld != g->ldc || p->qkv != g->c) return 0;
+  if (g->config != 0 || !proj_shape(g, p, A)) return 0;
   const uintptr_t a16 = (uintptr_t)A.q_out | (uintptr_t)A.k_out | (uintptr_t)A.v_out | (uintptr_t)A.vhat_out | (uintptr_t)A.gate_out | (A.has_ve ? (uintptr_t)A.ve_table : 0);
   if (a16 % 16 != 0) return 0;
   if (A.k_cache && ((((uintptr_t)A.k_cache | (uintptr_t)A.v_cache) % 8) != 0 || A.scb % 4 != 0 || A.scs % 4 != 0)) return 0;
@@ -311,9 +316,21 @@ extern "C" int uvmi_qkv_proj(const struct uvmi_qkv_proj_args* a, void* stream) {
   if (rc) return rc;
   hipStream_t st = (hipStream_t)stream;
   const uvmi_gemm_args* g = a->gemm;
-  const int rows = g->a && g->w && g->c ? proj_rows(g, a->post, A) : 0;
+  const int rows = g->a && g->w && g->c && !a->sums ? proj_rows(g, a->post, A) : 0;
   if (rows == 0) {
-    rc = uvmi_gemm_tn_ex(g, stream);
+    // Many rows, on tiles loaded straight into LDS: the query heads' part is an epilogue of the projection, so they are not written, read and written
+    // again (two thirds of what the post-processing moves).  Projection and post-processing, us: 3328 rows 18.2 -> 15.8, 5000 21.0 -> 16.5, 9000
+    // 28.5 -> 22.8; with sums 18 432 rows 37.4 -> 33.7, 33 216 61.5 -> 55.9, 65 536 109 -> 87.  Below, on the streaming tiles, which cut heads apart
+    // and split K over waves, the two launches stay: 2600 rows 15.7 against 15.4 on 128 x 128 tiles with it, 1700 13.1 / 15.3.
+    if (proj_shape(g, a->post, A) && qkv_post_rows_ok(a->post)) {
+      if (gemm_query_post(g, QueryPost{A.q_out, A.pos, A.rope ? A.rope_tab : nullptr, A.rope_n, A.eps}, a->sums, a->sums_ld, st)) {
+        qkv_post_kv_launch(g->dtype, A, st);
+        UVMI_CHECK_LAUNCH("uvmi_qkv_proj");
+        return UVMI_OK;
+      }
+    }
+    const struct uvmi_gemm_sums_args s = {g, a->sums, a->sums_ld};
+    rc = a->sums ? uvmi_gemm_sums(&s, stream) : uvmi_gemm_tn_ex(g, stream);
     return rc ? rc : uvmi_qkv_post(a->post, stream);
   }
 #define UVMI_Q(DT) do { if (rows == 16) launch_qkv<DT, 1, 2>(g, A, st); else if (rows == 32) launch_qkv<DT, 2, 2>(g, A, st); else launch_qkv<DT, 4, 1>(g, A, st); } while (0)

@@ -232,11 +232,13 @@ class UVEngine:
 
     def _gemm_sums(self, a: Tensor, w: Tensor, out: Tensor, epilogue: int = STORE, **kw):
         """_gemm of a pass that keeps its hidden's sums of squares (_sums_ok), in what buf h is for other plans."""
-        h = self.buf["h"]
         g = gemm_args(a, w, out, epilogue, **kw)
-        self._op(L.OP_GEMM_SUMS, L.GemmSumsArgs(C.addressof(g), h.data_ptr(), (self.max_tokens + 3) // 4 * 4), (g, a, w, out, h))
+        self._op(L.OP_GEMM_SUMS, L.GemmSumsArgs(C.addressof(g), *self._sums()), (g, a, w, out, self.buf["h"]))
         if self._rec is not None:
             self._rec.field(g, "M", "n")
+
+    def _sums(self) -> tuple[int, int]:
+        return self.buf["h"].data_ptr(), (self.max_tokens + 3) // 4 * 4
 
     def _sums_ok(self, n: int) -> bool:
         """Whether the residual updates of a packed pass sum the squares of the hidden they write for the projections that take its norm.
@@ -259,10 +261,10 @@ class UVEngine:
         self._op(L.OP_NORM, args, (), rows="n", **({} if advance is None else {"advance": "pos"}))
 
     def _qkv_post(self, l: int, tok: Tensor, pos: Tensor, rows: Tensor | None, last_pos: Tensor | None, st: KVState | None,
-                  n: int, write_cache: bool = True, ext: bool = False, gemm=None):
+                  n: int, write_cache: bool = True, ext: bool = False, gemm=None, sums: bool = False):
         """ext: the rows come from the extended projection (buf qkvx), whose last columns are the gates' logits: the
         normalised block input is then not read.  gemm: the argument block of that projection, which has yet to be made: the two
-        are one operation."""
+        are one operation; sums: with the rows' norm from the sums that the residual update before it left (_gemm_sums)."""
         cfg, b, W = self.cfg, self.buf, self.w.layers[l]
         glob = cfg.is_global(l)
         a = L.QkvPostArgs()
@@ -308,7 +310,7 @@ class UVEngine:
         if gemm is None:
             self._op(L.OP_QKV_POST, a, keep, **per_call)
         else:
-            self._op(L.OP_QKV_PROJ, L.QkvProjArgs(C.addressof(gemm), C.addressof(a)), (gemm, a, keep))
+            self._op(L.OP_QKV_PROJ, L.QkvProjArgs(C.addressof(gemm), C.addressof(a), *(self._sums() if sums else (None, 0))), (gemm, a, keep, b["h"]))
             if self._rec is not None:
                 self._rec.field(gemm, "M", "n")
                 for field, name in per_call.items():
@@ -632,13 +634,11 @@ class UVEngine:
         project = self._gemm_sums if sums else self._gemm
         for l, W in enumerate(self.w.layers):
             gemm = None
-            if sums and l > 0:
-                self._gemm_sums(x, W["wqkv_ext"], b["qkvx"][:n], norm_eps=self.eps)
-            elif n <= self.fold_qkv_rows and last_pos is not None:   # (decode rows alone: the projection of the fused attention's plans, to the same bits)
+            if n <= self.fold_qkv_rows and last_pos is not None:   # (decode rows alone: the projection of the fused attention's plans, to the same bits)
                 gemm = gemm_args(b["xn" if l == 0 else "x"][:n], W["wqkv_ext"], b["qkvx"][:n], norm_eps=None if l == 0 else self.eps, config=gc)
             else:
                 self._project_qkv(l, n, n <= self.fold_qkv_rows, config=gc)
-            self._qkv_post(l, tok, pos, rows, last_pos, st, n, ext=True, gemm=gemm)
+            self._qkv_post(l, tok, pos, rows, last_pos, st, n, ext=True, gemm=gemm, sums=sums and l > 0)
             if oproj and not sums:   # (the attention's launch, or one behind it)
                 attn(l, b["q"][:n], gemm_args(zg, W["wo"], x, RESID, resid=x, ca=W["resid_attn"], cb=W["post_attn"], config=gc))
             else:
