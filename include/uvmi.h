@@ -271,6 +271,10 @@ int uvmi_gemm_resid_tile(const uvmi_gemm_args* a);
  * sums 16-byte aligned, ld a multiple of 4 and at least M. */
 struct uvmi_gemm_sums_args { const uvmi_gemm_args* gemm; float* sums; int64_t ld; };
 int uvmi_gemm_sums(const struct uvmi_gemm_sums_args* a, void* stream);
+/* The logits (SOFTCAP) of rows rows[0 .. M-1] of the a_rows rows at gemm->a (rows NULL: of rows 0 .. M-1); the launch also counts the n_advance
+ * positions at advance (or NULL) up by one.  Rows out of range are taken as the nearest in range. */
+struct uvmi_head_args { const uvmi_gemm_args* gemm; const int64_t* rows; int64_t a_rows; int64_t* advance; int64_t n_advance; };
+int uvmi_head(const struct uvmi_head_args* a, void* stream);
 
 /* ------------------------------------------------------------------------------------------------------------
  * Packed (cu_seqlens) causal self-attention with an optional sliding window over unquantized K/V: the attention of

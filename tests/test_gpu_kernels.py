@@ -1332,6 +1332,38 @@ def test_rows_squares_summed_where_they_are_written(dtype, M, d, config):
         assert torch.equal(out, want)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N", [(1, 4096), (37, 4096), (129, 4096), (400, 32768), (2100, 32768)])
+@pytest.mark.parametrize("gather", [False, True])
+def test_head_of_some_rows_with_the_positions_counted_up(dtype, M, N, gather):
+    """uvmi_head: the bits of the softcapped product of the rows that it names (out of range: the nearest), or of all, on one 128-row tile, several and 256-row
+    ones, one and several to a workgroup; positions go up by one, whatever their number, and nothing beside them."""
+    import ctypes as C
+    from ultraviolet_amd import _lib as L
+    from ultraviolet_amd.kernels.gemm import SOFTCAP, gemm_args, gemm_tn
+    g = torch.Generator(device="cuda").manual_seed(M)
+    n = 3 * M + 5 if gather else M
+    x, w = (torch.randn(s, 640, device="cuda", generator=g).to(dtype) for s in (n, N))
+    kw = dict(norm_eps=1e-6, ca=23.0, cb=5.0, cap_c=7.5)
+    rows = torch.randint(0, n, (M,), device="cuda", generator=g)
+    rows[-1] = n + 3
+    pos = torch.arange(1003, device="cuda")
+    out = torch.empty(M, N, device="cuda")
+    ga = gemm_args(x[:M], w, out, SOFTCAP, **kw)
+    h = L.HeadArgs(C.addressof(ga), rows.data_ptr() if gather else None, n, pos.data_ptr(), 1001)
+    L.check(L.lib().uvmi_head(C.byref(h), L.stream_ptr(x)), "uvmi_head")
+    assert torch.equal(out, gemm_tn(x[rows.clamp(max=n - 1)].contiguous() if gather else x, w, epilogue=SOFTCAP, **kw))
+    assert torch.equal(pos, torch.arange(1003, device="cuda") + (torch.arange(1003, device="cuda") < 1001))
+    if M > 1:   # another epilogue, a hidden too large, positions behind no rows: refused
+        for bad in (dict(epilogue=0), dict(a_rows=1 << 21), dict(M=0)):
+            gb = gemm_args(x[:M], w, out, SOFTCAP, **kw)
+            hb = L.HeadArgs(C.addressof(gb), rows.data_ptr(), bad.get("a_rows", n), pos.data_ptr(), 1001)
+            for k, v in bad.items():
+                if k != "a_rows":
+                    setattr(gb, k, v)
+            assert L.lib().uvmi_head(C.byref(hb), L.stream_ptr(x)) < 0
+
+
 @pytest.mark.parametrize("change", [dict(config=3), dict(M=64), dict(ld=8), dict(ld=131), dict(epilogue=0), dict(norm_a=1), dict(K=2048)])
 def test_sums_of_squares_are_refused_elsewhere(change):
     """Other forms of the GEMM, few rows, pitches that do not hold the rows, epilogues that neither write nor read sums: refused, nothing launched."""

@@ -157,6 +157,10 @@ class GemmSumsArgs(C.Structure):   # struct uvmi_gemm_sums_args: address of a Ge
     _fields_ = [("gemm", C.c_void_p), ("sums", C.c_void_p), ("ld", C.c_int64)]
 
 
+class HeadArgs(C.Structure):   # struct uvmi_head_args
+    _fields_ = [("gemm", C.c_void_p), ("rows", C.c_void_p), ("a_rows", C.c_int64), ("advance", C.c_void_p), ("n_advance", C.c_int64)]
+
+
 OP_GEMM, OP_DECODE_ATTN, OP_QKV_POST, OP_PREFILL_ATTN, OP_NORM, OP_QKV_PROJ, OP_PREFILL_ATTN_O, OP_GEMM_RESID, OP_GEMM_SUMS = range(9)   # UVMI_OP_*
 
 _lib = None
@@ -226,6 +230,7 @@ def lib() -> C.CDLL:
         L.uvmi_rope_table.argtypes = [C.c_void_p, C.c_int, C.c_int64, C.c_int, C.c_void_p, C.c_void_p]
         L.uvmi_gemm_tn_supported.argtypes = [C.c_int, C.c_int64, C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_int64, C.c_int]
         L.uvmi_gemm_tn_ex.argtypes = [C.POINTER(GemmArgs), C.c_void_p]
+        L.uvmi_head.argtypes = [C.POINTER(HeadArgs), C.c_void_p]
         L.uvmi_gemm_sums.argtypes = [C.POINTER(GemmSumsArgs), C.c_void_p]
         L.uvmi_gemm_resid.argtypes = [C.POINTER(GemmArgs), C.c_void_p]
         L.uvmi_gemm_resid_tile.argtypes = [C.POINTER(GemmArgs)]
@@ -287,4 +292,4 @@ EXPORTS = ["uvmi_version", "uvmi_last_error", "uvmi_device_cus", "uvmi_quantize_
            "uvmi_default_splits", "uvmi_decode_attn_splits", "uvmi_decode_attn_path", "uvmi_attn_oproj_rows", "uvmi_decode_attn_noalloc", "uvmi_decode_attn_probe", "uvmi_prefill_attn", "uvmi_prefill_attn_o", "uvmi_prefill_attn_workspace_bytes",
            "uvmi_prefill_attn_path", "uvmi_fused_sample", "uvmi_philox4x32_10",
            "uvmi_embed_norm", "uvmi_add_norm", "uvmi_qkv_post", "uvmi_qkv_proj", "uvmi_attn_post", "uvmi_swiglu", "uvmi_swiglu_norm",
-           "uvmi_prefill_attn_bwd", "uvmi_prefill_attn_bwd_workspace_bytes", "uvmi_sched_compact", "uvmi_sched_commit", "uvmi_sched_commit_dense", "uvmi_sched_admit", "uvmi_sched_expand", "uvmi_sched_harvest", "uvmi_sched_plan_admit", "uvmi_sched_step_plan", "uvmi_run_ops", "uvmi_prompt_tables", "uvmi_rope_table", "uvmi_gemm_tn_supported", "uvmi_gemm_tn", "uvmi_gemm_tn_ex", "uvmi_gemm_tn_path", "uvmi_gemm_resid", "uvmi_gemm_resid_tile", "uvmi_gemm_sums"]
+           "uvmi_prefill_attn_bwd", "uvmi_prefill_attn_bwd_workspace_bytes", "uvmi_sched_compact", "uvmi_sched_commit", "uvmi_sched_commit_dense", "uvmi_sched_admit", "uvmi_sched_expand", "uvmi_sched_harvest", "uvmi_sched_plan_admit", "uvmi_sched_step_plan", "uvmi_run_ops", "uvmi_prompt_tables", "uvmi_rope_table", "uvmi_gemm_tn_supported", "uvmi_gemm_tn", "uvmi_gemm_tn_ex", "uvmi_gemm_tn_path", "uvmi_gemm_resid", "uvmi_gemm_resid_tile", "uvmi_gemm_sums", "uvmi_head"]

@@ -8,7 +8,7 @@ using namespace uvmi;
 
 namespace uvmi {
 void gemm_tile_launch(const uvmi_gemm_args* a, hipStream_t st);                     // gemm_tile.hip
-void gemm_big_launch(const uvmi_gemm_args* a, int tile, int cus, hipStream_t st, float* sums = nullptr, int64_t sums_ld = 0, const QueryPost* q = nullptr);   // gemm_big.hip; tile: 128, 256, 192 (x 128: RESID)
+void gemm_big_launch(const uvmi_gemm_args* a, int tile, int cus, hipStream_t st, float* sums = nullptr, int64_t sums_ld = 0, const QueryPost* q = nullptr, const HeadRows* h = nullptr);   // gemm_big.hip; tile: 128, 256, 192 (x 128: RESID)
 int gemm_stream_form(const uvmi_gemm_args* a, int cus);                             // gemm_stream.hip
 void gemm_stream_tile(int form, int* rows, int* cols);
 void gemm_stream_launch(const uvmi_gemm_args* a, int form, int cus, hipStream_t st);
@@ -172,10 +172,11 @@ extern "C" int uvmi_gemm_resid_tile(const uvmi_gemm_args* a) {
 }
 
 extern "C" int uvmi_gemm_resid(const uvmi_gemm_args* a, void* stream) {
+  if (a && a->M < BIG_MIN_ROWS) return uvmi_gemm_tn_ex(a, stream);
   const int rc = check_gemm(a);
   if (rc) return rc;
   const int cus = compute_units();
-  if (a->M == 0 || !resid_192(a, cus)) return uvmi_gemm_tn_ex(a, stream);
+  if (!resid_192(a, cus)) return uvmi_gemm_tn_ex(a, stream);
   gemm_big_launch(a, 192, cus, (hipStream_t)stream);
   UVMI_CHECK_LAUNCH("uvmi_gemm_resid");
   return UVMI_OK;
@@ -217,4 +218,22 @@ bool uvmi::gemm_query_post(const uvmi_gemm_args* a, const QueryPost& q, float* s
   if (a->config == 0 && p.form == 256 && t256 > cus && !big_tiles_pay(a, t128, t256, cus, 20)) p.form = 128;
   gemm_big_launch(a, p.form, cus, st, sums, sums_ld, &q);
   return true;
+}
+
+extern "C" int uvmi_head(const struct uvmi_head_args* s, void* stream) {
+  UVMI_REQUIRE(s && s->gemm, UVMI_EINVAL, "uvmi_head: null pointer");
+  const uvmi_gemm_args* a = s->gemm;
+  const int rc = check_gemm(a);
+  if (rc) return rc;
+  UVMI_REQUIRE(a->epilogue == UVMI_GEMM_SOFTCAP, UVMI_EINVAL, "uvmi_head: the SOFTCAP epilogue only");
+  UVMI_REQUIRE(!s->rows || (s->a_rows > 0 && s->a_rows <= (1 << 20) && (s->a_rows + 64) * a->lda * 2 < (1LL << 30)), UVMI_EUNSUPPORTED,
+               "uvmi_head: rows of a hidden of %lld rows with a pitch of %lld", (long long)s->a_rows, (long long)a->lda);
+  UVMI_REQUIRE(!s->advance || s->n_advance >= 0, UVMI_EINVAL, "uvmi_head: negative count");
+  UVMI_REQUIRE(a->M > 0 || !s->advance || s->n_advance == 0, UVMI_EINVAL, "uvmi_head: positions to count up behind no rows");
+  if (a->M == 0) return UVMI_OK;
+  const int cus = compute_units();
+  const HeadRows h = {s->rows, (int)s->a_rows, s->advance, s->n_advance};
+  gemm_big_launch(a, gemm_path(a, cus).form, cus, (hipStream_t)stream, nullptr, 0, nullptr, &h);
+  UVMI_CHECK_LAUNCH("uvmi_head");
+  return UVMI_OK;
 }

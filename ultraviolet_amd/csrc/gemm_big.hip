@@ -57,6 +57,7 @@ struct BigParams {
   float eps, ca, cb, cap_c;
   float* sums; uint32_t sums_ld4; int parts;   // NORM 2: read; EPI 2 (or null): written.  parts x sums_ld4 bytes
   QueryPost q;                                 // EPI 4
+  HeadRows h;                                  // EPI 3
 };
 constexpr int SUM_PARTS = 16;
 
@@ -92,7 +93,8 @@ __device__ __forceinline__ int fresh_lane() {
 }
 
 // EPI 0: C = A W^T (M, N).  EPI 1: W rows are [gate 16 | up 16] slabs; C = silu(gate) * up, (M, N / 2).
-// EPI 2: C = ca * R + cb * (A W^T).  EPI 3: C fp32 = ca * sigmoid((x + cb) / cap_c) of the rounded product x.  NORM: A stands
+// EPI 2: C = ca * R + cb * (A W^T).  EPI 3: C fp32 = ca * sigmoid((x + cb) / cap_c) of the rounded product x, of rows of A that
+// h.rows names (or all), with h.advance counted up behind it.  NORM: A stands
 // for its RMS-normalised rows, whose squares are summed here (1) or were by the launches that wrote them (2: a number per row and 64
 // columns, which an EPI 2 launch leaves).
 // EPI 4: EPI 0 whose columns 0 .. 511, a wave's 64 of them a query head, are normed, rotated (QK-norm and RoPE, with the roundings of
@@ -145,7 +147,9 @@ void gemm_big_kernel(BigParams P) {
 #pragma unroll
     for (int i = 0; i < LA; i++) {
       const int rl = 8 * (LA * wave + i) + (ln >> 3);   // row inside the tile
-      offA[i] = (uint32_t)min(m0 + rl, P.M - 1) * P.lda2 + 16 * ((ln & 7) ^ ((rl >> 1) & 7));
+      int m = min(m0 + rl, P.M - 1);
+      if (EPI == 3 && P.h.rows) m = (int)min(max(P.h.rows[m], (int64_t)0), (int64_t)P.h.a_rows - 1);
+      offA[i] = (uint32_t)m * P.lda2 + 16 * ((ln & 7) ^ ((rl >> 1) & 7));
     }
 #pragma unroll
     for (int i = 0; i < 4; i++) {
@@ -155,7 +159,7 @@ void gemm_big_kernel(BigParams P) {
   };
   offsets();
   // (buffer loads: 32-bit offsets and the slab as a scalar, where global ones keep eight 64-bit addresses)
-  const __amdgpu_buffer_rsrc_t rA = __builtin_amdgcn_make_buffer_rsrc((void*)P.a, 0, (int)((uint32_t)(P.M - 1) * P.lda2 + (uint32_t)P.K * 2), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rA = __builtin_amdgcn_make_buffer_rsrc((void*)P.a, 0, (int)((uint32_t)((EPI == 3 && P.h.rows ? P.h.a_rows : P.M) - 1) * P.lda2 + (uint32_t)P.K * 2), 0x00020000);
   const __amdgpu_buffer_rsrc_t rW = __builtin_amdgcn_make_buffer_rsrc((void*)P.w, 0, (int)((uint32_t)(P.N - 1) * P.ldw2 + (uint32_t)P.K * 2), 0x00020000);
   auto issue = [&](unsigned char* sa, unsigned char* sb, int kt) {
 #pragma unroll
@@ -534,6 +538,8 @@ void gemm_big_kernel(BigParams P) {
     L += step;
     clear();
   }
+  if (EPI == 3 && P.h.advance && blockIdx.x == 0)
+    for (int64_t i = 64 * wave + fresh_lane(); i < P.h.n_advance; i += BIG_THREADS<FI>) P.h.advance[i] += 1;
 }
 
 template <int DT, int FI>
@@ -562,8 +568,8 @@ static void launch_big(const uvmi_gemm_args* a, const BigParams& P, int cus, hip
 
 // Arguments are validated by the caller (uvmi_gemm_tn_ex), which also checks K >= 128.  tile: 256, 128 or (RESID without
 // the pre-norm: uvmi_gemm_resid) 192 rows.  sums: as uvmi_gemm_sums has it, q: STORE of K >= 256 and the
-// extended projection's columns; or null.
-void gemm_big_launch(const uvmi_gemm_args* a, int tile, int cus, hipStream_t st, float* sums, int64_t sums_ld, const QueryPost* q) {
+// extended projection's columns, h: SOFTCAP; or null.
+void gemm_big_launch(const uvmi_gemm_args* a, int tile, int cus, hipStream_t st, float* sums, int64_t sums_ld, const QueryPost* q, const HeadRows* h) {
   BigParams P;
   P.a = a->a; P.w = a->w; P.c = a->c; P.r = a->resid;
   P.lda2 = (uint32_t)a->lda * 2; P.ldw2 = (uint32_t)a->ldw * 2; P.ldc = a->ldc; P.ldr = a->ldr;
@@ -572,6 +578,7 @@ void gemm_big_launch(const uvmi_gemm_args* a, int tile, int cus, hipStream_t st,
   P.tiles_m = (int)((a->M + tile - 1) / tile);
   P.tiles_n = (a->N + cols - 1) / cols;
   P.q = q ? *q : QueryPost{};
+  P.h = h ? *h : HeadRows{};
   P.sums = sums; P.sums_ld4 = (uint32_t)sums_ld * 4; P.parts = ((a->norm_a ? a->K : a->N) + 63) / 64;
   P.eps = a->eps; P.ca = a->ca; P.cb = a->cb; P.cap_c = a->cap_c;
   const double bytes_a = (double)a->M * a->K, bytes_w = (double)a->N * a->K;

@@ -1,4 +1,5 @@
-// The post-processing of the QKV projection as the kernels take it: model_ops.hip, and qkv_proj.hip, where it is part of the projection's launch.
+// The post-processing of the QKV projection as the kernels take it: model_ops.hip, and qkv_proj.hip, where it is part of the projection's launch; and what
+// else a launch of gemm_big.hip does beside its product.
 #pragma once
 #include "common.h"
 
@@ -21,6 +22,9 @@ struct QkvArgs {
 // The query heads' part of it, as an epilogue of the projection takes it: columns 0 .. 511 are 8 heads, whose normed and rotated rows go to out
 // (n, 512); a row whose position the table does not hold is normed only.
 struct QueryPost { void* out; const int64_t* pos; const float* tab; int rope_n; float eps; };   // tab: null without a rotation
+
+// The head's rows of the hidden (null: all of them) and the positions that its launch counts up (or null): uvmi_head.
+struct HeadRows { const int64_t* rows; int a_rows; int64_t* advance; int64_t n_advance; };
 
 // model_ops.hip: uvmi_qkv_post's checks and the kernels' arguments.
 int qkv_post_prepare(const uvmi_qkv_post_args* a, QkvArgs* out);

@@ -766,17 +766,47 @@ class UVEngine:
         elementwise passes over the (n, V) output took 130 us at 512 rows)."""
         a, bb, c = self.cfg.softcap
         W = self.w.embed
-        if hidden.dtype in (torch.bfloat16, torch.float16) and hidden.dim() == 2 and hidden.size(0) > 0 and hidden.dtype == W.dtype and W.size(1) >= 128 and W.size(0) % 16 == 0:
+        if hidden.dim() == 2 and hidden.size(0) > 0 and self._own_logits_ok(hidden.dtype):
             hidden = hidden.contiguous()
             if gemm_supported(hidden, W, SOFTCAP):
                 return gemm_tn(hidden, W, epilogue=SOFTCAP, ca=a, cb=bb, cap_c=c)
         return a * torch.sigmoid((self.head(hidden).float() + bb) / c)
+
+    def _own_logits_ok(self, dtype: torch.dtype) -> bool:
+        W = self.w.embed
+        return dtype in (torch.bfloat16, torch.float16) and dtype == W.dtype and W.size(1) >= 128 and W.size(0) % 16 == 0
+
+    def _raw_logits_ok(self) -> bool:
+        W = self.w.embed
+        return self._own_logits_ok(self.dtype) and W.stride(1) == 1 and W.stride(0) % 8 == 0 and W.data_ptr() % 16 == 0 and W.size(1) % 64 == 0
+
+    def _raw_logits(self, hidden: Tensor, rows: Tensor | None = None, advance: Tensor | None = None) -> Tensor:
+        """logits() of rows `rows` (all) of what a trunk left un-normalised in buf x: the final norm is the row scale of the product, the rows are
+        gathered by the GEMM's loads and positions `advance` counted up by its launch.  (One launch less a decode step, two
+        less a prefill: a step of 37 rows 245.7 -> 242.1 us, of 512 413.5 -> 409.9, a prefill of 93 tokens, which waits for the host, 245 -> 241.)"""
+        ca, cb, c = self.cfg.softcap
+        W = self.w.embed
+        n = hidden.size(0) if rows is None else rows.numel()
+        out = torch.empty(n, W.size(0), dtype=torch.float32, device=hidden.device)
+        g = gemm_args(hidden[:n], W, out, SOFTCAP, norm_eps=self.eps, ca=ca, cb=cb, cap_c=c)
+        h = L.HeadArgs(C.addressof(g), None if rows is None else rows.data_ptr(), hidden.size(0), None if advance is None else advance.data_ptr(),
+                       0 if advance is None else advance.numel())
+        L.check(L.lib().uvmi_head(C.byref(h), L.stream_ptr(out)), "uvmi_head")
+        return out
 
     # ------------------------------------------------------------------------------------------------ decode
     @torch.no_grad()
     def decode_step(self, tok: Tensor, st: KVState, num_splits: dict | None = None, fuse: bool = True) -> Tensor:
         """One token for all B rows at per-row st.pos (reference: decode_step_fast, fast_decode.py:272-334): append K/V
         at pos first, attend lo..pos, then st.pos += 1.  Returns the final normed hidden (B, d)."""
+        return self._decode(tok, st, num_splits, fuse, False)
+
+    @torch.no_grad()
+    def decode_logits(self, tok: Tensor, st: KVState, num_splits: dict | None = None) -> Tensor:
+        """logits(decode_step(tok, st, num_splits)); where the step's plan leaves the hidden as it is, the head takes the final norm."""
+        return self._decode(tok, st, num_splits, True, True)
+
+    def _decode(self, tok: Tensor, st: KVState, num_splits: dict | None, fuse: bool, head: bool) -> Tensor:
         cfg = self.cfg
         B = tok.numel()
         pos, starts = st.pos, st.starts
@@ -790,12 +820,16 @@ class UVEngine:
                 # (a recorded list takes addresses only, so what its launches assume of the arrays is checked on every call)
                 assert all(t.dtype == torch.int64 and t.is_contiguous() and t.numel() >= B for t in (tok, pos, starts))
                 whole = B == pos.numel()     # (a step of fewer rows than the state has still moves every position)
+                if head and 0 < B <= 1 << 16 and self._raw_logits_ok():
+                    h = self._planned("decode-raw", st, kind, B, dict(n=B, tok=tok.data_ptr(), pos=pos.data_ptr(), starts=starts.data_ptr()),
+                                      lambda: self._trunk(tok, pos, B, None, st=st, fused_attn=fused, final_norm=False))
+                    return self._raw_logits(h, advance=pos)
                 h = self._planned("decode" if whole else "decode-part", st, kind, B,
                                   dict(n=B, tok=tok.data_ptr(), pos=pos.data_ptr(), starts=starts.data_ptr()),
                                   lambda: self._trunk(tok, pos, B, None, st=st, fused_attn=fused, advance=whole))
                 if not whole:
                     st.pos.add_(1)
-                return h
+                return self.logits(h) if head else h
 
         def attn(l, q):
             key = "global" if cfg.is_global(l) else "local"
@@ -808,7 +842,7 @@ class UVEngine:
 
         h = self._trunk(tok, pos, B, attn, st=st, fused_attn=fused)
         st.pos.add_(1)
-        return h
+        return self.logits(h) if head else h
 
     # ------------------------------------------------------------------------------------------------ prefill
     def _staging(self, n: int):
@@ -951,17 +985,30 @@ class UVEngine:
         return self._prefill(self._pack(prompts, rows, st.max_len, left_pad, st), st)
 
     @torch.no_grad()
+    def prefill_logits(self, prompts: list[list[int]], rows: list[int], st: KVState, left_pad: bool = True) -> Tensor:
+        """logits(prefill(prompts, rows, st, left_pad)), without the launches that gather and norm the prompts' last rows."""
+        return self._prefill(self._pack(prompts, rows, st.max_len, left_pad, st), st, True)
+
+    @torch.no_grad()
     def prefill_matrix(self, idx: Tensor, lens, rows, st: KVState, check: Tensor | None = None):
         """prefill(left_pad=True) of the prompts that stand right-aligned in idx (n, T), an int64 matrix on the engine's device: the
         last lens[a] (host) tokens of row a.  The token ids never visit the host.  check: n int64 of the device that have to be
         zero; also returns a function that gives them without waiting for the pass.  A prompt whose entry is not zero leaves
         the state as it is - cache row, pos and starts -, so the caller may raise when it sees that."""
+        return self._prefill_matrix(idx, lens, rows, st, check, False)
+
+    @torch.no_grad()
+    def prefill_matrix_logits(self, idx: Tensor, lens, rows, st: KVState, check: Tensor | None = None):
+        """prefill_matrix with the logits of the prompts' last rows in place of their hidden."""
+        return self._prefill_matrix(idx, lens, rows, st, check, True)
+
+    def _prefill_matrix(self, idx: Tensor, lens, rows, st: KVState, check: Tensor | None, head: bool):
         assert idx.dtype == torch.int64 and idx.is_contiguous() and idx.size(0) == len(lens) and idx.size(1) >= int(lens.max())
         pk = self._pack(None, rows, st.max_len, True, st, idx, lens, check, check_zero=check is not None)
-        h = self._prefill(pk, st)
+        h = self._prefill(pk, st, head)
         return h if check is None else (h, pk["check"])
 
-    def _prefill(self, pk: dict, st: KVState) -> Tensor:
+    def _prefill(self, pk: dict, st: KVState, head: bool = False) -> Tensor:
         N = pk["N"]
 
         def attn(l, q, gemm=None):
@@ -974,7 +1021,10 @@ class UVEngine:
                                                                 cu=cu.data_ptr(), n_seg=cu.numel() - 1), run)
         else:
             h = run()
-        return self._normed(h.index_select(0, pk["last_idx"]))   # (the norm of the prompts' last rows only)
+        if head and self.hidden_is_raw and pk["last_idx"].numel() <= 1 << 16 and self._raw_logits_ok():
+            return self._raw_logits(h, rows=pk["last_idx"])
+        h = self._normed(h.index_select(0, pk["last_idx"]))   # (the norm of the prompts' last rows only)
+        return self.logits(h) if head else h
 
     # ------------------------------------------------------------------------------------------------ generation
     @torch.no_grad()

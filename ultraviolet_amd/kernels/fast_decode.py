@@ -141,13 +141,12 @@ def prefill_fast(self, idx: Tensor, starts: Tensor, st: KVState, rows: Tensor | 
         # which the pass's first launch leaves in host memory, is checked behind it (where it is not zero, that launch keeps the pass
         # away from the state).  (Waiting for it first leaves the GPU idle
         # for 90 us of a 93-token prefill's 460.)
-        h, seen = eng.prefill_matrix(idx, np.array([T]), rows_l, st, check=starts)
-        lg = eng.logits(h)
+        lg, seen = eng.prefill_matrix_logits(idx, np.array([T]), rows_l, st, check=starts)
         assert int(seen()[0]) == 0, longest
     else:
         lens = T - starts.cpu().numpy().astype(np.int64)     # (the only thing the host needs from the device)
         assert lens.max() == T, longest
-        lg = eng.logits(eng.prefill_matrix(idx, lens, rows_l, st))
+        lg = eng.prefill_matrix_logits(idx, lens, rows_l, st)
     if hasattr(st, "host_pos"):
         st.host_pos[np.asarray(rows_l)] = T
     return lg
@@ -164,10 +163,10 @@ def prefill_packed_host(self, prompts, rows, st: KVState, dev=None) -> Tensor:
     rows_l = [int(r) for r in rows]
     T = max(len(p) for p in prompts)
     assert T <= st.max_len
-    h = eng.prefill([list(p) for p in prompts], rows_l, st, left_pad=True)
+    lg = eng.prefill_logits([list(p) for p in prompts], rows_l, st, left_pad=True)
     if hasattr(st, "host_pos"):
         st.host_pos[np.asarray(rows_l)] = T
-    return eng.logits(h)
+    return lg
 
 
 @torch.no_grad()
@@ -179,10 +178,10 @@ def decode_step_fast(self, tok: Tensor, st: KVState, g_len: int = 0, skip_attn: 
     assert not skip_attn, "skip_attn is a profiling switch of the reference and is not supported"
     assert backend in ("auto", "hip"), f"backend {backend!r}: this library has one backend"
     eng = _engine(self, full_check=False)
-    h = eng.decode_step(tok, st, num_splits)
+    out = (eng.decode_step if return_hidden else eng.decode_logits)(tok, st, num_splits)
     if hasattr(st, "host_pos"):
         st.host_pos += 1
-    return h if return_hidden else eng.logits(h)
+    return out
 
 
 def patch_model(model, kv_dtype: str | None = "fp16", num_splits: dict | None = None, backend: str = "auto",
