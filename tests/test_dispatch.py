@@ -81,6 +81,24 @@ def test_splits_of_a_call_that_names_none(monkeypatch, q_dtype, kv_dtype):
                     assert s * n <= 256 and ctx // s >= 128
 
 
+@pytest.mark.parametrize("V,d,n,of", [(32768, 640, 1, 1), (32768, 640, 65536, 1 << 20), (32768, 640, 65537, 65537), (32768, 640, 64, (1 << 29) // 640 - 64),
+                                      (32768, 640, 64, (1 << 20) + 1), (524288, 1024, 8, 8), (524224, 1024, 8, 8), (524208, 1024, 8, 8), (4096, 8192, 65536, 65536),
+                                      (4096, 8192, 65472, 65472), (4096, 8192, 65471, 65471), (4096, 8256, 8, 8), (4096, 96, 8, 8), (4104, 640, 8, 8), (4096, 64, 8, 8)])
+def test_logits_of_raw_hidden_are_asked_for_where_the_library_takes_them(V, d, n, of):
+    # (beyond, the logits come from the normed hidden as they did: a vocabulary or hidden past 32-bit offsets is no error)
+    from types import SimpleNamespace
+
+    from ultraviolet_amd import _lib as L
+    from ultraviolet_amd.engine.model import UVEngine
+    from ultraviolet_amd.kernels.gemm import SOFTCAP
+    W = torch.empty(V, d, dtype=torch.bfloat16, device="meta")
+    e = SimpleNamespace(w=SimpleNamespace(embed=W), dtype=torch.bfloat16)
+    e._own_logits_ok = lambda dtype: UVEngine._own_logits_ok(e, dtype)
+    lib = lambda rows: L.lib().uvmi_gemm_tn_supported(L.dtype_code(W.dtype), rows, V, d, d, d, V, SOFTCAP) == 1
+    takes = lib(n) and d >= 128 and (of == n or (of <= 1 << 20 and (of + 64) * d * 2 < 1 << 30))   # (uvmi_head's line for a gathered hidden)
+    assert UVEngine._raw_logits_ok(e, n, of) == takes
+
+
 def test_guard_of_recorded_passes_sees_what_changes():
     """Everything that launches took an address or a number from: a tensor replaced, moved under its object, a scalar, an entry that
     comes or goes - in the weights and in the state; by torch's comparison of addresses and by the list of them."""

@@ -776,9 +776,13 @@ class UVEngine:
         W = self.w.embed
         return dtype in (torch.bfloat16, torch.float16) and dtype == W.dtype and W.size(1) >= 128 and W.size(0) % 16 == 0
 
-    def _raw_logits_ok(self) -> bool:
+    def _raw_logits_ok(self, n: int, of: int | None = None) -> bool:
+        """Whether _raw_logits takes n rows, of a hidden of `of` (n): what uvmi_head does, whose offsets into hidden and embedding are 32-bit."""
         W = self.w.embed
-        return self._own_logits_ok(self.dtype) and W.stride(1) == 1 and W.stride(0) % 8 == 0 and W.data_ptr() % 16 == 0 and W.size(1) % 64 == 0
+        of = n if of is None else of
+        V, d = W.shape
+        return (0 < n <= 1 << 16 and of <= 1 << 20 and self._own_logits_ok(self.dtype) and W.stride(1) == 1 and W.stride(0) % 8 == 0 and W.data_ptr() % 16 == 0
+                and d % 64 == 0 and d <= 8192 and (V + 64) * W.stride(0) < 1 << 29 and (max(n, of) + 64) * d < 1 << 29)
 
     def _raw_logits(self, hidden: Tensor, rows: Tensor | None = None, advance: Tensor | None = None) -> Tensor:
         """logits() of rows `rows` (all) of what a trunk left un-normalised in buf x: the final norm is the row scale of the product, the rows are
@@ -820,7 +824,7 @@ class UVEngine:
                 # (a recorded list takes addresses only, so what its launches assume of the arrays is checked on every call)
                 assert all(t.dtype == torch.int64 and t.is_contiguous() and t.numel() >= B for t in (tok, pos, starts))
                 whole = B == pos.numel()     # (a step of fewer rows than the state has still moves every position)
-                if head and 0 < B <= 1 << 16 and self._raw_logits_ok():
+                if head and self._raw_logits_ok(B):
                     h = self._planned("decode-raw", st, kind, B, dict(n=B, tok=tok.data_ptr(), pos=pos.data_ptr(), starts=starts.data_ptr()),
                                       lambda: self._trunk(tok, pos, B, None, st=st, fused_attn=fused, final_norm=False))
                     return self._raw_logits(h, advance=pos)
@@ -1021,7 +1025,7 @@ class UVEngine:
                                                                 cu=cu.data_ptr(), n_seg=cu.numel() - 1), run)
         else:
             h = run()
-        if head and self.hidden_is_raw and pk["last_idx"].numel() <= 1 << 16 and self._raw_logits_ok():
+        if head and self.hidden_is_raw and self._raw_logits_ok(pk["last_idx"].numel(), h.size(0)):
             return self._raw_logits(h, rows=pk["last_idx"])
         h = self._normed(h.index_select(0, pk["last_idx"]))   # (the norm of the prompts' last rows only)
         return self.logits(h) if head else h
