@@ -69,6 +69,28 @@ def test_ragged_and_edges(dtype, lens, window):
     _check(q, k, v, cu, window, 2e-3 if dtype == torch.float16 else 4e-3, expect_path=1)
 
 
+@pytest.mark.parametrize("tiles", range(1, 10))
+@pytest.mark.parametrize("H,window", [(8, None), (5, 40), (4, None), (2, 40)])
+def test_even_and_odd_counts_of_key_tiles(tiles, H, window):
+    # (one sequence's last block walks every count of 32-key tiles, the sequence behind it starts inside a tile; bars as above)
+    q, k, v, cu = _case([32 * tiles - 3, 32 * tiles + 1], H, 1, 64, torch.float16, seed=tiles)
+    _check(q, k, v, cu, window, 2e-3, expect_path=1)
+
+
+@pytest.mark.parametrize("H", [8, 4, 2])
+def test_tiles_outside_a_blocks_keys_are_not_touched(H):
+    # (NaN in the values of a sequence whose tiles no other sequence's rows share stays in that sequence)
+    q, k, v, cu = _case([64, 32, 96, 32, 32], H, 1, 64, torch.float16)
+    from ultraviolet_amd.kernels.varlen_attn import packed_attention
+    clean = packed_attention(*(t.to(DEV) for t in (q, k, v, cu)), SC)
+    v[64:96] = float("nan")
+    v[192:224] = float("nan")
+    got = packed_attention(*(t.to(DEV) for t in (q, k, v, cu)), SC)
+    for a, b in ((0, 64), (96, 192), (224, 256)):
+        assert torch.equal(got[a:b], clean[a:b])
+    assert got[64:96].isnan().all() and got[192:224].isnan().all()
+
+
 @pytest.mark.parametrize("H,K", [(1, 1), (4, 1), (5, 1), (8, 2), (6, 2), (16, 2), (8, 8)])
 def test_head_groupings(H, K):
     q, k, v, cu = _case([40, 130, 9], H, K, 64, torch.float16, seed=H * 10 + K)

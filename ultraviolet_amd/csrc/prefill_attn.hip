@@ -6,7 +6,7 @@
 //
 // prefill_attn_mfma_hd64 (head_dim 64, 16-bit q/k/v of one dtype, up to 8 query heads per kv head):
 //   * a wave owns 16 consecutive packed tokens x 2 query heads of one kv head, and walks the keys in 32-key
-//     super-tiles.  Query blocks are aligned to the packed index, not to the sequences: a block that straddles a
+//     super-tiles, two of them a step where the four waves share a block (below).  Query blocks are aligned to the packed index, not to the sequences: a block that straddles a
 //     boundary walks the union of its rows' key ranges and masks per (row, key), so the grid is ceil(N / 16) blocks
 //     with no search for "which sequence is block i in";
 //   * S^T = K . Q^T with v_mfma_f32_16x16x32 (A = 16 keys x 32 dims, B = 32 dims x 16 rows): a lane of the accumulator
@@ -17,18 +17,19 @@
 //     do the K operands (16-byte reads, lane = key m, dims 8g..8g+7 of each half);
 //   * the 4 waves of a workgroup are the 4 head pairs of a query block (2 blocks x 2 pairs for up to 4 query heads per kv head, 4
 //     blocks for up to 2) of one kv head and walk the same keys, so a super-tile of K and V is fetched once per workgroup, from
-//     global memory straight into one of three LDS stages, two tiles ahead; one barrier per tile; a wave skips the tiles outside
-//     its own block's key range;
+//     global memory straight into one of two LDS stages of two tiles, a stage ahead; one barrier per stage, an odd count's first tile ahead of
+//     the pairs (behind them, the accumulators of two step forms met in copies: 33 registers of the single form's spilled).  Where the
+//     waves are of different blocks, a wave skips the tiles outside its own block's key range;
+//   * a step of two tiles (PAIR) takes one maximum, one exponential and one rescale of the accumulators for 64 keys: of ~65 vector instructions a head and
+//     tile 33 are a step's, not a key's.  It holds 158 registers, three waves per SIMD (at four, 128, 45 of them spill and everything
+//     takes twice as long); single tiles at four waves in the same loop: 64 x 512 tokens 45.1 us against 41.9, window 256 35.7 / 34.8;
 //   * online softmax per (row, head) in the exp2 domain; tiles that every row of the block sees completely skip the
-//     mask arithmetic: one branch per tile, around the mask alone (as two versions of the whole tile, the accumulators of the two met
-//     in copies, 40 registers a tile, and it took 153 registers instead of 118, three waves per SIMD instead of four);
+//     mask arithmetic: one branch per tile, around the mask alone (two versions of the whole tile would meet in copies of the accumulators);
 //   * workgroup ids are remapped so that each XCD (one L2 each) owns a contiguous range of query blocks and therefore
 //     whole sequences, the last blocks first: they see the most keys.
-// What bounds it: vector instructions (74 % of the cycles that a SIMD is busy; the matrix cores 22 %; 64 x 512 tokens, both windows), ~135 a
-// tile and head pair of which 36 are exponentials, at 3.3 of the four waves per SIMD that it has room for.  With four heads per wave it held 255 registers, two waves per SIMD, staged
-// K and V through registers, and made eight trips to memory one after the other for its epilogue.  us, before -> now, with the
-// epilogue: 93 tokens 9.4 -> 5.3; 400 16.6 -> 8.6; 64 x 64 .. 512 tokens 41.2 -> 30.8, window 256 34.2 -> 25.2; 64 x 512 62.2 -> 43.4 and
-// 46.3 -> 34.8; 4 x 2048 without 77.6 -> 43.5; 61 x 16 .. 1024, window 256, 42.1 -> 34.6.
+// What bounds it: vector instructions, at three waves per SIMD.  us with the segment table's launch, one tile a step (118 registers, four waves) -> now: 93
+// tokens 6.7 -> 6.6; 400 12.1 -> 10.9; 64 x 64 .. 512 tokens 32.6 -> 28.9, window 256 26.3 -> 25.5; 64 x 512 45.2 -> 41.9 and
+// 37.6 -> 34.7; 4 x 2048 47.2 -> 42.0; 61 x 16 .. 1024 59.5 -> 53.6, window 256 38.5 -> 36.2; 10 x 300 on 4 query and 2 kv heads 11.7 -> 11.6.
 //
 // Everything else (fp32 K/V, other head dims) goes token by token through the decode kernel's generic path with the
 // packed K/V as a batch-stride-0 "cache".
@@ -37,6 +38,7 @@
 #include "gemm_util.h"
 
 #include <climits>
+#include <type_traits>
 
 namespace uvmi {
 
@@ -87,10 +89,12 @@ __device__ __forceinline__ float max3(float a, float b, float c) { return __buil
 // the device idle: what is repeated takes no time, and a launch of the projection alone lasts 3.4 us at 93 rows, nearly all of it its start
 // and a trip for the weights.  A whole prefill, us: 30 tokens 267 -> 245, 93 296 -> 274, 300 347 -> 323 (64 columns a part: up to 384 tokens),
 // 500 400 -> 377, 700 444 -> 422 (128: up to 768; 780 tokens, where an XCD has more workgroups than compute units, 469 -> 479).
-template <int DT, int ODT, int OP>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OP ? 1 : 4))) void prefill_attn_mfma_hd64(PrefillParams P) {
+//
+// PAIR: the waves of a workgroup share one query block (n_hg = 4), and a step takes both tiles of a stage.
+template <int DT, int ODT, int OP, bool PAIR>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OP ? 1 : (PAIR ? 3 : 4)))) void prefill_attn_mfma_hd64(PrefillParams P) {
   // one object per stage: the compiler can then tell that reads of one do not touch the one a load is filling
-  __shared__ __attribute__((aligned(1024))) unsigned char s0[2][4096], s1[2][4096], s2[2][4096];  // [K, V][32 keys x 128 B]
+  __shared__ __attribute__((aligned(1024))) unsigned char s0[2][2][4096], s1[2][2][4096];  // [tile][K, V][32 keys x 128 B]
   constexpr int OW = 16 * OP;   // weight rows of a wave, a load each
   __shared__ __attribute__((aligned(1024))) unsigned char sw[OP ? 4 * OW * 1024 : 16];
   const int tid = threadIdx.x;
@@ -155,8 +159,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OP ? 1 : 4)
   const int kend_wg = min(row0 + qbw * 16, P.N);
   const int nk = (kend_wg - kbeg_wg + 31) >> 5;   // >= 1
 
-  // ---- K / V super-tiles go from global memory straight into one of three LDS stages, two tiles ahead: wave w moves keys 8 w .. 8 w + 7
-  // of K and of V, 16 bytes per lane.  Keys are clamped to N - 1 (a clamped key is masked).  K rows keep their 16-byte chunks
+  // ---- K / V tiles go from global memory straight into one of two LDS stages of two tiles each, a stage ahead: wave w moves keys
+  // 8 w .. 8 w + 7 of K and of V, 16 bytes per lane.  Keys are clamped to N - 1 (a clamped key is masked).  K rows keep their 16-byte chunks
   // xor-ed with (key / 2) % 8, V rows theirs with 2 (key / 2 % 4), which makes the operand reads (lane = key m, chunk 4 s + g;
   // eight keys' 32 bytes per 32 lanes) free of bank conflicts.
   const uint16_t* kbase = (const uint16_t*)P.k + (int64_t)kvh * P.skh;
@@ -166,13 +170,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OP ? 1 : 4)
   const __amdgpu_buffer_rsrc_t rV = __builtin_amdgcn_make_buffer_rsrc((void*)vbase, 0, (int)((uint32_t)(P.N - 1) * svn2 + 128), 0x00020000);
   const int lkey = 8 * wave + (lane >> 3), lch = lane & 7;
   const uint32_t kch = (uint32_t)((lch ^ ((lkey >> 1) & 7)) << 4), vch = (uint32_t)((lch ^ (lkey & 6)) << 4);
-  auto issue = [&](unsigned char (*S)[4096], int k) {
+  auto issue = [&](unsigned char (*S)[4096], int k) {   // tile k
     const uint32_t r = (uint32_t)min(kbeg_wg + 32 * k + lkey, P.N - 1);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rK, (__attribute__((address_space(3))) void*)(S[0] + 1024 * wave), 16, r * skn2 + kch, 0, 0, 0);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rV, (__attribute__((address_space(3))) void*)(S[1] + 1024 * wave), 16, r * svn2 + vch, 0, 0, 0);
   };
-  issue(s0, 0);
-  if (nk > 1) issue(s1, 1);
+  const bool odd = nk & 1;   // an odd count's first tile is a step of its own, ahead of the pairs, in the second stage
+  if (odd) issue(s1[0], 0);
+  if (nk > 1) issue(s0[0], odd), issue(s0[1], odd + 1);
+  if (!odd && nk > 3) issue(s1[0], 2), issue(s1[1], 3);
   if constexpr (OP > 0) {   // row i of the wave's weight rows, 1 KB, keeps its 16-byte chunks xor-ed with i % 16
     const __amdgpu_buffer_rsrc_t rO = __builtin_amdgcn_make_buffer_rsrc((void*)P.o_w, 0, (int)((uint32_t)(P.o_n - 1) * (uint32_t)P.o_ldw * 2 + 1024u), 0x00020000);
 #pragma unroll
@@ -195,86 +201,114 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OP ? 1 : 4)
 #pragma unroll
   for (int t = 0; t < 4; t++) vld[t] = (uint32_t)(4 * g + (m >> 2)) * 128 + (uint32_t)(((2 * t + ((m & 3) >> 1)) ^ ((4 * g + (m >> 2)) & 6)) << 4) + 8 * (m & 1);
 
-  auto step = [&](const unsigned char (*S)[4096], int k) __attribute__((always_inline)) {
+  // NT tiles from tile k on: one maximum, one rescale of the accumulators for all of their keys
+  auto step = [&](const unsigned char (*S)[2][4096], int k, auto nt) __attribute__((always_inline)) {
+    constexpr int NT = decltype(nt)::value;
     const int tb = kbeg_wg + 32 * k;
-    if (tb < kbeg || tb >= kend) return;   // (wave-uniform)
-    pu4 K[4];      // [tile A dims 0..31, tile A dims 32..63, tile B dims 0..31, tile B dims 32..63]: key m, dims 8g..8g+7
-    K[0] = *(const pu4*)(S[0] + kld0);
-    K[1] = *(const pu4*)(S[0] + kld1);
-    K[2] = *(const pu4*)(S[0] + 2048 + kld0);
-    K[3] = *(const pu4*)(S[0] + 2048 + kld1);
-    pu4 VA[4];     // V^T operands: row m is head dim 16 t + m; slots 0..3 are keys 4g+j of tile A, 4..7 of tile B
+    if (!PAIR && (tb < kbeg || tb >= kend)) return;   // (wave-uniform)
+    float t[HPW][8 * NT];
 #pragma unroll
-    for (int tt = 0; tt < 4; tt++) {
-      const pu2 a = ld_tr16(S[1] + vld[tt]), b = ld_tr16(S[1] + 2048 + vld[tt]);
-      VA[tt] = pu4{a.x, a.y, b.x, b.y};
-    }
-    float t[HPW][8];
+    for (int j = 0; j < NT; j++) {
+      pu4 K[4];      // [tile A dims 0..31, tile A dims 32..63, tile B dims 0..31, tile B dims 32..63]: key m, dims 8g..8g+7
+      K[0] = *(const pu4*)(S[j][0] + kld0);
+      K[1] = *(const pu4*)(S[j][0] + kld1);
+      K[2] = *(const pu4*)(S[j][0] + 2048 + kld0);
+      K[3] = *(const pu4*)(S[j][0] + 2048 + kld1);
 #pragma unroll
-    for (int hh = 0; hh < HPW; hh++) {
-      pf4 sA = mfma16<DT>(K[0], Q[hh][0], pf4{0.f, 0.f, 0.f, 0.f});
-      pf4 sB = mfma16<DT>(K[2], Q[hh][0], pf4{0.f, 0.f, 0.f, 0.f});
-      sA = mfma16<DT>(K[1], Q[hh][1], sA);
-      sB = mfma16<DT>(K[3], Q[hh][1], sB);
+      for (int hh = 0; hh < HPW; hh++) {
+        pf4 sA = mfma16<DT>(K[0], Q[hh][0], pf4{0.f, 0.f, 0.f, 0.f});
+        pf4 sB = mfma16<DT>(K[2], Q[hh][0], pf4{0.f, 0.f, 0.f, 0.f});
+        sA = mfma16<DT>(K[1], Q[hh][1], sA);
+        sB = mfma16<DT>(K[3], Q[hh][1], sB);
 #pragma unroll
-      for (int i = 0; i < 4; i++) { t[hh][i] = sA[i]; t[hh][4 + i] = sB[i]; }
-    }
-    if (tb < lo_last || tb + 31 > r0) {   // some row of the block does not see all of the tile
-      const uint32_t kA = (uint32_t)(tb + 4 * g - lo_n);
-#pragma unroll
-      for (int i = 0; i < 8; i++) {
-        const bool out = kA + (i & 3) + 16 * (i >> 2) >= n_keys;
-#pragma unroll
-        for (int hh = 0; hh < HPW; hh++)
-          if (out) t[hh][i] = -INFINITY;
+        for (int i = 0; i < 4; i++) { t[hh][8 * j + i] = sA[i]; t[hh][8 * j + 4 + i] = sB[i]; }
       }
     }
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+      if (tb + 32 * j < lo_last || tb + 32 * j + 31 > r0) {   // some row of the block does not see all of the tile
+        const uint32_t kA = (uint32_t)(tb + 32 * j + 4 * g - lo_n);
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+          const bool out = kA + (i & 3) + 16 * (i >> 2) >= n_keys;
+#pragma unroll
+          for (int hh = 0; hh < HPW; hh++)
+            if (out) t[hh][8 * j + i] = -INFINITY;
+        }
+      }
+    float mc[HPW];
 #pragma unroll
     for (int hh = 0; hh < HPW; hh++) {
       // (the maximum that hands NaN on: one instruction for three values, where the one that ignores it needs each made quiet first; a
       // score that is NaN makes its row NaN either way)
-      const float mx = max3(max3(max3(t[hh][0], t[hh][1], t[hh][2]), t[hh][3], t[hh][4]), max3(t[hh][5], t[hh][6], t[hh][7]), mrun[hh]);
-      {  // rescale by alpha = exp2((m_old - m_new) c), 1 where the row's maximum did not grow.  Unconditional: a branch
-         // here would split the heads into separate blocks and stop the scheduler from overlapping one head's
-         // softmax arithmetic with the next head's MFMAs.  (A reference point that may lag behind the maximum, as the decode
-         // kernel's, costs precision here: the largest probability is then no longer 1, which is exact in 16 bits.)
-        const float mnew = xmaximum(mx);
-        const float alpha = mnew == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f((mrun[hh] - mnew) * c);
+      float mx = max3(t[hh][0], t[hh][1], mrun[hh]);
 #pragma unroll
-        for (int tt = 0; tt < 4; tt++) O[hh][tt] *= alpha;
-        lrun[hh] *= alpha;
-        mrun[hh] = mnew;
+      for (int i = 2; i < 8 * NT; i += 2) mx = max3(t[hh][i], t[hh][i + 1], mx);
+      // rescale by alpha = exp2((m_old - m_new) c), 1 where the row's maximum did not grow.  Unconditional: a branch
+      // here would split the heads into separate blocks and stop the scheduler from overlapping one head's
+      // softmax arithmetic with the next head's MFMAs.  (A reference point that may lag behind the maximum, as the decode
+      // kernel's, costs precision here: the largest probability is then no longer 1, which is exact in 16 bits.)
+      const float mnew = xmaximum(mx);
+      const float alpha = mnew == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f((mrun[hh] - mnew) * c);
+#pragma unroll
+      for (int tt = 0; tt < 4; tt++) O[hh][tt] *= alpha;
+      lrun[hh] *= alpha;
+      mrun[hh] = mnew;
+      mc[hh] = mnew == -INFINITY ? 0.f : mnew * c;
+    }
+#pragma unroll
+    for (int j = 0; j < NT; j++) {
+      pu4 VA[4];     // V^T operands: row m is head dim 16 t + m; slots 0..3 are keys 4g+j of tile A, 4..7 of tile B
+#pragma unroll
+      for (int tt = 0; tt < 4; tt++) {
+        const pu2 a = ld_tr16(S[j][1] + vld[tt]), b = ld_tr16(S[j][1] + 2048 + vld[tt]);
+        VA[tt] = pu4{a.x, a.y, b.x, b.y};
       }
-      const float mc = mrun[hh] == -INFINITY ? 0.f : mrun[hh] * c;
-      float p[8];
 #pragma unroll
-      for (int i = 0; i < 8; i++) p[i] = __builtin_amdgcn_exp2f(fmaf(t[hh][i], c, -mc));
-      lrun[hh] += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
-      const pu4 PB = pu4{pack2<DT>(p[0], p[1]), pack2<DT>(p[2], p[3]), pack2<DT>(p[4], p[5]), pack2<DT>(p[6], p[7])};
+      for (int hh = 0; hh < HPW; hh++) {
+        float p[8];
 #pragma unroll
-      for (int tt = 0; tt < 4; tt++) O[hh][tt] = mfma16<DT>(VA[tt], PB, O[hh][tt]);
+        for (int i = 0; i < 8; i++) p[i] = __builtin_amdgcn_exp2f(fmaf(t[hh][8 * j + i], c, -mc[hh]));
+        lrun[hh] += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+        const pu4 PB = pu4{pack2<DT>(p[0], p[1]), pack2<DT>(p[2], p[3]), pack2<DT>(p[4], p[5]), pack2<DT>(p[6], p[7])};
+#pragma unroll
+        for (int tt = 0; tt < 4; tt++) O[hh][tt] = mfma16<DT>(VA[tt], PB, O[hh][tt]);
+      }
     }
   };
-  // iteration k: tile k has landed (own loads: the wait, which leaves tile k + 1's in flight; the other waves': the barrier) and every
-  // wave is done with tile k - 1, whose stage takes tile k + 2
-  auto iteration = [&](unsigned char (*S)[4096], unsigned char (*SN)[4096], int k) {
-    if (OP > 0 && k < 2) {   // (the weight rows were requested behind tile 1)
-      if (k + 1 < nk) wait_vm<2 + OW>(); else wait_vm<OW>();
+  typedef std::integral_constant<int, 1> one;
+  typedef std::integral_constant<int, 2> two;
+  // a step's tiles have landed (own loads: the wait; the other waves': the barrier) and every wave is done with the other stage
+  auto landed = [&] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+  auto full = [&](unsigned char (*S)[2][4096], unsigned char (*SN)[2][4096], int k) __attribute__((always_inline)) {   // tiles k and k + 1
+    if (k < 2) {   // (the weight rows were requested behind the tiles that went out at the start)
+      if (k == 0 && nk > 3) wait_vm<4 + OP * 16>(); else wait_vm<OP * 16>();
+    } else if (OP > 0 && k == 2) {
+      wait_vm<OP * 16>();
     } else {
-      if (k + 1 < nk) wait_vm<2>(); else wait_vm<0>();
+      wait_vm<0>();
     }
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (k + 2 < nk) issue(SN, k + 2);
-    step(S, k);
+    landed();
+    if (k > 0 && k + 2 < nk) issue(SN[0], k + 2), issue(SN[1], k + 3);
+    if constexpr (PAIR) {
+      step(S, k, two{});
+    } else {
+      step(S, k, one{});
+      step(S + 1, k + 1, one{});
+    }
   };
   int k = 0;
-  for (; k + 3 <= nk; k += 3) {
-    iteration(s0, s2, k);
-    iteration(s1, s0, k + 1);
-    iteration(s2, s1, k + 2);
+  if (odd) {
+    if (nk > 1) wait_vm<4 + OP * 16>(); else wait_vm<OP * 16>();
+    landed();
+    step(s1, 0, one{});
+    k = 1;
   }
-  if (k < nk) iteration(s0, s2, k);
-  if (k + 1 < nk) iteration(s1, s0, k + 1);
+  for (; k + 4 <= nk; k += 4) {
+    full(s0, s1, k);
+    full(s1, s0, k + 2);
+  }
+  if (k < nk) full(s0, s1, k);
   if constexpr (OP > 0) __syncthreads();   // (the stages take the heads' outputs)
 
   // ---- normalise and store: lane (row m, group g) holds head dims 16 t + 4 g + i, t, i = 0 .. 3
@@ -453,22 +487,28 @@ static int launch_mfma(const uvmi_prefill_attn_args* a, const int32_t* seg_start
     const dim3 parts(nblk, (unsigned)(o->N / (64 * pieces)));
 #define UVMI_LO(DT)                                                                                                       \
   do {                                                                                                                    \
-    if (pieces == 1) hipLaunchKernelGGL((prefill_attn_mfma_hd64<DT, DT, 1>), parts, blk, 0, st, P);                       \
-    else hipLaunchKernelGGL((prefill_attn_mfma_hd64<DT, DT, 2>), parts, blk, 0, st, P);                                   \
+    if (pieces == 1) hipLaunchKernelGGL((prefill_attn_mfma_hd64<DT, DT, 1, true>), parts, blk, 0, st, P);                       \
+    else hipLaunchKernelGGL((prefill_attn_mfma_hd64<DT, DT, 2, true>), parts, blk, 0, st, P);                                   \
   } while (0)
     if (a->q_dtype == UVMI_F16) UVMI_LO(UVMI_F16); else UVMI_LO(UVMI_BF16);
 #undef UVMI_LO
     UVMI_CHECK_LAUNCH("uvmi_prefill_attn_o");
     return UVMI_OK;
   }
+#define UVMI_LP(QD, OD)                                                                                                  \
+  do {                                                                                                                   \
+    if (P.n_hg == 4) hipLaunchKernelGGL((prefill_attn_mfma_hd64<QD, OD, 0, true>), grid, blk, 0, st, P);                  \
+    else hipLaunchKernelGGL((prefill_attn_mfma_hd64<QD, OD, 0, false>), grid, blk, 0, st, P);                            \
+  } while (0)
 #define UVMI_L(QD)                                                                                                       \
   do {                                                                                                                   \
-    if (od == UVMI_F16) hipLaunchKernelGGL((prefill_attn_mfma_hd64<QD, UVMI_F16, 0>), grid, blk, 0, st, P);          \
-    else if (od == UVMI_BF16) hipLaunchKernelGGL((prefill_attn_mfma_hd64<QD, UVMI_BF16, 0>), grid, blk, 0, st, P);   \
-    else hipLaunchKernelGGL((prefill_attn_mfma_hd64<QD, UVMI_F32, 0>), grid, blk, 0, st, P);                         \
+    if (od == UVMI_F16) UVMI_LP(QD, UVMI_F16);                                                                           \
+    else if (od == UVMI_BF16) UVMI_LP(QD, UVMI_BF16);                                                                    \
+    else UVMI_LP(QD, UVMI_F32);                                                                                          \
   } while (0)
   if (a->q_dtype == UVMI_F16) UVMI_L(UVMI_F16); else UVMI_L(UVMI_BF16);
 #undef UVMI_L
+#undef UVMI_LP
   UVMI_CHECK_LAUNCH("uvmi_prefill_attn");
   return UVMI_OK;
 }
