@@ -281,6 +281,16 @@ def test_backward_odd_head_groups_at_block_edges(H, K, n):
             assert np.abs(a - b).max() <= 2 * 2.0 ** -7 * np.abs(b).max() + 1e-6, (lens, np.abs(a - b).max(), np.abs(b).max())
 
 
+@pytest.mark.parametrize("tiles", range(1, 8))
+@pytest.mark.parametrize("H,K,window", [(8, 1, None), (5, 1, 40), (4, 1, None), (6, 2, 40)])
+def test_backward_even_and_odd_counts_of_key_tiles(tiles, H, K, window):
+    """dq with one and two heads of a wave over every count of 32-key tiles; two roundings of the largest gradient."""
+    got, ref = _grad_case([32 * tiles - 3, 32 * tiles + 1], H, K, torch.float16, window, seed=tiles)
+    for a, b in zip(got, ref):
+        assert np.isfinite(a).all()
+        assert np.abs(a - b).max() <= 2 * 2.0 ** -10 * np.abs(b).max() + 1e-6, (np.abs(a - b).max(), np.abs(b).max())
+
+
 @pytest.mark.parametrize("window", [2, 31, 32, 33, 64, 65, 96, 97, 330, 331, 332, 2 ** 31 - 1])
 def test_attention_and_backward_at_the_mask_rules(window):
     """Windows around the places where a 32-key tile stops needing a mask, or a wave of 32 keys stops seeing a 32-query tile: both

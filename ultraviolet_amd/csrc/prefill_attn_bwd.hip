@@ -17,6 +17,7 @@
 //                   the queries that see its keys and the heads of the group; dk and dv stay in registers.
 #include "common.h"
 #include "attn_mfma_util.h"
+#include "gemm_util.h"
 
 #include <climits>
 
@@ -233,8 +234,8 @@ __global__ __launch_bounds__(64) void bwd_dkv_kernel(BwdParams P) {
 // ------------------------------------------------------------------------------------------------ the MFMA form
 // Same mathematics on the matrix cores, on the forward kernel's operand layouts (prefill_attn.hip):
 //   * the rows' log-sum-exp (log2 domain) is the forward's, or comes from one more run of the forward kernel without output;
-//   * bwd_dq_mfma: a workgroup owns 16 query rows of one kv head, wave w the query heads 2w, 2w+1 of the group.  K and V
-//     super-tiles (32 keys) are staged once per workgroup in LDS, as in the forward.  S^T = K Q^T and dP^T = V dO^T have the same shape: a lane
+//   * bwd_dq_mfma: a workgroup owns 16 query rows of one kv head, wave w the query heads 2w, 2w+1 of the group (w up to four of them).  K and V
+//     super-tiles (32 keys) are staged once per workgroup in LDS, two tiles to a barrier, as in the forward.  S^T = K Q^T and dP^T = V dO^T have the same shape: a lane
 //     of either accumulator holds 4 consecutive keys of one query row for two 16-key tiles, so p = exp2(c s - lse) and
 //     ds = p (dp - D) are lane-local, and the 8 values of ds, rounded to the input type, are the lane's slice of the B
 //     operand of dQ^T += K^T dS^T (K^T operands from the transposing LDS read, as V^T in the
@@ -306,10 +307,16 @@ __device__ __forceinline__ void store_dims16(void* base, int64_t off, const pf4*
     *(uint2*)(p + 16 * t) = uint2{pack2<DT>(acc[t][0] * mul, acc[t][1] * mul), pack2<DT>(acc[t][2] * mul, acc[t][3] * mul)};
 }
 
-template <int DT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void bwd_dq_mfma(BwdMParams P) {
+// HB: heads of a wave.  Two for a group of five to eight, 164 registers and three waves per SIMD (at four, 128, 51 of them spill; a head to each of
+// eight waves, 102 registers, reads the staged tiles twice as often and is no faster: 61 sequences of up to 1024 tokens, no window, dq and dk / dv,
+// 149 us against 143); one for up to four, where two left two or three waves without a head.  What bounds it: issue (vector instructions 47 % and
+// matrix ones 30 % of the cycles of a SIMD).  us, dq and dk / dv together, with a barrier for every tile -> for two: 64 x 64 .. 512 tokens 75.7 -> 73.8, 4 x
+// 2048 106.2 -> 103.1, 61 x 16 .. 1024 145.8 -> 143.1 and with a window of 256 88.5 -> 86.3; 4 query heads, two kv heads, 10 x 300 19.9 -> 16.9, one, 20 x 700
+// 55.6 -> 48.7.
+template <int DT, int HB>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HB == 1 ? 4 : 3))) void bwd_dq_mfma(BwdMParams P) {
   // one object per stage: the compiler can then tell that reads of one do not touch the one a load is filling
-  __shared__ __attribute__((aligned(1024))) unsigned char s0[2][4096], s1[2][4096], s2[2][4096];  // [K, V][32 keys x 128 B]
+  __shared__ __attribute__((aligned(1024))) unsigned char s0[2][2][4096], s1[2][2][4096];  // [tile][K, V][32 keys x 128 B]
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int per = gridDim.x >> 3;
   const int bid = (blockIdx.x & 7) * per + (blockIdx.x >> 3);   // an XCD (ids congruent mod 8) gets a contiguous range
@@ -321,23 +328,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void b
   const int r0 = qb * 16, row = r0 + m;
   const int rowc = row < P.N ? row : P.N - 1;
   // ---- what depends on the row alone goes out first: Q^T, dO^T and O operands (lane = row m, dims 32 s + 8 g ..), the row's statistics
-  pu4 Q[2][2], GO[2][2], Ov[2][2];
-  float lse2[2];
-  bool hok[2];
+  pu4 Q[HB][2], GO[HB][2], Ov[HB][2];
+  float lse2[HB];
+  bool hok[HB];
   int lo_n = P.seg_start[rowc];
   int n_end = (int)load_index(P.cu, P.idx64, P.n_seg);   // tokens at or after it are padding
 #pragma unroll
-  for (int hh = 0; hh < 2; hh++) {
-    const int hq = 2 * wave + hh;
+  for (int hh = 0; hh < HB; hh++) {
+    const int hq = HB * wave + hh;
     hok[hh] = hq < G;
     const int head = kvh * G + (hok[hh] ? hq : G - 1);
     const int64_t base = ((int64_t)rowc * P.H + head) * 64 + 8 * g;
-    Q[hh][0] = *(const pu4*)((const uint16_t*)P.q + base);
-    Q[hh][1] = *(const pu4*)((const uint16_t*)P.q + base + 32);
-    GO[hh][0] = *(const pu4*)((const uint16_t*)P.go + base);
-    GO[hh][1] = *(const pu4*)((const uint16_t*)P.go + base + 32);
-    Ov[hh][0] = *(const pu4*)((const uint16_t*)P.o + base);
-    Ov[hh][1] = *(const pu4*)((const uint16_t*)P.o + base + 32);
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      Q[hh][s] = *(const pu4*)((const uint16_t*)P.q + base + 32 * s);
+      GO[hh][s] = *(const pu4*)((const uint16_t*)P.go + base + 32 * s);
+      Ov[hh][s] = *(const pu4*)((const uint16_t*)P.o + base + 32 * s);
+    }
     lse2[hh] = P.lse[(int64_t)head * P.lse_ld + rowc];
   }
   __builtin_amdgcn_sched_barrier(0);
@@ -354,7 +361,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void b
   const int nk = __builtin_amdgcn_readfirstlane((kend - kbeg + 31) >> 5);
   const uint32_t n_keys = row_ok ? (uint32_t)(row - lo_n + 1) : 0u;   // the row sees keys lo_n .. lo_n + n_keys - 1 (none ahead of the first sequence)
 
-  // ---- K / V tiles go from global memory straight into one of three LDS stages, two tiles ahead: wave w moves rows 8 w .. 8 w + 7
+  // ---- K / V tiles go from global memory straight into one of two LDS stages of two tiles, a stage ahead: wave w moves rows 8 w .. 8 w + 7
   const uint32_t rstride = (uint32_t)P.KH * 128;
   const int kv_bytes = (int)((uint32_t)P.N * rstride - (uint32_t)kvh * 128);
   const __amdgpu_buffer_rsrc_t rK = __builtin_amdgcn_make_buffer_rsrc((void*)((const uint16_t*)P.k + (int64_t)kvh * 64), 0, kv_bytes, 0x00020000);
@@ -363,16 +370,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void b
   const uint32_t lch = (uint32_t)(((lane & 7) ^ tile_swizzle(lkey)) << 4);
   auto issue = [&](unsigned char (*S)[4096], int k) {   // (keys are clamped: a clamped key is masked)
     const uint32_t off = (uint32_t)min(kbeg + 32 * k + lkey, P.N - 1) * rstride + lch;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rK, (__attribute__((address_space(3))) void*)(S[0] + 1024 * wave), 16, off, 0, 0, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rV, (__attribute__((address_space(3))) void*)(S[1] + 1024 * wave), 16, off, 0, 0, 0);
+    load_lds16(rK, S[0] + 1024 * wave, off, 0);
+    load_lds16(rV, S[1] + 1024 * wave, off, 0);
   };
-  if (nk > 0) issue(s0, 0);
-  if (nk > 1) issue(s1, 1);
+  const bool odd = nk & 1;   // an odd count's first tile is a step of its own, ahead of the pairs, in the second stage
+  if (odd) issue(s1[0], 0);
+  if (nk > 1) issue(s0[0], odd), issue(s0[1], odd + 1);
+  if (!odd && nk > 3) issue(s1[0], 2), issue(s1[1], 3);
 
   // ---- D = dO . O; -D is where the accumulators of dP^T start
-  pf4 nD[2], dQ[2][4];
+  pf4 nD[HB], dQ[HB][4];
 #pragma unroll
-  for (int hh = 0; hh < 2; hh++) {
+  for (int hh = 0; hh < HB; hh++) {
     float d = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; i++) d = dot2w<DT>(GO[hh][1][i], Ov[hh][1][i], dot2w<DT>(GO[hh][0][i], Ov[hh][0][i], d));
@@ -389,10 +398,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void b
     at.rows(S[1], VA);
 #pragma unroll
     for (int t = 0; t < 4; t++) KT[t] = at.cols(S[0], t);
-    float p[2][8];
-    pf4 dP[2][2];
+    float p[HB][8];
+    pf4 dP[HB][2];
 #pragma unroll
-    for (int hh = 0; hh < 2; hh++) {
+    for (int hh = 0; hh < HB; hh++) {
       pf4 sA = pf4{0.f, 0.f, 0.f, 0.f}, sB = sA, pA = nD[hh], pB = pA;
       sA = mfma16<DT>(KA[0], Q[hh][0], sA);
       sB = mfma16<DT>(KA[2], Q[hh][0], sB);
@@ -413,12 +422,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void b
 #pragma unroll
       for (int i = 0; i < 8; i++) {
         const bool out = kA + (i & 3) + 16 * (i >> 2) >= n_keys;
-        if (out) p[0][i] = 0.f;
-        if (out) p[1][i] = 0.f;
+#pragma unroll
+        for (int hh = 0; hh < HB; hh++)
+          if (out) p[hh][i] = 0.f;
       }
     }
 #pragma unroll
-    for (int hh = 0; hh < 2; hh++) {
+    for (int hh = 0; hh < HB; hh++) {
       float ds[8];
 #pragma unroll
       for (int i = 0; i < 8; i++) ds[i] = p[hh][i] * dP[hh][i >> 2][i & 3];
@@ -428,28 +438,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void b
     }
   };
   const bool work = hok[0];   // (wave-uniform: a wave without a head only helps with the loads)
-  // iteration k: tile k has landed (own loads: the wait, which leaves tile k + 1's in flight; the other waves': the barrier) and every
-  // wave is done with tile k - 1, whose stage takes tile k + 2
-  auto iteration = [&](unsigned char (*S)[4096], unsigned char (*SN)[4096], int k) {
-    if (k + 1 < nk) __builtin_amdgcn_s_waitcnt(0x0f72); else __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(2) / (0)
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (k + 2 < nk) issue(SN, k + 2);
-    if (work) step(S, kbeg + 32 * k);
+  // a stage's tiles have landed (own loads: the wait; the other waves': the barrier) and every wave is done with the other stage
+  auto landed = [&] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+  auto full = [&](unsigned char (*S)[2][4096], unsigned char (*SN)[2][4096], int k) __attribute__((always_inline)) {   // tiles k and k + 1
+    if (k == 0 && nk > 3) wait_vm<4>(); else wait_vm<0>();
+    landed();
+    if (k > 0 && k + 2 < nk) issue(SN[0], k + 2), issue(SN[1], k + 3);
+    if (work) {
+      step(S[0], kbeg + 32 * k);
+      step(S[1], kbeg + 32 * k + 32);
+    }
   };
   int k = 0;
-  for (; k + 3 <= nk; k += 3) {
-    iteration(s0, s2, k);
-    iteration(s1, s0, k + 1);
-    iteration(s2, s1, k + 2);
+  if (odd) {
+    if (nk > 1) wait_vm<4>(); else wait_vm<0>();
+    landed();
+    if (work) step(s1[0], kbeg);
+    k = 1;
   }
-  if (k < nk) iteration(s0, s2, k);
-  if (k + 1 < nk) iteration(s1, s0, k + 1);
+  for (; k + 4 <= nk; k += 4) {
+    full(s0, s1, k);
+    full(s1, s0, k + 2);
+  }
+  if (k < nk) full(s0, s1, k);
   // ---- dq = scale dQ; lane (row m, group g) holds head dims 16 t + 4 g + i (zeros for padding rows)
   if (row < P.N) {
 #pragma unroll
-    for (int hh = 0; hh < 2; hh++) {
+    for (int hh = 0; hh < HB; hh++) {
       if (!hok[hh]) continue;
-      const int head = kvh * G + 2 * wave + hh;
+      const int head = kvh * G + HB * wave + hh;
       if (g == 0) P.dsum[(int64_t)head * P.ls + row] = row_ok ? nD[hh][0] : 0.f;
       store_dims16<DT>(P.dq, ((int64_t)row * P.H + head) * 64 + 4 * g, dQ[hh], P.scale);
     }
@@ -755,9 +772,14 @@ extern "C" int uvmi_prefill_attn_bwd(const uvmi_prefill_attn_bwd_args* a, void* 
     M.N = a->N; M.H = a->H; M.KH = a->KH; M.G = G; M.window = window;
     M.scale = a->scale; M.scale_log2 = a->scale * 1.4426950408889634f;
     M.n_wg = ((a->N + 15) / 16) * a->KH;
-    const dim3 blk4(256), gq((unsigned)((M.n_wg + 7) / 8 * 8));
-    if (a->dtype == UVMI_F16) hipLaunchKernelGGL((bwd_dq_mfma<UVMI_F16>), gq, blk4, 0, st, M);
-    else hipLaunchKernelGGL((bwd_dq_mfma<UVMI_BF16>), gq, blk4, 0, st, M);
+    const dim3 gq((unsigned)((M.n_wg + 7) / 8 * 8));
+#define UVMI_DQ(DT)                                                                                    \
+  do {                                                                                                 \
+    if (M.G > 4) hipLaunchKernelGGL((bwd_dq_mfma<DT, 2>), gq, dim3(256), 0, st, M);                    \
+    else hipLaunchKernelGGL((bwd_dq_mfma<DT, 1>), gq, dim3(256), 0, st, M);                            \
+  } while (0)
+    if (a->dtype == UVMI_F16) UVMI_DQ(UVMI_F16); else UVMI_DQ(UVMI_BF16);
+#undef UVMI_DQ
     UVMI_CHECK_LAUNCH("uvmi_prefill_attn_bwd(dq)");
     int cus = uvmi_device_cus();
     if (cus <= 0) cus = 256;
