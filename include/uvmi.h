@@ -309,7 +309,7 @@ typedef struct uvmi_prefill_attn_args {
 /* The MFMA kernel runs when hd == 64, H / KH <= 8, q and k/v share a 16-bit dtype and rows are 16-byte aligned
  * (probabilities are rounded to that dtype for P.V, accumulation is fp32); anything else that uvmi_decode_attn's
  * generic kernel accepts runs there, token by token.  Two launches: the segment table (unless segments_ready), then the
- * attention. */
+ * attention; of at most 64 sequences the MFMA kernel forms the table itself. */
 int uvmi_prefill_attn(const uvmi_prefill_attn_args* a, void* stream);
 size_t uvmi_prefill_attn_workspace_bytes(int N);
 /* 1 = MFMA kernel, 0 = generic kernel, negative = unsupported */

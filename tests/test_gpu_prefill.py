@@ -77,6 +77,30 @@ def test_even_and_odd_counts_of_key_tiles(tiles, H, window):
     _check(q, k, v, cu, window, 2e-3, expect_path=1)
 
 
+@pytest.mark.parametrize("n_seg", [1, 2, 63, 64, 65])
+@pytest.mark.parametrize("H,first,idx", [(8, 0, torch.int32), (4, 3, torch.int64), (2, 40, torch.int32)])
+def test_segment_table_of_few_and_many_sequences(n_seg, H, first, idx):
+    """Up to 64 sequences, empty ones among them, the attention finds its rows' sequences itself; the table that it leaves is the one of the launch for more
+    of them, which the same boundaries with empty sequences behind them get."""
+    from ultraviolet_amd.kernels.varlen_attn import packed_attention
+    r = np.random.default_rng(n_seg)
+    lens = r.integers(0, 20, size=n_seg) + (n_seg == 1)
+    N = first + int(lens.sum()) + 5   # (tokens ahead of the first sequence and behind the last)
+    cu = torch.from_numpy(first + np.concatenate([[0], np.cumsum(lens)])).to(idx)
+    many = torch.cat([cu, cu[-1:].expand(70)])
+    q, k, v, _ = (t.to(DEV) for t in _case([N], H, 1, 64, torch.float16, seed=n_seg))
+    got = []
+    for c in (cu, many):
+        ws = torch.zeros(2 * ((4 * N + 255) // 256 * 256), dtype=torch.uint8, device=DEV)
+        got.append((packed_attention(q, k, v, c.to(DEV), SC, 30, workspace=ws), ws))
+    seg = [w.view(torch.int32)[:N].cpu().numpy() for _, w in got]
+    c, i = cu.numpy(), np.arange(N)
+    want = c[np.maximum(np.searchsorted(c[:-1], i, side="right") - 1, 0)]
+    assert (seg[0] == np.where(want <= i, want, i + 1)).all()
+    end = int(cu[-1])   # (what follows the last sequence belongs to the empty ones in `many`)
+    assert (seg[0][:end] == seg[1][:end]).all() and torch.equal(got[0][0][:end], got[1][0][:end])
+
+
 @pytest.mark.parametrize("H", [8, 4, 2])
 def test_tiles_outside_a_blocks_keys_are_not_touched(H):
     # (NaN in the values of a sequence whose tiles no other sequence's rows share stays in that sequence)
