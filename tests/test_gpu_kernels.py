@@ -1364,6 +1364,24 @@ def test_head_of_some_rows_with_the_positions_counted_up(dtype, M, N, gather):
             assert L.lib().uvmi_head(C.byref(hb), L.stream_ptr(x)) < 0
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,tile", [(768, 128), (769, 256), (1000, 256)])
+def test_softcapped_head_where_its_tile_changes(dtype, M, tile):
+    """The tile that is named, on either side of the line, and every logit within a rounding of the product (the softcap's slope is at most 23 / 30) of float64."""
+    from ultraviolet_amd.kernels.gemm import SOFTCAP, gemm_args, gemm_path, gemm_tn
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x, w = (torch.randn(s, 640, device="cuda", generator=g).to(dtype) for s in (M, 32768))
+    w = (w.float() / 8).to(dtype)
+    kw = dict(epilogue=SOFTCAP, norm_eps=1e-6, ca=23.0, cb=5.0, cap_c=7.5)
+    got = gemm_tn(x, w, **kw)
+    assert gemm_path(gemm_args(x, w, got, **kw))[1] == tile
+    for r in range(0, M, 256):   # (a few rows at a time: the float64 logits of all of them are half a gigabyte)
+        a = x[r:r + 256].double()
+        p = (a * torch.rsqrt((a * a).mean(1, keepdim=True) + 1e-6)) @ w.double().t()
+        ulp = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+        assert ((got[r:r + 256] - 23.0 * torch.sigmoid((p + 5.0) / 7.5)).abs() <= 23 / 30 * 1.02 * ulp * p.abs() + 1e-4).all()
+
+
 @pytest.mark.parametrize("change", [dict(config=3), dict(M=64), dict(ld=8), dict(ld=131), dict(epilogue=0), dict(norm_a=1), dict(K=2048)])
 def test_sums_of_squares_are_refused_elsewhere(change):
     """Other forms of the GEMM, few rows, pitches that do not hold the rows, epilogues that neither write nor read sums: refused, nothing launched."""

@@ -83,10 +83,13 @@ static Path gemm_path(const uvmi_gemm_args* a, int cus) {
   // (also a product of fewer rows whose 256 x 256 tiles still come to two rounds of the device or more - the tied head,
   // 2048 x 32768: 104 us against 129 us on 128 x 128 tiles - or, none of their columns padding, to one full round where 128 x 128
   // tiles, two to a compute unit, take a second one: 512 x 32768 26.6 us against 29.9, with the softcap 33.7 against 47.7 and
-  // from 384 rows on 28.3 against 35.6; 288 rows 27.9 against 26.4, 384 without the softcap 26.6 against 24.1)
+  // from 384 rows on 28.3 against 35.6; 288 rows 27.9 against 26.4, 384 without the softcap 26.6 against 24.1).  With the softcap two rounds are
+  // taken from 769 rows on, where 128 x 128 tiles come to more than three: 800 rows 54.5 / 51.4 us in a stream of its own and 60.9 / 73.5 behind other
+  // work, as a step has it, 900 rows 56.3 / 59.7 and 65.0 / 78.5, 1000 rows 58.9 / 61.8 and 71.2 / 97.8 (two decode steps of 800 rows 990 -> 976 us,
+  // 900 rows 1066 -> 1032, 1000 rows 1107 -> 1052); one and a half rounds, 648 - 768 rows, and one of 257 - 352 are within half a percent of a step either way.
   const int64_t t128 = ((a->M + 127) / 128) * (((int64_t)a->N + 127) / 128), t256 = ((a->M + 255) / 256) * (((int64_t)a->N + 255) / 256);
   const bool one_round = a->N % 256 == 0 && a->M >= (a->epilogue == UVMI_GEMM_SOFTCAP ? 384 : 512) && t256 <= cus && 8 * t256 >= 7 * (int64_t)cus && t128 > 2 * (int64_t)cus;
-  const bool many_big_tiles = one_round || (a->M >= 1024 && t256 >= 2 * (int64_t)cus);
+  const bool many_big_tiles = one_round || (a->M >= (a->epilogue == UVMI_GEMM_SOFTCAP ? 769 : 1024) && t256 >= 2 * (int64_t)cus);
   const bool rows_ok = a->M >= (a->epilogue == UVMI_GEMM_SWIGLU ? BIG_MIN_ROWS_SWIGLU : BIG_MIN_ROWS);
   if (a->config == 5) return {UVMI_GEMM_PATH_BIG, 256};
   if (a->config == 0 && (many_big_tiles || rows_ok) && big_ok(a)) {
