@@ -1555,3 +1555,31 @@ def test_a_greedy_row_does_not_depend_on_the_rows_beside_it(dtype, V):
     for lo, hi in ((0, 1), (1, 256), (255, 511), (300, 557), (599, 600)):
         t, p = greedy_sample(x[lo:hi], (23.0, 5.0, 7.5))
         assert torch.equal(t, tok[lo:hi]) and torch.equal(p, lp[lo:hi]), (lo, hi)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("d", [2, 126, 130, 638, 640, 642, 768, 2046, 2048])
+@pytest.mark.parametrize("rows", [1, 6])
+def test_norms_at_the_edges_of_their_forms(dtype, d, rows):
+    """Embedding with norm and the residual norm around 640 columns, where the form of five pairs a lane ends, and at the widths that leave a lane without its
+    last pair; token ids out of range are the nearest; in place.  A value is one rounding from float64 of what it was formed from (fp32: a few)."""
+    from ultraviolet_amd import _lib as L
+    g = torch.Generator(device="cuda").manual_seed(d + rows)
+    table, y = (torch.randn(n, d, device="cuda", generator=g).to(dtype) for n in (50, rows))
+    tok = torch.tensor([3, 49, 0, -5, 70, 17][:rows], device="cuda")
+    code, eps, st = L.dtype_code(dtype), 1e-6, L.stream_ptr(table)
+    x, n, x2, n2 = (torch.full((rows, d), 7.0, device="cuda", dtype=dtype) for _ in range(4))
+    L.check(L.lib().uvmi_embed_norm(table.data_ptr(), code, table.size(0), tok.data_ptr(), rows, d, eps, x.data_ptr(), n.data_ptr(), st), "uvmi_embed_norm")
+    L.check(L.lib().uvmi_add_norm(x.data_ptr(), y.data_ptr(), code, 0.75, 1.25, rows, d, eps, x2.data_ptr(), n2.data_ptr(), st), "uvmi_add_norm")
+    same = x.clone()
+    L.check(L.lib().uvmi_add_norm(same.data_ptr(), same.data_ptr(), code, 1.0, 0.0, rows, d, eps, None, same.data_ptr(), st), "uvmi_add_norm")
+    ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -21}[dtype]
+
+    def near(a, want):
+        assert ((a.double() - want).abs() <= 1.02 * ulp * want.abs() + 1e-6).all()
+    rms = lambda t: t.double() * torch.rsqrt((t.double() ** 2).mean(1, keepdim=True) + eps)
+    near(x, rms(table[tok.clamp(0, 49)]))
+    near(n, rms(x))
+    near(x2, 0.75 * x.double() + 1.25 * y.double())
+    near(n2, rms(x2))
+    near(same, rms(x))
