@@ -183,7 +183,8 @@ size_t uvmi_decode_attn_workspace_bytes(int B, int H, int KH, int hd, int num_sp
  * items to fill the device, each chunk >= min_chunk keys, at most 64.  n_cus <= 0: query the current device. */
 int uvmi_default_splits(int64_t n_bk, int ctx, int n_cus);
 /* The splits that decode_attention takes where its caller names none: as many as pay for the combine pass behind them on this geometry (n_bk =
- * rows x kv heads, G query heads per kv head, S slots, ctx the most keys a row attends); uvmi_default_splits where the generic kernel serves it. */
+ * rows x kv heads, G query heads per kv head, S slots, ctx the most keys a row attends); uvmi_default_splits where the generic kernel serves it.  The
+ * geometry alone is asked about: a call whose strides or addresses the matrix-core kernel does not take (uvmi_decode_attn_path 0) is cut by uvmi_default_splits. */
 int uvmi_decode_attn_splits(int q_dtype, int kv_dtype, int64_t n_bk, int G, int hd, int S, int ring, int ctx, int n_cus);
 /* 1 if uvmi_decode_attn runs the MFMA kernel for these arguments (head_dim 64, up to 8 query heads per kv head, an
  * int8 cache with fp16 scales or a cache held unquantized in the q dtype, aligned rows), 0 if the generic kernel (any

@@ -81,6 +81,58 @@ def test_splits_of_a_call_that_names_none(monkeypatch, q_dtype, kv_dtype):
                     assert s * n <= 256 and ctx // s >= 128
 
 
+def _cache(kv_dtype, S, pitch, at=0, KH=1):
+    """(2, KH, S, 64) with rows `pitch` elements apart from element `at` on."""
+    return torch.zeros(at + 2 * KH * S * pitch, dtype=kv_dtype)[at:].view(2, KH, S, pitch)[..., :64]
+
+
+@pytest.mark.parametrize("kv_dtype,S,pitch,k_at,v_at,s_at,q_at,scale,ring", [
+    (torch.int8, 2048, 64, 0, 0, 0, 0, 0.1, False), (torch.int8, 2048, 72, 0, 0, 0, 0, 0.1, False), (torch.int8, 2048, 80, 0, 0, 0, 0, 0.1, False),
+    (torch.int8, 2048, 64, 8, 0, 0, 0, 0.1, False), (torch.int8, 2048, 64, 16, 4, 4, 8, 0.1, False), (torch.int8, 2048, 64, 0, 2, 0, 0, 0.1, False),
+    (torch.int8, 2048, 64, 0, 0, 2, 0, 0.1, False), (torch.int8, 2048, 64, 0, 0, 0, 4, 0.1, False), (torch.int8, 2048, 64, 0, 0, 0, 0, -0.1, False),
+    (torch.int8, 2048, 64, 0, 0, 0, 0, 0.0, False), (torch.int8, 2048, 64, 0, 0, 0, 0, 0.1, True), (torch.int8, 2052, 64, 0, 0, 0, 0, 0.1, True),
+    (torch.float16, 2048, 64, 0, 0, 0, 0, 0.1, False), (torch.float16, 2048, 68, 0, 0, 0, 0, 0.1, False), (torch.float16, 2048, 72, 8, 4, 0, 8, 0.1, False),
+    (torch.float16, 2048, 64, 4, 0, 0, 0, 0.1, False), (torch.float16, 2048, 64, 0, 2, 0, 0, 0.1, False), (torch.bfloat16, 2048, 64, 0, 0, 0, 0, 0.1, False)])
+def test_splits_of_a_call_follow_the_kernel_that_serves_it(monkeypatch, kv_dtype, S, pitch, k_at, v_at, s_at, q_at, scale, ring):
+    """Strides and addresses that the matrix-core kernel does not take leave a call to the generic one, whose rows are cut by default_splits: in eager
+    calls by uvmi_decode_attn_path's answer, in traced ones by the same rules over strides and offsets."""
+    taken = []
+    monkeypatch.setattr(D, "_device_cus", lambda index: 256)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(D.L, "require_cuda", lambda *t: None)
+    monkeypatch.setattr(D, "_launch", lambda q, *a, **k: taken.append(a[9]) or torch.zeros_like(q))
+    monkeypatch.setattr(D, "_decode_attn_op", lambda q, *a, **k: taken.append(a[9]) or torch.zeros_like(q))
+    q = torch.zeros(q_at + 2 * 8 * 64, dtype=torch.float16)[q_at:].view(2, 8, 64)
+    k, v = _cache(kv_dtype, S, pitch, k_at), _cache(kv_dtype, S, pitch, v_at)
+    ks, vs = (torch.zeros(s_at + 2 * S, dtype=torch.float16)[s_at:].view(2, 1, S) for _ in range(2)) if kv_dtype == torch.int8 else (None, None)
+    pos = torch.zeros(2, dtype=torch.long)
+    a, keep = D.build_attn_args(q, k, v, pos, pos, scale, 0, ring, ks, vs, 1, torch.zeros_like(q))
+    served = D.L.lib().uvmi_decode_attn_path(ctypes.byref(a))
+    splits = lambda: D.decode_attention(q, k, v, pos, pos, scale, ring=ring, k_scale=ks, v_scale=vs)
+    splits()
+    with _Passing():
+        splits()
+    want = D._own_splits(q.dtype, kv_dtype, 2, 8, 64, S, ring, S) if served == 1 else D.default_splits(2, S)
+    assert served in (0, 1) and taken == [want] * 2 and (served == 1 or want == 8)
+
+
+def test_splits_of_a_compiled_call(monkeypatch):
+    """torch.compile takes the whole call, and cuts it by its strides."""
+    monkeypatch.setattr(D, "_device_cus", lambda index: 256)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(D.L, "require_cuda", lambda *t: None)
+    taken = []
+
+    def backend(gm, example):
+        taken.extend(n.args[10] for n in gm.graph.nodes if "decode_attn" in str(n.target))
+        return lambda *a: (torch.zeros(2, 8, 64),)
+    q, pos = torch.zeros(2, 8, 64).half(), torch.zeros(2, dtype=torch.long)
+    for pitch in (64, 68):
+        torch._dynamo.reset()
+        torch.compile(lambda k: D.decode_attention(q, k, k, pos, pos, 0.1), backend=backend, fullgraph=True)(_cache(torch.float16, 2048, pitch))
+    assert taken == [D._own_splits(torch.float16, torch.float16, 2, 8, 64, 2048, False, 2048), D.default_splits(2, 2048)]
+
+
 @pytest.mark.parametrize("V,d,n,of", [(32768, 640, 1, 1), (32768, 640, 65536, 1 << 20), (32768, 640, 65537, 65537), (32768, 640, 64, (1 << 29) // 640 - 64),
                                       (32768, 640, 64, (1 << 20) + 1), (524288, 1024, 8, 8), (524224, 1024, 8, 8), (524208, 1024, 8, 8), (4096, 8192, 65536, 65536),
                                       (4096, 8192, 65472, 65472), (4096, 8192, 65471, 65471), (4096, 8256, 8, 8), (4096, 96, 8, 8), (4104, 640, 8, 8), (4096, 64, 8, 8)])

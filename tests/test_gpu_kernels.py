@@ -1196,6 +1196,29 @@ def test_eager_calls_go_through_the_native_path(monkeypatch, kw):
         D.decode_attention(q, k, v, pos, starts, 0.1, k_scale=ks, v_scale=vs, **kw)
 
 
+@pytest.mark.parametrize("int8,pitch,served", [(True, 64, 1), (True, 72, 0), (False, 64, 1), (False, 68, 0)])
+def test_native_call_is_cut_for_the_kernel_that_serves_it(int8, pitch, served):
+    """A key pitch that the matrix-core kernel does not take: rows are cut as default_splits has it, not by the other kernel's rule (2000 int8
+    keys in one piece).  A call in one piece allocates its output alone, equal cuts give equal bits."""
+    import ctypes
+
+    from ultraviolet_amd.kernels import decode_attn as D
+    B, S = 4, 2000
+    q, k, v, ks, vs = (None if t is None else t.to(DEV) for t in attn_case(B, 1, 8, 64, S, int8, dtype=torch.float16))
+    wide = torch.zeros(B, 1, S, pitch, device=DEV, dtype=k.dtype)
+    wide[..., :64] = k
+    k = wide[..., :64]
+    pos, starts = torch.arange(B, device=DEV) * 600 + 100, torch.zeros(B, dtype=torch.long, device=DEV)
+    a, keep = D.build_attn_args(q, k, v, pos, starts, 0.14, 0, False, ks, vs, 1, torch.empty_like(q))
+    assert D.L.lib().uvmi_decode_attn_path(ctypes.byref(a)) == served
+    want = D._own_splits(q.dtype, k.dtype, B, 8, 64, S, False, S, DEV) if served else D.default_splits(B, S, DEV)
+    allocations = lambda: torch.cuda.memory_stats()["allocation.all.allocated"]
+    before = allocations()
+    got = D.decode_attention(q, k, v, pos, starts, 0.14, k_scale=ks, v_scale=vs)
+    assert allocations() - before == (2 if want > 1 else 1) and (served or want == 7)
+    assert torch.equal(got, D.decode_attention(q, k, v, pos, starts, 0.14, k_scale=ks, v_scale=vs, num_splits=want))
+
+
 def test_native_call_refuses_what_the_general_one_refuses(monkeypatch):
     """The library's refusals come back as the same exception; nothing is launched."""
     from ultraviolet_amd import _lib as L

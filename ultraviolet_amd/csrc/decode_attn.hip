@@ -1422,7 +1422,8 @@ extern "C" int uvmi_default_splits(int64_t n_bk, int ctx, int n_cus) {
 // than 128 keys gain nothing.  us on the GPU, rows up to that many keys without / with splits: int8 4 rows of 4096 11.0 / 7.9, of 2048 7.4 / 7.5; 64 rows of
 // 4096 12.2 / 10.2, of 2048 8.1 / 8.6; 100 rows of 4096 in two 12.5 / 13.1; 178 rows of 2048 8.6 / 12.4; 16-bit 16 rows of 1024
 // 8.7 / 7.7, of 2048 13.6 / 7.9; 64 rows of 2048 13.7 / 9.6; 128 rows of 2048 14.7 / 13.4, of 4096 24.9 / 20.5; 178 rows of 4096 25.4 / 32.1.
-// The generic kernel, a wave to an item, keeps uvmi_default_splits.
+// The generic kernel, a wave to an item, keeps uvmi_default_splits, also where it serves such a geometry for its strides or addresses, which the caller asks
+// uvmi_decode_attn_path about (an int8 cache at a key pitch of 72: 1 row of 2000 keys 205 us so and 1066 uncut, 64 rows 535 / 1975).
 extern "C" int uvmi_decode_attn_splits(int q_dtype, int kv_dtype, int64_t n_bk, int G, int hd, int S, int ring, int ctx, int n_cus) {
   const bool kv16 = kv_dtype == q_dtype;
   const bool mfma = hd == 64 && G <= 8 && (q_dtype == UVMI_F16 || q_dtype == UVMI_BF16) && (kv16 || kv_dtype == UVMI_I8) && S >= 32 &&

@@ -122,8 +122,17 @@ PyObject* py_decode_attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (args[10] == Py_None) a.ring = a.window > 0;
   else if (PyBool_Check(args[10])) a.ring = args[10] == Py_True;
   else Py_RETURN_NONE;
+  const int fp32 = PyObject_IsTrue(args[13]);
+  if (fp32 < 0) return nullptr;
+  if (!as_int(args[14], a.chunk_keys)) Py_RETURN_NONE;
+  at::Tensor out, ws;
+  auto allocate = [&] {
+    out = at::empty(q.sizes(), fp32 ? q.options().dtype(at::kFloat) : q.options());
+    a.out = out.data_ptr(); a.out_dtype = dtype_code(out); a.sob = out.stride(0); a.soh = out.stride(1);
+  };
   if (args[12] != Py_None) {
     if (!as_int(args[12], a.num_splits)) Py_RETURN_NONE;
+    allocate();
   } else {
     int ctx = 0;
     if (args[11] != Py_None && !as_int(args[11], ctx)) Py_RETURN_NONE;
@@ -138,18 +147,18 @@ PyObject* py_decode_attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
       if (!r || !as_int(r, cus)) return nullptr;
       device_cus[dev].store(cus, std::memory_order_relaxed);
     }
-    a.num_splits = uvmi_decode_attn_splits(qd, kd, static_cast<int64_t>(a.B) * a.KH, a.KH > 0 ? a.H / a.KH : 0, a.hd, a.S, a.ring, ctx, cus);
+    allocate();
+    // (how a row is best cut depends on the kernel that serves the call, which its strides and addresses have a say in)
+    a.num_splits = 1;
+    const int64_t work = static_cast<int64_t>(a.B) * a.KH;
+    if (uvmi_decode_attn_path(&a) == 1) a.num_splits = uvmi_decode_attn_splits(qd, kd, work, a.H / a.KH, a.hd, a.S, a.ring, ctx, cus);
+    else a.num_splits = uvmi_default_splits(work, ctx, cus);
   }
-  const int fp32 = PyObject_IsTrue(args[13]);
-  if (fp32 < 0) return nullptr;
-  if (!as_int(args[14], a.chunk_keys)) Py_RETURN_NONE;
   THPObjectPtr dev(PyLong_FromLong(q.get_device()));
   THPObjectPtr st(dev ? PyObject_CallFunctionObjArgs(raw_stream_fn, dev.get(), nullptr) : nullptr);
   if (!st) return nullptr;
   void* stream = PyLong_AsVoidPtr(st);
   if (PyErr_Occurred()) return nullptr;
-  at::Tensor out = at::empty(q.sizes(), fp32 ? q.options().dtype(at::kFloat) : q.options()), ws;
-  a.out = out.data_ptr(); a.out_dtype = dtype_code(out); a.sob = out.stride(0); a.soh = out.stride(1);
   if (a.num_splits > 1) {
     a.workspace_bytes = uvmi_decode_attn_workspace_bytes(a.B, a.H, a.KH, a.hd, a.num_splits);
     ws = at::empty({static_cast<int64_t>(a.workspace_bytes)}, q.options().dtype(at::kByte));

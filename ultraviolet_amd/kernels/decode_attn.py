@@ -87,6 +87,37 @@ def _own_splits(q_dtype, kv_dtype, n_bk: int, G: int, hd: int, S: int, ring: boo
     return s if saved >= (1000 if kv16 else 2900) else 1
 
 
+def _matrix_cores(q: Tensor, k: Tensor, v: Tensor, k_scale: Tensor | None, v_scale: Tensor | None, scale: float, ring: bool, address) -> bool:
+    """uvmi_decode_attn_path of a call whose output is a new tensor, for calls that are traced.  address: of a tensor, up to a multiple of 16."""
+    hd, S, kv16 = q.size(-1), k.size(2), k.dtype == q.dtype
+    if (hd != 64 or not 1 <= q.size(1) // max(k.size(1), 1) <= 8 or q.dtype not in (torch.float16, torch.bfloat16) or not (kv16 or k.dtype == torch.int8)
+            or not scale > 0 or S < 32 or (ring and S % 32) or (not kv16 and S % 4)):
+        return False
+
+    def aligned(t, n, strides, of):   # to n bytes, the strides to `of` elements
+        return address(t) % n == 0 and not any(s % of for s in strides)
+    if not (0 <= k.stride(2) <= (1 << 19 if kv16 else 1 << 20) and 0 <= v.stride(2) <= (1 << 19 if kv16 else 1 << 20)):
+        return False
+    if not (aligned(q, 16, q.stride()[:2], 8) and aligned(k, 16, k.stride()[:3], 8 if kv16 else 16) and aligned(v, 8 if kv16 else 4, v.stride()[:3], 4)):
+        return False
+    return kv16 or (k_scale is not None and v_scale is not None and aligned(k_scale, 8, k_scale.stride()[:2], 4) and aligned(v_scale, 8, v_scale.stride()[:2], 4))
+
+
+def _splits_of(q: Tensor, k: Tensor, v: Tensor, k_scale: Tensor | None, v_scale: Tensor | None, scale: float, ring: bool, ctx: int) -> int:
+    """The splits of a call that names none: how a row is best cut depends on the kernel that serves the call, which strides and addresses have a
+    say in.  (A traced operand has no address yet: its offset in its storage stands for it, and under torch.compile, which knows none, nothing.)"""
+    if plain_eager(q, k, v, k_scale, v_scale):
+        address = torch.Tensor.data_ptr
+    elif torch.compiler.is_compiling():
+        address = lambda t: 0
+    else:
+        address = lambda t: t.storage_offset() * t.element_size()
+    n, G, S = q.size(0) * k.size(1), q.size(1) // k.size(1) if k.size(1) else 0, k.size(2)
+    if _matrix_cores(q, k, v, k_scale, v_scale, scale, ring, address):
+        return _own_splits(q.dtype, k.dtype, n, G, q.size(2), S, ring, ctx, q.device)
+    return default_splits(n, ctx, q.device)
+
+
 def supported(q: Tensor, k_cache: Tensor) -> bool:
     """True when the MFMA kernel serves this geometry (reference: decode_attn_cuda.supported,
     decode_attn_cuda.py:265-270): head_dim 64, up to 8 query heads per kv head, an int8 cache or one in the q dtype.  Other
@@ -243,12 +274,12 @@ def decode_attention(q: Tensor, k_cache: Tensor, v_cache: Tensor, pos: Tensor, s
         ring = window > 0
     if rows is not None:
         rows = rows.to(pos.dtype).contiguous()
+    q = q.contiguous() if q.stride(-1) != 1 else q
     if num_splits is None:
         ctx = ctx_hint or S
         if window > 0:
             ctx = min(ctx, window)
-        num_splits = _own_splits(q.dtype, k_cache.dtype, B * KH, H // KH if KH else 0, hd, S, bool(ring), int(ctx), q.device)
-    q = q.contiguous() if q.stride(-1) != 1 else q
+        num_splits = _splits_of(q, k_cache, v_cache, k_scale, v_scale, float(scale), bool(ring), int(ctx))
     if pos.dtype != starts.dtype:
         starts = starts.to(pos.dtype)
     pos, starts = pos.contiguous(), starts.contiguous()
