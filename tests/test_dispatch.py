@@ -151,6 +151,30 @@ def test_logits_of_raw_hidden_are_asked_for_where_the_library_takes_them(V, d, n
     assert UVEngine._raw_logits_ok(e, n, of) == takes
 
 
+@pytest.mark.parametrize("d", [192, 256, 640, 1024, 1088])
+@pytest.mark.parametrize("H,f", [(1, 640), (2, 640), (8, 64), (8, 128), (1, 64), (8, 1664), (128, 8192)])
+@pytest.mark.parametrize("n", [12287, 12288, 40000, 65536, 65537])
+def test_passes_keep_sums_of_squares_where_the_library_takes_all_four_products(d, H, f, n):
+    """A width that uvmi_gemm_sums refuses for one of them runs as it did without.  (Asked with sums that lie where they may not, the library answers for the
+    shape first and launches nothing.)"""
+    from types import SimpleNamespace as N
+
+    from ultraviolet_amd import _lib as L
+    from ultraviolet_amd.engine.model import UVEngine
+    from ultraviolet_amd.engine.weights import UVWeights
+    from ultraviolet_amd.kernels.gemm import RESID, STORE, SWIGLU
+    cfg = N(d_model=d, n_heads=H, n_kv_heads=1, head_dim=64, d_ff=f)
+    e = N(cfg=cfg, big_rows=12288, fold_qkv_rows=1 << 17, gemm_config=0)
+    ext = UVWeights.qkv_ext_rows(cfg)
+
+    def refused(epilogue, cols, K, out, norm):
+        g = L.GemmArgs(a=256, w=256, c=256, dtype=L.dtype_code(torch.bfloat16), M=n, N=cols, K=K, lda=K, ldw=K, ldc=out, epilogue=epilogue, norm_a=norm, eps=1e-6,
+                       resid=256 if epilogue == RESID else None, ldr=out)
+        return L.lib().uvmi_gemm_sums(ctypes.byref(L.GemmSumsArgs(ctypes.addressof(g), 4, 1 << 17)), None) == -2
+    takes = not any(refused(*p) for p in [(STORE, ext, d, ext, 1), (RESID, d, H * 64, d, 0), (SWIGLU, 2 * f, d, f, 1), (RESID, d, f, d, 0)])
+    assert UVEngine._sums_ok(e, n) == takes or (n == 65536 and f == 8192)   # (which no product of this library takes, with sums or without)
+
+
 def test_guard_of_recorded_passes_sees_what_changes():
     """Everything that launches took an address or a number from: a tensor replaced, moved under its object, a scalar, an entry that
     comes or goes - in the weights and in the state; by torch's comparison of addresses and by the list of them."""

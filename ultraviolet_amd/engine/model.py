@@ -244,8 +244,11 @@ class UVEngine:
         """Whether the residual updates of a packed pass sum the squares of the hidden they write for the projections that take its norm.
         Formed again in every tile that reads it, it is a sixteenth of their matrix instructions: gate-up at 18 432 rows 86 us against 79 so, extended
         projection 22.7 / 21.4; at 33 216 rows 144 / 133, 37.7 / 35.9; the updates pay 0.4 - 1 us each (a pass of 64 prompts 2252 -> 2200 us, a
-        mixed one 3901 -> 3824).  All four have to run on the kernels of many rows."""
-        return n >= max(self.big_rows, 12288) and n <= min(self.fold_qkv_rows, 1 << 16) and self.gemm_config == 0 and 256 <= self.cfg.d_model <= 1024
+        mixed one 3901 -> 3824).  All four have to run on the kernels of many rows (uvmi_gemm_sums' rule: the updates' two contractions are over the
+        heads' columns and over d_ff)."""
+        cfg = self.cfg
+        return (n >= max(self.big_rows, 12288) and n <= min(self.fold_qkv_rows, 1 << 16) and self.gemm_config == 0 and 256 <= cfg.d_model <= 1024
+                and cfg.n_heads * cfg.head_dim >= 128 and cfg.d_ff >= 128)
 
     def _embed_norm(self, tok: Tensor, n: int):
         b = self.buf
