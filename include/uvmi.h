@@ -40,8 +40,8 @@ extern "C" {
 #define UVMI_I32 4
 #define UVMI_I64 5
 
-/* Revision of the argument structs below (uvmi_version() returns the value the library was built with). */
-#define UVMI_ABI_VERSION 8
+/* Revision of the argument structs and entry points below (uvmi_version() returns the value the library was built with). */
+#define UVMI_ABI_VERSION 9
 int uvmi_version(void);
 const char* uvmi_last_error(void);
 /* Number of compute units of the current device (used by the split heuristics); <0 on error. */

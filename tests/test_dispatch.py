@@ -276,6 +276,36 @@ def test_native_path_of_another_build_is_not_loaded(monkeypatch, tmp_path):
         none_of_it("does not load")
 
 
+@pytest.mark.parametrize("lacks", ["prefill_attn_args_bytes", "varlen_attention", "revision"])
+def test_native_path_that_lacks_something_is_another_build(monkeypatch, lacks):
+    """An extension without what this one asks it for is refused as one of another revision is, and calls take the general path."""
+    from types import SimpleNamespace as N
+
+    from ultraviolet_amd.kernels import varlen_attn as V
+    L = D.L
+    real = L.eager()
+    old = N(**{a: getattr(real, a) for a in dir(real) if not a.startswith("__") and a != lacks})
+    monkeypatch.setattr(L, "_eager", None)
+    monkeypatch.setattr(L.importlib.util, "spec_from_file_location", lambda *a: N(loader=N(exec_module=lambda m: None)))
+    monkeypatch.setattr(L.importlib.util, "module_from_spec", lambda spec: old)
+    with pytest.raises(L.UvmiError, match="rebuild"):
+        L.eager()
+    for native, n in ((D._native, 15), (V._native, 6)):
+        native.cache_clear()
+        with pytest.warns(UserWarning, match="rebuild"):
+            assert native()(*[None] * n) is None
+        native.cache_clear()
+
+
+def test_library_that_lacks_an_entry_point_is_refused(monkeypatch):
+    from types import SimpleNamespace as N
+    L = D.L
+    monkeypatch.setattr(L, "_lib", None)
+    monkeypatch.setattr(L.C, "CDLL", lambda path: N(uvmi_version=lambda: L.ABI_VERSION))
+    with pytest.raises(L.UvmiError, match="uvmi_decode_attn_splits.*rebuild"):
+        L.lib()
+
+
 def test_library_is_built_where_the_extension_cannot_be(monkeypatch, tmp_path, capsys):
     """A compiler or headers that are missing cost the extension only, and an older one does not stay."""
     from ultraviolet_amd.csrc import build as B

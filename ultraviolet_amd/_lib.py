@@ -164,7 +164,7 @@ class HeadArgs(C.Structure):   # struct uvmi_head_args
 OP_GEMM, OP_DECODE_ATTN, OP_QKV_POST, OP_PREFILL_ATTN, OP_NORM, OP_QKV_PROJ, OP_PREFILL_ATTN_O, OP_GEMM_RESID, OP_GEMM_SUMS = range(9)   # UVMI_OP_*
 
 _lib = None
-ABI_VERSION = 8   # UVMI_ABI_VERSION of include/uvmi.h
+ABI_VERSION = 9   # UVMI_ABI_VERSION of include/uvmi.h
 
 
 def lib() -> C.CDLL:
@@ -178,6 +178,9 @@ def lib() -> C.CDLL:
         if L.uvmi_version() != ABI_VERSION:   # the ctypes structs below mirror one revision of include/uvmi.h
             raise UvmiError(f"{LIB_PATH} was built for revision {L.uvmi_version()} of include/uvmi.h, these bindings are for "
                             f"{ABI_VERSION}: rebuild it with `python -m ultraviolet_amd.csrc.build`")
+        missing = [n for n in EXPORTS if not hasattr(L, n)]
+        if missing:
+            raise UvmiError(f"{LIB_PATH} lacks {', '.join(missing)}: rebuild it with `python -m ultraviolet_amd.csrc.build`")
         L.uvmi_last_error.restype = C.c_char_p
         L.uvmi_decode_attn_workspace_bytes.restype = C.c_size_t
         L.uvmi_decode_attn_workspace_bytes.argtypes = [C.c_int] * 5
@@ -261,9 +264,11 @@ def eager():
         except ImportError as e:
             raise UvmiError(f"{EAGER_PATH} does not load: {e}") from e
         # (it fills the argument structs itself, and calls whichever libuvmi.so the loader found for it)
-        sizes = (mod.attn_args_bytes, mod.prefill_attn_args_bytes, mod.prefill_attn_bwd_args_bytes)
-        if not (mod.revision == mod.library_revision == ABI_VERSION and sizes == tuple(C.sizeof(t) for t in (AttnArgs, PrefillAttnArgs, PrefillAttnBwdArgs))):
-            raise UvmiError(f"{EAGER_PATH} was built for revision {mod.revision} of include/uvmi.h and calls a library of revision {mod.library_revision}, these "
+        # (an attribute that it does not have is another build's, too)
+        revision, library, *sizes = (getattr(mod, a, None) for a in ("revision", "library_revision", "attn_args_bytes", "prefill_attn_args_bytes", "prefill_attn_bwd_args_bytes"))
+        if not (revision == library == ABI_VERSION and sizes == [C.sizeof(t) for t in (AttnArgs, PrefillAttnArgs, PrefillAttnBwdArgs)]
+                and hasattr(mod, "decode_attention") and hasattr(mod, "varlen_attention")):
+            raise UvmiError(f"{EAGER_PATH} was built for revision {revision} of include/uvmi.h and calls a library of revision {library}, these "
                             f"bindings are for {ABI_VERSION}: rebuild it with `python -m ultraviolet_amd.csrc.build`")
         _eager = mod
     return _eager
