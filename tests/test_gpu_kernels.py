@@ -1606,3 +1606,9 @@ def test_norms_at_the_edges_of_their_forms(dtype, d, rows):
     near(x2, 0.75 * x.double() + 1.25 * y.double())
     near(n2, rms(x2))
     near(same, rms(x))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("d", [128, 256, 258, 384, 386, 512, 514, 770, 896, 898, 1024, 1026, 1280, 1282, 1536, 1538])
+def test_norms_at_the_edges_of_every_form(dtype, d):
+    test_norms_at_the_edges_of_their_forms(dtype, d, 6)

@@ -85,6 +85,8 @@ __device__ __forceinline__ void st8(void* p, int64_t i, const float (&v)[8]) {
 // A row is a chain of trips - its token, its elements, its stores - and its elements are requested together: pairs past the row are read from its last one
 // and count as zeros.  (With a branch around each pair every load was waited for by itself, five of them at d = 640.)  Embedding
 // and norm, d = 640, us in a stream: 1 row 3.3 -> 2.9, 512 rows 3.8 -> 2.9, 18 432 rows 17.5 -> 13.3, 33 216 29.2 -> 21.5 (5.9 TB/s); the same bits.
+// Requests past the row's end cost what the row's own do, so NP is the width's: residual norm of 33 216 rows with branches / in the form of 5 or 16 pairs /
+// now, d = 64 9.3 / 11.9 / 6.4, 642 29.0 / 31.9 / 26.7, 768 31.6 / 32.3 / 30.0, 1280 67.0 / 60.1 / 60.2; 4096 rows of 768 6.0 / 7.1 / 5.1.
 template <int DT, int MODE, int NP>
 __global__ __launch_bounds__(256) void norm_kernel(const void* __restrict__ xin, const void* __restrict__ yin,
                                                    const int64_t* __restrict__ tok, int64_t vocab, float a, float b,
@@ -112,8 +114,8 @@ __global__ __launch_bounds__(256) void norm_kernel(const void* __restrict__ xin,
 #pragma unroll
   for (int i = 0; i < NP; i++) {
     if (MODE == 1) {
-      v0[i] = round_t<DT>(a * v0[i] + b * y0[i]);
-      v1[i] = round_t<DT>(a * v1[i] + b * y1[i]);
+      v0[i] = round_t<DT>(fmaf(a, v0[i], b * y0[i]));   // (which product is rounded is said, for the forms' results to be the same bits)
+      v1[i] = round_t<DT>(fmaf(a, v1[i], b * y1[i]));
     }
     if (lane + 64 * i >= np) v0[i] = v1[i] = 0.f;
     ss += v0[i] * v0[i] + v1[i] * v1[i];
@@ -735,6 +737,15 @@ static void dispatch_dt(int dt, F&& f) {
   else f(std::integral_constant<int, UVMI_F32>{});
 }
 
+// the smallest of the forms (ascending) that has `need` pairs a lane, the last one if none has
+template <int NP, int... MORE, typename F>
+static void norm_form(int need, F&& go) {
+  if constexpr (sizeof...(MORE) > 0) {
+    if (need > NP) return norm_form<MORE...>(need, go);
+  }
+  go(std::integral_constant<int, NP>{});
+}
+
 namespace uvmi {
 int norm_run(const uvmi_norm_args* a, void* stream) {
   const bool embed = a->tok != nullptr;
@@ -750,7 +761,7 @@ int norm_run(const uvmi_norm_args* a, void* stream) {
       if (embed) hipLaunchKernelGGL((norm_kernel<D, 0, n>), grid, blk, 0, (hipStream_t)stream, a->x, nullptr, a->tok, a->vocab, 0.f, 0.f, a->h_out, a->n_out, a->rows, a->d, a->eps, a->advance);
       else hipLaunchKernelGGL((norm_kernel<D, 1, n>), grid, blk, 0, (hipStream_t)stream, a->x, a->y, nullptr, 0, a->a, a->b, a->h_out, a->n_out, a->rows, a->d, a->eps, a->advance);
     };
-    if (a->d <= 640) go(std::integral_constant<int, 5>{}); else go(std::integral_constant<int, 16>{});
+    norm_form<1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 16>((a->d + 127) / 128, go);
   });
   UVMI_CHECK_LAUNCH(embed ? "uvmi_embed_norm" : "uvmi_add_norm");
   return UVMI_OK;
