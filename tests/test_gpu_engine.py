@@ -1106,3 +1106,43 @@ def test_a_refused_single_prompt_leaves_the_state_alone(dtype, kv):
         assert all([torch.equal(a, b) for a, b in zip(before, tensors)]) and np.array_equal(st.host_pos, host)
     m.prefill(idx, torch.zeros(1, dtype=torch.long, device=DEV), st, rows=rows)
     assert st.pos.tolist() == [11, 21, 11] and st.host_pos.tolist() == [11, 21, 11] and not torch.equal(before[0][1], st.k[0][1])
+
+
+@pytest.mark.parametrize("dtype,kv", [(torch.bfloat16, "int8"), (torch.bfloat16, "fp16"), (torch.float16, "int8"), (torch.float32, "int8")])
+@pytest.mark.parametrize("rows", [8, 5, 40])
+def test_logits_with_the_norm_in_the_heads_launch_equal_those_of_the_normed_hidden(monkeypatch, dtype, kv, rows):
+    """decode_logits and prefill_logits against logits() of decode_step and prefill, the first time and from the recorded pass, also in steps of fewer rows than the
+    state has, which still move every position; the states end alike.  The normed hidden is rounded ahead of the product in the one and not in the other, and
+    both round the product: u sum |n w| + 2 u |n w| (u: half a step of the activation type), times the softcap's steepest slope."""
+    from ultraviolet_amd.engine import KVState
+    cfg, _, eng, _ = _setup(window=32, dtype=dtype)
+    n = 40 if rows == 40 else 8
+    prompts = _prompts(cfg, np.arange(n) % 13 + 1)
+    a, b = (KVState(cfg, n, 64, DEV, kv_dtype=kv, dtype=dtype if dtype != torch.float32 else torch.bfloat16) for _ in range(2))
+    ca, _, c = cfg.softcap
+    u = {torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -12, torch.float32: 0.0}[dtype]
+    W = eng.w.embed.double()
+    raw = []
+    of_raw = eng._raw_logits
+    monkeypatch.setattr(eng, "_raw_logits", lambda *a, **k: raw.append(1) or of_raw(*a, **k))
+
+    def near(got, hidden):
+        h = hidden.double()
+        bound = ca / c / 4 * (u * (h.abs() @ W.abs().T) + 2 * u * (h @ W.T).abs() + 1e-6 * (h.abs() @ W.abs().T)) + 1e-5
+        assert got.dtype == torch.float32 and ((got.double() - eng.logits(hidden).double()).abs() <= bound).all()
+    if rows == n:
+        for _ in range(2):
+            hidden = eng.prefill(prompts, list(range(n)), a).clone()
+            near(eng.prefill_logits(prompts, list(range(n)), b), hidden)
+    else:
+        for st in (a, b):
+            eng.prefill(prompts, list(range(n)), st)
+    tok = torch.as_tensor(np.random.default_rng(1).integers(1, cfg.vocab_size, size=(4, rows)), device=DEV)
+    for t in range(4):
+        pos = a.pos.clone()
+        hidden = eng.decode_step(tok[t], a).clone()
+        near(eng.decode_logits(tok[t], b), hidden)
+        assert torch.equal(a.pos, pos + 1) and torch.equal(b.pos, a.pos)
+    assert len(raw) == (0 if dtype == torch.float32 else 4 + 2 * (rows == n))
+    for l in range(cfg.n_layers):
+        assert torch.equal(a.k[l], b.k[l]) and torch.equal(a.v[l], b.v[l])
