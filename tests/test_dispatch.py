@@ -175,6 +175,16 @@ def test_passes_keep_sums_of_squares_where_the_library_takes_all_four_products(d
     assert UVEngine._sums_ok(e, n) == takes or (n == 65536 and f == 8192)   # (which no product of this library takes, with sums or without)
 
 
+@pytest.mark.parametrize("M,N,K,tile", [(12288, 256, 256, 0), (16000, 256, 640, 0), (24576, 256, 2048, 0), (32768, 256, 512, 0), (33216, 256, 512, 192), (16000, 64, 512, 0),
+                                        (40000, 128, 1664, 0), (21760, 384, 1024, 0), (22000, 384, 1024, 192), (13056, 640, 512, 0), (14000, 640, 512, 192), (18432, 640, 1664, 192)])
+def test_residual_updates_of_one_round_keep_the_smaller_tiles(M, N, K, tile):
+    """192 x 128 tiles are for updates whose 128 x 128 ones are more than a round of the device (512 of them on 256 compute units)."""
+    from ultraviolet_amd import _lib as L
+    from ultraviolet_amd.kernels.gemm import RESID
+    g = L.GemmArgs(a=256, w=256, c=256, dtype=L.dtype_code(torch.bfloat16), M=M, N=N, K=K, lda=K, ldw=K, ldc=N, epilogue=RESID, resid=256, ldr=N)
+    assert L.lib().uvmi_gemm_resid_tile(ctypes.byref(g)) == tile
+
+
 def test_guard_of_recorded_passes_sees_what_changes():
     """Everything that launches took an address or a number from: a tensor replaced, moved under its object, a scalar, an entry that
     comes or goes - in the weights and in the state; by torch's comparison of addresses and by the list of them."""

@@ -156,7 +156,9 @@ extern "C" int uvmi_gemm_tn(const void* a, const void* w, void* c, int dtype, in
 // tiles 1.7 of one of 128 x 128 ones.  us, 128 / 192 / 256, 640 columns, K 1664 and 512: 12 288 rows 30.1 / 38.1 / 45.0 and 15.2 /
 // 18.5 / 22.1; 14 000 46.3 / 38.3 / 45.3 and 21.2 / 19.7 / 22.5; 18 432 47.3 / 41.6 / 48.6 and 22.6 / 21.5 / 23.8; 20 000 52.1 / 56.9 / 47.7 and
 // 26.2 / 28.1 / 24.3; 24 576 54.9 / 57.0 / 86.5 and 27.3 / 28.0 / 41.3; 28 000 71.6 / 61.6 / 88.9 and 32.7 / 29.6 / 41.8; 33 216 77.2 / 79.0 /
-// 90.6 and 37.6 / 36.5 / 43.8; 50 000 106.8 / 116.2 / 131.9 and 49.4 / 52.4 / 60.4.
+// 90.6 and 37.6 / 36.5 / 43.8; 50 000 106.8 / 116.2 / 131.9 and 49.4 / 52.4 / 60.4.  Those are last rounds, which start while the one before ends: an update
+// whose 128 x 128 tiles are one round has no use for larger ones (256 columns, K 256, 512 and 2048: 16 000 rows 7.4 / 9.0, 9.7 / 11.7 and 26.8 / 28.7; 24 576 10.2 / 10.1,
+// 15.2 / 14.5 and 30.9 / 32.8; two rounds, 33 216 rows, 16.4 / 14.2, 22.1 / 18.4 and 49.7 in 256 x 256 ones / 43.2; 128 columns, K 1664, 40 000 rows 31.1 / 34.9).
 static bool resid_192(const uvmi_gemm_args* a, int cus) {
   if (a->epilogue != UVMI_GEMM_RESID || a->norm_a || a->config != 0 || a->M < BIG_MIN_ROWS || !big_ok(a)) return false;
   const int64_t slots = 2 * (int64_t)cus, n128 = ((int64_t)a->N + 127) / 128;
@@ -165,8 +167,10 @@ static bool resid_192(const uvmi_gemm_args* a, int cus) {
     return tiles / slots * full + (rest == 0 ? 0 : (rest <= cus ? part : full));
   };
   const int64_t t256 = ((a->M + 255) / 256) * (((int64_t)a->N + 255) / 256);
+  const int64_t t128 = ((a->M + 127) / 128) * n128;
+  if (t128 <= slots) return false;
   const int64_t c192 = rounds(((a->M + 191) / 192) * n128, 148, 59);
-  return c192 < rounds(((a->M + 127) / 128) * n128, 100, 64) && c192 < (t256 + cus - 1) / cus * 170;
+  return c192 < rounds(t128, 100, 64) && c192 < (t256 + cus - 1) / cus * 170;
 }
 
 extern "C" int uvmi_gemm_resid_tile(const uvmi_gemm_args* a) {
