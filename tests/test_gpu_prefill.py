@@ -344,6 +344,18 @@ def test_backward_of_keys_by_heads_and_strides(G, K, lens, window):
         assert np.abs(a - b).max() <= 2 * 2.0 ** -10 * np.abs(b).max() + 1e-6, (np.abs(a - b).max(), np.abs(b).max())
 
 
+@pytest.mark.parametrize("G,K,lens,window", [(8, 1, [64], None), (8, 1, [63], None), (8, 2, [70] * 66, None), (5, 1, [200, 1, 90], 65), (3, 1, [330, 5, 200], 170), (4, 1, [160], None),
+                                             (2, 1, [641, 640], None), (2, 1, [900], 700), (1, 1, [1290], None), (1, 2, [1400], 1300), (8, 10, [820, 3], None), (2, 10, [900], None),
+                                             (1, 10, [1300], None)])
+def test_backward_of_keys_by_mean_sequence_and_window(G, K, lens, window):
+    """dk / dv on either side of the lines that give it eight waves a workgroup or four: the mean sequence, cut to the window, for every padding of the head
+    group, up to a workgroup per compute unit and beyond.  Tolerance as above."""
+    got, ref = _grad_case(lens, G * K, K, torch.float16, window, seed=9)
+    for a, b in zip(got, ref):
+        assert np.isfinite(a).all()
+        assert np.abs(a - b).max() <= 2 * 2.0 ** -10 * np.abs(b).max() + 1e-6, (np.abs(a - b).max(), np.abs(b).max())
+
+
 @pytest.mark.parametrize("window", [33, 167, 168, 2 ** 31 - 1])
 def test_plain_backward_with_windows_that_hide_few_keys_and_none(window):
     """16 query heads on a kv head, which the plain kernels serve: windows up to the largest that an int holds.  Tolerance as above."""

@@ -720,6 +720,21 @@ extern "C" size_t uvmi_prefill_attn_bwd_workspace_bytes(int N, int H) {
   return ((size_t)2 * (size_t)(H > 0 ? H : 0) * ls + 2 * ls) * 4 + 256;   // lse, D (H, ls); segment table, scratch (ls)
 }
 
+// Whether dk / dv takes eight waves a workgroup rather than four: a wave for each of 8 heads, or twice the strides of query tiles, so the row of tiles
+// of the keys that the most queries see, which a launch lasts as long as, is half as long.  Its waves have to have tiles: `keys` is the mean
+// sequence, cut to the window.  us, dq and dk / dv, four / eight, workgroups with compute units of their own: 8 heads 2500 tokens in sequences of
+// 16 14.3 / 15.1, of 40 15.2 / 15.5, of 100 19.2 / 18.4, of 250 34.5 / 30.0; 4 heads of 100 13.3 / 13.9, of 250 21.9 / 20.3; 2 heads of 250 14.8 / 15.3, of 700
+// 27.7 / 25.8, 4096 tokens with a window of 256 13.2 / 13.9; one head 1500 tokens 26.4 / 25.8, with a window 11.7 / 12.6.  Eight waves leave a unit one
+// workgroup: up to two rounds of them pay where sequences are long and no window shortens them (8 heads 16 of 1024 99.8 / 83.2, 24 of up to 1024 95.0 / 79.3, 3 of
+// 4096 286 / 294, 30 of 512 58.1 / 61.3; 4 heads 57.8 / 50.4, 56.4 / 50.5, 158 / 163, 37.6 / 41.5; 2 heads 37.7 / 36.6, one 28.8 / 30.3), with short ones they do not
+// (8 heads 20 000 tokens in sequences of 16 38.8 / 45.6, of 100 45.8 / 53.7; 10 000 of 40 26.3 / 31.4), nor with a window (24 of up to 1024 68.2 / 70.9) or a third round
+// (10 of 2048 210 / 218; 39 of up to 933 95.0 / 93.4 is the exception).
+static bool dkv_wide(int G, int64_t n_wg, int64_t mean, int window, int cus) {
+  const int64_t keys = window > 0 && window < mean ? window : mean, least = G > 4 ? 64 : (G > 2 ? 160 : (G > 1 ? 640 : 1280));
+  if (n_wg <= cus) return keys >= least;
+  return window == 0 && G > 1 && n_wg <= 2 * (int64_t)cus && keys >= (least > 400 ? least : 400);
+}
+
 extern "C" int uvmi_prefill_attn_bwd(const uvmi_prefill_attn_bwd_args* a, void* stream) {
   UVMI_REQUIRE(a, UVMI_EINVAL, "uvmi_prefill_attn_bwd: null arguments");
   UVMI_REQUIRE(a->N >= 0 && a->H > 0 && a->KH > 0 && a->H % a->KH == 0 && a->n_seg >= 0, UVMI_EINVAL, "uvmi_prefill_attn_bwd: bad sizes");
@@ -784,11 +799,7 @@ extern "C" int uvmi_prefill_attn_bwd(const uvmi_prefill_attn_bwd_args* a, void* 
     int cus = uvmi_device_cus();
     if (cus <= 0) cus = 256;
     M.n_wg = ((a->N + 31) / 32) * a->KH;
-    // A wave for each of 8 heads where workgroups have compute units of their own, or where there is no window: a launch lasts as long as the keys
-    // that the most queries see, whose row of tiles is then half as long (forward and backward, 16 sequences of up to 1024 tokens, 260
-    // workgroups, 96.7 us against 107.7; 24, 390, 114.5 / 117.4; 39 of up to 933, 582, 139.1 / 142.3; 61, 991, 213.0 / 212.1).  A window
-    // makes the rows short, and two workgroups on a unit cover each other's ends (24 sequences 70.9 / 68.2, 61 138.4 / 129.0).
-    const bool wide = M.n_wg <= cus || (window == 0 && 2 * M.n_wg <= 5 * cus);
+    const bool wide = dkv_wide(G, M.n_wg, a->n_seg > 0 ? a->N / a->n_seg : a->N, window, cus);
     const dim3 gk((unsigned)((M.n_wg + 7) / 8 * 8));
 #define UVMI_DKV_W(DT, GP)                                                                   \
   do {                                                                                       \
