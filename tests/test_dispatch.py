@@ -116,6 +116,16 @@ def test_splits_of_a_call_follow_the_kernel_that_serves_it(monkeypatch, kv_dtype
     assert served in (0, 1) and taken == [want] * 2 and (served == 1 or want == 8)
 
 
+def test_rows_that_default_splits_leaves_whole_are_whole_by_either_rule():
+    """What the native call rests on: it asks for the kernel that serves a call only where default_splits would cut its rows."""
+    lib = D.L.lib()
+    for q, kv in ((torch.float16, torch.int8), (torch.bfloat16, torch.bfloat16)):
+        for n in (0, 1, 2, 64, 127, 128, 129, 255, 256, 257, 5000):
+            for ctx in (*range(0, 6000, 61), 511, 512, 767, 768, 999, 1000, 1024, 2900, 100000):
+                if lib.uvmi_default_splits(n, ctx, 256) == 1:
+                    assert lib.uvmi_decode_attn_splits(D.L.dtype_code(q), D.L.dtype_code(kv), n, 8, 64, 1 << 20, 0, ctx, 256) == 1
+
+
 def test_splits_of_a_compiled_call(monkeypatch):
     """torch.compile takes the whole call, and cuts it by its strides."""
     monkeypatch.setattr(D, "_device_cus", lambda index: 256)

@@ -149,10 +149,11 @@ PyObject* py_decode_attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
     }
     allocate();
     // (how a row is best cut depends on the kernel that serves the call, which its strides and addresses have a say in)
-    a.num_splits = 1;
+    // (the generic kernel's rule cuts wherever the other one does: where it does not, there is nothing to ask)
     const int64_t work = static_cast<int64_t>(a.B) * a.KH;
-    if (uvmi_decode_attn_path(&a) == 1) a.num_splits = uvmi_decode_attn_splits(qd, kd, work, a.H / a.KH, a.hd, a.S, a.ring, ctx, cus);
-    else a.num_splits = uvmi_default_splits(work, ctx, cus);
+    const int generic = uvmi_default_splits(work, ctx, cus);
+    a.num_splits = 1;
+    if (generic > 1) a.num_splits = uvmi_decode_attn_path(&a) == 1 ? uvmi_decode_attn_splits(qd, kd, work, a.H / a.KH, a.hd, a.S, a.ring, ctx, cus) : generic;
   }
   THPObjectPtr dev(PyLong_FromLong(q.get_device()));
   THPObjectPtr st(dev ? PyObject_CallFunctionObjArgs(raw_stream_fn, dev.get(), nullptr) : nullptr);
