@@ -107,7 +107,9 @@ def test_splits_of_a_call_follow_the_kernel_that_serves_it(monkeypatch, kv_dtype
     ks, vs = (torch.zeros(s_at + 2 * S, dtype=torch.float16)[s_at:].view(2, 1, S) for _ in range(2)) if kv_dtype == torch.int8 else (None, None)
     pos = torch.zeros(2, dtype=torch.long)
     a, keep = D.build_attn_args(q, k, v, pos, pos, scale, 0, ring, ks, vs, 1, torch.zeros_like(q))
-    served = D.L.lib().uvmi_decode_attn_path(ctypes.byref(a))
+    path = D.L.lib().uvmi_decode_attn_path
+    monkeypatch.setattr(path, "argtypes", [ctypes.POINTER(D.L.AttnArgs)])   # (another test binds the library to a structure of its own)
+    served = path(ctypes.byref(a))
     splits = lambda: D.decode_attention(q, k, v, pos, pos, scale, ring=ring, k_scale=ks, v_scale=vs)
     splits()
     with _Passing():
