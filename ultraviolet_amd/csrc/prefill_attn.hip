@@ -22,14 +22,18 @@
 //     waves are of different blocks, a wave skips the tiles outside its own block's key range;
 //   * a step of two tiles (PAIR) takes one maximum, one exponential and one rescale of the accumulators for 64 keys: of ~65 vector instructions a head and
 //     tile 33 are a step's, not a key's.  It holds 158 registers, three waves per SIMD (at four, 128, 45 of them spill and everything
-//     takes twice as long); single tiles at four waves in the same loop: 64 x 512 tokens 45.1 us against 41.9, window 256 35.7 / 34.8;
+//     takes twice as long); single tiles at four waves in the same loop, both behind a launch for the segment table: 64 x 512 tokens 45.1 us
+//     against 41.9, window 256 35.7 / 34.8;
 //   * online softmax per (row, head) in the exp2 domain; tiles that every row of the block sees completely skip the
 //     mask arithmetic: one branch per tile, around the mask alone (two versions of the whole tile would meet in copies of the accumulators);
 //   * workgroup ids are remapped so that each XCD (one L2 each) owns a contiguous range of query blocks and therefore
 //     whole sequences, the last blocks first: they see the most keys.
-// What bounds it: vector instructions, at three waves per SIMD.  us with the segment table's launch, one tile a step (118 registers, four waves) -> now: 93
-// tokens 6.7 -> 6.6; 400 12.1 -> 10.9; 64 x 64 .. 512 tokens 32.6 -> 28.9, window 256 26.3 -> 25.5; 64 x 512 45.2 -> 41.9 and
-// 37.6 -> 34.7; 4 x 2048 47.2 -> 42.0; 61 x 16 .. 1024 59.5 -> 53.6, window 256 38.5 -> 36.2; 10 x 300 on 4 query and 2 kv heads 11.7 -> 11.6.
+// What bounds it: vector instructions, at three waves per SIMD.  us of calls in a graph, one tile a step (118 registers, four waves) behind a launch
+// for the segment table -> now, two tiles and the rows' sequences found here (up to 64 of them): 93 tokens 6.4 -> 5.0; 400 11.7 -> 9.1; 64 x 64 .. 512
+// tokens 30.2 -> 25.2, window 256 24.7 -> 22.1; 64 x 512 42.4 -> 38.4 and 35.5 -> 31.8; 4 x 2048 45.3 -> 38.3; 61 x 16 .. 1024 58.9 -> 50.8, window 256 38.3 ->
+// 33.5; 10 x 300 on 4 query and 2 kv heads 11.5 -> 9.9.  Groups of up to 4 query heads per kv head, table at hand, take single tiles from the same stages: 2 - 8 %
+// faster (8 and 2 heads 1 x 4096 71.2 -> 66.2, 61 x 16 .. 1024 55.8 -> 55.1) but for equal long sequences whose workgroups come to between one and two a compute
+// unit (2 x 4096 90.3 -> 94.7, 4 x 2048 43.5 -> 45.4); three stages of one tile are no faster there in this kernel (91.7) and slower elsewhere (1 x 4096 71.6).
 //
 // Everything else (fp32 K/V, other head dims) goes token by token through the decode kernel's generic path with the
 // packed K/V as a batch-stride-0 "cache".

@@ -790,7 +790,9 @@ class UVEngine:
     def _raw_logits(self, hidden: Tensor, rows: Tensor | None = None, advance: Tensor | None = None) -> Tensor:
         """logits() of rows `rows` (all) of what a trunk left un-normalised in buf x: the final norm is the row scale of the product, the rows are
         gathered by the GEMM's loads and positions `advance` counted up by its launch.  (One launch less a decode step, two
-        less a prefill: a step of 37 rows 245.7 -> 242.1 us, of 512 413.5 -> 409.9, a prefill of 93 tokens, which waits for the host, 245 -> 241.)"""
+        less a prefill: a step of 37 rows 245.7 -> 242.1 us, of 512 413.5 -> 409.9, a prefill of 93 tokens, which waits for the host, 245 -> 241.  Of
+        one row, where a head on 128-row tiles costs 2 us more with the norm in it and the host is as slow as the GPU, 188 -> 182 and 190 -> 181 on two machines,
+        medians of 8 and 4 processes; from 1 to 384 rows no count is slower by more than the runs of one differ.)"""
         ca, cb, c = self.cfg.softcap
         W = self.w.embed
         n = hidden.size(0) if rows is None else rows.numel()

@@ -1,7 +1,7 @@
 """Packed (cu_seqlens) causal attention with an optional sliding window: host side of uvmi_prefill_attn.
 
 Mirrors ultraviolet/kernels/varlen_attn.py of the reference: the forward (:87-93) on the MFMA kernel, and the backward
-(:56-84) in a first, plain form (uvmi_prefill_attn_bwd), wired into autograd as the reference wires its custom ops.
+(:56-84; uvmi_prefill_attn_bwd: matrix cores, or its plain form for groups of more than 8 query heads), wired into autograd as the reference wires its custom ops.
 q / k / v must be device tensors; there is no CPU path."""
 from __future__ import annotations
 
